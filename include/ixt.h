@@ -387,8 +387,9 @@ int ixt_set_sampling_ranges(ixt_ctx* ctx, const int32_t* lo_hi, int nranges);
  *   "ring_cfg"               0 (default): tile chosen per shape; 1: 128 x 128, 2: 128 rows x 64 columns, 3: 64 x 32
  *   "ring_split"             1: ixt_op_dot's ring GEMM runs split over the 512-k chains (one f32 slice per chain)
  *   "ring_wlayout"           1: ixt_op_dot stores its weights in the ring layout ([n/128][k/64][16 fragments]: one sequential stream per block)
- *   "attn_tile"              1 (default): prefill calls of at least "attn_tile_min_rows" rows (default 64) run the tiled attention: 16 (8 past
- *                            ~1500 keys) consecutive rows per block share every K / V load; 0: one block per (row, kv head) as for decode rows
+ *   "attn_tile"              1 (default): prefill calls of at least "attn_tile_min_rows" rows (default 64) run the tiled attention, 16 (other
+ *                            page sizes: 8 past ~1500 keys) consecutive rows per block: on the f32 matrix units for 32-token pages and at most 4096
+ *                            keys, on the vector units otherwise; 2: always on the vector units; 0: one block per (row, kv head) as for decode rows
  *   "unembed_tall"           1 (default): the unembedding at 129..256 rows uses 256 x 128 tiles (weights enter the chip once); 0: 128 x 128
  *   "ring_two_per_cu"        1 (default): ring GEMMs (and the unembedding) of 1024 rows and more with at least 320 tiles of 128 x 128 use 32-k chunks
  *                            in 4 slots (64 KiB of LDS: two blocks per CU overlap each other's prologue and epilogue); 0: the 64-k chunk form

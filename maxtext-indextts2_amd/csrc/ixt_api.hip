@@ -1151,6 +1151,7 @@ static int tile_attn_t(ixt_ctx* c, int layer, int R, int lmax, size_t lds, hipSt
   LAUNCHCHK();
   return IXT_OK;
 }
+static bool mtile_attn_fits(const ixt_ctx* c, int lmax) { return c->attn_tile == 1 && c->geom.P == 32 && lmax <= 4096; }   // k_attn_mtile
 static size_t tile_attn_lds(const ixt_ctx* c, int nq, int lmax) {
   const int ppb = 4 * (64 / (c->D / 4));   // pages of a PV pass
   return sizeof(float) * ((size_t)nq * lmax + (size_t)nq * ((c->geom.mpg + 3) & ~3) + (size_t)ppb * (nq / 2) * c->D);
@@ -1158,10 +1159,16 @@ static size_t tile_attn_lds(const ixt_ctx* c, int nq, int lmax) {
 static bool tile_attn_fits(const ixt_ctx* c, int R, int len_hint, bool decode) {
   if (decode || !c->attn_tile || R < c->attn_tile_min_rows) return false;
   const int lmax = (std::min(len_hint, c->Tmax) + 3) & ~3;
-  return tile_attn_lds(c, 8, lmax) <= 150 * 1024;
+  return mtile_attn_fits(c, lmax) || tile_attn_lds(c, 8, lmax) <= 150 * 1024;
 }
 static int launch_attention_tile(ixt_ctx* c, int layer, int R, int len_hint, hipStream_t st, float cap = 0.0f, int window = 0) {
   const int lmax = (std::min(len_hint, c->Tmax) + 3) & ~3;
+  if (mtile_attn_fits(c, lmax)) {
+    TileAttnArgs ta;
+    ta.row_slot = c->row_slot; ta.row_pos = c->row_pos; ta.row_active = c->row_active; ta.page_map = c->ps.page_map;
+    ta.qbuf = c->qbuf; ta.kpages = c->kpages_l[layer]; ta.vpages = c->vpages_l[layer]; ta.out = c->ao; ta.g = c->geom; ta.R = R; ta.lmax = lmax; ta.cap = cap; ta.window = window;
+    if (launch_mtile_attn(ta, c->D, c->GQ, st)) { LAUNCHCHK(); return IXT_OK; }
+  }
   const bool wide = tile_attn_lds(c, 16, lmax) <= 150 * 1024 && c->D <= 128;   // (head_dim 256 with 16 vectors: 100+ bytes of scratch per lane)
   const size_t lds = tile_attn_lds(c, wide ? 16 : 8, lmax);
 #define ATT(HD_, GQ_)                                                                             \

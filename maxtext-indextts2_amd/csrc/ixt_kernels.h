@@ -1702,7 +1702,8 @@ __global__ __launch_bounds__(256) void k_attn_decode_w(DecAttnArgs a, int npairs
 //      vectors run side by side.  Softmax: one wave per four query vectors, their phases interleaved.
 //      PV: lane = (page, 4 d), page chains for all NQ vectors in registers; the page sums meet in LDS, where the thread that owns
 //      (vector, d) adds them up four pages at a time and in order.  Rows of a tile that sit in different page groups (a tile across the
-//      border of two packed prompts) are worked off group by group.  grid = (nkv, ceil(R / TQ)), block 256;
+//      border of two packed prompts) are worked off group by group.  (Pages of 32 tokens and up to 4096 keys: k_attn_mtile, ixt_tile_attn.h;
+//      this form is for the other page sizes and longer prefixes.)  grid = (nkv, ceil(R / TQ)), block 256;
 //      LDS = NQ x lmax scores + 4 x mpg page sums + (256 / (HD / 4)) x NQ / 2 x HD page chains.
 struct TileAttnArgs {
   const int32_t* row_slot; const int32_t* row_pos; const int32_t* row_active; const int32_t* page_map;
@@ -1715,6 +1716,7 @@ struct TileAttnArgs {
   float cap;                          // > 0: score = ixt_tanh(score / cap) * cap before the max (attn_logits_soft_cap, attentions.py:1257-1259), as k_attn_pv
   int window;                         // > 0: keys j <= pos - window are invisible (LOCAL_SLIDING, attentions.py:625-631): e_j = p_j = +0, every sum unchanged
 };
+bool launch_mtile_attn(const TileAttnArgs& ta, int hd, int gq, hipStream_t st);   // ixt_tile_attn.hip; false: no such head geometry
 typedef uint32_t ixt_u32x16 __attribute__((ext_vector_type(16)));
 typedef float ixt_f32x2 __attribute__((ext_vector_type(2)));
 typedef const __attribute__((address_space(4))) ixt_u32x16* ixt_cq16p;   // constant address space: uniform reads become scalar loads

@@ -1,0 +1,335 @@
+// ixt_tile_attn.h -- prefill attention on the f32 matrix units, for pages of 32 tokens.
+//
+// v_mfma_f32_16x16x4_f32 adds its four products to the accumulator one after the other, k ascending, each step one IEEE fma (subnormals kept): on
+// 10^6 cells of random bf16 and f32 operands, down to subnormal sums, its result is the chain of four fmaf bit for bit.  So the contract's chains --
+// a score is one fma chain over d, an output one fma chain over the tokens of a page -- run on it unchanged, at 140 TFLOP/s where the vector units'
+// chains (k_attn_tile) reached 17.
+#pragma once
+#include "ixt_kernels.h"
+
+typedef float ixt_f32x4 __attribute__((ext_vector_type(4)));
+
+// rows 1 and 3 of `a` (16 lanes each) against rows 0 and 2 of `b` / the upper half of `a` against the lower half of `b`
+__device__ __forceinline__ void ixt_swap16(uint32_t& a, uint32_t& b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+  a = r[0]; b = r[1];
+}
+__device__ __forceinline__ void ixt_swap32(uint32_t& a, uint32_t& b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+  a = r[0]; b = r[1];
+}
+
+// 32 consecutive d of 16 keys, lane (key, c) holding the bf16 d = 8 c .. 8 c + 7, as the matrix operands of eight steps: out[s] on lane (key, c) is
+// d = 4 s + c.  `sel`: v_perm selector of the lane's half of a dword, as f32.
+__device__ __forceinline__ void ixt_k_operands(const u32x4& w, uint32_t sel, float (&out)[8]) {
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    uint32_t a = h ? w.z : w.x, b = h ? w.w : w.y;
+    ixt_swap32(a, b);
+    uint32_t a1 = a, b1 = b;
+    ixt_swap16(a, a1);
+    ixt_swap16(b, b1);
+    out[0 + h] = __uint_as_float(__builtin_amdgcn_perm(a, 0u, sel)); out[2 + h] = __uint_as_float(__builtin_amdgcn_perm(a1, 0u, sel));
+    out[4 + h] = __uint_as_float(__builtin_amdgcn_perm(b, 0u, sel)); out[6 + h] = __uint_as_float(__builtin_amdgcn_perm(b1, 0u, sel));
+  }
+}
+
+// block = (kv head, 16 query vectors = 16 / GQ consecutive rows x GQ heads), NW waves.  Super-block (4 pages, 128 keys) n NW + w belongs to wave w in
+// round n; its 128 x 16 scores stay in that wave's registers from the score products to the output products, so the keys one block holds are
+// 128 NW NR and nothing of them goes through LDS or memory.
+//   Scores: matrix rows = keys, columns = query vectors.  Row i of tile t is token 4 t + i % 4 of page i / 4: a lane then holds the 32 tokens of ONE
+//   page (its 16-lane group) for one query vector, and the page's sum of exponentials is a sum over its own registers, in order.  K is read once, 16
+//   bytes a lane, and turned into operands by lane swaps; the query operand comes from LDS, one read per eight products.
+//   Softmax: max over lanes and waves; page sums meet in LDS and every lane adds its vector's in page order.  e / l with one reciprocal per lane:
+//   two corrections of the quotient give the correctly rounded one where no remainder is subnormal (e >= 2^-96); otherwise the divide itself.
+//   Outputs: matrix rows = value columns, P as the other operand after a 4 x 4 transpose of lane groups and registers.  A lane's 16 bytes of V are 8
+//   columns of one token: column 8 i + x belongs to row i of tile x.  Page chains start from zero, four pages add up in order; the super-blocks of a
+//   round meet in LDS, where the thread that owns (vector, column) adds them in order.
+// A key that a row does not see has P = +0 (k_attn_tile says why that is exact); tokens past the end are re-reads of the last one.
+// Rows of other page groups in the tile are worked off group by group.  grid = (kv heads, tiles, 1 or the number of 128-column parts of a value):
+// with z = 2 the two halves of head_dim 256 go to two blocks, each taking the scores anew -- for launches that leave CUs idle otherwise.
+// Bound by the matrix units and, between their phases, by the vector work of the softmax (a block's waves are in the same phase).  Measured against
+// k_attn_tile, 16 heads of 128: 8 packed prompts (1525 rows, <= 251 keys) 128.6 -> 69.6 us; 1024 rows at <= 1024 / 2048 / 3072 keys 282 -> 106,
+// 860 -> 215, 1143 -> 356 us; 828 rows at <= 3900 keys 1496 -> 455 us (52 TFLOP/s).  8 heads of 256 on 4, 256 rows at <= 3072 keys: 320 -> 130 us.
+// Two waves per block for <= 256 keys: with four, two of them had nothing to do (90.2 us).
+template <int HD, int GQ, int NW, int NR>
+__global__ __launch_bounds__(NW * 64, NR == 1 && NW <= 4 ? 3 : 2) void k_attn_mtile(TileAttnArgs a) {
+  constexpr int TQ = 16 / GQ;
+  constexpr int NB = HD / 32;
+  constexpr int VW = HD >= 128 ? 128 : HD;     // value columns of one output pass
+  constexpr int NE = VW / 16;                  // matrix tiles of them
+  constexpr int NEH = NE / 2, CH = VW / 2, OP = CH + 4;
+  constexpr int NTOT = 16 * CH / (NW * 64);    // (vector, column) totals per thread and half
+  static_assert(16 % GQ == 0 && HD % 64 == 0 && (HD <= 128 || HD % 128 == 0), "tile geometry");
+  __shared__ __attribute__((aligned(16))) float qs[HD / 4 * 64];         // step s, lane l: d = 4 s + l / 16 of vector l % 16
+  __shared__ float psum[NW * NR * 4 * 16];                               // [page][vector]
+  __shared__ float wmax[NW * 16];
+  __shared__ __attribute__((aligned(16))) float ob[NW * 16 * OP];        // [wave][vector][half the columns]
+  __shared__ int s_pos[TQ], s_slot[TQ];
+  const AttnGeom& g = a.g;
+  const int kvh = blockIdx.x, r0 = (gridDim.y - 1 - blockIdx.y) * TQ;    // the rows with the most keys first
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, i16 = lane & 15, lg = lane >> 4;
+  const int n_out = g.nq * HD;
+  if (tid < TQ) {
+    const int r = r0 + tid;
+    const bool ok = r < a.R && a.row_active[r] != 0;
+    s_pos[tid] = ok ? a.row_pos[r] : -1;
+    s_slot[tid] = ok ? a.row_slot[r] : -1;
+  }
+  for (int it = tid; it < 16 * (HD / 8); it += NW * 64) {
+    const int v = it & 15, c = it >> 4;
+    const u32x4 w = *reinterpret_cast<const u32x4*>(a.qbuf + ((size_t)min(r0 + v / GQ, a.R - 1) * g.nq + kvh * GQ + v % GQ) * HD + c * 8);
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+      qs[(2 * c + (x >> 1)) * 64 + (2 * x & 3) * 16 + v] = bflo(w[x]);
+      qs[(2 * c + (x >> 1)) * 64 + ((2 * x & 3) + 1) * 16 + v] = bfhi(w[x]);
+    }
+  }
+  __syncthreads();
+  unsigned pending = 0;
+#pragma unroll
+  for (int i = 0; i < TQ; ++i) {
+    const bool act = __builtin_amdgcn_readfirstlane(s_pos[i]) >= 0;
+    if (act) pending |= 1u << i;
+    else if (r0 + i < a.R && blockIdx.z == 0) {          // idle row: zeros, as the per-row kernel writes
+      for (int idx = tid; idx < GQ * HD; idx += NW * 64) a.out[xidx(r0 + i, kvh * GQ * HD + idx, n_out)] = 0;
+    }
+  }
+  const uint32_t sel = (lg & 1) ? 0x07060c0cu : 0x05040c0cu;
+  while (pending != 0) {
+    // the rows of the leader's page group
+    const int lead = __builtin_ctz(pending);
+    const int slot = __builtin_amdgcn_readfirstlane(s_slot[lead]);
+    unsigned grp = 0;
+    int posmax = -1;
+#pragma unroll
+    for (int i = 0; i < TQ; ++i) {
+      const int ps_ = __builtin_amdgcn_readfirstlane(s_pos[i]), sl_ = __builtin_amdgcn_readfirstlane(s_slot[i]);
+      const bool in = ((pending >> i) & 1u) && sl_ == slot && ps_ < a.lmax;
+      if (in) { grp |= 1u << i; posmax = max(posmax, ps_); }
+    }
+    if (((grp >> lead) & 1u) == 0) {                     // the leader reaches beyond the keys a block holds (the caller's max_len guard prevents it): zeros
+      if (blockIdx.z == 0)
+        for (int idx = tid; idx < GQ * HD; idx += NW * 64) a.out[xidx(r0 + lead, kvh * GQ * HD + idx, n_out)] = 0;
+      pending &= ~(1u << lead);
+      continue;
+    }
+    pending &= ~grp;
+    const int kv_all = posmax + 1, pages_all = (kv_all + 31) >> 5, nsb = (pages_all + IXT_SB - 1) / IXT_SB;
+    const int32_t* prow = a.page_map + (size_t)slot * g.mpg;
+    const int mypos = ((grp >> (i16 / GQ)) & 1u) ? s_pos[i16 / GQ] : -1;
+
+    // ---- scores
+    ixt_f32x4 S[NR][8];
+    float mx = -INFINITY, mn = INFINITY;
+#pragma unroll
+    for (int n = 0; n < NR; ++n) {
+      const int sb = n * NW + wave;
+#pragma unroll
+      for (int t = 0; t < 8; ++t) S[n][t] = ixt_f32x4(0.0f);
+      if (sb < nsb) {
+        const bf16_t* kp = a.kpages + kpage_off(g, prow[min(4 * sb + (i16 >> 2), pages_all - 1)], kvh, lg, i16 & 3);
+        u32x4 kr[2][8];
+#pragma unroll
+        for (int t = 0; t < 8; ++t) kr[0][t] = *reinterpret_cast<const u32x4*>(kp + t * 32);
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+          if (b + 1 < NB) {                              // the next 32 d fly while these are multiplied
+#pragma unroll
+            for (int t = 0; t < 8; ++t) kr[(b + 1) & 1][t] = *reinterpret_cast<const u32x4*>(kp + (b + 1) * 1024 + t * 32);
+          }
+          float q8[8];
+#pragma unroll
+          for (int s = 0; s < 8; ++s) q8[s] = qs[(8 * b + s) * 64 + lane];
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int t = 0; t < 8; t += 2) {
+            float x[8], y[8];
+            ixt_k_operands(kr[b & 1][t], sel, x);
+            ixt_k_operands(kr[b & 1][t + 1], sel, y);
+#pragma unroll
+            for (int s = 0; s < 8; ++s) {
+              S[n][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[s], q8[s], S[n][t], 0, 0, 0);
+              S[n][t + 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(y[s], q8[s], S[n][t + 1], 0, 0, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);           // two tiles' operands at a time: the scores need the registers
+          }
+        }
+        // lane (vector i16, group lg): register r of tile t is token 4 t + r of page 4 sb + lg
+        const int lim = mypos - sb * 128 - lg * 32, lo = a.window > 0 ? lim - a.window : -1;
+        if (a.cap > 0.0f) {
+#pragma unroll
+          for (int t = 0; t < 8; ++t) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) S[n][t][r] = ixt_tanh(S[n][t][r] / a.cap) * a.cap;
+            __builtin_amdgcn_sched_barrier(0);
+          }
+        }
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int k = 4 * t + r;
+            mn = fminf(mn, S[n][t][r]);
+            mx = (k <= lim && k > lo) ? fmaxf(mx, S[n][t][r]) : mx;
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+    }
+    // ---- softmax
+    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    if (lane < 16) wmax[wave * 16 + lane] = mx;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < NW; ++w) mx = fmaxf(mx, wmax[w * 16 + i16]);
+#pragma unroll
+    for (int n = 0; n < NR; ++n) {
+      const int sb = n * NW + wave;
+      if (sb < nsb) {
+        const int lim = mypos - sb * 128 - lg * 32, lo = a.window > 0 ? lim - a.window : -1;
+        float sacc = 0.0f;
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int k = 4 * t + r;
+            const float e = ixt_exp(S[n][t][r] - mx);
+            S[n][t][r] = (k <= lim && k > lo) ? e : 0.0f;
+            sacc = sacc + S[n][t][r];
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        psum[(4 * sb + lg) * 16 + i16] = sacc;
+      }
+    }
+    __syncthreads();
+    float l = 0.0f;
+    for (int p = 0; p < nsb * 4; p += 4) {
+      const float s0 = psum[p * 16 + i16], s1 = psum[p * 16 + 16 + i16], s2 = psum[p * 16 + 32 + i16], s3 = psum[p * 16 + 48 + i16];
+      l = l + s0; l = l + s1; l = l + s2; l = l + s3;
+    }
+    if (!(l > 0.0f)) l = 1.0f;                           // a vector of another group
+    const float rl = 1.0f / l;
+    uint32_t P[NR][8][2];                                // bf16 pairs: pages 2 k (low half) and 2 k + 1 of the super-block, token 4 t + lg
+    auto weights = [&](auto quotient) {
+#pragma unroll
+      for (int n = 0; n < NR; ++n) {
+        if (n * NW + wave < nsb) {
+#pragma unroll
+          for (int t = 0; t < 8; ++t) {
+            uint32_t u[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) u[r] = __float_as_uint(rbf(quotient(S[n][t][r])));
+            // register = token of the lane's page -> register = page, lane group = token
+            ixt_swap32(u[0], u[2]); ixt_swap32(u[1], u[3]);
+            ixt_swap16(u[0], u[1]); ixt_swap16(u[2], u[3]);
+#pragma unroll
+            for (int k = 0; k < 2; ++k) P[n][t][k] = (u[2 * k] >> 16) | u[2 * k + 1];
+            __builtin_amdgcn_sched_barrier(0);
+          }
+        }
+      }
+    };
+    if (__any(mypos >= 0 && mn - mx < -66.0f)) weights([&](float e) { return e / l; });
+    else weights([&](float e) {
+      float q = e * rl;
+      q = __builtin_fmaf(__builtin_fmaf(-q, l, e), rl, q);
+      return __builtin_fmaf(__builtin_fmaf(-q, l, e), rl, q);
+    });
+    // ---- outputs
+    for (int part = blockIdx.z; part < HD / VW; part += gridDim.z) {
+      float tot[2][NTOT];
+#pragma unroll
+      for (int k = 0; k < NTOT; ++k) { tot[0][k] = 0.0f; tot[1][k] = 0.0f; }
+#pragma unroll
+      for (int n = 0; n < NR; ++n) {
+        if (n * NW >= nsb) break;
+        const int sb = n * NW + wave;
+        ixt_f32x4 ss[NE];
+#pragma unroll
+        for (int x = 0; x < NE; ++x) ss[x] = ixt_f32x4(0.0f);
+        if (sb < nsb) {
+          const int np = min(IXT_SB, pages_all - sb * IXT_SB);
+#pragma unroll
+          for (int t = 0; t < 8; ++t) asm volatile("" : "+v"(P[n][t][0]), "+v"(P[n][t][1]));   // unpacked here, a step at a time, and not ahead of the loops
+          u32x4 va[4], vb[4];
+          auto fetch = [&](u32x4 (&v)[4], int p, int t0) {
+            const char* vp = reinterpret_cast<const char*>(a.vpages + vpage_off(g, prow[p], kvh, 0) + part * VW);
+            const int last = min(32, kv_all - p * 32) - 1;
+            int at = lg;
+            asm volatile("" : "+v"(at));                 // the addresses of this fetch only: ahead of the loops they would take the scores' registers
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+              const char* q = vp + (uint32_t)((min(4 * (t0 + t) + at, last) * HD + i16 * NE) * 2);
+              if constexpr (NE == 8) v[t] = *reinterpret_cast<const u32x4*>(q);
+              else { const uint2 w = *reinterpret_cast<const uint2*>(q); v[t].x = w.x; v[t].y = w.y; }
+            }
+          };
+          fetch(va, sb * IXT_SB, 0);
+#pragma unroll
+          for (int pg = 0; pg < IXT_SB; ++pg) {
+            if (pg < np) {
+              const int p = sb * IXT_SB + pg;
+              ixt_f32x4 acc[NE];
+#pragma unroll
+              for (int x = 0; x < NE; ++x) acc[x] = ixt_f32x4(0.0f);
+              fetch(vb, p, 4);
+              __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+              for (int t = 0; t < 4; ++t) {
+                const float pv = (pg & 1) ? bfhi(P[n][t][pg >> 1]) : bflo(P[n][t][pg >> 1]);
+#pragma unroll
+                for (int x = 0; x < NE; ++x)
+                  acc[x] = __builtin_amdgcn_mfma_f32_16x16x4f32((x & 1) ? bfhi(va[t][x >> 1]) : bflo(va[t][x >> 1]), pv, acc[x], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+              }
+              if (pg + 1 < np) fetch(va, p + 1, 0);
+              __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+              for (int t = 0; t < 4; ++t) {
+                const float pv = (pg & 1) ? bfhi(P[n][4 + t][pg >> 1]) : bflo(P[n][4 + t][pg >> 1]);
+#pragma unroll
+                for (int x = 0; x < NE; ++x)
+                  acc[x] = __builtin_amdgcn_mfma_f32_16x16x4f32((x & 1) ? bfhi(vb[t][x >> 1]) : bflo(vb[t][x >> 1]), pv, acc[x], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+              }
+#pragma unroll
+              for (int x = 0; x < NE; ++x)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) ss[x][r] = ss[x][r] + acc[x][r];
+            }
+          }
+        }
+        // lane: vector i16, columns NE (4 lg + r) + x
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          __syncthreads();
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int x = 0; x < NEH; ++x) ob[(wave * 16 + i16) * OP + (4 * lg + r) * NEH + x] = ss[h * NEH + x][r];
+          __syncthreads();
+#pragma unroll
+          for (int k = 0; k < NTOT; ++k) {
+            const int idx = tid + k * NW * 64, v = idx / CH, c = idx % CH;
+            const int nsb_v = ((grp >> (v / GQ)) & 1u) ? (((s_pos[v / GQ] + 32) >> 5) + IXT_SB - 1) / IXT_SB : 0;
+#pragma unroll
+            for (int w = 0; w < NW; ++w)
+              if (n * NW + w < nsb_v) tot[h][k] = tot[h][k] + ob[(w * 16 + v) * OP + c];
+          }
+        }
+      }
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int k = 0; k < NTOT; ++k) {
+          const int idx = tid + k * NW * 64, v = idx / CH, c = idx % CH;
+          const int d = part * VW + c / NEH * NE + h * NEH + c % NEH;
+          if ((grp >> (v / GQ)) & 1u) a.out[xidx(r0 + v / GQ, (kvh * GQ + v % GQ) * HD + d, n_out)] = f2bf(tot[h][k]);
+        }
+    }
+    __syncthreads();                                     // the LDS arrays are reused by the next group
+  }
+}

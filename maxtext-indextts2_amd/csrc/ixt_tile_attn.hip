@@ -1,0 +1,21 @@
+// ixt_tile_attn.hip -- launches of k_attn_mtile (an object of its own: it compiles beside the others).
+#include "ixt_tile_attn.h"
+
+// The smallest form that holds the call's longest prefix (ta.lmax keys, at most 4096).
+template <int HD, int GQ>
+static void mtile_attn_t(const TileAttnArgs& ta, hipStream_t st) {
+  constexpr int TQ = 16 / GQ;
+  const int tiles = (ta.R + TQ - 1) / TQ;
+  const dim3 grid(ta.g.nkv, tiles, HD > 128 && ta.g.nkv * tiles <= 128 ? HD / 128 : 1);   // half of the CUs idle: the halves of a value side by side
+  if (ta.lmax <= 256) hipLaunchKernelGGL((k_attn_mtile<HD, GQ, 2, 1>), grid, dim3(128), 0, st, ta);
+  else if (ta.lmax <= 512) hipLaunchKernelGGL((k_attn_mtile<HD, GQ, 4, 1>), grid, dim3(256), 0, st, ta);
+  else if (ta.lmax <= 1024) hipLaunchKernelGGL((k_attn_mtile<HD, GQ, 8, 1>), grid, dim3(512), 0, st, ta);
+  else if (ta.lmax <= 2048) hipLaunchKernelGGL((k_attn_mtile<HD, GQ, 8, 2>), grid, dim3(512), 0, st, ta);
+  else hipLaunchKernelGGL((k_attn_mtile<HD, GQ, 8, 4>), grid, dim3(512), 0, st, ta);
+}
+bool launch_mtile_attn(const TileAttnArgs& ta, int hd, int gq, hipStream_t st) {
+#define ATT(HD_, GQ_) if (hd == HD_ && gq == GQ_) { mtile_attn_t<HD_, GQ_>(ta, st); return true; }
+  ATT(128, 1) ATT(128, 2) ATT(128, 4) ATT(64, 1) ATT(64, 2) ATT(64, 4) ATT(256, 1) ATT(256, 2) ATT(256, 4)
+#undef ATT
+  return false;
+}
