@@ -12,6 +12,7 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <initializer_list>
 #include <string>
 #include <vector>
 
@@ -184,23 +185,9 @@ extern "C" int ixt_train_refresh_bf16(ixt_trainer* t, void* stream) {
 }
 
 // ---------------------------------------------------------------------------------------------------------------- launches
-// Scratch for split reductions (set by the step: a buffer that is idle while the layers' backward GEMMs run).
-static float* g_splitk_buf = nullptr;
-static size_t g_splitk_floats = 0;
-static int gemm(hipStream_t st, const bf16_t* A, long sam, long sak, const bf16_t* B, long sbk, long sbn, void* C, long scm, int M, int N, int K, int out_bf16,
-                int accumulate, int nb1 = 1, int nb2 = 1, long sab1 = 0, long sab2 = 0, long sbb1 = 0, long sbb2 = 0, long scb1 = 0, long scb2 = 0) {
-  // A weight gradient of few output tiles over a long reduction (2048 x 2048 over 16384 tokens: 256 tiles, one block per CU, 287 TFLOP/s): the
-  // reduction is cut in four batch parts whose products are added up in order (k_t_sum_parts).
-  constexpr int KS = 4;
-  if (!out_bf16 && !accumulate && nb1 * nb2 == 1 && scm == N && K >= 2048 && K % (KS * TG_BK) == 0 && (long)((N + 127) / 128) * ((M + 127) / 128) <= 256 &&
-      g_splitk_buf != nullptr && (size_t)KS * M * N <= g_splitk_floats) {
-    const int rc = gemm(st, A, sam, sak, B, sbk, sbn, g_splitk_buf, N, M, N, K / KS, 0, 0, KS, 1, (long)(K / KS) * sak, 0, (long)(K / KS) * sbk, 0, (long)M * N, 0);
-    if (rc != IXT_OK) return rc;
-    hipLaunchKernelGGL(k_t_sum_parts, dim3((unsigned)(((long)M * N + 255) / 256)), dim3(256), 0, st, g_splitk_buf, KS, (long)M * N, reinterpret_cast<float*>(C));
-    TLAUNCH();
-    return IXT_OK;
-  }
-  TGemm g;
+static int gemm_batched(hipStream_t st, const bf16_t* A, long sam, long sak, const bf16_t* B, long sbk, long sbn, void* C, long scm, int M, int N, int K, int out_bf16,
+                        int accumulate, int nb1, int nb2, long sab1, long sab2, long sbb1, long sbb2, long scb1, long scb2) {
+  TGemmB g;
   g.A = A; g.sam = sam; g.sak = sak; g.sab1 = sab1; g.sab2 = sab2;
   g.B = B; g.sbk = sbk; g.sbn = sbn; g.sbb1 = sbb1; g.sbb2 = sbb2;
   g.C = C; g.scm = scm; g.scb1 = scb1; g.scb2 = scb2;
@@ -208,11 +195,84 @@ static int gemm(hipStream_t st, const bf16_t* A, long sam, long sak, const bf16_
   if ((sam != 1 && sak != 1) || (sbk != 1 && sbn != 1)) return t_set_err(IXT_ERR_INVALID, "gemm: an operand has no unit stride");
   const dim3 grid((N + 127) / 128, (M + 127) / 128, nb1 * nb2);
   const bool ta = sak != 1, tb = sbk != 1;     // the operand's rows, not k, are contiguous: its tile is read transposed from LDS
-  if (ta && tb) hipLaunchKernelGGL((k_tgemm<true, true>), grid, dim3(256), 0, st, g);
-  else if (ta) hipLaunchKernelGGL((k_tgemm<true, false>), grid, dim3(256), 0, st, g);
-  else if (tb) hipLaunchKernelGGL((k_tgemm<false, true>), grid, dim3(256), 0, st, g);
-  else hipLaunchKernelGGL((k_tgemm<false, false>), grid, dim3(256), 0, st, g);
+  if (ta && tb) hipLaunchKernelGGL((k_tgemm_batched<true, true>), grid, dim3(256), 0, st, g);
+  else if (ta) hipLaunchKernelGGL((k_tgemm_batched<true, false>), grid, dim3(256), 0, st, g);
+  else if (tb) hipLaunchKernelGGL((k_tgemm_batched<false, true>), grid, dim3(256), 0, st, g);
+  else hipLaunchKernelGGL((k_tgemm_batched<false, false>), grid, dim3(256), 0, st, g);
   TLAUNCH();
+  return IXT_OK;
+}
+
+// The three products of a linear layer y = x W, W [K][N]: x W (W's columns contiguous), dy W^T (its k contiguous), x^T dy (both by columns).
+enum { TL_XW, TL_DX, TL_DW };
+template <bool TA, bool TB, int BM>
+static int gemm_launch(hipStream_t st, TGemm& g) {
+  constexpr int BN = BM, NS = 4, lds = NS * (BM + BN) * 64, MI = BM == 64 ? 2 : BM == 128 ? 4 : 8, NI = BM == 64 ? 2 : 4, WN = BM == 256 ? 4 : 2;
+  const auto kernel = k_tgemm<TA, TB, MI, NI, 2, WN, NS>;
+  static bool attr_done = false;
+  if (!attr_done) {
+    TCHK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+    attr_done = true;
+  }
+  g.mt = (g.M + BM - 1) / BM;
+  for (int i = 0; i < 3; ++i) g.nt[i] = i < g.nprob ? (g.N[i] + BN - 1) / BN : 0;
+  const int total = g.mt * (g.nt[0] + g.nt[1] + g.nt[2]) * g.parts;
+  hipLaunchKernelGGL(kernel, dim3(8 * ((total + 7) / 8)), dim3(128 * WN), lds, st, g);
+  TLAUNCH();
+  return IXT_OK;
+}
+struct TOperand { const bf16_t* x; const bf16_t* w; void* c; int n; };   // TL_DX: n is the reduction (the layer's outputs), c of the first entry the result
+// M: rows (tokens; TL_DW: the layer's inputs); K: reduction (TL_DX: the entries' n); scratch: for reductions cut in parts, or nullptr
+static int gemm(hipStream_t st, int what, int M, int K, std::initializer_list<TOperand> ops, int out, long ld_x, int N_dx = 0, const bf16_t* res = nullptr, float* scratch = nullptr,
+                size_t scratch_floats = 0) {
+  TGemm g{};
+  g.M = M; g.R = res; g.out = out; g.parts = 1;
+  int i = 0;
+  for (const TOperand& o : ops) {
+    g.A[i] = o.x; g.B[i] = o.w; g.C[i] = o.c;
+    if (what == TL_XW) { g.lda[i] = ld_x; g.ldb[i] = o.n; g.ldc[i] = o.n; g.N[i] = o.n; g.K[i] = K; }
+    else if (what == TL_DX) { g.lda[i] = o.n; g.ldb[i] = o.n; g.ldc[i] = N_dx; g.N[i] = N_dx; g.K[i] = o.n; }
+    else { g.lda[i] = ld_x; g.ldb[i] = o.n; g.ldc[i] = o.n; g.N[i] = o.n; g.K[i] = K; }
+    ++i;
+  }
+  g.nprob = i;
+  auto tiles = [&](int b) {
+    long t = 0;
+    for (int k = 0; k < g.nprob; ++k) t += (g.N[k] + b - 1) / b;
+    return t * ((M + b - 1) / b);
+  };
+  // A weight gradient of few output tiles over a long reduction (2048 x 2048 over 16384 tokens: 64 tiles of 256 x 256) is cut in four parts, whose
+  // products are added up in order (k_t_sum_parts).  The cut is a matter of the shape alone, so that no choice of tiles changes a sum.
+  if (out == TG_F32 && scratch != nullptr && g.K[0] >= 2048 && g.K[0] % 256 == 0) {
+    bool all = true;
+    long need = 0;
+    for (int k = 0; k < g.nprob; ++k) {
+      all = all && (long)((g.N[k] + 127) / 128) * ((M + 127) / 128) <= 256;
+      need += 4L * M * g.N[k];
+    }
+    if (all && (size_t)need <= scratch_floats) {
+      g.parts = 4;
+      g.kpart = g.K[0] / 4;
+      float* at = scratch;
+      for (int k = 0; k < g.nprob; ++k) { g.C[k] = at; g.cpart[k] = (long)M * g.N[k]; at += 4 * g.cpart[k]; }
+    }
+  }
+  // 256 x 256 tiles wherever they occupy three quarters of the CUs; 128 x 128 down to 200 of those, 64 x 64 below.  Measured in us, 128 / 64:
+  // 96 tiles of 128 x 128 with K 768 15.1 / 9.9, K 2048 29.2 / 18.9; 192 tiles, K 2048 32.2 / 24.6; 256 tiles, K 768 14.8 / 17.7; 512 tiles 22.6 / 28.9.
+  const int bm = tiles(256) * g.parts >= 192 ? 256 : tiles(128) * g.parts >= 200 ? 128 : 64;
+#define GO(TA_, TB_) TTRY(bm == 256 ? (gemm_launch<TA_, TB_, 256>(st, g)) : bm == 128 ? (gemm_launch<TA_, TB_, 128>(st, g)) : (gemm_launch<TA_, TB_, 64>(st, g)))
+  if (what == TL_XW) GO(false, true);
+  else if (what == TL_DX) GO(false, false);
+  else GO(true, true);
+#undef GO
+  if (g.parts > 1) {
+    int k = 0;
+    for (const TOperand& o : ops) {
+      hipLaunchKernelGGL(k_t_sum_parts, dim3((unsigned)((g.cpart[k] + 255) / 256)), dim3(256), 0, st, reinterpret_cast<const float*>(g.C[k]), g.parts, g.cpart[k], reinterpret_cast<float*>(o.c));
+      TLAUNCH();
+      ++k;
+    }
+  }
   return IXT_OK;
 }
 #define EW(n) dim3((unsigned)(((long)(n) + 255) / 256)), dim3(256), 0, st
@@ -222,7 +282,6 @@ extern "C" int ixt_train_forward_backward(ixt_trainer* t, const int32_t* inputs,
   if (!t || !inputs || !positions || !segmentation || !targets || !targets_segmentation || !loss_and_weights_dev)
     return t_set_err(IXT_ERR_INVALID, "null argument");
   if (!t->p) return t_set_err(IXT_ERR_INVALID, "bind the parameter buffers first");
-  g_splitk_buf = nullptr; g_splitk_floats = 0;
   hipStream_t st = (hipStream_t)stream;
   const int E = t->E, H = t->H, D = t->D, F = t->F, V = t->V, S = t->S, T = t->T, QN = t->QN, B = t->B, KVH = t->KVH, G = t->G, KN = t->KN;
   const long HD = (long)H * D;
@@ -237,52 +296,38 @@ extern "C" int ixt_train_forward_backward(ixt_trainer* t, const int32_t* inputs,
     LayerAct& a = t->act[l];
     const ixt_trainer::LOff& o = t->lo[l];
     hipLaunchKernelGGL(k_t_rmsnorm_fwd, dim3(T), dim3(256), 0, st, a.h_in, pb + o.ln1, a.xn1, a.r1, E, eps);
-    TTRY(gemm(st, a.xn1, E, 1, pb + o.wq, QN, 1, a.q, QN, T, QN, E, 1, 0));
-    TTRY(gemm(st, a.xn1, E, 1, pb + o.wk, KN, 1, a.k, KN, T, KN, E, 1, 0));
-    TTRY(gemm(st, a.xn1, E, 1, pb + o.wv, KN, 1, a.v, KN, T, KN, E, 1, 0));
+    TTRY(gemm(st, TL_XW, T, E, {{a.xn1, pb + o.wq, a.q, QN}, {a.xn1, pb + o.wk, a.k, KN}, {a.xn1, pb + o.wv, a.v, KN}}, TG_BF16, E));
     hipLaunchKernelGGL((k_t_rope<false>), dim3(T, H), dim3(D / 2), 0, st, a.q, positions, t->rope_sin, t->rope_cos, H, D);
     hipLaunchKernelGGL((k_t_rope<false>), dim3(T, KVH), dim3(D / 2), 0, st, a.k, positions, t->rope_sin, t->rope_cos, KVH, D);
     // scores[b,h] = Q_h K_(h / G)^T (sm_scale 1: the query kernel carries 1/sqrt(d), attentions.py:1900-1904).  Grouped-query attention
     // (attentions.py:1206-1271: query heads reshaped to [kv heads, G]): query head kvh G + g of every kv head in launch g, batches (b, kvh).
     for (int g = 0; g < G; ++g)
-      TTRY(gemm(st, a.q + (long)g * D, HD, 1, a.k, 1, KN, t->scores + (long)g * S * S, S, S, S, D, 0, 0, B, KVH, (long)S * HD, (long)G * D, (long)S * KN, D,
+      TTRY(gemm_batched(st, a.q + (long)g * D, HD, 1, a.k, 1, KN, t->scores + (long)g * S * S, S, S, S, D, 0, 0, B, KVH, (long)S * HD, (long)G * D, (long)S * KN, D,
                 (long)H * S * S, (long)G * S * S));
     if (S <= 256 * TS_MAXV) hipLaunchKernelGGL(k_t_softmax_fwd_reg, dim3(S, B * H), dim3(256), 0, st, t->scores, segmentation, a.P, S, H);
     else hipLaunchKernelGGL(k_t_softmax_fwd, dim3(S, B * H), dim3(256), 0, st, t->scores, segmentation, a.P, S, H);
     for (int g = 0; g < G; ++g)
-      TTRY(gemm(st, a.P + (long)g * S * S, S, 1, a.v, KN, 1, a.ao + (long)g * D, HD, S, D, S, 1, 0, B, KVH, (long)H * S * S, (long)G * S * S, (long)S * KN, D,
+      TTRY(gemm_batched(st, a.P + (long)g * S * S, S, 1, a.v, KN, 1, a.ao + (long)g * D, HD, S, D, S, 1, 0, B, KVH, (long)H * S * S, (long)G * S * S, (long)S * KN, D,
                 (long)S * HD, (long)G * D));
-    TTRY(gemm(st, a.ao, QN, 1, pb + o.wo, E, 1, t->tmp_bf, E, T, E, QN, 1, 0));
-    hipLaunchKernelGGL(k_t_add_bf16, EW((long)T * E), a.h_in, t->tmp_bf, a.h_mid, (long)T * E);
+    TTRY(gemm(st, TL_XW, T, QN, {{a.ao, pb + o.wo, a.h_mid, E}}, TG_BF16_RES, QN, 0, a.h_in));
     hipLaunchKernelGGL(k_t_rmsnorm_fwd, dim3(T), dim3(256), 0, st, a.h_mid, pb + o.ln2, a.xn2, a.r2, E, eps);
-    TTRY(gemm(st, a.xn2, E, 1, pb + o.wi0, F, 1, a.a, F, T, F, E, 1, 0));
-    TTRY(gemm(st, a.xn2, E, 1, pb + o.wi1, F, 1, a.b, F, T, F, E, 1, 0));
+    TTRY(gemm(st, TL_XW, T, E, {{a.xn2, pb + o.wi0, a.a, F}, {a.xn2, pb + o.wi1, a.b, F}}, TG_BF16, E));
     hipLaunchKernelGGL(k_t_swiglu_fwd, EW((long)T * F), a.a, a.b, a.act, (long)T * F);
-    TTRY(gemm(st, a.act, F, 1, pb + o.wout, E, 1, t->tmp_bf, E, T, E, F, 1, 0));
     bf16_t* h_next = l + 1 < t->L ? t->act[l + 1].h_in : t->h_final;
-    hipLaunchKernelGGL(k_t_add_bf16, EW((long)T * E), a.h_mid, t->tmp_bf, h_next, (long)T * E);
+    TTRY(gemm(st, TL_XW, T, F, {{a.act, pb + o.wout, h_next, E}}, TG_BF16_RES, F, 0, a.h_mid));
     TLAUNCH();
   }
   hipLaunchKernelGGL(k_t_rmsnorm_fwd, dim3(T), dim3(256), 0, st, t->h_final, pb + t->o_fnorm, t->xn_f, t->r_f, E, eps);
-  g_splitk_buf = nullptr; g_splitk_floats = 0;          // (the logits buffer is in use below)
   // ------------------------------------------------------------------ logits, loss and their gradients, a chunk of rows at a time
   TCHK(hipMemsetAsync(t->dxn, 0, sizeof(float) * (size_t)T * E, st));
   for (int t0 = 0; t0 < T; t0 += t->Tc) {
     const int n = T - t0 < t->Tc ? T - t0 : t->Tc;
-    TTRY(gemm(st, t->xn_f + (long)t0 * E, E, 1, pb + t->o_logits, V, 1, t->logits, V, n, V, E, 0, 0));
+    const bf16_t* xn = t->xn_f + (long)t0 * E;
+    TTRY(gemm(st, TL_XW, n, E, {{xn, pb + t->o_logits, t->logits, V}}, TG_F32, E));
     hipLaunchKernelGGL(k_t_xent, dim3(n), dim3(256), 0, st, t->logits, targets + t0, targets_segmentation + t0, t->dlog, t->row_loss + t0, V);
     // d xn_f = dlogits . W^T ; dW += xn_f^T . dlogits
-    // (n x E outputs are only 256 tiles of 128 x 128 over K = V: the reduction is cut in KS parts -- batch dimension of the GEMM -- whose products
-    //  land in the idle score buffer and are added up in order; one part per CU took 8.8 ms per chunk at 253 TFLOP/s)
-    const int KS = (V % (4 * TG_BK) == 0 && V >= 65536 && (size_t)4 * n * E <= (size_t)B * H * S * S) ? 4 : 1;
-    if (KS > 1) {
-      TTRY(gemm(st, t->dlog, V, 1, pb + t->o_logits, 1, V, t->scores, E, n, E, V / KS, 0, 0, KS, 1, V / KS, 0, V / KS, 0, (long)n * E, 0));
-      hipLaunchKernelGGL(k_t_sum_parts, EW((long)n * E), t->scores, KS, (long)n * E, t->dxn + (long)t0 * E);
-      TLAUNCH();
-    } else {
-      TTRY(gemm(st, t->dlog, V, 1, pb + t->o_logits, 1, V, t->dxn + (long)t0 * E, E, n, E, V, 0, 0));
-    }
-    TTRY(gemm(st, t->xn_f + (long)t0 * E, 1, E, t->dlog, V, 1, t->g + t->o_logits, V, E, V, n, 0, 1));
+    TTRY(gemm(st, TL_DX, n, V, {{t->dlog, pb + t->o_logits, t->dxn + (long)t0 * E, V}}, TG_F32, V, E, nullptr, t->scores, V >= 65536 ? (size_t)B * H * S * S : 0));   // (the score buffer is idle)
+    TTRY(gemm(st, TL_DW, E, n, {{xn, t->dlog, t->g + t->o_logits, V}}, TG_F32_ADD, E));
   }
   hipLaunchKernelGGL(k_t_reduce, dim3(1), dim3(256), 0, st, t->row_loss, (long)T, 0, loss_and_weights_dev, 0);
   // total_weights = number of target positions with a non-zero segment id (train.py:309)
@@ -290,7 +335,8 @@ extern "C" int ixt_train_forward_backward(ixt_trainer* t, const int32_t* inputs,
   hipLaunchKernelGGL(k_t_reduce, dim3(1), dim3(256), 0, st, t->row_loss, (long)T, 0, loss_and_weights_dev + 1, 0);
   TLAUNCH();
   // ------------------------------------------------------------------ backward
-  g_splitk_buf = t->logits; g_splitk_floats = (size_t)t->Tc * V;   // idle from here on: scratch of the split weight-gradient GEMMs
+  float* const spare = t->logits;                          // idle from here on: scratch of the cut weight-gradient products
+  const size_t spare_n = (size_t)t->Tc * V;
   TCHK(hipMemsetAsync(t->dh, 0, sizeof(float) * (size_t)T * E, st));
   hipLaunchKernelGGL(k_t_rmsnorm_bwd, dim3((T + TN_RPB - 1) / TN_RPB), dim3(256), 0, st, t->dxn, t->h_final, pb + t->o_fnorm, t->r_f, t->dh, t->g + t->o_fnorm, E, (long)T);
   for (int l = t->L - 1; l >= 0; --l) {
@@ -298,52 +344,50 @@ extern "C" int ixt_train_forward_backward(ixt_trainer* t, const int32_t* inputs,
     const ixt_trainer::LOff& o = t->lo[l];
     // MLP: h_out = h_mid + wo(act)
     hipLaunchKernelGGL(k_t_f32_to_bf16, EW((long)T * E), t->dh, t->dy_bf, (long)T * E);
-    TTRY(gemm(st, t->dy_bf, E, 1, pb + o.wout, 1, E, t->dact, F, T, F, E, 1, 0));                       // d act = dy . Wout^T
-    TTRY(gemm(st, a.act, 1, F, t->dy_bf, E, 1, t->g + o.wout, E, F, E, T, 0, 0));                        // d Wout = act^T . dy
+    TTRY(gemm(st, TL_DX, T, E, {{t->dy_bf, pb + o.wout, t->dact, E}}, TG_BF16, E, F));                   // d act = dy . Wout^T
+    TTRY(gemm(st, TL_DW, F, T, {{a.act, t->dy_bf, t->g + o.wout, E}}, TG_F32, F, 0, nullptr, spare, spare_n));   // d Wout = act^T . dy
     hipLaunchKernelGGL(k_t_swiglu_bwd, EW((long)T * F), t->dact, a.a, a.b, t->da, t->db, (long)T * F);
-    TTRY(gemm(st, t->da, F, 1, pb + o.wi0, 1, F, t->dxn, E, T, E, F, 0, 0));                             // d xn2 = da . Wi0^T + db . Wi1^T
-    TTRY(gemm(st, t->db, F, 1, pb + o.wi1, 1, F, t->dxn, E, T, E, F, 0, 1));
-    TTRY(gemm(st, a.xn2, 1, E, t->da, F, 1, t->g + o.wi0, F, E, F, T, 0, 0));
-    TTRY(gemm(st, a.xn2, 1, E, t->db, F, 1, t->g + o.wi1, F, E, F, T, 0, 0));
+    TTRY(gemm(st, TL_DX, T, F, {{t->da, pb + o.wi0, t->dxn, F}}, TG_F32, F, E, nullptr, spare, spare_n));   // d xn2 = da . Wi0^T + db . Wi1^T
+    TTRY(gemm(st, TL_DX, T, F, {{t->db, pb + o.wi1, t->dxn, F}}, TG_F32_ADD, F, E));
+    TTRY(gemm(st, TL_DW, E, T, {{a.xn2, t->da, t->g + o.wi0, F}, {a.xn2, t->db, t->g + o.wi1, F}}, TG_F32, E, 0, nullptr, spare, spare_n));
     hipLaunchKernelGGL(k_t_rmsnorm_bwd, dim3((T + TN_RPB - 1) / TN_RPB), dim3(256), 0, st, t->dxn, a.h_mid, pb + o.ln2, a.r2, t->dh, t->g + o.ln2, E, (long)T);
     // attention: h_mid = h_in + out(ao)
     hipLaunchKernelGGL(k_t_f32_to_bf16, EW((long)T * E), t->dh, t->dy_bf, (long)T * E);
-    TTRY(gemm(st, t->dy_bf, E, 1, pb + o.wo, 1, E, t->d_ao, QN, T, QN, E, 1, 0));                        // d ao = dy . Wo^T
-    TTRY(gemm(st, a.ao, 1, QN, t->dy_bf, E, 1, t->g + o.wo, E, QN, E, T, 0, 0));                          // d Wo = ao^T . dy
+    TTRY(gemm(st, TL_DX, T, E, {{t->dy_bf, pb + o.wo, t->d_ao, E}}, TG_BF16, E, QN));                    // d ao = dy . Wo^T
+    TTRY(gemm(st, TL_DW, QN, T, {{a.ao, t->dy_bf, t->g + o.wo, E}}, TG_F32, QN, 0, nullptr, spare, spare_n));   // d Wo = ao^T . dy
     // dP = d_ao V^T (f32) ; dV = P^T d_ao ; dS = P o (dP - rowsum(dP o P)) ; dQ = dS K ; dK = dS^T Q.  With G query heads per kv head, dV and dK
     // are the sums over the group: accumulated in f32 over the G launches, rounded to bf16 once.
     for (int g = 0; g < G; ++g)
-      TTRY(gemm(st, t->d_ao + (long)g * D, HD, 1, a.v, 1, KN, t->scores + (long)g * S * S, S, S, S, D, 0, 0, B, KVH, (long)S * HD, (long)G * D, (long)S * KN, D,
+      TTRY(gemm_batched(st, t->d_ao + (long)g * D, HD, 1, a.v, 1, KN, t->scores + (long)g * S * S, S, S, S, D, 0, 0, B, KVH, (long)S * HD, (long)G * D, (long)S * KN, D,
                 (long)H * S * S, (long)G * S * S));
     if (G == 1) {
-      TTRY(gemm(st, a.P, 1, S, t->d_ao, HD, 1, t->dv, HD, S, D, S, 1, 0, B, H, (long)H * S * S, (long)S * S, (long)S * HD, D, (long)S * HD, D));
+      TTRY(gemm_batched(st, a.P, 1, S, t->d_ao, HD, 1, t->dv, HD, S, D, S, 1, 0, B, H, (long)H * S * S, (long)S * S, (long)S * HD, D, (long)S * HD, D));
     } else {
       for (int g = 0; g < G; ++g)
-        TTRY(gemm(st, a.P + (long)g * S * S, 1, S, t->d_ao + (long)g * D, HD, 1, t->dvf, KN, S, D, S, 0, g > 0, B, KVH, (long)H * S * S, (long)G * S * S,
+        TTRY(gemm_batched(st, a.P + (long)g * S * S, 1, S, t->d_ao + (long)g * D, HD, 1, t->dvf, KN, S, D, S, 0, g > 0, B, KVH, (long)H * S * S, (long)G * S * S,
                   (long)S * HD, (long)G * D, (long)S * KN, D));
       hipLaunchKernelGGL(k_t_f32_to_bf16, EW((long)T * KN), t->dvf, t->dv, (long)T * KN);
     }
     if (S <= 256 * TS_MAXV) hipLaunchKernelGGL(k_t_softmax_bwd_reg, dim3(S, B * H), dim3(256), 0, st, t->scores, a.P, t->dS, S);
     else hipLaunchKernelGGL(k_t_softmax_bwd, dim3(S, B * H), dim3(256), 0, st, t->scores, a.P, t->dS, S);
     for (int g = 0; g < G; ++g)
-      TTRY(gemm(st, t->dS + (long)g * S * S, S, 1, a.k, KN, 1, t->dq + (long)g * D, HD, S, D, S, 1, 0, B, KVH, (long)H * S * S, (long)G * S * S, (long)S * KN, D,
+      TTRY(gemm_batched(st, t->dS + (long)g * S * S, S, 1, a.k, KN, 1, t->dq + (long)g * D, HD, S, D, S, 1, 0, B, KVH, (long)H * S * S, (long)G * S * S, (long)S * KN, D,
                 (long)S * HD, (long)G * D));
     if (G == 1) {
-      TTRY(gemm(st, t->dS, 1, S, a.q, HD, 1, t->dk, HD, S, D, S, 1, 0, B, H, (long)H * S * S, (long)S * S, (long)S * HD, D, (long)S * HD, D));
+      TTRY(gemm_batched(st, t->dS, 1, S, a.q, HD, 1, t->dk, HD, S, D, S, 1, 0, B, H, (long)H * S * S, (long)S * S, (long)S * HD, D, (long)S * HD, D));
     } else {
       for (int g = 0; g < G; ++g)
-        TTRY(gemm(st, t->dS + (long)g * S * S, 1, S, a.q + (long)g * D, HD, 1, t->dkf, KN, S, D, S, 0, g > 0, B, KVH, (long)H * S * S, (long)G * S * S,
+        TTRY(gemm_batched(st, t->dS + (long)g * S * S, 1, S, a.q + (long)g * D, HD, 1, t->dkf, KN, S, D, S, 0, g > 0, B, KVH, (long)H * S * S, (long)G * S * S,
                   (long)S * HD, (long)G * D, (long)S * KN, D));
       hipLaunchKernelGGL(k_t_f32_to_bf16, EW((long)T * KN), t->dkf, t->dk, (long)T * KN);
     }
     hipLaunchKernelGGL((k_t_rope<true>), dim3(T, H), dim3(D / 2), 0, st, t->dq, positions, t->rope_sin, t->rope_cos, H, D);
     hipLaunchKernelGGL((k_t_rope<true>), dim3(T, KVH), dim3(D / 2), 0, st, t->dk, positions, t->rope_sin, t->rope_cos, KVH, D);
-    TTRY(gemm(st, t->dq, QN, 1, pb + o.wq, 1, QN, t->dxn, E, T, E, QN, 0, 0));                           // d xn1 = dq Wq^T + dk Wk^T + dv Wv^T
-    TTRY(gemm(st, t->dk, KN, 1, pb + o.wk, 1, KN, t->dxn, E, T, E, KN, 0, 1));
-    TTRY(gemm(st, t->dv, KN, 1, pb + o.wv, 1, KN, t->dxn, E, T, E, KN, 0, 1));
-    TTRY(gemm(st, a.xn1, 1, E, t->dq, QN, 1, t->g + o.wq, QN, E, QN, T, 0, 0));
-    TTRY(gemm(st, a.xn1, 1, E, t->dk, KN, 1, t->g + o.wk, KN, E, KN, T, 0, 0));
-    TTRY(gemm(st, a.xn1, 1, E, t->dv, KN, 1, t->g + o.wv, KN, E, KN, T, 0, 0));
+    // d xn1 = dq Wq^T + dk Wk^T + dv Wv^T
+    TTRY(gemm(st, TL_DX, T, QN, {{t->dq, pb + o.wq, t->dxn, QN}}, TG_F32, QN, E, nullptr, spare, spare_n));
+    TTRY(gemm(st, TL_DX, T, KN, {{t->dk, pb + o.wk, t->dxn, KN}}, TG_F32_ADD, KN, E));
+    TTRY(gemm(st, TL_DX, T, KN, {{t->dv, pb + o.wv, t->dxn, KN}}, TG_F32_ADD, KN, E));
+    TTRY(gemm(st, TL_DW, E, T, {{a.xn1, t->dq, t->g + o.wq, QN}, {a.xn1, t->dk, t->g + o.wk, KN}, {a.xn1, t->dv, t->g + o.wv, KN}}, TG_F32, E, 0, nullptr, spare, spare_n));
     hipLaunchKernelGGL(k_t_rmsnorm_bwd, dim3((T + TN_RPB - 1) / TN_RPB), dim3(256), 0, st, t->dxn, a.h_in, pb + o.ln1, a.r1, t->dh, t->g + o.ln1, E, (long)T);
     TLAUNCH();
   }

@@ -1,0 +1,223 @@
+// ixt_train_gemm.h -- the matrix products of the training step: C[m][n] (+)= sum_k A(m, k) B(k, n), bf16 operands of which either index may be the
+// contiguous one, f32 accumulation.
+//
+// Block = (16 MI WM) x (16 NI WN), waves WM x WN, 32 k at a time through a ring of NS LDS slots filled by LDS-DMA; a wave's tile is 16 MI x 16 NI.
+// What bounds it: LDS reads against matrix cores.  Per 32 k a wave reads MI + NI KiB and issues MI NI products of 16 cycles; eight waves of 128 x 64
+// read 96 KiB (768 cycles of the LDS) under 1024 cycles of products, four of 64 x 64 32 KiB (256) under 256: hence the 256 x 256 block wherever
+// its tiles fill the chip.  With few tiles a wave is alone on its SIMD and bound by its own instructions: smaller tiles, more waves (gemm_launch has
+// the rule).  The next 32 k are read from LDS and fetched from memory between the rows of products, not in front of them.
+// Measured (bf16): 16384 x 2048 x 7168 1.06 PFLOP/s, its input gradient 1.12, its weight gradient 1.13, 8192^3 1.24 (0.45 - 0.53 with 128 x 128 x 64
+// tiles staged through registers; torch's product of 8192^3 1.37 on this card); without the fetches 1.4 - 1.7.
+//   k contiguous:   slot image [row][32 k], four 16-byte pieces a row, piece c of row r at c ^ ((r >> 2) & 3): the 16 rows a half wave reads lie on
+//                   disjoint banks
+//   row contiguous: slot image [k][row], 32-byte pieces, piece u of row k at u ^ (k & 7) (64 rows: u ^ (k / 2 & 3)); ds_read_tr16 hands a 4 x 16 block to 16 lanes column-wise, so
+//                   the transpose costs nothing; the eight k rows a half wave touches lie on disjoint banks
+// Both put k = 4 q .. 4 q + 3 and 16 + 4 q .. on lane group q, 32 k after 32 k into one accumulator (the order of sums of k_tgemm_batched).  A piece past
+// K comes from a zeroed word instead, a row past M or N is a re-read of a valid one (its results are not stored), so dimensions need only be
+// multiples of 8.
+// One launch takes up to three products of the same M (`nprob`: the q, k and v projections, their gradients); `parts` > 1 cuts the reduction, part p
+// writing its own f32 C.  Blocks of one XCD take neighbouring tiles.
+#pragma once
+#include "ixt_device.h"
+
+typedef float tf32x4 __attribute__((ext_vector_type(4)));
+typedef short tbf16x8 __attribute__((ext_vector_type(8)));
+typedef short tbf16x4 __attribute__((ext_vector_type(4)));
+
+enum { TG_F32 = 0, TG_F32_ADD = 1, TG_BF16 = 2, TG_BF16_RES = 3 };   // C = acc, C += acc, C = bf16(acc), C = bf16(R + bf16(acc))
+
+struct TGemm {
+  const bf16_t* A[3]; long lda[3];       // stride of the index that is not contiguous
+  const bf16_t* B[3]; long ldb[3];
+  void* C[3]; long ldc[3];
+  const bf16_t* R;                       // TG_BF16_RES: as C[0]
+  int M, N[3], K[3];
+  int nprob, parts, kpart;               // parts > 1: part p covers k in [p kpart, (p + 1) kpart) and writes C + p * cpart
+  long cpart[3];
+  int out;
+  int mt, nt[3];                         // tiles
+};
+
+static __device__ const uint32_t tg_zero[4] = {0u, 0u, 0u, 0u};
+
+template <bool TA, bool TB, int MI, int NI, int WM, int WN, int NS>
+__global__ __launch_bounds__(WM * WN * 64, 2) void k_tgemm(TGemm g) {
+  constexpr int BM = 16 * MI * WM, BN = 16 * NI * WN, NW = WM * WN;
+  constexpr int NA = BM / 16, NB = BN / 16, NJ = (NA + NB) / NW;          // KiB of a chunk; a wave fetches NJ of them
+  constexpr int SLOT = (BM + BN) * 32;                                    // elements
+  static_assert(NA % NW == 0 && NB % NW == 0, "a fetch is of one operand");
+  extern __shared__ __attribute__((aligned(16))) bf16_t lds[];            // [NS][A image | B image]
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, r16 = lane & 15, q = lane >> 4;
+  const int wm = wave / WN, wn = wave % WN;
+  // XCD x takes a run of tiles (part by part); eight row tiles share their columns' operand
+  const int ntn = g.nt[0] + g.nt[1] + g.nt[2], total = g.mt * ntn, per = (total * g.parts + 7) >> 3;
+  const int id = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+  if (id >= total * g.parts) return;                                      // whole block
+  const int part = id / total, tile = id - part * total;
+  const int grp = tile / (8 * ntn), rows = min(8, g.mt - grp * 8), in = tile - grp * 8 * ntn;
+  int tn = in / rows;
+  const int tm = grp * 8 + in % rows;
+  int prob = 0;
+  while (prob < g.nprob - 1 && tn >= g.nt[prob]) tn -= g.nt[prob++];
+  const int m0 = tm * BM, n0 = tn * BN, N = g.N[prob];
+
+  int segk, segend;                                                       // k: next to fetch, end
+  const char *pa, *pb;                                                    // the tile's first row at segk; bytes between chunks
+  long adva, advb;
+  uint32_t off[NJ];                                                       // the lane's place in a chunk, in bytes
+  // piece f of a chunk's image (KiB): the k of this lane's 16 bytes, and row
+  auto place = [&](bool tr, int bx, int f, int& k, int& x) {
+    if (tr) {
+      const int pr = bx / 8, sl = lane % pr;
+      k = f * (64 / pr) + lane / pr;
+      x = (((sl >> 1) ^ (bx == 64 ? k >> 1 & 3 : k & 7)) << 4) + (sl & 1) * 8;
+    } else {
+      x = f * 16 + (lane >> 2);
+      k = ((lane & 3) ^ ((x >> 2) & 3)) * 8;
+    }
+  };
+  {
+    const long la = g.lda[prob], lb = g.ldb[prob];
+    segk = g.parts > 1 ? part * g.kpart : 0;
+    segend = g.parts > 1 ? min(g.K[prob], segk + g.kpart) : g.K[prob];
+    pa = reinterpret_cast<const char*>(g.A[prob] + (TA ? (long)segk * la + m0 : (long)m0 * la + segk));
+    pb = reinterpret_cast<const char*>(g.B[prob] + (TB ? (long)segk * lb + n0 : (long)n0 * lb + segk));
+    adva = TA ? 64 * la : 64; advb = TB ? 64 * lb : 64;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      const int f = wave + NW * j;
+      const bool isa = j * NW < NA;
+      int k, x;
+      place(isa ? TA : TB, isa ? BM : BN, isa ? f : f - NA, k, x);
+      const int lim = (isa ? g.M - m0 : N - n0) - ((isa ? TA : TB) ? 8 : 1);
+      x = min(x, lim);
+      off[j] = (uint32_t)((isa ? TA : TB) ? k * (int)(isa ? la : lb) + x : x * (int)(isa ? la : lb) + k) * 2u;
+    }
+  }
+  const int chunks = (segend - segk + 31) >> 5;
+  bool whole = false;
+  auto next_chunk = [&]() {                                               // past the last chunk: zeros, so that the counts stay
+    whole = segk + 32 <= segend;
+  };
+  // Issued by hand (nothing else in this kernel uses m0): the builtin makes the compiler wait for every fetch in flight ahead of a transposed LDS read.  (No register is written; the waits
+  // are counted in the loop.)
+  const uint32_t lds0 = (uint32_t)(uintptr_t)((__attribute__((address_space(3))) bf16_t*)lds);
+  auto issue = [&](int slot, int j) {                                     // piece j of this wave's share of the next chunk
+    const bool isa = j * NW < NA;
+    const uint32_t dst = __builtin_amdgcn_readfirstlane(lds0 + (uint32_t)(slot * SLOT + (wave + NW * j) * 512) * 2u);
+    if (whole) {
+      asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(off[j]), "s"(isa ? pa : pb) : "memory");
+    } else {
+      const char* p = (isa ? pa : pb) + off[j];
+      int k, x;
+      place(isa ? TA : TB, isa ? BM : BN, isa ? wave + NW * j : wave + NW * j - NA, k, x);
+      if (segk + k >= segend) p = reinterpret_cast<const char*>(tg_zero);
+      asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(dst), "v"(p) : "memory");
+    }
+  };
+  auto advance = [&]() { segk += 32; pa += adva; pb += advb; };
+  const int trf = (r16 >> 2) | (q & 1) << 2;                              // k & 7 of the lane's row in a transposed read: 4 q + r16 / 4
+  auto operand = [&](const bf16_t* img, int x, int bx, bool tr) -> tbf16x8 {
+    tbf16x4 lo, hi;
+    if (tr) {                                                             // lane 4 a + p of a group: k row a, columns 4 p ..
+      int f = bx == 64 ? trf >> 1 : trf;                                  // (k + 16: the same piece)
+      asm volatile("" : "+v"(f));                                         // an address at a time: all of them ahead of the loop are 12 registers
+      const bf16_t* p = img + (4 * q + (r16 >> 2)) * bx + (((x >> 4) ^ f) << 4) + 4 * (r16 & 3);
+      lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) tbf16x4*)p);
+      hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) tbf16x4*)(p + 16 * bx));
+    } else {
+      const bf16_t* p = img + (x + r16) * 32 + (q & 1) * 4;
+      const int f = (r16 >> 2) & 3;
+      lo = *reinterpret_cast<const tbf16x4*>(p + (((q >> 1) ^ f) << 3));
+      hi = *reinterpret_cast<const tbf16x4*>(p + ((((q >> 1) + 2) ^ f) << 3));
+    }
+    return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+  };
+  auto row_a = [&](int slot, int i) { return operand(lds + slot * SLOT, (wm * MI + i) * 16, BM, TA); };
+  auto row_b = [&](int slot, int i) { return operand(lds + slot * SLOT + BM * 32, (wn * NI + i) * 16, BN, TB); };
+  tf32x4 acc[MI][NI];
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int j = 0; j < NI; ++j) acc[i][j] = tf32x4(0.0f);
+  tbf16x8 fa[MI], fb[2][NI];
+#pragma unroll
+  for (int c = 0; c < NS; ++c) {
+    next_chunk();
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) issue(c, j);
+    advance();
+  }
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 1) * NJ) : "memory");
+  __builtin_amdgcn_s_barrier();
+#pragma unroll
+  for (int j = 0; j < NI; ++j) fb[0][j] = row_b(0, j);
+#pragma unroll
+  for (int i = 0; i < MI; ++i) fa[i] = row_a(0, i);
+  auto step = [&](int c, int cur) {
+    // chunk c + 1 has landed once the (NS - 2) younger ones are all that is outstanding; this wave's reads of chunk c are done, so behind the
+    // barrier its slot can be filled again
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((NS - 2) * NJ) : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    next_chunk();
+    const int nxt = (c + 1) % NS, old = c % NS;
+    // a row of products, then a share of the reads of chunk c + 1 and of the fetches of chunk c + NS: they ride under the products
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+#pragma unroll
+      for (int j = 0; j < NI; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[cur][j], fa[i], acc[i][j], 0, 0, 0);
+      fa[i] = row_a(nxt, i);
+      if (i < NI) fb[cur ^ 1][i] = row_b(nxt, i);
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+        if (j * MI / NJ == i) issue(old, j);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    advance();
+  };
+  for (int c = 0; c < chunks; c += 2) {                                   // (an odd count: the last products are with zeros)
+    step(c, 0);
+    step(c + 1, 1);
+  }
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");             // nothing may land in LDS that the next block owns
+  // lane: m = r16, n = 4 q + register
+  const int out = g.out, nw = n0 + wn * NI * 16 + q * 4;
+#pragma unroll
+  for (int i = 0; i < MI; ++i) {
+    const int m = m0 + (wm * MI + i) * 16 + r16;
+    if (m >= g.M) continue;
+    const long row = (long)m * g.ldc[prob] + nw;
+    if (out == TG_F32 || out == TG_F32_ADD) {
+      float* c = reinterpret_cast<float*>(g.C[prob]) + part * g.cpart[prob] + row;
+      if (out == TG_F32_ADD) {
+        tf32x4 old[NI];
+#pragma unroll
+        for (int j = 0; j < NI; ++j) old[j] = nw + j * 16 < N ? *reinterpret_cast<const tf32x4*>(c + j * 16) : tf32x4(0.0f);
+#pragma unroll
+        for (int j = 0; j < NI; ++j) acc[i][j] = old[j] + acc[i][j];
+      }
+#pragma unroll
+      for (int j = 0; j < NI; ++j)
+        if (nw + j * 16 < N) *reinterpret_cast<tf32x4*>(c + j * 16) = acc[i][j];
+    } else {
+      bf16_t* c = reinterpret_cast<bf16_t*>(g.C[prob]) + row;
+      if (out == TG_BF16_RES) {
+        uint2 h[NI];
+#pragma unroll
+        for (int j = 0; j < NI; ++j) h[j] = nw + j * 16 < N ? *reinterpret_cast<const uint2*>(g.R + row + j * 16) : make_uint2(0u, 0u);
+#pragma unroll
+        for (int j = 0; j < NI; ++j) {
+          acc[i][j][0] = bflo(h[j].x) + rbf(acc[i][j][0]); acc[i][j][1] = bfhi(h[j].x) + rbf(acc[i][j][1]);
+          acc[i][j][2] = bflo(h[j].y) + rbf(acc[i][j][2]); acc[i][j][3] = bfhi(h[j].y) + rbf(acc[i][j][3]);
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < NI; ++j) {
+        uint2 o;
+        o.x = pack2(f2bf(acc[i][j][0]), f2bf(acc[i][j][1])); o.y = pack2(f2bf(acc[i][j][2]), f2bf(acc[i][j][3]));
+        if (nw + j * 16 < N) *reinterpret_cast<uint2*>(c + j * 16) = o;
+      }
+    }
+  }
+}

@@ -6,11 +6,9 @@
 // bit-exact contract of the decode path, so reductions here use whatever order is fastest unless stated.
 #pragma once
 #include "ixt_device.h"
+#include "ixt_train_gemm.h"
 
-typedef float tf32x4 __attribute__((ext_vector_type(4)));
-typedef short tbf16x8 __attribute__((ext_vector_type(8)));
-
-// ---------------------------------------------------------------------------------------------------------------- general GEMM
+// ---------------------------------------------------------------------------------------------------------------- batched GEMM of the attention
 // C[m][n] (+)= sum_k A(m, k) B(k, n) for bf16 operands with arbitrary element strides (either index may be the contiguous one), f32
 // accumulation, two-level batch (z = z1 * nb2 + z2).  Block = 128 x 128 x 64, 4 waves as 2 x 2, wave = 64 x 64 = 4 x 4 MFMA tiles.
 // An operand tile lies in LDS the way it lies in memory, so every global 16-byte vector is one 16-byte LDS store:
@@ -22,7 +20,7 @@ typedef short tbf16x8 __attribute__((ext_vector_type(8)));
 // of the 32-block (the sum over k does not care which lane group carries which k, as long as both operands agree) -- with it the two
 // transposed reads of a half-wave cover 8 consecutive k-rows.
 // MFMA roles: A-operand = B tile rows (n), B-operand = A tile rows (m), so a lane ends with 4 consecutive n of one m.
-struct TGemm {
+struct TGemmB {
   const bf16_t* A; long sam, sak, sab1, sab2;
   const bf16_t* B; long sbk, sbn, sbb1, sbb2;
   void* C; long scm, scb1, scb2;      // C row stride (n contiguous)
@@ -83,7 +81,7 @@ __device__ __forceinline__ tbf16x8 tg_frag(const uint2 (&f)[2]) {
 }
 
 template <bool TA, bool TB>
-__global__ __launch_bounds__(256) void k_tgemm(TGemm g) {
+__global__ __launch_bounds__(256) void k_tgemm_batched(TGemmB g) {
   __shared__ __attribute__((aligned(16))) bf16_t As[TG_TILE];
   __shared__ __attribute__((aligned(16))) bf16_t Bs[TG_TILE];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;

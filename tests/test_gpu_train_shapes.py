@@ -1,0 +1,44 @@
+"""The training step's matrix products and attention at the edges of their tiles, against the f32 oracle: gradients of every tensor within the 2 % that
+rounding the backward signals to bf16 gives (tests/test_gpu_train.py), the loss within 1e-4."""
+import importlib
+
+import pytest
+
+from oracle import train_oracle as TO
+from test_gpu_train import f32_params, packed_batch, train_config
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = {
+    # nothing a multiple of 32, reductions that end inside a chunk, tiles of every product cut off
+    "ragged": dict(base_emb_dim=200, base_num_query_heads=5, base_num_kv_heads=5, head_dim=40, base_mlp_dim=328, vocab_size=1000, max_target_length=72, per_device_batch_size=3.0),
+    # 256 x 256 tiles with cut-off rows, columns and reductions (the vocabulary's products), a second chunk of 16 logits rows
+    "large tiles": dict(base_emb_dim=72, base_num_query_heads=2, base_num_kv_heads=2, head_dim=64, base_mlp_dim=136, vocab_size=6152, max_target_length=688, per_device_batch_size=3.0),
+    # reductions cut in parts, the last part shorter; groups of query heads
+    "cut reductions": dict(base_emb_dim=264, base_num_query_heads=4, base_num_kv_heads=2, head_dim=128, base_mlp_dim=520, vocab_size=4104, max_target_length=712, per_device_batch_size=3.0),
+    # one row, shorter than any tile
+    "short": dict(base_emb_dim=64, base_num_query_heads=2, base_num_kv_heads=1, head_dim=64, base_mlp_dim=72, vocab_size=264, max_target_length=8, per_device_batch_size=1.0),
+}
+
+
+@pytest.mark.parametrize("shape", list(SHAPES))
+def test_train_step_at_tile_edges(shape):
+  import torch
+  tr = importlib.import_module("maxtext-indextts2_amd.train")
+  cfg = train_config(**SHAPES[shape])
+  params = f32_params(cfg, 8)
+  trainer = tr.Trainer(cfg)
+  trainer.load_params(params)
+  orc = TO.TrainOracle(cfg, params)
+  b = packed_batch(cfg, 41)
+  m = trainer.train_step(b)
+  grads = {k: v.clone() for k, v in trainer.param_views(trainer.grads).items()}
+  o = orc.train_step(b)
+  assert m["learning/total_weights"] == o["learning/total_weights"]
+  assert abs(m["learning/loss"] - o["learning/loss"]) <= 1e-4 * abs(o["learning/loss"]), (m["learning/loss"], o["learning/loss"])
+  for k, g in grads.items():
+    ref, got = o["grads"][k], g.cpu() / (o["learning/total_weights"] + 1e-8)
+    err = float((got - ref).norm()) / (float(ref.norm()) + 1e-12)
+    assert err < 2e-2, (k, err)
+  del trainer
+  torch.cuda.synchronize()
