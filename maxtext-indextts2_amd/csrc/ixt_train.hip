@@ -58,7 +58,7 @@ struct ixt_trainer {
   float* r_f = nullptr;
   // workspaces
   float *scores = nullptr, *dh = nullptr, *dxn = nullptr, *logits = nullptr, *row_loss = nullptr, *scal = nullptr, *part = nullptr;
-  bf16_t *tmp_bf = nullptr, *dS = nullptr, *d_ao = nullptr, *dq = nullptr, *dk = nullptr, *dv = nullptr, *dact = nullptr, *da = nullptr, *db = nullptr, *dlog = nullptr,
+  bf16_t *dS = nullptr, *d_ao = nullptr, *dq = nullptr, *dk = nullptr, *dv = nullptr, *dact = nullptr, *da = nullptr, *db = nullptr, *dlog = nullptr,
          *dy_bf = nullptr;
   float *dkf = nullptr, *dvf = nullptr;   // grouped-query attention: dK / dV summed over a group's query heads in f32 before they round to bf16
   std::vector<void*> allocs;
@@ -127,8 +127,7 @@ extern "C" int ixt_train_create(const ixt_train_config* c, ixt_trainer** out) {
   A(tmalloc(t, &t->scores, BH * S * S)); A(tmalloc(t, &t->dh, T * E)); A(tmalloc(t, &t->dxn, T * E));
   A(tmalloc(t, &t->logits, (size_t)t->Tc * V)); A(tmalloc(t, &t->dlog, (size_t)t->Tc * V)); A(tmalloc(t, &t->row_loss, T)); A(tmalloc(t, &t->scal, (size_t)16));
   A(tmalloc(t, &t->part, (size_t)4096));
-  const size_t big = T * (size_t)(F > QN ? (F > E ? F : E) : (QN > E ? QN : E));
-  A(tmalloc(t, &t->tmp_bf, big)); A(tmalloc(t, &t->dS, BH * S * S)); A(tmalloc(t, &t->d_ao, T * QN)); A(tmalloc(t, &t->dq, T * QN)); A(tmalloc(t, &t->dk, T * KN));
+  A(tmalloc(t, &t->dS, BH * S * S)); A(tmalloc(t, &t->d_ao, T * QN)); A(tmalloc(t, &t->dq, T * QN)); A(tmalloc(t, &t->dk, T * KN));
   A(tmalloc(t, &t->dv, T * KN));
   if (t->G > 1) { A(tmalloc(t, &t->dkf, T * KN)); A(tmalloc(t, &t->dvf, T * KN)); } A(tmalloc(t, &t->dact, T * F)); A(tmalloc(t, &t->da, T * F)); A(tmalloc(t, &t->db, T * F)); A(tmalloc(t, &t->dy_bf, T * E));
 #undef A
@@ -179,7 +178,7 @@ extern "C" int ixt_train_bind(ixt_trainer* t, float* params, float* grads, float
 }
 extern "C" int ixt_train_refresh_bf16(ixt_trainer* t, void* stream) {
   if (!t || !t->p) return t_set_err(IXT_ERR_INVALID, "bind the parameter buffers first");
-  hipLaunchKernelGGL(k_t_cast_bf16, dim3((unsigned)((t->total + 255) / 256)), dim3(256), 0, (hipStream_t)stream, t->p, t->pb, t->total);
+  hipLaunchKernelGGL(k_t_cast_bf16, dim3((unsigned)((t->total / 4 + 255) / 256)), dim3(256), 0, (hipStream_t)stream, t->p, t->pb, t->total);
   TLAUNCH();
   return IXT_OK;
 }
@@ -268,12 +267,21 @@ static int gemm(hipStream_t st, int what, int M, int K, std::initializer_list<TO
   if (g.parts > 1) {
     int k = 0;
     for (const TOperand& o : ops) {
-      hipLaunchKernelGGL(k_t_sum_parts, dim3((unsigned)((g.cpart[k] + 255) / 256)), dim3(256), 0, st, reinterpret_cast<const float*>(g.C[k]), g.parts, g.cpart[k], reinterpret_cast<float*>(o.c));
+      hipLaunchKernelGGL(k_t_sum_parts, dim3((unsigned)((g.cpart[k] / 4 + 255) / 256)), dim3(256), 0, st, reinterpret_cast<const float*>(g.C[k]), g.parts, g.cpart[k], reinterpret_cast<float*>(o.c));
       TLAUNCH();
       ++k;
     }
   }
   return IXT_OK;
+}
+// 16 rows per block (16384 x 2048: 182 -> 141 us with the next row in flight and the bf16 copy included), fewer below 8192 rows: a block's rows
+// are a chain, but every block adds its sums to the same E words
+static void rmsnorm_bwd(hipStream_t st, const float* dy, const bf16_t* x, const bf16_t* scale, const float* rstd, float* dh, bf16_t* dh_bf, float* dscale, int E, long T) {
+  const int rpb = T < 512 ? 1 : T < 8192 ? (int)(T / 512) : 16;
+  const dim3 grid((unsigned)((T + rpb - 1) / rpb));
+  if (E <= 1024) hipLaunchKernelGGL(k_t_rmsnorm_bwd<4>, grid, dim3(256), 0, st, dy, x, scale, rstd, dh, dh_bf, dscale, E, T, rpb);
+  else if (E <= 2048) hipLaunchKernelGGL(k_t_rmsnorm_bwd<8>, grid, dim3(256), 0, st, dy, x, scale, rstd, dh, dh_bf, dscale, E, T, rpb);
+  else hipLaunchKernelGGL(k_t_rmsnorm_bwd<TN_FPT>, grid, dim3(256), 0, st, dy, x, scale, rstd, dh, dh_bf, dscale, E, T, rpb);
 }
 #define EW(n) dim3((unsigned)(((long)(n) + 255) / 256)), dim3(256), 0, st
 
@@ -287,7 +295,16 @@ extern "C" int ixt_train_forward_backward(ixt_trainer* t, const int32_t* inputs,
   const long HD = (long)H * D;
   const bf16_t* pb = t->pb;
   const float eps = t->cfg.normalization_layer_epsilon;
-  TCHK(hipMemsetAsync(t->g, 0, sizeof(float) * t->total, st));
+  // The gradients that several blocks add to start from zero: the embedding's and the norms' (the last one behind the loop's); every other one is stored
+  // whole.  The gaps between parameters, where there are any, are part of the norm: cleared with everything else.
+  bool gaps = false;
+  for (const ParamInfo& p : t->params) gaps = gaps || p.numel % 64 != 0;
+  const long stride = t->L > 1 ? t->lo[1].ln1 - t->lo[0].ln1 : 0;
+  const long n0 = gaps ? t->total : (long)V * E;
+  float* const g0 = gaps ? t->g : t->g + t->o_emb;
+  hipLaunchKernelGGL(k_t_zero, dim3((unsigned)((n0 + 1023) / 1024 + ((long)2 * t->L * E + 1023) / 1024)), dim3(256), 0, st, g0, n0, t->g + t->lo[0].ln1, t->g + t->lo[0].ln2, stride, t->L, E);
+  hipLaunchKernelGGL(k_t_zero, dim3((unsigned)((E + 1023) / 1024)), dim3(256), 0, st, t->g + t->o_fnorm, (long)E, t->g, t->g, 0L, 0, 4);
+  TLAUNCH();
   // ------------------------------------------------------------------ forward (layers/* in train mode)
   bf16_t* h = t->act[0].h_in;
   hipLaunchKernelGGL(k_embed, dim3((E / 8 + 255) / 256, T), dim3(256), 0, st, pb + t->o_emb, inputs, h, E, V);
@@ -297,8 +314,7 @@ extern "C" int ixt_train_forward_backward(ixt_trainer* t, const int32_t* inputs,
     const ixt_trainer::LOff& o = t->lo[l];
     hipLaunchKernelGGL(k_t_rmsnorm_fwd, dim3(T), dim3(256), 0, st, a.h_in, pb + o.ln1, a.xn1, a.r1, E, eps);
     TTRY(gemm(st, TL_XW, T, E, {{a.xn1, pb + o.wq, a.q, QN}, {a.xn1, pb + o.wk, a.k, KN}, {a.xn1, pb + o.wv, a.v, KN}}, TG_BF16, E));
-    hipLaunchKernelGGL((k_t_rope<false>), dim3(T, H), dim3(D / 2), 0, st, a.q, positions, t->rope_sin, t->rope_cos, H, D);
-    hipLaunchKernelGGL((k_t_rope<false>), dim3(T, KVH), dim3(D / 2), 0, st, a.k, positions, t->rope_sin, t->rope_cos, KVH, D);
+    hipLaunchKernelGGL((k_t_rope<false>), EW((long)T * (H + KVH) * (D / 8)), a.q, a.k, positions, t->rope_sin, t->rope_cos, H, KVH, D, (long)T);
     // scores[b,h] = Q_h K_(h / G)^T (sm_scale 1: the query kernel carries 1/sqrt(d), attentions.py:1900-1904).  Grouped-query attention
     // (attentions.py:1206-1271: query heads reshaped to [kv heads, G]): query head kvh G + g of every kv head in launch g, batches (b, kvh).
     for (int g = 0; g < G; ++g)
@@ -312,22 +328,21 @@ extern "C" int ixt_train_forward_backward(ixt_trainer* t, const int32_t* inputs,
     TTRY(gemm(st, TL_XW, T, QN, {{a.ao, pb + o.wo, a.h_mid, E}}, TG_BF16_RES, QN, 0, a.h_in));
     hipLaunchKernelGGL(k_t_rmsnorm_fwd, dim3(T), dim3(256), 0, st, a.h_mid, pb + o.ln2, a.xn2, a.r2, E, eps);
     TTRY(gemm(st, TL_XW, T, E, {{a.xn2, pb + o.wi0, a.a, F}, {a.xn2, pb + o.wi1, a.b, F}}, TG_BF16, E));
-    hipLaunchKernelGGL(k_t_swiglu_fwd, EW((long)T * F), a.a, a.b, a.act, (long)T * F);
+    hipLaunchKernelGGL(k_t_swiglu_fwd, EW((long)T * F / 8), a.a, a.b, a.act, (long)T * F);
     bf16_t* h_next = l + 1 < t->L ? t->act[l + 1].h_in : t->h_final;
     TTRY(gemm(st, TL_XW, T, F, {{a.act, pb + o.wout, h_next, E}}, TG_BF16_RES, F, 0, a.h_mid));
     TLAUNCH();
   }
   hipLaunchKernelGGL(k_t_rmsnorm_fwd, dim3(T), dim3(256), 0, st, t->h_final, pb + t->o_fnorm, t->xn_f, t->r_f, E, eps);
   // ------------------------------------------------------------------ logits, loss and their gradients, a chunk of rows at a time
-  TCHK(hipMemsetAsync(t->dxn, 0, sizeof(float) * (size_t)T * E, st));
   for (int t0 = 0; t0 < T; t0 += t->Tc) {
     const int n = T - t0 < t->Tc ? T - t0 : t->Tc;
     const bf16_t* xn = t->xn_f + (long)t0 * E;
-    TTRY(gemm(st, TL_XW, n, E, {{xn, pb + t->o_logits, t->logits, V}}, TG_F32, E));
-    hipLaunchKernelGGL(k_t_xent, dim3(n), dim3(256), 0, st, t->logits, targets + t0, targets_segmentation + t0, t->dlog, t->row_loss + t0, V);
+    TTRY(gemm(st, TL_XW, n, E, {{xn, pb + t->o_logits, t->logits, V}}, TG_BF16, E));
+    hipLaunchKernelGGL(k_t_xent, dim3(n), dim3(256), 0, st, reinterpret_cast<const bf16_t*>(t->logits), targets + t0, targets_segmentation + t0, t->dlog, t->row_loss + t0, V);
     // d xn_f = dlogits . W^T ; dW += xn_f^T . dlogits
     TTRY(gemm(st, TL_DX, n, V, {{t->dlog, pb + t->o_logits, t->dxn + (long)t0 * E, V}}, TG_F32, V, E, nullptr, t->scores, V >= 65536 ? (size_t)B * H * S * S : 0));   // (the score buffer is idle)
-    TTRY(gemm(st, TL_DW, E, n, {{xn, t->dlog, t->g + t->o_logits, V}}, TG_F32_ADD, E));
+    TTRY(gemm(st, TL_DW, E, n, {{xn, t->dlog, t->g + t->o_logits, V}}, t0 == 0 ? TG_F32 : TG_F32_ADD, E));
   }
   hipLaunchKernelGGL(k_t_reduce, dim3(1), dim3(256), 0, st, t->row_loss, (long)T, 0, loss_and_weights_dev, 0);
   // total_weights = number of target positions with a non-zero segment id (train.py:309)
@@ -337,22 +352,20 @@ extern "C" int ixt_train_forward_backward(ixt_trainer* t, const int32_t* inputs,
   // ------------------------------------------------------------------ backward
   float* const spare = t->logits;                          // idle from here on: scratch of the cut weight-gradient products
   const size_t spare_n = (size_t)t->Tc * V;
-  TCHK(hipMemsetAsync(t->dh, 0, sizeof(float) * (size_t)T * E, st));
-  hipLaunchKernelGGL(k_t_rmsnorm_bwd, dim3((T + TN_RPB - 1) / TN_RPB), dim3(256), 0, st, t->dxn, t->h_final, pb + t->o_fnorm, t->r_f, t->dh, t->g + t->o_fnorm, E, (long)T);
+  hipLaunchKernelGGL(k_t_zero, dim3((unsigned)(((long)T * E + 1023) / 1024)), dim3(256), 0, st, t->dh, (long)T * E, t->g, t->g, 0L, 0, 4);
+  rmsnorm_bwd(st, t->dxn, t->h_final, pb + t->o_fnorm, t->r_f, t->dh, t->dy_bf, t->g + t->o_fnorm, E, T);
   for (int l = t->L - 1; l >= 0; --l) {
     LayerAct& a = t->act[l];
     const ixt_trainer::LOff& o = t->lo[l];
     // MLP: h_out = h_mid + wo(act)
-    hipLaunchKernelGGL(k_t_f32_to_bf16, EW((long)T * E), t->dh, t->dy_bf, (long)T * E);
     TTRY(gemm(st, TL_DX, T, E, {{t->dy_bf, pb + o.wout, t->dact, E}}, TG_BF16, E, F));                   // d act = dy . Wout^T
     TTRY(gemm(st, TL_DW, F, T, {{a.act, t->dy_bf, t->g + o.wout, E}}, TG_F32, F, 0, nullptr, spare, spare_n));   // d Wout = act^T . dy
-    hipLaunchKernelGGL(k_t_swiglu_bwd, EW((long)T * F), t->dact, a.a, a.b, t->da, t->db, (long)T * F);
+    hipLaunchKernelGGL(k_t_swiglu_bwd, EW((long)T * F / 8), t->dact, a.a, a.b, t->da, t->db, (long)T * F);
     TTRY(gemm(st, TL_DX, T, F, {{t->da, pb + o.wi0, t->dxn, F}}, TG_F32, F, E, nullptr, spare, spare_n));   // d xn2 = da . Wi0^T + db . Wi1^T
     TTRY(gemm(st, TL_DX, T, F, {{t->db, pb + o.wi1, t->dxn, F}}, TG_F32_ADD, F, E));
     TTRY(gemm(st, TL_DW, E, T, {{a.xn2, t->da, t->g + o.wi0, F}, {a.xn2, t->db, t->g + o.wi1, F}}, TG_F32, E, 0, nullptr, spare, spare_n));
-    hipLaunchKernelGGL(k_t_rmsnorm_bwd, dim3((T + TN_RPB - 1) / TN_RPB), dim3(256), 0, st, t->dxn, a.h_mid, pb + o.ln2, a.r2, t->dh, t->g + o.ln2, E, (long)T);
+    rmsnorm_bwd(st, t->dxn, a.h_mid, pb + o.ln2, a.r2, t->dh, t->dy_bf, t->g + o.ln2, E, T);
     // attention: h_mid = h_in + out(ao)
-    hipLaunchKernelGGL(k_t_f32_to_bf16, EW((long)T * E), t->dh, t->dy_bf, (long)T * E);
     TTRY(gemm(st, TL_DX, T, E, {{t->dy_bf, pb + o.wo, t->d_ao, E}}, TG_BF16, E, QN));                    // d ao = dy . Wo^T
     TTRY(gemm(st, TL_DW, QN, T, {{a.ao, t->dy_bf, t->g + o.wo, E}}, TG_F32, QN, 0, nullptr, spare, spare_n));   // d Wo = ao^T . dy
     // dP = d_ao V^T (f32) ; dV = P^T d_ao ; dS = P o (dP - rowsum(dP o P)) ; dQ = dS K ; dK = dS^T Q.  With G query heads per kv head, dV and dK
@@ -366,7 +379,7 @@ extern "C" int ixt_train_forward_backward(ixt_trainer* t, const int32_t* inputs,
       for (int g = 0; g < G; ++g)
         TTRY(gemm_batched(st, a.P + (long)g * S * S, 1, S, t->d_ao + (long)g * D, HD, 1, t->dvf, KN, S, D, S, 0, g > 0, B, KVH, (long)H * S * S, (long)G * S * S,
                   (long)S * HD, (long)G * D, (long)S * KN, D));
-      hipLaunchKernelGGL(k_t_f32_to_bf16, EW((long)T * KN), t->dvf, t->dv, (long)T * KN);
+      hipLaunchKernelGGL(k_t_f32_to_bf16, EW((long)T * KN / 8), t->dvf, t->dv, (long)T * KN);
     }
     if (S <= 256 * TS_MAXV) hipLaunchKernelGGL(k_t_softmax_bwd_reg, dim3(S, B * H), dim3(256), 0, st, t->scores, a.P, t->dS, S);
     else hipLaunchKernelGGL(k_t_softmax_bwd, dim3(S, B * H), dim3(256), 0, st, t->scores, a.P, t->dS, S);
@@ -379,16 +392,15 @@ extern "C" int ixt_train_forward_backward(ixt_trainer* t, const int32_t* inputs,
       for (int g = 0; g < G; ++g)
         TTRY(gemm_batched(st, t->dS + (long)g * S * S, 1, S, a.q + (long)g * D, HD, 1, t->dkf, KN, S, D, S, 0, g > 0, B, KVH, (long)H * S * S, (long)G * S * S,
                   (long)S * HD, (long)G * D, (long)S * KN, D));
-      hipLaunchKernelGGL(k_t_f32_to_bf16, EW((long)T * KN), t->dkf, t->dk, (long)T * KN);
+      hipLaunchKernelGGL(k_t_f32_to_bf16, EW((long)T * KN / 8), t->dkf, t->dk, (long)T * KN);
     }
-    hipLaunchKernelGGL((k_t_rope<true>), dim3(T, H), dim3(D / 2), 0, st, t->dq, positions, t->rope_sin, t->rope_cos, H, D);
-    hipLaunchKernelGGL((k_t_rope<true>), dim3(T, KVH), dim3(D / 2), 0, st, t->dk, positions, t->rope_sin, t->rope_cos, KVH, D);
+    hipLaunchKernelGGL((k_t_rope<true>), EW((long)T * (H + KVH) * (D / 8)), t->dq, t->dk, positions, t->rope_sin, t->rope_cos, H, KVH, D, (long)T);
     // d xn1 = dq Wq^T + dk Wk^T + dv Wv^T
     TTRY(gemm(st, TL_DX, T, QN, {{t->dq, pb + o.wq, t->dxn, QN}}, TG_F32, QN, E, nullptr, spare, spare_n));
     TTRY(gemm(st, TL_DX, T, KN, {{t->dk, pb + o.wk, t->dxn, KN}}, TG_F32_ADD, KN, E));
     TTRY(gemm(st, TL_DX, T, KN, {{t->dv, pb + o.wv, t->dxn, KN}}, TG_F32_ADD, KN, E));
     TTRY(gemm(st, TL_DW, E, T, {{a.xn1, t->dq, t->g + o.wq, QN}, {a.xn1, t->dk, t->g + o.wk, KN}, {a.xn1, t->dv, t->g + o.wv, KN}}, TG_F32, E, 0, nullptr, spare, spare_n));
-    hipLaunchKernelGGL(k_t_rmsnorm_bwd, dim3((T + TN_RPB - 1) / TN_RPB), dim3(256), 0, st, t->dxn, a.h_in, pb + o.ln1, a.r1, t->dh, t->g + o.ln1, E, (long)T);
+    rmsnorm_bwd(st, t->dxn, a.h_in, pb + o.ln1, a.r1, t->dh, l > 0 ? t->dy_bf : nullptr, t->g + o.ln1, E, T);
     TLAUNCH();
   }
   hipLaunchKernelGGL(k_t_embed_bwd, dim3((E + 255) / 256, T), dim3(256), 0, st, t->dh, inputs, t->g + t->o_emb, E, V);

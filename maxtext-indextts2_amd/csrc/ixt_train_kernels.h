@@ -155,9 +155,36 @@ __global__ __launch_bounds__(256) void k_tgemm_batched(TGemmB g) {
 }
 
 // ---------------------------------------------------------------------------------------------------------------- elementwise / rows
-static __global__ void k_t_cast_bf16(const float* __restrict__ src, bf16_t* __restrict__ dst, long n) {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) dst[i] = f2bf(src[i]);
+// Rows of bf16 are moved 16 bytes a lane; where a sum has a place in the arithmetic, its terms stay with the threads they always had (thread t: t, t +
+// 256, ..), so that the losses and gradients of a step do not depend on how the rows are read.
+__device__ __forceinline__ void t_unpack8(const u32x4& w, float (&v)[8]) {
+#pragma unroll
+  for (int k = 0; k < 4; ++k) { v[2 * k] = bflo(w[k]); v[2 * k + 1] = bfhi(w[k]); }
+}
+__device__ __forceinline__ u32x4 t_pack8(const float (&v)[8]) {
+  u32x4 w;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) w[k] = pack2(f2bf(v[2 * k]), f2bf(v[2 * k + 1]));
+  return w;
+}
+// zeros: n values at `at`, then `count` times two runs of `run` values at a and b, `stride` apart (n, run, offsets multiples of 4).
+// grid = (ceil(n / 1024) + ceil(2 count run / 1024)), block 256.
+static __global__ void k_t_zero(float* __restrict__ at, long n, float* __restrict__ a, float* __restrict__ b, long stride, int count, int run) {
+  const float4 z = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  const long nb = (n + 1023) / 1024;
+  if ((long)blockIdx.x < nb) {
+    const long i = ((long)blockIdx.x * 256 + threadIdx.x) * 4;
+    if (i < n) *reinterpret_cast<float4*>(at + i) = z;
+    return;
+  }
+  const long i = (((long)blockIdx.x - nb) * 256 + threadIdx.x) * 4, l = i / (2 * run), e = i - l * 2 * run;
+  if (l < count) *reinterpret_cast<float4*>((e < run ? a + e : b + e - run) + l * stride) = z;
+}
+static __global__ void k_t_cast_bf16(const float* __restrict__ src, bf16_t* __restrict__ dst, long n) {   // n a multiple of 64 (the parameters' layout)
+  const long i = ((long)blockIdx.x * blockDim.x + threadIdx.x) * 4;
+  if (i >= n) return;
+  const float4 v = *reinterpret_cast<const float4*>(src + i);
+  *reinterpret_cast<uint2*>(dst + i) = make_uint2(pack2(f2bf(v.x), f2bf(v.y)), pack2(f2bf(v.z), f2bf(v.w)));
 }
 
 __device__ __forceinline__ float t_block_sum(float v, float* red) {   // 256 threads
@@ -169,74 +196,127 @@ __device__ __forceinline__ float t_block_sum(float v, float* red) {   // 256 thr
   return red[0] + red[1] + red[2] + red[3];
 }
 
-// RMSNorm forward (normalizations.py:57-70): y = bf16(bf16(x r) scale), r = rsqrt(mean(x^2) + eps) saved per row.  grid = T, block 256.
+// RMSNorm forward (normalizations.py:57-70): y = bf16(bf16(x r) scale), r = rsqrt(mean(x^2) + eps) saved per row.  E % 8 == 0, E <= 4096.  grid = T, block 256.
 static __global__ __launch_bounds__(256) void k_t_rmsnorm_fwd(const bf16_t* __restrict__ x, const bf16_t* __restrict__ scale, bf16_t* __restrict__ y,
                                                        float* __restrict__ rstd, int E, float eps) {
   __shared__ float red[4];
+  __shared__ __attribute__((aligned(16))) bf16_t xs[4096];
   const long row = blockIdx.x;
+  const int tid = threadIdx.x;
+  u32x4 w[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int e = (tid + i * 256) * 8;
+    if (e < E) { w[i] = *reinterpret_cast<const u32x4*>(x + row * E + e); *reinterpret_cast<u32x4*>(xs + e) = w[i]; }
+  }
+  __syncthreads();
   float s = 0.0f;
-  for (int e = threadIdx.x; e < E; e += 256) { const float v = bf2f(x[row * E + e]); s += v * v; }
+  for (int e = tid; e < E; e += 256) { const float v = bf2f(xs[e]); s += v * v; }
   const float tot = t_block_sum(s, red);
   const float r = 1.0f / sqrtf(tot / (float)E + eps);
-  if (threadIdx.x == 0) rstd[row] = r;
-  for (int e = threadIdx.x; e < E; e += 256) y[row * E + e] = f2bf(rbf(bf2f(x[row * E + e]) * r) * bf2f(scale[e]));
-}
-// backward: dy f32 [T][E] (the sum of the consumers' input gradients); dx (f32) is ADDED to dh (the residual-stream gradient);
-// dscale: a block walks TN_RPB rows and keeps its features' partial sums in registers -- one f32 atomic per feature and BLOCK (one per feature
-// and row took 466 us per launch at 16384 x 2048: 2048 addresses under 33 M atomics).  grid = ceil(T / TN_RPB), block 256, E <= 256 TN_FPT.
-#define TN_RPB 16
-#define TN_FPT 16
-static __global__ __launch_bounds__(256) void k_t_rmsnorm_bwd(const float* __restrict__ dy, const bf16_t* __restrict__ x, const bf16_t* __restrict__ scale,
-                                                       const float* __restrict__ rstd, float* __restrict__ dh, float* __restrict__ dscale, int E, long T) {
-  __shared__ float red[4];
-  float ds[TN_FPT];
+  if (tid == 0) rstd[row] = r;
 #pragma unroll
-  for (int i = 0; i < TN_FPT; ++i) ds[i] = 0.0f;
-  const long row0 = (long)blockIdx.x * TN_RPB;
-  for (long row = row0; row < row0 + TN_RPB && row < T; ++row) {
-    const float r = rstd[row];
-    float s = 0.0f;
-    for (int e = threadIdx.x; e < E; e += 256) {
-      const float xh = bf2f(x[row * E + e]) * r;
-      s += dy[row * E + e] * bf2f(scale[e]) * xh;
+  for (int i = 0; i < 2; ++i) {
+    const int e = (tid + i * 256) * 8;
+    if (e < E) {
+      float v[8], c[8];
+      t_unpack8(w[i], v);
+      t_unpack8(*reinterpret_cast<const u32x4*>(scale + e), c);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[k] = rbf(v[k] * r) * c[k];
+      *reinterpret_cast<u32x4*>(y + row * E + e) = t_pack8(v);
     }
+  }
+}
+// backward: dy f32 [T][E] (the sum of the consumers' input gradients); dx (f32) is ADDED to dh (the residual-stream gradient), and the sum goes out as
+// bf16, too (dh_bf, the next products' operand; nullptr: nobody wants it).
+// dscale: a block walks `rpb` rows and keeps its features' partial sums in registers -- one f32 atomic per feature and BLOCK (one per feature and row
+// took 466 us per launch at 16384 x 2048: 2048 addresses under 33 M atomics).  A row's operands stay in registers between the two passes over it and
+// the next row's are in flight meanwhile.  grid = ceil(T / rpb), block 256, E <= 256 FPT.
+#define TN_FPT 16
+template <int FPT>
+static __global__ __launch_bounds__(256) void k_t_rmsnorm_bwd(const float* __restrict__ dy, const bf16_t* __restrict__ x, const bf16_t* __restrict__ scale,
+                                                       const float* __restrict__ rstd, float* __restrict__ dh, bf16_t* __restrict__ dh_bf, float* __restrict__ dscale, int E, long T,
+                                                       int rpb) {
+  __shared__ float red[4];
+  float ds[FPT], sc[FPT], gy[FPT], xv[FPT], hv[FPT];
+#pragma unroll
+  for (int i = 0; i < FPT; ++i) {
+    const int e = threadIdx.x + i * 256;
+    ds[i] = 0.0f;
+    sc[i] = e < E ? bf2f(scale[e]) : 0.0f;
+  }
+  const long row0 = (long)blockIdx.x * rpb, row1 = row0 + rpb < T ? row0 + rpb : T;
+  auto fetch = [&](long row) {
+#pragma unroll
+    for (int i = 0; i < FPT; ++i) {
+      const int e = threadIdx.x + i * 256;
+      if (e < E) { gy[i] = dy[row * E + e]; xv[i] = bf2f(x[row * E + e]); hv[i] = dh[row * E + e]; }
+    }
+  };
+  fetch(row0);
+  for (long row = row0; row < row1; ++row) {
+    const float r = rstd[row];
+    float s = 0.0f, g0[FPT], xh[FPT], h0[FPT];
+#pragma unroll
+    for (int i = 0; i < FPT; ++i) { g0[i] = gy[i]; xh[i] = xv[i] * r; h0[i] = hv[i]; }
+    if (row + 1 < row1) fetch(row + 1);
+#pragma unroll
+    for (int i = 0; i < FPT; ++i)
+      if (threadIdx.x + i * 256 < E) s += g0[i] * sc[i] * xh[i];
     const float mean = t_block_sum(s, red) / (float)E;
 #pragma unroll
-    for (int i = 0; i < TN_FPT; ++i) {
+    for (int i = 0; i < FPT; ++i) {
       const int e = threadIdx.x + i * 256;
       if (e < E) {
-        const float xh = bf2f(x[row * E + e]) * r, gy = dy[row * E + e];
-        dh[row * E + e] += r * (gy * bf2f(scale[e]) - xh * mean);
-        ds[i] += gy * xh;
+        const float h = h0[i] + r * (g0[i] * sc[i] - xh[i] * mean);
+        dh[row * E + e] = h;
+        if (dh_bf != nullptr) dh_bf[row * E + e] = f2bf(h);
+        ds[i] += g0[i] * xh[i];
       }
     }
   }
 #pragma unroll
-  for (int i = 0; i < TN_FPT; ++i) {
+  for (int i = 0; i < FPT; ++i) {
     const int e = threadIdx.x + i * 256;
     if (e < E) atomicAdd(dscale + e, ds[i]);
   }
 }
 // out[i] = parts[0][i] + parts[1][i] + ... (split-K partial products, in order)
-static __global__ void k_t_sum_parts(const float* __restrict__ parts, int nparts, long n, float* __restrict__ out) {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+static __global__ void k_t_sum_parts(const float* __restrict__ parts, int nparts, long n, float* __restrict__ out) {   // n a multiple of 64
+  const long i = ((long)blockIdx.x * blockDim.x + threadIdx.x) * 4;
   if (i >= n) return;
-  float t = parts[i];
-  for (int p = 1; p < nparts; ++p) t += parts[(long)p * n + i];
-  out[i] = t;
+  float4 t = *reinterpret_cast<const float4*>(parts + i);
+  for (int p = 1; p < nparts; ++p) {
+    const float4 v = *reinterpret_cast<const float4*>(parts + (long)p * n + i);
+    t.x += v.x; t.y += v.y; t.z += v.z; t.w += v.w;
+  }
+  *reinterpret_cast<float4*>(out + i) = t;
 }
 
-// RoPE (embeddings.py:277-315) on x bf16 [T][H][D] with per-token positions; INV: the transposed rotation (backward).  grid = (T, H), block D/2.
+// RoPE (embeddings.py:277-315) on q bf16 [T][H][D] and k [T][KVH][D] with per-token positions; INV: the transposed rotation (backward).  A thread turns
+// four pairs (D % 8 == 0).  grid = ceil(T (H + KVH) (D / 8) / 256), block 256.
 template <bool INV>
-__global__ void k_t_rope(bf16_t* __restrict__ x, const int32_t* __restrict__ pos, const bf16_t* __restrict__ sn, const bf16_t* __restrict__ cs, int H, int D) {
-  const long t = blockIdx.x;
-  const int h = blockIdx.y, i = threadIdx.x, half = D / 2;
-  if (i >= half) return;
-  bf16_t* p = x + (t * H + h) * D;
-  const float x1 = bf2f(p[i]), x2 = bf2f(p[half + i]);
-  const float s = bf2f(sn[(long)pos[t] * half + i]), c = bf2f(cs[(long)pos[t] * half + i]);
-  if (!INV) { p[i] = f2bf(rbf(x1 * c) - rbf(x2 * s)); p[half + i] = f2bf(rbf(x2 * c) + rbf(x1 * s)); }
-  else { p[i] = f2bf(x1 * c + x2 * s); p[half + i] = f2bf(x2 * c - x1 * s); }
+__global__ void k_t_rope(bf16_t* __restrict__ q, bf16_t* __restrict__ k, const int32_t* __restrict__ pos, const bf16_t* __restrict__ sn, const bf16_t* __restrict__ cs, int H, int KVH,
+                         int D, long T) {
+  const int quads = D / 8, half = D / 2;
+  const long id = (long)blockIdx.x * 256 + threadIdx.x;
+  const long t = id / ((H + KVH) * quads);
+  if (t >= T) return;
+  const int in = (int)(id - t * ((H + KVH) * quads)), h = in / quads, i = (in - h * quads) * 4;
+  bf16_t* p = (h < H ? q + (t * H + h) * D : k + (t * KVH + h - H) * D) + i;
+  const long at = (long)pos[t] * half + i;
+  const uint2 a = *reinterpret_cast<const uint2*>(p), b = *reinterpret_cast<const uint2*>(p + half), sw = *reinterpret_cast<const uint2*>(sn + at), cw = *reinterpret_cast<const uint2*>(cs + at);
+  const float x1[4] = {bflo(a.x), bfhi(a.x), bflo(a.y), bfhi(a.y)}, x2[4] = {bflo(b.x), bfhi(b.x), bflo(b.y), bfhi(b.y)};
+  const float s[4] = {bflo(sw.x), bfhi(sw.x), bflo(sw.y), bfhi(sw.y)}, c[4] = {bflo(cw.x), bfhi(cw.x), bflo(cw.y), bfhi(cw.y)};
+  bf16_t u[4], v[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    if (!INV) { u[j] = f2bf(rbf(x1[j] * c[j]) - rbf(x2[j] * s[j])); v[j] = f2bf(rbf(x2[j] * c[j]) + rbf(x1[j] * s[j])); }
+    else { u[j] = f2bf(x1[j] * c[j] + x2[j] * s[j]); v[j] = f2bf(x2[j] * c[j] - x1[j] * s[j]); }
+  }
+  *reinterpret_cast<uint2*>(p) = make_uint2(pack2(u[0], u[1]), pack2(u[2], u[3]));
+  *reinterpret_cast<uint2*>(p + half) = make_uint2(pack2(v[0], v[1]), pack2(v[2], v[3]));
 }
 
 // Attention softmax over scores f32 [BH][S][S] with the train-mode mask (attentions.py:586-618: same segment AND col <= row), P bf16 out.
@@ -337,32 +417,39 @@ static __global__ __launch_bounds__(256) void k_t_softmax_bwd_reg(const float* _
 }
 
 // SwiGLU (linears.py:449-464) forward: act = bf16(bf16(a sg) b), sg = bf16(sigmoid(a)); backward through the unrounded formula.
-static __global__ void k_t_swiglu_fwd(const bf16_t* __restrict__ a, const bf16_t* __restrict__ b, bf16_t* __restrict__ act, long n) {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) act[i] = ixt_swiglu(bf2f(a[i]), bf2f(b[i]));
+static __global__ void k_t_swiglu_fwd(const bf16_t* __restrict__ a, const bf16_t* __restrict__ b, bf16_t* __restrict__ act, long n) {   // n a multiple of 8
+  const long i = ((long)blockIdx.x * blockDim.x + threadIdx.x) * 8;
+  if (i >= n) return;
+  const u32x4 aw = *reinterpret_cast<const u32x4*>(a + i), bw = *reinterpret_cast<const u32x4*>(b + i);
+  u32x4 o;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) o[k] = pack2(ixt_swiglu(bflo(aw[k]), bflo(bw[k])), ixt_swiglu(bfhi(aw[k]), bfhi(bw[k])));
+  *reinterpret_cast<u32x4*>(act + i) = o;
 }
 static __global__ void k_t_swiglu_bwd(const bf16_t* __restrict__ dact, const bf16_t* __restrict__ a, const bf16_t* __restrict__ b, bf16_t* __restrict__ da,
                                bf16_t* __restrict__ db, long n) {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  const long i = ((long)blockIdx.x * blockDim.x + threadIdx.x) * 8;
   if (i >= n) return;
-  const float av = bf2f(a[i]), bv = bf2f(b[i]), g = bf2f(dact[i]);
-  const float sg = 1.0f / (1.0f + ixt_exp(-av));
-  da[i] = f2bf(g * bv * sg * (1.0f + av * (1.0f - sg)));
-  db[i] = f2bf(g * av * sg);
+  float av[8], bv[8], g[8], oa[8], ob[8];
+  t_unpack8(*reinterpret_cast<const u32x4*>(a + i), av);
+  t_unpack8(*reinterpret_cast<const u32x4*>(b + i), bv);
+  t_unpack8(*reinterpret_cast<const u32x4*>(dact + i), g);
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const float sg = 1.0f / (1.0f + ixt_exp(-av[k]));
+    oa[k] = g[k] * bv[k] * sg * (1.0f + av[k] * (1.0f - sg));
+    ob[k] = g[k] * av[k] * sg;
+  }
+  *reinterpret_cast<u32x4*>(da + i) = t_pack8(oa);
+  *reinterpret_cast<u32x4*>(db + i) = t_pack8(ob);
 }
 
-// residual stream: h_out = bf16(h + y) (llama2.py:127, :157); gradient helpers
-static __global__ void k_t_add_bf16(const bf16_t* __restrict__ a, const bf16_t* __restrict__ b, bf16_t* __restrict__ out, long n) {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) out[i] = f2bf(bf2f(a[i]) + bf2f(b[i]));
-}
-static __global__ void k_t_f32_to_bf16(const float* __restrict__ a, bf16_t* __restrict__ out, long n) {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) out[i] = f2bf(a[i]);
-}
-static __global__ void k_t_bf16_to_f32(const bf16_t* __restrict__ a, float* __restrict__ out, long n, int add) {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) out[i] = (add ? out[i] : 0.0f) + bf2f(a[i]);
+static __global__ void k_t_f32_to_bf16(const float* __restrict__ a, bf16_t* __restrict__ out, long n) {   // n a multiple of 8
+  const long i = ((long)blockIdx.x * blockDim.x + threadIdx.x) * 8;
+  if (i >= n) return;
+  const float4 u = *reinterpret_cast<const float4*>(a + i), v = *reinterpret_cast<const float4*>(a + i + 4);
+  const float w[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
+  *reinterpret_cast<u32x4*>(out + i) = t_pack8(w);
 }
 
 // embedding: forward gather (embeddings.py:154) = k_embed of ixt_kernels.h; backward scatter-add of dh f32 [T][E] into dE f32 [V][E]
@@ -375,29 +462,52 @@ static __global__ void k_t_embed_bwd(const float* __restrict__ dh, const int32_t
   atomicAdd(dE + (long)id * E + e, dh[t * E + e]);
 }
 
-// cross entropy with the reference's VJP (max_utils.py:563-654, z_loss = 0) on a chunk of f32 logits [Tc][V] (already bf16-rounded values,
-// decoders.py:570,586): loss_row = log(sum exp(l - max)) + max - l[target]; dlogits = (softmax - onehot) * weight, bf16.  grid = Tc, block 256.
-static __global__ __launch_bounds__(256) void k_t_xent(const float* __restrict__ logits, const int32_t* __restrict__ targets, const int32_t* __restrict__ tseg,
+// cross entropy with the reference's VJP (max_utils.py:563-654, z_loss = 0) on a chunk of logits [Tc][V] (bf16, decoders.py:570,586):
+// loss_row = log(sum exp(l - max)) + max - l[target]; dlogits = (softmax - onehot) * weight, bf16.  The row is read 2048 columns at a time, 16 bytes a
+// thread; the sum's terms reach the threads that own them (column mod 256) through LDS.  grid = Tc, block 256.
+static __global__ __launch_bounds__(256) void k_t_xent(const bf16_t* __restrict__ logits, const int32_t* __restrict__ targets, const int32_t* __restrict__ tseg,
                                                 bf16_t* __restrict__ dlogits, float* __restrict__ row_loss, int V) {
   __shared__ float red[4];
+  __shared__ __attribute__((aligned(16))) bf16_t tile[2][2048];
   const long row = blockIdx.x;
-  const float* l = logits + row * V;
+  const int tid = threadIdx.x;
+  const bf16_t* l = logits + row * V;
   float m = -INFINITY;
-  for (int j = threadIdx.x; j < V; j += 256) m = fmaxf(m, rbf(l[j]));
+  for (int j = tid * 8; j < V; j += 2048) {
+    float v[8];
+    t_unpack8(*reinterpret_cast<const u32x4*>(l + j), v);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) m = fmaxf(m, v[k]);
+  }
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
   __syncthreads();
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+  if ((tid & 63) == 0) red[tid >> 6] = m;
   __syncthreads();
   m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
   float s = 0.0f;
-  for (int j = threadIdx.x; j < V; j += 256) s += ixt_exp(rbf(l[j]) - m);
+  u32x4 w = tid * 8 < V ? *reinterpret_cast<const u32x4*>(l + tid * 8) : u32x4(0u);
+  int buf = 0;
+  for (int j0 = 0; j0 < V; j0 += 2048, buf ^= 1) {
+    *reinterpret_cast<u32x4*>(&tile[buf][tid * 8]) = w;
+    __syncthreads();                                     // (the other buffer is written next: one barrier per tile)
+    if (j0 + 2048 + tid * 8 < V) w = *reinterpret_cast<const u32x4*>(l + j0 + 2048 + tid * 8);
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (j0 + i * 256 + tid < V) s += ixt_exp(bf2f(tile[buf][i * 256 + tid]) - m);
+  }
   s = t_block_sum(s, red);
-  const float w = tseg[row] != 0 ? 1.0f : 0.0f;
+  const float wt = tseg[row] != 0 ? 1.0f : 0.0f;
   const int tg = targets[row];
-  if (threadIdx.x == 0) row_loss[row] = w * (logf(s) + m - rbf(l[tg]));
-  const float inv = w / s;
-  for (int j = threadIdx.x; j < V; j += 256) dlogits[row * V + j] = f2bf(ixt_exp(rbf(l[j]) - m) * inv - (j == tg ? w : 0.0f));
+  if (tid == 0) row_loss[row] = wt * (logf(s) + m - bf2f(l[tg]));
+  const float inv = wt / s;
+  for (int j = tid * 8; j < V; j += 2048) {
+    float v[8];
+    t_unpack8(*reinterpret_cast<const u32x4*>(l + j), v);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = ixt_exp(v[k] - m) * inv - (j + k == tg ? wt : 0.0f);
+    *reinterpret_cast<u32x4*>(dlogits + row * V + j) = t_pack8(v);
+  }
 }
 
 // out[i] = 1 where s[i] != 0 (the weight of a target position, train.py:308-309)
@@ -419,7 +529,16 @@ static __global__ __launch_bounds__(256) void k_t_reduce(const float* __restrict
 static __global__ __launch_bounds__(256) void k_t_sumsq_partial(const float* __restrict__ x, long n, float* __restrict__ part) {
   __shared__ float red[4];
   float s = 0.0f;
-  for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long)gridDim.x * 256) { const float v = x[i]; s += v * v; }
+  const long step = (long)gridDim.x * 256;
+  long i = (long)blockIdx.x * 256 + threadIdx.x;
+  for (; i + 7 * step < n; i += 8 * step) {              // eight loads in flight, added one after the other
+    float v[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = x[i + k * step];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) s += v[k] * v[k];
+  }
+  for (; i < n; i += step) { const float v = x[i]; s += v * v; }
   s = t_block_sum(s, red);
   if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
