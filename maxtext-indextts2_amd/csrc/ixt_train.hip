@@ -184,41 +184,57 @@ extern "C" int ixt_train_refresh_bf16(ixt_trainer* t, void* stream) {
 }
 
 // ---------------------------------------------------------------------------------------------------------------- launches
-static int gemm_batched(hipStream_t st, const bf16_t* A, long sam, long sak, const bf16_t* B, long sbk, long sbn, void* C, long scm, int M, int N, int K, int out_bf16,
-                        int accumulate, int nb1, int nb2, long sab1, long sab2, long sbb1, long sbb2, long scb1, long scb2) {
-  TGemmB g;
-  g.A = A; g.sam = sam; g.sak = sak; g.sab1 = sab1; g.sab2 = sab2;
-  g.B = B; g.sbk = sbk; g.sbn = sbn; g.sbb1 = sbb1; g.sbb2 = sbb2;
-  g.C = C; g.scm = scm; g.scb1 = scb1; g.scb2 = scb2;
-  g.M = M; g.N = N; g.K = K; g.nb2 = nb2; g.out_bf16 = out_bf16; g.accumulate = accumulate;
-  if ((sam != 1 && sak != 1) || (sbk != 1 && sbn != 1)) return t_set_err(IXT_ERR_INVALID, "gemm: an operand has no unit stride");
-  const dim3 grid((N + 127) / 128, (M + 127) / 128, nb1 * nb2);
-  const bool ta = sak != 1, tb = sbk != 1;     // the operand's rows, not k, are contiguous: its tile is read transposed from LDS
-  if (ta && tb) hipLaunchKernelGGL((k_tgemm_batched<true, true>), grid, dim3(256), 0, st, g);
-  else if (ta) hipLaunchKernelGGL((k_tgemm_batched<true, false>), grid, dim3(256), 0, st, g);
-  else if (tb) hipLaunchKernelGGL((k_tgemm_batched<false, true>), grid, dim3(256), 0, st, g);
-  else hipLaunchKernelGGL((k_tgemm_batched<false, false>), grid, dim3(256), 0, st, g);
-  TLAUNCH();
-  return IXT_OK;
-}
-
 // The three products of a linear layer y = x W, W [K][N]: x W (W's columns contiguous), dy W^T (its k contiguous), x^T dy (both by columns).
 enum { TL_XW, TL_DX, TL_DW };
-template <bool TA, bool TB, int BM>
+template <bool TA, bool TB, int BM, int BN = BM>
 static int gemm_launch(hipStream_t st, TGemm& g) {
-  constexpr int BN = BM, NS = 4, lds = NS * (BM + BN) * 64, MI = BM == 64 ? 2 : BM == 128 ? 4 : 8, NI = BM == 64 ? 2 : 4, WN = BM == 256 ? 4 : 2;
-  const auto kernel = k_tgemm<TA, TB, MI, NI, 2, WN, NS>;
+  // waves and their tiles: 256 x 256: 2 x 4 of 128 x 64; 256 x 128: 4 x 2 and 128 x 128: 2 x 2 of 64 x 64; 128 x 64: 4 of 32 x 64; 64 x 64: 2 x 2 of 32 x 32
+  constexpr int WM = BN == BM ? 2 : 4, WN = BN == 256 ? 4 : BN == 64 && BM == 128 ? 1 : 2, MI = BM / 16 / WM, NI = BN / 16 / WN, NS = 4, lds = NS * (BM + BN) * 64;
+  const auto kernel = k_tgemm<TA, TB, MI, NI, WM, WN, NS>;
   static bool attr_done = false;
   if (!attr_done) {
     TCHK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds));
     attr_done = true;
   }
+  if (g.nb1 == 0) g.nb1 = g.nb2 = 1;
   g.mt = (g.M + BM - 1) / BM;
   for (int i = 0; i < 3; ++i) g.nt[i] = i < g.nprob ? (g.N[i] + BN - 1) / BN : 0;
-  const int total = g.mt * (g.nt[0] + g.nt[1] + g.nt[2]) * g.parts;
-  hipLaunchKernelGGL(kernel, dim3(8 * ((total + 7) / 8)), dim3(128 * WN), lds, st, g);
+  const int total = g.mt * (g.nt[0] + g.nt[1] + g.nt[2]) * g.parts * g.nb1 * g.nb2;
+  hipLaunchKernelGGL(kernel, dim3(8 * ((total + 7) / 8)), dim3(64 * WM * WN), lds, st, g);
   TLAUNCH();
   return IXT_OK;
+}
+// One product per (batch row, kv head), element strides between them for each operand.  The score-sized ones (a head's S x S) take square tiles, those
+// with head_dim columns tall ones; the smaller tile of each pair where the larger would leave CUs without a block (causal tiles count half).
+static int attn_gemm(hipStream_t st, bool ta, bool tb, const bf16_t* A, long lda, const bf16_t* B, long ldb, void* C, long ldc, int M, int N, int K, int out, int causal, int nb1, int nb2,
+                     long sa1, long sa2, long sb1, long sb2, long sc1, long sc2) {
+  TGemm g{};
+  g.A[0] = A; g.lda[0] = lda; g.B[0] = B; g.ldb[0] = ldb; g.C[0] = C; g.ldc[0] = ldc;
+  g.M = M; g.N[0] = N; g.K[0] = K; g.nprob = g.parts = 1; g.out = out; g.causal = causal;
+  g.nb1 = nb1; g.nb2 = nb2; g.sa1 = sa1; g.sa2 = sa2; g.sb1 = sb1; g.sb2 = sb2; g.sc1 = sc1; g.sc2 = sc2;
+  auto blocks = [&](int bm, int bn) { return (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn) * nb1 * nb2 / (causal == TC_LOWER ? 2 : 1); };
+  if (!tb) {
+    if (blocks(256, 256) >= 512) return gemm_launch<false, false, 256>(st, g);
+    if (blocks(128, 128) >= 200) return gemm_launch<false, false, 128>(st, g);
+    return gemm_launch<false, false, 64>(st, g);
+  }
+  if (N > 64 && blocks(256, 128) >= 512) return ta ? gemm_launch<true, true, 256, 128>(st, g) : gemm_launch<false, true, 256, 128>(st, g);
+  if (blocks(128, 64) >= 200) return ta ? gemm_launch<true, true, 128, 64>(st, g) : gemm_launch<false, true, 128, 64>(st, g);
+  return ta ? gemm_launch<true, true, 64>(st, g) : gemm_launch<false, true, 64>(st, g);
+}
+static void softmax_fwd(hipStream_t st, const float* scores, const int32_t* seg, bf16_t* P, int S, int B, int H) {
+  const dim3 grid(S, B * H);
+  if (S <= 512) hipLaunchKernelGGL(k_t_softmax_fwd_reg<2>, grid, dim3(256), 0, st, scores, seg, P, S, H);
+  else if (S <= 2048) hipLaunchKernelGGL(k_t_softmax_fwd_reg<8>, grid, dim3(256), 0, st, scores, seg, P, S, H);
+  else if (S <= 4096) hipLaunchKernelGGL(k_t_softmax_fwd_reg<16>, grid, dim3(256), 0, st, scores, seg, P, S, H);
+  else hipLaunchKernelGGL(k_t_softmax_fwd, grid, dim3(256), 0, st, scores, seg, P, S, H);
+}
+static void softmax_bwd(hipStream_t st, const float* dP, const bf16_t* P, bf16_t* dS, int S, int BH) {
+  const dim3 grid(S, BH);
+  if (S <= 512) hipLaunchKernelGGL(k_t_softmax_bwd_reg<2>, grid, dim3(256), 0, st, dP, P, dS, S);
+  else if (S <= 2048) hipLaunchKernelGGL(k_t_softmax_bwd_reg<8>, grid, dim3(256), 0, st, dP, P, dS, S);
+  else if (S <= 4096) hipLaunchKernelGGL(k_t_softmax_bwd_reg<16>, grid, dim3(256), 0, st, dP, P, dS, S);
+  else hipLaunchKernelGGL(k_t_softmax_bwd, grid, dim3(256), 0, st, dP, P, dS, S);
 }
 struct TOperand { const bf16_t* x; const bf16_t* w; void* c; int n; };   // TL_DX: n is the reduction (the layer's outputs), c of the first entry the result
 // M: rows (tokens; TL_DW: the layer's inputs); K: reduction (TL_DX: the entries' n); scratch: for reductions cut in parts, or nullptr
@@ -317,14 +333,12 @@ extern "C" int ixt_train_forward_backward(ixt_trainer* t, const int32_t* inputs,
     hipLaunchKernelGGL((k_t_rope<false>), EW((long)T * (H + KVH) * (D / 8)), a.q, a.k, positions, t->rope_sin, t->rope_cos, H, KVH, D, (long)T);
     // scores[b,h] = Q_h K_(h / G)^T (sm_scale 1: the query kernel carries 1/sqrt(d), attentions.py:1900-1904).  Grouped-query attention
     // (attentions.py:1206-1271: query heads reshaped to [kv heads, G]): query head kvh G + g of every kv head in launch g, batches (b, kvh).
+    const long SS = (long)S * S;
     for (int g = 0; g < G; ++g)
-      TTRY(gemm_batched(st, a.q + (long)g * D, HD, 1, a.k, 1, KN, t->scores + (long)g * S * S, S, S, S, D, 0, 0, B, KVH, (long)S * HD, (long)G * D, (long)S * KN, D,
-                (long)H * S * S, (long)G * S * S));
-    if (S <= 256 * TS_MAXV) hipLaunchKernelGGL(k_t_softmax_fwd_reg, dim3(S, B * H), dim3(256), 0, st, t->scores, segmentation, a.P, S, H);
-    else hipLaunchKernelGGL(k_t_softmax_fwd, dim3(S, B * H), dim3(256), 0, st, t->scores, segmentation, a.P, S, H);
+      TTRY(attn_gemm(st, false, false, a.q + (long)g * D, HD, a.k, KN, t->scores + g * SS, S, S, S, D, TG_F32, TC_LOWER, B, KVH, (long)S * HD, (long)G * D, (long)S * KN, D, H * SS, G * SS));
+    softmax_fwd(st, t->scores, segmentation, a.P, S, B, H);
     for (int g = 0; g < G; ++g)
-      TTRY(gemm_batched(st, a.P + (long)g * S * S, S, 1, a.v, KN, 1, a.ao + (long)g * D, HD, S, D, S, 1, 0, B, KVH, (long)H * S * S, (long)G * S * S, (long)S * KN, D,
-                (long)S * HD, (long)G * D));
+      TTRY(attn_gemm(st, false, true, a.P + g * SS, S, a.v, KN, a.ao + (long)g * D, HD, S, D, S, TG_BF16, TC_K_TO_ROW, B, KVH, H * SS, G * SS, (long)S * KN, D, (long)S * HD, (long)G * D));
     TTRY(gemm(st, TL_XW, T, QN, {{a.ao, pb + o.wo, a.h_mid, E}}, TG_BF16_RES, QN, 0, a.h_in));
     hipLaunchKernelGGL(k_t_rmsnorm_fwd, dim3(T), dim3(256), 0, st, a.h_mid, pb + o.ln2, a.xn2, a.r2, E, eps);
     TTRY(gemm(st, TL_XW, T, E, {{a.xn2, pb + o.wi0, a.a, F}, {a.xn2, pb + o.wi1, a.b, F}}, TG_BF16, E));
@@ -370,28 +384,26 @@ extern "C" int ixt_train_forward_backward(ixt_trainer* t, const int32_t* inputs,
     TTRY(gemm(st, TL_DW, QN, T, {{a.ao, t->dy_bf, t->g + o.wo, E}}, TG_F32, QN, 0, nullptr, spare, spare_n));   // d Wo = ao^T . dy
     // dP = d_ao V^T (f32) ; dV = P^T d_ao ; dS = P o (dP - rowsum(dP o P)) ; dQ = dS K ; dK = dS^T Q.  With G query heads per kv head, dV and dK
     // are the sums over the group: accumulated in f32 over the G launches, rounded to bf16 once.
+    const long SS = (long)S * S;
     for (int g = 0; g < G; ++g)
-      TTRY(gemm_batched(st, t->d_ao + (long)g * D, HD, 1, a.v, 1, KN, t->scores + (long)g * S * S, S, S, S, D, 0, 0, B, KVH, (long)S * HD, (long)G * D, (long)S * KN, D,
-                (long)H * S * S, (long)G * S * S));
+      TTRY(attn_gemm(st, false, false, t->d_ao + (long)g * D, HD, a.v, KN, t->scores + g * SS, S, S, S, D, TG_F32, TC_LOWER, B, KVH, (long)S * HD, (long)G * D, (long)S * KN, D, H * SS, G * SS));
     if (G == 1) {
-      TTRY(gemm_batched(st, a.P, 1, S, t->d_ao, HD, 1, t->dv, HD, S, D, S, 1, 0, B, H, (long)H * S * S, (long)S * S, (long)S * HD, D, (long)S * HD, D));
+      TTRY(attn_gemm(st, true, true, a.P, S, t->d_ao, HD, t->dv, HD, S, D, S, TG_BF16, TC_K_FROM_ROW, B, H, H * SS, SS, (long)S * HD, D, (long)S * HD, D));
     } else {
       for (int g = 0; g < G; ++g)
-        TTRY(gemm_batched(st, a.P + (long)g * S * S, 1, S, t->d_ao + (long)g * D, HD, 1, t->dvf, KN, S, D, S, 0, g > 0, B, KVH, (long)H * S * S, (long)G * S * S,
-                  (long)S * HD, (long)G * D, (long)S * KN, D));
+        TTRY(attn_gemm(st, true, true, a.P + g * SS, S, t->d_ao + (long)g * D, HD, t->dvf, KN, S, D, S, g > 0 ? TG_F32_ADD : TG_F32, TC_K_FROM_ROW, B, KVH, H * SS, G * SS, (long)S * HD,
+                       (long)G * D, (long)S * KN, D));
       hipLaunchKernelGGL(k_t_f32_to_bf16, EW((long)T * KN / 8), t->dvf, t->dv, (long)T * KN);
     }
-    if (S <= 256 * TS_MAXV) hipLaunchKernelGGL(k_t_softmax_bwd_reg, dim3(S, B * H), dim3(256), 0, st, t->scores, a.P, t->dS, S);
-    else hipLaunchKernelGGL(k_t_softmax_bwd, dim3(S, B * H), dim3(256), 0, st, t->scores, a.P, t->dS, S);
+    softmax_bwd(st, t->scores, a.P, t->dS, S, B * H);
     for (int g = 0; g < G; ++g)
-      TTRY(gemm_batched(st, t->dS + (long)g * S * S, S, 1, a.k, KN, 1, t->dq + (long)g * D, HD, S, D, S, 1, 0, B, KVH, (long)H * S * S, (long)G * S * S, (long)S * KN, D,
-                (long)S * HD, (long)G * D));
+      TTRY(attn_gemm(st, false, true, t->dS + g * SS, S, a.k, KN, t->dq + (long)g * D, HD, S, D, S, TG_BF16, TC_K_TO_ROW, B, KVH, H * SS, G * SS, (long)S * KN, D, (long)S * HD, (long)G * D));
     if (G == 1) {
-      TTRY(gemm_batched(st, t->dS, 1, S, a.q, HD, 1, t->dk, HD, S, D, S, 1, 0, B, H, (long)H * S * S, (long)S * S, (long)S * HD, D, (long)S * HD, D));
+      TTRY(attn_gemm(st, true, true, t->dS, S, a.q, HD, t->dk, HD, S, D, S, TG_BF16, TC_K_FROM_ROW, B, H, H * SS, SS, (long)S * HD, D, (long)S * HD, D));
     } else {
       for (int g = 0; g < G; ++g)
-        TTRY(gemm_batched(st, t->dS + (long)g * S * S, 1, S, a.q + (long)g * D, HD, 1, t->dkf, KN, S, D, S, 0, g > 0, B, KVH, (long)H * S * S, (long)G * S * S,
-                  (long)S * HD, (long)G * D, (long)S * KN, D));
+        TTRY(attn_gemm(st, true, true, t->dS + g * SS, S, a.q + (long)g * D, HD, t->dkf, KN, S, D, S, g > 0 ? TG_F32_ADD : TG_F32, TC_K_FROM_ROW, B, KVH, H * SS, G * SS, (long)S * HD,
+                       (long)G * D, (long)S * KN, D));
       hipLaunchKernelGGL(k_t_f32_to_bf16, EW((long)T * KN / 8), t->dkf, t->dk, (long)T * KN);
     }
     hipLaunchKernelGGL((k_t_rope<true>), EW((long)T * (H + KVH) * (D / 8)), t->dq, t->dk, positions, t->rope_sin, t->rope_cos, H, KVH, D, (long)T);

@@ -12,11 +12,12 @@
 //                   disjoint banks
 //   row contiguous: slot image [k][row], 32-byte pieces, piece u of row k at u ^ (k & 7) (64 rows: u ^ (k / 2 & 3)); ds_read_tr16 hands a 4 x 16 block to 16 lanes column-wise, so
 //                   the transpose costs nothing; the eight k rows a half wave touches lie on disjoint banks
-// Both put k = 4 q .. 4 q + 3 and 16 + 4 q .. on lane group q, 32 k after 32 k into one accumulator (the order of sums of k_tgemm_batched).  A piece past
+// Both put k = 4 q .. 4 q + 3 and 16 + 4 q .. on lane group q, 32 k after 32 k into one accumulator .  A piece past
 // K comes from a zeroed word instead, a row past M or N is a re-read of a valid one (its results are not stored), so dimensions need only be
 // multiples of 8.
 // One launch takes up to three products of the same M (`nprob`: the q, k and v projections, their gradients); `parts` > 1 cuts the reduction, part p
-// writing its own f32 C.  Blocks of one XCD take neighbouring tiles.
+// writing its own f32 C.  The attention's products run as batches, with the tiles and the reduction that the causal mask leaves: what it takes away is
+// zero, and a product of zeros leaves the accumulator as it is.  Blocks of one XCD take neighbouring tiles.
 #pragma once
 #include "ixt_device.h"
 
@@ -36,7 +37,11 @@ struct TGemm {
   long cpart[3];
   int out;
   int mt, nt[3];                         // tiles
+  // attention: nb1 x nb2 products of the same shape (nprob = parts = 1), element strides between them; `causal`: what the mask leaves
+  int nb1, nb2, causal;
+  long sa1, sa2, sb1, sb2, sc1, sc2;
 };
+enum { TC_NONE = 0, TC_LOWER = 1, TC_K_TO_ROW = 2, TC_K_FROM_ROW = 3 };   // C's tiles on and below the diagonal; k up to the tile's last row; k from its first row
 
 static __device__ const uint32_t tg_zero[4] = {0u, 0u, 0u, 0u};
 
@@ -50,16 +55,18 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void k_tgemm(TGemm g) {
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, r16 = lane & 15, q = lane >> 4;
   const int wm = wave / WN, wn = wave % WN;
   // XCD x takes a run of tiles (part by part); eight row tiles share their columns' operand
-  const int ntn = g.nt[0] + g.nt[1] + g.nt[2], total = g.mt * ntn, per = (total * g.parts + 7) >> 3;
+  const int ntn = g.nt[0] + g.nt[1] + g.nt[2], total = g.mt * ntn, every = total * g.parts * g.nb1 * g.nb2, per = (every + 7) >> 3;
   const int id = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
-  if (id >= total * g.parts) return;                                      // whole block
-  const int part = id / total, tile = id - part * total;
+  if (id >= every) return;                                                // whole block
+  const int z = id / total, tile = id - z * total, part = g.parts > 1 ? z : 0, z1 = z / g.nb2, z2 = z - z1 * g.nb2;
   const int grp = tile / (8 * ntn), rows = min(8, g.mt - grp * 8), in = tile - grp * 8 * ntn;
   int tn = in / rows;
   const int tm = grp * 8 + in % rows;
   int prob = 0;
   while (prob < g.nprob - 1 && tn >= g.nt[prob]) tn -= g.nt[prob++];
   const int m0 = tm * BM, n0 = tn * BN, N = g.N[prob];
+  if (g.causal == TC_LOWER && n0 > m0 + BM - 1) return;                   // whole block
+  const long za = z1 * g.sa1 + z2 * g.sa2, zb = z1 * g.sb1 + z2 * g.sb2, zc = z1 * g.sc1 + z2 * g.sc2;
 
   int segk, segend;                                                       // k: next to fetch, end
   const char *pa, *pb;                                                    // the tile's first row at segk; bytes between chunks
@@ -80,8 +87,10 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void k_tgemm(TGemm g) {
     const long la = g.lda[prob], lb = g.ldb[prob];
     segk = g.parts > 1 ? part * g.kpart : 0;
     segend = g.parts > 1 ? min(g.K[prob], segk + g.kpart) : g.K[prob];
-    pa = reinterpret_cast<const char*>(g.A[prob] + (TA ? (long)segk * la + m0 : (long)m0 * la + segk));
-    pb = reinterpret_cast<const char*>(g.B[prob] + (TB ? (long)segk * lb + n0 : (long)n0 * lb + segk));
+    if (g.causal == TC_K_TO_ROW) segend = min(segend, m0 + BM);
+    if (g.causal == TC_K_FROM_ROW) segk = m0;
+    pa = reinterpret_cast<const char*>(g.A[prob] + za + (TA ? (long)segk * la + m0 : (long)m0 * la + segk));
+    pb = reinterpret_cast<const char*>(g.B[prob] + zb + (TB ? (long)segk * lb + n0 : (long)n0 * lb + segk));
     adva = TA ? 64 * la : 64; advb = TB ? 64 * lb : 64;
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
@@ -168,7 +177,9 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void k_tgemm(TGemm g) {
 #pragma unroll
       for (int j = 0; j < NI; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[cur][j], fa[i], acc[i][j], 0, 0, 0);
       fa[i] = row_a(nxt, i);
-      if (i < NI) fb[cur ^ 1][i] = row_b(nxt, i);
+#pragma unroll
+      for (int j = 0; j < NI; ++j)
+        if (j * MI / NI == i) fb[cur ^ 1][j] = row_b(nxt, j);
 #pragma unroll
       for (int j = 0; j < NJ; ++j)
         if (j * MI / NJ == i) issue(old, j);
@@ -189,7 +200,7 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void k_tgemm(TGemm g) {
     if (m >= g.M) continue;
     const long row = (long)m * g.ldc[prob] + nw;
     if (out == TG_F32 || out == TG_F32_ADD) {
-      float* c = reinterpret_cast<float*>(g.C[prob]) + part * g.cpart[prob] + row;
+      float* c = reinterpret_cast<float*>(g.C[prob]) + (g.parts > 1 ? part * g.cpart[prob] : zc) + row;
       if (out == TG_F32_ADD) {
         tf32x4 old[NI];
 #pragma unroll
@@ -201,7 +212,7 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void k_tgemm(TGemm g) {
       for (int j = 0; j < NI; ++j)
         if (nw + j * 16 < N) *reinterpret_cast<tf32x4*>(c + j * 16) = acc[i][j];
     } else {
-      bf16_t* c = reinterpret_cast<bf16_t*>(g.C[prob]) + row;
+      bf16_t* c = reinterpret_cast<bf16_t*>(g.C[prob]) + zc + row;
       if (out == TG_BF16_RES) {
         uint2 h[NI];
 #pragma unroll

@@ -8,152 +8,6 @@
 #include "ixt_device.h"
 #include "ixt_train_gemm.h"
 
-// ---------------------------------------------------------------------------------------------------------------- batched GEMM of the attention
-// C[m][n] (+)= sum_k A(m, k) B(k, n) for bf16 operands with arbitrary element strides (either index may be the contiguous one), f32
-// accumulation, two-level batch (z = z1 * nb2 + z2).  Block = 128 x 128 x 64, 4 waves as 2 x 2, wave = 64 x 64 = 4 x 4 MFMA tiles.
-// An operand tile lies in LDS the way it lies in memory, so every global 16-byte vector is one 16-byte LDS store:
-//   k contiguous  (TR = false): image [row][k], pitch 72 elements; a lane's fragment = two 8-byte reads
-//   row contiguous (TR = true):  image [k][row], pitch 144 elements; a lane's fragment = two ds_read_b64_tr_b16 (the LDS hands a 4 x 16 block
-//                                to 16 lanes column-wise: the transpose costs nothing; pitch 288 B puts the 8 k-rows a 32-lane half touches on
-//                                8 disjoint bank groups)
-// Both forms use ONE assignment of the 32 k of an MFMA to the lanes: lane group q (= lane / 16) holds k = 4q .. 4q+3 and 16+4q .. 16+4q+3
-// of the 32-block (the sum over k does not care which lane group carries which k, as long as both operands agree) -- with it the two
-// transposed reads of a half-wave cover 8 consecutive k-rows.
-// MFMA roles: A-operand = B tile rows (n), B-operand = A tile rows (m), so a lane ends with 4 consecutive n of one m.
-struct TGemmB {
-  const bf16_t* A; long sam, sak, sab1, sab2;
-  const bf16_t* B; long sbk, sbn, sbb1, sbb2;
-  void* C; long scm, scb1, scb2;      // C row stride (n contiguous)
-  int M, N, K, nb2;
-  int out_bf16;                       // 1: C is bf16, else f32
-  int accumulate;                     // f32 output only: C += result
-};
-
-#define TG_LD 72      // [row][k] image: 64 k + 8 elements of padding (144-byte rows)
-#define TG_LDT 144    // [k][row] image: 128 rows + 16 elements of padding (288-byte rows)
-#define TG_BK 64
-#define TG_TILE (64 * TG_LDT)   // elements of one operand image (the larger of 128 x 72 and 64 x 144: equal)
-// One operand tile = 128 rows x 64 k = 1024 vectors of 8 elements, 4 per thread: fetched into registers (tg_fetch) while the previous
-// tile is being multiplied, written to LDS afterwards (tg_store) -- the global latency runs under the MFMAs.
-template <bool TR>
-__device__ __forceinline__ void tg_fetch(u32x4 (&r)[4], const bf16_t* __restrict__ g, long s_row, long s_k, int row0, int k0, int nrows, int K, int tid) {
-#pragma unroll
-  for (int it = 0; it < 4; ++it) {
-    const int v = tid + it * 256;
-    r[it] = u32x4(0);
-    if (!TR) {
-      const int rr = v >> 3, kk = (v & 7) * 8;
-      if (row0 + rr < nrows && k0 + kk < K) r[it] = *reinterpret_cast<const u32x4*>(g + (long)(row0 + rr) * s_row + (k0 + kk));
-    } else {   // rows are the contiguous index (s_row == 1): 8 consecutive rows at one k per load
-      const int rr = (v & 15) * 8, kk = v >> 4;
-      if (row0 + rr < nrows && k0 + kk < K) r[it] = *reinterpret_cast<const u32x4*>(g + (long)(k0 + kk) * s_k + (row0 + rr));
-    }
-  }
-}
-template <bool TR>
-__device__ __forceinline__ void tg_store(bf16_t* __restrict__ lds, const u32x4 (&r)[4], int tid) {
-#pragma unroll
-  for (int it = 0; it < 4; ++it) {
-    const int v = tid + it * 256;
-    if (!TR) *reinterpret_cast<u32x4*>(lds + (v >> 3) * TG_LD + (v & 7) * 8) = r[it];
-    else *reinterpret_cast<u32x4*>(lds + (v >> 4) * TG_LDT + (v & 15) * 8) = r[it];
-  }
-}
-// the 8 k of lane group q for rows row0 .. row0 + 15 of a tile, k-block ks (see the k assignment above)
-template <bool TR>
-__device__ __forceinline__ void tg_frag_issue(uint2 (&f)[2], const bf16_t* lds, int row0, int ks, int lane) {
-  const int r_in = lane & 15, q = lane >> 4;
-  if constexpr (!TR) {
-    const bf16_t* p = lds + (row0 + r_in) * TG_LD + ks * 32 + 4 * q;
-    f[0] = *reinterpret_cast<const uint2*>(p);
-    f[1] = *reinterpret_cast<const uint2*>(p + 16);
-  } else {
-    // lane 4a + p of a 16-lane group: row (k) a of the block, columns (tile rows) 4p .. 4p+3
-    const bf16_t* p = lds + (ks * 32 + 4 * q + (r_in >> 2)) * TG_LDT + row0 + 4 * (r_in & 3);
-    const uint32_t addr = (uint32_t)(uintptr_t)((const __attribute__((address_space(3))) void*)(p));
-    asm volatile("ds_read_b64_tr_b16 %0, %1" : "=v"(f[0]) : "v"(addr) : "memory");
-    asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(f[1]) : "v"(addr), "n"(16 * TG_LDT * 2) : "memory");
-  }
-}
-__device__ __forceinline__ tbf16x8 tg_frag(const uint2 (&f)[2]) {
-  u32x4 v; v.x = f[0].x; v.y = f[0].y; v.z = f[1].x; v.w = f[1].y;
-  return __builtin_bit_cast(tbf16x8, v);
-}
-
-template <bool TA, bool TB>
-__global__ __launch_bounds__(256) void k_tgemm_batched(TGemmB g) {
-  __shared__ __attribute__((aligned(16))) bf16_t As[TG_TILE];
-  __shared__ __attribute__((aligned(16))) bf16_t Bs[TG_TILE];
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int z1 = blockIdx.z / g.nb2, z2 = blockIdx.z % g.nb2;
-  const bf16_t* A = g.A + z1 * g.sab1 + z2 * g.sab2;
-  const bf16_t* B = g.B + z1 * g.sbb1 + z2 * g.sbb2;
-  const int m0 = blockIdx.y * 128, n0 = blockIdx.x * 128;
-  const int wr = wave >> 1, wc = wave & 1;
-  const int r_in = lane & 15, q = lane >> 4;
-  tf32x4 acc[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = tf32x4(0.0f);
-  u32x4 ra[4], rbv[4];
-  tg_fetch<TA>(ra, A, g.sam, g.sak, m0, 0, g.M, g.K, tid);
-  tg_fetch<TB>(rbv, B, g.sbn, g.sbk, n0, 0, g.N, g.K, tid);
-  for (int k0 = 0; k0 < g.K; k0 += TG_BK) {
-    tg_store<TA>(As, ra, tid);
-    tg_store<TB>(Bs, rbv, tid);
-    __syncthreads();
-    if (k0 + TG_BK < g.K) {                       // the next tile's loads fly while this one is multiplied
-      tg_fetch<TA>(ra, A, g.sam, g.sak, m0, k0 + TG_BK, g.M, g.K, tid);
-      tg_fetch<TB>(rbv, B, g.sbn, g.sbk, n0, k0 + TG_BK, g.N, g.K, tid);
-    }
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      uint2 fa[4][2], fb[4][2];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) tg_frag_issue<TA>(fa[i], As, wr * 64 + i * 16, ks, lane);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) tg_frag_issue<TB>(fb[j], Bs, wc * 64 + j * 16, ks, lane);
-      // the transposed reads are issued by hand: the compiler neither counts them nor knows that their registers fill late -- the wait
-      // takes the fragment registers as operands, so nothing that uses them can be scheduled ahead of it
-      if constexpr (TA) asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(fa[0][0]), "+v"(fa[0][1]), "+v"(fa[1][0]), "+v"(fa[1][1]), "+v"(fa[2][0]), "+v"(fa[2][1]), "+v"(fa[3][0]), "+v"(fa[3][1]) :: "memory");
-      if constexpr (TB) asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(fb[0][0]), "+v"(fb[0][1]), "+v"(fb[1][0]), "+v"(fb[1][1]), "+v"(fb[2][0]), "+v"(fb[2][1]), "+v"(fb[3][0]), "+v"(fb[3][1]) :: "memory");
-      tbf16x8 af[4], bf[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) af[i] = tg_frag(fa[i]);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) bf[j] = tg_frag(fb[j]);
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[j], af[i], acc[i][j], 0, 0, 0);
-    }
-    __syncthreads();
-  }
-  // D[i = n row][j = m col]: lane holds m = .. + r_in, n = .. + q * 4 + reg
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int m = m0 + wr * 64 + i * 16 + r_in;
-    if (m >= g.M) continue;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int n = n0 + wc * 64 + j * 16 + q * 4;
-      if (n >= g.N) continue;
-      const long off = z1 * g.scb1 + z2 * g.scb2 + (long)m * g.scm + n;
-      if (g.out_bf16) {
-        uint2 o;
-        o.x = pack2(f2bf(acc[i][j][0]), f2bf(acc[i][j][1])); o.y = pack2(f2bf(acc[i][j][2]), f2bf(acc[i][j][3]));
-        *reinterpret_cast<uint2*>(reinterpret_cast<bf16_t*>(g.C) + off) = o;
-      } else {
-        float4* p = reinterpret_cast<float4*>(reinterpret_cast<float*>(g.C) + off);
-        float4 v = make_float4(acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]);
-        if (g.accumulate) { const float4 o = *p; v.x += o.x; v.y += o.y; v.z += o.z; v.w += o.w; }
-        *p = v;
-      }
-    }
-  }
-}
-
 // ---------------------------------------------------------------------------------------------------------------- elementwise / rows
 // Rows of bf16 are moved 16 bytes a lane; where a sum has a place in the arithmetic, its terms stay with the threads they always had (thread t: t, t +
 // 256, ..), so that the losses and gradients of a step do not depend on how the rows are read.
@@ -319,15 +173,20 @@ __global__ void k_t_rope(bf16_t* __restrict__ q, bf16_t* __restrict__ k, const i
   *reinterpret_cast<uint2*>(p + half) = make_uint2(pack2(v[0], v[1]), pack2(v[2], v[3]));
 }
 
-// Attention softmax over scores f32 [BH][S][S] with the train-mode mask (attentions.py:586-618: same segment AND col <= row), P bf16 out.
+// Attention softmax over scores f32 [BH][S][S] with the train-mode mask (attentions.py:586-618: same segment AND col <= row), P bf16 out.  Columns up to
+// the end of the row's 256-column block are written (zeros past the row): the products that follow go no further.  The row stays in registers
+// (S <= 256 MAXV; longer rows are read again), bf16 goes out 16 bytes a lane through LDS; thread t owns the columns t, t + 256, ..
 // grid = (S, BH), block 256; one row per block.
+__device__ __forceinline__ void t_store_tiles(const bf16_t* tile, bf16_t* __restrict__ out, int n, int tid) {   // n a multiple of 8
+  for (int j = tid * 8; j < n; j += 2048) *reinterpret_cast<u32x4*>(out + j) = *reinterpret_cast<const u32x4*>(tile + j);
+}
 static __global__ __launch_bounds__(256) void k_t_softmax_fwd(const float* __restrict__ sc, const int32_t* __restrict__ seg, bf16_t* __restrict__ P, int S, int H) {
   __shared__ float red[4];
   const int row = blockIdx.x;
   const long bh = blockIdx.y, b = bh / H;
   const float* s = sc + (bh * S + row) * S;
   bf16_t* p = P + (bh * S + row) * S;
-  const int myseg = seg[b * S + row];
+  const int myseg = seg[b * S + row], end = min(S, (row / 256 + 1) * 256);
   float m = -INFINITY;
   for (int j = threadIdx.x; j <= row; j += 256)
     if (seg[b * S + j] == myseg) m = fmaxf(m, s[j]);
@@ -341,79 +200,87 @@ static __global__ __launch_bounds__(256) void k_t_softmax_fwd(const float* __res
   for (int j = threadIdx.x; j <= row; j += 256)
     if (seg[b * S + j] == myseg) l += ixt_exp(s[j] - m);
   l = t_block_sum(l, red);
-  for (int j = threadIdx.x; j < S; j += 256) {
+  for (int j = threadIdx.x; j < end; j += 256) {
     const bool on = j <= row && seg[b * S + j] == myseg;
     p[j] = on ? f2bf(ixt_exp(s[j] - m) / l) : (bf16_t)0;
   }
 }
-// The same row in ONE pass over memory (S <= 256 TS_MAXV): a thread's scores and segment tests stay in registers, every exponential is taken once.
-// Same values as the three-pass form bit for bit (same per-thread order of the partial sums); 1.70 -> see DESIGN.md section 9.
-#define TS_MAXV 16
+template <int MAXV>
 static __global__ __launch_bounds__(256) void k_t_softmax_fwd_reg(const float* __restrict__ sc, const int32_t* __restrict__ seg, bf16_t* __restrict__ P, int S, int H) {
   __shared__ float red[4];
-  const int row = blockIdx.x;
+  __shared__ __attribute__((aligned(16))) bf16_t tile[256 * MAXV];
+  const int row = blockIdx.x, tid = threadIdx.x;
   const long bh = blockIdx.y, b = bh / H;
   const float* s = sc + (bh * S + row) * S;
-  bf16_t* p = P + (bh * S + row) * S;
-  const int myseg = seg[b * S + row];
-  float v[TS_MAXV];
-  unsigned onmask = 0;
+  const int myseg = seg[b * S + row], nv = row / 256 + 1;
+  float v[MAXV];
+  unsigned on = 0;
   float m = -INFINITY;
 #pragma unroll
-  for (int i = 0; i < TS_MAXV; ++i) {
-    const int j = threadIdx.x + i * 256;
-    const bool on = j <= row && seg[b * S + min(j, S - 1)] == myseg;     // (row < S: j <= row is inside the row)
-    v[i] = on ? s[j] : -INFINITY;
-    if (on) { onmask |= 1u << i; m = fmaxf(m, v[i]); }
+  for (int i = 0; i < MAXV; ++i) {
+    const int j = tid + i * 256;
+    v[i] = -INFINITY;
+    if (i < nv && j <= row && seg[b * S + j] == myseg) { on |= 1u << i; v[i] = s[j]; }
   }
 #pragma unroll
+  for (int i = 0; i < MAXV; ++i) m = fmaxf(m, v[i]);
+#pragma unroll
   for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+  if ((tid & 63) == 0) red[tid >> 6] = m;
   __syncthreads();
   m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
   float l = 0.0f;
 #pragma unroll
-  for (int i = 0; i < TS_MAXV; ++i) {
-    if ((onmask >> i) & 1u) { v[i] = ixt_exp(v[i] - m); l += v[i]; } else v[i] = 0.0f;
+  for (int i = 0; i < MAXV; ++i) {
+    if (i < nv) { v[i] = ((on >> i) & 1u) ? ixt_exp(v[i] - m) : 0.0f; l += v[i]; }
   }
   l = t_block_sum(l, red);
 #pragma unroll
-  for (int i = 0; i < TS_MAXV; ++i) {
-    const int j = threadIdx.x + i * 256;
-    if (j < S) p[j] = ((onmask >> i) & 1u) ? f2bf(v[i] / l) : (bf16_t)0;
-  }
+  for (int i = 0; i < MAXV; ++i)
+    if (i < nv) tile[tid + i * 256] = f2bf(v[i] / l);
+  __syncthreads();
+  t_store_tiles(tile, P + (bh * S + row) * S, min(S, nv * 256), tid);
 }
-// dS = P o (dP - sum_j dP P), bf16 out (in place of nothing: separate buffer).  grid = (S, BH), block 256.
+// dS = P o (dP - sum_j dP P), bf16 out (a separate buffer), columns as above.  grid = (S, BH), block 256.
 static __global__ __launch_bounds__(256) void k_t_softmax_bwd(const float* __restrict__ dP, const bf16_t* __restrict__ P, bf16_t* __restrict__ dS, int S) {
   __shared__ float red[4];
-  const long base = ((long)blockIdx.y * S + blockIdx.x) * S;
+  const int row = blockIdx.x, end = min(S, (row / 256 + 1) * 256);
+  const long base = ((long)blockIdx.y * S + row) * S;
   float s = 0.0f;
-  for (int j = threadIdx.x; j < S; j += 256) s += dP[base + j] * bf2f(P[base + j]);
+  for (int j = threadIdx.x; j <= row; j += 256) s += dP[base + j] * bf2f(P[base + j]);
   const float dot = t_block_sum(s, red);
-  for (int j = threadIdx.x; j < S; j += 256) { const float p = bf2f(P[base + j]); dS[base + j] = f2bf(p * (dP[base + j] - dot)); }
+  for (int j = threadIdx.x; j < end; j += 256) {
+    const float p = j <= row ? bf2f(P[base + j]) : 0.0f;
+    dS[base + j] = j <= row ? f2bf(p * (dP[base + j] - dot)) : (bf16_t)0;
+  }
 }
-// one pass (S <= 256 TS_MAXV); columns beyond the row hold P = 0 (the causal mask): their dP is not read
+template <int MAXV>
 static __global__ __launch_bounds__(256) void k_t_softmax_bwd_reg(const float* __restrict__ dP, const bf16_t* __restrict__ P, bf16_t* __restrict__ dS, int S) {
   __shared__ float red[4];
-  const int row = blockIdx.x;
+  __shared__ __attribute__((aligned(16))) bf16_t tile[256 * MAXV];
+  const int row = blockIdx.x, tid = threadIdx.x, nv = row / 256 + 1, n = min(S, nv * 256);
   const long base = ((long)blockIdx.y * S + row) * S;
-  float g[TS_MAXV], pv[TS_MAXV];
+  float g[MAXV], pv[MAXV];
+#pragma unroll
+  for (int i = 0; i < MAXV; ++i) {
+    const int j = tid + i * 256;
+    g[i] = i < nv && j <= row ? dP[base + j] : 0.0f;
+  }
+  for (int j = tid * 8; j < n; j += 2048) *reinterpret_cast<u32x4*>(tile + j) = *reinterpret_cast<const u32x4*>(P + base + j);
+  __syncthreads();
   float s = 0.0f;
 #pragma unroll
-  for (int i = 0; i < TS_MAXV; ++i) {
-    const int j = threadIdx.x + i * 256;
-    const bool in = j <= row;
-    pv[i] = in ? bf2f(P[base + j]) : 0.0f;
-    g[i] = in ? dP[base + j] : 0.0f;
-    s += g[i] * pv[i];
+  for (int i = 0; i < MAXV; ++i) {
+    const int j = tid + i * 256;
+    pv[i] = i < nv && j <= row ? bf2f(tile[j]) : 0.0f;
+    if (i < nv) s += g[i] * pv[i];
   }
   const float dot = t_block_sum(s, red);
 #pragma unroll
-  for (int i = 0; i < TS_MAXV; ++i) {
-    const int j = threadIdx.x + i * 256;
-    if (j < S) dS[base + j] = f2bf(pv[i] * (g[i] - dot));
-  }
+  for (int i = 0; i < MAXV; ++i)
+    if (i < nv) tile[tid + i * 256] = f2bf(pv[i] * (g[i] - dot));
+  __syncthreads();
+  t_store_tiles(tile, dS + base, n, tid);
 }
 
 // SwiGLU (linears.py:449-464) forward: act = bf16(bf16(a sg) b), sg = bf16(sigmoid(a)); backward through the unrounded formula.
