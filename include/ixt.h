@@ -384,15 +384,16 @@ int ixt_set_sampling_ranges(ixt_ctx* ctx, const int32_t* lo_hi, int nranges);
  *                            128-column x 64-row blocks (default: never)
  *   "ring_min_rows"          from this many rows (default 128) every dot of the model runs as the LDS-ring GEMM with fused epilogues
  *                            (QKV + RoPE + page write, residual, SwiGLU, sampling; csrc/ixt_gemm.h); ixt_op_dot uses its f32 epilogue
- *   "ring_cfg"               0 (default): tile chosen per shape; 1: 128 x 128, 2: 128 rows x 64 columns, 3: 64 x 32
+ *   "ring_cfg"               0 (default): tile chosen per shape; 1: 128 x 128, 2: 128 rows x 64 columns, 3: 64 x 32, 4: 256 x 128, 5: 64 x 64,
+ *                            6: 64 x 16, 7: 128 x 128 with 32-k chunks, two blocks on a CU
  *   "ring_split"             1: ixt_op_dot's ring GEMM runs split over the 512-k chains (one f32 slice per chain)
  *   "ring_wlayout"           1: ixt_op_dot stores its weights in the ring layout ([n/128][k/64][16 fragments]: one sequential stream per block)
  *   "attn_tile"              1 (default): prefill calls of at least "attn_tile_min_rows" rows (default 64) run the tiled attention, 16 (other
  *                            page sizes: 8 past ~1500 keys) consecutive rows per block: on the f32 matrix units for 32-token pages and at most 4096
  *                            keys, on the vector units otherwise; 2: always on the vector units; 0: one block per (row, kv head) as for decode rows
- *   "unembed_tall"           1 (default): the unembedding at 129..256 rows uses 256 x 128 tiles (weights enter the chip once); 0: 128 x 128
- *   "ring_two_per_cu"        1 (default): ring GEMMs (and the unembedding) of 1024 rows and more with at least 320 tiles of 128 x 128 use 32-k chunks
- *                            in 4 slots (64 KiB of LDS: two blocks per CU overlap each other's prologue and epilogue); 0: the 64-k chunk form
+ *   "unembed_tall"           1 (default): the unembedding may take 256 x 128 tiles (at 129..256 rows its weights enter the chip once); 0: never
+ *   "ring_two_per_cu"        1 (default): ring GEMMs (and the unembedding) may take 128 x 128 tiles with 32-k chunks in 4 slots (64 KiB of LDS: two
+ *                            blocks per CU overlap each other's prologue and epilogue); 0: never
  *   "ring_down"              MLP down-projection on the ring path: 1 ring GEMM + residual epilogue, 0 split-K tiles + slice-sum kernel,
  *                            -1 (default) by shape */
 int ixt_set_option(ixt_ctx* ctx, const char* name, int value);

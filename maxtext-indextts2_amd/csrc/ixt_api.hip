@@ -684,15 +684,40 @@ static void timing_end(ixt_ctx* c, hipStream_t st, int idx) {
 }
 
 // --------------------------------------------------------------------------------------- LDS-ring GEMM (ixt_gemm.h)
-// Tiles: 1 = 128 x 128 (8 waves as 2 x 4, 4 ring slots of 32 KiB), 2 = 128 rows x 64 columns (8 waves, 5 x 24 KiB), 3 = 64 x 32 (4 waves, 6 x 24 KiB,
-// 128-k chunks).
-static int ring_pick(const ixt_ctx* c, int epi, int R, int N) {
-  if (c->ring_cfg >= 1 && c->ring_cfg <= 3 && !(epi == GEPI_SWIGLU && c->ring_cfg == 3) && !(epi == GEPI_UNEMBED && c->ring_cfg != 1)) return c->ring_cfg;
-  if (epi == GEPI_UNEMBED) return 1;
-  const long b1 = (long)((N + 127) / 128) * ((R + 127) / 128), b2 = (long)((N + 63) / 64) * ((R + 127) / 128);
-  if (b1 >= 192) return 1;                    // the chip has 256 CUs and a block owns one (LDS): fewer blocks leave CUs without work
-  if (b2 >= 160 || epi == GEPI_SWIGLU) return 2;
-  return 3;
+// Tiles (rows x columns): 1 = 128 x 128 (8 waves as 2 x 4, 4 slots of 32 KiB), 2 = 128 x 64 (8 waves, 5 x 24 KiB), 3 = 64 x 32 (4 waves, 6 x 24 KiB,
+// 128-k chunks), 4 = 256 x 128 (8 waves of 64 x 64, 3 x 48 KiB), 5 = 64 x 64 (4 waves, 4 x 16 KiB: two blocks share a CU), 6 = 64 x 16 (4 waves, 6 x 20 KiB,
+// 128-k chunks), 7 = 128 x 128 with 32-k chunks (4 x 16 KiB, two blocks share a CU).
+//
+// A launch takes as many rounds as its fullest XCD has blocks for its 32 CUs, and a round of one tile takes the same time whatever the sizes: what one 64-k
+// chunk takes, in units of 10 ns, measured on 9 numbers of rows (128 .. 2048) x 8 projections (K 2048 .. 9216, N 2048 .. 18432) -- tile 4: 100, 1: 62, 2: 44,
+// 5: 31 (52 for two blocks of a CU), 3: 22, 6: 19, 7: 66 (122 for two).  The least estimate is within 6 % of the fastest tile on all but 3 of these 72
+// (within 12 %); the rule that looked at the number of 128 x 128 tiles alone took 62 us where this takes 40 (256 x 2304 outputs, K 9216) and 122 where this
+// takes 102 (1525 x 14336, K 2048).
+static int ring_pick(const ixt_ctx* c, int epi, int R, int N, bool routed, bool wring) {
+  if (c->ring_cfg >= 1 && c->ring_cfg <= 7 && !(epi == GEPI_SWIGLU && (c->ring_cfg == 3 || c->ring_cfg == 6)) && !(epi == GEPI_UNEMBED && c->ring_cfg != 1) && !(routed && c->ring_cfg == 4) &&
+      !(wring && c->ring_cfg == 7)) return c->ring_cfg;
+  if (routed) {   // every expert's rows are one or two groups of 128, whatever the launch's total: the blocks that have work are not known here
+    const long b1 = (long)((N + 127) / 128) * ((R + 127) / 128), b2 = (long)((N + 63) / 64) * ((R + 127) / 128);
+    return b1 >= 192 ? 1 : b2 >= 160 || epi == GEPI_SWIGLU ? 2 : 3;
+  }
+  static const struct { int id, rows, cols, one, two; } tiles[] = {{4, 256, 128, 100, 0}, {7, 128, 128, 66, 122}, {1, 128, 128, 62, 0}, {2, 128, 64, 44, 0},
+                                                                    {5, 64, 64, 31, 52},  {3, 64, 32, 22, 0},     {6, 64, 16, 19, 0}};
+  int best = 1;
+  long least = -1;
+  for (const auto& t : tiles) {
+    if ((epi == GEPI_SWIGLU && t.cols < 64) || (epi == GEPI_UNEMBED && t.cols < 64)) continue;   // gate pairs are two column tiles of a wave; few waves a row for the sampling
+    if ((t.id == 7 && (!c->ring_two_per_cu || wring)) || (t.id == 4 && epi == GEPI_UNEMBED && !c->unembed_tall)) continue;
+    const long per_xcd = (long)(((N + t.cols - 1) / t.cols + 7) / 8) * ((R + t.rows - 1) / t.rows);
+    long cost;
+    if (t.two) {
+      const long rest = per_xcd % 64;
+      cost = per_xcd / 64 * t.two + (rest == 0 ? 0 : rest <= 32 ? t.one : t.two);
+    } else {
+      cost = (per_xcd + 31) / 32 * t.one;
+    }
+    if (least < 0 || cost < least) { least = cost; best = t.id; }
+  }
+  return best;
 }
 
 template <int WR, int WC, int RB, int CT, int KS, int NS, int EPI, int SPLIT>
@@ -719,7 +744,7 @@ int launch_ring(ixt_ctx* c, int epi, const bf16_t* x, const bf16_t* w, int K, in
                 int* wave_cols) {
   if (K % IXT_KALIGN || N % 16) return set_err(IXT_ERR_UNSUPPORTED, "ring gemm: K %% 128 or N %% 16");
   const int chains = (K + IXT_CHAIN - 1) / IXT_CHAIN;
-  const int cfg = ring_pick(c, epi, R, N);
+  const int cfg = ring_pick(c, epi, R, N, e.rb_exp != nullptr, wring != 0);
   double ebytes = 0.0;
   switch (epi) {
     case GEPI_F32: ebytes = (double)(split ? chains : 1) * R * N * 4.0; break;
@@ -731,47 +756,36 @@ int launch_ring(ixt_ctx* c, int epi, const bf16_t* x, const bf16_t* w, int K, in
   }
   const int ti = timing_begin(c, st, (double)K * N * 2.0 + (double)R * K * 2.0 + ebytes);
   int rc = IXT_ERR_UNSUPPORTED;
-#define RING_A(EPI_, SPLIT_) ring_launch_t<2, 4, 4, 2, 2, 4, EPI_, SPLIT_>(x, w, K, N, R, chains, wring, e, st, wave_cols)
-#define RING_B(EPI_) ring_launch_t<2, 4, 4, 1, 2, 5, EPI_, 0>(x, w, K, N, R, chains, wring, e, st, wave_cols)
-#define RING_C(EPI_) ring_launch_t<2, 2, 2, 1, 4, 6, EPI_, 0>(x, w, K, N, R, chains, wring, e, st, wave_cols)
-#define RING(EPI_) do { if (cfg == 1) rc = RING_A(EPI_, 0); else if (cfg == 2) rc = RING_B(EPI_); else rc = RING_C(EPI_); } while (0)
-  // Prefill-sized launches (several rounds of blocks per CU): the 128 x 128 tile with 32-k chunks in 4 slots = 64 KiB of LDS, so TWO blocks
-  // share a CU and one's prologue (first chunk's latency) and epilogue run under the other's main loop: 7.6 -> 6.7 ms of GEMMs per 2048-row
-  // pass.  At 256 rows a launch has at most one block per CU anyway and the 64-k chunks (half the barriers) are faster.
-#define RING_P(EPI_) ring_launch_t<2, 4, 4, 2, 1, 4, EPI_, 0>(x, w, K, N, R, chains, wring, e, st, wave_cols)
-  // (launches of up to 256 tiles -- O / MLP down at 2048 rows -- have one block per CU either way, and there the 64-k chunks win: 8.5 against 8.7 ms
-  // per pass with 512 tiles of 128 x 64 in 72 KiB; from 384 tiles on -- QKV at 1024 rows -- the two-per-CU form wins)
-  // (routed experts: every expert's rows are ONE or two row groups -- the 256-row regime per expert, whatever the launch's total: 64-k chunks.  Mixtral-8x7B
-  //  256-token prefill 29.8 -> 26.7 ms)
-  const bool two_per_cu = c->ring_two_per_cu && R >= 1024 && cfg == 1 && !split && e.rb_exp == nullptr && (long)((N + 127) / 128) * ((R + 127) / 128) >= 320;
-  if (two_per_cu && epi == GEPI_RESID) rc = RING_P(GEPI_RESID);
-  else if (two_per_cu && epi == GEPI_QKV) rc = RING_P(GEPI_QKV);
-  else if (two_per_cu && epi == GEPI_SWIGLU) rc = RING_P(GEPI_SWIGLU);
-  else if (two_per_cu && epi == GEPI_F32) rc = RING_P(GEPI_F32);
-  else if (two_per_cu && epi == GEPI_TANHNORM) rc = RING_P(GEPI_TANHNORM);
-  else if (two_per_cu && epi == GEPI_ACT) rc = RING_P(GEPI_ACT);
-  else if (epi == GEPI_F32 && split) rc = RING_A(GEPI_F32, 1);
-  else if (epi == GEPI_F32) RING(GEPI_F32);
-  else if (epi == GEPI_RESID) RING(GEPI_RESID);
-  else if (epi == GEPI_TANHNORM) RING(GEPI_TANHNORM);
-  else if (epi == GEPI_ACT) RING(GEPI_ACT);
-  else if (epi == GEPI_QKV) RING(GEPI_QKV);
-  else if (two_per_cu && epi == GEPI_UNEMBED) rc = RING_P(GEPI_UNEMBED);
-  else if (epi == GEPI_UNEMBED) {
-    // the unembedding at 129..256 rows: ONE block owns all rows of its 128 columns (8 waves of 64 x 64: 256 x 128 tile, 3 slots of 48 KiB), so the
-    // 1 GB kernel enters the chip once instead of once per 128-row group
-    if (c->unembed_tall && R > 128 && R <= 256) rc = ring_launch_t<4, 2, 4, 4, 2, 3, GEPI_UNEMBED, 0>(x, w, K, N, R, chains, wring, e, st, wave_cols);
-    else rc = RING_A(GEPI_UNEMBED, 0);
+#define RING_T(WR_, WC_, RB_, CT_, KS_, NS_, EPI_, SPLIT_) ring_launch_t<WR_, WC_, RB_, CT_, KS_, NS_, EPI_, SPLIT_>(x, w, K, N, R, chains, wring, e, st, wave_cols)
+#define RING_WIDE(EPI_)                                                    \
+  case 1: rc = RING_T(2, 4, 4, 2, 2, 4, EPI_, 0); break;                   \
+  case 4: rc = RING_T(4, 2, 4, 4, 2, 3, EPI_, 0); break;                   \
+  case 5: rc = RING_T(2, 2, 2, 2, 2, 4, EPI_, 0); break;                   \
+  case 7: rc = RING_T(2, 4, 4, 2, 1, 4, EPI_, 0); break
+#define RING(EPI_)                                                         \
+  switch (cfg) {                                                           \
+    RING_WIDE(EPI_);                                                       \
+    case 2: rc = RING_T(2, 4, 4, 1, 2, 5, EPI_, 0); break;                 \
+    case 3: rc = RING_T(2, 2, 2, 1, 4, 6, EPI_, 0); break;                 \
+    case 6: rc = RING_T(4, 1, 1, 1, 4, 6, EPI_, 0); break;                 \
   }
-  else if (epi == GEPI_SWIGLU) {
-    if (cfg == 1) rc = RING_A(GEPI_SWIGLU, 0);
-    else rc = ring_launch_t<2, 2, 4, 2, 2, 5, GEPI_SWIGLU, 0>(x, w, K, N, R, chains, wring, e, st, wave_cols);   // gate pairs need two tiles per wave: 4 waves
+#define RING_PAIRS(EPI_)                                                   \
+  switch (cfg) {                                                           \
+    RING_WIDE(EPI_);                                                       \
+    case 2: rc = RING_T(2, 2, 4, 2, 2, 5, EPI_, 0); break;                 \
   }
+  if (epi == GEPI_F32 && split) rc = RING_T(2, 4, 4, 2, 2, 4, GEPI_F32, 1);
+  else if (epi == GEPI_F32) RING(GEPI_F32)
+  else if (epi == GEPI_RESID) RING(GEPI_RESID)
+  else if (epi == GEPI_TANHNORM) RING(GEPI_TANHNORM)
+  else if (epi == GEPI_ACT) RING(GEPI_ACT)
+  else if (epi == GEPI_QKV) RING(GEPI_QKV)
+  else if (epi == GEPI_UNEMBED) RING_PAIRS(GEPI_UNEMBED)
+  else if (epi == GEPI_SWIGLU) RING_PAIRS(GEPI_SWIGLU)
+#undef RING_T
+#undef RING_WIDE
 #undef RING
-#undef RING_A
-#undef RING_B
-#undef RING_C
-#undef RING_P
+#undef RING_PAIRS
   timing_end(c, st, ti);
   if (rc == IXT_ERR_UNSUPPORTED) return set_err(rc, "ring gemm: epilogue %d", epi);
   return rc;

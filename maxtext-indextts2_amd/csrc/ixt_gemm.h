@@ -5,15 +5,16 @@
 //   * both operands are stored in HBM in fragment order (1 KiB = one wave-instruction), so a K-chunk of a block tile is a list of
 //     fragments that LDS-DMA (`global_load_lds_dwordx4`: 64 lanes x 16 B, no VGPRs) drops into an LDS ring slot exactly as the MFMAs
 //     read them (lane-linear, conflict-free ds_read_b128);
-//   * NS ring slots, NS - 1 chunks in flight per block behind a counted `s_waitcnt vmcnt(N)` and ONE raw s_barrier per chunk (the
-//     memory latency of a chunk is hidden behind the two or more chunks ahead of it; k_gemm had one chunk in flight and waited for
-//     every one of them);
+//   * NS ring slots behind a counted `s_waitcnt vmcnt(N)` and ONE raw s_barrier per chunk: the latency of a chunk is hidden behind the
+//     chunks ahead of it, and the reads of the next 32 k run under the products of these;
 //   * a block owns whole (tile, all chains) work items: the chain totals stay in registers and the epilogue consumes them on chip --
 //     no f32 slice leaves the chip except in the op-level / split forms.
 // Block = WR x WC waves; wave tile = RB 16-row blocks x CT 16-column tiles; block tile = 16 WR RB rows x 16 WC CT columns.
-// Measured with in-kernel stamps (tools/ring_probe.hip): an LDS-DMA issue holds its wave for about 75 cycles and MFMA issue is in order,
-// so one wave per SIMD runs load issue and MFMAs back to back (128 x 128 x 64-k chunk: 1 550 cycles); with TWO waves per SIMD (8-wave
-// blocks) one wave's MFMAs run under the other's load issue.
+// What bounds it: a 128 x 128 tile fetches as many bytes a chunk as the CU's 64 B a cycle bring in the time of its products (512 cycles of each per 64 k;
+// measured 31 TB/s over the chip from L2), and a fetch that finds the queue full holds its wave and the MFMAs behind it.  256 x 128 tiles need 3/4 of
+// that and win wherever the launch has enough of them: 14336 columns, K 2048, 1525 rows: 122 us (735 TFLOP/s) with 128 x 128 tiles whose chunk was
+// read and then multiplied, 112 with the reads under the products, 102 (881 TFLOP/s) with 256 x 128.  Tried without gain: the fetches of a SIMD's two waves in
+// different halves of a chunk, hot weights, chunk-contiguous operands.
 //
 // Epilogues (EPI):
 //   GEPI_F32      f32 [slice][R][N] (op-level entry point, split-K form)
@@ -98,6 +99,14 @@ template <int N_>
 __device__ __forceinline__ void ring_wait() {
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N_) : "memory");
 }
+// at most min(M, younger) chunks of NJ fetches outstanding, and no LDS read
+template <int NJ, int M>
+__device__ __forceinline__ void ring_wait_chunks(int younger) {
+  if constexpr (M > 0) {
+    if (younger < M) return ring_wait_chunks<NJ, M - 1>(younger);
+  }
+  ring_wait<M * NJ>();
+}
 
 //   grid = (8 ceil(ncolg / 8) zb, SPLIT ? chains : 1), block 64 WR WC, dynamic LDS = NS (WC CT + WR RB) KS KiB.
 //   Row groups of one column group are block ids b, b + 8, ..: same XCD, the weights meet in its L2.
@@ -113,11 +122,10 @@ __global__ __launch_bounds__(WR * WC * 64, 2) void k_gemm_ring(const u32x4* __re
   constexpr int NXF = TR * KS;         // activation fragments
   constexpr int NF = NWF + NXF;
   constexpr int NJ = NF / NW;          // fragments a wave fetches per chunk
-  constexpr int D = NS - 1;            // chunks in flight
-  static_assert(NF % NW == 0 && 16 % KS == 0 && (D - 1) * NJ < 64, "ring geometry");
+  static_assert(NF % NW == 0 && 16 % KS == 0 && (NS - 1) * NJ < 64 && NS > 1 && (KS == 1 || KS % 2 == 0), "ring geometry");
   static_assert(EPI != GEPI_SWIGLU || CT % 2 == 0, "gate pairs need two tiles per wave");
   extern __shared__ __attribute__((aligned(16))) u32x4 st[];   // [NS][NF fragments][64 lanes]
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int bx = blockIdx.x;
   const int colg = (bx / (8 * zb)) * 8 + (bx & 7), rowg = (bx >> 3) % zb;
   if (colg >= ncolg) return;                                    // whole block: no barrier is skipped
@@ -131,133 +139,141 @@ __global__ __launch_bounds__(WR * WC * 64, 2) void k_gemm_ring(const u32x4* __re
   const int nchunks = nsteps / KS;
   const int wr = wave / WC, wc = wave % WC;
   const int r_in = lane & 15, cq = lane >> 4;
-  const u32x4* src[NJ];
-  // weights: fragment order [tile][k-step] (wring == 0: the layout of the small-batch kernels) or the ring layout (r8frag)
-  const size_t wadv = wring ? (size_t)KS * 8 * 64 : (size_t)KS * 64;   // fragments (x 64 lanes) between two chunks of one tile
+  // weights: fragment order [tile][k-step] (wring == 0: the layout of the small-batch kernels) or the ring layout (r8frag).  A wave's pieces of a chunk:
+  // one offset a piece from the first fragment of the block's tiles, one scalar address that moves from chunk to chunk
+  const size_t wadv = (wring ? (size_t)KS * 8 : (size_t)KS) * 1024;    // bytes between two chunks of one tile
+  uint32_t off[NJ];
 #pragma unroll
   for (int j = 0; j < NJ; ++j) {
     const int f = wave + NW * j;
     if (f < NWF) {
       const int tile = wring ? colg * TC + f / KS : min(colg * TC + f / KS, ntile - 1);    // past the end: a valid (wring: padding) tile, results dropped
-      src[j] = wt + (wring ? r8frag(tile, f % KS, nsteps) : (size_t)tile * nsteps + (f % KS)) * 64 + lane;
+      off[j] = (uint32_t)(wring ? r8frag(tile, f % KS, nsteps) - r8frag(colg * TC, 0, nsteps) : (size_t)(tile - colg * TC) * nsteps + (f % KS)) * 1024u;
     } else {
       const int rb = min(rowg * TR + (f - NWF) / KS, nrbk - 1);
-      src[j] = xt + ((size_t)rb * nsteps + ((f - NWF) % KS)) * 64 + lane;
+      off[j] = (uint32_t)((rb - rowg * TR) * nsteps + (f - NWF) % KS) * 1024u;
     }
+    off[j] += lane * 16;
   }
   constexpr int CPC = (F8 ? 8 : 16) / KS;                       // chunks per 512-k chain
   const int chb = SPLIT ? (int)blockIdx.y * CPC : 0;
   const int che = SPLIT ? min(nchunks, chb + CPC) : nchunks;
-#define IXT_RISSUE(CH_, SLOT_)                                                                                         \
-  do {                                                                                                                 \
-    _Pragma("unroll") for (int j = 0; j < NJ; ++j)                                                                     \
-      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src[j] + (size_t)(CH_) * (wave + NW * j < NWF ? wadv : (size_t)KS * 64)), \
-                                       (__attribute__((address_space(3))) void*)(st + ((SLOT_) * NF + wave + NW * j) * 64), 16, 0, 0); \
-  } while (0)
+  const char* pw = reinterpret_cast<const char*>(wt + (wring ? r8frag(colg * TC, 0, nsteps) : (size_t)colg * TC * nsteps) * 64) + chb * wadv;
+  const char* px = reinterpret_cast<const char*>(xt + (size_t)rowg * TR * nsteps * 64) + (size_t)chb * KS * 1024;
+  const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)((__attribute__((address_space(3))) u32x4*)st));
+  // piece j of the next chunk to fetch, into a slot.  Issued by hand (no register is written, nothing else in this kernel uses m0): behind the builtin the
+  // compiler may wait for every fetch in flight before an LDS read; the waits are counted in the loop.
+  auto issue = [&](int slot, int j) {
+    const uint32_t dst = lds0 + (uint32_t)(slot * NF + wave + NW * j) * 1024u;
+    if (NW * j + NW <= NWF) asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(off[j]), "s"(pw) : "memory");
+    else if (NW * j >= NWF) asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(off[j]), "s"(px) : "memory");
+    else {
+      const uint64_t p = wave + NW * j < NWF ? (uint64_t)(uintptr_t)pw : (uint64_t)(uintptr_t)px;
+      asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(off[j]), "s"(p) : "memory");
+    }
+  };
+  auto advance = [&]() { pw += wadv; px += (size_t)KS * 1024; };
 #pragma unroll
-  for (int c = 0; c < D; ++c)
-    if (chb + c < che) IXT_RISSUE(chb + c, c);
+  for (int c = 0; c < NS; ++c)
+    if (chb + c < che) {
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) issue(c, j);
+      advance();
+    }
   f32x4 acc[CT][RB], tot[CT][RB];
 #pragma unroll
   for (int i = 0; i < CT; ++i)
 #pragma unroll
     for (int b = 0; b < RB; ++b) { acc[i][b] = f32x4(0.0f); tot[i][b] = f32x4(0.0f); }
+  bf16x8 wf[CT], xf[2][RB];
+  auto wfrag = [&](int slot, int ks, int i) { return __builtin_bit_cast(bf16x8, st[(slot * NF + (wc * CT + i) * KS + ks) * 64 + lane]); };
+  auto xfrag = [&](int slot, int ks, int b) { return __builtin_bit_cast(bf16x8, st[(slot * NF + NWF + (wr * RB + b) * KS + ks) * 64 + lane]); };
+  ring_wait_chunks<NJ, NS - 1>(che - chb - 1);                  // chunk chb
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+#pragma unroll
+  for (int b = 0; b < RB; ++b) xf[0][b] = xfrag(0, 0, b);
+#pragma unroll
+  for (int i = 0; i < CT; ++i) wf[i] = wfrag(0, 0, i);
   int slot = 0;                                                 // ring slot of chunk ch
-#ifdef IXT_RING_STAMPS   // diagnostic build (tools/ring_probe.hip): where an iteration spends its cycles; never defined in the product
-  unsigned long long st0 = 0, st1 = 0, st2 = 0, st3 = 0, st4 = 0, sum_wait = 0, sum_bar = 0, sum_issue = 0, sum_comp = 0;
-#define IXT_STAMP(T_) do { __builtin_amdgcn_sched_barrier(0); asm volatile("s_memtime %0\n\ts_waitcnt lgkmcnt(0)" : "=s"(T_) :: "memory"); __builtin_amdgcn_sched_barrier(0); } while (0)
-#else
-#define IXT_STAMP(T_) do { } while (0)
-#endif
-  for (int ch = chb; ch < che; ++ch) {
-    IXT_STAMP(st0);
-    // chunk ch has landed once at most min(D - 1, chunks after it) x NJ of this wave's younger loads are outstanding; the LDS reads
-    // of the previous chunk are retired (lgkmcnt(0)) before the barrier lets any wave refill their slot
-    const int rem = che - 1 - ch;
-    if (rem >= D - 1) ring_wait<(D - 1) * NJ>();
-    else if (D > 2 && rem == 2) ring_wait<(D > 2 ? 2 : 0) * NJ>();
-    else if (D > 1 && rem == 1) ring_wait<(D > 1 ? 1 : 0) * NJ>();
-    else if (D > 3 && rem == 3) ring_wait<(D > 3 ? 3 : 0) * NJ>();
-    else ring_wait<0>();
-    IXT_STAMP(st1);
-    __builtin_amdgcn_s_barrier();
-    IXT_STAMP(st2);
-    // All LDS reads of the chunk first (their latency then runs under the issue of the refill loads), then the MFMAs in groups of RB
-    // with the NJ refill loads of chunk ch + D dealt between the groups: an LDS-DMA issue costs the wave about 50 cycles, a group of
-    // 4 MFMAs keeps the matrix pipe busy for 64, so the refill rides under the MFMAs instead of in front of them.
-    const u32x4* sb = st + (size_t)slot * NF * 64;
-    bf16x8 wf[KS][CT], xf[KS][RB];
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-#pragma unroll
-      for (int i = 0; i < CT; ++i) wf[ks][i] = __builtin_bit_cast(bf16x8, sb[((wc * CT + i) * KS + ks) * 64 + lane]);
-#pragma unroll
-      for (int b = 0; b < RB; ++b) xf[ks][b] = __builtin_bit_cast(bf16x8, sb[(NWF + (wr * RB + b) * KS + ks) * 64 + lane]);
+  bool refill = false;
+  int fill = 0;
+  // One k-step: products of the fragments in registers, with the reads of the next step's fragments and the refill of the slot that was read out last dealt
+  // between them, so that the matrix cores, the LDS and the fetches run side by side (reading a chunk and then multiplying it took turns: 1 500 cycles a
+  // 64-k chunk of a 128 x 128 tile, of which the products are 512).  Ahead of a chunk's last step its fragments are all in registers and the next chunk has
+  // to be there: one counted wait and one barrier a chunk, behind which its slot is free for chunk ch + NS.
+  auto step = [&](int ch, int ks, int cur) {
+    const bool last = ks == KS - 1;
+    if (last) {
+      ring_wait_chunks<NJ, NS - 2>(che - ch - 2);
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      refill = ch + NS < che;
+      fill = slot;
+      slot = slot + 1 == NS ? 0 : slot + 1;
     }
-    IXT_STAMP(st3);
-    const bool refill = ch + D < che;
-    const int fill = slot == 0 ? NS - 1 : slot - 1;             // the slot of chunk ch - 1 = that of chunk ch + D
-    constexpr int NG = KS * CT;                                 // MFMA groups of an iteration
+    const int nks = last ? 0 : ks + 1, from = ks == KS - 1 ? 0 : ks + 1;   // `from`: position of this step among the KS steps of a refill
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
+    for (int i = 0; i < CT; ++i) {
 #pragma unroll
-      for (int i = 0; i < CT; ++i) {
-#pragma unroll
-        for (int b = 0; b < RB; ++b) {
-          if constexpr (F8) {
-            typedef long l2 __attribute__((ext_vector_type(2)));
-            const l2 wl = __builtin_bit_cast(l2, wf[ks][i]), xl = __builtin_bit_cast(l2, xf[ks][b]);
-            acc[i][b] = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(wl[0], xl[0], acc[i][b], 0, 0, 0);
-            acc[i][b] = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(wl[1], xl[1], acc[i][b], 0, 0, 0);
-          } else {
-            acc[i][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[ks][i], xf[ks][b], acc[i][b], 0, 0, 0);
-          }
-        }
-        const int gi = ks * CT + i;
-        if (refill) {
-#pragma unroll
-          for (int j = 0; j < NJ; ++j)
-            if (j * NG / NJ == gi)                              // load j rides behind group j NG / NJ
-              __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src[j] + (size_t)(ch + D) * (wave + NW * j < NWF ? wadv : (size_t)KS * 64)),
-                                               (__attribute__((address_space(3))) void*)(st + (fill * NF + wave + NW * j) * 64), 16, 0, 0);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    }
-    if (((ch + 1) % CPC) == 0 || ch + 1 == che) {               // a 512-k chain is complete
-      if constexpr (F8) {                                       // scale the chain by (activation block scale) x (column scale)
-        const int chain = ch / CPC, nchains = (nchunks + CPC - 1) / CPC;
-#pragma unroll
-        for (int b = 0; b < RB; ++b) {
-          const int row = min((rowg * TR + wr * RB + b) * 16 + r_in, R - 1);
-          const float a = e.xscale[(size_t)row * nchains + chain];
-#pragma unroll
-          for (int i = 0; i < CT; ++i) {
-            const int tile = min(colg * TC + wc * CT + i, ntile - 1);
-            const float4 sn = *reinterpret_cast<const float4*>(e.wscale + tile * 16 + cq * 4);
-            acc[i][b][0] *= a * sn.x; acc[i][b][1] *= a * sn.y; acc[i][b][2] *= a * sn.z; acc[i][b][3] *= a * sn.w;
-          }
+      for (int b = 0; b < RB; ++b) {
+        if constexpr (F8) {
+          typedef long l2 __attribute__((ext_vector_type(2)));
+          const l2 wl = __builtin_bit_cast(l2, wf[i]), xl = __builtin_bit_cast(l2, xf[cur][b]);
+          acc[i][b] = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(wl[0], xl[0], acc[i][b], 0, 0, 0);
+          acc[i][b] = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(wl[1], xl[1], acc[i][b], 0, 0, 0);
+        } else {
+          acc[i][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[i], xf[cur][b], acc[i][b], 0, 0, 0);
         }
       }
+      wf[i] = wfrag(slot, nks, i);
 #pragma unroll
-      for (int i = 0; i < CT; ++i)
+      for (int b = 0; b < RB; ++b)
+        if (b * CT / RB == i) xf[cur ^ 1][b] = xfrag(slot, nks, b);
+      const int gi = from * CT + i;
+      if (refill) {
 #pragma unroll
-        for (int b = 0; b < RB; ++b) { tot[i][b] = tot[i][b] + acc[i][b]; acc[i][b] = f32x4(0.0f); }
+        for (int j = 0; j < NJ; ++j)
+          if (j * (KS * CT) / NJ == gi) issue(fill, j);
+      }
+      __builtin_amdgcn_sched_barrier(0);
     }
-    slot = slot + 1 == NS ? 0 : slot + 1;
-#ifdef IXT_RING_STAMPS
-    IXT_STAMP(st4);
-    sum_wait += st1 - st0; sum_bar += st2 - st1; sum_issue += st3 - st2; sum_comp += st4 - st3;
-#endif
+    if (refill && from == KS - 1) advance();
+  };
+  // a 512-k chain is complete
+  auto chain_end = [&](int ch) {
+    if constexpr (F8) {                                         // scale the chain by (activation block scale) x (column scale)
+      const int chain = ch / CPC, nchains = (nchunks + CPC - 1) / CPC;
+#pragma unroll
+      for (int b = 0; b < RB; ++b) {
+        const int row = min((rowg * TR + wr * RB + b) * 16 + r_in, R - 1);
+        const float a = e.xscale[(size_t)row * nchains + chain];
+#pragma unroll
+        for (int i = 0; i < CT; ++i) {
+          const int tile = min(colg * TC + wc * CT + i, ntile - 1);
+          const float4 sn = *reinterpret_cast<const float4*>(e.wscale + tile * 16 + cq * 4);
+          acc[i][b][0] *= a * sn.x; acc[i][b][1] *= a * sn.y; acc[i][b][2] *= a * sn.z; acc[i][b][3] *= a * sn.w;
+        }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < CT; ++i)
+#pragma unroll
+      for (int b = 0; b < RB; ++b) { tot[i][b] = tot[i][b] + acc[i][b]; acc[i][b] = f32x4(0.0f); }
+  };
+  if constexpr (KS == 1) {                                      // (an even number of chunks: K is a multiple of 128)
+    for (int ch = chb; ch < che; ch += 2) {
+      step(ch, 0, 0);
+      step(ch + 1, 0, 1);
+      if (((ch + 2) % CPC) == 0 || ch + 2 == che) chain_end(ch);
+    }
+  } else {
+    for (int ch = chb; ch < che; ++ch) {
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) step(ch, ks, ks & 1);
+      if (((ch + 1) % CPC) == 0 || ch + 1 == che) chain_end(ch);
+    }
   }
-#ifdef IXT_RING_STAMPS
-  if (lane == 0 && e.amax_val != nullptr) {   // the probe passes a buffer of its own here: [block][wave][4] cycle sums
-    unsigned long long* dbg = reinterpret_cast<unsigned long long*>(e.amax_val) + ((size_t)bx * NW + wave) * 4;
-    dbg[0] = sum_wait; dbg[1] = sum_bar; dbg[2] = sum_issue; dbg[3] = sum_comp;
-  }
-#endif
-#undef IXT_STAMP
-#undef IXT_RISSUE
 
   // ---------------------------------------------------------------- epilogues
   if constexpr (EPI == GEPI_F32) {

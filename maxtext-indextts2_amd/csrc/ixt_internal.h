@@ -95,13 +95,13 @@ struct ixt_ctx {
   int gemm_prefix_halves = 0;   // measured at 256 rows on the MLP up-projection: decode step 5.39 vs 4.84 ms: off
   int gemm_split_min_blocks = 300;   // 128 x 128 x one-chain blocks (at C2 / 256 rows: the QKV and MLP-down kernels; +2.4 % end to end)
   int unembed_gemm = 1;
-  // LDS-ring GEMM with fused epilogues (ixt_gemm.h) from this many rows; ring_cfg forces a tile (1: 128 x 128, 2: 128 x 64, 3: 64 x 32)
+  // LDS-ring GEMM with fused epilogues (ixt_gemm.h) from this many rows; ring_cfg forces a tile (ring_pick)
   int ring_min_rows = 128, ring_cfg = 0, ring_split = 0, ring_wlayout = 0;
   // MLP down-projection on the ring path: 1 = ring GEMM with the residual epilogue; 0 = split-K tiles (one f32 slice per 512-k chain, two blocks
   // per CU) + slice-sum / residual / norm kernel; -1 (default) = by shape: the ring form needs at least 192 whole-K blocks of 128 x 128 or 128 x 64
   int ring_down = -1;
-  int unembed_tall = 1;      // 256 x 128 tiles for the unembedding at 129..256 rows (0: 128 x 128)
-  int ring_two_per_cu = 1;   // ring GEMMs of >= 1024 rows: 32-k chunks in 4 slots (64 KiB of LDS), two blocks per CU
+  int unembed_tall = 1;      // 256 x 128 tiles for the unembedding (0: never)
+  int ring_two_per_cu = 1;   // 128 x 128 ring tiles with 32-k chunks in 4 slots (64 KiB of LDS), two blocks per CU (0: never)
   int attn_tile = 1;         // prefill rows: tiled attention (k_attn_tile) from attn_tile_min_rows rows on
   int attn_tile_min_rows = 64;
   int attn_wave_pairs = 0;   // measured at 256 rows, 765 keys: 339 us per launch (4.7 TB/s) against 305 us (5.3 TB/s) for the block form
