@@ -711,7 +711,7 @@ static int ring_pick(const ixt_ctx* c, int epi, int R, int N, bool routed, bool 
     long cost;
     if (t.two) {
       const long rest = per_xcd % 64;
-      cost = per_xcd / 64 * t.two + (rest == 0 ? 0 : rest <= 32 ? t.one : t.two);
+      cost = per_xcd / 64 * t.two + (rest == 0 ? 0 : rest > 32 ? t.two : per_xcd > 64 ? t.two - t.one : t.one);   // (a last, half round runs beside the end of the one before it)
     } else {
       cost = (per_xcd + 31) / 32 * t.one;
     }
@@ -984,10 +984,16 @@ int launch_dot(ixt_ctx* c, const bf16_t* x, const bf16_t* w, int K, int N, int R
 }
 
 
+// Rows from which a pass of the llama blocks and the unembedding run on the ring GEMM.  From 17 on (up to 16 the kernels of ixt_small.h serve): 64-row tiles of
+// 64, 32 or 16 columns stream the weights as fast as the split-K dots and their epilogues leave no slices to add up (attention has its q and keys ready
+// instead of adding QKV slices).  48 rows of the 1B model, one layer: QKV 11.3 -> 12.1 us and attention 47.1 -> 42.3, O and norm 11.9 -> 13.3,
+// MLP up and gate 23.8 -> 14.7; unembedding 267 -> 220.  A decode step 2.08 -> 1.83 ms; a prompt of 57 tokens 1.57 -> 1.35 ms.
+static int ring_model_rows(const ixt_ctx* c) { return c->ring_min_rows > 128 ? c->ring_min_rows : std::min(c->ring_min_rows, c->ring_mid_rows); }
+
 // logits (optional store) + greedy argmax for R rows of normed hidden states
 static int launch_unembed(ixt_ctx* c, const bf16_t* yT, int R, float* logits_out, int32_t* argmax_out, hipStream_t st) {
   const int K = c->E, N = c->V;
-  if (R >= c->ring_min_rows && c->unembed_gemm) {   // many rows: the LDS-ring GEMM with the sampling epilogue
+  if (R >= ring_model_rows(c) && c->unembed_gemm) {   // the LDS-ring GEMM with the sampling epilogue
     if ((size_t)R * ((N / 16 + 1) / 2) > c->amax_cap) return set_err(IXT_ERR_INVALID, "argmax workspace too small");   // one pair per row and wave column (>= 2 tiles)
     GemmEpi e{};
     e.out = logits_out; e.amax_val = c->amax_val; e.amax_idx = c->amax_idx; e.cr = c->sample_cols;
@@ -1472,7 +1478,7 @@ static int forward_rows_gemma2(ixt_ctx* c, int R, const int32_t* tokens, int len
 // decode: one new token per row (rows never read each other's new K).
 //
 // Two launch sequences per layer, same arithmetic:
-//   R >= ring_min_rows  LDS-ring GEMMs with fused epilogues (ixt_gemm.h): QKV (+ RoPE, q -> qbuf, K/V -> pages), attention from qbuf
+//   R >= 17 (ring_model_rows)  LDS-ring GEMMs with fused epilogues (ixt_gemm.h): QKV (+ RoPE, q -> qbuf, K/V -> pages), attention from qbuf
 //                       and the pages, O-proj (+ residual), norm, MLP-up (+ SwiGLU), MLP-down (+ residual), norm: 7 launches, no f32
 //                       slice leaves the chip;
 //   fewer rows          split-K dots into f32 slices: dot_qkv, [front | qkv_finalize + scores], pv, combine, dot_o, rownorm (slice sum
@@ -1675,7 +1681,7 @@ static int forward_rows(ixt_ctx* c, int R, const int32_t* tokens, int len_hint, 
   bf16_t* hcur = c->h_a;
   bf16_t* hnext = c->h_b;
   const bool final_fused = nl == R && lrow0 == 0 && lrows == nullptr;   // decode: every row is unembedded
-  const bool ring = R >= c->ring_min_rows && !c->moe && !c->fp8;   // fp8: the dots write scaled f32 slices, the bf16 path's row kernels take it from there   // Mixtral: the split-K dots (every expert is a launch sequence of its own)
+  const bool ring = R >= ring_model_rows(c) && !c->moe && !c->fp8;   // fp8: the dots write scaled f32 slices, the bf16 path's row kernels take it from there   // Mixtral: the split-K dots (every expert is a launch sequence of its own)
   const int fused_min = c->attn_fused_min_blocks;
   const size_t fused_lds = sizeof(float) * ((size_t)c->GQ * c->D + 2 * c->D + (size_t)c->GQ * (c->geom.Tmax + 3) + c->geom.mpg + 12 + (size_t)c->geom.nsb_max * c->D);
   const bool attn_one_launch = R * c->KV >= fused_min && fused_lds <= 64 * 1024;
@@ -2182,7 +2188,7 @@ extern "C" int ixt_set_option(ixt_ctx* c, const char* name, int value) {
       {"attn_fused_min_blocks", &c->attn_fused_min_blocks, 1}, {"gemm_prefix_halves", &c->gemm_prefix_halves, 0},
       {"gemm_split_min_blocks", &c->gemm_split_min_blocks, 1}, {"gemm_min_blocks", &c->gemm_min_blocks, 1}, {"gemm_min_rows", &c->gemm_min_rows, 1},
       {"unembed_gemm", &c->unembed_gemm, 0}, {"attn_wave_pairs", &c->attn_wave_pairs, 0}, {"attn_tile", &c->attn_tile, 0}, {"attn_tile_min_rows", &c->attn_tile_min_rows, 1}, {"dot_stream_min_blocks", &c->dot_stream_min_blocks, 1},
-      {"ring_min_rows", &c->ring_min_rows, 1}, {"ring_cfg", &c->ring_cfg, 0}, {"ring_split", &c->ring_split, 0}, {"ring_wlayout", &c->ring_wlayout, 0}, {"ring_down", &c->ring_down, -1}, {"unembed_tall", &c->unembed_tall, 0}, {"ring_two_per_cu", &c->ring_two_per_cu, 0},
+      {"ring_min_rows", &c->ring_min_rows, 1}, {"ring_mid_rows", &c->ring_mid_rows, 17}, {"ring_cfg", &c->ring_cfg, 0}, {"ring_split", &c->ring_split, 0}, {"ring_wlayout", &c->ring_wlayout, 0}, {"ring_down", &c->ring_down, -1}, {"unembed_tall", &c->unembed_tall, 0}, {"ring_two_per_cu", &c->ring_two_per_cu, 0},
       {"small_rows", &c->small_rows, 0}, {"small_tpb", &c->small_tpb, 0}, {"small_attn_waves", &c->small_attn_waves, 4}, {"small_attn_max_blocks", &c->small_attn_max_blocks, 0}, {"dot_small", &c->dot_small, 0}, {"small_norm", &c->small_norm, 0}, {"small_prefetch", &c->small_prefetch, 0}, {"small_prefetch_blocks", &c->small_prefetch_blocks, 1}, {"moe_grouped", &c->moe_grouped, 0}, {"small_attn_split", &c->small_attn_split, 0}, {"moe_route_blocks", &c->moe_route_blocks, 0}, {"gemma_tile", &c->gemma_tile, 0}, {"moe_fused_gate", &c->moe_fused_gate, 0}, {"moe_mid_pairs", &c->moe_mid_pairs, 0},
   };
   for (const Opt& o : opts) {

@@ -96,7 +96,7 @@ struct ixt_ctx {
   int gemm_split_min_blocks = 300;   // 128 x 128 x one-chain blocks (at C2 / 256 rows: the QKV and MLP-down kernels; +2.4 % end to end)
   int unembed_gemm = 1;
   // LDS-ring GEMM with fused epilogues (ixt_gemm.h) from this many rows; ring_cfg forces a tile (ring_pick)
-  int ring_min_rows = 128, ring_cfg = 0, ring_split = 0, ring_wlayout = 0;
+  int ring_min_rows = 128, ring_mid_rows = 17, ring_cfg = 0, ring_split = 0, ring_wlayout = 0;
   // MLP down-projection on the ring path: 1 = ring GEMM with the residual epilogue; 0 = split-K tiles (one f32 slice per 512-k chain, two blocks
   // per CU) + slice-sum / residual / norm kernel; -1 (default) = by shape: the ring form needs at least 192 whole-K blocks of 128 x 128 or 128 x 64
   int ring_down = -1;

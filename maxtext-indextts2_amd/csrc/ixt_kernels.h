@@ -569,27 +569,37 @@ static __global__ void k_transpose_x(const bf16_t* x, bf16_t* xT, int R, int K) 
 }
 
 // final (max, first index) over the per-tile pairs.  grid = R, block 256.
-static __global__ __launch_bounds__(256) void k_argmax_final(const float* amax_val, const int32_t* amax_idx, int ntiles, int32_t* out_idx) {
-  __shared__ float bv[256];
-  __shared__ int bi[256];
+static __global__ __launch_bounds__(256) void k_argmax_final(const float* __restrict__ amax_val, const int32_t* __restrict__ amax_idx, int ntiles, int32_t* out_idx) {
+  __shared__ float bv[4];
+  __shared__ int bi[4];
   const int r = blockIdx.x, tid = threadIdx.x;
+  const float* pv = amax_val + (size_t)r * ntiles;
+  const int32_t* pi = amax_idx + (size_t)r * ntiles;
   float best = -INFINITY;
   int bidx = 0x7fffffff;
-  for (int t = tid; t < ntiles; t += 256) {
-    const float v = amax_val[(size_t)r * ntiles + t];
-    const int i2 = amax_idx[(size_t)r * ntiles + t];
-    if (v > best || (v == best && i2 < bidx)) { best = v; bidx = i2; }
+  auto take = [&](float v, int i2) { if (v > best || (v == best && i2 < bidx)) { best = v; bidx = i2; } };
+  int t = tid;
+  for (; t + 7 * 256 < ntiles; t += 8 * 256) {   // eight pairs in flight: one at a time is a memory latency each (8256 pairs: 17 us -> 7)
+    float v[8];
+    int i2[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) { v[j] = pv[t + j * 256]; i2[j] = pi[t + j * 256]; }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) take(v[j], i2[j]);
   }
-  bv[tid] = best; bi[tid] = bidx;
+  for (; t < ntiles; t += 256) take(pv[t], pi[t]);
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    const float v = __shfl_xor(best, off, 64);
+    const int i2 = __shfl_xor(bidx, off, 64);
+    take(v, i2);
+  }
+  if ((tid & 63) == 0) { bv[tid >> 6] = best; bi[tid >> 6] = bidx; }
   __syncthreads();
-  for (int s2 = 128; s2 > 0; s2 >>= 1) {
-    if (tid < s2) {
-      const float v = bv[tid + s2]; const int i2 = bi[tid + s2];
-      if (v > bv[tid] || (v == bv[tid] && i2 < bi[tid])) { bv[tid] = v; bi[tid] = i2; }
-    }
-    __syncthreads();
+  if (tid == 0) {
+    for (int w = 1; w < 4; ++w) take(bv[w], bi[w]);
+    out_idx[r] = bidx == 0x7fffffff ? 0 : bidx;
   }
-  if (tid == 0) out_idx[r] = bi[0] == 0x7fffffff ? 0 : bi[0];
 }
 
 // h_out = bf16(h_in + bf16(sum of slices))  (llama2.py:127, :157).  grid = (ceil(E/256), R), block 128, 2 columns per thread.

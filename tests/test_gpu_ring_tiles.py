@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 
 import helpers as H
-from test_gpu_ops import _dot_case, ctx  # noqa: F401  (fixture)
+from test_gpu_ops import _dot_case, _st, _vp, ctx  # noqa: F401  (fixture)
 
 pytestmark = pytest.mark.gpu
 
@@ -26,3 +26,23 @@ def test_forced_tile(ctx, cfg_id, R, K, N):
 def test_chosen_tile(ctx, R, K, N):
   rng = np.random.default_rng(R + K + N)
   _dot_case(ctx, H.rand_bf16(rng, (R, K)), H.rand_bf16(rng, (K, N), 0.05))
+
+
+@pytest.mark.parametrize("R", [17, 48, 64, 65, 127])
+def test_unembedding_of_some_rows(ctx, R):
+  """17 .. 127 rows: the sampling epilogue on 64-row tiles (rounded logits and the first index of the maximum), a vocabulary that is no multiple of a tile."""
+  torch, O = ctx["torch"], ctx["O"]
+  cfg = H.make_config(per_device_batch_size=float(R), pagedattn_num_pages=256, vocab_size=4112)
+  w = H.synth.synth_weights(cfg, 3)
+  eng, _ = H.make_engine(cfg, w)
+  E, V = cfg.emb_dim, cfg.vocab_size
+  y = H.rand_bf16(np.random.default_rng(R), (R, E))
+  lg = np.zeros((R, V), np.float32)
+  wl = w["params/decoder/logits_dense/kernel"].reshape(E, V)
+  O.lib().orc_dot_rows(O._p(y, O._u16p), E, R, O._p(wl, O._u16p), E, V, O._p(lg, O._f32p), V)
+  lg = O.bf16_to_f32(O.f32_to_bf16(lg)).reshape(R, V)
+  logits = torch.empty((R, V), dtype=torch.float32, device="cuda")
+  amax = torch.empty((R,), dtype=torch.int32, device="cuda")
+  H.lib.check(eng.lib.ixt_op_unembed_argmax(eng._ctx, _vp(H.dev_bf16(y)), R, _vp(logits), _vp(amax), _st(torch)))
+  assert np.array_equal(logits.cpu().numpy().view(np.uint32), lg.view(np.uint32))
+  assert np.array_equal(amax.cpu().numpy(), np.argmax(lg, axis=-1).astype(np.int32))
