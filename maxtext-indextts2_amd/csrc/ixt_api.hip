@@ -1135,7 +1135,7 @@ static void launch_scores_pv(ixt_ctx* c, int layer, int R, int len_hint, hipStre
 }
 
 template <int HD, int GQ>
-static void launch_decode_attn(ixt_ctx* c, int layer, int R, const DotResult& dr, bool newtok, hipStream_t st) {
+static void launch_decode_attn(ixt_ctx* c, int layer, int R, const DotResult& dr, bool newtok, bool decode, hipStream_t st) {
   const AttnGeom& g = c->geom;
   DecAttnArgs da;
   da.part = c->part; da.slices = dr.slices; da.slice_stride = dr.slice_stride; da.ncols = c->NQKV;
@@ -1150,8 +1150,9 @@ static void launch_decode_attn(ixt_ctx* c, int layer, int R, const DotResult& dr
     return;
   }
   const size_t lds = sizeof(float) * ((size_t)GQ * HD + 2 * HD + (size_t)GQ * ((g.Tmax + 3) & ~3) + ((g.mpg + 3) & ~3) + 8 + (size_t)g.nsb_max * HD);
-  if (newtok) hipLaunchKernelGGL((k_attn_decode<HD, GQ, true>), dim3(g.nkv, R), dim3(256), lds, st, da);
-  else hipLaunchKernelGGL((k_attn_decode<HD, GQ, false>), dim3(g.nkv, R), dim3(256), lds, st, da);
+  if (newtok) hipLaunchKernelGGL((k_attn_decode<HD, GQ, true, true>), dim3(g.nkv, R), dim3(256), lds, st, da);
+  else if (decode) hipLaunchKernelGGL((k_attn_decode<HD, GQ, false, true>), dim3(g.nkv, R), dim3(256), lds, st, da);
+  else hipLaunchKernelGGL((k_attn_decode<HD, GQ, false, false>), dim3(g.nkv, R), dim3(256), lds, st, da);
 }
 
 // prefill rows (q in qbuf, K/V already in the pages): NQ query vectors per block share every K / V load.  false: the score rows of
@@ -1199,10 +1200,10 @@ static int launch_attention_tile(ixt_ctx* c, int layer, int R, int len_hint, hip
 }
 
 // decode rows, enough (row, kv head) pairs to fill the chip: the whole attention in one launch (writes c->ao)
-static int launch_attention_fused(ixt_ctx* c, int layer, int R, const DotResult& qkv, bool newtok, hipStream_t st) {
+static int launch_attention_fused(ixt_ctx* c, int layer, int R, const DotResult& qkv, bool newtok, bool decode, hipStream_t st) {
 #define ATT(HD_, GQ_)                                                                             \
   if (c->D == HD_ && c->GQ == GQ_) {                                                              \
-    launch_decode_attn<HD_, GQ_>(c, layer, R, qkv, newtok, st);                                   \
+    launch_decode_attn<HD_, GQ_>(c, layer, R, qkv, newtok, decode, st);                                   \
     LAUNCHCHK();                                                                                  \
     return IXT_OK;                                                                                \
   }
@@ -1629,7 +1630,7 @@ static int forward_rows_small(ixt_ctx* c, int R, const int32_t* tokens, int len_
       } else if (attn_small) {
         TRY(launch_attn_small(c, l, R, st, w.wi, (size_t)E * 2 * F));                                             // while the attention runs: the wi kernel
       } else if (fused_lds <= 64 * 1024) {
-        TRY(launch_attention_fused(c, l, R, DotResult{0, 0, 0}, false, st));
+        TRY(launch_attention_fused(c, l, R, DotResult{0, 0, 0}, false, decode, st));
       } else {
         TRY(launch_attention_partials(c, l, R, len_hint, DotResult{0, 0, 0}, false, st));
         hipLaunchKernelGGL(k_attn_combine, dim3(R), dim3(256), 0, st, c->pvpart, c->row_pos, c->row_active, c->ao, c->geom, 1);
@@ -1701,7 +1702,7 @@ static int forward_rows(ixt_ctx* c, int R, const int32_t* tokens, int len_hint, 
         const DotResult none{0, 0, 0};
         const int ta = decode ? timing_begin(c, st, 0.0, 1) : -1;
         if (decode && attn_small_fits(c, R)) TRY(launch_attn_small(c, l, R, st));   // (small_attn_max_blocks raised: the 8-wave form with everything in flight)
-        else TRY(launch_attention_fused(c, l, R, none, false, st));   // q from qbuf, every key / value (the new ones too) from the pages
+        else TRY(launch_attention_fused(c, l, R, none, false, decode, st));   // q from qbuf, every key / value (the new ones too) from the pages
         timing_end(c, st, ta);
       } else {
         TRY(launch_attention_partials(c, l, R, len_hint, DotResult{0, 0, 0}, false, st));
@@ -1756,7 +1757,7 @@ static int forward_rows(ixt_ctx* c, int R, const int32_t* tokens, int len_hint, 
       timing_end(c, st, ta);
     } else if (attn_one_launch) {   // decode rows, and prefill rows after k_qkv_finalize
       const int ta = decode ? timing_begin(c, st, 0.0, 1) : -1;   // K/V bytes depend on the rows' lengths: the caller prices them
-      TRY(launch_attention_fused(c, l, R, dr, decode, st));
+      TRY(launch_attention_fused(c, l, R, dr, decode, decode, st));
       timing_end(c, st, ta);
     } else {
       TRY(launch_attention_partials(c, l, R, len_hint, dr, decode, st));
