@@ -720,22 +720,30 @@ static int ring_pick(const ixt_ctx* c, int epi, int R, int N, bool routed, bool 
   return best;
 }
 
-template <int WR, int WC, int RB, int CT, int KS, int NS, int EPI, int SPLIT>
-static int ring_launch_t(const bf16_t* x, const bf16_t* w, int K, int N, int R, int chains, int wring, const GemmEpi& e, hipStream_t st, int* wave_cols) {
+template <int WR, int WC, int RB, int CT, int KS, int NS, int EPI, int SPLIT, bool ONCE>
+static int ring_launch_o(const bf16_t* x, const bf16_t* w, int K, int N, int R, int chains, int wring, const GemmEpi& e, hipStream_t st, int* wave_cols) {
   constexpr int TC = WC * CT, TR = WR * RB;
   const int ncolg = (N / 16 + TC - 1) / TC, zb = (R + 16 * TR - 1) / (16 * TR);
   constexpr size_t lds = (size_t)NS * (TC + TR) * KS * 1024;
   static bool attr_done = false;
   if (!attr_done) {   // more than 64 KiB of dynamic LDS needs the attribute once per kernel
-    HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gemm_ring<WR, WC, RB, CT, KS, NS, EPI, SPLIT>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gemm_ring<WR, WC, RB, CT, KS, NS, EPI, SPLIT, false, ONCE>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     attr_done = true;
   }
   dim3 grid(((ncolg + 7) / 8) * 8 * zb, SPLIT ? chains : 1, 1);
-  hipLaunchKernelGGL((k_gemm_ring<WR, WC, RB, CT, KS, NS, EPI, SPLIT>), grid, dim3(WR * WC * 64), lds, st, reinterpret_cast<const u32x4*>(x),
+  hipLaunchKernelGGL((k_gemm_ring<WR, WC, RB, CT, KS, NS, EPI, SPLIT, false, ONCE>), grid, dim3(WR * WC * 64), lds, st, reinterpret_cast<const u32x4*>(x),
                      reinterpret_cast<const u32x4*>(w), K, N, R, ncolg, zb, wring, e);
   LAUNCHCHK();
   if (wave_cols) *wave_cols = WC * ncolg;
   return IXT_OK;
+}
+// the widest kernels (gated units, unembedding) with all rows in one row group: weights streamed past the caches
+template <int WR, int WC, int RB, int CT, int KS, int NS, int EPI, int SPLIT>
+static int ring_launch_t(const bf16_t* x, const bf16_t* w, int K, int N, int R, int chains, int wring, const GemmEpi& e, hipStream_t st, int* wave_cols) {
+  if constexpr (EPI == GEPI_SWIGLU || EPI == GEPI_UNEMBED) {
+    if (R <= 16 * WR * RB) return ring_launch_o<WR, WC, RB, CT, KS, NS, EPI, SPLIT, true>(x, w, K, N, R, chains, wring, e, st, wave_cols);
+  }
+  return ring_launch_o<WR, WC, RB, CT, KS, NS, EPI, SPLIT, false>(x, w, K, N, R, chains, wring, e, st, wave_cols);
 }
 
 // x in xidx layout, w in widx layout (wring: ring layout); the epilogue's operands in `e`.  split (GEPI_F32 only): one f32 slice per

@@ -112,7 +112,7 @@ __device__ __forceinline__ void ring_wait_chunks(int younger) {
 //   Row groups of one column group are block ids b, b + 8, ..: same XCD, the weights meet in its L2.
 //   F8 (ixt_fp8.h): both operands are e4m3 fragments of 64 k (still 1 KiB: the ring moves them exactly as bf16 fragments of 32 k); a fragment
 //   feeds two v_mfma_f32_16x16x32_fp8_fp8; at the end of every 512-k chain the accumulator is scaled by (a_rc s_n) before it joins the total.
-template <int WR, int WC, int RB, int CT, int KS, int NS, int EPI, int SPLIT, bool F8 = false>
+template <int WR, int WC, int RB, int CT, int KS, int NS, int EPI, int SPLIT, bool F8 = false, bool ONCE = false>
 __global__ __launch_bounds__(WR * WC * 64, 2) void k_gemm_ring(const u32x4* __restrict__ xt, const u32x4* __restrict__ wt, int K, int N, int R,
                                                                int ncolg, int zb, int wring, GemmEpi e) {
   constexpr int NW = WR * WC;          // waves
@@ -162,15 +162,15 @@ __global__ __launch_bounds__(WR * WC * 64, 2) void k_gemm_ring(const u32x4* __re
   const char* px = reinterpret_cast<const char*>(xt + (size_t)rowg * TR * nsteps * 64) + (size_t)chb * KS * 1024;
   const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)((__attribute__((address_space(3))) u32x4*)st));
   // piece j of the next chunk to fetch, into a slot.  Issued by hand (no register is written, nothing else in this kernel uses m0): behind the builtin the
-  // compiler may wait for every fetch in flight before an LDS read; the waits are counted in the loop.
+  // compiler may wait for every fetch in flight before an LDS read; the waits are counted in the loop.  ONCE (one row group): no other block reads these
+  // weights, so they are streamed past the caches (264192 columns, K 2048: 48 rows 219 -> 203 us, 256 rows 386 -> 359; several row groups of small tiles lose
+  // by it, and a branch here instead of a second kernel costs them up to 10 %).
   auto issue = [&](int slot, int j) {
     const uint32_t dst = lds0 + (uint32_t)(slot * NF + wave + NW * j) * 1024u;
-    if (NW * j + NW <= NWF) asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(off[j]), "s"(pw) : "memory");
-    else if (NW * j >= NWF) asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(off[j]), "s"(px) : "memory");
-    else {
-      const uint64_t p = wave + NW * j < NWF ? (uint64_t)(uintptr_t)pw : (uint64_t)(uintptr_t)px;
-      asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(off[j]), "s"(p) : "memory");
-    }
+    if (NW * j >= NWF || (NW * j + NW > NWF && wave + NW * j >= NWF))
+      asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(off[j]), "s"(px) : "memory");
+    else if constexpr (ONCE) asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(dst), "v"(off[j]), "s"(pw) : "memory");
+    else asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(off[j]), "s"(pw) : "memory");
   };
   auto advance = [&]() { pw += wadv; px += (size_t)KS * 1024; };
 #pragma unroll
