@@ -51,6 +51,10 @@ struct ixt_trainer {
   bf16_t* pb = nullptr;   // bf16 copies of the parameters (owned here)
   // offsets
   long o_emb, o_fnorm, o_logits;
+  // Rows of the vocabulary (bf16 copy of the logits kernel, the last parameter; logits and their gradients) lie Vp apart: V + 64.  Where 2 V bytes is an odd
+  // multiple of some power of two (264192: 129 x 2^12), the 256 rows a tile fetches side by side lie in few memory channels, and the product whose reduction
+  // runs along them took 3.30 ms a chunk of 2048 rows (0.67 PFLOP/s); 128 bytes more a row: 1.72 (1.29; only one of the two operands: 2.9)
+  long Vp;
   struct LOff { long ln1, wq, wk, wv, wo, ln2, wi0, wi1, wout; };
   std::vector<LOff> lo;
   std::vector<LayerAct> act;
@@ -93,6 +97,7 @@ extern "C" int ixt_train_create(const ixt_train_config* c, ixt_trainer** out) {
   t->KVH = c->num_kv_heads; t->G = t->H / t->KVH; t->KN = t->KVH * t->D;
   t->Tc = c->logits_chunk > 0 ? c->logits_chunk : 2048;
   if (t->Tc > t->T) t->Tc = t->T;
+  t->Vp = t->V >= 4096 ? t->V + 64 : t->V;
   const long E = t->E, F = t->F, V = t->V, QN = t->QN, KN = t->KN;
   add_param(t, "params/token_embedder/embedding", V * E, &t->o_emb);
   t->lo.resize(t->L);
@@ -115,7 +120,7 @@ extern "C" int ixt_train_create(const ixt_train_config* c, ixt_trainer** out) {
   auto fail = [&](int code) { ixt_train_destroy(t); return code; };
 #define A(expr) do { rc = (expr); if (rc != IXT_OK) return fail(rc); } while (0)
   const size_t T = t->T, S = t->S, BH = (size_t)t->B * t->H;
-  A(tmalloc(t, &t->pb, (size_t)t->total));
+  A(tmalloc(t, &t->pb, (size_t)t->total + (size_t)E * (t->Vp - V)));
   t->act.resize(t->L);
   for (int i = 0; i < t->L; ++i) {
     LayerAct& a = t->act[i];
@@ -125,7 +130,7 @@ extern "C" int ixt_train_create(const ixt_train_config* c, ixt_trainer** out) {
   }
   A(tmalloc(t, &t->h_final, T * E)); A(tmalloc(t, &t->xn_f, T * E)); A(tmalloc(t, &t->r_f, T));
   A(tmalloc(t, &t->scores, BH * S * S)); A(tmalloc(t, &t->dh, T * E)); A(tmalloc(t, &t->dxn, T * E));
-  A(tmalloc(t, &t->logits, (size_t)t->Tc * V)); A(tmalloc(t, &t->dlog, (size_t)t->Tc * V)); A(tmalloc(t, &t->row_loss, T)); A(tmalloc(t, &t->scal, (size_t)16));
+  A(tmalloc(t, &t->logits, (size_t)t->Tc * V)); A(tmalloc(t, &t->dlog, (size_t)t->Tc * t->Vp)); A(tmalloc(t, &t->row_loss, T)); A(tmalloc(t, &t->scal, (size_t)16));
   A(tmalloc(t, &t->part, (size_t)4096));
   A(tmalloc(t, &t->dS, BH * S * S)); A(tmalloc(t, &t->d_ao, T * QN)); A(tmalloc(t, &t->dq, T * QN)); A(tmalloc(t, &t->dk, T * KN));
   A(tmalloc(t, &t->dv, T * KN));
@@ -178,7 +183,8 @@ extern "C" int ixt_train_bind(ixt_trainer* t, float* params, float* grads, float
 }
 extern "C" int ixt_train_refresh_bf16(ixt_trainer* t, void* stream) {
   if (!t || !t->p) return t_set_err(IXT_ERR_INVALID, "bind the parameter buffers first");
-  hipLaunchKernelGGL(k_t_cast_bf16, dim3((unsigned)((t->total / 4 + 255) / 256)), dim3(256), 0, (hipStream_t)stream, t->p, t->pb, t->total);
+  hipLaunchKernelGGL(k_t_cast_bf16, dim3((unsigned)((t->o_logits / 4 + 255) / 256)), dim3(256), 0, (hipStream_t)stream, t->p, t->pb, t->o_logits, 0L);
+  hipLaunchKernelGGL(k_t_cast_bf16, dim3((unsigned)((t->V / 4 + 255) / 256), t->E), dim3(256), 0, (hipStream_t)stream, t->p + t->o_logits, t->pb + t->o_logits, (long)t->V, t->Vp);
   TLAUNCH();
   return IXT_OK;
 }
@@ -236,7 +242,8 @@ static void softmax_bwd(hipStream_t st, const float* dP, const bf16_t* P, bf16_t
   else if (S <= 4096) hipLaunchKernelGGL(k_t_softmax_bwd_reg<16>, grid, dim3(256), 0, st, dP, P, dS, S);
   else hipLaunchKernelGGL(k_t_softmax_bwd, grid, dim3(256), 0, st, dP, P, dS, S);
 }
-struct TOperand { const bf16_t* x; const bf16_t* w; void* c; int n; };   // TL_DX: n is the reduction (the layer's outputs), c of the first entry the result
+// TL_DX: n is the reduction (the layer's outputs), c of the first entry the result; ldw: where the rows of w (TL_XW: and of c) lie further apart than n
+struct TOperand { const bf16_t* x; const bf16_t* w; void* c; int n; long ldw = 0; };
 // M: rows (tokens; TL_DW: the layer's inputs); K: reduction (TL_DX: the entries' n); scratch: for reductions cut in parts, or nullptr
 static int gemm(hipStream_t st, int what, int M, int K, std::initializer_list<TOperand> ops, int out, long ld_x, int N_dx = 0, const bf16_t* res = nullptr, float* scratch = nullptr,
                 size_t scratch_floats = 0) {
@@ -245,9 +252,10 @@ static int gemm(hipStream_t st, int what, int M, int K, std::initializer_list<TO
   int i = 0;
   for (const TOperand& o : ops) {
     g.A[i] = o.x; g.B[i] = o.w; g.C[i] = o.c;
-    if (what == TL_XW) { g.lda[i] = ld_x; g.ldb[i] = o.n; g.ldc[i] = o.n; g.N[i] = o.n; g.K[i] = K; }
-    else if (what == TL_DX) { g.lda[i] = o.n; g.ldb[i] = o.n; g.ldc[i] = N_dx; g.N[i] = N_dx; g.K[i] = o.n; }
-    else { g.lda[i] = ld_x; g.ldb[i] = o.n; g.ldc[i] = o.n; g.N[i] = o.n; g.K[i] = K; }
+    const long ldw = o.ldw ? o.ldw : o.n;
+    if (what == TL_XW) { g.lda[i] = ld_x; g.ldb[i] = g.ldc[i] = ldw; g.N[i] = o.n; g.K[i] = K; }
+    else if (what == TL_DX) { g.lda[i] = ld_x; g.ldb[i] = ldw; g.ldc[i] = N_dx; g.N[i] = N_dx; g.K[i] = o.n; }
+    else { g.lda[i] = ld_x; g.ldb[i] = ldw; g.ldc[i] = o.n; g.N[i] = o.n; g.K[i] = K; }
     ++i;
   }
   g.nprob = i;
@@ -352,11 +360,11 @@ extern "C" int ixt_train_forward_backward(ixt_trainer* t, const int32_t* inputs,
   for (int t0 = 0; t0 < T; t0 += t->Tc) {
     const int n = T - t0 < t->Tc ? T - t0 : t->Tc;
     const bf16_t* xn = t->xn_f + (long)t0 * E;
-    TTRY(gemm(st, TL_XW, n, E, {{xn, pb + t->o_logits, t->logits, V}}, TG_BF16, E));
-    hipLaunchKernelGGL(k_t_xent, dim3(n), dim3(256), 0, st, reinterpret_cast<const bf16_t*>(t->logits), targets + t0, targets_segmentation + t0, t->dlog, t->row_loss + t0, V);
+    TTRY(gemm(st, TL_XW, n, E, {{xn, pb + t->o_logits, t->logits, V, t->Vp}}, TG_BF16, E));
+    hipLaunchKernelGGL(k_t_xent, dim3(n), dim3(256), 0, st, reinterpret_cast<const bf16_t*>(t->logits), targets + t0, targets_segmentation + t0, t->dlog, t->row_loss + t0, V, t->Vp);
     // d xn_f = dlogits . W^T ; dW += xn_f^T . dlogits
-    TTRY(gemm(st, TL_DX, n, V, {{t->dlog, pb + t->o_logits, t->dxn + (long)t0 * E, V}}, TG_F32, V, E, nullptr, t->scores, V >= 65536 ? (size_t)B * H * S * S : 0));   // (the score buffer is idle)
-    TTRY(gemm(st, TL_DW, E, n, {{xn, t->dlog, t->g + t->o_logits, V}}, t0 == 0 ? TG_F32 : TG_F32_ADD, E));
+    TTRY(gemm(st, TL_DX, n, V, {{t->dlog, pb + t->o_logits, t->dxn + (long)t0 * E, V, t->Vp}}, TG_F32, t->Vp, E, nullptr, t->scores, V >= 65536 ? (size_t)B * H * S * S : 0));   // (the score buffer is idle)
+    TTRY(gemm(st, TL_DW, E, n, {{xn, t->dlog, t->g + t->o_logits, V, t->Vp}}, t0 == 0 ? TG_F32 : TG_F32_ADD, E));
   }
   hipLaunchKernelGGL(k_t_reduce, dim3(1), dim3(256), 0, st, t->row_loss, (long)T, 0, loss_and_weights_dev, 0);
   // total_weights = number of target positions with a non-zero segment id (train.py:309)
@@ -432,7 +440,9 @@ extern "C" int ixt_train_apply(ixt_trainer* t, float total_weights, float clip_t
   a.lr = lr; a.b1 = b1; a.b2 = b2; a.eps = eps; a.eps_root = eps_root; a.wd = weight_decay;
   a.bc1 = 1.0f - powf(b1, (float)count);
   a.bc2 = 1.0f - powf(b2, (float)count);
-  hipLaunchKernelGGL(k_t_adamw, EW(t->total), t->p, t->g, t->mu, t->nu, t->pb, t->scal + 1, t->total, a);
+  const long ol = t->o_logits;
+  hipLaunchKernelGGL(k_t_adamw, EW(ol), t->p, t->g, t->mu, t->nu, t->pb, t->scal + 1, ol, 0L, a);
+  hipLaunchKernelGGL(k_t_adamw, dim3((unsigned)((t->V + 255) / 256), t->E), dim3(256), 0, st, t->p + ol, t->g + ol, t->mu + ol, t->nu + ol, t->pb + ol, t->scal + 1, (long)t->V, t->Vp, a);
   TLAUNCH();
   return IXT_OK;
 }

@@ -34,11 +34,12 @@ static __global__ void k_t_zero(float* __restrict__ at, long n, float* __restric
   const long i = (((long)blockIdx.x - nb) * 256 + threadIdx.x) * 4, l = i / (2 * run), e = i - l * 2 * run;
   if (l < count) *reinterpret_cast<float4*>((e < run ? a + e : b + e - run) + l * stride) = z;
 }
-static __global__ void k_t_cast_bf16(const float* __restrict__ src, bf16_t* __restrict__ dst, long n) {   // n a multiple of 64 (the parameters' layout)
+// rows of n (a multiple of 4), ld apart in dst.  grid.y = rows
+static __global__ void k_t_cast_bf16(const float* __restrict__ src, bf16_t* __restrict__ dst, long n, long ld) {
   const long i = ((long)blockIdx.x * blockDim.x + threadIdx.x) * 4;
   if (i >= n) return;
-  const float4 v = *reinterpret_cast<const float4*>(src + i);
-  *reinterpret_cast<uint2*>(dst + i) = make_uint2(pack2(f2bf(v.x), f2bf(v.y)), pack2(f2bf(v.z), f2bf(v.w)));
+  const float4 v = *reinterpret_cast<const float4*>(src + blockIdx.y * n + i);
+  *reinterpret_cast<uint2*>(dst + blockIdx.y * ld + i) = make_uint2(pack2(f2bf(v.x), f2bf(v.y)), pack2(f2bf(v.z), f2bf(v.w)));
 }
 
 __device__ __forceinline__ float t_block_sum(float v, float* red) {   // 256 threads
@@ -333,12 +334,12 @@ static __global__ void k_t_embed_bwd(const float* __restrict__ dh, const int32_t
 // loss_row = log(sum exp(l - max)) + max - l[target]; dlogits = (softmax - onehot) * weight, bf16.  The row is read 2048 columns at a time, 16 bytes a
 // thread; the sum's terms reach the threads that own them (column mod 256) through LDS.  grid = Tc, block 256.
 static __global__ __launch_bounds__(256) void k_t_xent(const bf16_t* __restrict__ logits, const int32_t* __restrict__ targets, const int32_t* __restrict__ tseg,
-                                                bf16_t* __restrict__ dlogits, float* __restrict__ row_loss, int V) {
+                                                bf16_t* __restrict__ dlogits, float* __restrict__ row_loss, int V, long ld) {
   __shared__ float red[4];
   __shared__ __attribute__((aligned(16))) bf16_t tile[2][2048];
   const long row = blockIdx.x;
   const int tid = threadIdx.x;
-  const bf16_t* l = logits + row * V;
+  const bf16_t* l = logits + row * ld;
   float m = -INFINITY;
   for (int j = tid * 8; j < V; j += 2048) {
     float v[8];
@@ -373,7 +374,7 @@ static __global__ __launch_bounds__(256) void k_t_xent(const bf16_t* __restrict_
     t_unpack8(*reinterpret_cast<const u32x4*>(l + j), v);
 #pragma unroll
     for (int k = 0; k < 8; ++k) v[k] = ixt_exp(v[k] - m) * inv - (j + k == tg ? wt : 0.0f);
-    *reinterpret_cast<u32x4*>(dlogits + row * V + j) = t_pack8(v);
+    *reinterpret_cast<u32x4*>(dlogits + row * ld + j) = t_pack8(v);
   }
 }
 
@@ -414,9 +415,9 @@ static __global__ __launch_bounds__(256) void k_t_sumsq_partial(const float* __r
 // correction with `count` (1 at the first step), decoupled weight decay, p -= lr * update; the bf16 copy of the parameter is refreshed.
 struct AdamArgs { float lr, b1, b2, eps, eps_root, wd, bc1, bc2; };
 static __global__ void k_t_adamw(float* __restrict__ p, const float* __restrict__ g, float* __restrict__ mu, float* __restrict__ nu, bf16_t* __restrict__ pb,
-                          const float* __restrict__ gscale, long n, AdamArgs a) {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
+                          const float* __restrict__ gscale, long n, long ld, AdamArgs a) {
+  const long x = (long)blockIdx.x * blockDim.x + threadIdx.x, i = blockIdx.y * n + x;
+  if (x >= n) return;
   const float gv = g[i] * gscale[0];
   const float m = a.b1 * mu[i] + (1.0f - a.b1) * gv;
   const float v = a.b2 * nu[i] + (1.0f - a.b2) * gv * gv;
@@ -424,7 +425,7 @@ static __global__ void k_t_adamw(float* __restrict__ p, const float* __restrict_
   const float upd = (m / a.bc1) / (sqrtf(v / a.bc2 + a.eps_root) + a.eps) + a.wd * p[i];
   const float np_ = p[i] - a.lr * upd;
   p[i] = np_;
-  pb[i] = f2bf(np_);
+  pb[blockIdx.y * ld + x] = f2bf(np_);
 }
 // gscale[0] = (1 / denom) * min(1, clip / (norm / denom)) with norm = sqrt(sumsq[0]); norms_out = {raw grad norm, clipped grad norm}
 static __global__ void k_t_clip_scale(const float* __restrict__ sumsq, float denom, float clip, float* __restrict__ gscale, float* __restrict__ norms_out) {
