@@ -192,11 +192,11 @@ extern "C" int ixt_train_refresh_bf16(ixt_trainer* t, void* stream) {
 // ---------------------------------------------------------------------------------------------------------------- launches
 // The three products of a linear layer y = x W, W [K][N]: x W (W's columns contiguous), dy W^T (its k contiguous), x^T dy (both by columns).
 enum { TL_XW, TL_DX, TL_DW };
-template <bool TA, bool TB, int BM, int BN = BM>
+template <bool TA, bool TB, int BM, int BN = BM, bool FOLD = false>
 static int gemm_launch(hipStream_t st, TGemm& g) {
   // waves and their tiles: 256 x 256: 2 x 4 of 128 x 64; 256 x 128: 4 x 2 and 128 x 128: 2 x 2 of 64 x 64; 128 x 64: 4 of 32 x 64; 64 x 64: 2 x 2 of 32 x 32
   constexpr int WM = BN == BM ? 2 : 4, WN = BN == 256 ? 4 : BN == 64 && BM == 128 ? 1 : 2, MI = BM / 16 / WM, NI = BN / 16 / WN, NS = 4, lds = NS * (BM + BN) * 64;
-  const auto kernel = k_tgemm<TA, TB, MI, NI, WM, WN, NS>;
+  const auto kernel = k_tgemm<TA, TB, MI, NI, WM, WN, NS, FOLD>;
   static bool attr_done = false;
   if (!attr_done) {
     TCHK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds));
@@ -244,11 +244,13 @@ static void softmax_bwd(hipStream_t st, const float* dP, const bf16_t* P, bf16_t
 }
 // TL_DX: n is the reduction (the layer's outputs), c of the first entry the result; ldw: where the rows of w (TL_XW: and of c) lie further apart than n
 struct TOperand { const bf16_t* x; const bf16_t* w; void* c; int n; long ldw = 0; };
+// TL_DX of several entries: the sum of their products.
 // M: rows (tokens; TL_DW: the layer's inputs); K: reduction (TL_DX: the entries' n); scratch: for reductions cut in parts, or nullptr
 static int gemm(hipStream_t st, int what, int M, int K, std::initializer_list<TOperand> ops, int out, long ld_x, int N_dx = 0, const bf16_t* res = nullptr, float* scratch = nullptr,
                 size_t scratch_floats = 0) {
   TGemm g{};
   g.M = M; g.R = res; g.out = out; g.parts = 1;
+  const int sums = what == TL_DX ? (int)ops.size() : 1;
   int i = 0;
   for (const TOperand& o : ops) {
     g.A[i] = o.x; g.B[i] = o.w; g.C[i] = o.c;
@@ -258,7 +260,7 @@ static int gemm(hipStream_t st, int what, int M, int K, std::initializer_list<TO
     else { g.lda[i] = ld_x; g.ldb[i] = ldw; g.ldc[i] = o.n; g.N[i] = o.n; g.K[i] = K; }
     ++i;
   }
-  g.nprob = i;
+  g.nprob = sums > 1 ? 1 : i;
   auto tiles = [&](int b) {
     long t = 0;
     for (int k = 0; k < g.nprob; ++k) t += (g.N[k] + b - 1) / b;
@@ -279,6 +281,31 @@ static int gemm(hipStream_t st, int what, int M, int K, std::initializer_list<TO
       float* at = scratch;
       for (int k = 0; k < g.nprob; ++k) { g.C[k] = at; g.cpart[k] = (long)M * g.N[k]; at += 4 * g.cpart[k]; }
     }
+  }
+  // Sums, and cuts, inside the block (FOLD) where whole reductions give the chip enough tiles and the largest tile is not the one to take: 2048 x 768 outputs,
+  // three products with K 768 33 -> 29 us, two with K 2048 49 -> 47; the weight gradients of 768 x 2304 over 2048 tokens 33 -> 22.  Fewer tiles than CUs
+  // keep the parts (768 x 768: 14 us against 19).
+  bool fold = what != TL_XW && tiles(256) * g.parts < 192 && (sums > 1 || g.parts > 1) && (g.parts == 1 || tiles(64) >= 256);
+  for (const TOperand& o : ops) fold = fold && (sums == 1 || (o.n == g.K[0] && o.ldw == 0));
+  if (fold) {
+    g.nsum = sums;
+    if (g.parts > 1) {
+      g.fold = g.kpart / 32;
+      g.parts = 1;
+      int k = 0;
+      for (const TOperand& o : ops) g.C[k++] = o.c;
+    }
+    const bool b128 = tiles(128) >= 200;
+    if (what == TL_DX) return b128 ? gemm_launch<false, false, 128, 128, true>(st, g) : gemm_launch<false, false, 64, 64, true>(st, g);
+    return b128 ? gemm_launch<true, true, 128, 128, true>(st, g) : gemm_launch<true, true, 64, 64, true>(st, g);
+  }
+  if (sums > 1) {
+    int k = 0;
+    for (const TOperand& o : ops) {
+      const TOperand one{o.x, o.w, ops.begin()->c, o.n, o.ldw};
+      TTRY(gemm(st, what, M, o.n, {one}, k++ == 0 ? out : TG_F32_ADD, o.n, N_dx, res, scratch, scratch_floats));
+    }
+    return IXT_OK;
   }
   // 256 x 256 tiles wherever they occupy three quarters of the CUs; 128 x 128 down to 200 of those, 64 x 64 below.  Measured in us, 128 / 64:
   // 96 tiles of 128 x 128 with K 768 15.1 / 9.9, K 2048 29.2 / 18.9; 192 tiles, K 2048 32.2 / 24.6; 256 tiles, K 768 14.8 / 17.7; 512 tiles 22.6 / 28.9.
@@ -383,8 +410,7 @@ extern "C" int ixt_train_forward_backward(ixt_trainer* t, const int32_t* inputs,
     TTRY(gemm(st, TL_DX, T, E, {{t->dy_bf, pb + o.wout, t->dact, E}}, TG_BF16, E, F));                   // d act = dy . Wout^T
     TTRY(gemm(st, TL_DW, F, T, {{a.act, t->dy_bf, t->g + o.wout, E}}, TG_F32, F, 0, nullptr, spare, spare_n));   // d Wout = act^T . dy
     hipLaunchKernelGGL(k_t_swiglu_bwd, EW((long)T * F / 8), t->dact, a.a, a.b, t->da, t->db, (long)T * F);
-    TTRY(gemm(st, TL_DX, T, F, {{t->da, pb + o.wi0, t->dxn, F}}, TG_F32, F, E, nullptr, spare, spare_n));   // d xn2 = da . Wi0^T + db . Wi1^T
-    TTRY(gemm(st, TL_DX, T, F, {{t->db, pb + o.wi1, t->dxn, F}}, TG_F32_ADD, F, E));
+    TTRY(gemm(st, TL_DX, T, F, {{t->da, pb + o.wi0, t->dxn, F}, {t->db, pb + o.wi1, t->dxn, F}}, TG_F32, F, E, nullptr, spare, spare_n));   // d xn2 = da . Wi0^T + db . Wi1^T
     TTRY(gemm(st, TL_DW, E, T, {{a.xn2, t->da, t->g + o.wi0, F}, {a.xn2, t->db, t->g + o.wi1, F}}, TG_F32, E, 0, nullptr, spare, spare_n));
     rmsnorm_bwd(st, t->dxn, a.h_mid, pb + o.ln2, a.r2, t->dh, t->dy_bf, t->g + o.ln2, E, T);
     // attention: h_mid = h_in + out(ao)
@@ -416,9 +442,7 @@ extern "C" int ixt_train_forward_backward(ixt_trainer* t, const int32_t* inputs,
     }
     hipLaunchKernelGGL((k_t_rope<true>), EW((long)T * (H + KVH) * (D / 8)), t->dq, t->dk, positions, t->rope_sin, t->rope_cos, H, KVH, D, (long)T);
     // d xn1 = dq Wq^T + dk Wk^T + dv Wv^T
-    TTRY(gemm(st, TL_DX, T, QN, {{t->dq, pb + o.wq, t->dxn, QN}}, TG_F32, QN, E, nullptr, spare, spare_n));
-    TTRY(gemm(st, TL_DX, T, KN, {{t->dk, pb + o.wk, t->dxn, KN}}, TG_F32_ADD, KN, E));
-    TTRY(gemm(st, TL_DX, T, KN, {{t->dv, pb + o.wv, t->dxn, KN}}, TG_F32_ADD, KN, E));
+    TTRY(gemm(st, TL_DX, T, QN, {{t->dq, pb + o.wq, t->dxn, QN}, {t->dk, pb + o.wk, t->dxn, KN}, {t->dv, pb + o.wv, t->dxn, KN}}, TG_F32, QN, E, nullptr, spare, spare_n));
     TTRY(gemm(st, TL_DW, E, T, {{a.xn1, t->dq, t->g + o.wq, QN}, {a.xn1, t->dk, t->g + o.wk, KN}, {a.xn1, t->dv, t->g + o.wv, KN}}, TG_F32, E, 0, nullptr, spare, spare_n));
     rmsnorm_bwd(st, t->dxn, a.h_in, pb + o.ln1, a.r1, t->dh, l > 0 ? t->dy_bf : nullptr, t->g + o.ln1, E, T);
     TLAUNCH();

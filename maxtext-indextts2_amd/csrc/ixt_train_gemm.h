@@ -18,6 +18,8 @@
 // One launch takes up to three products of the same M (`nprob`: the q, k and v projections, their gradients); `parts` > 1 cuts the reduction, part p
 // writing its own f32 C.  The attention's products run as batches, with the tiles and the reduction that the causal mask leaves: what it takes away is
 // zero, and a product of zeros leaves the accumulator as it is.  Blocks of one XCD take neighbouring tiles.
+// FOLD: where the tiles fill the chip without cutting the reduction, its parts, and products that are added up (the gradients of q, k and v), follow one
+// another in the block and join a second set of accumulators, in the same order: no partial C in memory, no kernel that adds them, one launch.
 #pragma once
 #include "ixt_device.h"
 
@@ -40,12 +42,14 @@ struct TGemm {
   // attention: nb1 x nb2 products of the same shape (nprob = parts = 1), element strides between them; `causal`: what the mask leaves
   int nb1, nb2, causal;
   long sa1, sa2, sb1, sb2, sc1, sc2;
+  // FOLD: C[0] = the sum of `nsum` products of the same K and strides (nprob = 1 then); product 0, or each of nprob, adds up `fold` chunks of 32 k at a time (0: all)
+  int nsum, fold;
 };
 enum { TC_NONE = 0, TC_LOWER = 1, TC_K_TO_ROW = 2, TC_K_FROM_ROW = 3 };   // C's tiles on and below the diagonal; k up to the tile's last row; k from its first row
 
 static __device__ const uint32_t tg_zero[4] = {0u, 0u, 0u, 0u};
 
-template <bool TA, bool TB, int MI, int NI, int WM, int WN, int NS>
+template <bool TA, bool TB, int MI, int NI, int WM, int WN, int NS, bool FOLD = false>
 __global__ __launch_bounds__(WM * WN * 64, 2) void k_tgemm(TGemm g) {
   constexpr int BM = 16 * MI * WM, BN = 16 * NI * WN, NW = WM * WN;
   constexpr int NA = BM / 16, NB = BN / 16, NJ = (NA + NB) / NW;          // KiB of a chunk; a wave fetches NJ of them
@@ -103,7 +107,8 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void k_tgemm(TGemm g) {
       off[j] = (uint32_t)((isa ? TA : TB) ? k * (int)(isa ? la : lb) + x : x * (int)(isa ? la : lb) + k) * 2u;
     }
   }
-  const int chunks = (segend - segk + 31) >> 5;
+  const int chunks1 = (segend - segk + 31) >> 5, chunks = FOLD ? g.nsum * chunks1 : chunks1;
+  int sum = 0;                                                            // FOLD: the product that is fetched
   bool whole = false;
   auto next_chunk = [&]() {                                               // past the last chunk: zeros, so that the counts stay
     whole = segk + 32 <= segend;
@@ -124,7 +129,17 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void k_tgemm(TGemm g) {
       asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(dst), "v"(p) : "memory");
     }
   };
-  auto advance = [&]() { segk += 32; pa += adva; pb += advb; };
+  auto advance = [&]() {
+    segk += 32; pa += adva; pb += advb;
+    if constexpr (FOLD) {
+      if (segk >= segend && sum + 1 < g.nsum) {
+        ++sum;
+        segk = 0;
+        pa = reinterpret_cast<const char*>(g.A[sum] + (TA ? (long)m0 : (long)m0 * g.lda[0]));
+        pb = reinterpret_cast<const char*>(g.B[sum] + (TB ? (long)n0 : (long)n0 * g.ldb[0]));
+      }
+    }
+  };
   const int trf = (r16 >> 2) | (q & 1) << 2;                              // k & 7 of the lane's row in a transposed read: 4 q + r16 / 4
   auto operand = [&](const bf16_t* img, int x, int bx, bool tr) -> tbf16x8 {
     tbf16x4 lo, hi;
@@ -187,9 +202,34 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void k_tgemm(TGemm g) {
     }
     advance();
   };
+  tf32x4 tot[FOLD ? MI : 1][FOLD ? NI : 1];
+  int next = FOLD && g.fold > 0 ? g.fold : chunks1;
+  bool first = true;
+  auto fold = [&](int done) {                                             // a cut of a reduction, or a whole one, joins the sum
+    if constexpr (FOLD) {
+      if (done != next) return;
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NI; ++j) {
+          tot[i][j] = first ? acc[i][j] : tot[i][j] + acc[i][j];
+          acc[i][j] = tf32x4(0.0f);
+        }
+      first = false;
+      next += done < chunks1 ? g.fold : chunks1;
+    }
+  };
   for (int c = 0; c < chunks; c += 2) {                                   // (an odd count: the last products are with zeros)
     step(c, 0);
+    fold(c + 1);
     step(c + 1, 1);
+    fold(c + 2);
+  }
+  if constexpr (FOLD) {
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NI; ++j) acc[i][j] = tot[i][j];
   }
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");             // nothing may land in LDS that the next block owns
   // lane: m = r16, n = 4 q + register
