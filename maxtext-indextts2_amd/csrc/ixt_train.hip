@@ -61,7 +61,7 @@ struct ixt_trainer {
   bf16_t *h_final = nullptr, *xn_f = nullptr, *rope_sin = nullptr, *rope_cos = nullptr;
   float* r_f = nullptr;
   // workspaces
-  float *scores = nullptr, *dh = nullptr, *dxn = nullptr, *logits = nullptr, *row_loss = nullptr, *scal = nullptr, *part = nullptr;
+  float *scores = nullptr, *dh = nullptr, *dxn = nullptr, *logits = nullptr, *row_loss = nullptr, *scal = nullptr, *part = nullptr, *norm_part = nullptr;   // norm_part: [norms][blocks][E], rows of at most 1024 (rmsnorm_bwd)
   bf16_t *dS = nullptr, *d_ao = nullptr, *dq = nullptr, *dk = nullptr, *dv = nullptr, *dact = nullptr, *da = nullptr, *db = nullptr, *dlog = nullptr,
          *dy_bf = nullptr;
   float *dkf = nullptr, *dvf = nullptr;   // grouped-query attention: dK / dV summed over a group's query heads in f32 before they round to bf16
@@ -77,6 +77,9 @@ static int tmalloc(ixt_trainer* t, T_** p, size_t n) {
   return IXT_OK;
 }
 
+// the norms' backward (k_t_rmsnorm_bwd)
+static int norm_rows(long T) { return T < 512 ? 1 : T < 8192 ? (int)(T / 512) : 16; }   // rows of a block
+static long norm_blocks(long T) { return (T + norm_rows(T) - 1) / norm_rows(T); }
 static void add_param(ixt_trainer* t, const std::string& name, long numel, long* off) {
   *off = t->total;
   t->params.push_back({name, t->total, numel});
@@ -132,6 +135,7 @@ extern "C" int ixt_train_create(const ixt_train_config* c, ixt_trainer** out) {
   A(tmalloc(t, &t->scores, BH * S * S)); A(tmalloc(t, &t->dh, T * E)); A(tmalloc(t, &t->dxn, T * E));
   A(tmalloc(t, &t->logits, (size_t)t->Tc * V)); A(tmalloc(t, &t->dlog, (size_t)t->Tc * t->Vp)); A(tmalloc(t, &t->row_loss, T)); A(tmalloc(t, &t->scal, (size_t)16));
   A(tmalloc(t, &t->part, (size_t)4096));
+  if (E <= 1024) A(tmalloc(t, &t->norm_part, (size_t)(2 * t->L + 1) * norm_blocks(t->T) * E));
   A(tmalloc(t, &t->dS, BH * S * S)); A(tmalloc(t, &t->d_ao, T * QN)); A(tmalloc(t, &t->dq, T * QN)); A(tmalloc(t, &t->dk, T * KN));
   A(tmalloc(t, &t->dv, T * KN));
   if (t->G > 1) { A(tmalloc(t, &t->dkf, T * KN)); A(tmalloc(t, &t->dvf, T * KN)); } A(tmalloc(t, &t->dact, T * F)); A(tmalloc(t, &t->da, T * F)); A(tmalloc(t, &t->db, T * F)); A(tmalloc(t, &t->dy_bf, T * E));
@@ -327,12 +331,12 @@ static int gemm(hipStream_t st, int what, int M, int K, std::initializer_list<TO
 }
 // 16 rows per block (16384 x 2048: 182 -> 141 us with the next row in flight and the bf16 copy included), fewer below 8192 rows: a block's rows
 // are a chain, but every block adds its sums to the same E words
-static void rmsnorm_bwd(hipStream_t st, const float* dy, const bf16_t* x, const bf16_t* scale, const float* rstd, float* dh, bf16_t* dh_bf, float* dscale, int E, long T) {
-  const int rpb = T < 512 ? 1 : T < 8192 ? (int)(T / 512) : 16;
-  const dim3 grid((unsigned)((T + rpb - 1) / rpb));
-  if (E <= 1024) hipLaunchKernelGGL(k_t_rmsnorm_bwd<4>, grid, dim3(256), 0, st, dy, x, scale, rstd, dh, dh_bf, dscale, E, T, rpb);
-  else if (E <= 2048) hipLaunchKernelGGL(k_t_rmsnorm_bwd<8>, grid, dim3(256), 0, st, dy, x, scale, rstd, dh, dh_bf, dscale, E, T, rpb);
-  else hipLaunchKernelGGL(k_t_rmsnorm_bwd<TN_FPT>, grid, dim3(256), 0, st, dy, x, scale, rstd, dh, dh_bf, dscale, E, T, rpb);
+static void rmsnorm_bwd(hipStream_t st, const float* dy, const bf16_t* x, const bf16_t* scale, const float* rstd, float* dh, bf16_t* dh_bf, float* dscale, float* part, int E, long T) {
+  const int rpb = norm_rows(T);
+  const dim3 grid((unsigned)norm_blocks(T));
+  if (E <= 1024) hipLaunchKernelGGL(k_t_rmsnorm_bwd<4>, grid, dim3(256), 0, st, dy, x, scale, rstd, dh, dh_bf, dscale, part, E, T, rpb);
+  else if (E <= 2048) hipLaunchKernelGGL(k_t_rmsnorm_bwd<8>, grid, dim3(256), 0, st, dy, x, scale, rstd, dh, dh_bf, dscale, part, E, T, rpb);
+  else hipLaunchKernelGGL(k_t_rmsnorm_bwd<TN_FPT>, grid, dim3(256), 0, st, dy, x, scale, rstd, dh, dh_bf, dscale, part, E, T, rpb);
 }
 #define EW(n) dim3((unsigned)(((long)(n) + 255) / 256)), dim3(256), 0, st
 
@@ -402,7 +406,8 @@ extern "C" int ixt_train_forward_backward(ixt_trainer* t, const int32_t* inputs,
   float* const spare = t->logits;                          // idle from here on: scratch of the cut weight-gradient products
   const size_t spare_n = (size_t)t->Tc * V;
   hipLaunchKernelGGL(k_t_zero, dim3((unsigned)(((long)T * E + 1023) / 1024)), dim3(256), 0, st, t->dh, (long)T * E, t->g, t->g, 0L, 0, 4);
-  rmsnorm_bwd(st, t->dxn, t->h_final, pb + t->o_fnorm, t->r_f, t->dh, t->dy_bf, t->g + t->o_fnorm, E, T);
+  const auto norm_part = [&](int q) { return t->norm_part != nullptr ? t->norm_part + (size_t)q * norm_blocks(T) * E : nullptr; };
+  rmsnorm_bwd(st, t->dxn, t->h_final, pb + t->o_fnorm, t->r_f, t->dh, t->dy_bf, t->g + t->o_fnorm, norm_part(2 * t->L), E, T);
   for (int l = t->L - 1; l >= 0; --l) {
     LayerAct& a = t->act[l];
     const ixt_trainer::LOff& o = t->lo[l];
@@ -412,7 +417,7 @@ extern "C" int ixt_train_forward_backward(ixt_trainer* t, const int32_t* inputs,
     hipLaunchKernelGGL(k_t_swiglu_bwd, EW((long)T * F / 8), t->dact, a.a, a.b, t->da, t->db, (long)T * F);
     TTRY(gemm(st, TL_DX, T, F, {{t->da, pb + o.wi0, t->dxn, F}, {t->db, pb + o.wi1, t->dxn, F}}, TG_F32, F, E, nullptr, spare, spare_n));   // d xn2 = da . Wi0^T + db . Wi1^T
     TTRY(gemm(st, TL_DW, E, T, {{a.xn2, t->da, t->g + o.wi0, F}, {a.xn2, t->db, t->g + o.wi1, F}}, TG_F32, E, 0, nullptr, spare, spare_n));
-    rmsnorm_bwd(st, t->dxn, a.h_mid, pb + o.ln2, a.r2, t->dh, t->dy_bf, t->g + o.ln2, E, T);
+    rmsnorm_bwd(st, t->dxn, a.h_mid, pb + o.ln2, a.r2, t->dh, t->dy_bf, t->g + o.ln2, norm_part(t->L + l), E, T);
     // attention: h_mid = h_in + out(ao)
     TTRY(gemm(st, TL_DX, T, E, {{t->dy_bf, pb + o.wo, t->d_ao, E}}, TG_BF16, E, QN));                    // d ao = dy . Wo^T
     TTRY(gemm(st, TL_DW, QN, T, {{a.ao, t->dy_bf, t->g + o.wo, E}}, TG_F32, QN, 0, nullptr, spare, spare_n));   // d Wo = ao^T . dy
@@ -444,9 +449,12 @@ extern "C" int ixt_train_forward_backward(ixt_trainer* t, const int32_t* inputs,
     // d xn1 = dq Wq^T + dk Wk^T + dv Wv^T
     TTRY(gemm(st, TL_DX, T, QN, {{t->dq, pb + o.wq, t->dxn, QN}, {t->dk, pb + o.wk, t->dxn, KN}, {t->dv, pb + o.wv, t->dxn, KN}}, TG_F32, QN, E, nullptr, spare, spare_n));
     TTRY(gemm(st, TL_DW, E, T, {{a.xn1, t->dq, t->g + o.wq, QN}, {a.xn1, t->dk, t->g + o.wk, KN}, {a.xn1, t->dv, t->g + o.wv, KN}}, TG_F32, E, 0, nullptr, spare, spare_n));
-    rmsnorm_bwd(st, t->dxn, a.h_in, pb + o.ln1, a.r1, t->dh, l > 0 ? t->dy_bf : nullptr, t->g + o.ln1, E, T);
+    rmsnorm_bwd(st, t->dxn, a.h_in, pb + o.ln1, a.r1, t->dh, l > 0 ? t->dy_bf : nullptr, t->g + o.ln1, norm_part(l), E, T);
     TLAUNCH();
   }
+  if (t->norm_part != nullptr)
+    hipLaunchKernelGGL(k_t_scale_grads, dim3((E + 63) / 64, 2 * t->L + 1), dim3(1024), 0, st, t->norm_part, (int)norm_blocks(T), E, t->g, t->L, t->lo[0].ln1, t->lo[0].ln2,
+                       t->L > 1 ? t->lo[1].ln1 - t->lo[0].ln1 : 0L, t->o_fnorm);
   hipLaunchKernelGGL(k_t_embed_bwd, dim3((E + 255) / 256, T), dim3(256), 0, st, t->dh, inputs, t->g + t->o_emb, E, V);
   TLAUNCH();
   return IXT_OK;

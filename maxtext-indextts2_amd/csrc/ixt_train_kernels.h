@@ -85,14 +85,15 @@ static __global__ __launch_bounds__(256) void k_t_rmsnorm_fwd(const bf16_t* __re
 }
 // backward: dy f32 [T][E] (the sum of the consumers' input gradients); dx (f32) is ADDED to dh (the residual-stream gradient), and the sum goes out as
 // bf16, too (dh_bf, the next products' operand; nullptr: nobody wants it).
-// dscale: a block walks `rpb` rows and keeps its features' partial sums in registers -- one f32 atomic per feature and BLOCK (one per feature and row
+// dscale: a block walks `rpb` rows and keeps its features' partial sums in registers -- written out for k_t_scale_grads (part), or one f32 atomic per
+// feature and BLOCK (short rows: the atomics were 10 of 23 us at 2048 x 768; 13 of 145 at 16384 x 2048) (one per feature and row
 // took 466 us per launch at 16384 x 2048: 2048 addresses under 33 M atomics).  A row's operands stay in registers between the two passes over it and
 // the next row's are in flight meanwhile.  grid = ceil(T / rpb), block 256, E <= 256 FPT.
 #define TN_FPT 16
 template <int FPT>
 static __global__ __launch_bounds__(256) void k_t_rmsnorm_bwd(const float* __restrict__ dy, const bf16_t* __restrict__ x, const bf16_t* __restrict__ scale,
-                                                       const float* __restrict__ rstd, float* __restrict__ dh, bf16_t* __restrict__ dh_bf, float* __restrict__ dscale, int E, long T,
-                                                       int rpb) {
+                                                       const float* __restrict__ rstd, float* __restrict__ dh, bf16_t* __restrict__ dh_bf, float* __restrict__ dscale, float* __restrict__ part,
+                                                       int E, long T, int rpb) {
   __shared__ float red[4];
   float ds[FPT], sc[FPT], gy[FPT], xv[FPT], hv[FPT];
 #pragma unroll
@@ -134,7 +135,33 @@ static __global__ __launch_bounds__(256) void k_t_rmsnorm_bwd(const float* __res
 #pragma unroll
   for (int i = 0; i < FPT; ++i) {
     const int e = threadIdx.x + i * 256;
-    if (e < E) atomicAdd(dscale + e, ds[i]);
+    if (e < E) {
+      if (part != nullptr) part[(long)blockIdx.x * E + e] = ds[i];
+      else atomicAdd(dscale + e, ds[i]);
+    }
+  }
+}
+// the scale gradients of all norms from their blocks' parts [norms][n][E]: norm y is first (y < L), second (y < 2 L) or final; offsets into the gradients.
+// grid = (ceil(E / 64), 2 L + 1), block 1024 = 64 features x 16 runs of parts
+static __global__ __launch_bounds__(1024) void k_t_scale_grads(const float* __restrict__ part, int n, int E, float* __restrict__ g, int L, long o1, long o2, long layer, long o_final) {
+  __shared__ float run[16][64];
+  const int f = threadIdx.x & 63, r = threadIdx.x >> 6, e = blockIdx.x * 64 + f, y = blockIdx.y;
+  const float* p = part + ((long)y * n + (long)n * r / 16) * E + e;
+  const int m = (long)n * (r + 1) / 16 - (long)n * r / 16;
+  float s = 0.0f;
+  if (e < E)
+    for (int i = 0; i < m; i += 8) {
+      float v[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[k] = i + k < m ? p[(long)(i + k) * E] : 0.0f;
+#pragma unroll
+      for (int k = 0; k < 8; ++k) s += v[k];
+    }
+  run[r][f] = s;
+  __syncthreads();
+  if (r == 0 && e < E) {
+    for (int k = 1; k < 16; ++k) s += run[k][f];
+    g[(y < L ? o1 + y * layer : y < 2 * L ? o2 + (y - L) * layer : o_final) + e] = s;
   }
 }
 // out[i] = parts[0][i] + parts[1][i] + ... (split-K partial products, in order)
