@@ -1405,9 +1405,18 @@ static int launch_logits_post(ixt_ctx* c, float* lg, int nl, int normalize, floa
   return IXT_OK;
 }
 
+static int launch_gnorm(const GNormArgs& ga, int R, hipStream_t st) {
+  if (ga.E <= 4096) hipLaunchKernelGGL(k_gnorm<2>, dim3(R), dim3(256), 0, st, ga);
+  else if (ga.E <= 8192) hipLaunchKernelGGL(k_gnorm<4>, dim3(R), dim3(256), 0, st, ga);
+  else if (ga.E <= 16384) hipLaunchKernelGGL(k_gnorm<8>, dim3(R), dim3(256), 0, st, ga);
+  else return set_err(IXT_ERR_UNSUPPORTED, "gemma norm: emb_dim %d above 16384", ga.E);
+  LAUNCHCHK();
+  return IXT_OK;
+}
 // The Gemma-2 block over R rows (layers/gemma2.py:69-236): per (attention, MLP) sub-layer
 //   QKV dot -> k_qkv_finalize (RoPE, q -> qbuf, K/V -> pages) -> scores / softmax + PV (soft cap; sliding window on the even, "local"
-//   sub-layers) / combine -> O dot -> k_gnorm (post norm, residual, pre-MLP norm) -> wi dot -> GELU gate -> down dot -> k_gnorm (post norm,
+//   sub-layers) / combine -> O dot -> k_gnorm (post norm, residual, pre-MLP norm) -> wi dot -> GELU gate (from 17 rows on, RoPE and page write, and the gate, are epilogues of
+//   their products) -> down dot -> k_gnorm (post norm,
 //   residual, the next pre-attention norm or the final norm).  Prefill and decode rows take the same launches: every row's K/V is in its
 //   page before any score is computed, and a row never sees a key beyond its own position.
 // Logits: unembedding (dense kernel, or the transposed embedding when logits_via_embedding), then k_logits_post (/ sqrt(emb), soft cap,
@@ -1420,25 +1429,34 @@ static int forward_rows_gemma2(ixt_ctx* c, int R, const int32_t* tokens, int len
   bf16_t* hcur = c->h_a;
   bf16_t* hnext = c->h_b;
   const bool all_rows = nl == R && lrow0 == 0 && lrows == nullptr;
-  const size_t glds = sizeof(float) * ((size_t)E + 128);
+  const bool ring = R >= ring_model_rows(c) && !c->fp8;   // QKV and the gate as epilogues of the products
   const bool attn_tiled = c->gemma_tile && tile_attn_fits(c, R, len_hint, false) && attn_split_factor(c, R) <= 1;
   TRY(launch_rownorm(c, 0, R, tokens, nullptr, nullptr, hcur, c->layers[0].ln1, c->xn, st));
   for (int l = 0; l < c->L; ++l) {
     const LayerW& w = c->layers[l];
-    TRY(launch_dot(c, c->xn, w.wqkv, E, c->NQKV, R, c->part, c->part_floats, false, st, &dr));
-    QkvArgs qa;
-    qa.part = c->part; qa.slices = dr.slices; qa.slice_stride = dr.slice_stride; qa.ncols = c->NQKV;
-    qa.row_slot = c->row_slot; qa.row_pos = c->row_pos; qa.row_active = c->row_active; qa.page_map = c->ps.page_map;
     // gemma2.py: even sub-layers are the local ones; gemma3.py:35-47: five local layers, then a global one
     const bool local = c->gemma3 ? (l % 6 != 5) : (l % 2 == 0);
     const bool lrope = local && c->rope_sin_local != nullptr;
-    qa.rope_sin = lrope ? c->rope_sin_local : c->rope_sin; qa.rope_cos = lrope ? c->rope_cos_local : c->rope_cos; qa.qbuf = c->qbuf;
-    qa.kpages = c->kpages_l[l]; qa.vpages = c->vpages_l[l];
-    qa.g = c->geom;
-    qa.qnorm = w.qn; qa.knorm = w.kn; qa.eps = cf.normalization_layer_epsilon;
-    qa.q_scalar = (cf.query_pre_attn_scalar != 0.0f && cf.query_pre_attn_scalar != 1.0f) ? host_rbf(cf.query_pre_attn_scalar) : 0.0f;
-    hipLaunchKernelGGL(k_qkv_finalize, dim3(R, c->Q + 2 * c->KV), dim3(64), 0, st, qa);
-    LAUNCHCHK();
+    const bf16_t *rsin = lrope ? c->rope_sin_local : c->rope_sin, *rcos = lrope ? c->rope_cos_local : c->rope_cos;
+    const float q_scalar = (cf.query_pre_attn_scalar != 0.0f && cf.query_pre_attn_scalar != 1.0f) ? host_rbf(cf.query_pre_attn_scalar) : 0.0f;
+    if (ring && w.qn == nullptr && w.kn == nullptr) {   // no norm over a head: RoPE and the page write are an epilogue
+      GemmEpi e{};
+      e.row_slot = c->row_slot; e.row_pos = c->row_pos; e.row_active = c->row_active; e.page_map = c->ps.page_map;
+      e.rope_sin = rsin; e.rope_cos = rcos; e.qbuf = c->qbuf; e.kpages = c->kpages_l[l]; e.vpages = c->vpages_l[l]; e.g = c->geom; e.q_scalar = q_scalar;
+      TRY(launch_ring(c, GEPI_QKV, c->xn, w.wqkv, E, c->NQKV, R, e, false, st));
+    } else {
+      TRY(launch_dot(c, c->xn, w.wqkv, E, c->NQKV, R, c->part, c->part_floats, false, st, &dr));
+      QkvArgs qa;
+      qa.part = c->part; qa.slices = dr.slices; qa.slice_stride = dr.slice_stride; qa.ncols = c->NQKV;
+      qa.row_slot = c->row_slot; qa.row_pos = c->row_pos; qa.row_active = c->row_active; qa.page_map = c->ps.page_map;
+      qa.rope_sin = rsin; qa.rope_cos = rcos; qa.qbuf = c->qbuf;
+      qa.kpages = c->kpages_l[l]; qa.vpages = c->vpages_l[l];
+      qa.g = c->geom;
+      qa.qnorm = w.qn; qa.knorm = w.kn; qa.eps = cf.normalization_layer_epsilon;
+      qa.q_scalar = q_scalar;
+      hipLaunchKernelGGL(k_qkv_finalize, dim3(R, c->Q + 2 * c->KV), dim3(64), 0, st, qa);
+      LAUNCHCHK();
+    }
     const int attn_split = attn_split_factor(c, R);   // few rows (decode): the keys of a head over several blocks of ONE launch instead of scores / PV / combine
     if (attn_split > 1) {
       TRY(launch_attn_split(c, l, R, attn_split, st, cf.attn_logits_soft_cap, local ? cf.sliding_window_size : 0));
@@ -1457,16 +1475,20 @@ static int forward_rows_gemma2(ixt_ctx* c, int R, const int32_t* tokens, int len
     GNormArgs ga;
     ga.part = c->part; ga.slices = dr.slices; ga.slice_stride = dr.slice_stride; ga.h_in = hcur; ga.h_out = hnext;
     ga.post = w.pan; ga.next = w.ln2; ga.xn_out = c->xn; ga.E = E; ga.eps = cf.normalization_layer_epsilon;
-    hipLaunchKernelGGL(k_gnorm, dim3(R), dim3(256), glds, st, ga);
-    LAUNCHCHK();
-    TRY(launch_dot(c, c->xn, w.wi, E, 2 * F, R, c->part, c->part_floats, false, st, &dr));
-    hipLaunchKernelGGL(k_geglu_part, dim3((F + 2047) / 2048, R), dim3(256), 0, st, c->part, dr.slices, dr.slice_stride, F, c->hact);
-    LAUNCHCHK();
+    TRY(launch_gnorm(ga, R, st));
+    if (ring) {
+      GemmEpi eu{};
+      eu.act = c->hact; eu.glu = -1;
+      TRY(launch_ring(c, GEPI_SWIGLU, c->xn, w.wi, E, 2 * F, R, eu, false, st));
+    } else {
+      TRY(launch_dot(c, c->xn, w.wi, E, 2 * F, R, c->part, c->part_floats, false, st, &dr));
+      hipLaunchKernelGGL(k_geglu_part, dim3((F + 2047) / 2048, R), dim3(256), 0, st, c->part, dr.slices, dr.slice_stride, F, c->hact);
+      LAUNCHCHK();
+    }
     TRY(launch_dot(c, c->hact, w.wout, F, E, R, c->part, c->part_floats, false, st, &dr));
     ga.part = c->part; ga.slices = dr.slices; ga.slice_stride = dr.slice_stride; ga.h_in = hnext; ga.h_out = hcur;
     ga.post = w.pfn; ga.next = l + 1 < c->L ? c->layers[l + 1].ln1 : (all_rows ? c->final_norm : nullptr);
-    hipLaunchKernelGGL(k_gnorm, dim3(R), dim3(256), glds, st, ga);
-    LAUNCHCHK();
+    TRY(launch_gnorm(ga, R, st));
   }
   if (nl > 0) {
     if (nl > c->NLmax) return set_err(IXT_ERR_INVALID, "too many logits rows (%d > %d)", nl, c->NLmax);

@@ -21,7 +21,7 @@
 //   GEPI_UNEMBED  greedy sampling (decoders.py:566-587, inference_utils.py:74-75): bf16-rounded logits on request, one
 //                 (max, first index) pair per row and wave column for k_argmax_final
 //   GEPI_RESID    h_out = bf16(h_in + bf16(t))                                   (llama2.py:127, :157)
-//   GEPI_SWIGLU   act = bf16(bf16(silu(bf16(t_0))) * bf16(t_1))                  (linears.py:449-464); the fused wi kernel stores
+//   GEPI_SWIGLU   act = bf16(bf16(silu(bf16(t_0))) * bf16(t_1)), or the gelu gate  (linears.py:449-464); the fused wi kernel stores
 //                 wi_0 tile j and wi_1 tile j as column tiles 2j, 2j+1, so both gates of a feature are in one wave
 //   GEPI_ACT      act = bf16(unit(t)), a unit without a gate (ixt_act)
 //   GEPI_TANHNORM residual and norms of a decoder with tanh norms (TanhNormEpi)
@@ -88,10 +88,11 @@ struct GemmEpi {
   const bf16_t* rope_sin; const bf16_t* rope_cos;
   bf16_t* qbuf; bf16_t* kpages; bf16_t* vpages;
   AttnGeom g;
+  float q_scalar;                                       // QKV: queries times this bf16 value behind RoPE (0: none)
   const float* xscale; const float* wscale;             // F8: activation scales [rows][chains], column scales [N] (ixt_fp8.h)
   size_t sstride;                                       // F8 + routed experts: floats between two experts' column scales
   TanhNormEpi tn;                                       // TANHNORM (with act)
-  int glu; float glu_limit; const float* act_par;       // ACT: the unit's kind and its numbers; SWIGLU: glu != 0 takes that gated unit of the f32 totals instead (ixt_glu)
+  int glu; float glu_limit; const float* act_par;       // ACT: the unit's kind and its numbers; SWIGLU: glu > 0 takes that gated unit of the f32 totals instead (ixt_glu), glu < 0 ixt_geglu
   const int32_t* rb_exp; size_t wstride;                // routed experts: expert of every 16-row block (-1: none), 16-byte units between experts' kernels
 };
 
@@ -373,7 +374,8 @@ __global__ __launch_bounds__(WR * WC * 64, 2) void k_gemm_ring(const u32x4* __re
           bf16_t o[4];
 #pragma unroll
           for (int j = 0; j < 4; ++j)
-            o[j] = e.glu ? f2bf(ixt_glu(e.glu, tot[i][b][j], tot[i + 1][b][j], e.glu_limit)) : ixt_swiglu(rbf(tot[i][b][j]), rbf(tot[i + 1][b][j]));
+            o[j] = e.glu > 0 ? f2bf(ixt_glu(e.glu, tot[i][b][j], tot[i + 1][b][j], e.glu_limit)) : e.glu < 0 ? ixt_geglu(rbf(tot[i][b][j]), rbf(tot[i + 1][b][j]))
+                                                                                                          : ixt_swiglu(rbf(tot[i][b][j]), rbf(tot[i + 1][b][j]));
           uint2 ov;
           ov.x = pack2(o[0], o[1]); ov.y = pack2(o[2], o[3]);
           *reinterpret_cast<uint2*>(e.act + xidx(row, f0, F)) = ov;
@@ -428,6 +430,10 @@ __global__ __launch_bounds__(WR * WC * 64, 2) void k_gemm_ring(const u32x4* __re
             v[j] = cq < 2 ? rbf(rbf(v[j] * cs[j]) - rbf(other * sn[j])) : rbf(rbf(v[j] * cs[j]) + rbf(other * sn[j]));
           }
           }
+        }
+        if (hh < g.nq && e.q_scalar != 0.0f) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) v[j] = rbf(v[j] * e.q_scalar);
         }
         if (tile >= ntile || !row_ok) continue;
         uint2 ov;

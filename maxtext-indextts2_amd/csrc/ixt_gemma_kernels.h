@@ -11,7 +11,8 @@
 // o = bf16(bf16(o * rsqrt(mean(o^2) + eps)) * post)       when post != nullptr   (gemma2.py:107-116, :135-143)
 // h = bf16(h_in + o) -> h_out                             (gemma2.py:118, :146)
 // xn = bf16(bf16(h * rsqrt(mean(h^2) + eps)) * next)      when next != nullptr (the following pre-norm), dot kernel's x layout
-// grid = R, block 256, dynamic LDS = (E + 128) floats.
+// A thread keeps its chunks of 8 features (tid + 256 it, E <= 2048 ITS) in registers from the sums to the last norm, and everything it reads is in flight
+// before the first of the two sums over the row (one read behind the other: 7.8 us a launch of 256 rows of 2304 -> 6.4).   grid = R, block 256.
 // =====================================================================================================
 struct GNormArgs {
   const float* part; int slices; size_t slice_stride;
@@ -21,96 +22,90 @@ struct GNormArgs {
   int E; float eps;
 };
 
+template <int ITS>
 static __global__ __launch_bounds__(256) void k_gnorm(GNormArgs a) {
-  extern __shared__ __attribute__((aligned(16))) float smem[];
-  float* row = smem;             // [E] o, then h
-  float* blk = smem + a.E;       // [<=64] block sums of o^2
-  float* blk2 = blk + 64;        // [<=64] block sums of h^2
+  __shared__ float blk[2][4 * ITS];                        // block sums of o^2, of h^2
   const int r = blockIdx.x, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int E = a.E, nch = E / 8, nblk = (nch + 63) / 64;
-  // pass 1: o and its sum of squares
-  for (int it = 0; it * 4 < nblk; ++it) {
-    const int b = it * 4 + wave;
-    const int ch = b * 64 + lane;
-    float v = 0.0f;
-    if (b < nblk && ch < nch) {
-      float o[8];
+  float o[ITS][8];
+  u32x4 hin[ITS], post[ITS], next[ITS];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) o[j] = 0.0f;
-      for (int s = 0; s < a.slices; ++s) {
+  for (int it = 0; it < ITS; ++it) {
+    const int ch = it * 256 + tid;
+    hin[it] = post[it] = next[it] = u32x4(0u);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) o[it][j] = 0.0f;
+    if (ch < nch) {
+      hin[it] = *reinterpret_cast<const u32x4*>(a.h_in + (size_t)r * E + ch * 8);
+      if (a.post != nullptr) post[it] = *reinterpret_cast<const u32x4*>(a.post + ch * 8);
+      if (a.next != nullptr) next[it] = *reinterpret_cast<const u32x4*>(a.next + ch * 8);
+    }
+  }
+  for (int s = 0; s < a.slices; ++s) {
+#pragma unroll
+    for (int it = 0; it < ITS; ++it) {
+      const int ch = it * 256 + tid;
+      if (ch < nch) {
         const float* p = a.part + (size_t)s * a.slice_stride + (size_t)r * E + ch * 8;
         const float4 p0 = *reinterpret_cast<const float4*>(p), p1 = *reinterpret_cast<const float4*>(p + 4);
-        o[0] = o[0] + p0.x; o[1] = o[1] + p0.y; o[2] = o[2] + p0.z; o[3] = o[3] + p0.w;
-        o[4] = o[4] + p1.x; o[5] = o[5] + p1.y; o[6] = o[6] + p1.z; o[7] = o[7] + p1.w;
-      }
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        o[j] = rbf(o[j]);
-        row[ch * 8 + j] = o[j];
-        v = __builtin_fmaf(o[j], o[j], v);
+        o[it][0] = o[it][0] + p0.x; o[it][1] = o[it][1] + p0.y; o[it][2] = o[it][2] + p0.z; o[it][3] = o[it][3] + p0.w;
+        o[it][4] = o[it][4] + p1.x; o[it][5] = o[it][5] + p1.y; o[it][6] = o[it][6] + p1.z; o[it][7] = o[it][7] + p1.w;
       }
     }
-    if (b < nblk) {
+  }
+  // the sum of squares of a row: 64 chunks of 8 features at a time (a wave's), in order
+  auto square_sum = [&](float* sums) {
+#pragma unroll
+    for (int it = 0; it < ITS; ++it) {
+      float v = 0.0f;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v = __builtin_fmaf(o[it][j], o[it][j], v);
 #pragma unroll
       for (int off = 1; off < 64; off <<= 1) v = v + __shfl_xor(v, off, 64);
-      if (lane == 0) blk[b] = v;
+      if (lane == 0) sums[it * 4 + wave] = v;
     }
-  }
-  __syncthreads();
-  float rs1 = 0.0f;
-  if (a.post != nullptr) {
+    __syncthreads();
     float total = 0.0f;
-    for (int b = 0; b < nblk; ++b) total = total + blk[b];
-    rs1 = 1.0f / sqrtf(total / (float)E + a.eps);
-  }
-  // pass 2: post norm, residual, sum of squares of h (each thread revisits the chunks it wrote)
-  for (int it = 0; it * 4 < nblk; ++it) {
-    const int b = it * 4 + wave;
-    const int ch = b * 64 + lane;
-    float v = 0.0f;
-    if (b < nblk && ch < nch) {
-      const u32x4 hv = *reinterpret_cast<const u32x4*>(a.h_in + (size_t)r * E + ch * 8);
-      const float hin[8] = {bflo(hv.x), bfhi(hv.x), bflo(hv.y), bfhi(hv.y), bflo(hv.z), bfhi(hv.z), bflo(hv.w), bfhi(hv.w)};
-      float sc[8];
-      if (a.post != nullptr) {
-        const u32x4 sv = *reinterpret_cast<const u32x4*>(a.post + ch * 8);
-        sc[0] = bflo(sv.x); sc[1] = bfhi(sv.x); sc[2] = bflo(sv.y); sc[3] = bfhi(sv.y);
-        sc[4] = bflo(sv.z); sc[5] = bfhi(sv.z); sc[6] = bflo(sv.w); sc[7] = bfhi(sv.w);
-      }
-      float h[8];
+    for (int b = 0; b < nblk; ++b) total = total + sums[b];
+    return 1.0f / sqrtf(total / (float)E + a.eps);
+  };
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        float o = row[ch * 8 + j];
-        if (a.post != nullptr) o = rbf(rbf(o * rs1) * sc[j]);
-        h[j] = rbf(hin[j] + o);
-        row[ch * 8 + j] = h[j];
-        v = __builtin_fmaf(h[j], h[j], v);
-      }
+  for (int it = 0; it < ITS; ++it)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) o[it][j] = rbf(o[it][j]);
+  const float rs1 = a.post != nullptr ? square_sum(blk[0]) : 0.0f;
+#pragma unroll
+  for (int it = 0; it < ITS; ++it) {
+    const float hf[8] = {bflo(hin[it].x), bfhi(hin[it].x), bflo(hin[it].y), bfhi(hin[it].y), bflo(hin[it].z), bfhi(hin[it].z), bflo(hin[it].w), bfhi(hin[it].w)};
+    const float sc[8] = {bflo(post[it].x), bfhi(post[it].x), bflo(post[it].y), bfhi(post[it].y), bflo(post[it].z), bfhi(post[it].z), bflo(post[it].w), bfhi(post[it].w)};
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      float v = o[it][j];
+      if (a.post != nullptr) v = rbf(rbf(v * rs1) * sc[j]);
+      o[it][j] = rbf(hf[j] + v);
+    }
+    const int ch = it * 256 + tid;
+    if (ch < nch) {
       u32x4 ov;
-      ov.x = pack2(f2bf(h[0]), f2bf(h[1])); ov.y = pack2(f2bf(h[2]), f2bf(h[3]));
-      ov.z = pack2(f2bf(h[4]), f2bf(h[5])); ov.w = pack2(f2bf(h[6]), f2bf(h[7]));
+      ov.x = pack2(f2bf(o[it][0]), f2bf(o[it][1])); ov.y = pack2(f2bf(o[it][2]), f2bf(o[it][3]));
+      ov.z = pack2(f2bf(o[it][4]), f2bf(o[it][5])); ov.w = pack2(f2bf(o[it][6]), f2bf(o[it][7]));
       *reinterpret_cast<u32x4*>(a.h_out + (size_t)r * E + ch * 8) = ov;
     }
-    if (b < nblk) {
-#pragma unroll
-      for (int off = 1; off < 64; off <<= 1) v = v + __shfl_xor(v, off, 64);
-      if (lane == 0) blk2[b] = v;
-    }
   }
-  __syncthreads();
-  if (a.next == nullptr) return;
-  float total = 0.0f;
-  for (int b = 0; b < nblk; ++b) total = total + blk2[b];
-  const float rs = 1.0f / sqrtf(total / (float)E + a.eps);
-  for (int ch = tid; ch < nch; ch += 256) {
-    const u32x4 sv = *reinterpret_cast<const u32x4*>(a.next + ch * 8);
-    const float sc[8] = {bflo(sv.x), bfhi(sv.x), bflo(sv.y), bfhi(sv.y), bflo(sv.z), bfhi(sv.z), bflo(sv.w), bfhi(sv.w)};
-    bf16_t o[8];
+  if (a.next == nullptr) return;                           // whole grid
+  const float rs = square_sum(blk[1]);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) o[j] = f2bf(rbf(row[ch * 8 + j] * rs) * sc[j]);
-    u32x4 ov;
-    ov.x = pack2(o[0], o[1]); ov.y = pack2(o[2], o[3]); ov.z = pack2(o[4], o[5]); ov.w = pack2(o[6], o[7]);
-    *reinterpret_cast<u32x4*>(a.xn_out + xidx(r, ch * 8, E)) = ov;
+  for (int it = 0; it < ITS; ++it) {
+    const int ch = it * 256 + tid;
+    if (ch < nch) {
+      const float sc[8] = {bflo(next[it].x), bfhi(next[it].x), bflo(next[it].y), bfhi(next[it].y), bflo(next[it].z), bfhi(next[it].z), bflo(next[it].w), bfhi(next[it].w)};
+      bf16_t y[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) y[j] = f2bf(rbf(o[it][j] * rs) * sc[j]);
+      u32x4 ov;
+      ov.x = pack2(y[0], y[1]); ov.y = pack2(y[2], y[3]); ov.z = pack2(y[4], y[5]); ov.w = pack2(y[6], y[7]);
+      *reinterpret_cast<u32x4*>(a.xn_out + xidx(r, ch * 8, E)) = ov;
+    }
   }
 }
 

@@ -46,3 +46,14 @@ def test_unembedding_of_some_rows(ctx, R):
   H.lib.check(eng.lib.ixt_op_unembed_argmax(eng._ctx, _vp(H.dev_bf16(y)), R, _vp(logits), _vp(amax), _st(torch)))
   assert np.array_equal(logits.cpu().numpy().view(np.uint32), lg.view(np.uint32))
   assert np.array_equal(amax.cpu().numpy(), np.argmax(lg, axis=-1).astype(np.int32))
+
+
+@pytest.mark.parametrize("rows", [16, 17, 64, 65, 127])
+def test_gelu_gate_and_query_scale_epilogues(rows):
+  """A Gemma-2 prompt of that many rows, one prefill call: up to 16 rows split-K dots with kernels of their own, from 17 on RoPE, the query scale, the page
+  write and the gelu gate as epilogues; then a few steps, token by token against the oracle."""
+  from test_gpu_engine import run_pair
+  cfg = H.make_config("gemma2-tiny", max_prefill_predict_length=128, max_target_length=160, per_device_batch_size=2.0, pagedattn_num_pages=64, head_dim=128,
+                      base_num_query_heads=4, base_num_kv_heads=2, sliding_window_size=24)
+  w = H.synth.synth_weights(cfg, 9)
+  run_pair(cfg, w, [(H.synth.synth_prompt(cfg.vocab_size, 128, 70)[0], rows)], steps=4)
