@@ -992,16 +992,18 @@ int launch_dot(ixt_ctx* c, const bf16_t* x, const bf16_t* w, int K, int N, int R
 }
 
 
-// Rows from which a pass of the llama blocks and the unembedding run on the ring GEMM.  From 17 on (up to 16 the kernels of ixt_small.h serve): 64-row tiles of
-// 64, 32 or 16 columns stream the weights as fast as the split-K dots and their epilogues leave no slices to add up (attention has its q and keys ready
-// instead of adding QKV slices).  48 rows of the 1B model, one layer: QKV 11.3 -> 12.1 us and attention 47.1 -> 42.3, O and norm 11.9 -> 13.3,
-// MLP up and gate 23.8 -> 14.7; unembedding 267 -> 220.  A decode step 2.08 -> 1.83 ms; a prompt of 57 tokens 1.57 -> 1.35 ms.
-static int ring_model_rows(const ixt_ctx* c) { return c->ring_min_rows > 128 ? c->ring_min_rows : std::min(c->ring_min_rows, c->ring_mid_rows); }
+// Rows from which a pass of the llama blocks (or Gemma's: RoPE and the gate) and the unembedding run on the ring GEMM.  64-row tiles of 64, 32 or 16 columns
+// stream the weights as fast as the split-K dots and their epilogues leave no slices to add up (attention has its q and keys ready instead of adding QKV
+// slices).  48 rows of the 1B model, one layer: QKV 11.3 -> 12.1 us and attention 47.1 -> 42.3, O and norm 11.9 -> 13.3, MLP up and gate 23.8 -> 14.7;
+// unembedding 267 -> 220.  A decode step of 48 rows 2.08 -> 1.83 ms, a prompt of 57 tokens 1.57 -> 1.35 ms.  Prompts from 17 rows on (up to 16 the kernels
+// of ixt_small.h serve; 20 rows 1.32 -> 1.26 ms); decode rows and the unembedding from 33 on: two row blocks a fragment stream as fast without a tile's idle
+// half (24 rows 1.36 -> 1.41 ms a step with the ring).
+static int ring_model_rows(const ixt_ctx* c, bool decode) { return c->ring_min_rows > 128 ? c->ring_min_rows : std::min(c->ring_min_rows, c->ring_mid_rows + (decode ? 16 : 0)); }
 
 // logits (optional store) + greedy argmax for R rows of normed hidden states
 static int launch_unembed(ixt_ctx* c, const bf16_t* yT, int R, float* logits_out, int32_t* argmax_out, hipStream_t st) {
   const int K = c->E, N = c->V;
-  if (R >= ring_model_rows(c) && c->unembed_gemm) {   // the LDS-ring GEMM with the sampling epilogue
+  if (R >= ring_model_rows(c, true) && c->unembed_gemm) {   // the LDS-ring GEMM with the sampling epilogue
     if ((size_t)R * ((N / 16 + 1) / 2) > c->amax_cap) return set_err(IXT_ERR_INVALID, "argmax workspace too small");   // one pair per row and wave column (>= 2 tiles)
     GemmEpi e{};
     e.out = logits_out; e.amax_val = c->amax_val; e.amax_idx = c->amax_idx; e.cr = c->sample_cols;
@@ -1158,8 +1160,12 @@ static void launch_decode_attn(ixt_ctx* c, int layer, int R, const DotResult& dr
     return;
   }
   const size_t lds = sizeof(float) * ((size_t)GQ * HD + 2 * HD + (size_t)GQ * ((g.Tmax + 3) & ~3) + ((g.mpg + 3) & ~3) + 8 + (size_t)g.nsb_max * HD);
-  if (newtok) hipLaunchKernelGGL((k_attn_decode<HD, GQ, true, true>), dim3(g.nkv, R), dim3(256), lds, st, da);
-  else if (decode) hipLaunchKernelGGL((k_attn_decode<HD, GQ, false, true>), dim3(g.nkv, R), dim3(256), lds, st, da);
+  // streamed past the caches where the launch is bound by the memory's rate: with fewer blocks its latency counts, and that is longer (10.7 -> 12.1 us for 16 blocks,
+  // 3 % of a step at 384 blocks of 12 heads)
+  const bool once = decode && (long)R * g.nkv >= 512;
+  if (newtok && once) hipLaunchKernelGGL((k_attn_decode<HD, GQ, true, true>), dim3(g.nkv, R), dim3(256), lds, st, da);
+  else if (newtok) hipLaunchKernelGGL((k_attn_decode<HD, GQ, true, false>), dim3(g.nkv, R), dim3(256), lds, st, da);
+  else if (once) hipLaunchKernelGGL((k_attn_decode<HD, GQ, false, true>), dim3(g.nkv, R), dim3(256), lds, st, da);
   else hipLaunchKernelGGL((k_attn_decode<HD, GQ, false, false>), dim3(g.nkv, R), dim3(256), lds, st, da);
 }
 
@@ -1429,7 +1435,7 @@ static int forward_rows_gemma2(ixt_ctx* c, int R, const int32_t* tokens, int len
   bf16_t* hcur = c->h_a;
   bf16_t* hnext = c->h_b;
   const bool all_rows = nl == R && lrow0 == 0 && lrows == nullptr;
-  const bool ring = R >= ring_model_rows(c) && !c->fp8;   // QKV and the gate as epilogues of the products
+  const bool ring = R >= ring_model_rows(c, false) && !c->fp8;   // QKV and the gate as epilogues of the products
   const bool attn_tiled = c->gemma_tile && tile_attn_fits(c, R, len_hint, false) && attn_split_factor(c, R) <= 1;
   TRY(launch_rownorm(c, 0, R, tokens, nullptr, nullptr, hcur, c->layers[0].ln1, c->xn, st));
   for (int l = 0; l < c->L; ++l) {
@@ -1509,7 +1515,7 @@ static int forward_rows_gemma2(ixt_ctx* c, int R, const int32_t* tokens, int len
 // decode: one new token per row (rows never read each other's new K).
 //
 // Two launch sequences per layer, same arithmetic:
-//   R >= 17 (ring_model_rows)  LDS-ring GEMMs with fused epilogues (ixt_gemm.h): QKV (+ RoPE, q -> qbuf, K/V -> pages), attention from qbuf
+//   R >= 17, decode rows 33 (ring_model_rows)  LDS-ring GEMMs with fused epilogues (ixt_gemm.h): QKV (+ RoPE, q -> qbuf, K/V -> pages), attention from qbuf
 //                       and the pages, O-proj (+ residual), norm, MLP-up (+ SwiGLU), MLP-down (+ residual), norm: 7 launches, no f32
 //                       slice leaves the chip;
 //   fewer rows          split-K dots into f32 slices: dot_qkv, [front | qkv_finalize + scores], pv, combine, dot_o, rownorm (slice sum
@@ -1712,10 +1718,10 @@ static int forward_rows(ixt_ctx* c, int R, const int32_t* tokens, int len_hint, 
   bf16_t* hcur = c->h_a;
   bf16_t* hnext = c->h_b;
   const bool final_fused = nl == R && lrow0 == 0 && lrows == nullptr;   // decode: every row is unembedded
-  const bool ring = R >= ring_model_rows(c) && !c->moe && !c->fp8;   // fp8: the dots write scaled f32 slices, the bf16 path's row kernels take it from there   // Mixtral: the split-K dots (every expert is a launch sequence of its own)
   const int fused_min = c->attn_fused_min_blocks;
   const size_t fused_lds = sizeof(float) * ((size_t)c->GQ * c->D + 2 * c->D + (size_t)c->GQ * (c->geom.Tmax + 3) + c->geom.mpg + 12 + (size_t)c->geom.nsb_max * c->D);
   const bool attn_one_launch = R * c->KV >= fused_min && fused_lds <= 64 * 1024;
+  const bool ring = R >= ring_model_rows(c, decode) && !c->moe && !c->fp8;   // fp8: the dots write scaled f32 slices, the bf16 path's row kernels take it from there   // Mixtral: the split-K dots (every expert is a launch sequence of its own)
   const bool attn_tiled = tile_attn_fits(c, R, len_hint, decode);   // prefill rows: consecutive rows share their page group's K and V loads
   TRY(launch_rownorm(c, 0, R, tokens, nullptr, nullptr, hcur, c->layers[0].ln1, c->xn, st));
   for (int l = 0; l < c->L; ++l) {
@@ -1731,8 +1737,8 @@ static int forward_rows(ixt_ctx* c, int R, const int32_t* tokens, int len_hint, 
       } else if (attn_one_launch) {
         const DotResult none{0, 0, 0};
         const int ta = decode ? timing_begin(c, st, 0.0, 1) : -1;
-        if (decode && attn_small_fits(c, R)) TRY(launch_attn_small(c, l, R, st));   // (small_attn_max_blocks raised: the 8-wave form with everything in flight)
-        else TRY(launch_attention_fused(c, l, R, none, false, decode, st));   // q from qbuf, every key / value (the new ones too) from the pages
+        // (four waves a block: with more than one block on a CU the eight-wave form is the slower one, 40 rows x 12 heads of 64: 20.3 against 13.7 us)
+        TRY(launch_attention_fused(c, l, R, none, false, decode, st));   // q from qbuf, every key / value (the new ones too) from the pages
         timing_end(c, st, ta);
       } else {
         TRY(launch_attention_partials(c, l, R, len_hint, DotResult{0, 0, 0}, false, st));

@@ -28,9 +28,9 @@ def test_chosen_tile(ctx, R, K, N):
   _dot_case(ctx, H.rand_bf16(rng, (R, K)), H.rand_bf16(rng, (K, N), 0.05))
 
 
-@pytest.mark.parametrize("R", [17, 48, 64, 65, 127])
+@pytest.mark.parametrize("R", [32, 33, 64, 65, 127])
 def test_unembedding_of_some_rows(ctx, R):
-  """17 .. 127 rows: the sampling epilogue on 64-row tiles (rounded logits and the first index of the maximum), a vocabulary that is no multiple of a tile."""
+  """33 .. 127 rows: the sampling epilogue on 64-row tiles (rounded logits and the first index of the maximum), a vocabulary that is no multiple of a tile."""
   torch, O = ctx["torch"], ctx["O"]
   cfg = H.make_config(per_device_batch_size=float(R), pagedattn_num_pages=256, vocab_size=4112)
   w = H.synth.synth_weights(cfg, 3)
