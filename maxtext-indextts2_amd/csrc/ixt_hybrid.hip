@@ -756,12 +756,26 @@ template <> int hdot<bf16_t>(ixt_ctx* c, const bf16_t* x, const HMat& w, int R, 
   *res = Slices{out, dr.slices, dr.slice_stride, w.Np};
   return IXT_OK;
 }
-template <> int hdot<float>(ixt_ctx*, const float* x, const HMat& w, int R, float* out, size_t out_floats, hipStream_t st, Slices* res) {
+// f32: rows in blocks of 16, 32 or 64 (groups: 16), two column tiles a wave where that still gives every CU a block; a slice per 512 k where the whole form
+// leaves CUs without two blocks (2048 columns of 8 rows, K 7168: 32 blocks -> 448)
+static int launch_dot32(const float* x, const HMat& w, size_t wstride, int R, const int32_t* rb, float* out, size_t out_floats, hipStream_t st, Slices* res) {
   if ((size_t)R * w.Np > out_floats) return set_err(IXT_ERR_INVALID, "dot: output workspace too small");
-  hipLaunchKernelGGL(k_dot32, dim3((w.Np + 63) / 64, (R + 15) / 16), dim3(256), 0, st, x, (const float*)w.w, w.Kp, w.Np, R, out, (const int32_t*)nullptr, (size_t)0);
+  const int chains = (w.Kp + 511) / 512, nrb = rb != nullptr || R <= 16 ? 1 : R <= 32 ? 2 : 4;
+  const bool wide = nrb == 4 && (long)((w.Np + 127) / 128) * ((R + 63) / 64) >= 256;
+  dim3 grid((w.Np + (wide ? 127 : 63)) / (wide ? 128 : 64), (R + 16 * nrb - 1) / (16 * nrb), 1);
+  if ((long)grid.x * grid.y < 512 && (size_t)chains * R * w.Np <= out_floats) grid.z = chains;
+#define DOT32(C_, B_, D_) hipLaunchKernelGGL((k_dot32<C_, B_, D_>), grid, dim3(256), 0, st, x, (const float*)w.w, w.Kp, w.Np, R, out, rb, wstride)
+  if (nrb == 1) DOT32(1, 1, 8);
+  else if (nrb == 2) DOT32(1, 2, 8);
+  else if (wide) DOT32(2, 4, 4);
+  else DOT32(1, 4, 4);
+#undef DOT32
   LAUNCHCHK();
-  *res = Slices{out, 1, (size_t)R * w.Np, w.Np};
+  *res = Slices{out, (int)grid.z, (size_t)R * w.Np, w.Np};
   return IXT_OK;
+}
+template <> int hdot<float>(ixt_ctx*, const float* x, const HMat& w, int R, float* out, size_t out_floats, hipStream_t st, Slices* res) {
+  return launch_dot32(x, w, 0, R, nullptr, out, out_floats, st, res);
 }
 // a product of few columns over a long K, some rows: whole-K blocks would leave most of the chip idle, so the reduction is cut into slices (128 x 160 outputs, K
 // 4096: 7 against 16 us; from 1024 rows on the whole form is as fast)
@@ -798,11 +812,7 @@ template <> int hdot_grouped<bf16_t>(ixt_ctx* c, const bf16_t* x, const HMat& w,
   return IXT_OK;
 }
 template <> int hdot_grouped<float>(ixt_ctx*, const float* x, const HMat& w, size_t stride, int rows, int, const int32_t* rb, float* out, size_t out_floats, hipStream_t st, Slices* res) {
-  if ((size_t)rows * w.Np > out_floats) return set_err(IXT_ERR_INVALID, "grouped dot: output workspace too small");
-  hipLaunchKernelGGL(k_dot32, dim3((w.Np + 63) / 64, (rows + 15) / 16), dim3(256), 0, st, x, (const float*)w.w, w.Kp, w.Np, rows, out, rb, stride);
-  LAUNCHCHK();
-  *res = Slices{out, 1, (size_t)rows * w.Np, w.Np};
-  return IXT_OK;
+  return launch_dot32(x, w, stride, rows, rb, out, out_floats, st, res);
 }
 // product with a unit without a gate (from IXT_ACT_RELU2 on) behind it -> act(T) of the down product
 template <typename T> static int hact_unit(ixt_ctx* c, const T* x, const HMat& w, size_t stride, int rows, int group_rows, const int32_t* rb, int kind, const float* par, T* out, hipStream_t st);

@@ -102,36 +102,79 @@ __device__ __forceinline__ float hw_softplus(float z) {
 }
 
 // ---------------------------------------------------------------------------------------------------- f32 dot
-// out[r][n] = sum_k x[r][k] w[n][k], k ascending by fma.  x [R][Kp], w [Np][Kp] row-major f32, Kp % 32 == 0, Np % 16 == 0.  Grouped: 16-row block rb
-// uses the matrix of group rb_exp[rb] (-1: none), wstride floats apart.  grid (ceil(Np / 64), ceil(R / 16)), block 256 (16 rows x 16 column lanes).
-static __global__ __launch_bounds__(256) void k_dot32(const float* __restrict__ x, const float* __restrict__ w, int Kp, int Np, int R, float* __restrict__ out,
-                                               const int32_t* __restrict__ rb_exp, size_t wstride) {
-  __shared__ float xs[16][33], ws[64][33];
-  const int tid = threadIdx.x, n0 = blockIdx.x * 64, r0 = blockIdx.y * 16;
+// out[r][n] = sum_k x[r][k] w[n][k] on the f32 matrix units (16 x 16 x 4: a chain of four fma).  x [R][Kp], w [Np][Kp] row-major f32, Kp % 32 == 0, Np % 16 == 0.
+// A wave owns 16 CB columns and 16 RB rows; a lane's 16 bytes of a row are four k, and product e of a step of 16 takes k = e, 4 + e, 8 + e, 12 + e, so the operands
+// come as they lie in memory.  512 k are one accumulator chain and the chains are added in order, in the wave (grid.z = 1) or as slices by whoever reads them
+// (grid.z = chains): the same sums whatever R, RB and the split are.  D steps of both operands are in flight.
+// What bounds it: few rows the weights (a lane row's 64 bytes a load: 3.7 TB/s; non-temporal loads lose the other half of each line, 5 % slower), many rows the
+// matrix units and the reads of operands (CB = 2 halves those of x: 2434 rows, 14336 columns, K 2048 2482 -> 1826 us, 78 TFLOP/s).  Tiles of 16 x 32 and 64 x 32
+// staged through LDS, one barrier pair per 32 k, on vector units, took 710 us for 2048 columns of 8 rows, K 2048 and 7168: now 10 and 17.
+// Grouped: 16-row block rb uses the matrix of group rb_exp[rb] (-1: none), wstride floats apart; RB = 1.
+// grid (ceil(Np / (64 CB)), ceil(R / (16 RB)), chains or 1), block 256.
+template <int CB, int RB, int D>
+static __global__ __launch_bounds__(256, 2) void k_dot32(const float* __restrict__ x, const float* __restrict__ w, int Kp, int Np, int R, float* __restrict__ out,
+                                                  const int32_t* __restrict__ rb_exp, size_t wstride) {
+  static_assert(32 % D == 0, "chains end with a group of steps");
+  typedef float f4 __attribute__((ext_vector_type(4)));
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, i16 = lane & 15, lg = lane >> 4;
+  const int n0 = (blockIdx.x * 4 + wave) * 16 * CB, r0 = blockIdx.y * 16 * RB;
+  if (n0 >= Np) return;
   if (rb_exp != nullptr) {
     const int ex = rb_exp[blockIdx.y];
     if (ex < 0) return;
     w += (size_t)ex * wstride;
   }
-  const int tr = tid >> 4, tc = tid & 15;
-  float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-  for (int k0 = 0; k0 < Kp; k0 += 32) {
-    for (int i = tid; i < 16 * 32; i += 256) xs[i >> 5][i & 31] = (r0 + (i >> 5) < R) ? x[(size_t)(r0 + (i >> 5)) * Kp + k0 + (i & 31)] : 0.0f;
-    for (int i = tid; i < 64 * 32; i += 256) ws[i >> 5][i & 31] = (n0 + (i >> 5) < Np) ? w[(size_t)(n0 + (i >> 5)) * Kp + k0 + (i & 31)] : 0.0f;
-    __syncthreads();
-#pragma unroll 8
-    for (int k = 0; k < 32; ++k) {
-      const float xv = xs[tr][k];
+  const int steps = Kp >> 4, s0 = gridDim.z > 1 ? blockIdx.z * 32 : 0, s1 = gridDim.z > 1 ? min(steps, s0 + 32) : steps;
+  const float *wp[CB], *xp[RB];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) acc[j] = fmaf(xv, ws[tc + 16 * j][k], acc[j]);
+  for (int i = 0; i < CB; ++i) wp[i] = w + (size_t)min(n0 + i * 16 + i16, Np - 1) * Kp + 4 * lg;
+#pragma unroll
+  for (int b = 0; b < RB; ++b) xp[b] = x + (size_t)min(r0 + b * 16 + i16, R - 1) * Kp + 4 * lg;
+  f4 wv[D][CB], xv[D][RB], acc[CB][RB], tot[CB][RB];
+  auto fetch = [&](int d, int s) {
+    const int at = min(s, s1 - 1) * 16;
+#pragma unroll
+    for (int i = 0; i < CB; ++i) wv[d][i] = *reinterpret_cast<const f4*>(wp[i] + at);
+#pragma unroll
+    for (int b = 0; b < RB; ++b) xv[d][b] = *reinterpret_cast<const f4*>(xp[b] + at);
+  };
+#pragma unroll
+  for (int d = 0; d < D; ++d) fetch(d, s0 + d);
+#pragma unroll
+  for (int i = 0; i < CB; ++i)
+#pragma unroll
+    for (int b = 0; b < RB; ++b) acc[i][b] = f4(0.0f);
+  bool first = true;
+  for (int s = s0; s < s1; s += D) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      if (s + d < s1) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int i = 0; i < CB; ++i)
+#pragma unroll
+            for (int b = 0; b < RB; ++b) acc[i][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[d][i][e], xv[d][b][e], acc[i][b], 0, 0, 0);
+      }
+      fetch(d, s + D + d);
+      __builtin_amdgcn_sched_barrier(0);
     }
-    __syncthreads();
-  }
-  if (r0 + tr < R) {
+    if (((s + D) & 31) == 0 || s + D >= s1) {              // a chain is complete
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-      if (n0 + tc + 16 * j < Np) out[(size_t)(r0 + tr) * Np + n0 + tc + 16 * j] = acc[j];
+      for (int i = 0; i < CB; ++i)
+#pragma unroll
+        for (int b = 0; b < RB; ++b) { tot[i][b] = first ? acc[i][b] : tot[i][b] + acc[i][b]; acc[i][b] = f4(0.0f); }
+      first = false;
+    }
   }
+  out += (size_t)blockIdx.z * R * Np;
+#pragma unroll
+  for (int i = 0; i < CB; ++i)
+#pragma unroll
+    for (int b = 0; b < RB; ++b) {
+      const int r = r0 + b * 16 + i16;                     // lane: row, columns 4 lg ..
+      if (r < R && n0 + i * 16 < Np) *reinterpret_cast<f4*>(out + (size_t)r * Np + n0 + i * 16 + 4 * lg) = tot[i][b];
+    }
 }
 
 // ---------------------------------------------------------------------------------------------------- weights
