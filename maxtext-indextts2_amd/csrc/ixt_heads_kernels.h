@@ -151,9 +151,7 @@ __global__ __launch_bounds__(256) void k_heads_any(const T* __restrict__ qb, Hea
       float s = -INFINITY;
       if (j <= pos) {
         const T* kp = kpages + (((size_t)prow[j / g.P] * g.G + kh) * g.P + j % g.P) * g.dkp + mi * g.dmp;
-        float a = 0.0f;
-        for (int k = 0; k < g.d; ++k) a = fmaf(qm[k], to_f(kp[k]), a);
-        s = a * g.scale;
+        s = key_dot(qm, kp, g.d) * g.scale;
         if (g.cap > 0.0f) s = g.cap * tanhf(s / g.cap);
       }
       float tm = s;
@@ -172,13 +170,7 @@ __global__ __launch_bounds__(256) void k_heads_any(const T* __restrict__ qb, Hea
       const int nk = min(256, pos - j0 + 1);
 #pragma unroll
       for (int i = 0; i < 4; ++i) acc[i] *= al;
-      for (int kk = 0; kk < nk; ++kk) {
-        const T* vp = vpages + (((size_t)prow[(j0 + kk) / g.P] * g.G + kh) * g.P + (j0 + kk) % g.P) * g.dvp;
-        const float w = p[kk];
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (tid + 256 * i < g.dv) acc[i] = fmaf(w, to_f(vp[tid + 256 * i]), acc[i]);
-      }
+      weighted_rows(p, nk, g.dv, acc, [&](int kk) { return vpages + (((size_t)prow[(j0 + kk) / g.P] * g.G + kh) * g.P + (j0 + kk) % g.P) * g.dvp; });
       __syncthreads();
     }
     const float f = mi == 0 ? 1.0f / l : -*mp.lambda / l;
