@@ -138,6 +138,23 @@ __device__ __forceinline__ float tanh_f32(float x) {
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
+// LDS-DMA by hand: 16 bytes a lane from memory to LDS, lane l's to byte `dst` + 16 l (dst uniform, it goes through M0).  No register is written, and the kernels
+// count the waits themselves: behind the builtin the compiler waits for every fetch in flight ahead of an LDS read that it cannot tell from their targets.
+// A write of M0 has to stand one wait state in front of a fetch that uses it (the compiler puts this s_nop there for the builtin, but does not look into
+// asm), and M0 is named as overwritten: otherwise a fetch of the compiler's own may go to the slot of this one.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"          // (M0 is a reserved register: the compiler keeps nothing in it across this)
+#define IXT_LDS_DMA "s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 "
+// from base + off, base uniform; ONCE: past the caches
+template <bool ONCE = false> __device__ __forceinline__ void lds_dma16(uint32_t dst, const void* base, uint32_t off) {
+  if constexpr (ONCE) asm volatile(IXT_LDS_DMA "%1, %2 nt" ::"s"(dst), "v"(off), "s"(base) : "memory", "m0");
+  else asm volatile(IXT_LDS_DMA "%1, %2" ::"s"(dst), "v"(off), "s"(base) : "memory", "m0");
+}
+// from a lane's own address
+__device__ __forceinline__ void lds_dma16(uint32_t dst, const void* src) { asm volatile(IXT_LDS_DMA "%1, off" ::"s"(dst), "v"(src) : "memory", "m0"); }
+#undef IXT_LDS_DMA
+#pragma clang diagnostic pop
+
 // agent-scope (L1-bypassing) accesses for state one wave re-reads after writing it
 __device__ __forceinline__ int ldg_i32(const int32_t* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ __forceinline__ void stg_i32(int32_t* p, int v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }

@@ -162,16 +162,13 @@ __global__ __launch_bounds__(WR * WC * 64, 2) void k_gemm_ring(const u32x4* __re
   const char* pw = reinterpret_cast<const char*>(wt + (wring ? r8frag(colg * TC, 0, nsteps) : (size_t)colg * TC * nsteps) * 64) + chb * wadv;
   const char* px = reinterpret_cast<const char*>(xt + (size_t)rowg * TR * nsteps * 64) + (size_t)chb * KS * 1024;
   const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)((__attribute__((address_space(3))) u32x4*)st));
-  // piece j of the next chunk to fetch, into a slot.  Issued by hand (no register is written, nothing else in this kernel uses m0): behind the builtin the
-  // compiler may wait for every fetch in flight before an LDS read; the waits are counted in the loop.  ONCE (one row group): no other block reads these
-  // weights, so they are streamed past the caches (264192 columns, K 2048: 48 rows 219 -> 203 us, 256 rows 386 -> 359; several row groups of small tiles lose
+  // piece j of the next chunk to fetch, into a slot; the waits are counted in the loop.  ONCE (one row group): no other block reads these weights, so they are streamed past the caches (264192 columns, K 2048: 48 rows 219 -> 203 us, 256 rows 386 -> 359; several row groups of small tiles lose
   // by it, and a branch here instead of a second kernel costs them up to 10 %).
   auto issue = [&](int slot, int j) {
     const uint32_t dst = lds0 + (uint32_t)(slot * NF + wave + NW * j) * 1024u;
     if (NW * j >= NWF || (NW * j + NW > NWF && wave + NW * j >= NWF))
-      asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(off[j]), "s"(px) : "memory");
-    else if constexpr (ONCE) asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(dst), "v"(off[j]), "s"(pw) : "memory");
-    else asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(off[j]), "s"(pw) : "memory");
+      lds_dma16(dst, px, off[j]);
+    else lds_dma16<ONCE>(dst, pw, off[j]);
   };
   auto advance = [&]() { pw += wadv; px += (size_t)KS * 1024; };
 #pragma unroll

@@ -113,20 +113,18 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void k_tgemm(TGemm g) {
   auto next_chunk = [&]() {                                               // past the last chunk: zeros, so that the counts stay
     whole = segk + 32 <= segend;
   };
-  // Issued by hand (nothing else in this kernel uses m0): the builtin makes the compiler wait for every fetch in flight ahead of a transposed LDS read.  (No register is written; the waits
-  // are counted in the loop.)
   const uint32_t lds0 = (uint32_t)(uintptr_t)((__attribute__((address_space(3))) bf16_t*)lds);
-  auto issue = [&](int slot, int j) {                                     // piece j of this wave's share of the next chunk
+  auto issue = [&](int slot, int j) {                                     // piece j of this wave's share of the next chunk; the waits are counted in the loop
     const bool isa = j * NW < NA;
     const uint32_t dst = __builtin_amdgcn_readfirstlane(lds0 + (uint32_t)(slot * SLOT + (wave + NW * j) * 512) * 2u);
     if (whole) {
-      asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(off[j]), "s"(isa ? pa : pb) : "memory");
+      lds_dma16(dst, isa ? pa : pb, off[j]);
     } else {
       const char* p = (isa ? pa : pb) + off[j];
       int k, x;
       place(isa ? TA : TB, isa ? BM : BN, isa ? wave + NW * j : wave + NW * j - NA, k, x);
       if (segk + k >= segend) p = reinterpret_cast<const char*>(tg_zero);
-      asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(dst), "v"(p) : "memory");
+      lds_dma16(dst, p);
     }
   };
   auto advance = [&]() {
