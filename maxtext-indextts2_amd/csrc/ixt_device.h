@@ -154,6 +154,12 @@ template <bool ONCE = false> __device__ __forceinline__ void lds_dma16(uint32_t 
 __device__ __forceinline__ void lds_dma16(uint32_t dst, const void* src) { asm volatile(IXT_LDS_DMA "%1, off" ::"s"(dst), "v"(src) : "memory", "m0"); }
 #undef IXT_LDS_DMA
 #pragma clang diagnostic pop
+// barrier of a block behind which LDS is read that such fetches (or other waves) filled.  The builtin orders nothing for the compiler, which does not see
+// the fetches write: without the fence a read may move in front of it.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
 
 // agent-scope (L1-bypassing) accesses for state one wave re-reads after writing it
 __device__ __forceinline__ int ldg_i32(const int32_t* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }

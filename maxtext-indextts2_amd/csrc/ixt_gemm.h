@@ -187,8 +187,7 @@ __global__ __launch_bounds__(WR * WC * 64, 2) void k_gemm_ring(const u32x4* __re
   auto wfrag = [&](int slot, int ks, int i) { return __builtin_bit_cast(bf16x8, st[(slot * NF + (wc * CT + i) * KS + ks) * 64 + lane]); };
   auto xfrag = [&](int slot, int ks, int b) { return __builtin_bit_cast(bf16x8, st[(slot * NF + NWF + (wr * RB + b) * KS + ks) * 64 + lane]); };
   ring_wait_chunks<NJ, NS - 1>(che - chb - 1);                  // chunk chb
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
+  lds_barrier();
 #pragma unroll
   for (int b = 0; b < RB; ++b) xf[0][b] = xfrag(0, 0, b);
 #pragma unroll
@@ -204,8 +203,7 @@ __global__ __launch_bounds__(WR * WC * 64, 2) void k_gemm_ring(const u32x4* __re
     const bool last = ks == KS - 1;
     if (last) {
       ring_wait_chunks<NJ, NS - 2>(che - ch - 2);
-      __builtin_amdgcn_s_barrier();
-      asm volatile("" ::: "memory");
+      lds_barrier();
       refill = ch + NS < che;
       fill = slot;
       slot = slot + 1 == NS ? 0 : slot + 1;

@@ -171,7 +171,7 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void k_tgemm(TGemm g) {
     advance();
   }
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 1) * NJ) : "memory");
-  __builtin_amdgcn_s_barrier();
+  lds_barrier();
 #pragma unroll
   for (int j = 0; j < NI; ++j) fb[0][j] = row_b(0, j);
 #pragma unroll
@@ -180,8 +180,7 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void k_tgemm(TGemm g) {
     // chunk c + 1 has landed once the (NS - 2) younger ones are all that is outstanding; this wave's reads of chunk c are done, so behind the
     // barrier its slot can be filled again
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((NS - 2) * NJ) : "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
+    lds_barrier();
     next_chunk();
     const int nxt = (c + 1) % NS, old = c % NS;
     // a row of products, then a share of the reads of chunk c + 1 and of the fetches of chunk c + NS: they ride under the products

@@ -68,3 +68,11 @@ def test_wait_states(source, tmp_path):
   assert "inline-asm" not in done.stderr
   fetches, m0, address = _distances(out.read_text())
   assert fetches > 20 and m0 is not None and m0 >= 1 and address >= 5, (fetches, m0, address)
+
+
+def test_barriers_order_the_reads_behind_them():
+  """The barrier builtin is no memory operation to the compiler: kernels use lds_barrier, which adds the fence."""
+  bare = [n for n in sorted(os.listdir(build.CSRC)) if n != "ixt_device.h" and "__builtin_amdgcn_s_barrier" in open(os.path.join(build.CSRC, n), encoding="utf-8").read()]
+  with open(os.path.join(build.CSRC, "ixt_device.h"), encoding="utf-8") as f:
+    body = re.search(r"void lds_barrier\(\) \{(.*?)\n\}", f.read(), re.S)
+  assert bare == [] and body and re.search(r's_barrier\(\);\s*asm volatile\("" ::: "memory"\);', body[1])
