@@ -298,7 +298,7 @@ extern "C" int ixt_create(const ixt_config* cfg, ixt_ctx** out) {
   }
   A(dmalloc(x, &x->scores, (size_t)R * x->Q * x->Tmax));
   A(dmalloc(x, &x->pvpart, (size_t)R * x->Q * x->nsb_max * x->D));
-  x->amax_cap = (size_t)x->NLmax * ((V + 15) / 16);
+  x->amax_cap = (size_t)x->NLmax * std::max(4, (V + 15) / 16);   // (ring_pairs)
   A(dmalloc(x, &x->amax_val, x->amax_cap));
   A(dmalloc(x, &x->amax_idx, x->amax_cap));
   {
@@ -720,6 +720,12 @@ static int ring_pick(const ixt_ctx* c, int epi, int R, int N, bool routed, bool 
   return best;
 }
 
+// (max, index) pairs that an unembedding with this tile leaves of a row: one a wave column of whole column groups (4 even of a vocabulary of 16 columns)
+static size_t ring_pairs(int cfg, int N) {
+  const int n = N / 16;
+  return cfg == 1 || cfg == 7 ? (n + 7) / 8 * 4 : cfg == 4 ? (n + 7) / 8 * 2 : (n + 3) / 4 * 2;
+}
+
 template <int WR, int WC, int RB, int CT, int KS, int NS, int EPI, int SPLIT, bool ONCE>
 static int ring_launch_o(const bf16_t* x, const bf16_t* w, int K, int N, int R, int chains, int wring, const GemmEpi& e, hipStream_t st, int* wave_cols) {
   constexpr int TC = WC * CT, TR = WR * RB;
@@ -753,6 +759,7 @@ int launch_ring(ixt_ctx* c, int epi, const bf16_t* x, const bf16_t* w, int K, in
   if (K % IXT_KALIGN || N % 16) return set_err(IXT_ERR_UNSUPPORTED, "ring gemm: K %% 128 or N %% 16");
   const int chains = (K + IXT_CHAIN - 1) / IXT_CHAIN;
   const int cfg = ring_pick(c, epi, R, N, e.rb_exp != nullptr, wring != 0);
+  if (epi == GEPI_UNEMBED && (size_t)R * ring_pairs(cfg, N) > c->amax_cap) return set_err(IXT_ERR_INVALID, "argmax workspace too small");
   double ebytes = 0.0;
   switch (epi) {
     case GEPI_F32: ebytes = (double)(split ? chains : 1) * R * N * 4.0; break;
@@ -1004,7 +1011,6 @@ static int ring_model_rows(const ixt_ctx* c, bool decode) { return c->ring_min_r
 static int launch_unembed(ixt_ctx* c, const bf16_t* yT, int R, float* logits_out, int32_t* argmax_out, hipStream_t st) {
   const int K = c->E, N = c->V;
   if (R >= ring_model_rows(c, true) && c->unembed_gemm) {   // the LDS-ring GEMM with the sampling epilogue
-    if ((size_t)R * ((N / 16 + 1) / 2) > c->amax_cap) return set_err(IXT_ERR_INVALID, "argmax workspace too small");   // one pair per row and wave column (>= 2 tiles)
     GemmEpi e{};
     e.out = logits_out; e.amax_val = c->amax_val; e.amax_idx = c->amax_idx; e.cr = c->sample_cols;
     int wave_cols = 0;

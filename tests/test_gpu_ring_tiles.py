@@ -28,14 +28,15 @@ def test_chosen_tile(ctx, R, K, N):
   _dot_case(ctx, H.rand_bf16(rng, (R, K)), H.rand_bf16(rng, (K, N), 0.05))
 
 
-@pytest.mark.parametrize("R", [32, 33, 64, 65, 127])
-def test_unembedding_of_some_rows(ctx, R):
-  """33 .. 127 rows: the sampling epilogue on 64-row tiles (rounded logits and the first index of the maximum), a vocabulary that is no multiple of a tile."""
+@pytest.mark.parametrize("R,V", [(32, 4112), (33, 4112), (64, 4112), (65, 4112), (127, 4112), (40, 16), (130, 16), (130, 48), (40, 80), (130, 144)])
+def test_unembedding_of_some_rows(ctx, R, V):
+  """33 rows and more: the sampling epilogue on 64-row tiles (rounded logits and the first index of the maximum), a vocabulary that is no multiple of a
+  tile, down to one that ends inside the first column group (its pairs of maximum and index are those of a whole one)."""
   torch, O = ctx["torch"], ctx["O"]
-  cfg = H.make_config(per_device_batch_size=float(R), pagedattn_num_pages=256, vocab_size=4112)
+  cfg = H.make_config(per_device_batch_size=float(R), pagedattn_num_pages=256, vocab_size=V)
   w = H.synth.synth_weights(cfg, 3)
   eng, _ = H.make_engine(cfg, w)
-  E, V = cfg.emb_dim, cfg.vocab_size
+  E = cfg.emb_dim
   y = H.rand_bf16(np.random.default_rng(R), (R, E))
   lg = np.zeros((R, V), np.float32)
   wl = w["params/decoder/logits_dense/kernel"].reshape(E, V)
