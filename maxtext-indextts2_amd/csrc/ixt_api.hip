@@ -1743,8 +1743,10 @@ static int forward_rows(ixt_ctx* c, int R, const int32_t* tokens, int len_hint, 
       } else if (attn_one_launch) {
         const DotResult none{0, 0, 0};
         const int ta = decode ? timing_begin(c, st, 0.0, 1) : -1;
-        // (four waves a block: with more than one block on a CU the eight-wave form is the slower one, 40 rows x 12 heads of 64: 20.3 against 13.7 us)
-        TRY(launch_attention_fused(c, l, R, none, false, decode, st));   // q from qbuf, every key / value (the new ones too) from the pages
+        // at most one block on a CU: eight waves with everything in flight (128 rows x 1 kv head of two query heads of 128, 1500 keys: 421 us a step of four layers with
+        // four waves, 351 with eight; 700 keys 302 -> 260; 64 keys 231 -> 229); with more the four-wave form is the faster one (40 rows x 12 heads of 64: 20.3 against 13.7 us)
+        if (decode && (long)R * c->KV <= c->small_attn_max_blocks / 2 && attn_small_fits(c, R)) TRY(launch_attn_small(c, l, R, st));
+        else TRY(launch_attention_fused(c, l, R, none, false, decode, st));   // q from qbuf, every key / value (the new ones too) from the pages
         timing_end(c, st, ta);
       } else {
         TRY(launch_attention_partials(c, l, R, len_hint, DotResult{0, 0, 0}, false, st));

@@ -106,7 +106,8 @@ struct ixt_ctx {
   int attn_tile_min_rows = 64;
   int attn_wave_pairs = 0;   // measured at 256 rows, 765 keys: 339 us per launch (4.7 TB/s) against 305 us (5.3 TB/s) for the block form
   // few rows (one row block): five launches per layer (ixt_small.h).  small_rows: most rows of that path (0: off); small_tpb: column tiles per
-  // block of k_sdot (0: by shape); small_attn_waves: waves per (row, kv head) block of k_attn_small (4: k_attn_decode instead)
+  // block of k_sdot (0: by shape); small_attn_waves: waves per (row, kv head) block of k_attn_small (4: k_attn_decode instead);
+  // small_attn_max_blocks: most (row, kv head) pairs for it, half as many on the ring path
   int small_rows = 16, small_tpb = 0, small_attn_waves = 16, small_attn_max_blocks = 512;
   int dot_small = 0;         // ixt_op_dot through k_sdot where it fits (tests)
   // few rows: the keys of a (row, kv head) split over `S` blocks of k_attn_split (S = min(small_attn_split, 256 / (rows * kv heads)); < 2: k_attn_small)
