@@ -19,3 +19,13 @@ def test_steps_of_few_kv_heads(rows, kv, heads, dim):
   eight = run_pair(cfg, w, prompts, steps=4)
   four = run_pair(cfg, w, prompts, steps=4, options={"small_attn_max_blocks": 0})
   assert np.array_equal(eight, four)
+
+
+@pytest.mark.parametrize("rows,dim", [(63, 64), (65, 256)])
+def test_steps_of_capped_rows(rows, dim):
+  """Gemma-2 decode rows on both sides of the tiled attention's first row: every row has pages of its own, so the per-row kernels serve them."""
+  cfg = H.make_config("gemma2-tiny", per_device_batch_size=float(rows), head_dim=dim, max_prefill_predict_length=48, max_target_length=64, pagedattn_num_pages=2 * rows + 2,
+                      pagedattn_tokens_per_page=32, sliding_window_size=24, base_num_decoder_layers=1)
+  w = H.synth.synth_weights(cfg, rows)
+  prompts = [(H.synth.synth_prompt(cfg.vocab_size, 48, i)[0], 1 + (29 * i) % 48) for i in range(rows)]
+  run_pair(cfg, w, prompts, steps=4)
