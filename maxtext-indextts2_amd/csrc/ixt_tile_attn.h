@@ -46,8 +46,9 @@ __device__ __forceinline__ void ixt_k_operands(const u32x4& w, uint32_t sel, flo
 //   columns of one token: column 8 i + x belongs to row i of tile x.  Page chains start from zero, four pages add up in order; the super-blocks of a
 //   round meet in LDS, where the thread that owns (vector, column) adds them in order.
 // A key that a row does not see has P = +0 (k_attn_tile says why that is exact); tokens past the end are re-reads of the last one.
-// Rows of other page groups in the tile are worked off group by group.  grid = (kv heads, tiles, 1 or the number of 128-column parts of a value):
-// with z = 2 the two halves of head_dim 256 go to two blocks, each taking the scores anew -- for launches that leave CUs idle otherwise.
+// Rows of other page groups in the tile are worked off group by group, dealt among `shares` blocks.  grid = (kv heads, tiles, parts x shares): parts = 1 or
+// the number of 128-column parts of a value (the two halves of head_dim 256 in two blocks, each taking the scores anew), shares = 1 or more, both for
+// launches that leave CUs idle otherwise.
 // Bound by the matrix units and, between their phases, by the vector work of the softmax (a block's waves are in the same phase).  Measured against
 // k_attn_tile, 16 heads of 128: 8 packed prompts (1525 rows, <= 251 keys) 128.6 -> 69.6 us; 1024 rows at <= 1024 / 2048 / 3072 keys 282 -> 106,
 // 860 -> 215, 1143 -> 356 us; 828 rows at <= 3900 keys 1496 -> 455 us (52 TFLOP/s).  8 heads of 256 on 4, 256 rows at <= 3072 keys: 320 -> 130 us.
@@ -69,6 +70,7 @@ __global__ __launch_bounds__(NW * 64, NR == 1 && NW <= 4 ? 3 : 2) void k_attn_mt
   const AttnGeom& g = a.g;
   const int kvh = blockIdx.x, r0 = (gridDim.y - 1 - blockIdx.y) * TQ;    // the rows with the most keys first
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, i16 = lane & 15, lg = lane >> 4;
+  const int part0 = blockIdx.z % a.parts, share = blockIdx.z / a.parts, shares = gridDim.z / a.parts;
   const int n_out = g.nq * HD;
   if (tid < TQ) {
     const int r = r0 + tid;
@@ -96,6 +98,7 @@ __global__ __launch_bounds__(NW * 64, NR == 1 && NW <= 4 ? 3 : 2) void k_attn_mt
     }
   }
   const uint32_t sel = (lg & 1) ? 0x07060c0cu : 0x05040c0cu;
+  int turn = 0;                                          // whose group comes next
   while (pending != 0) {
     // the rows of the leader's page group
     const int lead = __builtin_ctz(pending);
@@ -115,6 +118,9 @@ __global__ __launch_bounds__(NW * 64, NR == 1 && NW <= 4 ? 3 : 2) void k_attn_mt
       continue;
     }
     pending &= ~grp;
+    const bool mine = turn == share;
+    turn = turn + 1 == shares ? 0 : turn + 1;
+    if (!mine) continue;
     const int kv_all = posmax + 1, pages_all = (kv_all + 31) >> 5, nsb = (pages_all + IXT_SB - 1) / IXT_SB;
     const int32_t* prow = a.page_map + (size_t)slot * g.mpg;
     const int mypos = ((grp >> (i16 / GQ)) & 1u) ? s_pos[i16 / GQ] : -1;
@@ -239,7 +245,7 @@ __global__ __launch_bounds__(NW * 64, NR == 1 && NW <= 4 ? 3 : 2) void k_attn_mt
       return __builtin_fmaf(__builtin_fmaf(-q, l, e), rl, q);
     });
     // ---- outputs
-    for (int part = blockIdx.z; part < HD / VW; part += gridDim.z) {
+    for (int part = part0; part < HD / VW; part += a.parts) {
       float tot[2][NTOT];
 #pragma unroll
       for (int k = 0; k < NTOT; ++k) { tot[0][k] = 0.0f; tot[1][k] = 0.0f; }

@@ -1,12 +1,18 @@
 // ixt_tile_attn.hip -- launches of k_attn_mtile (an object of its own: it compiles beside the others).
 #include "ixt_tile_attn.h"
 
+#include <algorithm>
+
 // The smallest form that holds the call's longest prefix (ta.lmax keys, at most 4096).
 template <int HD, int GQ>
-static void mtile_attn_t(const TileAttnArgs& ta, hipStream_t st) {
+static void mtile_attn_t(TileAttnArgs ta, hipStream_t st) {
   constexpr int TQ = 16 / GQ;
-  const int tiles = (ta.R + TQ - 1) / TQ;
-  const dim3 grid(ta.g.nkv, tiles, HD > 128 && ta.g.nkv * tiles <= 128 ? HD / 128 : 1);   // half of the CUs idle: the halves of a value side by side
+  const int tiles = (ta.R + TQ - 1) / TQ, blocks = ta.g.nkv * tiles;
+  // half of the CUs idle: the halves of a value side by side; still half of them: the page groups of a tile, too.  A tile of a prompt has one, and the other blocks
+  // end at once (64 and 100 rows: the same time); one of a mixed step's decoded tokens has up to TQ, and one behind the other 64 rows at 128 keys with heads of 256
+  // took 2.40 ms a step of four sub-layers (per-vector units: 2.35), dealt out 1.84; 16 heads of 128, four layers: 64 keys 2.45 -> 1.77, 1500 keys 4.50 -> 2.58
+  ta.parts = HD > 128 && blocks <= 128 ? HD / 128 : 1;
+  const dim3 grid(ta.g.nkv, tiles, ta.parts * std::min(TQ, std::max(1, 256 / (blocks * ta.parts))));
   if (ta.lmax <= 256) hipLaunchKernelGGL((k_attn_mtile<HD, GQ, 2, 1>), grid, dim3(128), 0, st, ta);
   else if (ta.lmax <= 512) hipLaunchKernelGGL((k_attn_mtile<HD, GQ, 4, 1>), grid, dim3(256), 0, st, ta);
   else if (ta.lmax <= 1024) hipLaunchKernelGGL((k_attn_mtile<HD, GQ, 8, 1>), grid, dim3(512), 0, st, ta);

@@ -47,3 +47,36 @@ def test_matrix_tile_with_cap_and_window(hd, nq, nkv, window):
   a = _prefill_long(cfg, w, toks, 250, {"gemma_tile": 1, "attn_tile_min_rows": 1})
   b = _prefill_long(cfg, w, toks, 250, {"gemma_tile": 0})
   _same(a, b)
+
+
+@pytest.mark.parametrize("model,hd,nq,nkv", [("ixt-tiny", 64, 4, 2), ("ixt-tiny", 128, 8, 8), ("gemma2-tiny", 256, 4, 2)])
+@pytest.mark.parametrize("portion", [2, 40])
+def test_rows_of_many_page_groups(model, hd, nq, nkv, portion):
+  """One mixed step: 62 rows that continue sequences of their own (up to as many page groups in a tile as it has rows, dealt among blocks where CUs are idle)
+  and a portion of a prompt; logits, tokens and new K/V against the per-row kernels."""
+  import torch
+  slots, longest = 63, 300
+  cfg = H.make_config(model, per_device_batch_size=float(slots), head_dim=hd, base_num_query_heads=nq, base_num_kv_heads=nkv, base_num_decoder_layers=1,
+                      max_prefill_predict_length=longest, max_target_length=longest + 64, pagedattn_tokens_per_page=32, pagedattn_num_pages=slots * 12 + 1)
+  w = H.synth.synth_weights(cfg, 31)
+  rng = np.random.default_rng(portion)
+  lens = [int(n) for n in rng.integers(1, longest, slots)]
+  toks = [rng.integers(1, cfg.vocab_size, n + 64).astype(np.int32) for n in lens]
+
+  def step(options):
+    eng, params = H.make_engine(cfg, w)
+    for name, value in options.items():
+      H.lib.check(eng.lib.ixt_set_option(eng._ctx, name.encode(), value))
+    for slot, n in enumerate(lens):
+      eng.prefill(params=params, padded_tokens=toks[slot][:n], true_length=n, slot=slot)
+    entries = [(slot, n, toks[slot][n:n + 1], [0]) for slot, n in enumerate(lens[:-1])]
+    entries.append((slots - 1, lens[-1], toks[-1][lens[-1]:lens[-1] + portion], [portion - 1]))
+    logits, first = eng.step(entries)
+    kv = [H.bits(t).copy() for slot in (0, 7, slots - 1) for t in eng.gather_kv(0, slot, lens[slot] + 1)]
+    out = logits.cpu().numpy().view(np.uint32), first.cpu().numpy(), kv
+    torch.cuda.synchronize()
+    return out
+
+  a, b = step({"attn_tile_min_rows": 1}), step({"attn_tile": 0})
+  assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1])
+  assert all(np.array_equal(x, y) for x, y in zip(a[2], b[2]))
