@@ -51,9 +51,11 @@ struct ixt_trainer {
   bf16_t* pb = nullptr;   // bf16 copies of the parameters (owned here)
   // offsets
   long o_emb, o_fnorm, o_logits;
-  // Rows of the vocabulary (bf16 copy of the logits kernel, the last parameter; logits and their gradients) lie Vp apart: V + 64.  Where 2 V bytes is an odd
-  // multiple of some power of two (264192: 129 x 2^12), the 256 rows a tile fetches side by side lie in few memory channels, and the product whose reduction
-  // runs along them took 3.30 ms a chunk of 2048 rows (0.67 PFLOP/s); 128 bytes more a row: 1.72 (1.29; only one of the two operands: 2.9)
+  // Rows of the vocabulary (bf16 copy of the logits kernel, the last parameter; logits and their gradients) lie Vp apart: an odd number of 128-byte lines, V or V + 64
+  // columns.  With 127 or 129 times 2^12 bytes the 256 rows a tile fetches side by side lie in few memory channels: the product whose reduction runs along them
+  // took 3.30 ms a chunk of 2048 rows of 264192 columns (0.67 PFLOP/s), one line further apart 1.72 (1.29; only one of the two operands: 2.9).  A whole step,
+  // one layer of 2048, 4096 tokens: 264192 columns 25.6 -> 22.5 ms, 260096 24.8 -> 23.6; where V is an odd number of lines already, 64 more make it worse
+  // (131008, then rows of 2^18 bytes: 12.91 -> 13.11 ms; 262080 24.09 -> 24.32); every other of 40 vocabularies, 16384 to 280576, is the same within 1.5 %
   long Vp;
   struct LOff { long ln1, wq, wk, wv, wo, ln2, wi0, wi1, wout; };
   std::vector<LOff> lo;
@@ -100,7 +102,7 @@ extern "C" int ixt_train_create(const ixt_train_config* c, ixt_trainer** out) {
   t->KVH = c->num_kv_heads; t->G = t->H / t->KVH; t->KN = t->KVH * t->D;
   t->Tc = c->logits_chunk > 0 ? c->logits_chunk : 2048;
   if (t->Tc > t->T) t->Tc = t->T;
-  t->Vp = t->V >= 4096 ? t->V + 64 : t->V;
+  t->Vp = t->V >= 4096 && (t->V + 32) / 64 % 2 == 0 ? t->V + 64 : t->V;
   const long E = t->E, F = t->F, V = t->V, QN = t->QN, KN = t->KN;
   add_param(t, "params/token_embedder/embedding", V * E, &t->o_emb);
   t->lo.resize(t->L);

@@ -16,6 +16,8 @@ SHAPES = {
     "large tiles": dict(base_emb_dim=72, base_num_query_heads=2, base_num_kv_heads=2, head_dim=64, base_mlp_dim=136, vocab_size=6152, max_target_length=688, per_device_batch_size=3.0),
     # reductions cut in parts, the last part shorter; groups of query heads
     "cut reductions": dict(base_emb_dim=264, base_num_query_heads=4, base_num_kv_heads=2, head_dim=128, base_mlp_dim=520, vocab_size=4104, max_target_length=712, per_device_batch_size=3.0),
+    # a vocabulary of an odd number of 128-byte lines: its rows lie as far apart as they are long, also from 4096 columns on
+    "odd lines": dict(base_emb_dim=72, base_num_query_heads=2, base_num_kv_heads=2, head_dim=64, base_mlp_dim=136, vocab_size=4160, max_target_length=72, per_device_batch_size=2.0),
     # one row, shorter than any tile
     "short": dict(base_emb_dim=64, base_num_query_heads=2, base_num_kv_heads=1, head_dim=64, base_mlp_dim=72, vocab_size=264, max_target_length=8, per_device_batch_size=1.0),
 }
