@@ -90,15 +90,16 @@ def _prefill_long(cfg, w, toks, chunk, options):
 
 
 @pytest.mark.parametrize("hd,nq,nkv", [(128, 2, 2), (64, 4, 1)])
-def test_tile_long_context_equals_row_kernel(hd, nq, nkv):
-  """2300 keys: the wide tile (16 query vectors) up to ~1900 keys, the narrow one (8) beyond; every chunk's first token, the last logits
-  and the whole K/V equal what the one-block-per-row kernel produces (which the oracle pins at the shorter ranges above)."""
+@pytest.mark.parametrize("tile", [1, 2])
+def test_tile_long_context_equals_row_kernel(hd, nq, nkv, tile):
+  """2300 keys, on the matrix units (1) and on the vector units (2: the wide tile, 16 query vectors, up to ~1900 keys, the narrow one, 8, beyond); every chunk's
+  first token, the last logits and the whole K/V equal what the one-block-per-row kernel produces (which the oracle pins at the shorter ranges above)."""
   cfg = H.make_config(base_emb_dim=256, base_num_query_heads=nq, base_num_kv_heads=nkv, head_dim=hd, base_mlp_dim=384, base_num_decoder_layers=2,
                       vocab_size=1024, model_name="default", per_device_batch_size=1.0, use_chunked_prefill=True, prefill_chunk_size=128,
                       max_prefill_predict_length=128, max_target_length=2432, pagedattn_tokens_per_page=32, pagedattn_num_pages=80)
   w = H.synth.synth_weights(cfg, 21)
   toks = np.random.default_rng(5).integers(1, cfg.vocab_size, size=2300).astype(np.int32)
-  a = _prefill_long(cfg, w, toks, 128, {"attn_tile": 1, "attn_tile_min_rows": 1})
+  a = _prefill_long(cfg, w, toks, 128, {"attn_tile": tile, "attn_tile_min_rows": 1})
   b = _prefill_long(cfg, w, toks, 128, {"attn_tile": 0})
   assert np.array_equal(a[0], b[0])
   assert np.array_equal(a[1], b[1])

@@ -1,5 +1,5 @@
 """The prefill attention on the f32 matrix units (k_attn_mtile: 32-token pages) against the kernels that walk one row at a time: token ids, f32 logits
-and K/V bit for bit at the edges of its forms (256, 512, 1024, 2048 keys), with windows and soft caps, and with scores so far apart that the
+and K/V bit for bit at the edges of its forms (256, 512, 1024, 2048, 4096 keys), with windows and soft caps, and with scores so far apart that the
 quotients of the softmax leave the range of the corrected reciprocal (e below 2^-96)."""
 import numpy as np
 import pytest
@@ -35,7 +35,20 @@ def test_matrix_tile_equals_row_kernel(hd, nq, nkv, length, chunk, spread):
   _same(a, b)
 
 
-@pytest.mark.parametrize("hd,nq,nkv", [(256, 4, 2), (256, 8, 2), (64, 4, 2)])
+@pytest.mark.parametrize("hd,nq,nkv", [(128, 8, 2), (64, 2, 2)])
+def test_matrix_tile_of_the_longest_prefixes(hd, nq, nkv):
+  """4200 keys: all four rounds of the last form (3073 .. 4096 keys), then the vector units, which take over past 4096; four query heads a kv head."""
+  cfg = H.make_config(base_emb_dim=256, base_num_query_heads=nq, base_num_kv_heads=nkv, head_dim=hd, base_mlp_dim=384, base_num_decoder_layers=1,
+                      vocab_size=1024, model_name="default", per_device_batch_size=1.0, use_chunked_prefill=True, prefill_chunk_size=256,
+                      max_prefill_predict_length=256, max_target_length=4352, pagedattn_tokens_per_page=32, pagedattn_num_pages=140)
+  w = H.synth.synth_weights(cfg, 37)
+  toks = np.random.default_rng(hd).integers(1, cfg.vocab_size, size=4200).astype(np.int32)
+  matrix, vector, rows = (_prefill_long(cfg, w, toks, 240, {"attn_tile": tile, "attn_tile_min_rows": 1}) for tile in (1, 2, 0))
+  _same(matrix, rows)
+  _same(vector, rows)
+
+
+@pytest.mark.parametrize("hd,nq,nkv", [(256, 4, 2), (256, 8, 2), (64, 4, 2), (256, 2, 2)])
 @pytest.mark.parametrize("window", [70, 4096])
 def test_matrix_tile_with_cap_and_window(hd, nq, nkv, window):
   """Local and global sub-layers, capped scores; 256-column values (two output passes, in one block and in two)."""

@@ -14,8 +14,16 @@ SHAPES = {
     "ragged": dict(base_emb_dim=200, base_num_query_heads=5, base_num_kv_heads=5, head_dim=40, base_mlp_dim=328, vocab_size=1000, max_target_length=72, per_device_batch_size=3.0),
     # 256 x 256 tiles with cut-off rows, columns and reductions (the vocabulary's products), a second chunk of 16 logits rows
     "large tiles": dict(base_emb_dim=72, base_num_query_heads=2, base_num_kv_heads=2, head_dim=64, base_mlp_dim=136, vocab_size=6152, max_target_length=688, per_device_batch_size=3.0),
-    # reductions cut in parts, the last part shorter; groups of query heads
-    "cut reductions": dict(base_emb_dim=264, base_num_query_heads=4, base_num_kv_heads=2, head_dim=128, base_mlp_dim=520, vocab_size=4104, max_target_length=712, per_device_batch_size=3.0),
+    # long reductions that are not cut (2136 tokens: only multiples of 256 are); groups of query heads
+    "long reductions": dict(base_emb_dim=264, base_num_query_heads=4, base_num_kv_heads=2, head_dim=128, base_mlp_dim=520, vocab_size=4104, max_target_length=712, per_device_batch_size=3.0),
+    # reductions cut in four: inside the block (the weight gradients of 2048 x 768 and of three times 768 x 768 over 2304 tokens; the sum of two products over
+    # 2048 features, the first of them cut), and as parts that a kernel adds (768 x 768); the
+    # scratch for them is the chunk's logits: 2048 x 6152
+    "cut reductions": dict(base_emb_dim=768, base_num_query_heads=12, base_num_kv_heads=12, head_dim=64, base_mlp_dim=2048, vocab_size=6152, max_target_length=768, per_device_batch_size=3.0),
+    # sums of two and of three products in 128 x 128 tiles (4096 x 832), reductions that end inside a chunk
+    "sums in large tiles": dict(base_emb_dim=832, base_num_query_heads=13, base_num_kv_heads=13, head_dim=64, base_mlp_dim=1032, vocab_size=264, max_target_length=512, per_device_batch_size=8.0),
+    # enough heads for the attention's largest tiles (256 x 256 scores, 256 x 128 outputs), rows 8 beyond a tile
+    "large attention tiles": dict(base_emb_dim=72, base_num_query_heads=16, base_num_kv_heads=16, head_dim=128, base_mlp_dim=136, vocab_size=264, max_target_length=264, per_device_batch_size=16.0),
     # a vocabulary of an odd number of 128-byte lines: its rows lie as far apart as they are long, also from 4096 columns on
     "odd lines": dict(base_emb_dim=72, base_num_query_heads=2, base_num_kv_heads=2, head_dim=64, base_mlp_dim=136, vocab_size=4160, max_target_length=72, per_device_batch_size=2.0),
     # one row, shorter than any tile
