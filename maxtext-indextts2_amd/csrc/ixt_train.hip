@@ -273,7 +273,8 @@ static int gemm(hipStream_t st, int what, int M, int K, std::initializer_list<TO
     return t * ((M + b - 1) / b);
   };
   // A weight gradient of few output tiles over a long reduction (2048 x 2048 over 16384 tokens: 64 tiles of 256 x 256) is cut in four parts, whose
-  // products are added up in order (k_t_sum_parts).  The cut is a matter of the shape alone, so that no choice of tiles changes a sum.
+  // products are added up in order (k_t_sum_parts); a reduction that is no multiple of 256 is not cut.  The cut is a matter of the shape alone, so that no
+  // choice of tiles changes a sum.
   if (out == TG_F32 && scratch != nullptr && g.K[0] >= 2048 && g.K[0] % 256 == 0) {
     bool all = true;
     long need = 0;
@@ -301,9 +302,8 @@ static int gemm(hipStream_t st, int what, int M, int K, std::initializer_list<TO
       int k = 0;
       for (const TOperand& o : ops) g.C[k++] = o.c;
     }
-    const bool b128 = tiles(128) >= 200;
-    if (what == TL_DX) return b128 ? gemm_launch<false, false, 128, 128, true>(st, g) : gemm_launch<false, false, 64, 64, true>(st, g);
-    return b128 ? gemm_launch<true, true, 128, 128, true>(st, g) : gemm_launch<true, true, 64, 64, true>(st, g);
+    if (what == TL_DX) return tiles(128) >= 200 ? gemm_launch<false, false, 128, 128, true>(st, g) : gemm_launch<false, false, 64, 64, true>(st, g);
+    return gemm_launch<true, true, 64, 64, true>(st, g);   // (cut in four: fewer than 48 tiles of 256 x 256, 192 of 128 x 128 at most)
   }
   if (sums > 1) {
     int k = 0;
