@@ -20,7 +20,8 @@ typedef struct ixt_train_config {
   float normalization_layer_epsilon, rope_min_timescale, rope_max_timescale;
   int32_t batch;          /* rows of this GPU's batch = per_device_batch_size (train.py:271-275) */
   int32_t seq_len;        /* max_target_length (base.yml:527) */
-  int32_t logits_chunk;   /* rows whose [rows, vocab] f32 logits are alive at a time (0: 2048) */
+  int32_t logits_chunk;   /* rows whose [rows, vocab] logits (bf16) and their gradients are alive at a time (0: 2048).  rows x vocab f32 words are set aside
+                             for them, which the backward pass uses for the parts of long reductions */
 } ixt_train_config;
 
 typedef struct ixt_trainer ixt_trainer;
