@@ -370,7 +370,7 @@ int ixt_set_sampling_ranges(ixt_ctx* ctx, const int32_t* lo_hi, int nranges);
 
 /* Launch-shape knobs of this build (no counterpart in the reference; results never depend on them, tests use them to drive
  * every kernel variant on small configurations):
- *   "attn_fused_min_blocks"  decode attention runs as one launch per layer once rows x kv_heads reaches this (default 128)
+ *   "attn_fused_min_blocks"  decode attention runs as one launch per layer once rows x kv_heads reaches this (default 64)
  *   "gemm_min_rows", "gemm_min_blocks"  a dot of at least this many rows (default 128) and 128 x 128 blocks (default 150) runs as
  *                            the tiled GEMM kernel (all of K per block, one f32 slice) instead of split-K
  *   "gemm_split_min_blocks"  below gemm_min_blocks: the same tiles split over the 512-k chains (one slice per chain) once there are
@@ -384,8 +384,8 @@ int ixt_set_sampling_ranges(ixt_ctx* ctx, const int32_t* lo_hi, int nranges);
  *                            128-column x 64-row blocks (default: never)
  *   "ring_min_rows"          from this many rows (default 128) a dot runs as the LDS-ring GEMM (QKV + RoPE + page write, residual, SwiGLU, sampling as
  *                            its epilogues; csrc/ixt_gemm.h); ixt_op_dot uses its f32 epilogue
- *   "ring_mid_rows"          prompts' passes of the llama and Gemma blocks take it from this many rows (default 17), decode steps of the llama blocks and
- *                            unembeddings from 16 more, unless ring_min_rows is above 128
+ *   "ring_mid_rows"          passes of the Gemma blocks and prompts' passes of the llama blocks take it from this many rows (default 17), decode steps of the
+ *                            llama blocks and unembeddings from 16 more, unless ring_min_rows is above 128
  *   "ring_cfg"               0 (default): tile chosen per shape; 1: 128 x 128, 2: 128 rows x 64 columns, 3: 64 x 32, 4: 256 x 128, 5: 64 x 64,
  *                            6: 64 x 16, 7: 128 x 128 with 32-k chunks, two blocks on a CU
  *   "ring_split"             1: ixt_op_dot's ring GEMM runs split over the 512-k chains (one f32 slice per chain)

@@ -1004,7 +1004,8 @@ int launch_dot(ixt_ctx* c, const bf16_t* x, const bf16_t* w, int K, int N, int R
 // slices).  48 rows of the 1B model, one layer: QKV 11.3 -> 12.1 us and attention 47.1 -> 42.3, O and norm 11.9 -> 13.3, MLP up and gate 23.8 -> 14.7;
 // unembedding 267 -> 220.  A decode step of 48 rows 2.08 -> 1.83 ms, a prompt of 57 tokens 1.57 -> 1.35 ms.  Prompts from 17 rows on (up to 16 the kernels
 // of ixt_small.h serve; 20 rows 1.32 -> 1.26 ms); decode rows and the unembedding from 33 on: two row blocks a fragment stream as fast without a tile's idle
-// half (24 rows 1.36 -> 1.41 ms a step with the ring).
+// half (24 rows 1.36 -> 1.41 ms a step with the ring).  Gemma's decode rows from 17 on, too (24 rows, four sub-layers: 687 -> 668 us a step).  Hybrid decoders and the
+// routed blocks' QKV and O start at ring_min_rows.
 static int ring_model_rows(const ixt_ctx* c, bool decode) { return c->ring_min_rows > 128 ? c->ring_min_rows : std::min(c->ring_min_rows, c->ring_mid_rows + (decode ? 16 : 0)); }
 
 // logits (optional store) + greedy argmax for R rows of normed hidden states
