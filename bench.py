@@ -1,19 +1,19 @@
 #!/usr/bin/env python3
-"""Headline benchmark: audio tokens / second over prefill + decode of the 1B IndexTTS2-style decoder (BASELINE.json
-configs[1], "C2"), data-parallel over N GPUs of one node (one process per GPU, no collective on the data path).
+"""Headline benchmark: audio tokens / second over prefill + decode of the 1B IndexTTS2-style decoder ("C2": 264 192-row
+vocabulary), data-parallel over N GPUs of one node (one process per GPU, no collective on the data path).
 
   python bench.py --gpus N --steps K --warmup W            (N > 1: this process starts N rank processes itself, before any GPU call)
   python -m torch.distributed.run --nnodes=1 --nproc-per-node N --master-addr 127.0.0.1 --master-port P bench.py --gpus N ...
 
 A "step" is one pass of the hot path over one batch of synthetic input: `--batch` (default 256) utterances per GPU,
-each a 256-token prompt (4 s reference speech + 128-char text, SURVEY.md section 8d) prefilled -- `--prefill-pack` (default 8)
+each a 256-token prompt (4 s reference speech + 128-char text) prefilled -- `--prefill-pack` (default 8)
 prompts per pass over the weights through the engine's prefill_concat / insert_partial (maxengine.py:719-836, 1206-1318) -- then
 `--decode-steps` (default 1024) greedy generate calls for all slots, then ONE fetch of all generated ids to the host (decode.py:162-184
-reads them; SURVEY.md section 8e "results gathered on host as int32 ids").  Tokens counted = generated audio tokens
+reads them; results are gathered on the host as int32 ids).  Tokens counted = generated audio tokens
 including the first one from prefill (decode.py:162-178: T-P generate calls yield T-P+1 tokens per utterance).
 Protocol = the reference's micro-benchmark (inference_microbenchmark.py:149-197): warm-up passes, then a timed loop closed by a device sync.
 
-The driver's command is `python3 bench.py --gpus 1 --steps 20 --warmup 5` under a 600 s limit: 25 passes of the default batch take about
+`python3 bench.py --gpus 1 --steps 20 --warmup 5` is meant to end within 600 s: 25 passes of the default batch take about
 175 s.  Everything after the timed region runs against a wall-clock budget (`--budget-s`, counted from process start): `roofline` and
 `cpu_baseline` always, the extra rows under `detail` (one / eight utterances, the 4096-token chunked prefill, one pass each at 512 and 1024
 utterances per GPU) only while the budget allows; rows left out are named in `detail.skipped`.
@@ -59,14 +59,14 @@ def parse(argv=None):
   ap.add_argument("--no-graph", action="store_true")
   ap.add_argument("--no-cpu-baseline", action="store_true")
   ap.add_argument("--no-roofline", action="store_true")
-  ap.add_argument("--no-batch-rows", action="store_true", help="skip the B=1 / B=8 rows of SURVEY.md section 8(d)")
+  ap.add_argument("--no-batch-rows", action="store_true", help="skip the rows of one and of eight utterances")
   ap.add_argument("--no-detail", action="store_true", help="no prefill / decode split events inside the timed passes (profiling runs)")
   ap.add_argument("--no-big-rows", action="store_true", help="skip the one-pass rows at larger batches")
   ap.add_argument("--no-fetch", action="store_true", help="do not fetch the generated ids to the host at the end of a pass (counter runs)")
   ap.add_argument("--cpu-batch", type=int, default=16, help="utterances of the CPU baseline sample")
   ap.add_argument("--cpu-slice-steps", type=int, default=2)
   ap.add_argument("--cpu-check-steps", type=int, default=4, help="decode steps of utterance 0 the parity oracle replays to check the fetched ids")
-  ap.add_argument("--cpu-threads", type=int, default=16, help="threads of the CPU baseline (the GPU box's CPU share for one GPU is 16)")
+  ap.add_argument("--cpu-threads", type=int, default=16, help="threads of the CPU baseline (one GPU's share of its host: 16)")
   ap.add_argument("--sync-every", type=int, default=0, help="synchronise the stream every N engine calls (profiling runs: bounds the launch backlog)")
   ap.add_argument("--backend", default="nccl", help="torch.distributed backend (nccl = RCCL; gloo for the CPU rehearsal)")
   ap.add_argument("--opt", action="append", default=[], help="library option name=value (ixt_set_option), e.g. kv_head_major=1; experiments")
@@ -399,7 +399,7 @@ def detail_split(args, nums, B, P, t_prefill, t_decode):
   mean_ctx = P + args.decode_steps / 2.0
   step_bytes = (nums["body_params"] + nums["unembed_params"]) * 2 + B * mean_ctx * nums["kv_bytes_per_token"] + B * nums["kv_bytes_per_token"]
   step_flops = B * 2.0 * (nums["body_params"] + nums["unembed_params"]) + B * mean_ctx * nums["kv_bytes_per_token"]
-  prefill_flops = 2.0 * P * nums["body_params"] + 4.0 * 16 * 128 * 16 * P * P / 2 + 2.0 * nums["unembed_params"]   # SURVEY 8(d): last-row logits only
+  prefill_flops = 2.0 * P * nums["body_params"] + 4.0 * 16 * 128 * 16 * P * P / 2 + 2.0 * nums["unembed_params"]   # last-row logits only
   return {"prefill_ms_per_utterance": t_prefill / B * 1e3, "prefill_mfu": prefill_flops / (t_prefill / B) / MFMA_BF16_PEAK,
           "decode_ms_per_step": ms_step, "decode_tokens_per_s": B / (ms_step * 1e-3),
           "decode_step_algorithmic_bytes": step_bytes, "decode_hbm_frac": step_bytes / (ms_step * 1e-3) / HBM_PEAK,
@@ -503,7 +503,7 @@ def roofline(args, wl, eng, cfg, nums, prompts, B):
 
 
 def batch_row(args, b, weights, prompts_dev, nums):
-  """the same model at B = 1 (latency) and B = 8 utterances per GPU against the HBM bounds of BASELINE.md section 4."""
+  """The same model at B = 1 (latency) and B = 8 utterances per GPU against the HBM bounds of their bytes."""
   import torch
   pyconfig = importlib.import_module("maxtext-indextts2_amd.pyconfig")
   maxengine = importlib.import_module("maxtext-indextts2_amd.maxengine")
@@ -535,7 +535,7 @@ def batch_row(args, b, weights, prompts_dev, nums):
 
 
 def long_prefill_row(args, weights, nums, total=4096, chunk=None):
-  """BASELINE.json configs[3]'s prefill shape on the C2 model: ONE prompt of `total` tokens through the engine's chunked prefill (chunks of
+  """A long prefill on the C2 model: ONE prompt of `total` tokens through the engine's chunked prefill (chunks of
   `chunk` rows, default --prefill-len; each chunk attends to everything before it through the pages: k_attn_tile with a growing key range)."""
   import numpy as np
   import torch
@@ -573,8 +573,8 @@ def long_prefill_row(args, weights, nums, total=4096, chunk=None):
 
 def cpu_baseline(args, cfg, weights, prompts, gpu_ids=None):
   """The reference ALGORITHM on this host's CPU cores (oracle/ref_algo_cpu.py: dense two-segment cache, both full buffers read at every step,
-  [1, P, V] prefill logits, bf16 values / f32 accumulation), on a bounded sample of the workload.  JAX (the north star's `jax.devices('cpu')`)
-  is not installed anywhere in this pipeline; this torch-CPU restatement is the labelled stand-in of BASELINE.md section 3.
+  [1, P, V] prefill logits, bf16 values / f32 accumulation), on a bounded sample of the workload.  JAX (`jax.devices('cpu')`)
+  is not installed; this torch-CPU restatement is the labelled stand-in.
   `gpu_ids` (the ids the last timed pass fetched) are CHECKED here against the parity oracle (oracle/ixt_oracle.c: utterance 0, the first
   1 + `--cpu-check-steps` ids, bit-exact contract) and against the independent f32 restatement's first token."""
   import numpy as np
@@ -582,7 +582,7 @@ def cpu_baseline(args, cfg, weights, prompts, gpu_ids=None):
   from oracle import ref_algo_cpu as RA
   host_w = {k: v.detach().contiguous().view(torch.int16).cpu().numpy().view(np.uint16) for k, v in weights.items()}
   cb = max(1, min(args.cpu_batch, args.batch))
-  # the GPU box gives one GPU's job 16 CPUs whatever os.cpu_count() says: more threads than that only thrash
+  # one GPU's job has 16 CPUs of its host whatever os.cpu_count() says: more threads than that only thrash
   threads = min(args.cpu_threads, os.cpu_count() or 1)
   _log(f"cpu baseline: {cb} utterances on {threads} threads")
   r = RA.measure(cfg, host_w, prompts, cb, args.prefill_len, args.decode_steps, slice_steps=args.cpu_slice_steps, threads=threads, log=_log)

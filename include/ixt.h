@@ -2,7 +2,7 @@
  * ixt.h -- C ABI of libixt.so: the MI355X (gfx950) hot path of an IndexTTS2-style
  * semantic-token LM: chunked prompt prefill + per-step audio-token decode over a paged KV cache.
  *
- * Boundary rules (SURVEY.md section 8b): plain C, `int` status return (0 = ok, negative = ixt_status,
+ * Boundary rules: plain C, `int` status return (0 = ok, negative = ixt_status,
  * never throws), device pointers are plain `void*`/typed pointers owned by the caller unless stated,
  * every compute call takes an explicit hipStream_t (passed as void*), no allocation after
  * ixt_create/ixt_load_weight, one ctx per GPU, calls on one ctx externally serialised (the reference
@@ -122,7 +122,7 @@ typedef struct ixt_config {
   int32_t max_packed_rows;         /* build knob: most rows of one ixt_prefill_rows call (0: max_prefill_predict_length) */
   int32_t staging_groups;          /* build knob: page groups behind the decode slots that a packed prefill (MaxEngine.prefill_concat,
                                       maxengine.py:719-836) fills before insert_partial hands their pages to slots; 0 = none */
-  /* Decoder block variant (SURVEY.md section 8(f) item 3).  All zero = the llama2 block (llama2.py:54-169).
+  /* Decoder block variant.  All zero = the llama2 block (llama2.py:54-169).
    * IXT_BLOCK_GEMMA2 (layers/gemma2.py:69-236, configs/models/gemma2-2b.yml): `num_decoder_layers` counts the reference's merged
    * [local, global] layers; the context then holds 2 x num_decoder_layers (attention, MLP) sub-layers -- sub-layer 2 i is layer i's
    * "local" half, 2 i + 1 its "global" half -- and every `layer` argument of this header (ixt_kv_gather, ixt_op_kv_write,
@@ -141,7 +141,7 @@ typedef struct ixt_config {
    * :2246-2248).  Read for gemma3 only: */
   float local_rope_max_timescale;  /* base.yml:603, attentions.py:2085-2088: RoPE base of the local layers; <= 0: rope_max_timescale */
   float query_pre_attn_scalar;     /* gemma3.py:50-58, attentions.py:2262-2264: q = bf16(q * bf16(scalar)) after RoPE; 0 or 1: none */
-  /* IXT_BLOCK_MIXTRAL (SURVEY.md section 8(f) item 4; layers/mixtral.py:52-170, layers/moe.py:205-1490, configs/models/mixtral-8x7b.yml): the
+  /* IXT_BLOCK_MIXTRAL (layers/mixtral.py:52-170, layers/moe.py:205-1490, configs/models/mixtral-8x7b.yml): the
    * llama2 wiring with the MLP replaced by a routed mixture -- gate logits (moe.py:170-204), jax.lax.top_k + softmax over the k logits
    * (:326-345), the selected experts' silu MLPs, sum_k weight_k y_k in f32 (:455-484).  Weights: `MoeBlock_0/gate/kernel` [emb, experts],
    * `MoeBlock_0/wi_0`, `MoeBlock_0/wi_1` [experts, emb, mlp], `MoeBlock_0/wo` [experts, mlp, emb]; the pre-MoE norm is
@@ -153,8 +153,8 @@ typedef struct ixt_config {
    * and the other experts' slices are skipped.  ep_size <= 1: every expert.  A sharded context serves ixt_op_moe_route / ixt_op_moe_experts
    * (the two sides of the caller's exchange); the fused engine entry points need every expert and refuse. */
   int32_t ep_rank, ep_size;
-  /* base.yml:93 `quantization: "fp8"` (BASELINE.json configs[3]).  The reference installs fp8 for training only (quantizations.py:289-298) and refuses
-   * it in decode (decode.py:127-128), so the scheme is this build's own, "IXT-FP8-v1" (csrc/ixt_fp8.h, DESIGN.md section 3b): the four projection
+  /* base.yml:93 `quantization: "fp8"`.  The reference installs fp8 for training only (quantizations.py:289-298) and refuses
+   * it in decode (decode.py:127-128), so the scheme is this build's own, "IXT-FP8-v1" (csrc/ixt_fp8.h): the four projection
    * kernels of every layer (and every expert) are kept as e4m3 with one f32 scale per output column, activations are quantised to e4m3 per row
    * and 512-k block on the way in, the products run on v_mfma_f32_16x16x32_fp8_fp8 with f32 accumulation; embedding, norms, attention and the
    * logits head stay bf16.  Not bit-comparable with the bf16 path: tests/test_gpu_fp8.py states the error. */
@@ -208,7 +208,7 @@ int ixt_pages_reset(ixt_ctx* ctx, void* stream);
 /* PageManager.update_prefill_pages (page_manager.py:493-536): release the group, then first-fit reserve
  * ceil(true_length/page) pages; silently leaves the group empty when resources are short (:305-311). */
 int ixt_pages_reserve(ixt_ctx* ctx, int slot, int true_length, void* stream);
-/* Build extension for chunked prefill over pages (no reference counterpart, see DESIGN.md): keep the
+/* Build extension for chunked prefill over pages (no reference counterpart): keep the
  * group's pages and grow the allocation to total_length tokens. */
 int ixt_pages_extend(ixt_ctx* ctx, int slot, int total_length, void* stream);
 /* PageManager.update_decode_pages (page_manager.py:331-412,538-566). */
@@ -363,7 +363,7 @@ int ixt_timing_get(ixt_ctx* ctx, const char* family, double* avg_us, int64_t* la
 
 
 /* Greedy sampling restricted to the union of `nranges` (0..4) half-open column ranges lo_hi[2i], lo_hi[2i+1] (host array);
- * nranges == 0 lifts the restriction.  SURVEY.md section 8(f) item 1: the expanded vocabulary keeps the audio codes in rows
+ * nranges == 0 lifts the restriction.  The expanded vocabulary keeps the audio codes in rows
  * 6..104 and 256001..264093 (audio_token_mapping_adjusted.json, generator vocab_expansion/extend_tokenizer.py:29-46); with
  * these two ranges every generated id maps back to an audio code.  Logits are returned unmasked. */
 int ixt_set_sampling_ranges(ixt_ctx* ctx, const int32_t* lo_hi, int nranges);

@@ -1,5 +1,5 @@
 /*
- * ixt_train.h -- C ABI of the training step of libixt.so (SURVEY.md section 8 f2, BASELINE.json configs[2]): forward + backward of the
+ * ixt_train.h -- C ABI of the training step of libixt.so: forward + backward of the
  * llama2 block stack on one GPU's share of the batch, cross entropy with the reference's custom VJP, global-norm clip and AdamW.
  * Same boundary rules as ixt.h: plain C, int status, explicit stream, no allocation after create.  Parameters, gradients and the AdamW
  * moments live in FLAT f32 device buffers owned by the CALLER, laid out as ixt_train_param_info describes, so that the data-parallel

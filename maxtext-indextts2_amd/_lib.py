@@ -143,7 +143,7 @@ def load():
 
 
 def check(rc: int):
-  """Map ixt_status to the reference's exception conventions (error conventions)."""
+  """Map ixt_status to the reference's exception conventions."""
   if rc == IXT_OK:
     return
   msg = load().ixt_last_error().decode("utf-8", "replace")

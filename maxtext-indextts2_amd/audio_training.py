@@ -1,7 +1,7 @@
 """Counterpart of the reference's example_audio_training.py (repo root of the reference) and of the batch contract its training path
 expects (MaxText/maxtext_utils.py:85-99 `get_shaped_batch`; MaxText/input_pipeline/synthetic_data_processing.py:66-78 for how the six arrays
 relate).  The reference's own Emilia iterators raise NotImplementedError (input_pipeline/_emilia_audio_processing.py:44-49) and its example
-calls a `pyconfig.load_config` that does not exist (header facts), so "counterpart" means: the SAME override list parses, the
+calls a `pyconfig.load_config` that does not exist, so "counterpart" means: the SAME override list parses, the
 SAME tokenizer callback type is accepted, and the batches have the SAME six int32 [B, max_target_length] keys.
 
   audio bytes --(audio_tokenizer_fn: List[bytes] -> List[List[int]], ids in [0, 8192), example_audio_training.py:16-43)-->
@@ -21,7 +21,7 @@ AudioTokenizerFn = Callable[[List[bytes]], List[List[int]]]
 BATCH_KEYS = ("inputs", "inputs_position", "inputs_segmentation", "targets", "targets_position", "targets_segmentation")
 
 # example_audio_training.py:54-79, verbatim keys; vocab_size is 264192 here: the example's 264191 cannot hold max_embedding_index 264191
-# (SURVEY.md section 8, C2 note) and is refused below with that explanation
+# and is refused below with that explanation
 EXAMPLE_OVERRIDES = [
     "dataset_type=emilia_audio", "audio_token_mapping_path=vocab_expansion/audio_token_mapping_adjusted.json", "audio_batch_size=32",
     "emilia_language=EN", "base_emb_dim=2048", "vocab_size=264192", "global_batch_size_to_load=128", "max_target_length=2048", "steps=100000",

@@ -14,7 +14,7 @@ SOURCES = ["ixt_api.hip", "ixt_hybrid.hip", "ixt_hybrid_heads.hip", "ixt_hybrid_
 HEADERS = ["ixt_device.h", "ixt_kernels.h", "ixt_tile_attn.h", "ixt_gemma_kernels.h", "ixt_moe_kernels.h", "ixt_gemm.h", "ixt_small.h", "ixt_fp8.h", "ixt_hybrid_kernels.h", "ixt_heads_kernels.h", "ixt_retention_kernels.h", "ixt_scan_kernels.h", "ixt_internal.h", "ixt_hybrid.h", "ixt_train_gemm.h", "ixt_train_kernels.h", os.path.join("..", "..", "include", "ixt.h"),
            os.path.join("..", "..", "include", "ixt_train.h")]
 
-# -ffp-contract=off: the numerics contract (DESIGN.md section 3) allows fused multiply-adds only where the source
+# -ffp-contract=off: the numerics contract allows fused multiply-adds only where the source
 # says fmaf; correctly rounded f32 divide/sqrt and IEEE denormals are hipcc defaults and are stated explicitly.
 HIPCC_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=off", "-fno-fast-math",

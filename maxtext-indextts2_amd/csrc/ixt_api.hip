@@ -32,7 +32,7 @@ static float host_rbf(float f) {
 }
 
 static void host_rope_tables(const ixt_config& cfg, float max_timescale, std::vector<uint16_t>& sn, std::vector<uint16_t>& cs) {
-  // embeddings.py:270-307; every step's rounding is listed in DESIGN.md section 3.
+  // embeddings.py:270-307; every step is rounded as written here.
   const int half = cfg.head_dim / 2, T = cfg.max_target_length;
   sn.resize((size_t)T * half);
   cs.resize((size_t)T * half);
@@ -56,7 +56,7 @@ static void host_rope_tables(const ixt_config& cfg, float max_timescale, std::ve
 
 // LLaMARotaryEmbedding (embeddings.py:396-443): timescale_i = min (max / min)^(2 i / D) for the pair (2 i, 2 i + 1); with use_scale the
 // frequency 1 / timescale goes through the llama-3.1 rule: wavelengths below 8192 / 4 keep it, above 8192 divide it by 8, between the two the
-// smooth blend.  angle = position / timescale in f32; sin / cos evaluated in double and rounded to f32 (DESIGN.md section 3).
+// smooth blend.  angle = position / timescale in f32; sin / cos evaluated in double and rounded to f32.
 static void host_rope_tables_llama31(const ixt_config& cfg, std::vector<float>& sn, std::vector<float>& cs) {
   const int half = cfg.head_dim / 2, T = cfg.max_target_length;
   sn.resize((size_t)T * half);

@@ -1,4 +1,4 @@
-// ixt_device.h -- scalar numerics shared by every kernel ("IXT-MFMA-v2", DESIGN.md section 3).
+// ixt_device.h -- scalar numerics shared by every kernel ("IXT-MFMA-v2").
 // Compiled with -ffp-contract=off: a*b+c never fuses; every fused multiply-add is an explicit fmaf.
 #pragma once
 #include <hip/hip_runtime.h>

@@ -1,9 +1,9 @@
-// ixt_fp8.h -- the projections of a decoder layer with FP8 weights on the gfx950 fp8 matrix cores ("fp8 MFMA
-// weights"; included by ixt_api.hip).
+// ixt_fp8.h -- the projections of a decoder layer with FP8 weights on the gfx950 fp8 matrix cores
+// (included by ixt_api.hip).
 //
 // The reference has no fp8 inference behaviour to be equal to: `quantization: fp8 / nanoo_fp8` installs AQT hooks for TRAINING
-// (layers/quantizations.py:289-298) and decode refuses them (decode.py:127-128).  This build therefore DEFINES the scheme ("IXT-FP8-v1",
-// DESIGN.md section 3b) and states its error against the bf16 path instead of claiming bit equality:
+// (layers/quantizations.py:289-298) and decode refuses them (decode.py:127-128).  This build therefore DEFINES the scheme ("IXT-FP8-v1")
+// and states its error against the bf16 path instead of claiming bit equality:
 //   weights      W[k][n] (bf16 values) -> e4m3 (OCP: 4 exponent bits, 3 mantissa bits, max 448, no infinities) with one f32 scale per output
 //                column: s_n = amax_k |W[k][n]| / 448 (1 for an all-zero column), q = e4m3_rne(W / s_n)
 //   activations  x[r][k] (bf16 values) -> e4m3 with one f32 scale per row and 512-k block (the canonical dot's chain):

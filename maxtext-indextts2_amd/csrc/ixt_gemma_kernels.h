@@ -1,4 +1,4 @@
-// ixt_gemma_kernels.h -- row kernels of the Gemma-2 block (SURVEY.md section 8(f) item 3; layers/gemma2.py:69-236, decoders.py:552-565).
+// ixt_gemma_kernels.h -- row kernels of the Gemma-2 block (layers/gemma2.py:69-236, decoders.py:552-565).
 // The projections, RoPE, page writes and the attention kernels are the ones of the llama2 block (ixt_kernels.h); what differs is what
 // happens between them: the projection output is normalised before the residual add, the gate is GELU(tanh), and the logits are
 // divided by sqrt(emb) and soft-capped.  Same canonical orders as ixt_kernels.h (slices from 0; sum of squares: a lane's 8 features by

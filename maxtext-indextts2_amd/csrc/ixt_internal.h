@@ -134,7 +134,7 @@ struct ixt_ctx {
   float* moe_w = nullptr;       // [Rmax][TK]
   bf16_t* moe_y = nullptr;      // [Rmax][TK][E]
   // routed evaluation (k_moe_plan / k_moe_gather, grouped k_dotb / k_gemm_ring): copies of a row sit in the rows of their expert
-  int moe_grouped = 1;          // 0: every expert over all rows (round 2's form; experiments)
+  int moe_grouped = 1;          // 0: every expert over all rows (experiments)
   int moe_rows_cap = 0;         // copy rows incl. alignment padding the workspaces hold
   int32_t* moe_pos = nullptr;   // [Rmax TK] destination row of every copy
   int32_t* moe_rbexp = nullptr; // [moe_rows_cap / 16] expert of every 16-row block, -1: none

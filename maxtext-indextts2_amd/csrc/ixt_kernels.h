@@ -1,6 +1,6 @@
 // ixt_kernels.h -- gfx950 kernels of the hot path.  Wave = 64 lanes everywhere.
 //
-// HBM layouts (DESIGN.md section 4):
+// HBM layouts:
 //   weights      bf16, MFMA-fragment tiled [N/16][K/32][(k%32)/8][n%16][k%8]: a wave reads 1 KiB per k-step, contiguous along k
 //   K pages      bf16 [layer][page][kv_head][hd/8][tok][8]   (token-minor inside a d-chunk: a wave's
 //                score load is tokens_per_page x 16 B contiguous per page)
@@ -2325,7 +2325,7 @@ static __global__ __launch_bounds__(64) void k_pages_advance(PageStateDev s) {
 }
 static __global__ void k_pages_set_active(PageStateDev s, int g, int v) { s.has_active_page[g] = v; }
 
-// ---- build extensions around MaxEngine.insert (no reference counterpart; DESIGN.md section 6) ----------------------------------
+// ---- build extensions around MaxEngine.insert (no reference counterpart) ----------------------------------
 // insert of a prefix of `length` tokens into the slot that already holds its pages: has_active_page = 1 (maxengine.py:1189-1191) and the
 // length fields back to their post-prefill values -- a generate() between prefill(slot) and insert(slot) has advanced them.
 static __global__ void k_pages_resync(PageStateDev s, int g, int length) {

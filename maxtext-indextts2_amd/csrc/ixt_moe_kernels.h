@@ -1,6 +1,6 @@
-// ixt_moe_kernels.h -- row kernels of the Mixtral block (SURVEY.md section 8(f) item 4; layers/mixtral.py:52-170, layers/moe.py:170-204,
+// ixt_moe_kernels.h -- row kernels of the Mixtral block (layers/mixtral.py:52-170, layers/moe.py:170-204,
 // :326-345, :420-484, :855-942).  Attention, norms and the per-expert MLP dots are the llama2 block's kernels; this file holds the router
-// and the combination of the selected experts' outputs.  Canonical orders (DESIGN.md section 3): gate logit = the vector order of the
+// and the combination of the selected experts' outputs.  Canonical orders: gate logit = the vector order of the
 // RMSNorm statistics (a lane's 8 consecutive k by fma, xor tree over the wave, blocks of 512 k in order; bf16 result); top_k = repeated
 // first-index maximum; weights = bf16(exp*(v_j - v_0) / (e_0 + e_1 + ...)); mixture = fma chain over the k selected experts in top_k order.
 #pragma once
@@ -66,7 +66,7 @@ static __global__ __launch_bounds__(1024) void k_moe_route(const bf16_t* xn, con
 
 // The same router with the work turned round (n_exp a multiple of 8): one wave per BLOCK of 512 k, all experts at once.  A lane's 8 k of the
 // gate kernel are 8 n_exp consecutive bf16 (row-major [E][n_exp]): whole 16-byte loads, consecutive lanes on consecutive lines -- k_moe_route
-// reads the same bytes two at a time, once per expert wave (21.5 us per launch at 4096 x 8; this form: see DESIGN.md section 10).  The order is the
+// reads the same bytes two at a time, once per expert wave (21.5 us per launch at 4096 x 8; this form 8.3).  The order is the
 // contract's: a lane's 8 k by fma, xor tree over the wave, then the blocks' sums added in block order by one thread per expert.
 // grid = R, block = 64 min(blocks, 16).
 template <int NG>   // NG = n_exp / 8

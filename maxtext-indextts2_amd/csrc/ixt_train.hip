@@ -145,7 +145,7 @@ extern "C" int ixt_train_create(const ixt_train_config* c, ixt_trainer** out) {
   A(tmalloc(t, &t->dv, T * KN));
   if (t->G > 1) { A(tmalloc(t, &t->dkf, T * KN)); A(tmalloc(t, &t->dvf, T * KN)); } A(tmalloc(t, &t->dact, T * F)); A(tmalloc(t, &t->da, T * F)); A(tmalloc(t, &t->db, T * F)); A(tmalloc(t, &t->dy_bf, T * E));
 #undef A
-  // RoPE tables: the same host recipe as the decode path (embeddings.py:270-307; DESIGN.md section 3)
+  // RoPE tables: the same host recipe as the decode path (embeddings.py:270-307)
   {
     const int half = t->D / 2;
     std::vector<uint16_t> sn((size_t)S * half), cs((size_t)S * half);

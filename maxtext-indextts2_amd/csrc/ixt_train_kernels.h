@@ -1,4 +1,4 @@
-// ixt_train_kernels.h -- gfx950 kernels of the training step (SURVEY.md section 8 f2; MaxText/train.py:255-472): forward + backward of the
+// ixt_train_kernels.h -- gfx950 kernels of the training step (MaxText/train.py:255-472): forward + backward of the
 // llama2 block stack, cross entropy with its custom VJP (max_utils.py:563-654), global-norm clip (maxtext_utils.py:825-846) and AdamW
 // (optimizers.py:28-38).  Precision: bf16 activations and matmul operands, f32 accumulation (v_mfma_f32_16x16x32_bf16), f32 master
 // weights / gradients / optimizer state -- the reference's dtype=bfloat16, weight_dtype=float32 (base.yml:86, :130).

@@ -1,5 +1,5 @@
 """Data-parallel plumbing for N GPUs of one node: one process per GPU, utterances sharded across ranks, NO collective
-on the data path (SURVEY.md section 8e).  The only exchanges are host-side: a barrier around the timed region, a MAX
+on the data path.  The only exchanges are host-side: a barrier around the timed region, a MAX
 of the elapsed time, and a gather of the generated token ids.  Backend "nccl" is RCCL on ROCm; the CPU tests use gloo."""
 from __future__ import annotations
 
@@ -26,7 +26,7 @@ def init(backend: str, device: torch.device | None = None):
 
 
 def shard_utterances(n_total: int, rank: int, world: int) -> List[int]:
-  """Utterance u goes to rank u mod world (the assignment SURVEY.md section 8e names); returns this rank's global ids."""
+  """Utterance u goes to rank u mod world; returns this rank's global ids."""
   return [u for u in range(n_total) if u % world == rank]
 
 
@@ -63,10 +63,10 @@ def timed_region(one_pass, steps: int, warmup: int, sync_device, device: torch.d
 
 def exchange_gradients(grads: torch.Tensor, loss_and_weights: torch.Tensor, algorithm: str = "auto", bucket_elems: int = 64 << 20) -> None:
   """The data-parallel step of train_step: every rank ends with the SUM over ranks of the flat gradient buffer and of
-  [total_loss, total_weights] (GSPMD emits this all-reduce implicitly in the reference, SURVEY.md section 2.3; loss = sum / sum as in
+  [total_loss, total_weights] (GSPMD emits this all-reduce implicitly in the reference; loss = sum / sum as in
   train.py:307-322).  In place.  algorithm "rs_ag" (what "auto" picks): per bucket a reduce-scatter followed by an all-gather -- on the
   8 fully connected GPUs of a node every rank exchanges 1/8 of the bucket with each of its 7 peers at once, all xGMI links busy, where a
-  ring all-reduce is bound by one link (SURVEY.md section 5.8); "all_reduce": one all-reduce per bucket."""
+  ring all-reduce is bound by one link; "all_reduce": one all-reduce per bucket."""
   if not dist.is_initialized() or dist.get_world_size() == 1:
     return
   world = dist.get_world_size()

@@ -111,7 +111,7 @@ class PageManager:
     return PageState(self)
 
   def extend_prefill_pages(self, page_state: Optional[PageState], page_group_id: int, total_length: int) -> PageState:
-    """Build extension for chunked prefill over pages (DESIGN.md section 6)."""
+    """Build extension for chunked prefill over pages."""
     if page_group_id < 0 or page_group_id >= self.max_page_groups:
       raise ValueError(f"PageManager: page_group_id ({page_group_id}) out of range [0, {self.max_page_groups})")
     if total_length <= 0 or total_length > self.max_target_length:

@@ -1,7 +1,7 @@
 """MaxText/inference/paged_attention.py: PagedAttentionOp (:99-471) over the page pools of libixt.so.
 
 Prefill writes the chunk's K/V into the slot's pages (the INTENDED semantics of :403-444 -- the reference overwrites the whole pool there,
-a defect this build does not copy, DESIGN.md section 6) and attends with the causal offset of ref_ragged_paged_attention
+a defect this build does not copy) and attends with the causal offset of ref_ragged_paged_attention
 (paged_attention_kernel_v2.py:71-109); decode scatters the new token at the page manager's position (:446-471) and attends over the
 slot's sequence.  Returns (output, None, None) as the reference does for paged attention (attentions.py:2302: already normalised)."""
 from __future__ import annotations

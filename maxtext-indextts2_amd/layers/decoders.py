@@ -1,5 +1,5 @@
-"""MaxText/layers/decoders.py: Decoder (:242-800): embedding (:493-534), the unscanned layer loop (:762-789; paged attention needs it,
-SURVEY.md section 3.1), final norm + logits (:537-589)."""
+"""MaxText/layers/decoders.py: Decoder (:242-800): embedding (:493-534), the unscanned layer loop (:762-789; paged attention needs it),
+final norm + logits (:537-589)."""
 from __future__ import annotations
 
 from typing import Any, Optional

@@ -3,7 +3,7 @@ engine (/root/reference/MaxText/maxengine.py:100-1487) for the prefill / insert 
 `attention="paged"` semantics.  PyTorch is used for device memory and streams only; all arithmetic is in
 the HIP library.  Thread rule mirrors the reference: one engine per GPU, calls externally serialised.
 
-Differences that a caller can observe (all documented in DESIGN.md section 6):
+Differences that a caller can observe:
   * prefill writes K/V straight into the slot's pages, so `Prefix["cache"]` is a handle, and `insert`
     is a state copy (the reference's page-copy loop, maxengine.py:1106-1125, is unnecessary);
   * `decode_state` tensors are updated in place and returned (the reference donates them, :868, :1045);
@@ -121,7 +121,7 @@ class MaxEngine(engine_api.Engine):
       c.streams, c.logit_scale, c.logits_via_embedding = int(config.hybrid_streams), float(config.logit_scale), 1 if config.logits_via_embedding else 0
     elif config.dtype != "bfloat16":
       raise NotImplementedError(f"dtype {config.dtype}: only decoder_block hybrid runs in float32")
-    elif config.decoder_block in ("gemma2", "gemma3"):   # layers/gemma2.py:69-236, layers/gemma3.py:35-200 (SURVEY.md section 8(f) item 3)
+    elif config.decoder_block in ("gemma2", "gemma3"):   # layers/gemma2.py:69-236, layers/gemma3.py:35-200
       if tuple(config.mlp_activations) != ("gelu", "linear"):
         raise ValueError(f"decoder_block {config.decoder_block} is built with mlp_activations ['gelu', 'linear']")
       c.decoder_block = _lib.BLOCK_GEMMA2 if config.decoder_block == "gemma2" else _lib.BLOCK_GEMMA3
@@ -137,7 +137,7 @@ class MaxEngine(engine_api.Engine):
       c.normalize_embedding_logits = 1 if config.normalize_embedding_logits else 0
     elif tuple(config.mlp_activations) != ("silu", "linear"):
       raise ValueError(f"decoder_block {config.decoder_block} is built with mlp_activations ['silu', 'linear']")
-    elif config.decoder_block == "mixtral":            # layers/mixtral.py:52-170, layers/moe.py (SURVEY.md section 8(f) item 4)
+    elif config.decoder_block == "mixtral":            # layers/mixtral.py:52-170, layers/moe.py
       c.decoder_block = _lib.BLOCK_MIXTRAL
       c.num_experts, c.num_experts_per_tok = int(config.num_experts), int(config.num_experts_per_tok)
       c.ep_rank, c.ep_size = int(config.ixt_expert_parallel_rank), int(config.ixt_expert_parallel_size)
@@ -258,7 +258,7 @@ class MaxEngine(engine_api.Engine):
     self._params_loaded = True
     return {"params": "resident in HBM (libixt)", "engine": id(self)}
 
-  # ------------------------------------------------------------------ sampling columns (SURVEY 8(f) item 1)
+  # ------------------------------------------------------------------ sampling columns
   def set_sampling_ranges(self, ranges) -> None:
     """Restrict greedy sampling to the union of up to 4 half-open column ranges [(lo, hi), ...]; [] or None lifts it.
     With `AudioTokenMapping.audio_row_ranges()` every generated id is the row of an audio code.  Logits stay unmasked."""

@@ -1,4 +1,4 @@
-"""The work counts of MaxText/maxtext_utils.py that the measurements here are priced in (SURVEY.md section 8(d)): training TFLOP per step and
+"""The work counts of MaxText/maxtext_utils.py that the measurements here are priced in: training TFLOP per step and
 device (`calculate_tflops_training_per_device`, maxtext_utils.py:475-587 with the FFN helper :297-309 and the Gemma-2 / Gemma-3 attention
 variants :156-224) and prefill TFLOP (`calculate_prefill_tflops_per_device`, :590-614).  Same names, arguments and return tuples; pinned by the
 reference's own golden cases (tests/flop_calculation_test.py:99-208 -> tests/test_flop_counts_cpu.py)."""

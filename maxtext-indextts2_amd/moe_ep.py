@@ -1,4 +1,4 @@
-"""Expert-parallel exchange of the Mixtral block (SURVEY.md section 8(f) item 4): the one place of the inference path with a real exchange
+"""Expert-parallel exchange of the Mixtral block: the one place of the inference path with a real exchange
 step.  Experts are split over the ranks of a node (expert e lives on rank e // experts_per_rank); every rank routes its own rows
 (layers/moe.py:420-453 `permute`), sends each (row, k) copy to the rank that owns its expert, receives the copies for its experts,
 applies them, and sends the results back the way they came (moe.py:855-931: the reference does this with two `jax.lax.ragged_all_to_all`
@@ -80,7 +80,7 @@ def expert_parallel_apply(x: torch.Tensor, selected_experts: torch.Tensor, num_e
   """x [rows, emb] and selected_experts int [rows, k] of THIS rank -> y [rows, k, emb] with y[r, j] = expert_fn(selected_experts[r, j], x[r]),
   every expert evaluated on the rank that owns it (experts_per_rank = num_experts / world consecutive ids per rank).  expert_fn(e, rows)
   is called once per local expert that received rows, with the global expert id.  always_exchange: run the collectives on a one-rank
-  group too (exercises the RCCL calls on a one-GPU box).  The steps are the reference's (moe.py:799-942): permute -> all-gather of the
+  group too (exercises the RCCL calls on one GPU).  The steps are the reference's (moe.py:799-942): permute -> all-gather of the
   group sizes -> all-to-all (get_all_to_all_params) -> local_permute -> experts -> undo -> all-to-all back -> unpermute."""
   exchange = dist.is_initialized() and (dist.get_world_size(group) > 1 or always_exchange)
   world = dist.get_world_size(group) if exchange else 1

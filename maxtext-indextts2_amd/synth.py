@@ -1,4 +1,4 @@
-"""Synthetic weights / prompts (SURVEY.md section 8d) -- host-side numpy, shared by tests and bench.
+"""Synthetic weights / prompts -- host-side numpy, shared by tests and bench.
 
 Weights follow the reference's init distributions, drawn from numpy `Generator(PCG64(seed))`:
   * embedding ~ N(0, 1)                                 (layers/models.py:68)
@@ -257,7 +257,7 @@ def audio_id_to_row(a: np.ndarray) -> np.ndarray:
 
 
 def synth_prompt(vocab_size: int, prefill_length: int, seed: int = 1234, n_text: int = 46):
-  """SURVEY.md section 8d prompt: [BT] + n_text text ids + [BA] + audio rows, padded to prefill_length.
+  """A prompt: [BT] + n_text text ids + [BA] + audio rows, padded to prefill_length.
   Returns (padded int32[prefill_length], true_length).  Small vocabularies (test models) get uniform ids."""
   rng = np.random.Generator(np.random.PCG64(seed))
   true_length = int(prefill_length - rng.integers(0, 9)) if prefill_length >= 16 else int(prefill_length)

@@ -1,6 +1,6 @@
 """The training step of the reference (MaxText/train.py:255-472) on MI355X: `Trainer.train_step(batch)` = loss_fn + value_and_grad on this
 GPU's rows (HIP, include/ixt_train.h), the data-parallel gradient exchange (RCCL reduce-scatter + all-gather over xGMI through
-torch.distributed, SURVEY.md section 5.8 -- the only collective of the whole build), global-norm clip, AdamW, warmup-cosine schedule.
+torch.distributed -- the only collective of the whole build), global-norm clip, AdamW, warmup-cosine schedule.
 
 State layout: ONE flat f32 device buffer each for parameters, gradients, AdamW mu and nu (caller = this module owns them as torch tensors,
 the library reads and writes them in place); `param_views()` gives the MaxText tree ({"params/decoder/layers_3/mlp/wi_0/kernel": tensor}).

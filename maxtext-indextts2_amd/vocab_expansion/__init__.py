@@ -1,4 +1,4 @@
-"""Vocabulary expansion for audio codes (SURVEY.md section 8(f) item 1; reference: vocab_expansion/*, audio_token_mapping_adjusted.json).
+"""Vocabulary expansion for audio codes (reference: vocab_expansion/*, audio_token_mapping_adjusted.json).
 
   AudioTokenMapping   the reference's audio-id <-> embedding-row table (integer-exact)
   expand_embedder     append rows to `token_embedder/embedding` AND, when the head is untied, columns to

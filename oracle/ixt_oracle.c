@@ -4,12 +4,12 @@
  * A plain-C restatement of the reference's semantic-token LM hot path
  * (chunked prefill + per-step decode over a paged KV cache) with every
  * floating-point reduction written in ONE fixed, documented order
- * ("IXT-MFMA-v2", DESIGN.md section 3).  Only tests/, __graft_entry__.smoke()
+ * ("IXT-MFMA-v2").  Only tests/, __graft_entry__.smoke()
  * and bench.py's cpu_baseline leg may load this file's shared object.
  *
  * PARITY UNPINNED: the reference is JAX (not installed here; XLA:CPU's
  * accumulation order is unspecified by its source) and its tests carry no
- * numeric golden vectors for this path (SURVEY.md section 8c).  What IS pinned
+ * numeric golden vectors for this path.  What IS pinned
  * by the reference's own fixtures: the integer page-manager cases
  * (tests/inference/page_manager_test.py) and the audio-id mapping tables; see
  * oracle/oracle.py and tests/.
@@ -61,7 +61,7 @@ typedef struct orc_model {
   /* KV pages (oracle-private layout): [L][num_pages][page][nkv][hd] */
   uint16_t* kpages;
   uint16_t* vpages;
-  /* SURVEY.md section 8(f) item 3, Gemma-2 block (layers/gemma2.py:69-236): nlayers then counts (attention, MLP) sub-layers, two per
+  /* Gemma-2 block (layers/gemma2.py:69-236): nlayers then counts (attention, MLP) sub-layers, two per
    * reference layer: even = local sliding window, odd = global.  All zero / NULL: the llama2 block. */
   int32_t block;                      /* 0 llama2, 1 gemma2, 2 gemma3, 3 mixtral */
   float attn_cap;                     /* attn_logits_soft_cap (attentions.py:1257-1259), 0: none */
@@ -77,7 +77,7 @@ typedef struct orc_model {
   float q_scalar;                     /* query_pre_attn_scalar (gemma3.py:50-58, attentions.py:2262-2264): q * scalar after RoPE; 0 or 1: none */
   const uint16_t* rope_sin_local;     /* [max_pos][hd/2]: tables of the local layers (local_rope_max_timescale, attentions.py:2085-2088); NULL: rope_sin */
   const uint16_t* rope_cos_local;
-  /* Mixtral block (block == 3; SURVEY.md section 8(f) item 4; layers/mixtral.py:52-170, layers/moe.py:170-204, :326-345, :420-484, :855-942):
+  /* Mixtral block (block == 3; layers/mixtral.py:52-170, layers/moe.py:170-204, :326-345, :420-484, :855-942):
    * the llama2 wiring with the MLP replaced by a routed mixture: gate logits -> top_k experts -> softmax over the k logits ->
    * sum_k weight_k * MLP_{expert_k}(x).  ln2 is post_self_attention_layer_norm; wi0 / wi1 / wout hold all experts of a layer. */
   int32_t n_exp, top_k;               /* num_experts, num_experts_per_tok (<= 8) */
@@ -567,7 +567,7 @@ void orc_attend_row(const orc_model* m, int layer, const uint16_t* q, const int3
 }
 
 /* ---------------------------------------------------------------- sampling columns */
-/* greedy sampling restricted to a union of up to 4 half-open column ranges (the audio rows of
+/* Greedy sampling restricted to a union of up to 4 half-open column ranges (the audio rows of
  * the expanded vocabulary); n == 0: every column. */
 static int orc_nranges = 0;
 static int32_t orc_lo[4], orc_hi[4];

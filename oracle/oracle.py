@@ -9,7 +9,7 @@ in numpy / pure Python, the integer parts of the path:
   * audio-id <-> embedding-row mapping   /root/reference/vocab_expansion/extend_tokenizer.py:29-46
 
 PARITY UNPINNED for the floating-point path (no JAX here, no numeric goldens in the reference's
-tests; SURVEY.md section 8c).  PINNED for the integer page manager by the reference's own test
+tests).  PINNED for the integer page manager by the reference's own test
 cases (tests/test_page_manager_oracle.py re-states tests/inference/page_manager_test.py).
 
 Only tests/, __graft_entry__.smoke() and bench.py's cpu_baseline leg may import this module.
@@ -365,7 +365,7 @@ class OracleConfig:
   pagedattn_tokens_per_page: int = 32
   pagedattn_max_pages_per_group: int = -1
   max_slots: int = 1
-  # Gemma-2 block (SURVEY.md section 8(f) item 3; configs/models/gemma2-2b.yml): num_decoder_layers counts the reference's merged
+  # Gemma-2 block (configs/models/gemma2-2b.yml): num_decoder_layers counts the reference's merged
   # [local, global] layers; the model then has 2 x num_decoder_layers (attention, MLP) sub-layers and as many K/V page pools
   decoder_block: str = "llama2"
   attn_logits_soft_cap: float = 0.0

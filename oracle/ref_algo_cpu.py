@@ -1,6 +1,6 @@
 """CPU BASELINE of the reference ALGORITHM (test / measurement infrastructure, NOT product code, NOT the parity oracle).
 
-BASELINE.md section 3 / SURVEY.md section 8(d): the north star's CPU baseline is the reference on `jax.devices('cpu')`.  JAX is not
+The CPU baseline would be the reference on `jax.devices('cpu')`.  JAX is not
 installed in this pipeline, so the timed stand-in is this PyTorch-CPU restatement of what the reference *does* on that path -- the
 data movement and arithmetic volume that make up its time, not the bit patterns (those belong to oracle/ixt_oracle.c):
 

@@ -11,4 +11,4 @@ if os.path.dirname(os.path.abspath(__file__)) not in sys.path:
 
 
 def pytest_configure(config):
-  config.addinivalue_line("markers", "gpu: needs a real MI355X (run with -m gpu on the GPU box)")
+  config.addinivalue_line("markers", "gpu: needs a real MI355X (run with -m gpu)")

@@ -7,10 +7,10 @@
   tiny_decode.npz / c1_decode.npz / c2_decode.npz
                                      greedy token ids produced by the CPU ORACLE (oracle/ixt_oracle.c) on seeded synthetic
                                      weights and prompts.  These pin the oracle against drift and give the GPU tests a
-                                     full-size (C2, 1024-step) target without re-running the oracle on the GPU box.
+                                     full-size (C2, 1024-step) target without re-running the oracle beside the GPU.
 
 The floating-point fixtures are oracle outputs, NOT reference outputs (the reference needs JAX, which is not installed:
-parity unpinned, SURVEY.md section 8c).    c2_rows_130.npz / c2_rows_256.npz  C2 at the row counts the benchmark times (130 = two GEMM row groups, the second ragged; 256 = the
+parity unpinned).    c2_rows_130.npz / c2_rows_256.npz  C2 at the row counts the benchmark times (130 = two GEMM row groups, the second ragged; 256 = the
                                      bench default): ragged prompts, a few decode steps, token ids + per-row logits checksums
 usage: make_golden.py [mapping] [tiny] [c1] [c2] [c2_rows_130] [c2_rows_256]
 """

@@ -2,7 +2,7 @@
 
 The floating-point oracle (oracle/ixt_oracle.c) fixes one operation order ("IXT-MFMA-v2") that the kernels share, so HIP == oracle proves
 the kernels implement that contract, not that the contract is the reference's model; JAX is not installable here and the reference's tests
-hold no numeric fixtures for this path (DESIGN.md section 2).  The strongest evidence available is agreement with a restatement that shares
+hold no numeric fixtures for this path.  The strongest evidence available is agreement with a restatement that shares
 nothing with it: oracle/ref_algo_cpu.py is written from the reference's dense path -- two-segment dense KV cache with ONE shared ring index
 (inference/kvcache.py:490-831), full-length masked attention with the (max, sum) merge of the two segments (layers/attentions.py:1376-1466),
 [1, P, V] prefill logits -- on torch f32 matmuls in torch's own accumulation order, against the oracle's paged layout, matrix-instruction model
@@ -93,7 +93,7 @@ def test_tiny_dense_restatement_agrees_with_paged_oracle():
 
 
 def test_c1_dense_restatement_agrees_with_paged_oracle():
-  """BASELINE.json configs[0]'s 134M decoder (C1): one prompt, 32 greedy steps."""
+  """The 134M decoder (C1): one prompt, 32 greedy steps."""
   cfg = H.make_config(model_name="c1-134m", per_device_batch_size=1.0, max_prefill_predict_length=64, max_target_length=128,
                       pagedattn_tokens_per_page=32, pagedattn_num_pages=8)
   w = H.synth.synth_weights(cfg, 0)

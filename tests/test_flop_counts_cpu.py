@@ -1,6 +1,6 @@
 """The work counts the measurements are priced in (maxtext-indextts2_amd/maxtext_utils.py) against the golden cases the reference's own tests
-hold (tests/flop_calculation_test.py:99-208: 6 x tokens x published parameter count + causal attention, within 5 %), and against the figures
-SURVEY.md section 8(d) derives for this build's training and prefill rows."""
+hold (tests/flop_calculation_test.py:99-208: 6 x tokens x published parameter count + causal attention, within 5 %), and against figures
+worked out by hand for the training and prefill rows of the 1B model."""
 import importlib
 from types import SimpleNamespace
 
@@ -45,7 +45,7 @@ def test_mixtral_8x7b_reference_case():
 
 
 def test_c3_training_row_of_the_survey():
-  """SURVEY.md section 8(d): C2 dims, 8 x 2048 tokens per GPU -> learnable-weight 148.8 TFLOP + attention 6.6 TFLOP = 155.4 TFLOP per step."""
+  """C2 dims, 8 x 2048 tokens per GPU -> learnable-weight 148.8 TFLOP + attention 6.6 TFLOP = 155.4 TFLOP per step."""
   c = _cfg(per_device_batch_size=8, max_target_length=2048, emb_dim=2048, mlp_dim=7168, num_query_heads=16, num_kv_heads=16, num_decoder_layers=16,
            head_dim=128, vocab_size=264192)
   total, learnable, attention = mu.calculate_tflops_training_per_device(c, log=False)
@@ -64,7 +64,7 @@ def test_gemma_attention_variants_and_prefill_count():
             mlp_dim=10240, num_query_heads=8, num_kv_heads=4, num_decoder_layers=34, head_dim=256, vocab_size=262144)
   att3 = mu.calculate_tflops_training_per_device(g3, log=False)[2]
   assert abs(att3 - (5 * full + 29 * full / 8) / 2 * 3 / 1e12) < 1e-9           # 34 // 6 = 5 global layers, 29 with a 1024-key window
-  # prefill (SURVEY 8(d)): 2 x 256 x 973.2 M + causal attention 4.3e9 at C2
+  # prefill: 2 x 256 x 973.2 M + causal attention 4.3e9 at C2
   c2 = _cfg(num_query_heads=16, num_decoder_layers=16, head_dim=128)
   total, lw, att = mu.calculate_prefill_tflops_per_device(973.2e6, 256, c2, log=False)
   assert abs(lw - 2 * 256 * 973.2e6 / 1e12) < 1e-12 and abs(att - 4.3e9 / 1e12) < 1e-4 and abs(total - lw - att) < 1e-15

@@ -1,4 +1,4 @@
-"""The oracle's Gemma-2 block (SURVEY.md section 8(f) item 3; layers/gemma2.py:69-236, attentions.py:625-631 and :1257-1259,
+"""The oracle's Gemma-2 block (layers/gemma2.py:69-236, attentions.py:625-631 and :1257-1259,
 decoders.py:552-565), checked on the CPU: the scalar restatements against float64 formulas, and the invariants the reference's tests state for
 any decoder (chunked == unchunked, prefill + autoregress == longer prefill) plus the ones the Gemma features add (a window at least as long
 as the sequence changes nothing; a window of w hides exactly the keys at distance >= w; the cap bounds the logits)."""

@@ -1,4 +1,4 @@
-"""The oracle's Gemma-3 block (SURVEY.md section 8(f) item 3; layers/gemma3.py:35-200, attentions.py:1872-1888, :2085-2088, :2246-2265), checked
+"""The oracle's Gemma-3 block (layers/gemma3.py:35-200, attentions.py:1872-1888, :2085-2088, :2246-2265), checked
 on the CPU: the parameter names, the decoder invariants of the reference's tests (chunked == unchunked, prefill + autoregress == longer
 prefill) over a full [5 local, 1 global] pattern, and what the Gemma-3 features add (the head norm against its float64 formula, the local
 layers' own RoPE base, the layer pattern, q * query_pre_attn_scalar)."""

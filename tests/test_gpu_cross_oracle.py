@@ -63,7 +63,7 @@ def test_hip_agrees_with_the_dense_restatement_tiny():
 
 
 def test_hip_agrees_with_the_dense_restatement_c1():
-  """BASELINE.json configs[0]'s 134M decoder: one 64-token prompt, 32 greedy steps."""
+  """The 134M decoder: one 64-token prompt, 32 greedy steps."""
   cfg = H.make_config(model_name="c1-134m", per_device_batch_size=1.0, max_prefill_predict_length=64, max_target_length=128,
                       pagedattn_tokens_per_page=32, pagedattn_num_pages=8)
   w = H.synth.synth_weights(cfg, 0)

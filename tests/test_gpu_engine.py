@@ -132,7 +132,7 @@ def test_tiny_one_launch_decode_attention(B, nprompts, wave_pairs):
 
 
 def test_audio_only_sampling_ranges():
-  """greedy sampling restricted to column ranges (the audio rows of the expanded vocabulary): tokens equal the
+  """Greedy sampling restricted to column ranges (the audio rows of the expanded vocabulary): tokens equal the
   oracle's restricted argmax, all lie inside the ranges, and the returned logits are the unmasked ones (checked by run_pair)."""
   cfg = H.make_config(per_device_batch_size=3.0)
   w = H.synth.synth_weights(cfg, 6)

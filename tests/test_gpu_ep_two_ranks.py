@@ -1,4 +1,4 @@
-"""Expert parallelism on TWO processes sharing the test GPU (SURVEY.md section 8(f) item 4; layers/moe.py:785-938): each process builds a context that
+"""Expert parallelism on TWO processes sharing the test GPU (layers/moe.py:785-938): each process builds a context that
 holds HALF of the experts' kernels (ixt_config.ep_rank / ep_size), routes ITS OWN rows, and the fixed-capacity exchange of moe_ep.py
 (expert_parallel_apply_grouped) carries the (row, k) copies to the process that owns their expert and the results back; the mixture every process
 assembles must equal the oracle's (orc_moe_rows) bit for bit.  The collectives run on gloo (the box has one GPU: RCCL needs one device per rank), so

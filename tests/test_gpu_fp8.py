@@ -1,9 +1,9 @@
-"""GPU tests of IXT-FP8-v1 (`quantization: fp8`, BASELINE.json configs[3]; csrc/ixt_fp8.h).  The reference has no fp8 inference behaviour
+"""GPU tests of IXT-FP8-v1 (`quantization: fp8`; csrc/ixt_fp8.h).  The reference has no fp8 inference behaviour
 (quantizations.py:289-298 is training-only AQT, decode.py:127-128 refuses it), so nothing here is bit-compared with it.  What is checked:
   1. the device's e4m3 conversion == the OCP rule restated in oracle/fp8_ref.py, on a dense sweep of inputs;
   2. the fp8 dot (both kernel forms: split-K below 128 rows, the LDS-ring GEMM from 128 rows) == the float64 restatement of the same
      quantised operands within the matrix cores' accumulation noise (|err| <= 2e-5 x sum of |products|; measured: up to 4.4e-6 -- the instruction aligns
-     and truncates its products much as the bf16 one does, DESIGN.md section 3);
+     and truncates its products much as the bf16 one does);
   3. a model with fp8 projection kernels against the bf16 oracle on the same weights: the error IXT-FP8-v1 costs, stated as tolerances.
 """
 import ctypes

@@ -1,4 +1,4 @@
-"""Size-independent properties at the BASELINE.json sizes of the other two model families (configs[3] Gemma-2 2B with every layer, configs[4]
+"""Size-independent properties at the real sizes of the other two model families (Gemma-2 2B with every layer,
 Mixtral-8x7B widths with four layers), where the CPU oracle would take minutes: chunked prefill == one-chunk prefill, packed prefill == one
 by one, hipGraph decode == eager decode -- bit for bit, on weights drawn on the device (synth.DeviceTree).  The arithmetic itself is
 checked against the oracle at these widths with fewer layers in test_gpu_gemma2.py / test_gpu_mixtral.py."""
@@ -53,7 +53,7 @@ def _chunked_vs_whole_and_graph_vs_eager(model, steps=6, **kw):
 
 
 def test_gemma2_2b_every_layer_chunked_and_graph_invariance():
-  """configs/models/gemma2-2b.yml + the 2048 appended vocabulary rows of BASELINE configs[3], all 13 merged layers (26 sub-layers), window 4096."""
+  """configs/models/gemma2-2b.yml + the 2048 appended vocabulary rows, all 13 merged layers (26 sub-layers), window 4096."""
   _chunked_vs_whole_and_graph_vs_eager("gemma2-2b", vocab_size=256128 + 2048)
 
 
@@ -128,7 +128,7 @@ def _long_prompt_runs(model, total, plans, steps=3, **kw):
 
 
 def test_gemma2_2b_4096_token_chunked_prefill():
-  """BASELINE.json configs[3]'s workload shape: Gemma-2 2B + the 2048 appended vocabulary rows, every layer, ONE 4096-token prompt (the local
+  """A long prompt: Gemma-2 2B + the 2048 appended vocabulary rows, every layer, ONE 4096-token prompt (the local
   sub-layers' window is 4096: the last chunks see the whole prompt).  256-row chunks == 1024-row chunks == one 4096-row pass, hipGraph == eager."""
   _long_prompt_runs("gemma2-2b", 4096, [(256, True), (1024, False), (4096, True)], vocab_size=256128 + 2048)
 

@@ -1,4 +1,4 @@
-"""GPU parity of the Gemma-2 block (SURVEY.md section 8(f) item 3) against the oracle through the engine's call order: tokens, f32 logits
+"""GPU parity of the Gemma-2 block against the oracle through the engine's call order: tokens, f32 logits
 bits (after / sqrt(emb) and the soft cap), K and V of every sub-layer, PageState.  The tiny geometry has every Gemma-2 feature on and a
 sliding window (24) shorter than the sequences, so the local sub-layers really mask."""
 import numpy as np

@@ -1,4 +1,4 @@
-"""GPU parity of the Gemma-3 block (SURVEY.md section 8(f) item 3; layers/gemma3.py:35-200) against the oracle through the engine's call
+"""GPU parity of the Gemma-3 block (layers/gemma3.py:35-200) against the oracle through the engine's call
 order: tokens, f32 logits bits, K and V of every layer, PageState.  The tiny geometry has 7 layers (local x 5, global, local), a window (24)
 shorter than the sequences, two RoPE bases, the query / key head norms and q * head_dim ** -0.5."""
 import numpy as np

@@ -168,7 +168,7 @@ def _packed(prompts):
 
 
 def test_golden_c2_full_decode(c2_weights):
-  """BASELINE.json configs[1] at full size: every one of the 1025 token ids equals the oracle's."""
+  """The 1B model at full size: every one of the 1025 token ids equals the oracle's."""
   g, w = c2_weights
   cfg = H.make_config(model_name="indextts2-1b", per_device_batch_size=1.0, max_prefill_predict_length=256, max_target_length=1280,
                       pagedattn_tokens_per_page=32, pagedattn_num_pages=41)
@@ -234,7 +234,7 @@ def test_decode_harness_reproduces_tiny_golden(capsys):
 
 
 def test_expanded_checkpoint_end_to_end(tmp_path):
-  """SURVEY 8(f) item 1 through the product path: a flat checkpoint is extended by `expand_embedder` (embedding rows + logits
+  """Vocabulary expansion through the product path: a flat checkpoint is extended by `expand_embedder` (embedding rows + logits
   columns, padded to the GEMM tile), saved as .npz, loaded by MaxEngine.load_params() via `load_parameters_path`, and decodes
   the same ids as the oracle on the same expanded weights; sampling restricted to the appended rows picks only appended rows."""
   VE = H.importlib.import_module("maxtext-indextts2_amd.vocab_expansion")

@@ -1,4 +1,4 @@
-"""GPU parity of the Mixtral block (SURVEY.md section 8(f) item 4; layers/mixtral.py:52-170, layers/moe.py) against the oracle through the
+"""GPU parity of the Mixtral block (layers/mixtral.py:52-170, layers/moe.py) against the oracle through the
 engine's call order: tokens, f32 logits bits, K and V of every layer, PageState.  8 experts, 2 per token, 4 query heads per kv head."""
 import numpy as np
 import pytest
@@ -84,7 +84,7 @@ def test_mixtral_8x7b_widths():
 @pytest.mark.parametrize("rccl", [False, True])
 def test_routed_moe_module_with_exchange_matches_oracle(rccl):
   """layers.moe.RoutedMoE over the op-level entry points (route -> exchange -> per-expert MLP -> exchange -> combine) against the oracle's
-  mixture, bit for bit; rccl=True runs the two all-to-alls on a one-rank RCCL group (the expert-parallel code path on this one-GPU box)."""
+  mixture, bit for bit; rccl=True runs the two all-to-alls on a one-rank RCCL group (the expert-parallel code path on one GPU)."""
   import ctypes
   import importlib
   import torch
@@ -216,7 +216,7 @@ def test_expert_sharded_contexts_cover_the_mixture():
     y = torch.where(mine[:, None], part[:R * TK], y)
   whole = full.moe_experts(1, rows, ids)                                # the same through a context with every expert
   assert torch.equal(whole, y)
-  for e in range(NE):                                                   # and through the one-expert op of round 2
+  for e in range(NE):                                                   # and through the one-expert op
     sel = (ids == e).nonzero()[:, 0]
     if sel.numel():
       assert torch.equal(full.moe_expert(1, e, rows[sel].contiguous()), y[sel])

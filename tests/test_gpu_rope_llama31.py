@@ -1,4 +1,4 @@
-"""rope_type "llama3.1" (layers/embeddings.py:354-488 LLaMARotaryEmbedding; SURVEY.md section 8 row a8) on the GPU against the oracle, bit for bit:
+"""rope_type "llama3.1" (layers/embeddings.py:354-488 LLaMARotaryEmbedding) on the GPU against the oracle, bit for bit:
 every kernel that rotates -- the few-rows QKV launch, the split-K path's finalize / decode prologues, the ring GEMM's QKV epilogue, the op-level
 rope -- and the K cache export (the kernels rotate de-interleaved Q / K columns and store the results back in the model's feature order)."""
 import ctypes

@@ -1,5 +1,5 @@
-"""GPU parity of the training step (BASELINE.json configs[2] at test size): Trainer.train_step (HIP, include/ixt_train.h)
-against the f32 PyTorch oracle (oracle/train_oracle.py) on identical batches.  Bars: loss within 1e-4 relative at every step (north_star's
+"""GPU parity of the training step (at test size): Trainer.train_step (HIP, include/ixt_train.h)
+against the f32 PyTorch oracle (oracle/train_oracle.py) on identical batches.  Bars: loss within 1e-4 relative at every step (the project's
 training criterion); raw gradient norm within 3e-3 relative and every gradient tensor within 2 % in L2 of the oracle's (the product rounds its
 backward signals to bf16 where they feed the matrix cores; the oracle does not)."""
 import importlib
@@ -118,7 +118,7 @@ def test_free_running_trajectory_stays_close():
 
 
 def test_train_step_at_the_c3_widths():
-  """BASELINE.json configs[2]'s model at its real widths -- emb 2048, 16 heads of 128, mlp 7168, the 264 192-row audio-expanded vocabulary, 2048-token
+  """The 1B model at its real widths -- emb 2048, 16 heads of 128, mlp 7168, the 264 192-row audio-expanded vocabulary, 2048-token
   rows -- with 2 of its 16 layers and one row per step (the CPU oracle is an f32 torch autograd pass: the logits alone are 2 GB): loss within 1e-4
   relative with synchronised state, raw gradient norm within 3e-3, every gradient tensor within 2 %."""
   import torch

@@ -1,4 +1,4 @@
-"""The oracle's Mixtral block (SURVEY.md section 8(f) item 4; layers/mixtral.py:52-170, layers/moe.py:170-204, :326-345, :420-484, :855-942) on
+"""The oracle's Mixtral block (layers/mixtral.py:52-170, layers/moe.py:170-204, :326-345, :420-484, :855-942) on
 the CPU: routing against numpy (top_k order, ties, softmax over the k logits), the mixture against a float64 formula built from the
 oracle's own per-expert MLP, a one-expert mixture == the llama2 block bit for bit, and the decoder invariants of the reference's tests."""
 import ctypes

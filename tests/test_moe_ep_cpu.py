@@ -1,4 +1,4 @@
-"""Expert-parallel exchange (maxtext-indextts2_amd/moe_ep.py; SURVEY.md section 8(f) item 4): the integer bookkeeping against the cases the
+"""Expert-parallel exchange (maxtext-indextts2_amd/moe_ep.py): the integer bookkeeping against the cases the
 reference's own tests hold (tests/moe_test.py:788-900), and the two-all-to-all exchange on 2 gloo ranks against the single-process result."""
 import importlib
 import socket

@@ -1,5 +1,5 @@
 """CPU suite: the oracle against its committed golden vectors and against the invariants the reference's own tests
-state for this path (SURVEY.md section 4); host logic; and the C-ABI export check (no GPU compute)."""
+state for this path; host logic; and the C-ABI export check (no GPU compute)."""
 import ctypes
 import hashlib
 import os
@@ -97,7 +97,7 @@ def test_prefill_plus_autoregress_equals_longer_prefill(tiny):
 
 
 def test_batch_rows_are_independent(tiny):
-  """A slot's tokens do not depend on what the other slots hold (decode_batch rows are independent units, SURVEY 8e)."""
+  """A slot's tokens do not depend on what the other slots hold (decode_batch rows are independent units)."""
   cfg, w = tiny
   p0 = H.synth.synth_prompt(cfg.vocab_size, 32, 21)
   p1 = H.synth.synth_prompt(cfg.vocab_size, 32, 22)

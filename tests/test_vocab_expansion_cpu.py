@@ -1,4 +1,4 @@
-"""SURVEY.md section 8(f) item 1 on the CPU: the audio-id mapping (pinned by the reference's own data file, in array form under
+"""Vocabulary expansion on the CPU: the audio-id mapping (pinned by the reference's own data file, in array form under
 tests/golden/), the row-append tool, and the oracle's range-restricted greedy sampling."""
 import importlib
 import os
@@ -115,7 +115,7 @@ def test_oracle_sampling_ranges():
 
 
 def test_other_reference_mapping_files_agree(mapping):
-  """The reference ships three mapping data files (SURVEY.md section 8 a15); the adjusted one drives this build.  The other two
+  """The reference ships three mapping data files; the adjusted one drives this build.  The other two
   (vocab_expansion/audio_token_mapping.json, sha256 abf2cbca..., and audio_token_mapping_complete.json, sha256 6644cd61...) are pinned
   here in array form and must tell the same story: same audio-id -> embedding-row table, and tokenizer indices that differ from
   embedding rows by exactly the removed soft token at 262144 (extend_tokenizer.py:40-46)."""

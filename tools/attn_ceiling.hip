@@ -3,7 +3,7 @@
 // 8 KiB each per (page, head), pages scattered by a random page map).  This program reads exactly those bytes with no arithmetic:
 //   (a) "paged":   grid (16 heads, 256 rows) x 256 threads as k_attn_decode, each block its row's pages of its head -- K pieces first, then V pieces
 //   (b) "linear":  the same number of bytes as one contiguous stream, grid-stride (the streaming ceiling of the part)
-// Build + run on the GPU box:  hipcc --offload-arch=gfx950 -O3 tools/attn_ceiling.hip -o /tmp/attn_ceiling && /tmp/attn_ceiling
+// Build + run on an MI355X:  hipcc --offload-arch=gfx950 -O3 tools/attn_ceiling.hip -o /tmp/attn_ceiling && /tmp/attn_ceiling
 #include <hip/hip_runtime.h>
 #include <cstdio>
 #include <cstdint>

@@ -1,5 +1,5 @@
 #!/usr/bin/env python3
-"""Micro-benchmark of the canonical DOT kernel on the decode/prefill shapes of C2 (run on the GPU box)."""
+"""Micro-benchmark of the canonical DOT kernel on the decode/prefill shapes of C2 (run on an MI355X)."""
 import ctypes
 import importlib
 import os
@@ -29,7 +29,7 @@ def main():
   if max(rows) >= 128:
     variants += [("ring 128x128", {"ring_cfg": 1}), ("ring 128x64", {"ring_cfg": 2}), ("ring 64x32", {"ring_cfg": 3}), ("ring split", {"ring_split": 1}), ("ring 128x128 ring-layout W", {"ring_cfg": 1, "ring_wlayout": 1}),
                  ("ring 128x64 ring-layout W", {"ring_cfg": 2, "ring_wlayout": 1}), ("ring 64x32 ring-layout W", {"ring_cfg": 3, "ring_wlayout": 1}),
-                 ("k_gemm / k_dotb (round 1)", {"ring_min_rows": 1 << 30})]
+                 ("k_gemm / k_dotb", {"ring_min_rows": 1 << 30})]
   for R in rows:
    for label, opts in (variants if R >= 128 else variants[:1]):
     for k, v in opts.items():

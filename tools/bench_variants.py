@@ -1,5 +1,5 @@
 #!/usr/bin/env python3
-"""Rates of the two other model families of SURVEY.md section 8(f) at their BASELINE.json sizes, one GPU, synthetic
+"""Rates of the two other model families (Gemma-2 2B, Mixtral-8x7B), one GPU, synthetic
 weights drawn ON the device (the trees are 5 GB and 93 GB; the host-side generator of synth.py would take minutes):
 
   gemma2   Gemma-2 2B (configs/models/gemma2-2b.yml) + 2048 appended vocabulary rows: one 4096-token prompt through the chunked prefill in

@@ -1,7 +1,7 @@
 #!/usr/bin/env python3
-"""BASELINE.json configs[2] on ONE GPU's share: the 1B IndexTTS2-style decoder (vocab 264192), per-device batch 8 x 2048 tokens
+"""A training step on ONE GPU's share: the 1B IndexTTS2-style decoder (vocab 264192), per-device batch 8 x 2048 tokens
 (example_audio_training.py:69: max_target_length=2048; 64 utterances over 8 GPUs), a few train steps on a synthetic batch.
-Reports step time, tokens/s and TFLOP/s against SURVEY.md section 8(d)'s 155.4 TFLOP per step per GPU.  Run on the GPU box."""
+Reports step time, tokens/s and TFLOP/s against 155.4 TFLOP per step per GPU.  Run on an MI355X."""
 import importlib
 import json
 import os
@@ -43,7 +43,7 @@ def main():
     print(f"[train_bench] step {i}: loss {m['learning/loss']:.4f} raw_grad_norm {m['learning/raw_grad_norm']:.4f} lr {m['learning/current_learning_rate']:.2e} "
           f"{m['step_s']:.3f} s", file=sys.stderr, flush=True)
   best = min(m["step_s"] for m in out[1:]) if steps > 1 else out[0]["step_s"]
-  # the reference's own count (maxtext_utils.calculate_tflops_training_per_device; SURVEY.md 8(d): 155.4 TFLOP per step per GPU at 8 x 2048)
+  # the reference's own count (maxtext_utils.calculate_tflops_training_per_device): 155.4 TFLOP per step per GPU at 8 x 2048
   tflop = importlib.import_module("maxtext-indextts2_amd.maxtext_utils").calculate_tflops_training_per_device(cfg, log=False)[0]
   print(json.dumps({"config": f"C3 share: indextts2-1b, per_device_batch {pdb} x {S} tokens, 1 GPU", "steps": steps, "step_s": best, "tokens_per_s": pdb * S / best,
                     "tflop_per_s": tflop / best, "mfu_bf16": tflop / best / 2500.0, "losses": [m["learning/loss"] for m in out], "ln_vocab": float(np.log(cfg.vocab_size))}))
