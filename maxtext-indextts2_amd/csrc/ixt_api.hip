@@ -358,6 +358,7 @@ extern "C" int ixt_create(const ixt_config* cfg, ixt_ctx** out) {
   hipLaunchKernelGGL(k_pages_reset, dim3(1), dim3(64), 0, 0, x->ps);
   if (hipDeviceSynchronize() != hipSuccess) return fail(set_err(IXT_ERR_HIP, "page state init failed"));
   if (sdot_set_attributes() != IXT_OK) return fail(IXT_ERR_HIP);
+  if (!hybrid && step_init(x) != IXT_OK) return fail(IXT_ERR_HIP);
   *out = x;
   return IXT_OK;
 }
@@ -1648,6 +1649,17 @@ static bool small_path_ok(const ixt_ctx* c, int R) {
 static int forward_rows_small(ixt_ctx* c, int R, const int32_t* tokens, int len_hint, int lrow0, int nl, const int32_t* lrows, int32_t* argmax_out,
                               float* logits_out, bool decode, hipStream_t st) {
   const int E = c->E, F = c->F;
+  if (c->small_step && c->small_norm && !c->timing && step_fits(c, R) && !(decode && attn_split_factor(c, R) > 1)) {
+    const bf16_t* h = nullptr;
+    TRY(launch_step(c, R, tokens, decode ? 0 : c->one_segment ? R : c->Tmax, &h, st));
+    if (nl > 0) {
+      if (nl > c->NLmax) return set_err(IXT_ERR_INVALID, "too many logits rows (%d > %d)", nl, c->NLmax);
+      TRY(launch_rownorm(c, 2, nl, nullptr, nullptr, lrows ? h : h + (size_t)lrow0 * E, nullptr, c->final_norm, c->xn, st, 1, lrows));
+      TRY(launch_unembed(c, c->xn, nl, logits_out, argmax_out, st));
+    }
+    c->h_final = h; c->h_final_rows = R;
+    return IXT_OK;
+  }
   bf16_t* hcur = c->h_a;
   bf16_t* hnext = c->h_b;
   const bool down_small = sdot_plan(c, GEPI_RESID, false, F, E, R).ok;
@@ -2236,7 +2248,7 @@ extern "C" int ixt_set_option(ixt_ctx* c, const char* name, int value) {
       {"gemm_split_min_blocks", &c->gemm_split_min_blocks, 1}, {"gemm_min_blocks", &c->gemm_min_blocks, 1}, {"gemm_min_rows", &c->gemm_min_rows, 1},
       {"unembed_gemm", &c->unembed_gemm, 0}, {"attn_wave_pairs", &c->attn_wave_pairs, 0}, {"attn_tile", &c->attn_tile, 0}, {"attn_tile_min_rows", &c->attn_tile_min_rows, 1}, {"dot_stream_min_blocks", &c->dot_stream_min_blocks, 1},
       {"ring_min_rows", &c->ring_min_rows, 1}, {"ring_mid_rows", &c->ring_mid_rows, 17}, {"ring_cfg", &c->ring_cfg, 0}, {"ring_split", &c->ring_split, 0}, {"ring_wlayout", &c->ring_wlayout, 0}, {"ring_down", &c->ring_down, -1}, {"unembed_tall", &c->unembed_tall, 0}, {"ring_two_per_cu", &c->ring_two_per_cu, 0},
-      {"small_rows", &c->small_rows, 0}, {"small_tpb", &c->small_tpb, 0}, {"small_attn_waves", &c->small_attn_waves, 4}, {"small_attn_max_blocks", &c->small_attn_max_blocks, 0}, {"dot_small", &c->dot_small, 0}, {"small_norm", &c->small_norm, 0}, {"small_prefetch", &c->small_prefetch, 0}, {"small_prefetch_blocks", &c->small_prefetch_blocks, 1}, {"moe_grouped", &c->moe_grouped, 0}, {"small_attn_split", &c->small_attn_split, 0}, {"moe_route_blocks", &c->moe_route_blocks, 0}, {"gemma_tile", &c->gemma_tile, 0}, {"moe_fused_gate", &c->moe_fused_gate, 0}, {"moe_mid_pairs", &c->moe_mid_pairs, 0},
+      {"small_rows", &c->small_rows, 0}, {"small_tpb", &c->small_tpb, 0}, {"small_attn_waves", &c->small_attn_waves, 4}, {"small_attn_max_blocks", &c->small_attn_max_blocks, 0}, {"dot_small", &c->dot_small, 0}, {"small_step", &c->small_step, 0}, {"small_norm", &c->small_norm, 0}, {"small_prefetch", &c->small_prefetch, 0}, {"small_prefetch_blocks", &c->small_prefetch_blocks, 1}, {"moe_grouped", &c->moe_grouped, 0}, {"small_attn_split", &c->small_attn_split, 0}, {"moe_route_blocks", &c->moe_route_blocks, 0}, {"gemma_tile", &c->gemma_tile, 0}, {"moe_fused_gate", &c->moe_fused_gate, 0}, {"moe_mid_pairs", &c->moe_mid_pairs, 0},
   };
   for (const Opt& o : opts) {
     if (strcmp(name, o.name) != 0) continue;

@@ -122,6 +122,10 @@ struct ixt_ctx {
   size_t split_stride = 0;
   int small_prefetch = 0;    // few-rows path: prefetch blocks stream the next launch's kernel into the Infinity Cache (ixt_prefetch).  Measured SLOWER (one utterance 1.19 against 1.03 ms per step, eight 1.33 against 1.23: a launch cannot end before its prefetch has, and an Infinity-Cache hit is only 1.4 x an HBM stream): off
   int small_prefetch_blocks = 64;
+  int small_step = 1;        // few rows: all layers in one launch (k_step) where the shapes allow; 0: five launches a layer
+  struct StepLayer* step_layers = nullptr;   // [L] in HBM; nullptr: not this model
+  bf16_t* step_ws = nullptr;
+  int32_t* step_cnt = nullptr;
   int small_norm = 1;        // 1: the RMSNorm in front of the QKV / wi projections runs inside k_sdot; 0: k_rownorm launches (experiments)
   int dot_stream_min_blocks = 1 << 30;   // off: measured slower than split-K at 256 rows (decode 7.84 vs 7.68 ms/step, prefill 3.53 vs 3.31 ms)
   ColRanges sample_cols{};   // greedy sampling restricted to these columns (n == 0: all)
@@ -184,3 +188,7 @@ int launch_dot(ixt_ctx* c, const bf16_t* x, const bf16_t* w, int K, int N, int R
 SdotPlan sdot_plan(const ixt_ctx* c, int epi, bool norm, int K, int N, int R);
 int launch_sdot(ixt_ctx* c, int epi, bool norm, const bf16_t* x, const bf16_t* scale, const bf16_t* w, int K, int N, int R, const GemmEpi& e, hipStream_t st,
                 const bf16_t* pf = nullptr, size_t pf_elems = 0);
+// ---- few rows, all layers in one launch (ixt_step.hip)
+int step_init(ixt_ctx* c);
+bool step_fits(const ixt_ctx* c, int R);
+int launch_step(ixt_ctx* c, int R, const int32_t* tokens, int fresh, const bf16_t** hidden, hipStream_t st);
