@@ -126,6 +126,7 @@ struct ixt_ctx {
   struct StepLayer* step_layers = nullptr;   // [L] in HBM; nullptr: not this model
   bf16_t* step_ws = nullptr;
   int32_t* step_cnt = nullptr;
+  int32_t step_token = 0;
   int small_norm = 1;        // 1: the RMSNorm in front of the QKV / wi projections runs inside k_sdot; 0: k_rownorm launches (experiments)
   int dot_stream_min_blocks = 1 << 30;   // off: measured slower than split-K at 256 rows (decode 7.84 vs 7.68 ms/step, prefill 3.53 vs 3.31 ms)
   ColRanges sample_cols{};   // greedy sampling restricted to these columns (n == 0: all)

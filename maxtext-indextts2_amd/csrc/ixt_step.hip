@@ -2,6 +2,8 @@
 #include "ixt_internal.h"
 #include "ixt_step.h"
 
+#include <atomic>
+
 // Which shapes: those whose rows, normed, and whose attention's pages fit the LDS of a CU and whose (tile, chain) pairs fit a block; other models of few rows take the
 // launches of ixt_small.h.
 #define STEP_LDS (150 * 1024)
@@ -52,13 +54,15 @@ int step_init(ixt_ctx* c) {
   if (c->moe || c->gemma || c->fp8 || c->L < 1 || !step_plan(c, 1).ok) return IXT_OK;
   TRY(dmalloc(c, &c->step_layers, (size_t)c->L));
   TRY(dmalloc(c, &c->step_ws, (size_t)c->L * 16 * (2 * c->QN + 2 * c->E + c->F)));
-  TRY(dmalloc(c, &c->step_cnt, (size_t)c->L * STEP_PHASES * STEP_NS * 32));
+  TRY(dmalloc(c, &c->step_cnt, ((size_t)c->L * STEP_PHASES * STEP_NS + 1) * 32));
   std::vector<StepLayer> t((size_t)c->L);
   auto at = [&](const void* p) { return (int64_t)(reinterpret_cast<intptr_t>(p) - reinterpret_cast<intptr_t>(c->step_ws)); };
   for (int l = 0; l < c->L; ++l) {
     const LayerW& w = c->layers[l];
     t[l] = StepLayer{at(w.wqkv), at(w.wo), at(w.wi), at(w.wout), at(w.ln1), at(w.ln2), at(c->kpages_l[l]), at(c->vpages_l[l])};
   }
+  static std::atomic<int32_t> contexts{0};
+  c->step_token = contexts.fetch_add(1) % 0x7fffffff + 1;
   HIPCHK(hipMemcpy(c->step_layers, t.data(), sizeof(StepLayer) * t.size(), hipMemcpyHostToDevice));
   return IXT_OK;
 }
@@ -70,12 +74,12 @@ int launch_step(ixt_ctx* c, int R, const int32_t* tokens, int fresh, const bf16_
   a.layers = c->step_layers; a.ws = c->step_ws; a.lstride = (size_t)16 * (2 * c->QN + 2 * c->E + c->F);
   a.h0 = c->h_a; a.cnt = c->step_cnt; a.err = c->split_cnt + (size_t)16 * c->KV * 4;
   a.R = R; a.E = c->E; a.F = c->F; a.QN = c->QN; a.NQKV = c->NQKV; a.rpl = p.rpl; a.fresh = fresh;
-  a.per_layer = 0; a.attw = p.attw; a.att_floats = p.att_floats; a.early = p.early;
+  a.token = c->step_token; a.nl = c->L; a.per_layer = 0; a.attw = p.attw; a.att_floats = p.att_floats; a.early = p.early;
   for (int i = 0; i < STEP_PHASES; ++i) { a.nblk[i] = p.nblk[i]; a.tpb[i] = p.tpb[i]; a.per_layer += p.nblk[i]; }
   a.eps = c->cfg.normalization_layer_epsilon;
   a.row_slot = c->row_slot; a.row_pos = c->row_pos; a.row_active = c->row_active; a.page_map = c->ps.page_map;
   a.rope_sin = c->rope_sin; a.rope_cos = c->rope_cos; a.g = c->geom;
-  hipLaunchKernelGGL(k_step_begin, dim3(R), dim3(256), 0, st, tokens, c->embedding, c->E, c->h_a, c->step_cnt, c->L * STEP_PHASES * STEP_NS);
+  hipLaunchKernelGGL(k_step_begin, dim3(R), dim3(256), 0, st, tokens, c->embedding, c->E, c->h_a, c->step_cnt, c->L * STEP_PHASES * STEP_NS + 1, a.token, a.err);
   LAUNCHCHK();
   *hidden = c->step_ws + (size_t)c->L * a.lstride - (size_t)16 * c->E;
 #define ST(HD_, GQ_) if (c->D == HD_ && c->GQ == GQ_) return launch_step_t<HD_, GQ_>(a, c->L, p.lds, st);

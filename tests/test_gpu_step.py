@@ -71,3 +71,41 @@ def test_packed_rows():
     del eng
     torch.cuda.synchronize()
   assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
+
+
+def test_passes_of_two_engines_on_two_streams():
+  """Steps of two models in flight on two streams: the launches take turns (each would hold compute units that the other's blocks have to start on), and every
+  token is what a model alone gives."""
+  import torch
+  lens, steps = (33, 20), 200
+  cfgs = [_config(1, 2048, 16, 16, 128, 7168, 33 + steps, 2), _config(1, 768, 12, 12, 64, 2048, 33 + steps, 6)]
+  engines = [H.make_engine(cfg, H.synth.synth_weights(cfg, i)) for i, cfg in enumerate(cfgs)]
+  streams = [torch.cuda.Stream() for _ in cfgs]
+
+  def begin(i):
+    toks = H.synth.synth_prompt(cfgs[i].vocab_size, 33, i)[0]
+    eng, params = engines[i]
+    prefix, _ = eng.prefill(params=params, padded_tokens=toks, true_length=lens[i], slot=0)
+    return eng.insert(prefix, eng.init_decode_state(), 0)
+
+  def run(together):
+    out, states = [[], []], [None, None]
+    order = [0, 1] * steps if together else [0] * steps + [1] * steps
+    for i in (0, 1):
+      with torch.cuda.stream(streams[i]):
+        states[i] = begin(i)
+    torch.cuda.synchronize()
+    for i in order:
+      with torch.cuda.stream(streams[i]):
+        states[i], result = engines[i][0].generate(engines[i][1], states[i])
+        out[i].append(result.data.clone())
+      if not together:
+        streams[i].synchronize()
+    torch.cuda.synchronize()
+    for i in (0, 1):
+      assert engines[i][0].exchange_status() == 0
+      engines[i][0].release_pages(0)
+    return [torch.stack(o).cpu().numpy() for o in out]
+
+  alone, both = run(False), run(True)
+  assert all(np.array_equal(x, y) for x, y in zip(alone, both))
