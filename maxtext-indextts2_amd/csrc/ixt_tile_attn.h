@@ -7,6 +7,8 @@
 #pragma once
 #include "ixt_kernels.h"
 
+#include <type_traits>
+
 typedef float ixt_f32x4 __attribute__((ext_vector_type(4)));
 
 // rows 1 and 3 of `a` (16 lanes each) against rows 0 and 2 of `b` / the upper half of `a` against the lower half of `b`
@@ -49,10 +51,15 @@ __device__ __forceinline__ void ixt_k_operands(const u32x4& w, uint32_t sel, flo
 // Rows of other page groups in the tile are worked off group by group, dealt among `shares` blocks.  grid = (kv heads, tiles, parts x shares): parts = 1 or
 // the number of 128-column parts of a value (the two halves of head_dim 256 in two blocks, each taking the scores anew), shares = 1 or more, both for
 // launches that leave CUs idle otherwise.
-// Bound by the matrix units and, between their phases, by the vector work of the softmax (a block's waves are in the same phase).  Measured against
-// k_attn_tile, 16 heads of 128: 8 packed prompts (1525 rows, <= 251 keys) 128.6 -> 69.6 us; 1024 rows at <= 1024 / 2048 / 3072 keys 282 -> 106,
-// 860 -> 215, 1143 -> 356 us; 828 rows at <= 3900 keys 1496 -> 455 us (52 TFLOP/s).  8 heads of 256 on 4, 256 rows at <= 3072 keys: 320 -> 130 us.
-// Two waves per block for <= 256 keys: with four, two of them had nothing to do (90.2 us).
+// Bound by the matrix units and the vector units TOGETHER: an f32 product and a vector instruction of the same SIMD take turns, whichever waves they belong to (products
+// alone 150 TFLOP/s; one bf16 -> f32 conversion in front of each 116, eight in front of eight 129).  So what counts is vector instructions: operands of a
+// step converted together, no mask where every row sees every key (sees_all; the selects of a score were a branch each), weights rounded and packed two at a time ahead
+// of the transpose.  Tried without gain: the keys of the next super-block requested ahead, page numbers in a register, a priority for half of the waves;
+// 4-byte loads of the keys that need no lane swaps (2.3 x slower).  Keys and values widened to f32 by a launch ahead take another 15 % off here and cost 11 to 22 us for 1024 to
+// 3900 keys: level up to 2048.
+// Measured against k_attn_tile, 16 heads of 128, 1024 rows at <= 1024 / 2048 / 3072 keys 282 / 860 / 1143 us; before the instructions above and the forms
+// <4, 2> and <8, 3>: 112 / 215 / 351, now 88 / 195 / 302.  828 rows at <= 3900 keys 1496, 448, 411 us (57 TFLOP/s).  8 heads of 256 on 4, 256 rows at <= 3000 keys: 151 -> 130 us.
+// 8 packed prompts (1525 rows, <= 251 keys) 128.6, 68.8, 67.6: two waves per block for <= 256 keys, with four, two of them had nothing to do (90.2 us).
 template <int HD, int GQ, int NW, int NR>
 __global__ __launch_bounds__(NW * 64, NR == 1 && NW <= 4 ? 3 : 2) void k_attn_mtile(TileAttnArgs a) {
   constexpr int TQ = 16 / GQ;
@@ -104,12 +111,12 @@ __global__ __launch_bounds__(NW * 64, NR == 1 && NW <= 4 ? 3 : 2) void k_attn_mt
     const int lead = __builtin_ctz(pending);
     const int slot = __builtin_amdgcn_readfirstlane(s_slot[lead]);
     unsigned grp = 0;
-    int posmax = -1;
+    int posmax = -1, posmin = a.lmax;
 #pragma unroll
     for (int i = 0; i < TQ; ++i) {
       const int ps_ = __builtin_amdgcn_readfirstlane(s_pos[i]), sl_ = __builtin_amdgcn_readfirstlane(s_slot[i]);
       const bool in = ((pending >> i) & 1u) && sl_ == slot && ps_ < a.lmax;
-      if (in) { grp |= 1u << i; posmax = max(posmax, ps_); }
+      if (in) { grp |= 1u << i; posmax = max(posmax, ps_); posmin = min(posmin, ps_); }
     }
     if (((grp >> lead) & 1u) == 0) {                     // the leader reaches beyond the keys a block holds (the caller's max_len guard prevents it): zeros
       if (blockIdx.z == 0)
@@ -124,6 +131,9 @@ __global__ __launch_bounds__(NW * 64, NR == 1 && NW <= 4 ? 3 : 2) void k_attn_mt
     const int kv_all = posmax + 1, pages_all = (kv_all + 31) >> 5, nsb = (pages_all + IXT_SB - 1) / IXT_SB;
     const int32_t* prow = a.page_map + (size_t)slot * g.mpg;
     const int mypos = ((grp >> (i16 / GQ)) & 1u) ? s_pos[i16 / GQ] : -1;
+
+    // every row of the group sees every key of the super-block (a vector of another group may see any: it is not stored)
+    auto sees_all = [&](int sb) { return sb * 128 + 127 <= posmin && (a.window <= 0 || posmax - a.window < sb * 128); };
 
     // ---- scores
     ixt_f32x4 S[NR][8];
@@ -153,6 +163,7 @@ __global__ __launch_bounds__(NW * 64, NR == 1 && NW <= 4 ? 3 : 2) void k_attn_mt
             float x[8], y[8];
             ixt_k_operands(kr[b & 1][t], sel, x);
             ixt_k_operands(kr[b & 1][t + 1], sel, y);
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int s = 0; s < 8; ++s) {
               S[n][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[s], q8[s], S[n][t], 0, 0, 0);
@@ -171,16 +182,20 @@ __global__ __launch_bounds__(NW * 64, NR == 1 && NW <= 4 ? 3 : 2) void k_attn_mt
             __builtin_amdgcn_sched_barrier(0);
           }
         }
+        auto range = [&](auto masked) {
 #pragma unroll
-        for (int t = 0; t < 8; ++t) {
+          for (int t = 0; t < 8; ++t) {
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const int k = 4 * t + r;
-            mn = fminf(mn, S[n][t][r]);
-            mx = (k <= lim && k > lo) ? fmaxf(mx, S[n][t][r]) : mx;
+            for (int r = 0; r < 4; ++r) {
+              const int k = 4 * t + r;
+              mn = fminf(mn, S[n][t][r]);
+              mx = fmaxf(mx, !masked.value || (k <= lim && k > lo) ? S[n][t][r] : -INFINITY);
+            }
+            __builtin_amdgcn_sched_barrier(0);
           }
-          __builtin_amdgcn_sched_barrier(0);
-        }
+        };
+        if (sees_all(sb)) range(std::false_type());
+        else range(std::true_type());
       }
     }
     // ---- softmax
@@ -196,17 +211,21 @@ __global__ __launch_bounds__(NW * 64, NR == 1 && NW <= 4 ? 3 : 2) void k_attn_mt
       if (sb < nsb) {
         const int lim = mypos - sb * 128 - lg * 32, lo = a.window > 0 ? lim - a.window : -1;
         float sacc = 0.0f;
+        auto exps = [&](auto masked) {
 #pragma unroll
-        for (int t = 0; t < 8; ++t) {
+          for (int t = 0; t < 8; ++t) {
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const int k = 4 * t + r;
-            const float e = ixt_exp(S[n][t][r] - mx);
-            S[n][t][r] = (k <= lim && k > lo) ? e : 0.0f;
-            sacc = sacc + S[n][t][r];
+            for (int r = 0; r < 4; ++r) {
+              const int k = 4 * t + r;
+              const float e = ixt_exp(S[n][t][r] - mx);
+              S[n][t][r] = !masked.value || (k <= lim && k > lo) ? e : 0.0f;
+              sacc = sacc + S[n][t][r];
+            }
+            __builtin_amdgcn_sched_barrier(0);
           }
-          __builtin_amdgcn_sched_barrier(0);
-        }
+        };
+        if (sees_all(sb)) exps(std::false_type());
+        else exps(std::true_type());
         psum[(4 * sb + lg) * 16 + i16] = sacc;
       }
     }
@@ -219,20 +238,21 @@ __global__ __launch_bounds__(NW * 64, NR == 1 && NW <= 4 ? 3 : 2) void k_attn_mt
     if (!(l > 0.0f)) l = 1.0f;                           // a vector of another group
     const float rl = 1.0f / l;
     uint32_t P[NR][8][2];                                // bf16 pairs: pages 2 k (low half) and 2 k + 1 of the super-block, token 4 t + lg
+    const uint32_t half = (lg & 1) ? 0x07060302u : 0x05040100u;      // the lane group's token of either page
     auto weights = [&](auto quotient) {
 #pragma unroll
       for (int n = 0; n < NR; ++n) {
         if (n * NW + wave < nsb) {
 #pragma unroll
           for (int t = 0; t < 8; ++t) {
-            uint32_t u[4];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) u[r] = __float_as_uint(rbf(quotient(S[n][t][r])));
-            // register = token of the lane's page -> register = page, lane group = token
-            ixt_swap32(u[0], u[2]); ixt_swap32(u[1], u[3]);
-            ixt_swap16(u[0], u[1]); ixt_swap16(u[2], u[3]);
-#pragma unroll
-            for (int k = 0; k < 2; ++k) P[n][t][k] = (u[2 * k] >> 16) | u[2 * k + 1];
+            // bf16 pairs of tokens of the lane's page -> pairs of pages, lane group = token
+            uint32_t u = pack2(f2bf(quotient(S[n][t][0])), f2bf(quotient(S[n][t][1]))), v = pack2(f2bf(quotient(S[n][t][2])), f2bf(quotient(S[n][t][3])));
+            ixt_swap32(u, v);                            // u: pages 0, 1, v: pages 2, 3; lane groups 0, 1: tokens 0 and 1, 2, 3: tokens 2 and 3
+            uint32_t u1 = u, v1 = v;
+            ixt_swap16(u, u1);
+            ixt_swap16(v, v1);
+            P[n][t][0] = __builtin_amdgcn_perm(u1, u, half);
+            P[n][t][1] = __builtin_amdgcn_perm(v1, v, half);
             __builtin_amdgcn_sched_barrier(0);
           }
         }
@@ -281,14 +301,24 @@ __global__ __launch_bounds__(NW * 64, NR == 1 && NW <= 4 ? 3 : 2) void k_attn_mt
               ixt_f32x4 acc[NE];
 #pragma unroll
               for (int x = 0; x < NE; ++x) acc[x] = ixt_f32x4(0.0f);
+              // a step's operands all ahead of its products: one right in front of its own takes two empty cycles more
+              auto values = [&](const u32x4& v, float pv) {
+                float f[NE];
+#pragma unroll
+                for (int x = 0; x < NE; ++x) {
+                  f[x] = (x & 1) ? bfhi(v[x >> 1]) : bflo(v[x >> 1]);
+                  asm volatile("" : "+v"(f[x]));
+                }
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int x = 0; x < NE; ++x) acc[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(f[x], pv, acc[x], 0, 0, 0);
+              };
               fetch(vb, p, 4);
               __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
               for (int t = 0; t < 4; ++t) {
                 const float pv = (pg & 1) ? bfhi(P[n][t][pg >> 1]) : bflo(P[n][t][pg >> 1]);
-#pragma unroll
-                for (int x = 0; x < NE; ++x)
-                  acc[x] = __builtin_amdgcn_mfma_f32_16x16x4f32((x & 1) ? bfhi(va[t][x >> 1]) : bflo(va[t][x >> 1]), pv, acc[x], 0, 0, 0);
+                values(va[t], pv);
                 __builtin_amdgcn_sched_barrier(0);
               }
               if (pg + 1 < np) fetch(va, p + 1, 0);
@@ -296,9 +326,7 @@ __global__ __launch_bounds__(NW * 64, NR == 1 && NW <= 4 ? 3 : 2) void k_attn_mt
 #pragma unroll
               for (int t = 0; t < 4; ++t) {
                 const float pv = (pg & 1) ? bfhi(P[n][4 + t][pg >> 1]) : bflo(P[n][4 + t][pg >> 1]);
-#pragma unroll
-                for (int x = 0; x < NE; ++x)
-                  acc[x] = __builtin_amdgcn_mfma_f32_16x16x4f32((x & 1) ? bfhi(vb[t][x >> 1]) : bflo(vb[t][x >> 1]), pv, acc[x], 0, 0, 0);
+                values(vb[t], pv);
                 __builtin_amdgcn_sched_barrier(0);
               }
 #pragma unroll
@@ -313,9 +341,11 @@ __global__ __launch_bounds__(NW * 64, NR == 1 && NW <= 4 ? 3 : 2) void k_attn_mt
         for (int h = 0; h < 2; ++h) {
           __syncthreads();
 #pragma unroll
-          for (int r = 0; r < 4; ++r)
-#pragma unroll
-            for (int x = 0; x < NEH; ++x) ob[(wave * 16 + i16) * OP + (4 * lg + r) * NEH + x] = ss[h * NEH + x][r];
+          for (int r = 0; r < 4; ++r) {
+            float* o = ob + (wave * 16 + i16) * OP + (4 * lg + r) * NEH;
+            if constexpr (NEH == 4) *reinterpret_cast<float4*>(o) = make_float4(ss[h * NEH][r], ss[h * NEH + 1][r], ss[h * NEH + 2][r], ss[h * NEH + 3][r]);
+            else *reinterpret_cast<float2*>(o) = make_float2(ss[h * NEH][r], ss[h * NEH + 1][r]);
+          }
           __syncthreads();
 #pragma unroll
           for (int k = 0; k < NTOT; ++k) {

@@ -15,8 +15,14 @@ static void mtile_attn_t(TileAttnArgs ta, hipStream_t st) {
   const dim3 grid(ta.g.nkv, tiles, ta.parts * std::min(TQ, std::max(1, 256 / (blocks * ta.parts))));
   if (ta.lmax <= 256) hipLaunchKernelGGL((k_attn_mtile<HD, GQ, 2, 1>), grid, dim3(128), 0, st, ta);
   else if (ta.lmax <= 512) hipLaunchKernelGGL((k_attn_mtile<HD, GQ, 4, 1>), grid, dim3(256), 0, st, ta);
+  // more than one block a CU: two of four waves side by side (256 registers a wave; one block's softmax and exchange under the other's products), else all the waves a CU has room
+  // for in one.  16 heads of 128 at <= 1024 keys, us of <8, 1> / <4, 2>: 256 blocks 32.0 / 37.8, 320 61.2 / 57.9, 512 64.0 / 58.1, 1024 105 / 88.  With twice the keys two blocks' scores
+  // take every register: level
+  else if (ta.lmax <= 1024 && (int)(grid.x * grid.y * ta.parts) > 256) hipLaunchKernelGGL((k_attn_mtile<HD, GQ, 4, 2>), grid, dim3(256), 0, st, ta);
   else if (ta.lmax <= 1024) hipLaunchKernelGGL((k_attn_mtile<HD, GQ, 8, 1>), grid, dim3(512), 0, st, ta);
   else if (ta.lmax <= 2048) hipLaunchKernelGGL((k_attn_mtile<HD, GQ, 8, 2>), grid, dim3(512), 0, st, ta);
+  // (the scores of three rounds leave registers that those of four do not: 1024 rows at <= 3072 keys 322 -> 302 us)
+  else if (ta.lmax <= 3072) hipLaunchKernelGGL((k_attn_mtile<HD, GQ, 8, 3>), grid, dim3(512), 0, st, ta);
   else hipLaunchKernelGGL((k_attn_mtile<HD, GQ, 8, 4>), grid, dim3(512), 0, st, ta);
 }
 bool launch_mtile_attn(const TileAttnArgs& ta, int hd, int gq, hipStream_t st) {
