@@ -1743,6 +1743,40 @@ static int forward_rows(ixt_ctx* c, int R, const int32_t* tokens, int len_hint, 
   const bool attn_one_launch = R * c->KV >= fused_min && fused_lds <= 64 * 1024;
   const bool ring = R >= ring_model_rows(c, decode) && !c->moe && !c->fp8;   // fp8: the dots write scaled f32 slices, the bf16 path's row kernels take it from there   // Mixtral: the split-K dots (every expert is a launch sequence of its own)
   const bool attn_tiled = tile_attn_fits(c, R, len_hint, decode);   // prefill rows: consecutive rows share their page group's K and V loads
+  // q from its buffer, keys and values (the new ones too) from the pages
+  auto attention = [&](int l) -> int {
+    if (attn_tiled) {
+      TRY(launch_attention_tile(c, l, R, len_hint, st));
+    } else if (attn_one_launch) {
+      const DotResult none{0, 0, 0};
+      const int ta = decode ? timing_begin(c, st, 0.0, 1) : -1;
+      // at most one block on a CU: eight waves with everything in flight (128 rows x 1 kv head of two query heads of 128, 1500 keys: 421 us a step of four layers with
+      // four waves, 351 with eight; 700 keys 302 -> 260; 64 keys 231 -> 229); with more the four-wave form is the faster one (40 rows x 12 heads of 64: 20.3 against 13.7 us)
+      if (decode && (long)R * c->KV <= c->small_attn_max_blocks / 2 && attn_small_fits(c, R)) TRY(launch_attn_small(c, l, R, st));
+      else TRY(launch_attention_fused(c, l, R, none, false, decode, st));   // q from qbuf, every key / value (the new ones too) from the pages
+      timing_end(c, st, ta);
+    } else {
+      TRY(launch_attention_partials(c, l, R, len_hint, DotResult{0, 0, 0}, false, st));
+      hipLaunchKernelGGL(k_attn_combine, dim3(R), dim3(256), 0, st, c->pvpart, c->row_pos, c->row_active, c->ao, c->geom, 1);
+      LAUNCHCHK();
+    }
+    return IXT_OK;
+  };
+  if (c->mid_rows > 0 && !c->timing && !c->moe && !c->fp8 && mid_fits(c, R)) {
+    const bf16_t *h = nullptr, *xn = nullptr;
+    TRY(launch_mid(c, R, -1, tokens, false, nullptr, nullptr, st));
+    for (int l = 0; l < c->L; ++l) {
+      TRY(attention(l));
+      TRY(launch_mid(c, R, l, nullptr, final_fused, &h, &xn, st));
+    }
+    if (nl > 0) {
+      if (nl > c->NLmax) return set_err(IXT_ERR_INVALID, "too many logits rows (%d > %d)", nl, c->NLmax);
+      if (!final_fused) TRY(launch_rownorm(c, 2, nl, nullptr, nullptr, lrows ? h : h + (size_t)lrow0 * E, nullptr, c->final_norm, c->xn, st, 1, lrows));
+      TRY(launch_unembed(c, final_fused ? xn : c->xn, nl, logits_out, argmax_out, st));
+    }
+    c->h_final = h; c->h_final_rows = R;
+    return IXT_OK;
+  }
   TRY(launch_rownorm(c, 0, R, tokens, nullptr, nullptr, hcur, c->layers[0].ln1, c->xn, st));
   for (int l = 0; l < c->L; ++l) {
     const LayerW& w = c->layers[l];
@@ -1752,21 +1786,7 @@ static int forward_rows(ixt_ctx* c, int R, const int32_t* tokens, int len_hint, 
       e.row_slot = c->row_slot; e.row_pos = c->row_pos; e.row_active = c->row_active; e.page_map = c->ps.page_map;
       e.rope_sin = c->rope_sin; e.rope_cos = c->rope_cos; e.qbuf = c->qbuf; e.kpages = c->kpages_l[l]; e.vpages = c->vpages_l[l]; e.g = c->geom;
       TRY(launch_ring(c, GEPI_QKV, c->xn, w.wqkv, E, c->NQKV, R, e, false, st));
-      if (attn_tiled) {
-        TRY(launch_attention_tile(c, l, R, len_hint, st));
-      } else if (attn_one_launch) {
-        const DotResult none{0, 0, 0};
-        const int ta = decode ? timing_begin(c, st, 0.0, 1) : -1;
-        // at most one block on a CU: eight waves with everything in flight (128 rows x 1 kv head of two query heads of 128, 1500 keys: 421 us a step of four layers with
-        // four waves, 351 with eight; 700 keys 302 -> 260; 64 keys 231 -> 229); with more the four-wave form is the faster one (40 rows x 12 heads of 64: 20.3 against 13.7 us)
-        if (decode && (long)R * c->KV <= c->small_attn_max_blocks / 2 && attn_small_fits(c, R)) TRY(launch_attn_small(c, l, R, st));
-        else TRY(launch_attention_fused(c, l, R, none, false, decode, st));   // q from qbuf, every key / value (the new ones too) from the pages
-        timing_end(c, st, ta);
-      } else {
-        TRY(launch_attention_partials(c, l, R, len_hint, DotResult{0, 0, 0}, false, st));
-        hipLaunchKernelGGL(k_attn_combine, dim3(R), dim3(256), 0, st, c->pvpart, c->row_pos, c->row_active, c->ao, c->geom, 1);
-        LAUNCHCHK();
-      }
+      TRY(attention(l));
       GemmEpi eo{};
       eo.h_in = hcur; eo.h_out = hnext;
       TRY(launch_ring(c, GEPI_RESID, c->ao, w.wo, c->QN, E, R, eo, false, st));
@@ -2248,7 +2268,7 @@ extern "C" int ixt_set_option(ixt_ctx* c, const char* name, int value) {
       {"gemm_split_min_blocks", &c->gemm_split_min_blocks, 1}, {"gemm_min_blocks", &c->gemm_min_blocks, 1}, {"gemm_min_rows", &c->gemm_min_rows, 1},
       {"unembed_gemm", &c->unembed_gemm, 0}, {"attn_wave_pairs", &c->attn_wave_pairs, 0}, {"attn_tile", &c->attn_tile, 0}, {"attn_tile_min_rows", &c->attn_tile_min_rows, 1}, {"dot_stream_min_blocks", &c->dot_stream_min_blocks, 1},
       {"ring_min_rows", &c->ring_min_rows, 1}, {"ring_mid_rows", &c->ring_mid_rows, 17}, {"ring_cfg", &c->ring_cfg, 0}, {"ring_split", &c->ring_split, 0}, {"ring_wlayout", &c->ring_wlayout, 0}, {"ring_down", &c->ring_down, -1}, {"unembed_tall", &c->unembed_tall, 0}, {"ring_two_per_cu", &c->ring_two_per_cu, 0},
-      {"small_rows", &c->small_rows, 0}, {"small_tpb", &c->small_tpb, 0}, {"small_attn_waves", &c->small_attn_waves, 4}, {"small_attn_max_blocks", &c->small_attn_max_blocks, 0}, {"dot_small", &c->dot_small, 0}, {"small_step", &c->small_step, 0}, {"small_norm", &c->small_norm, 0}, {"small_prefetch", &c->small_prefetch, 0}, {"small_prefetch_blocks", &c->small_prefetch_blocks, 1}, {"moe_grouped", &c->moe_grouped, 0}, {"small_attn_split", &c->small_attn_split, 0}, {"moe_route_blocks", &c->moe_route_blocks, 0}, {"gemma_tile", &c->gemma_tile, 0}, {"moe_fused_gate", &c->moe_fused_gate, 0}, {"moe_mid_pairs", &c->moe_mid_pairs, 0},
+      {"small_rows", &c->small_rows, 0}, {"small_tpb", &c->small_tpb, 0}, {"small_attn_waves", &c->small_attn_waves, 4}, {"small_attn_max_blocks", &c->small_attn_max_blocks, 0}, {"dot_small", &c->dot_small, 0}, {"small_step", &c->small_step, 0}, {"mid_rows", &c->mid_rows, 0}, {"small_norm", &c->small_norm, 0}, {"small_prefetch", &c->small_prefetch, 0}, {"small_prefetch_blocks", &c->small_prefetch_blocks, 1}, {"moe_grouped", &c->moe_grouped, 0}, {"small_attn_split", &c->small_attn_split, 0}, {"moe_route_blocks", &c->moe_route_blocks, 0}, {"gemma_tile", &c->gemma_tile, 0}, {"moe_fused_gate", &c->moe_fused_gate, 0}, {"moe_mid_pairs", &c->moe_mid_pairs, 0},
   };
   for (const Opt& o : opts) {
     if (strcmp(name, o.name) != 0) continue;

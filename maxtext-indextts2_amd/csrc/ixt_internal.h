@@ -123,10 +123,14 @@ struct ixt_ctx {
   int small_prefetch = 0;    // few-rows path: prefetch blocks stream the next launch's kernel into the Infinity Cache (ixt_prefetch).  Measured SLOWER (one utterance 1.19 against 1.03 ms per step, eight 1.33 against 1.23: a launch cannot end before its prefetch has, and an Infinity-Cache hit is only 1.4 x an HBM stream): off
   int small_prefetch_blocks = 64;
   int small_step = 1;        // few rows: all layers in one launch (k_step) where the shapes allow; 0: five launches a layer
-  struct StepLayer* step_layers = nullptr;   // [L] in HBM; nullptr: not this model
+  struct StepLayer* step_layers = nullptr;   // [L] in HBM
   bf16_t* step_ws = nullptr;
   int32_t* step_cnt = nullptr;
   int32_t step_token = 0;
+  bool step_ok = false;      // k_step has its buffers
+  int mid_rows = 64;         // passes of 17 to so many rows (<= 64): a launch between two attentions (k_mid) where the shapes allow; 0: a launch a phase
+  bf16_t* mid_ws = nullptr;  // nullptr: not this model
+  int32_t* mid_cnt = nullptr;
   int small_norm = 1;        // 1: the RMSNorm in front of the QKV / wi projections runs inside k_sdot; 0: k_rownorm launches (experiments)
   int dot_stream_min_blocks = 1 << 30;   // off: measured slower than split-K at 256 rows (decode 7.84 vs 7.68 ms/step, prefill 3.53 vs 3.31 ms)
   ColRanges sample_cols{};   // greedy sampling restricted to these columns (n == 0: all)
@@ -192,4 +196,6 @@ int launch_sdot(ixt_ctx* c, int epi, bool norm, const bf16_t* x, const bf16_t* s
 // ---- few rows, all layers in one launch (ixt_step.hip)
 int step_init(ixt_ctx* c);
 bool step_fits(const ixt_ctx* c, int R);
+bool mid_fits(const ixt_ctx* c, int R);
+int launch_mid(ixt_ctx* c, int R, int l, const int32_t* tokens, bool final, const bf16_t** hidden, const bf16_t** normed, hipStream_t st);
 int launch_step(ixt_ctx* c, int R, const int32_t* tokens, int fresh, const bf16_t** hidden, hipStream_t st);

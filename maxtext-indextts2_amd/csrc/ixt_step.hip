@@ -1,5 +1,6 @@
-// ixt_step.hip -- the one-launch pass of few rows: which shapes take it, its buffers, its launch.
+// ixt_step.hip -- the one-launch pass of few rows, and the launches between the attentions of some: which shapes take them, their buffers, their launches.
 #include "ixt_internal.h"
+#include "ixt_mid.h"
 #include "ixt_step.h"
 
 #include <atomic>
@@ -49,11 +50,50 @@ static int launch_step_t(const StepArgs& a, int L, size_t lds, hipStream_t st) {
   LAUNCHCHK();
   return IXT_OK;
 }
-// the buffers of k_step, once, at ixt_create (the launch may be captured)
+// k_mid: up to 64 rows whose norm is four pieces of 512 features a lane's share at most; a projection's units (16 a block) as in ixt_mid.h
+struct MidPlan { bool ok; int early, nblk[MID_PHASES], tpb[MID_PHASES]; size_t lds; };
+static MidPlan mid_plan(const ixt_ctx* c, int R) {
+  MidPlan p{};
+  const int G = (R + 15) / 16;
+  if (G < 1 || G > 4 || c->E > 2048 || c->QN > 16 * IXT_CHAIN || c->F > 16 * IXT_CHAIN) return p;
+  int steps = 0;
+  auto dot = [&](int phase, int K, int ntile, int even, int least = 96) {
+    const int nc = (K + IXT_CHAIN - 1) / IXT_CHAIN;
+    int tpb = nc > 8 ? 1 : std::min(8, 16 / nc & ~1);
+    while (tpb > 2 && (ntile + tpb - 1) / tpb < least) tpb -= 2;      // (a small projection over more CUs)
+    if (even && tpb < 2) return false;
+    p.tpb[phase] = tpb;
+    p.nblk[phase] = (ntile + tpb - 1) / tpb;
+    if (tpb > 1 && K / 32 <= MID_BUF_STEPS) steps = std::max(steps, K / 32);
+    return true;
+  };
+  p.ok = dot(MID_O, c->QN, c->E / 16, 0) && dot(MID_UP, c->E, 2 * c->F / 16, 1) && dot(MID_DOWN, c->F, c->E / 16, 0) && dot(MID_QKV, c->E, c->NQKV / 16, 0, 160);
+  p.nblk[MID_DOWN] = (p.nblk[MID_DOWN] + 7 & ~7) * MID_SPLIT;
+  p.early = std::max(0, std::min(p.nblk[MID_UP], 256 - p.nblk[MID_O] - (R + MID_NW - 1) / MID_NW)) & ~7;
+  p.nblk[MID_N1] = p.nblk[MID_N2] = (R + MID_NW - 1) / MID_NW;
+  p.lds = (size_t)std::max({2 * steps, 16 * G, c->E / 64 + 1}) * 1024;
+  return p;
+}
+static bool step_model(const ixt_ctx* c) { return !c->moe && !c->gemma && !c->fp8 && c->L >= 1; }
+// Four row groups only where the weights of a layer are worth the phases' ends: ms a pass of 32 steps, a launch a phase / k_mid, 64 slots of the 1B model (121 MB a layer) 52.6 / 49.1, of the
+// 134M model (14 MB) 22.5 / 22.9; 33 of it 18.4 / 17.6, 20 19.3 / 16.2
+bool mid_fits(const ixt_ctx* c, int R) {
+  const size_t layer = ((size_t)c->E * (c->NQKV + 2 * c->F) + (size_t)(c->QN + c->F) * c->E) * sizeof(bf16_t);
+  return c->mid_ws != nullptr && R >= 17 && R <= std::min(layer >= (size_t)48 << 20 ? 64 : 48, c->mid_rows) && mid_plan(c, R).ok;
+}
+static size_t mid_words(const ixt_ctx* c) { return (size_t)(c->L + 1) * MID_PHASES * STEP_NS + 1; }      // lines of its counters
+// the buffers of k_step and k_mid, once, at ixt_create (the launch may be captured)
 int step_init(ixt_ctx* c) {
-  if (c->moe || c->gemma || c->fp8 || c->L < 1 || !step_plan(c, 1).ok) return IXT_OK;
+  const bool step = step_model(c) && step_plan(c, 1).ok, mid = step_model(c) && c->Rmax >= 17 && mid_plan(c, 17).ok;
+  if (!step && !mid) return IXT_OK;
+  const size_t step_elems = step ? (size_t)c->L * 16 * (2 * c->QN + 2 * c->E + c->F) : 0;
   TRY(dmalloc(c, &c->step_layers, (size_t)c->L));
-  TRY(dmalloc(c, &c->step_ws, (size_t)c->L * 16 * (2 * c->QN + 2 * c->E + c->F)));
+  TRY(dmalloc(c, &c->step_ws, step_elems + (mid ? (size_t)64 * (5 * c->E + c->F) : 0)));
+  if (mid) {
+    c->mid_ws = c->step_ws + step_elems;
+    TRY(dmalloc(c, &c->mid_cnt, mid_words(c) * 32));
+  }
+  c->step_ok = step;
   TRY(dmalloc(c, &c->step_cnt, ((size_t)c->L * STEP_PHASES * STEP_NS + 1) * 32));
   std::vector<StepLayer> t((size_t)c->L);
   auto at = [&](const void* p) { return (int64_t)(reinterpret_cast<intptr_t>(p) - reinterpret_cast<intptr_t>(c->step_ws)); };
@@ -66,7 +106,7 @@ int step_init(ixt_ctx* c) {
   HIPCHK(hipMemcpy(c->step_layers, t.data(), sizeof(StepLayer) * t.size(), hipMemcpyHostToDevice));
   return IXT_OK;
 }
-bool step_fits(const ixt_ctx* c, int R) { return c->step_layers != nullptr && step_plan(c, R).ok; }
+bool step_fits(const ixt_ctx* c, int R) { return c->step_ok && step_plan(c, R).ok; }
 // every layer of R rows; *hidden = the rows behind the last one.  fresh: step_attn
 int launch_step(ixt_ctx* c, int R, const int32_t* tokens, int fresh, const bf16_t** hidden, hipStream_t st) {
   const StepPlan p = step_plan(c, R);
@@ -86,4 +126,54 @@ int launch_step(ixt_ctx* c, int R, const int32_t* tokens, int fresh, const bf16_
   ST(128, 1) ST(128, 2) ST(64, 1) ST(64, 2)
 #undef ST
   return set_err(IXT_ERR_UNSUPPORTED, "step geometry hd=%d gq=%d", c->D, c->GQ);
+}
+
+static int launch_mid_t(const MidArgs& a, int G, int blocks, size_t lds, hipStream_t st) {
+  const auto kernel = G == 2 ? &k_mid<2> : G == 3 ? &k_mid<3> : &k_mid<4>;
+  static bool attr_done[5] = {};
+  if (!attr_done[G]) {
+    HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 2 * MID_BUF_STEPS * 1024));
+    attr_done[G] = true;
+  }
+  hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(MID_NW * 64), lds, st, a);
+  LAUNCHCHK();
+  return IXT_OK;
+}
+// What stands between the attentions of layers l and l + 1 (-1: the embedding and what is in front of the first attention).  Behind the last layer: the rows, *hidden, and with
+// `final` their norm for the head, *normed.
+int launch_mid(ixt_ctx* c, int R, int l, const int32_t* tokens, bool final, const bf16_t** hidden, const bf16_t** normed, hipStream_t st) {
+  const MidPlan p = mid_plan(c, R);
+  const int G = (R + 15) / 16, lines = MID_PHASES * STEP_NS;
+  bf16_t *h[2], *ws = c->mid_ws;
+  auto take = [&](size_t n) { bf16_t* q = ws; ws += n; return q; };
+  MidArgs a;
+  h[0] = take((size_t)64 * c->E); h[1] = take((size_t)64 * c->E);
+  a.hmid = take((size_t)64 * c->E); a.xn1 = take((size_t)64 * c->E); a.xn2 = take((size_t)64 * c->E); a.act = take((size_t)64 * c->F);
+  const bool end = l == c->L - 1;
+  a.layers = c->step_layers; a.base = c->step_ws; a.layer = l; a.next = end ? -1 : l + 1;
+  a.ao = c->ao; a.qbuf = c->qbuf; a.hin = h[(l + 2) & 1]; a.hout = h[(l + 1) & 1];
+  a.scale = end ? c->final_norm : c->layers[l + 1].ln1;
+  a.cnt = c->mid_cnt + (size_t)(l + 1) * lines * 32; a.err = c->split_cnt + (size_t)16 * c->KV * 4;
+  a.done = end ? c->mid_cnt + (size_t)(c->L + 1) * lines * 32 : nullptr;
+  a.R = R; a.E = c->E; a.F = c->F; a.QN = c->QN; a.NQKV = c->NQKV; a.token = c->step_token; a.last = final ? MID_N1 : MID_DOWN;
+  a.early = p.early;
+  a.eps = c->cfg.normalization_layer_epsilon;
+  a.row_slot = c->row_slot; a.row_pos = c->row_pos; a.row_active = c->row_active; a.page_map = c->ps.page_map;
+  a.rope_sin = c->rope_sin; a.rope_cos = c->rope_cos; a.g = c->geom;
+  int blocks = 0, before = -1;
+  for (int i = 0; i < MID_PHASES; ++i) {
+    const bool here = i <= MID_DOWN ? l >= 0 : i == MID_N1 ? !end || final : !end;
+    a.tpb[i] = p.tpb[i];
+    a.nblk[i] = here ? p.nblk[i] : 0;
+    a.prev[i] = before;
+    if (here) before = i;
+    blocks += a.nblk[i];
+  }
+  if (l < 0) {
+    hipLaunchKernelGGL(k_step_begin, dim3(R), dim3(256), 0, st, tokens, c->embedding, c->E, h[0], c->mid_cnt, (int)mid_words(c), a.token, a.err);
+    LAUNCHCHK();
+  }
+  if (hidden) *hidden = a.hout;
+  if (normed) *normed = a.xn1;
+  return launch_mid_t(a, G, blocks, p.lds, st);
 }
