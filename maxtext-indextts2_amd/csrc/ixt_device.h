@@ -161,6 +161,13 @@ __device__ __forceinline__ void lds_barrier() {
   asm volatile("" ::: "memory");
 }
 
+// 16 bytes past the XCD's L2 (sc1: agent scope).  A store of more than 8 bytes is still reading its registers when the next instruction issues: the wait state that the compiler puts
+// in front of a vector instruction that writes them has to stand here (without it one row of a wave in thousands of launches was wrong)
+template <typename V> __device__ __forceinline__ void stg16_agent(void* p, const V& v) {
+  static_assert(sizeof(V) == 16, "four registers");
+  asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(p), "v"(v) : "memory");
+}
+
 // agent-scope (L1-bypassing) accesses for state one wave re-reads after writing it
 __device__ __forceinline__ int ldg_i32(const int32_t* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ __forceinline__ void stg_i32(int32_t* p, int v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }

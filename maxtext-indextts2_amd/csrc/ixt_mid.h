@@ -39,8 +39,6 @@ struct MidArgs {
   const bf16_t *rope_sin, *rope_cos;
   AttnGeom g;
 };
-// 16 bytes past the XCD's L2, as step_st8 stores 8 (sc1: agent scope)
-__device__ __forceinline__ void mid_st16(void* p, const u32x4& v) { asm volatile("global_store_dwordx4 %0, %1, off sc1" ::"v"(p), "v"(v) : "memory"); }
 template <typename T> __device__ __forceinline__ T* mid_at(const MidArgs& a, int64_t off) { return reinterpret_cast<T*>(reinterpret_cast<char*>(a.base) + off); }
 __device__ __forceinline__ int32_t* mid_cnt(const MidArgs& a, int phase) { return a.cnt + (size_t)phase * STEP_NS * 32; }
 __device__ __forceinline__ void mid_wait(const MidArgs& a, int phase) {
@@ -342,7 +340,7 @@ __device__ __forceinline__ void mid_norm(const MidArgs& a, int blk, u32x4* sx) {
   bf16_t* dst = PHASE == MID_N1 ? a.xn1 : a.xn2;
   for (int i = threadIdx.x; i < nch * MID_NW; i += MID_NW * 64) {
     const int ch = i / MID_NW, rr = i % MID_NW;
-    if (blk * MID_NW + rr < a.R) mid_st16(dst + xidx(blk * MID_NW + rr, ch * 8, a.E), sx[ch * MID_NW + (rr ^ (ch & (MID_NW - 1)))]);
+    if (blk * MID_NW + rr < a.R) stg16_agent(dst + xidx(blk * MID_NW + rr, ch * 8, a.E), sx[ch * MID_NW + (rr ^ (ch & (MID_NW - 1)))]);
   }
   mid_arrive(a, PHASE, blk, MID_NW, &met);
 }

@@ -19,6 +19,11 @@ TRAIN = """#include "ixt_train_gemm.h"
 template __global__ void k_tgemm<true, true, 2, 2, 2, 2, 4, true>(TGemm);
 template __global__ void k_tgemm<false, false, 8, 4, 2, 4, 4, false>(TGemm);
 """
+MID = """#include "ixt_mid.h"
+template __global__ void k_mid<2>(MidArgs);
+template __global__ void k_mid<3>(MidArgs);
+template __global__ void k_mid<4>(MidArgs);
+"""
 
 
 def _registers(operand):
@@ -57,7 +62,7 @@ def test_the_scan_sees_both():
   assert _distances(near.replace(" global", " s_nop 3\n global")) == (1, 4, 5)
 
 
-@pytest.mark.parametrize("source", [RING, TRAIN], ids=["ring", "train"])
+@pytest.mark.parametrize("source", [RING, TRAIN, MID], ids=["ring", "train", "mid"])
 def test_wait_states(source, tmp_path):
   if not os.path.exists(build.hipcc()):
     pytest.skip("no hipcc here")
@@ -76,3 +81,16 @@ def test_barriers_order_the_reads_behind_them():
   with open(os.path.join(build.CSRC, "ixt_device.h"), encoding="utf-8") as f:
     body = re.search(r"void lds_barrier\(\) \{(.*?)\n\}", f.read(), re.S)
   assert bare == [] and body and re.search(r's_barrier\(\);\s*asm volatile\("" ::: "memory"\);', body[1])
+
+
+def test_wide_stores_are_followed_by_a_wait_state():
+  """A store of more than 8 bytes still reads its registers when the next instruction issues; the compiler keeps a vector instruction that writes them away from its
+  own stores and does not look into asm."""
+  found = 0
+  for n in sorted(os.listdir(build.CSRC)):
+    with open(os.path.join(build.CSRC, n), encoding="utf-8") as f:
+      for text in re.findall(r'asm(?: volatile)?\s*\(\s*"((?:[^"\\]|\\.)*)"', f.read()):
+        for at in re.finditer(r"(?:global|buffer|flat)_store_dwordx[34]", text):
+          found += 1
+          assert re.search(r"\\n\\ts_nop \d", text[at.end():]), (n, text)
+  assert found > 0
