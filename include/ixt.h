@@ -237,8 +237,8 @@ int ixt_pages_status(ixt_ctx* ctx, int32_t* out4, int reset, void* stream);
  * the words once it has completed (a throughput path checks the reservations of packed prefill N while pass N already runs). */
 int ixt_pages_status_async(ixt_ctx* ctx, int32_t* host_out4, void* stream);
 /* Few decode rows: the keys of a (row, kv head) are split over several thread blocks that exchange their softmax statistics through HBM
- * inside one launch (k_attn_split; option small_attn_split), or all layers of a pass run in one launch whose blocks wait for the phase before
- * theirs (k_step; option small_step).  These waits are bounded; out1 (HOST) = 1 if a wait ever gave up since the last
+ * inside one launch (k_attn_split; option small_attn_split), or all layers of a pass, or what lies between two attentions, run in one launch whose blocks wait for
+ * the phase before theirs (k_step, k_mid; options small_step, mid_rows), or a product's sum is handed from block to block (option ring_parts).  These waits are bounded; out1 (HOST) = 1 if a wait ever gave up since the last
  * reset (the affected step's numbers are then wrong -- the reference has no counterpart: its generate step, maxengine.py:838-935, is one XLA
  * program), 0 otherwise.  Synchronises `stream`; reset != 0 re-arms the exchange. */
 int ixt_exchange_status(ixt_ctx* ctx, int32_t* out1, int reset, void* stream);

@@ -340,6 +340,8 @@ extern "C" int ixt_create(const ixt_config* cfg, ixt_ctx** out) {
     }
   }
   }
+  A(dmalloc(x, &x->ring_flags, (size_t)RING_FLAGS));
+  if (hipMemset(x->ring_flags, 0, sizeof(int32_t) * RING_FLAGS) != hipSuccess) return fail(set_err(IXT_ERR_HIP, "flags"));
   A(dmalloc(x, &x->row_slot, (size_t)R));
   A(dmalloc(x, &x->row_pos, (size_t)R));
   A(dmalloc(x, &x->row_active, (size_t)R));
@@ -614,6 +616,7 @@ extern "C" int ixt_exchange_status(ixt_ctx* c, int32_t* out1, int reset, void* s
   int32_t* err = c->split_cnt + (size_t)16 * c->KV * 4;
   HIPCHK(hipMemcpyAsync(out1, err, sizeof(int32_t), hipMemcpyDeviceToHost, st));
   HIPCHK(hipStreamSynchronize(st));
+  if (reset && *out1 != 0) HIPCHK(hipMemsetAsync(c->ring_flags, 0, sizeof(int32_t) * RING_FLAGS, st));
   if (reset && *out1 != 0) HIPCHK(hipMemsetAsync(c->split_cnt, 0, sizeof(int32_t) * ((size_t)16 * c->KV * 4 + 4), st));   // a wait that gave up leaves its counters armed
   return IXT_OK;
 }
@@ -721,6 +724,15 @@ static int ring_pick(const ixt_ctx* c, int epi, int R, int N, bool routed, bool 
   return best;
 }
 
+// f32 sums of few tiles over a long K: three blocks a tile (k_gemm_ring, SPLIT 2) of 128 x 64, by the same estimate (a part's chunks, and 1.5 us a hand-over) against that of the
+// tile picked, which is one round
+static bool ring_parts_fit(const ixt_ctx* c, int cfg, int R, int N, int K) {
+  const int n = (K + IXT_CHAIN - 1) / IXT_CHAIN, colg = (N + 63) / 64, zb = (R + 127) / 128, longest = n - ((RING_PARTS - 1) * n / RING_PARTS - 1);
+  const int per_xcd = (colg + 7) / 8 * zb, one = cfg == 5 ? 31 : cfg == 3 ? 22 : cfg == 6 ? 19 : 0;
+  return c->ring_flags != nullptr && c->ring_parts && one > 0 && n >= 2 * RING_PARTS && longest <= RING_KEEP && per_xcd * RING_PARTS <= 32 && (size_t)per_xcd * 8 * 8 * RING_PARTS <= RING_FLAGS &&
+         8 * longest * 44 + 300 < 8 * n * one;
+}
+
 // (max, index) pairs that an unembedding with this tile leaves of a row: one a wave column of whole column groups (4 even of a vocabulary of 16 columns)
 static size_t ring_pairs(int cfg, int N) {
   const int n = N / 16;
@@ -737,7 +749,7 @@ static int ring_launch_o(const bf16_t* x, const bf16_t* w, int K, int N, int R, 
     HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gemm_ring<WR, WC, RB, CT, KS, NS, EPI, SPLIT, false, ONCE>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     attr_done = true;
   }
-  dim3 grid(((ncolg + 7) / 8) * 8 * zb, SPLIT ? chains : 1, 1);
+  dim3 grid(((ncolg + 7) / 8) * 8 * zb, SPLIT == 2 ? RING_PARTS : SPLIT ? chains : 1, 1);
   hipLaunchKernelGGL((k_gemm_ring<WR, WC, RB, CT, KS, NS, EPI, SPLIT, false, ONCE>), grid, dim3(WR * WC * 64), lds, st, reinterpret_cast<const u32x4*>(x),
                      reinterpret_cast<const u32x4*>(w), K, N, R, ncolg, zb, wring, e);
   LAUNCHCHK();
@@ -791,6 +803,11 @@ int launch_ring(ixt_ctx* c, int epi, const bf16_t* x, const bf16_t* w, int K, in
     case 2: rc = RING_T(2, 2, 4, 2, 2, 5, EPI_, 0); break;                 \
   }
   if (epi == GEPI_F32 && split) rc = RING_T(2, 4, 4, 2, 2, 4, GEPI_F32, 1);
+  else if (epi == GEPI_F32 && e.rb_exp == nullptr && !wring && c->ring_cfg == 0 && ring_parts_fit(c, cfg, R, N, K)) {
+    GemmEpi ep = e;
+    ep.flags = c->ring_flags; ep.err = c->split_cnt + (size_t)16 * c->KV * 4;
+    rc = ring_launch_t<2, 4, 4, 1, 2, 5, GEPI_F32, 2>(x, w, K, N, R, chains, wring, ep, st, wave_cols);
+  }
   else if (epi == GEPI_F32) RING(GEPI_F32)
   else if (epi == GEPI_RESID) RING(GEPI_RESID)
   else if (epi == GEPI_TANHNORM) RING(GEPI_TANHNORM)
@@ -2268,7 +2285,7 @@ extern "C" int ixt_set_option(ixt_ctx* c, const char* name, int value) {
       {"gemm_split_min_blocks", &c->gemm_split_min_blocks, 1}, {"gemm_min_blocks", &c->gemm_min_blocks, 1}, {"gemm_min_rows", &c->gemm_min_rows, 1},
       {"unembed_gemm", &c->unembed_gemm, 0}, {"attn_wave_pairs", &c->attn_wave_pairs, 0}, {"attn_tile", &c->attn_tile, 0}, {"attn_tile_min_rows", &c->attn_tile_min_rows, 1}, {"dot_stream_min_blocks", &c->dot_stream_min_blocks, 1},
       {"ring_min_rows", &c->ring_min_rows, 1}, {"ring_mid_rows", &c->ring_mid_rows, 17}, {"ring_cfg", &c->ring_cfg, 0}, {"ring_split", &c->ring_split, 0}, {"ring_wlayout", &c->ring_wlayout, 0}, {"ring_down", &c->ring_down, -1}, {"unembed_tall", &c->unembed_tall, 0}, {"ring_two_per_cu", &c->ring_two_per_cu, 0},
-      {"small_rows", &c->small_rows, 0}, {"small_tpb", &c->small_tpb, 0}, {"small_attn_waves", &c->small_attn_waves, 4}, {"small_attn_max_blocks", &c->small_attn_max_blocks, 0}, {"dot_small", &c->dot_small, 0}, {"small_step", &c->small_step, 0}, {"mid_rows", &c->mid_rows, 0}, {"small_norm", &c->small_norm, 0}, {"small_prefetch", &c->small_prefetch, 0}, {"small_prefetch_blocks", &c->small_prefetch_blocks, 1}, {"moe_grouped", &c->moe_grouped, 0}, {"small_attn_split", &c->small_attn_split, 0}, {"moe_route_blocks", &c->moe_route_blocks, 0}, {"gemma_tile", &c->gemma_tile, 0}, {"moe_fused_gate", &c->moe_fused_gate, 0}, {"moe_mid_pairs", &c->moe_mid_pairs, 0},
+      {"small_rows", &c->small_rows, 0}, {"small_tpb", &c->small_tpb, 0}, {"small_attn_waves", &c->small_attn_waves, 4}, {"small_attn_max_blocks", &c->small_attn_max_blocks, 0}, {"dot_small", &c->dot_small, 0}, {"ring_parts", &c->ring_parts, 0}, {"small_step", &c->small_step, 0}, {"mid_rows", &c->mid_rows, 0}, {"small_norm", &c->small_norm, 0}, {"small_prefetch", &c->small_prefetch, 0}, {"small_prefetch_blocks", &c->small_prefetch_blocks, 1}, {"moe_grouped", &c->moe_grouped, 0}, {"small_attn_split", &c->small_attn_split, 0}, {"moe_route_blocks", &c->moe_route_blocks, 0}, {"gemma_tile", &c->gemma_tile, 0}, {"moe_fused_gate", &c->moe_fused_gate, 0}, {"moe_mid_pairs", &c->moe_mid_pairs, 0},
   };
   for (const Opt& o : opts) {
     if (strcmp(name, o.name) != 0) continue;

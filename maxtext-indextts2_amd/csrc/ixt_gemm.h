@@ -93,6 +93,7 @@ struct GemmEpi {
   size_t sstride;                                       // F8 + routed experts: floats between two experts' column scales
   TanhNormEpi tn;                                       // TANHNORM (with act)
   int glu; float glu_limit; const float* act_par;       // ACT: the unit's kind and its numbers; SWIGLU: glu > 0 takes that gated unit of the f32 totals instead (ixt_glu), glu < 0 ixt_geglu
+  int32_t *flags, *err;                                 // SPLIT 2: a word a wave of a tile and part, zero between launches; a wait that gave up
   const int32_t* rb_exp; size_t wstride;                // routed experts: expert of every 16-row block (-1: none), 16-byte units between experts' kernels
 };
 
@@ -109,7 +110,13 @@ __device__ __forceinline__ void ring_wait_chunks(int younger) {
   ring_wait<M * NJ>();
 }
 
-//   grid = (8 ceil(ncolg / 8) zb, SPLIT ? chains : 1), block 64 WR WC, dynamic LDS = NS (WC CT + WR RB) KS KiB.
+// SPLIT 2 (GEPI_F32): a tile's chains in gridDim.y parts, one block each.  A sum's order stays: part 0 adds its chains up as it goes, a later part keeps each of its chains (at most RING_KEEP) in
+// registers, takes the sum so far from the part before it, wave by wave, adds its own in order and hands it on; the last one stores it.  Progress: a part waits for a block of lower
+// index on the same XCD (gridDim.x is a multiple of 8), which has started before it; the waits are bounded all the same.  For few tiles of a long K: 256 x 2304 outputs, K 9216, 41 us in
+// one part (144 tiles of 64 x 64 for 256 CUs), 35 in three equal ones (72 of 128 x 64), 31 with a chain more for each later part.
+#define RING_KEEP 7
+#define RING_SPIN_LIMIT (1 << 20)
+//   grid = (8 ceil(ncolg / 8) zb, SPLIT 1 ? chains : SPLIT 2 ? parts : 1), block 64 WR WC, dynamic LDS = NS (WC CT + WR RB) KS KiB.
 //   Row groups of one column group are block ids b, b + 8, ..: same XCD, the weights meet in its L2.
 //   F8 (ixt_fp8.h): both operands are e4m3 fragments of 64 k (still 1 KiB: the ring moves them exactly as bf16 fragments of 32 k); a fragment
 //   feeds two v_mfma_f32_16x16x32_fp8_fp8; at the end of every 512-k chain the accumulator is scaled by (a_rc s_n) before it joins the total.
@@ -157,8 +164,10 @@ __global__ __launch_bounds__(WR * WC * 64, 2) void k_gemm_ring(const u32x4* __re
     off[j] += lane * 16;
   }
   constexpr int CPC = (F8 ? 8 : 16) / KS;                       // chunks per 512-k chain
-  const int chb = SPLIT ? (int)blockIdx.y * CPC : 0;
-  const int che = SPLIT ? min(nchunks, chb + CPC) : nchunks;
+  const int nch = (nchunks + CPC - 1) / CPC, part = SPLIT == 2 ? (int)blockIdx.y : 0, parts = SPLIT == 2 ? (int)gridDim.y : 1;
+  // (a later part has a chain more: it waits for the one before)
+  const int chb = SPLIT == 2 ? (part == 0 ? 0 : nch * part / parts - 1) * CPC : SPLIT ? (int)blockIdx.y * CPC : 0;
+  const int che = SPLIT == 2 ? min(nchunks, (part + 1 == parts ? nch : nch * (part + 1) / parts - 1) * CPC) : SPLIT ? min(nchunks, chb + CPC) : nchunks;
   const char* pw = reinterpret_cast<const char*>(wt + (wring ? r8frag(colg * TC, 0, nsteps) : (size_t)colg * TC * nsteps) * 64) + chb * wadv;
   const char* px = reinterpret_cast<const char*>(xt + (size_t)rowg * TR * nsteps * 64) + (size_t)chb * KS * 1024;
   const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)((__attribute__((address_space(3))) u32x4*)st));
@@ -263,17 +272,76 @@ __global__ __launch_bounds__(WR * WC * 64, 2) void k_gemm_ring(const u32x4* __re
       step(ch + 1, 0, 1);
       if (((ch + 2) % CPC) == 0 || ch + 2 == che) chain_end(ch);
     }
-  } else {
+  } else if (SPLIT != 2 || part == 0) {
     for (int ch = chb; ch < che; ++ch) {
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) step(ch, ks, ks & 1);
       if (((ch + 1) % CPC) == 0 || ch + 1 == che) chain_end(ch);
     }
   }
+  if constexpr (SPLIT == 2) {
+    static_assert(EPI == GEPI_F32 && KS > 1 && !F8, "parts of f32 sums");
+    f32x4 keep[RING_KEEP][CT][RB];
+    if (part > 0) {
+#pragma unroll
+      for (int q = 0; q < RING_KEEP; ++q) {
+        for (int ch = chb + q * CPC; ch < min(che, chb + (q + 1) * CPC); ++ch) {
+#pragma unroll
+          for (int ks = 0; ks < KS; ++ks) step(ch, ks, ks & 1);
+        }
+#pragma unroll
+        for (int i = 0; i < CT; ++i)
+#pragma unroll
+          for (int b = 0; b < RB; ++b) { keep[q][i][b] = acc[i][b]; acc[i][b] = f32x4(0.0f); }
+      }
+    }
+    auto place = [&](int i, int b, float*& p) {
+      const int tile = colg * TC + wc * CT + i, row = (rowg * TR + wr * RB + b) * 16 + r_in;
+      p = e.out + (size_t)row * N + tile * 16 + cq * 4;
+      return tile < ntile && row < R;
+    };
+    int32_t* flag = e.flags + ((size_t)blockIdx.x * NW + wave) * parts;
+    float* p;
+    if (part > 0) {
+      for (int it = 0; __hip_atomic_load(flag + part - 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0;) {
+        if (++it > RING_SPIN_LIMIT) { __hip_atomic_store(e.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); break; }
+        __builtin_amdgcn_s_sleep(1);
+      }
+      asm volatile("" ::: "memory");
+#pragma unroll
+      for (int i = 0; i < CT; ++i)
+#pragma unroll
+        for (int b = 0; b < RB; ++b) {
+          if (!place(i, b, p)) continue;
+          unsigned long long* q = reinterpret_cast<unsigned long long*>(p);      // (past the L2: half of a line is another wave's, and may be older)
+          const unsigned long long lo = __hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), hi = __hip_atomic_load(q + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          tot[i][b] = f32x4{__uint_as_float((uint32_t)lo), __uint_as_float((uint32_t)(lo >> 32)), __uint_as_float((uint32_t)hi), __uint_as_float((uint32_t)(hi >> 32))};
+        }
+#pragma unroll
+      for (int q = 0; q < RING_KEEP; ++q)
+        if (chb + q * CPC < che) {
+#pragma unroll
+          for (int i = 0; i < CT; ++i)
+#pragma unroll
+            for (int b = 0; b < RB; ++b) tot[i][b] = tot[i][b] + keep[q][i][b];
+        }
+      if (lane == 0) __hip_atomic_store(flag + part - 1, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if (part < parts - 1) {
+#pragma unroll
+      for (int i = 0; i < CT; ++i)
+#pragma unroll
+        for (int b = 0; b < RB; ++b)
+          if (place(i, b, p)) stg16_agent(p, tot[i][b]);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      if (lane == 0) __hip_atomic_store(flag + part, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      return;
+    }
+  }
 
   // ---------------------------------------------------------------- epilogues
   if constexpr (EPI == GEPI_F32) {
-    float* out = e.out + (SPLIT ? (size_t)blockIdx.y * R * N : 0);
+    float* out = e.out + (SPLIT == 1 ? (size_t)blockIdx.y * R * N : 0);
 #pragma unroll
     for (int i = 0; i < CT; ++i) {
       const int tile = colg * TC + wc * CT + i;

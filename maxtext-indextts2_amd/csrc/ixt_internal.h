@@ -50,6 +50,8 @@ int hybrid_prompt_logits(ixt_ctx* c, int row0, int n, hipStream_t st);
 int forward_rows_hybrid(ixt_ctx* c, int R, const int32_t* tokens, int len_hint, int lrow0, int nl, const int32_t* lrows, int32_t* argmax_out, float* logits_out, bool decode,
                                hipStream_t st);
 
+#define RING_PARTS 3           // blocks of a tile whose f32 sum is cut (k_gemm_ring, SPLIT 2)
+#define RING_FLAGS 16384
 struct ixt_ctx {
   ixt_config cfg;
   HybridModel* hy = nullptr;
@@ -122,6 +124,8 @@ struct ixt_ctx {
   size_t split_stride = 0;
   int small_prefetch = 0;    // few-rows path: prefetch blocks stream the next launch's kernel into the Infinity Cache (ixt_prefetch).  Measured SLOWER (one utterance 1.19 against 1.03 ms per step, eight 1.33 against 1.23: a launch cannot end before its prefetch has, and an Infinity-Cache hit is only 1.4 x an HBM stream): off
   int small_prefetch_blocks = 64;
+  int ring_parts = 1;        // f32 sums of few tiles over a long K: three blocks a tile (k_gemm_ring, SPLIT 2)
+  int32_t* ring_flags = nullptr;
   int small_step = 1;        // few rows: all layers in one launch (k_step) where the shapes allow; 0: five launches a layer
   struct StepLayer* step_layers = nullptr;   // [L] in HBM
   bf16_t* step_ws = nullptr;
