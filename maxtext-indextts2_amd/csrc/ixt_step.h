@@ -9,7 +9,8 @@
 // Progress: a block waits for blocks of lower index only, and those are dispatched before it (each XCD takes its share of the grid in order), so the
 // lowest unfinished block never waits for one that has not started, whatever runs beside it and ends by itself.  Two such grids would not: each could hold the
 // XCD that the other's lowest block has to start on.  So one of them at a time is on the chip (step_turn): k_step_begin waits for the turn, the last block of the last layer gives it
-// on.  The waits are bounded all the same (step_wait).  Workgroups that draw their block's index from a counter, and stay, would need no turn: built, and slower
+// on.  The waits are bounded all the same (step_wait); processes that share a GPU have no turn between them
+// (options small_step and mid_rows).  Workgroups that draw their block's index from a counter, and stay, would need no turn: built, and slower
 // (us a step, 1 / 8 slots: 650 / 809 this, 833 / 1316 with the index drawn a block ahead, 780 / 956 behind the block's own wait; the draw holds up the wave's loads behind it).
 //
 // Data between blocks: written with agent-scope stores (past the XCD's L2), announced by a counter behind the stores' completion, and read by ordinary loads:
