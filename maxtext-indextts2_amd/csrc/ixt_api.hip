@@ -10,6 +10,8 @@
 #include <stdio.h>
 #include <stdlib.h>
 
+#include <mutex>
+
 static thread_local char g_err[512] = "";
 int set_err(int code, const char* fmt, ...) {
   va_list ap;
@@ -86,6 +88,17 @@ static void host_rope_tables_llama31(const ixt_config& cfg, std::vector<float>& 
       sn[(size_t)p * half + i] = (float)sin((double)ang);
       cs[(size_t)p * half + i] = (float)cos((double)ang);
     }
+}
+
+// the gate of the current GPU: one each, for the life of the process
+struct DeviceGate : IxtGate {};
+static DeviceGate* device_gate() {
+  static std::mutex mu;
+  static std::map<int, DeviceGate> gates;
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return nullptr;
+  std::lock_guard<std::mutex> lk(mu);
+  return &gates[dev];
 }
 
 static int sdot_set_attributes();
@@ -361,6 +374,11 @@ extern "C" int ixt_create(const ixt_config* cfg, ixt_ctx** out) {
   if (hipDeviceSynchronize() != hipSuccess) return fail(set_err(IXT_ERR_HIP, "page state init failed"));
   if (sdot_set_attributes() != IXT_OK) return fail(IXT_ERR_HIP);
   if (!hybrid && step_init(x) != IXT_OK) return fail(IXT_ERR_HIP);
+  if (x->step_ok || x->mid_ws != nullptr) {
+    if (hipEventCreateWithFlags(&x->pass_event, hipEventDisableTiming) != hipSuccess) return fail(set_err(IXT_ERR_HIP, "event"));
+    x->gate = device_gate();
+    if (x->gate) x->gate->join(x, x->pass_event, [] { return hipDeviceSynchronize() == hipSuccess; });
+  }
   *out = x;
   return IXT_OK;
 }
@@ -368,6 +386,8 @@ extern "C" int ixt_create(const ixt_config* cfg, ixt_ctx** out) {
 extern "C" int ixt_destroy(ixt_ctx* c) {
   if (!c) return IXT_OK;
   (void)hipDeviceSynchronize();
+  if (c->gate) c->gate->forget(c);
+  if (c->pass_event) (void)hipEventDestroy(c->pass_event);
   for (auto& kv : c->graphs) (void)hipGraphExecDestroy(kv.second.exec);
   for (auto& t : c->tpairs) { (void)hipEventDestroy(t.a); (void)hipEventDestroy(t.b); }
   for (void* p : c->allocs) (void)hipFree(p);
@@ -618,6 +638,11 @@ extern "C" int ixt_exchange_status(ixt_ctx* c, int32_t* out1, int reset, void* s
   HIPCHK(hipStreamSynchronize(st));
   if (reset && *out1 != 0) HIPCHK(hipMemsetAsync(c->ring_flags, 0, sizeof(int32_t) * RING_FLAGS, st));
   if (reset && *out1 != 0) HIPCHK(hipMemsetAsync(c->split_cnt, 0, sizeof(int32_t) * ((size_t)16 * c->KV * 4 + 4), st));   // a wait that gave up leaves its counters armed
+  return IXT_OK;
+}
+extern "C" int ixt_pass_forms(ixt_ctx* c, int32_t* out1) {
+  if (!c || !out1) return set_err(IXT_ERR_INVALID, "null argument");
+  *out1 = c->forms;
   return IXT_OK;
 }
 extern "C" int ixt_pages_status_async(ixt_ctx* c, int32_t* host_out4, void* stream) {
@@ -1663,10 +1688,14 @@ static bool small_path_ok(const ixt_ctx* c, int R) {
   return sdot_plan(c, GEPI_QKV, true, c->E, c->NQKV, R).ok && sdot_plan(c, GEPI_RESID, false, c->QN, c->E, R).ok &&
          sdot_plan(c, GEPI_SWIGLU, true, c->E, 2 * c->F, R).ok;
 }
+static bool takes_step(ixt_ctx* c, int R, bool decode) {
+  return c->small_step && c->small_norm && !c->timing && step_fits(c, R) && !(decode && attn_split_factor(c, R) > 1);
+}
+static bool takes_mid(const ixt_ctx* c, int R) { return c->mid_rows > 0 && !c->timing && !c->moe && !c->fp8 && mid_fits(c, R); }
 static int forward_rows_small(ixt_ctx* c, int R, const int32_t* tokens, int len_hint, int lrow0, int nl, const int32_t* lrows, int32_t* argmax_out,
                               float* logits_out, bool decode, hipStream_t st) {
   const int E = c->E, F = c->F;
-  if (c->small_step && c->small_norm && !c->timing && step_fits(c, R) && !(decode && attn_split_factor(c, R) > 1)) {
+  if (c->may_wait && takes_step(c, R, decode)) {
     const bf16_t* h = nullptr;
     TRY(launch_step(c, R, tokens, decode ? 0 : c->one_segment ? R : c->Tmax, &h, st));
     if (nl > 0) {
@@ -1779,7 +1808,7 @@ static int forward_rows(ixt_ctx* c, int R, const int32_t* tokens, int len_hint, 
     }
     return IXT_OK;
   };
-  if (c->mid_rows > 0 && !c->timing && !c->moe && !c->fp8 && mid_fits(c, R)) {
+  if (c->may_wait && takes_mid(c, R)) {
     const bf16_t *h = nullptr, *xn = nullptr;
     TRY(launch_mid(c, R, -1, tokens, false, nullptr, nullptr, st));
     for (int l = 0; l < c->L; ++l) {
@@ -1922,6 +1951,41 @@ static int forward_rows(ixt_ctx* c, int R, const int32_t* tokens, int len_hint, 
   return IXT_OK;
 }
 
+// While a pass of R rows is enqueued: may it take the launches whose blocks wait?  A stream that the caller captures may not: its graph is replayed without this call.
+class WaitPass {
+ public:
+  WaitPass(ixt_ctx* c, int R, bool decode, hipStream_t st) : c_(c), st_(st) {
+    c->forms = 0;
+    if (c->gate == nullptr || !(small_path_ok(c, R) ? takes_step(c, R, decode) : takes_mid(c, R))) return;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
+      (void)hipGetLastError();
+      return;
+    }
+    in_ = true;
+    c->may_wait = c->gate->enter(c, [](void* event) {
+      const bool ended = hipEventQuery((hipEvent_t)event) == hipSuccess;
+      if (!ended) (void)hipGetLastError();       // (not ready)
+      return ended;
+    });
+  }
+  ~WaitPass() {
+    if (!in_) return;
+    c_->may_wait = false;
+    c_->gate->leave(c_, [this](void* event) {
+      const bool marked = hipEventRecord((hipEvent_t)event, st_) == hipSuccess;
+      if (!marked) (void)hipGetLastError();
+      return marked;
+    });
+  }
+  WaitPass(const WaitPass&) = delete;
+
+ private:
+  ixt_ctx* c_;
+  hipStream_t st_;
+  bool in_ = false;
+};
+
 extern "C" int ixt_prefill_chunk(ixt_ctx* c, int slot, const int32_t* tokens_dev, int n_tokens, int start_pos, int32_t* first_token_dev,
                                  float* last_logits_dev, void* stream) {
   if (!c || !tokens_dev || !first_token_dev) return set_err(IXT_ERR_INVALID, "null argument");
@@ -1932,6 +1996,7 @@ extern "C" int ixt_prefill_chunk(ixt_ctx* c, int slot, const int32_t* tokens_dev
   hipLaunchKernelGGL(k_rows_prefill, dim3((n_tokens + 255) / 256), dim3(256), 0, st, c->row_slot, c->row_pos, c->row_active, slot, start_pos, n_tokens,
                      c->ps.num_pages_used, c->P);
   LAUNCHCHK();
+  const WaitPass pass(c, n_tokens, false, st);
   c->one_segment = true;
   const int rc = forward_rows(c, n_tokens, tokens_dev, start_pos + n_tokens, n_tokens - 1, 1, nullptr, first_token_dev, last_logits_dev, false, st);
   c->one_segment = false;
@@ -1980,6 +2045,7 @@ extern "C" int ixt_prefill_rows(ixt_ctx* c, int n_rows, const int32_t* tokens_de
   hipLaunchKernelGGL(k_rows_packed, dim3((n_rows + 255) / 256), dim3(256), 0, st, c->row_slot, c->row_pos, c->row_active, row_group_dev, row_pos_dev, n_rows,
                      c->ps.num_pages_used, c->P, c->G, c->Tmax, max_len, c->ps.status);
   LAUNCHCHK();
+  const WaitPass pass(c, n_rows, false, st);
   if (c->hy) return forward_rows(c, n_rows, tokens_dev, max_len, 0, n_logits, logits_rows_dev, first_tokens_dev, logits_dev, false, st);
   HIPCHK(hipMemcpyAsync(c->lrows, logits_rows_dev, sizeof(int32_t) * n_logits, hipMemcpyDeviceToDevice, st));
   return forward_rows(c, n_rows, tokens_dev, max_len, 0, n_logits, c->lrows, first_tokens_dev, logits_dev, false, st);
@@ -1996,6 +2062,7 @@ static int decode_rows(ixt_ctx* c, const int32_t* tokens_dev, const int32_t* pos
 extern "C" int ixt_decode_step(ixt_ctx* c, const int32_t* tokens_dev, const int32_t* pos_dev, int32_t* next_tokens_dev, float* logits_dev, void* stream) {
   if (!c || !tokens_dev || !pos_dev || !next_tokens_dev) return set_err(IXT_ERR_INVALID, "null argument");
   if (c->B > 1024) return set_err(IXT_ERR_UNSUPPORTED, "max_slots > 1024");
+  const WaitPass pass(c, c->B, true, (hipStream_t)stream);
   return decode_rows(c, tokens_dev, pos_dev, next_tokens_dev, logits_dev, 0, (hipStream_t)stream);
 }
 
@@ -2014,10 +2081,11 @@ extern "C" int ixt_generate(ixt_ctx* c, int32_t* tokens_dev, int32_t* next_pos_d
   if (!c || !tokens_dev || !next_pos_dev || !generated_dev || !result_data_dev) return set_err(IXT_ERR_INVALID, "null argument");
   if (c->B > 1024) return set_err(IXT_ERR_UNSUPPORTED, "max_slots > 1024");
   hipStream_t st = (hipStream_t)stream;
+  const WaitPass pass(c, c->B, true, st);
   if (!c->cfg.use_hip_graph || c->timing) return generate_body(c, tokens_dev, next_pos_dev, generated_dev, result_data_dev, logits_dev, st);
   if (!ixt_weights_complete(c)) return set_err(IXT_ERR_NOT_LOADED, "weights incomplete");
   char key[160];
-  snprintf(key, sizeof(key), "%p/%p/%p/%p/%p", (void*)tokens_dev, (void*)next_pos_dev, (void*)generated_dev, (void*)result_data_dev, (void*)logits_dev);
+  snprintf(key, sizeof(key), "%p/%p/%p/%p/%p/%d", (void*)tokens_dev, (void*)next_pos_dev, (void*)generated_dev, (void*)result_data_dev, (void*)logits_dev, c->may_wait ? 1 : 0);
   auto it = c->graphs.find(key);
   if (it == c->graphs.end()) {
     // capture on a private stream so the caller's stream state is untouched
@@ -2035,6 +2103,7 @@ extern "C" int ixt_generate(ixt_ctx* c, int32_t* tokens_dev, int32_t* next_pos_d
       return rc != IXT_OK ? rc : set_err(IXT_ERR_HIP, "hipStreamEndCapture: %s", hipGetErrorString(e));
     }
     GraphEntry ge;
+    ge.forms = c->forms;
     e = hipGraphInstantiate(&ge.exec, graph, nullptr, nullptr, 0);
     (void)hipGraphDestroy(graph);
     (void)hipStreamDestroy(cs);
@@ -2046,6 +2115,7 @@ extern "C" int ixt_generate(ixt_ctx* c, int32_t* tokens_dev, int32_t* next_pos_d
     it = c->graphs.emplace(std::string(key), ge).first;
   }
   HIPCHK(hipGraphLaunch(it->second.exec, st));
+  c->forms = it->second.forms;
   return IXT_OK;
 }
 

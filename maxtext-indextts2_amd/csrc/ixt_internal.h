@@ -1,6 +1,7 @@
 // ixt_internal.h -- what the host objects of libixt share: the ctx, error reporting, memory ownership and the launch helpers of the canonical dot.
 #pragma once
 #include "../../include/ixt.h"
+#include "ixt_gate.h"
 #include "ixt_kernels.h"
 
 #include <hip/hip_runtime.h>
@@ -36,6 +37,7 @@ struct TimingPair { hipEvent_t a, b; double bytes; int family; };   // family: 0
 
 struct GraphEntry {
   hipGraphExec_t exec;
+  int forms = 0;
 };
 
 struct HybridModel;           // IXT_BLOCK_HYBRID (ixt_hybrid.h)
@@ -130,8 +132,11 @@ struct ixt_ctx {
   struct StepLayer* step_layers = nullptr;   // [L] in HBM
   bf16_t* step_ws = nullptr;
   int32_t* step_cnt = nullptr;
-  int32_t step_token = 0;
   bool step_ok = false;      // k_step has its buffers
+  struct DeviceGate* gate = nullptr;   // the GPU's (ixt_gate.h); nullptr: this model has no form that waits
+  hipEvent_t pass_event = nullptr;     // behind the last pass that could have taken one
+  int forms = 0;             // IXT_FORM_* that the last pass took
+  bool may_wait = false;     // the pass being enqueued is through it: k_step, k_mid
   int mid_rows = 64;         // passes of 17 to so many rows (<= 64): a launch between two attentions (k_mid) where the shapes allow; 0: a launch a phase
   bf16_t* mid_ws = nullptr;  // nullptr: not this model
   int32_t* mid_cnt = nullptr;

@@ -30,8 +30,8 @@ struct MidArgs {
   int layer, next;              // the layer of O .. DOWN, and of N1 / QKV (-1: not in this launch)
   const bf16_t *ao, *hin, *scale;        // attention's output (xidx), rows [64][E]; N1's scale (next layer's, or the head's)
   bf16_t *hmid, *hout, *xn1, *xn2, *act, *qbuf;   // rows, rows, operands in xidx layout
-  int32_t *cnt, *err, *done;    // [MID_PHASES][STEP_NS] lines of this launch; done: the last phase of a pass counts here, else nullptr
-  int R, E, F, QN, NQKV, token, last;    // last: that phase
+  int32_t *cnt, *err;           // [MID_PHASES][STEP_NS] lines of this launch
+  int R, E, F, QN, NQKV;
   int early;                    // blocks of the gated units that start beside the output projection
   int nblk[MID_PHASES], tpb[MID_PHASES], prev[MID_PHASES];     // blocks, tiles of a block; the phase to wait for (-1: none)
   float eps;
@@ -44,9 +44,6 @@ __device__ __forceinline__ int32_t* mid_cnt(const MidArgs& a, int phase) { retur
 __device__ __forceinline__ void mid_wait(const MidArgs& a, int phase) {
   if (a.prev[phase] >= 0) step_wait(mid_cnt(a, a.prev[phase]), a.nblk[a.prev[phase]], a.err);
   else __syncthreads();
-}
-__device__ __forceinline__ void mid_arrive(const MidArgs& a, int phase, int blk, int waves, int* met) {
-  if (step_arrive(mid_cnt(a, phase), blk, waves, met) && a.done != nullptr && phase == a.last) step_turn_on(a.done, a.nblk[phase], a.token);
 }
 
 // Weights of phase `to` (kernel at `off`, K x ntile tiles), of those of its `nb` blocks that will run on this XCD (the grid, from block p0 on, is dealt to the XCDs in turn), into its L2:
@@ -294,7 +291,7 @@ __device__ __forceinline__ void mid_dot(const MidArgs& a, int blk, u32x4* sx) {
   if (PHASE == MID_UP) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // nothing may land in LDS that the next block owns
   // (behind QKV nobody waits: the launch ends)
   const int storing = min(MID_NW, njobs);                    // (of a last block with fewer tiles some arrive with nothing stored)
-  if (PHASE != MID_QKV && wave < storing) mid_arrive(a, PHASE, blk_all, storing, &met);
+  if (PHASE != MID_QKV && wave < storing) step_arrive(mid_cnt(a, PHASE), blk_all, storing, &met);
 }
 
 // the norm of eight rows, a wave a row (k_step's order of operations), as the operand of the projections behind it
@@ -342,7 +339,7 @@ __device__ __forceinline__ void mid_norm(const MidArgs& a, int blk, u32x4* sx) {
     const int ch = i / MID_NW, rr = i % MID_NW;
     if (blk * MID_NW + rr < a.R) stg16_agent(dst + xidx(blk * MID_NW + rr, ch * 8, a.E), sx[ch * MID_NW + (rr ^ (ch & (MID_NW - 1)))]);
   }
-  mid_arrive(a, PHASE, blk, MID_NW, &met);
+  step_arrive(mid_cnt(a, PHASE), blk, MID_NW, &met);
 }
 
 template <int G>

@@ -8,9 +8,8 @@
 //
 // Progress: a block waits for blocks of lower index only, and those are dispatched before it (each XCD takes its share of the grid in order), so the
 // lowest unfinished block never waits for one that has not started, whatever runs beside it and ends by itself.  Two such grids would not: each could hold the
-// XCD that the other's lowest block has to start on.  So one of them at a time is on the chip (step_turn): k_step_begin waits for the turn, the last block of the last layer gives it
-// on.  The waits are bounded all the same (step_wait); processes that share a GPU have no turn between them
-// (options small_step and mid_rows).  Workgroups that draw their block's index from a counter, and stay, would need no turn: built, and slower
+// XCD that the other's lowest block has to start on.  So the host admits one pass with them at a time (ixt_gate.h).  The waits are bounded all the same (step_wait).
+// Workgroups that draw their block's index from a counter, and stay, would end beside each other: built, and slower
 // (us a step, 1 / 8 slots: 650 / 809 this, 833 / 1316 with the index drawn a block ahead, 780 / 956 behind the block's own wait; the draw holds up the wave's loads behind it).
 //
 // Data between blocks: written with agent-scope stores (past the XCD's L2), announced by a counter behind the stores' completion, and read by ordinary loads:
@@ -43,13 +42,12 @@ struct StepArgs {
   bf16_t* ws;                   // per layer: q [16][QN], attention [16][QN], hidden [16][E], units [16][F], hidden [16][E]
   size_t lstride;               // elements of a layer's buffers
   const bf16_t* h0;             // [R][E] rows in front of the first layer
-  int32_t* cnt;                 // [L][STEP_PHASES][STEP_NS] x 32 words and one line more (step_turn_on), zero at the start
+  int32_t* cnt;                 // [L][STEP_PHASES][STEP_NS] x 32 words, zero at the start
   int32_t* err;
   int R, E, F, QN, NQKV, rpl, fresh;       // fresh: positions in front of a row's own that this pass writes, at most
   int nblk[STEP_PHASES], tpb[STEP_PHASES]; // blocks of a phase, tiles of a block
-  int nl, per_layer, attw, att_floats, early;   // layers; blocks of one; waves and LDS floats of a (row, kv head); blocks of the gated units that start early
+  int per_layer, attw, att_floats, early;   // blocks of a layer; waves and LDS floats of a (row, kv head); blocks of the gated units that start early
   float eps;
-  int32_t token;                // this context's in step_turn
   const int32_t *row_slot, *row_pos, *row_active, *page_map;
   const bf16_t *rope_sin, *rope_cos;
   AttnGeom g;
@@ -62,28 +60,10 @@ __device__ __forceinline__ void step_st8(bf16_t* p, uint32_t lo, uint32_t hi) {
 __device__ __forceinline__ int32_t* step_cnt(const StepArgs& a, int layer, int phase) { return a.cnt + ((size_t)layer * STEP_PHASES + phase) * STEP_NS * 32; }
 
 // arrival of a block, by the last of its `waves` storing waves, behind their stores; `met` in LDS is zero
-__device__ __forceinline__ bool step_arrive(int32_t* cnt, int blk, int waves, int* met) {
+__device__ __forceinline__ void step_arrive(int32_t* cnt, int blk, int waves, int* met) {
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  if ((threadIdx.x & 63) != 0 || (waves > 1 && __hip_atomic_fetch_add(met, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) != waves - 1)) return false;
+  if ((threadIdx.x & 63) != 0 || (waves > 1 && __hip_atomic_fetch_add(met, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) != waves - 1)) return;
   __hip_atomic_fetch_add(cnt + (blk & (STEP_NS - 1)) * 32, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  return true;
-}
-
-// Whose pass is on the chip: 0 or a context's token.  The streams of a process take turns.
-static __device__ int32_t step_turn;
-#define STEP_TURN_LIMIT (1 << 22)
-__device__ __forceinline__ void step_turn_take(int32_t token, int32_t* err) {
-  for (int it = 0;; ++it) {
-    int32_t seen = 0;
-    if (__hip_atomic_compare_exchange_strong(&step_turn, &seen, token, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) || seen == token) return;
-    if (it > STEP_TURN_LIMIT) { __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); return; }
-    __builtin_amdgcn_s_sleep(8);
-  }
-}
-// by the wave that announced one of the `n` blocks of the last phase; nobody waits any more when the last of them has
-__device__ __forceinline__ void step_turn_on(int32_t* done, int n, int32_t token) {
-  if (__hip_atomic_fetch_add(done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != n - 1) return;
-  __hip_atomic_compare_exchange_strong(&step_turn, &token, 0, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // The first wave waits until the counters hold all `n` arrivals, the others at the barrier.  Most blocks stand here long before their phase is due: they look at
@@ -350,8 +330,7 @@ __device__ __forceinline__ void step_dot(const StepArgs& a, int layer, int blk, 
       bf16_t* dst = (PHASE == STEP_O ? hm : hout) + (size_t)row * E + tile * 16 + cq * 4;
       step_st8(dst, pack2(f2bf(bflo(hv.x) + rbf(tot[0])), f2bf(bfhi(hv.x) + rbf(tot[1]))), pack2(f2bf(bflo(hv.y) + rbf(tot[2])), f2bf(bfhi(hv.y) + rbf(tot[3]))));
     }
-    const bool last = step_arrive(step_cnt(a, layer, PHASE), blk, min(tpb, ntile - blk * tpb), &met);
-    if (PHASE == STEP_DOWN && last && layer == a.nl - 1) step_turn_on(step_cnt(a, a.nl, 0), a.nblk[STEP_DOWN], a.token);
+    step_arrive(step_cnt(a, layer, PHASE), blk, min(tpb, ntile - blk * tpb), &met);
   } else if constexpr (PHASE == STEP_UP) {
     if (row_ok) {
       bf16_t o[4];
@@ -643,10 +622,9 @@ __global__ __launch_bounds__(STEP_NW * 64, STEP_NW / 4) void k_step(StepArgs a) 
   step_dot<STEP_DOWN>(a, layer, b - a.nblk[STEP_UP], step_lds);
 }
 
-// rows of the embedding in front of the first layer; the counters and the turn of the launch behind it
-__global__ __launch_bounds__(256) void k_step_begin(const int32_t* tokens, const bf16_t* embedding, int E, bf16_t* h0, int32_t* cnt, int ncnt, int32_t token, int32_t* err) {
+// rows of the embedding in front of the first layer; the counters of the launch behind it
+__global__ __launch_bounds__(256) void k_step_begin(const int32_t* tokens, const bf16_t* embedding, int E, bf16_t* h0, int32_t* cnt, int ncnt) {
   const bf16_t* src = embedding + (size_t)tokens[blockIdx.x] * E;
   for (int i = threadIdx.x; i < E / 8; i += 256) *reinterpret_cast<u32x4*>(h0 + (size_t)blockIdx.x * E + i * 8) = *reinterpret_cast<const u32x4*>(src + i * 8);
   for (int i = blockIdx.x * 256 + threadIdx.x; i < ncnt; i += gridDim.x * 256) cnt[(size_t)i * 32] = 0;
-  if (blockIdx.x == 0 && threadIdx.x == 0) step_turn_take(token, err);
 }

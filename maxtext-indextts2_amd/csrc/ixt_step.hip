@@ -3,8 +3,6 @@
 #include "ixt_mid.h"
 #include "ixt_step.h"
 
-#include <atomic>
-
 // Which shapes: those whose rows, normed, and whose attention's pages fit the LDS of a CU and whose (tile, chain) pairs fit a block; other models of few rows take the
 // launches of ixt_small.h.
 #define STEP_LDS (150 * 1024)
@@ -81,7 +79,7 @@ bool mid_fits(const ixt_ctx* c, int R) {
   const size_t layer = ((size_t)c->E * (c->NQKV + 2 * c->F) + (size_t)(c->QN + c->F) * c->E) * sizeof(bf16_t);
   return c->mid_ws != nullptr && R >= 17 && R <= std::min(layer >= (size_t)48 << 20 ? 64 : 48, c->mid_rows) && mid_plan(c, R).ok;
 }
-static size_t mid_words(const ixt_ctx* c) { return (size_t)(c->L + 1) * MID_PHASES * STEP_NS + 1; }      // lines of its counters
+static size_t mid_words(const ixt_ctx* c) { return (size_t)(c->L + 1) * MID_PHASES * STEP_NS; }      // lines of its counters
 // the buffers of k_step and k_mid, once, at ixt_create (the launch may be captured)
 int step_init(ixt_ctx* c) {
   const bool step = step_model(c) && step_plan(c, 1).ok, mid = step_model(c) && c->Rmax >= 17 && mid_plan(c, 17).ok;
@@ -94,15 +92,13 @@ int step_init(ixt_ctx* c) {
     TRY(dmalloc(c, &c->mid_cnt, mid_words(c) * 32));
   }
   c->step_ok = step;
-  TRY(dmalloc(c, &c->step_cnt, ((size_t)c->L * STEP_PHASES * STEP_NS + 1) * 32));
+  TRY(dmalloc(c, &c->step_cnt, (size_t)c->L * STEP_PHASES * STEP_NS * 32));
   std::vector<StepLayer> t((size_t)c->L);
   auto at = [&](const void* p) { return (int64_t)(reinterpret_cast<intptr_t>(p) - reinterpret_cast<intptr_t>(c->step_ws)); };
   for (int l = 0; l < c->L; ++l) {
     const LayerW& w = c->layers[l];
     t[l] = StepLayer{at(w.wqkv), at(w.wo), at(w.wi), at(w.wout), at(w.ln1), at(w.ln2), at(c->kpages_l[l]), at(c->vpages_l[l])};
   }
-  static std::atomic<int32_t> contexts{0};
-  c->step_token = contexts.fetch_add(1) % 0x7fffffff + 1;
   HIPCHK(hipMemcpy(c->step_layers, t.data(), sizeof(StepLayer) * t.size(), hipMemcpyHostToDevice));
   return IXT_OK;
 }
@@ -110,16 +106,17 @@ bool step_fits(const ixt_ctx* c, int R) { return c->step_ok && step_plan(c, R).o
 // every layer of R rows; *hidden = the rows behind the last one.  fresh: step_attn
 int launch_step(ixt_ctx* c, int R, const int32_t* tokens, int fresh, const bf16_t** hidden, hipStream_t st) {
   const StepPlan p = step_plan(c, R);
+  c->forms |= IXT_FORM_STEP;
   StepArgs a;
   a.layers = c->step_layers; a.ws = c->step_ws; a.lstride = (size_t)16 * (2 * c->QN + 2 * c->E + c->F);
   a.h0 = c->h_a; a.cnt = c->step_cnt; a.err = c->split_cnt + (size_t)16 * c->KV * 4;
   a.R = R; a.E = c->E; a.F = c->F; a.QN = c->QN; a.NQKV = c->NQKV; a.rpl = p.rpl; a.fresh = fresh;
-  a.token = c->step_token; a.nl = c->L; a.per_layer = 0; a.attw = p.attw; a.att_floats = p.att_floats; a.early = p.early;
+  a.per_layer = 0; a.attw = p.attw; a.att_floats = p.att_floats; a.early = p.early;
   for (int i = 0; i < STEP_PHASES; ++i) { a.nblk[i] = p.nblk[i]; a.tpb[i] = p.tpb[i]; a.per_layer += p.nblk[i]; }
   a.eps = c->cfg.normalization_layer_epsilon;
   a.row_slot = c->row_slot; a.row_pos = c->row_pos; a.row_active = c->row_active; a.page_map = c->ps.page_map;
   a.rope_sin = c->rope_sin; a.rope_cos = c->rope_cos; a.g = c->geom;
-  hipLaunchKernelGGL(k_step_begin, dim3(R), dim3(256), 0, st, tokens, c->embedding, c->E, c->h_a, c->step_cnt, c->L * STEP_PHASES * STEP_NS + 1, a.token, a.err);
+  hipLaunchKernelGGL(k_step_begin, dim3(R), dim3(256), 0, st, tokens, c->embedding, c->E, c->h_a, c->step_cnt, c->L * STEP_PHASES * STEP_NS);
   LAUNCHCHK();
   *hidden = c->step_ws + (size_t)c->L * a.lstride - (size_t)16 * c->E;
 #define ST(HD_, GQ_) if (c->D == HD_ && c->GQ == GQ_) return launch_step_t<HD_, GQ_>(a, c->L, p.lds, st);
@@ -143,6 +140,7 @@ static int launch_mid_t(const MidArgs& a, int G, int blocks, size_t lds, hipStre
 // `final` their norm for the head, *normed.
 int launch_mid(ixt_ctx* c, int R, int l, const int32_t* tokens, bool final, const bf16_t** hidden, const bf16_t** normed, hipStream_t st) {
   const MidPlan p = mid_plan(c, R);
+  c->forms |= IXT_FORM_MID;
   const int G = (R + 15) / 16, lines = MID_PHASES * STEP_NS;
   bf16_t *h[2], *ws = c->mid_ws;
   auto take = [&](size_t n) { bf16_t* q = ws; ws += n; return q; };
@@ -154,8 +152,7 @@ int launch_mid(ixt_ctx* c, int R, int l, const int32_t* tokens, bool final, cons
   a.ao = c->ao; a.qbuf = c->qbuf; a.hin = h[(l + 2) & 1]; a.hout = h[(l + 1) & 1];
   a.scale = end ? c->final_norm : c->layers[l + 1].ln1;
   a.cnt = c->mid_cnt + (size_t)(l + 1) * lines * 32; a.err = c->split_cnt + (size_t)16 * c->KV * 4;
-  a.done = end ? c->mid_cnt + (size_t)(c->L + 1) * lines * 32 : nullptr;
-  a.R = R; a.E = c->E; a.F = c->F; a.QN = c->QN; a.NQKV = c->NQKV; a.token = c->step_token; a.last = final ? MID_N1 : MID_DOWN;
+  a.R = R; a.E = c->E; a.F = c->F; a.QN = c->QN; a.NQKV = c->NQKV;
   a.early = p.early;
   a.eps = c->cfg.normalization_layer_epsilon;
   a.row_slot = c->row_slot; a.row_pos = c->row_pos; a.row_active = c->row_active; a.page_map = c->ps.page_map;
@@ -170,7 +167,7 @@ int launch_mid(ixt_ctx* c, int R, int l, const int32_t* tokens, bool final, cons
     blocks += a.nblk[i];
   }
   if (l < 0) {
-    hipLaunchKernelGGL(k_step_begin, dim3(R), dim3(256), 0, st, tokens, c->embedding, c->E, h[0], c->mid_cnt, (int)mid_words(c), a.token, a.err);
+    hipLaunchKernelGGL(k_step_begin, dim3(R), dim3(256), 0, st, tokens, c->embedding, c->E, h[0], c->mid_cnt, (int)mid_words(c));
     LAUNCHCHK();
   }
   if (hidden) *hidden = a.hout;

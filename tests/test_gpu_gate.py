@@ -1,0 +1,132 @@
+"""Several engines on one GPU: passes whose launches have blocks that wait for each other (k_step, k_mid) beside each other on streams and threads.  Every token is what
+a model alone gives, whichever form a pass took."""
+import ctypes
+import threading
+
+import numpy as np
+import pytest
+
+import helpers as H
+from test_gpu_step import _config
+
+pytestmark = pytest.mark.gpu
+
+STEP, MID = 1, 2
+FEW, SOME = (1, 2048, 16, 16, 128, 7168), (20, 512, 4, 4, 64, 1024)      # rows, emb, query heads, kv heads, dim, mlp
+
+
+def forms(eng):
+  out = ctypes.c_int32(-1)
+  H.lib.check(eng.lib.ixt_pass_forms(eng._ctx, ctypes.byref(out)))
+  return out.value
+
+
+class Run:
+  """One engine with its prompts prefilled and inserted, on a stream of its own."""
+
+  def __init__(self, shape, seed, steps, **keys):
+    import torch
+    self.torch, self.stream, self.tokens = torch, torch.cuda.Stream(), []
+    self.cfg = _config(*shape, 12 + steps, 2, **keys)
+    self.eng, self.params = H.make_engine(self.cfg, H.synth.synth_weights(self.cfg, seed))
+    self.begin()
+
+  def begin(self):
+    with self.torch.cuda.stream(self.stream):
+      self.state, self.tokens = self.eng.init_decode_state(), []
+      for slot in range(self.eng.max_concurrent_decodes):
+        prefix, _ = self.eng.prefill(params=self.params, padded_tokens=H.synth.synth_prompt(self.cfg.vocab_size, 12, slot)[0], true_length=1 + slot % 12, slot=slot)
+        self.state = self.eng.insert(prefix, self.state, slot)
+    self.torch.cuda.synchronize()
+
+  def step(self):
+    with self.torch.cuda.stream(self.stream):
+      self.state, result = self.eng.generate(self.params, self.state)
+      self.tokens.append(result.data.clone())
+    return forms(self.eng)
+
+  def result(self):
+    self.torch.cuda.synchronize()
+    assert self.eng.exchange_status() == 0
+    return self.torch.stack(self.tokens).cpu().numpy()
+
+
+def test_a_pass_beside_another():
+  """While passes of another engine are on their way an engine takes the forms without waits; behind them, and alone, those with."""
+  a, b = Run(FEW, 1, 130), Run(SOME, 2, 130)
+  assert [a.step() for _ in range(60)] == [STEP] * 60
+  assert b.step() == 0 and a.step() == 0
+  a.result()
+  b.result()
+  assert [b.step() for _ in range(60)] == [MID] * 60
+  assert a.step() == 0 and b.step() == 0
+  b.result()
+  assert a.step() == STEP
+  got = [a.result(), b.result()]
+  for r, n, tokens in zip((a, b), (63, 62), got):
+    r.begin()
+    for _ in range(n):
+      r.step()
+      r.stream.synchronize()
+    assert np.array_equal(tokens, r.result())
+
+
+def test_engines_on_threads():
+  runs = [Run(FEW, 1, 60), Run(SOME, 2, 60), Run(FEW[:1] + (768, 12, 12, 64, 2048), 3, 60)]
+  alone = []
+  for r in runs:
+    for _ in range(50):
+      r.step()
+    alone.append(r.result())
+    r.begin()
+  errors = []
+
+  def work(r):
+    try:
+      for _ in range(50):
+        r.step()
+    except Exception as e:  # pylint: disable=broad-except
+      errors.append(e)
+
+  threads = [threading.Thread(target=work, args=(r,)) for r in runs]
+  for t in threads:
+    t.start()
+  for t in threads:
+    t.join(60)
+  assert not errors and not any(t.is_alive() for t in threads)
+  for r, want in zip(runs, alone):
+    assert np.array_equal(r.result(), want)
+
+
+def test_an_engine_that_goes_leaves_the_gate_open():
+  a, b = Run(FEW, 1, 20), Run(FEW, 2, 20)
+  for _ in range(10):
+    a.step()
+  a.eng.close()
+  assert b.step() == STEP
+  b.result()
+
+
+@pytest.mark.parametrize("shape", [FEW, SOME])
+def test_a_stream_that_the_caller_captures(shape):
+  """Its graph is replayed without a call into the library, so it holds no launch that waits."""
+  import torch
+  r = Run(shape, 4, 20, ixt_use_hip_graph=False)
+  want = []
+  for _ in range(6):
+    assert r.step() == (STEP if shape is FEW else MID)
+  want = r.result()
+  r.begin()
+  r.step()
+  torch.cuda.synchronize()
+  graph = torch.cuda.CUDAGraph()
+  with torch.cuda.graph(graph, stream=r.stream):
+    r.state, result = r.eng.generate(r.params, r.state)
+  assert forms(r.eng) == 0
+  got = [r.tokens[0]]
+  for _ in range(5):
+    graph.replay()
+    got.append(result.data.clone())
+    torch.randn(1 << 20, device="cuda").sum().item()
+  assert r.eng.exchange_status() == 0
+  assert np.array_equal(torch.stack(got).cpu().numpy(), want)

@@ -74,8 +74,8 @@ def test_packed_rows():
 
 
 def test_passes_of_two_engines_on_two_streams():
-  """Steps of two models in flight on two streams: the launches take turns (each would hold compute units that the other's blocks have to start on), and every
-  token is what a model alone gives."""
+  """Steps of two models in flight on two streams: never two whole steps as one launch beside each other (each would hold compute units that the other's blocks have to
+  start on), and every token is what a model alone gives."""
   import torch
   lens, steps = (33, 20), 200
   cfgs = [_config(1, 2048, 16, 16, 128, 7168, 33 + steps, 2), _config(1, 768, 12, 12, 64, 2048, 33 + steps, 6)]
