@@ -374,7 +374,7 @@ extern "C" int ixt_create(const ixt_config* cfg, ixt_ctx** out) {
   if (hipDeviceSynchronize() != hipSuccess) return fail(set_err(IXT_ERR_HIP, "page state init failed"));
   if (sdot_set_attributes() != IXT_OK) return fail(IXT_ERR_HIP);
   if (!hybrid && step_init(x) != IXT_OK) return fail(IXT_ERR_HIP);
-  if (x->step_ok || x->mid_ws != nullptr) {
+  if (!hybrid) {
     if (hipEventCreateWithFlags(&x->pass_event, hipEventDisableTiming) != hipSuccess) return fail(set_err(IXT_ERR_HIP, "event"));
     x->gate = device_gate();
     if (x->gate) x->gate->join(x, x->pass_event, [] { return hipDeviceSynchronize() == hipSuccess; });
@@ -1411,7 +1411,7 @@ static int attn_split_capacity(ixt_ctx* c, size_t lds) {
   c->split_capacity = cap;
   return cap;
 }
-static int attn_split_factor(ixt_ctx* c, int R) {
+static int attn_split_blocks(ixt_ctx* c, int R) {
   const AttnGeom& g = c->geom;
   if (c->small_attn_split < 2 || R > 16 || g.P > 32 || !(c->D == 256 || c->D == 128 || c->D == 64) || !(c->GQ == 1 || c->GQ == 2 || c->GQ == 4)) return 1;
   const size_t lds = sizeof(float) * ((size_t)c->GQ * c->D + (size_t)c->GQ * ((g.Tmax + 3) & ~3) + ((g.mpg + 3) & ~3) + 32 + (size_t)c->GQ * 4 * c->D + (size_t)c->GQ * ((g.mpg + 3) & ~3));
@@ -1426,6 +1426,8 @@ static int attn_split_factor(ixt_ctx* c, int R) {
   if (S > 16) S = 16;
   return S < 2 ? 1 : S;
 }
+// those of the pass being enqueued: its blocks wait for each other (ixt_gate.h)
+static int attn_split_factor(ixt_ctx* c, int R) { return c->may_wait ? attn_split_blocks(c, R) : 1; }
 template <int HD, int GQ>
 static void launch_attn_split_t(ixt_ctx* c, int layer, int R, int S, hipStream_t st, float cap, int window) {
   const AttnGeom& g = c->geom;
@@ -1438,6 +1440,7 @@ static void launch_attn_split_t(ixt_ctx* c, int layer, int R, int S, hipStream_t
   w.cnt = c->split_cnt; w.ws = c->split_ws; w.stride = c->split_stride; w.err = c->split_cnt + (size_t)16 * c->KV * 4; w.mpgp = (g.mpg + 3) & ~3;
   w.cap = cap; w.window = window;
   const size_t lds = sizeof(float) * ((size_t)GQ * HD + (size_t)GQ * ((g.Tmax + 3) & ~3) + w.mpgp + 32 + (size_t)GQ * 4 * HD + (size_t)GQ * w.mpgp);
+  c->forms |= IXT_FORM_SPLIT;
   hipLaunchKernelGGL((k_attn_split<HD, GQ>), dim3(g.nkv, R, S), dim3(256), lds, st, da, w);
 }
 static int launch_attn_split(ixt_ctx* c, int layer, int R, int S, hipStream_t st, float cap = 0.0f, int window = 0) {
@@ -1689,9 +1692,13 @@ static bool small_path_ok(const ixt_ctx* c, int R) {
          sdot_plan(c, GEPI_SWIGLU, true, c->E, 2 * c->F, R).ok;
 }
 static bool takes_step(ixt_ctx* c, int R, bool decode) {
-  return c->small_step && c->small_norm && !c->timing && step_fits(c, R) && !(decode && attn_split_factor(c, R) > 1);
+  return c->small_step && c->small_norm && !c->timing && step_fits(c, R) && !(decode && attn_split_blocks(c, R) > 1);
 }
 static bool takes_mid(const ixt_ctx* c, int R) { return c->mid_rows > 0 && !c->timing && !c->moe && !c->fp8 && mid_fits(c, R); }
+static bool takes_waits(ixt_ctx* c, int R, bool decode) {
+  if ((decode || c->gemma) && attn_split_blocks(c, R) > 1) return true;
+  return small_path_ok(c, R) ? takes_step(c, R, decode) : takes_mid(c, R);
+}
 static int forward_rows_small(ixt_ctx* c, int R, const int32_t* tokens, int len_hint, int lrow0, int nl, const int32_t* lrows, int32_t* argmax_out,
                               float* logits_out, bool decode, hipStream_t st) {
   const int E = c->E, F = c->F;
@@ -1956,7 +1963,7 @@ class WaitPass {
  public:
   WaitPass(ixt_ctx* c, int R, bool decode, hipStream_t st) : c_(c), st_(st) {
     c->forms = 0;
-    if (c->gate == nullptr || !(small_path_ok(c, R) ? takes_step(c, R, decode) : takes_mid(c, R))) return;
+    if (c->gate == nullptr || !takes_waits(c, R, decode)) return;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
       (void)hipGetLastError();

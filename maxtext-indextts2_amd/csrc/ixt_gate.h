@@ -1,6 +1,6 @@
-// ixt_gate.h -- which pass may take the launches whose blocks wait for each other (k_step, k_mid).
+// ixt_gate.h -- which pass may take the launches whose blocks wait for each other (k_step, k_mid, k_attn_split).
 //
-// One such grid ends beside anything that ends by itself (ixt_step.h).  Two of them need not: each could hold the compute units that a block of the other has to start on.  So a pass takes these
+// One such grid ends beside anything that ends by itself (ixt_step.h, ixt_small.h).  Two of them need not: each could hold the compute units that a block of the other has to start on.  So a pass takes these
 // forms only while no other context has a pass on the GPU, and otherwise the forms without waits, which give the same bits.  Nobody stands still for the answer.  (A turn that
 // kernels wait for needs a launch behind them to give it on, which a hardware queue shared with another stream may hold back, or which an error on the way may never send.)
 //

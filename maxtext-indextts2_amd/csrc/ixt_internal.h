@@ -133,10 +133,10 @@ struct ixt_ctx {
   bf16_t* step_ws = nullptr;
   int32_t* step_cnt = nullptr;
   bool step_ok = false;      // k_step has its buffers
-  struct DeviceGate* gate = nullptr;   // the GPU's (ixt_gate.h); nullptr: this model has no form that waits
+  struct DeviceGate* gate = nullptr;   // the GPU's (ixt_gate.h); nullptr: a hybrid decoder, which has no form that waits
   hipEvent_t pass_event = nullptr;     // behind the last pass that could have taken one
   int forms = 0;             // IXT_FORM_* that the last pass took
-  bool may_wait = false;     // the pass being enqueued is through it: k_step, k_mid
+  bool may_wait = false;     // the pass being enqueued is through it: k_step, k_mid, k_attn_split
   int mid_rows = 64;         // passes of 17 to so many rows (<= 64): a launch between two attentions (k_mid) where the shapes allow; 0: a launch a phase
   bf16_t* mid_ws = nullptr;  // nullptr: not this model
   int32_t* mid_cnt = nullptr;

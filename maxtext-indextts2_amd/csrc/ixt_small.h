@@ -503,8 +503,8 @@ __global__ __launch_bounds__(NW * 64) void k_attn_small(DecAttnArgs a) {
 //   out = super-block sums added in order                         -> exchange 3: the LAST block to arrive adds them (and re-arms the counters)
 // Exchanges go through a small global workspace per (row, kv head): agent-scope stores, a counter, agent-scope loads; the waits are bounded
 // (IXT_SPIN_LIMIT polls, then the error word is set and the block goes on -- wrong numbers, which the caller reports, but never a hang).  All
-// S blocks of a launch are resident at once (the host launches no more blocks than the occupancy query says fit the chip), so nobody waits for a
-// block that cannot start.
+// S blocks of a launch are resident at once (the host launches no more blocks than the occupancy query says fit the chip, and no other grid whose blocks
+// wait is on it: ixt_gate.h), so nobody waits for a block that cannot start.
 // Wave w of a block owns page 4 sb + w of each of its super-blocks in both phases: scores with lane = key (P <= 64 lanes busy), PV with
 // lane = 2 or 4 features (HD / FPL <= 64 lanes busy), all of a page's loads in flight at once.  Soft cap and sliding window as in k_attn_pv.
 // grid = (nkv, R, S), block 256.  LDS = GQ HD + GQ Tmax' + mpg' + 32 + GQ 4 HD + GQ mpg' floats.

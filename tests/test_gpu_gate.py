@@ -1,4 +1,4 @@
-"""Several engines on one GPU: passes whose launches have blocks that wait for each other (k_step, k_mid) beside each other on streams and threads.  Every token is what
+"""Several engines on one GPU: passes whose launches have blocks that wait for each other (k_step, k_mid, k_attn_split) beside each other on streams and threads.  Every token is what
 a model alone gives, whichever form a pass took."""
 import ctypes
 import threading
@@ -11,7 +11,7 @@ from test_gpu_step import _config
 
 pytestmark = pytest.mark.gpu
 
-STEP, MID = 1, 2
+STEP, MID, SPLIT = 1, 2, 4
 FEW, SOME = (1, 2048, 16, 16, 128, 7168), (20, 512, 4, 4, 64, 1024)      # rows, emb, query heads, kv heads, dim, mlp
 
 
@@ -95,6 +95,24 @@ def test_engines_on_threads():
     t.join(60)
   assert not errors and not any(t.is_alive() for t in threads)
   for r, want in zip(runs, alone):
+    assert np.array_equal(r.result(), want)
+
+
+@pytest.mark.parametrize("beside", [FEW, SOME])
+def test_split_attention_beside_whole_steps(beside):
+  """Blocks of the split decode attention all count on being on the chip together; 5 slots of 4 kv heads leave those of a head on several of its parts."""
+  split = Run((5, 512, 8, 4, 128, 512), 6, 200, model_name="gemma2-tiny", sliding_window_size=64)
+  other = Run(beside, 7, 200)
+  alone = []
+  for r, form in ((split, SPLIT), (other, STEP if beside is FEW else MID)):
+    assert [r.step() for _ in range(60)] == [form] * 60
+    alone.append(r.result())
+    r.begin()
+  seen = set()
+  for _ in range(60):
+    seen |= {split.step(), other.step()}
+  assert 0 in seen
+  for r, want in zip((split, other), alone):
     assert np.array_equal(r.result(), want)
 
 
