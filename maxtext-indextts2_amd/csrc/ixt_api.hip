@@ -91,14 +91,18 @@ static void host_rope_tables_llama31(const ixt_config& cfg, std::vector<float>& 
 }
 
 // the gate of the current GPU: one each, for the life of the process
-struct DeviceGate : IxtGate {};
+struct DeviceGate : IxtGate {
+  using IxtGate::IxtGate;
+};
 static DeviceGate* device_gate() {
   static std::mutex mu;
-  static std::map<int, DeviceGate> gates;
+  static std::map<std::string, DeviceGate> gates;
   int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return nullptr;
+  char bus[64] = "";
+  if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetPCIBusId(bus, sizeof(bus), dev) != hipSuccess) return nullptr;
+  const std::string file = std::string("/tmp/libixt-gpu-") + bus + ".lock";
   std::lock_guard<std::mutex> lk(mu);
-  return &gates[dev];
+  return &gates.try_emplace(file, file).first->second;
 }
 
 static int sdot_set_attributes();

@@ -1,6 +1,9 @@
 """Several engines on one GPU: passes whose launches have blocks that wait for each other (k_step, k_mid, k_attn_split) beside each other on streams and threads.  Every token is what
 a model alone gives, whichever form a pass took."""
 import ctypes
+import gc
+import subprocess
+import sys
 import threading
 
 import numpy as np
@@ -23,12 +26,14 @@ def forms(eng):
 
 class Run:
   """One engine with its prompts prefilled and inserted, on a stream of its own."""
+  alive = []
 
   def __init__(self, shape, seed, steps, **keys):
     import torch
     self.torch, self.stream, self.tokens = torch, torch.cuda.Stream(), []
     self.cfg = _config(*shape, 12 + steps, 2, **keys)
     self.eng, self.params = H.make_engine(self.cfg, H.synth.synth_weights(self.cfg, seed))
+    Run.alive.append(self.eng)
     self.begin()
 
   def begin(self):
@@ -49,6 +54,15 @@ class Run:
     self.torch.cuda.synchronize()
     assert self.eng.exchange_status() == 0
     return self.torch.stack(self.tokens).cpu().numpy()
+
+
+@pytest.fixture(autouse=True)
+def closed():
+  """Engines that are still there count: those of earlier tests go first."""
+  gc.collect()
+  yield
+  while Run.alive:
+    Run.alive.pop().close()
 
 
 def test_a_pass_beside_another():
@@ -148,3 +162,33 @@ def test_a_stream_that_the_caller_captures(shape):
     torch.randn(1 << 20, device="cuda").sum().item()
   assert r.eng.exchange_status() == 0
   assert np.array_equal(torch.stack(got).cpu().numpy(), want)
+
+
+HOLD = """
+import fcntl, os, sys
+fd = os.open(sys.argv[1], os.O_RDWR | os.O_CREAT, 0o666)
+fcntl.lockf(fd, fcntl.LOCK_EX | fcntl.LOCK_NB)
+print("held", flush=True)
+sys.stdin.readline()
+"""
+
+
+def test_beside_another_process():
+  """While another process holds the GPU's lock, passes take the forms without waits; they take it when it has gone."""
+  import torch
+  alone = Run(FEW, 5, 20)
+  for _ in range(8):
+    alone.step()
+  want = alone.result()
+  alone.eng.close()                                      # (this process's engines let go of the lock)
+  props = torch.cuda.get_device_properties(0)
+  lock = f"/tmp/libixt-gpu-{props.pci_domain_id:04x}:{props.pci_bus_id:02x}:{props.pci_device_id:02x}.0.lock"
+  with subprocess.Popen([sys.executable, "-c", HOLD, lock], stdin=subprocess.PIPE, stdout=subprocess.PIPE, text=True) as other:
+    assert other.stdout.readline() == "held\n"
+    r = Run(FEW, 5, 20)
+    assert [r.step() for _ in range(4)] == [0] * 4
+    other.stdin.write("\n")
+    other.stdin.flush()
+    assert other.wait(30) == 0
+  assert [r.step() for _ in range(4)] == [STEP] * 4
+  assert np.array_equal(r.result(), want)
