@@ -25,6 +25,7 @@ typedef enum ixt_status {
   IXT_ERR_HIP = -2,          /* a HIP runtime call failed; see ixt_last_error()                  */
   IXT_ERR_UNSUPPORTED = -3,  /* configuration outside the built path (reference: NotImplementedError) */
   IXT_ERR_NOT_LOADED = -4,   /* a weight needed by the call was never loaded                     */
+  IXT_ERR_WAIT = -6,         /* a wait between blocks of a launch gave up in an EARLIER pass; its results are wrong      */
   IXT_ERR_RANGE = -5         /* slot / length out of range (page_manager.py:529-532)             */
 } ixt_status;
 
@@ -236,11 +237,14 @@ int ixt_pages_status(ixt_ctx* ctx, int32_t* out4, int reset, void* stream);
 /* The same four words copied to PINNED host memory in stream order, without waiting: the caller records an event behind the call and reads
  * the words once it has completed (a throughput path checks the reservations of packed prefill N while pass N already runs). */
 int ixt_pages_status_async(ixt_ctx* ctx, int32_t* host_out4, void* stream);
-/* Few decode rows: the keys of a (row, kv head) are split over several thread blocks that exchange their softmax statistics through HBM
- * inside one launch (k_attn_split; option small_attn_split), or all layers of a pass, or what lies between two attentions, run in one launch whose blocks wait for
- * the phase before theirs (k_step, k_mid; options small_step, mid_rows), or a product's sum is handed from block to block (option ring_parts).  These waits are bounded; out1 (HOST) = 1 if a wait ever gave up since the last
- * reset (the affected step's numbers are then wrong -- the reference has no counterpart: its generate step, maxengine.py:838-935, is one XLA
- * program), 0 otherwise.  Synchronises `stream`; reset != 0 re-arms the exchange. */
+/* Some launches have blocks that wait for each other: the keys of a (row, kv head) split over several blocks that exchange their softmax statistics through HBM (k_attn_split; option
+ * small_attn_split), all layers of a pass, or what lies between two attentions, in one launch whose blocks wait for the phase before theirs (k_step, k_mid; options small_step, mid_rows),
+ * a product's sum handed from block to block (option ring_parts).  These waits are bounded (option wait_polls).  If one gives up, the pass's numbers, and the keys and values it cached, are
+ * wrong (the reference has no counterpart: its generate step, maxengine.py:838-935, is one XLA program).  Then ixt_generate's result rows of that pass are not valid (second column 0), and
+ * the next ixt_prefill_*, ixt_decode_step or ixt_generate call on the context returns IXT_ERR_WAIT, once, without a pass of its own.
+ * ixt_wait_check: that report alone, without a pass; it waits for nothing, so a pass still on its way is not covered.
+ * ixt_exchange_status: synchronises `stream`; out1 (HOST) = 1 if a wait gave up that was not reported yet, else 0; reset != 0 takes it as reported. */
+int ixt_wait_check(ixt_ctx* ctx);
 int ixt_exchange_status(ixt_ctx* ctx, int32_t* out1, int reset, void* stream);
 /* The forms of launches that the last pass enqueued took, of those whose blocks wait for each other (IXT_FORM_*, ORed; out1: HOST).  Two passes of different contexts that are on a GPU
  * at the same time never both take one of these: the later one takes the forms without waits, with the same results (so do passes on a stream that the caller captures). */

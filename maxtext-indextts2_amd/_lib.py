@@ -76,6 +76,7 @@ SIGNATURES = {
     "ixt_pages_status": (ctypes.c_int, [vp, c_i32p, ctypes.c_int, vp]),
     "ixt_pages_status_async": (ctypes.c_int, [vp, vp, vp]),
     "ixt_exchange_status": (ctypes.c_int, [vp, c_i32p, ctypes.c_int, vp]),
+    "ixt_wait_check": (ctypes.c_int, [vp]),
     "ixt_pass_forms": (ctypes.c_int, [vp, c_i32p]),
     "ixt_state_status": (ctypes.c_int, [vp, c_i32p, ctypes.c_int, vp]),
     "ixt_set_residual_tap": (ctypes.c_int, [vp, vp, ctypes.c_int64]),

@@ -277,8 +277,6 @@ extern "C" int ixt_create(const ixt_config* cfg, ixt_ctx** out) {
   A(dmalloc(x, &s.active_page_position, (size_t)s.groups));
   if (hybrid) {
     x->hy = hybrid_new();
-    A(dmalloc(x, &x->split_cnt, (size_t)128));
-    HIPCHK(hipMemset(x->split_cnt, 0, sizeof(int32_t) * 128));
     A(hybrid_init(x));
   } else {
   // workspaces
@@ -357,6 +355,14 @@ extern "C" int ixt_create(const ixt_config* cfg, ixt_ctx** out) {
     }
   }
   }
+  A(dmalloc(x, &x->gave, (size_t)1));
+  void *fault = nullptr, *fault_dev = nullptr;
+  if (hipMemset(x->gave, 0, sizeof(int32_t)) != hipSuccess || hipHostMalloc(&fault, 64, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess)
+    return fail(set_err(IXT_ERR_HIP, "words of the waits"));
+  x->fault = (int32_t*)fault;
+  *x->fault = 0;
+  if (hipHostGetDevicePointer(&fault_dev, fault, 0) != hipSuccess) return fail(set_err(IXT_ERR_HIP, "words of the waits"));
+  x->fault_dev = (int32_t*)fault_dev;
   A(dmalloc(x, &x->ring_flags, (size_t)RING_FLAGS));
   if (hipMemset(x->ring_flags, 0, sizeof(int32_t) * RING_FLAGS) != hipSuccess) return fail(set_err(IXT_ERR_HIP, "flags"));
   A(dmalloc(x, &x->row_slot, (size_t)R));
@@ -392,6 +398,7 @@ extern "C" int ixt_destroy(ixt_ctx* c) {
   (void)hipDeviceSynchronize();
   if (c->gate) c->gate->forget(c);
   if (c->pass_event) (void)hipEventDestroy(c->pass_event);
+  if (c->fault) (void)hipHostFree(c->fault);
   for (auto& kv : c->graphs) (void)hipGraphExecDestroy(kv.second.exec);
   for (auto& t : c->tpairs) { (void)hipEventDestroy(t.a); (void)hipEventDestroy(t.b); }
   for (void* p : c->allocs) (void)hipFree(p);
@@ -637,12 +644,15 @@ extern "C" int ixt_pages_status(ixt_ctx* c, int32_t* out4, int reset, void* stre
 extern "C" int ixt_exchange_status(ixt_ctx* c, int32_t* out1, int reset, void* stream) {
   if (!c || !out1) return set_err(IXT_ERR_INVALID, "null argument");
   hipStream_t st = (hipStream_t)stream;
-  int32_t* err = c->split_cnt + (size_t)16 * c->KV * 4;
-  HIPCHK(hipMemcpyAsync(out1, err, sizeof(int32_t), hipMemcpyDeviceToHost, st));
   HIPCHK(hipStreamSynchronize(st));
+  *out1 = reset ? __atomic_exchange_n(c->fault, 0, __ATOMIC_ACQ_REL) : __atomic_load_n(c->fault, __ATOMIC_ACQUIRE);
   if (reset && *out1 != 0) HIPCHK(hipMemsetAsync(c->ring_flags, 0, sizeof(int32_t) * RING_FLAGS, st));
-  if (reset && *out1 != 0) HIPCHK(hipMemsetAsync(c->split_cnt, 0, sizeof(int32_t) * ((size_t)16 * c->KV * 4 + 4), st));   // a wait that gave up leaves its counters armed
   return IXT_OK;
+}
+extern "C" int ixt_wait_check(ixt_ctx* c) {
+  if (!c) return set_err(IXT_ERR_INVALID, "null ctx");
+  if (__atomic_load_n(c->fault, __ATOMIC_ACQUIRE) == 0 || __atomic_exchange_n(c->fault, 0, __ATOMIC_ACQ_REL) == 0) return IXT_OK;
+  return set_err(IXT_ERR_WAIT, "a wait between blocks of a launch gave up in an earlier pass: the results of that pass, and the keys and values it cached, are not to be trusted");
 }
 extern "C" int ixt_pass_forms(ixt_ctx* c, int32_t* out1) {
   if (!c || !out1) return set_err(IXT_ERR_INVALID, "null argument");
@@ -834,7 +844,7 @@ int launch_ring(ixt_ctx* c, int epi, const bf16_t* x, const bf16_t* w, int K, in
   if (epi == GEPI_F32 && split) rc = RING_T(2, 4, 4, 2, 2, 4, GEPI_F32, 1);
   else if (epi == GEPI_F32 && e.rb_exp == nullptr && !wring && c->ring_cfg == 0 && ring_parts_fit(c, cfg, R, N, K)) {
     GemmEpi ep = e;
-    ep.flags = c->ring_flags; ep.err = c->split_cnt + (size_t)16 * c->KV * 4;
+    ep.flags = c->ring_flags; ep.wait = c->wait();
     rc = ring_launch_t<2, 4, 4, 1, 2, 5, GEPI_F32, 2>(x, w, K, N, R, chains, wring, ep, st, wave_cols);
   }
   else if (epi == GEPI_F32) RING(GEPI_F32)
@@ -1441,7 +1451,7 @@ static void launch_attn_split_t(ixt_ctx* c, int layer, int R, int S, hipStream_t
   da.kpages = c->kpages_l[layer]; da.vpages = c->vpages_l[layer];
   da.out = c->ao; da.g = g; da.qbuf = c->qbuf;
   SplitWs w{};
-  w.cnt = c->split_cnt; w.ws = c->split_ws; w.stride = c->split_stride; w.err = c->split_cnt + (size_t)16 * c->KV * 4; w.mpgp = (g.mpg + 3) & ~3;
+  w.cnt = c->split_cnt; w.ws = c->split_ws; w.stride = c->split_stride; w.wait = c->wait(); w.mpgp = (g.mpg + 3) & ~3;
   w.cap = cap; w.window = window;
   const size_t lds = sizeof(float) * ((size_t)GQ * HD + (size_t)GQ * ((g.Tmax + 3) & ~3) + w.mpgp + 32 + (size_t)GQ * 4 * HD + (size_t)GQ * w.mpgp);
   c->forms |= IXT_FORM_SPLIT;
@@ -2000,6 +2010,7 @@ class WaitPass {
 extern "C" int ixt_prefill_chunk(ixt_ctx* c, int slot, const int32_t* tokens_dev, int n_tokens, int start_pos, int32_t* first_token_dev,
                                  float* last_logits_dev, void* stream) {
   if (!c || !tokens_dev || !first_token_dev) return set_err(IXT_ERR_INVALID, "null argument");
+  TRY(ixt_wait_check(c));
   TRY(check_group(c, slot));
   if (n_tokens <= 0 || n_tokens > c->Rmax) return set_err(IXT_ERR_RANGE, "prefill chunk of %d rows (max %d)", n_tokens, c->Rmax);
   if (start_pos < 0 || start_pos + n_tokens > c->Tmax) return set_err(IXT_ERR_RANGE, "prefill beyond max_target_length");
@@ -2049,6 +2060,7 @@ extern "C" int ixt_prefill_prompt_logp(ixt_ctx* c, const int32_t* tokens_dev, in
 extern "C" int ixt_prefill_rows(ixt_ctx* c, int n_rows, const int32_t* tokens_dev, const int32_t* row_group_dev, const int32_t* row_pos_dev, int max_len,
                                 int n_logits, const int32_t* logits_rows_dev, int32_t* first_tokens_dev, float* logits_dev, void* stream) {
   if (!c || !tokens_dev || !row_group_dev || !row_pos_dev || (n_logits > 0 && (!logits_rows_dev || !first_tokens_dev))) return set_err(IXT_ERR_INVALID, "null argument");
+  TRY(ixt_wait_check(c));
   if (n_rows <= 0 || n_rows > c->Rmax) return set_err(IXT_ERR_RANGE, "packed prefill of %d rows (max %d: ixt_config.max_packed_rows)", n_rows, c->Rmax);
   if (c->hy ? (n_logits < 0 || n_logits > n_rows) : (n_logits <= 0 || n_logits > c->NLmax || n_logits > n_rows)) return set_err(IXT_ERR_RANGE, "packed prefill with %d prompts (max %d)", n_logits, c->NLmax);
   if (max_len <= 0 || max_len > c->Tmax) max_len = c->Tmax;
@@ -2072,6 +2084,7 @@ static int decode_rows(ixt_ctx* c, const int32_t* tokens_dev, const int32_t* pos
 
 extern "C" int ixt_decode_step(ixt_ctx* c, const int32_t* tokens_dev, const int32_t* pos_dev, int32_t* next_tokens_dev, float* logits_dev, void* stream) {
   if (!c || !tokens_dev || !pos_dev || !next_tokens_dev) return set_err(IXT_ERR_INVALID, "null argument");
+  TRY(ixt_wait_check(c));
   if (c->B > 1024) return set_err(IXT_ERR_UNSUPPORTED, "max_slots > 1024");
   const WaitPass pass(c, c->B, true, (hipStream_t)stream);
   return decode_rows(c, tokens_dev, pos_dev, next_tokens_dev, logits_dev, 0, (hipStream_t)stream);
@@ -2082,7 +2095,7 @@ static int generate_body(ixt_ctx* c, int32_t* tokens_dev, int32_t* next_pos_dev,
   hipLaunchKernelGGL(k_pages_advance, dim3(1), dim3(64), 0, st, c->ps);
   LAUNCHCHK();
   TRY(decode_rows(c, tokens_dev, next_pos_dev, c->new_tok, logits_dev, 1, st));
-  hipLaunchKernelGGL(k_generate_epilogue, dim3(1), dim3(((c->B + 63) / 64) * 64), 0, st, c->new_tok, tokens_dev, next_pos_dev, generated_dev, result_data_dev, c->B);
+  hipLaunchKernelGGL(k_generate_epilogue, dim3(1), dim3(((c->B + 63) / 64) * 64), 0, st, c->new_tok, tokens_dev, next_pos_dev, generated_dev, result_data_dev, c->B, c->gave);
   LAUNCHCHK();
   return IXT_OK;
 }
@@ -2090,6 +2103,7 @@ static int generate_body(ixt_ctx* c, int32_t* tokens_dev, int32_t* next_pos_dev,
 extern "C" int ixt_generate(ixt_ctx* c, int32_t* tokens_dev, int32_t* next_pos_dev, int32_t* generated_dev, int32_t* result_data_dev, float* logits_dev,
                             void* stream) {
   if (!c || !tokens_dev || !next_pos_dev || !generated_dev || !result_data_dev) return set_err(IXT_ERR_INVALID, "null argument");
+  TRY(ixt_wait_check(c));
   if (c->B > 1024) return set_err(IXT_ERR_UNSUPPORTED, "max_slots > 1024");
   hipStream_t st = (hipStream_t)stream;
   const WaitPass pass(c, c->B, true, st);
@@ -2366,7 +2380,7 @@ extern "C" int ixt_set_option(ixt_ctx* c, const char* name, int value) {
       {"gemm_split_min_blocks", &c->gemm_split_min_blocks, 1}, {"gemm_min_blocks", &c->gemm_min_blocks, 1}, {"gemm_min_rows", &c->gemm_min_rows, 1},
       {"unembed_gemm", &c->unembed_gemm, 0}, {"attn_wave_pairs", &c->attn_wave_pairs, 0}, {"attn_tile", &c->attn_tile, 0}, {"attn_tile_min_rows", &c->attn_tile_min_rows, 1}, {"dot_stream_min_blocks", &c->dot_stream_min_blocks, 1},
       {"ring_min_rows", &c->ring_min_rows, 1}, {"ring_mid_rows", &c->ring_mid_rows, 17}, {"ring_cfg", &c->ring_cfg, 0}, {"ring_split", &c->ring_split, 0}, {"ring_wlayout", &c->ring_wlayout, 0}, {"ring_down", &c->ring_down, -1}, {"unembed_tall", &c->unembed_tall, 0}, {"ring_two_per_cu", &c->ring_two_per_cu, 0},
-      {"small_rows", &c->small_rows, 0}, {"small_tpb", &c->small_tpb, 0}, {"small_attn_waves", &c->small_attn_waves, 4}, {"small_attn_max_blocks", &c->small_attn_max_blocks, 0}, {"dot_small", &c->dot_small, 0}, {"ring_parts", &c->ring_parts, 0}, {"small_step", &c->small_step, 0}, {"mid_rows", &c->mid_rows, 0}, {"small_norm", &c->small_norm, 0}, {"small_prefetch", &c->small_prefetch, 0}, {"small_prefetch_blocks", &c->small_prefetch_blocks, 1}, {"moe_grouped", &c->moe_grouped, 0}, {"small_attn_split", &c->small_attn_split, 0}, {"moe_route_blocks", &c->moe_route_blocks, 0}, {"gemma_tile", &c->gemma_tile, 0}, {"moe_fused_gate", &c->moe_fused_gate, 0}, {"moe_mid_pairs", &c->moe_mid_pairs, 0},
+      {"small_rows", &c->small_rows, 0}, {"small_tpb", &c->small_tpb, 0}, {"small_attn_waves", &c->small_attn_waves, 4}, {"small_attn_max_blocks", &c->small_attn_max_blocks, 0}, {"dot_small", &c->dot_small, 0}, {"ring_parts", &c->ring_parts, 0}, {"small_step", &c->small_step, 0}, {"wait_polls", &c->wait_polls, 0}, {"mid_rows", &c->mid_rows, 0}, {"small_norm", &c->small_norm, 0}, {"small_prefetch", &c->small_prefetch, 0}, {"small_prefetch_blocks", &c->small_prefetch_blocks, 1}, {"moe_grouped", &c->moe_grouped, 0}, {"small_attn_split", &c->small_attn_split, 0}, {"moe_route_blocks", &c->moe_route_blocks, 0}, {"gemma_tile", &c->gemma_tile, 0}, {"moe_fused_gate", &c->moe_fused_gate, 0}, {"moe_mid_pairs", &c->moe_mid_pairs, 0},
   };
   for (const Opt& o : opts) {
     if (strcmp(name, o.name) != 0) continue;

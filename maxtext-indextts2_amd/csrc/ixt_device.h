@@ -168,6 +168,14 @@ template <typename V> __device__ __forceinline__ void stg16_agent(void* p, const
   asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(p), "v"(v) : "memory");
 }
 
+// Waits of a block for another one of its launch are bounded: `polls` looks, then the block says so and goes on.  `gave` is the pass's own word on the device (cleared in front of a pass; who
+// sees it set waits no more, and k_generate_epilogue marks the result), `fault` the context's in host memory, which the next call reports.
+struct IxtWait { int32_t *gave, *fault; int polls; };
+__device__ __forceinline__ void ixt_gave_up(const IxtWait& w) {
+  __hip_atomic_store(w.gave, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __hip_atomic_store(w.fault, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // agent-scope (L1-bypassing) accesses for state one wave re-reads after writing it
 __device__ __forceinline__ int ldg_i32(const int32_t* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ __forceinline__ void stg_i32(int32_t* p, int v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }

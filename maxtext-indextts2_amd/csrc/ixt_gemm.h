@@ -93,7 +93,8 @@ struct GemmEpi {
   size_t sstride;                                       // F8 + routed experts: floats between two experts' column scales
   TanhNormEpi tn;                                       // TANHNORM (with act)
   int glu; float glu_limit; const float* act_par;       // ACT: the unit's kind and its numbers; SWIGLU: glu > 0 takes that gated unit of the f32 totals instead (ixt_glu), glu < 0 ixt_geglu
-  int32_t *flags, *err;                                 // SPLIT 2: a word a wave of a tile and part, zero between launches; a wait that gave up
+  int32_t* flags;                                       // SPLIT 2: a word a wave of a tile and part, zero between launches
+  IxtWait wait;
   const int32_t* rb_exp; size_t wstride;                // routed experts: expert of every 16-row block (-1: none), 16-byte units between experts' kernels
 };
 
@@ -115,7 +116,6 @@ __device__ __forceinline__ void ring_wait_chunks(int younger) {
 // index on the same XCD (gridDim.x is a multiple of 8), which has started before it; the waits are bounded all the same.  For few tiles of a long K: 256 x 2304 outputs, K 9216, 41 us in
 // one part (144 tiles of 64 x 64 for 256 CUs), 35 in three equal ones (72 of 128 x 64), 31 with a chain more for each later part.
 #define RING_KEEP 7
-#define RING_SPIN_LIMIT (1 << 20)
 //   grid = (8 ceil(ncolg / 8) zb, SPLIT 1 ? chains : SPLIT 2 ? parts : 1), block 64 WR WC, dynamic LDS = NS (WC CT + WR RB) KS KiB.
 //   Row groups of one column group are block ids b, b + 8, ..: same XCD, the weights meet in its L2.
 //   F8 (ixt_fp8.h): both operands are e4m3 fragments of 64 k (still 1 KiB: the ring moves them exactly as bf16 fragments of 32 k); a fragment
@@ -304,7 +304,7 @@ __global__ __launch_bounds__(WR * WC * 64, 2) void k_gemm_ring(const u32x4* __re
     float* p;
     if (part > 0) {
       for (int it = 0; __hip_atomic_load(flag + part - 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0;) {
-        if (++it > RING_SPIN_LIMIT) { __hip_atomic_store(e.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); break; }
+        if (++it > e.wait.polls) { ixt_gave_up(e.wait); break; }
         __builtin_amdgcn_s_sleep(1);
       }
       asm volatile("" ::: "memory");

@@ -121,7 +121,7 @@ struct ixt_ctx {
   int moe_fused_gate = 1;    // routed experts at few copies: wi as whole-K blocks with the SwiGLU epilogue (0: split-K slices + k_swiglu_part)
   int gemma_tile = 1;        // Gemma blocks: tiled prefill attention (0: the per-row scores / PV / combine kernels)
   int moe_route_blocks = 1;  // router: one wave per 512-k block, all experts at once (0: one wave per expert)
-  int32_t* split_cnt = nullptr;   // [16][KV][4] arrival counters (zero between launches) + the error word behind them
+  int32_t* split_cnt = nullptr;   // [16][KV][4] arrival counters (zero between launches)
   float* split_ws = nullptr;      // [16][KV][split_stride]
   size_t split_stride = 0;
   int small_prefetch = 0;    // few-rows path: prefetch blocks stream the next launch's kernel into the Infinity Cache (ixt_prefetch).  Measured SLOWER (one utterance 1.19 against 1.03 ms per step, eight 1.33 against 1.23: a launch cannot end before its prefetch has, and an Infinity-Cache hit is only 1.4 x an HBM stream): off
@@ -178,6 +178,10 @@ struct ixt_ctx {
   float* xs8 = nullptr;         // [rows16][chains]
   std::vector<TimingPair> tpairs;
   size_t tused = 0;
+  // bounded waits between blocks of a launch (IxtWait)
+  int32_t *gave = nullptr, *fault = nullptr, *fault_dev = nullptr;   // fault: pinned host memory, and what the GPU knows it by
+  int wait_polls = 1 << 20;     // (0.5 to 1 s)
+  IxtWait wait() const { return IxtWait{gave, fault_dev, wait_polls}; }
   // graphs keyed by the pointer tuple of ixt_generate
   std::map<std::string, GraphEntry> graphs;
   bool capturing = false;

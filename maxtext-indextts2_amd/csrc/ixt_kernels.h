@@ -2135,16 +2135,20 @@ static __global__ void k_rows_decode(int32_t* row_slot, int32_t* row_pos, int32_
   }
 }
 // maxengine.py:913-935
+// gave: a wait of the pass gave up, its tokens are not valid (one block: cleared for the next pass)
 static __global__ void k_generate_epilogue(const int32_t* new_tok, int32_t* tokens, int32_t* next_pos, int32_t* generated,
-                                    int32_t* result, int B) {
+                                    int32_t* result, int B, int32_t* gave) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  const int bad = *gave;
+  __syncthreads();
+  if (i == 0) *gave = 0;
   if (i < B) {
     tokens[i] = new_tok[i];
     next_pos[i] = next_pos[i] + 1;
     const int gnew = generated[i] + 1;
     generated[i] = gnew;
     result[i * 3 + 0] = new_tok[i];
-    result[i * 3 + 1] = 1;
+    result[i * 3 + 1] = bad ? 0 : 1;
     result[i * 3 + 2] = gnew;
   }
 }

@@ -30,7 +30,8 @@ struct MidArgs {
   int layer, next;              // the layer of O .. DOWN, and of N1 / QKV (-1: not in this launch)
   const bf16_t *ao, *hin, *scale;        // attention's output (xidx), rows [64][E]; N1's scale (next layer's, or the head's)
   bf16_t *hmid, *hout, *xn1, *xn2, *act, *qbuf;   // rows, rows, operands in xidx layout
-  int32_t *cnt, *err;           // [MID_PHASES][STEP_NS] lines of this launch
+  int32_t* cnt;                 // [MID_PHASES][STEP_NS] lines of this launch
+  IxtWait wait;
   int R, E, F, QN, NQKV;
   int early;                    // blocks of the gated units that start beside the output projection
   int nblk[MID_PHASES], tpb[MID_PHASES], prev[MID_PHASES];     // blocks, tiles of a block; the phase to wait for (-1: none)
@@ -42,7 +43,7 @@ struct MidArgs {
 template <typename T> __device__ __forceinline__ T* mid_at(const MidArgs& a, int64_t off) { return reinterpret_cast<T*>(reinterpret_cast<char*>(a.base) + off); }
 __device__ __forceinline__ int32_t* mid_cnt(const MidArgs& a, int phase) { return a.cnt + (size_t)phase * STEP_NS * 32; }
 __device__ __forceinline__ void mid_wait(const MidArgs& a, int phase) {
-  if (a.prev[phase] >= 0) step_wait(mid_cnt(a, a.prev[phase]), a.nblk[a.prev[phase]], a.err);
+  if (a.prev[phase] >= 0) step_wait(mid_cnt(a, a.prev[phase]), a.nblk[a.prev[phase]], a.wait);
   else __syncthreads();
 }
 

@@ -502,19 +502,18 @@ __global__ __launch_bounds__(NW * 64) void k_attn_small(DecAttnArgs a) {
 //   p = bf16(e / l); PV: one fma chain over a page's tokens, the 4 pages of a super-block added in order   (local)
 //   out = super-block sums added in order                         -> exchange 3: the LAST block to arrive adds them (and re-arms the counters)
 // Exchanges go through a small global workspace per (row, kv head): agent-scope stores, a counter, agent-scope loads; the waits are bounded
-// (IXT_SPIN_LIMIT polls, then the error word is set and the block goes on -- wrong numbers, which the caller reports, but never a hang).  All
+// (IxtWait: wrong numbers, which the caller reports, but never a hang).  All
 // S blocks of a launch are resident at once (the host launches no more blocks than the occupancy query says fit the chip, and no other grid whose blocks
 // wait is on it: ixt_gate.h), so nobody waits for a block that cannot start.
 // Wave w of a block owns page 4 sb + w of each of its super-blocks in both phases: scores with lane = key (P <= 64 lanes busy), PV with
 // lane = 2 or 4 features (HD / FPL <= 64 lanes busy), all of a page's loads in flight at once.  Soft cap and sliding window as in k_attn_pv.
 // grid = (nkv, R, S), block 256.  LDS = GQ HD + GQ Tmax' + mpg' + 32 + GQ 4 HD + GQ mpg' floats.
 // =====================================================================================================
-#define IXT_SPIN_LIMIT (1 << 18)
 struct SplitWs {
   int32_t* cnt;     // [R][nkv][4] arrival counters (zero between launches)
   float* ws;        // [R][nkv][stride]: maxima [GQ][16], page sums [GQ][mpgp], super-block sums [GQ][nsb_max][HD]
   size_t stride;
-  int32_t* err;     // set to 1 when a wait gave up
+  IxtWait wait;
   int mpgp;
   float cap;        // > 0: score = ixt_tanh(score / cap) * cap before the max (attn_logits_soft_cap, attentions.py:1257-1259), as k_attn_pv
   int window;       // > 0: keys j <= pos - window are invisible (LOCAL_SLIDING, attentions.py:625-631): e_j = p_j = +0, every sum unchanged
@@ -559,7 +558,7 @@ __device__ __forceinline__ void ixt_xld16x2(const float* p0, const float* p1, si
   asm volatile("" : "+v"(u[0]), "+v"(u[1]), "+v"(u[2]), "+v"(u[3]), "+v"(u[4]), "+v"(u[5]), "+v"(u[6]), "+v"(u[7]),
                "+v"(u[8]), "+v"(u[9]), "+v"(u[10]), "+v"(u[11]), "+v"(u[12]), "+v"(u[13]), "+v"(u[14]), "+v"(u[15]) : : "memory");   // (after the wait: volatile statements keep their order)
 }
-__device__ __forceinline__ void ixt_arrive_and_wait(int32_t* cnt, int target, int32_t* err, int tid) {
+__device__ __forceinline__ void ixt_arrive_and_wait(int32_t* cnt, int target, const IxtWait& w, int tid) {
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this thread's exchange stores have completed (at agent scope: they are sc1 stores)
   __syncthreads();
   if (tid == 0) {
@@ -567,7 +566,7 @@ __device__ __forceinline__ void ixt_arrive_and_wait(int32_t* cnt, int target, in
     int it = 0;
     while (__hip_atomic_load(cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target) {
       __builtin_amdgcn_s_sleep(1);
-      if (++it > IXT_SPIN_LIMIT) { __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); break; }
+      if (++it > w.polls) { ixt_gave_up(w); break; }
     }
   }
   __syncthreads();
@@ -715,7 +714,7 @@ __global__ __launch_bounds__(256) void k_attn_split(DecAttnArgs a, SplitWs w) {
   }
   __syncthreads();
   if (tid < GQ) ixt_xst(gmx + tid * 16 + s, fmaxf(fmaxf(wred[tid * 4], wred[tid * 4 + 1]), fmaxf(wred[tid * 4 + 2], wred[tid * 4 + 3])));
-  ixt_arrive_and_wait(cnt, S, w.err, tid);
+  ixt_arrive_and_wait(cnt, S, w.wait, tid);
   if (tid < GQ) {
     float mv[16];
     ixt_xld16(gmx + tid * 16, 1, S, mv);
@@ -740,7 +739,7 @@ __global__ __launch_bounds__(256) void k_attn_split(DecAttnArgs a, SplitWs w) {
     for (int t = 0; t < n; ++t) sacc = sacc + ep[t];
     ixt_xst(gps + (size_t)q * w.mpgp + p0 + pl, sacc);
   }
-  ixt_arrive_and_wait(cnt + 1, S, w.err, tid);
+  ixt_arrive_and_wait(cnt + 1, S, w.wait, tid);
   for (int i = tid; i < GQ * pages; i += 256) lps[(i / pages) * w.mpgp + i % pages] = ixt_xld(gps + (size_t)(i / pages) * w.mpgp + i % pages);   // one load per thread, all in flight
   __syncthreads();
   if (tid < GQ) {

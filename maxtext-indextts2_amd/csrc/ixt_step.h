@@ -30,7 +30,6 @@
 
 enum { STEP_QKV = 0, STEP_ATT, STEP_O, STEP_UP, STEP_DOWN, STEP_PHASES };
 #define STEP_NS 32              // counters of a phase, in lines of their own: arrivals on one word take turns (24 on each cost 1 us)
-#define STEP_SPIN_LIMIT (1 << 20)
 #define STEP_NW 16              // waves of a block; one block a CU
 
 // A layer's weights and pages, as distances in bytes from the launch's workspace: a pointer that a kernel reads from memory is a generic one, and FLAT loads
@@ -43,7 +42,7 @@ struct StepArgs {
   size_t lstride;               // elements of a layer's buffers
   const bf16_t* h0;             // [R][E] rows in front of the first layer
   int32_t* cnt;                 // [L][STEP_PHASES][STEP_NS] x 32 words, zero at the start
-  int32_t* err;
+  IxtWait wait;
   int R, E, F, QN, NQKV, rpl, fresh;       // fresh: positions in front of a row's own that this pass writes, at most
   int nblk[STEP_PHASES], tpb[STEP_PHASES]; // blocks of a phase, tiles of a block
   int per_layer, attw, att_floats, early;   // blocks of a layer; waves and LDS floats of a (row, kv head); blocks of the gated units that start early
@@ -68,14 +67,14 @@ __device__ __forceinline__ void step_arrive(int32_t* cnt, int blk, int waves, in
 
 // The first wave waits until the counters hold all `n` arrivals, the others at the barrier.  Most blocks stand here long before their phase is due: they look at
 // one counter now and then until the phase has begun to end, and at all of them, without a pause, from there on.
-__device__ __forceinline__ void step_wait(const int32_t* cnt, int n, int32_t* err) {
+__device__ __forceinline__ void step_wait(const int32_t* cnt, int n, const IxtWait& w) {
   if (threadIdx.x < 64) {
     const int lane = threadIdx.x & (STEP_NS - 1), mine = (int)blockIdx.x & (STEP_NS - 1);
     const int due = (n + STEP_NS - 1 - lane) / STEP_NS;
     auto look = [&](int i) { return __hip_atomic_load(cnt + i * 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
     auto give_up = [&](int it) {         // some block gave up: nobody waits for it
-      if (it > STEP_SPIN_LIMIT) { __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); return true; }
-      return (it & 255) == 0 && __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
+      if (it > w.polls) { ixt_gave_up(w); return true; }
+      return (it & 255) == 0 && __hip_atomic_load(w.gave, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
     };
     int it = 0;
     if (mine < n) {
@@ -188,9 +187,9 @@ __device__ __forceinline__ void step_dot(const StepArgs& a, int layer, int blk, 
   bf16_t* hout = act + (size_t)16 * a.F;
   const bf16_t* hin = layer == 0 ? a.h0 : a.ws + (size_t)layer * a.lstride - (size_t)16 * E;
   if (PHASE == STEP_QKV) {
-    if (layer > 0) step_wait(step_cnt(a, layer - 1, STEP_DOWN), a.nblk[STEP_DOWN], a.err);
+    if (layer > 0) step_wait(step_cnt(a, layer - 1, STEP_DOWN), a.nblk[STEP_DOWN], a.wait);
   } else {
-    step_wait(step_cnt(a, layer, PHASE - 1), a.nblk[PHASE - 1], a.err);
+    step_wait(step_cnt(a, layer, PHASE - 1), a.nblk[PHASE - 1], a.wait);
   }
 
   f32x4 acc = f32x4(0.0f);
@@ -449,7 +448,7 @@ __device__ __forceinline__ void step_attn(const StepArgs& a, int layer, int blk,
     touch(vpages, 0, (old >> 3) * (per / 4));
     touch(kpages, 2 * aw * per, (old >> 5) * per);                 // (a page of keys is as large as one of values)
   }
-  step_wait(step_cnt(a, layer, STEP_QKV), a.nblk[STEP_QKV], a.err);
+  step_wait(step_cnt(a, layer, STEP_QKV), a.nblk[STEP_QKV], a.wait);
   for (int i = tid; i < GQ * HD; i += nt) qs[i] = bf2f(qsrc[i]);
   if (j0 >= old && j0 < kv_len) kload(j0);
   __syncthreads();
@@ -622,9 +621,10 @@ __global__ __launch_bounds__(STEP_NW * 64, STEP_NW / 4) void k_step(StepArgs a) 
   step_dot<STEP_DOWN>(a, layer, b - a.nblk[STEP_UP], step_lds);
 }
 
-// rows of the embedding in front of the first layer; the counters of the launch behind it
-__global__ __launch_bounds__(256) void k_step_begin(const int32_t* tokens, const bf16_t* embedding, int E, bf16_t* h0, int32_t* cnt, int ncnt) {
+// rows of the embedding in front of the first layer; the counters of the launch behind it, and the pass's word of waits given up
+__global__ __launch_bounds__(256) void k_step_begin(const int32_t* tokens, const bf16_t* embedding, int E, bf16_t* h0, int32_t* cnt, int ncnt, int32_t* gave) {
   const bf16_t* src = embedding + (size_t)tokens[blockIdx.x] * E;
   for (int i = threadIdx.x; i < E / 8; i += 256) *reinterpret_cast<u32x4*>(h0 + (size_t)blockIdx.x * E + i * 8) = *reinterpret_cast<const u32x4*>(src + i * 8);
   for (int i = blockIdx.x * 256 + threadIdx.x; i < ncnt; i += gridDim.x * 256) cnt[(size_t)i * 32] = 0;
+  if (blockIdx.x == 0 && threadIdx.x == 0) *gave = 0;
 }

@@ -109,14 +109,14 @@ int launch_step(ixt_ctx* c, int R, const int32_t* tokens, int fresh, const bf16_
   c->forms |= IXT_FORM_STEP;
   StepArgs a;
   a.layers = c->step_layers; a.ws = c->step_ws; a.lstride = (size_t)16 * (2 * c->QN + 2 * c->E + c->F);
-  a.h0 = c->h_a; a.cnt = c->step_cnt; a.err = c->split_cnt + (size_t)16 * c->KV * 4;
+  a.h0 = c->h_a; a.cnt = c->step_cnt; a.wait = c->wait();
   a.R = R; a.E = c->E; a.F = c->F; a.QN = c->QN; a.NQKV = c->NQKV; a.rpl = p.rpl; a.fresh = fresh;
   a.per_layer = 0; a.attw = p.attw; a.att_floats = p.att_floats; a.early = p.early;
   for (int i = 0; i < STEP_PHASES; ++i) { a.nblk[i] = p.nblk[i]; a.tpb[i] = p.tpb[i]; a.per_layer += p.nblk[i]; }
   a.eps = c->cfg.normalization_layer_epsilon;
   a.row_slot = c->row_slot; a.row_pos = c->row_pos; a.row_active = c->row_active; a.page_map = c->ps.page_map;
   a.rope_sin = c->rope_sin; a.rope_cos = c->rope_cos; a.g = c->geom;
-  hipLaunchKernelGGL(k_step_begin, dim3(R), dim3(256), 0, st, tokens, c->embedding, c->E, c->h_a, c->step_cnt, c->L * STEP_PHASES * STEP_NS);
+  hipLaunchKernelGGL(k_step_begin, dim3(R), dim3(256), 0, st, tokens, c->embedding, c->E, c->h_a, c->step_cnt, c->L * STEP_PHASES * STEP_NS, c->gave);
   LAUNCHCHK();
   *hidden = c->step_ws + (size_t)c->L * a.lstride - (size_t)16 * c->E;
 #define ST(HD_, GQ_) if (c->D == HD_ && c->GQ == GQ_) return launch_step_t<HD_, GQ_>(a, c->L, p.lds, st);
@@ -151,7 +151,7 @@ int launch_mid(ixt_ctx* c, int R, int l, const int32_t* tokens, bool final, cons
   a.layers = c->step_layers; a.base = c->step_ws; a.layer = l; a.next = end ? -1 : l + 1;
   a.ao = c->ao; a.qbuf = c->qbuf; a.hin = h[(l + 2) & 1]; a.hout = h[(l + 1) & 1];
   a.scale = end ? c->final_norm : c->layers[l + 1].ln1;
-  a.cnt = c->mid_cnt + (size_t)(l + 1) * lines * 32; a.err = c->split_cnt + (size_t)16 * c->KV * 4;
+  a.cnt = c->mid_cnt + (size_t)(l + 1) * lines * 32; a.wait = c->wait();
   a.R = R; a.E = c->E; a.F = c->F; a.QN = c->QN; a.NQKV = c->NQKV;
   a.early = p.early;
   a.eps = c->cfg.normalization_layer_epsilon;
@@ -167,7 +167,7 @@ int launch_mid(ixt_ctx* c, int R, int l, const int32_t* tokens, bool final, cons
     blocks += a.nblk[i];
   }
   if (l < 0) {
-    hipLaunchKernelGGL(k_step_begin, dim3(R), dim3(256), 0, st, tokens, c->embedding, c->E, h[0], c->mid_cnt, (int)mid_words(c));
+    hipLaunchKernelGGL(k_step_begin, dim3(R), dim3(256), 0, st, tokens, c->embedding, c->E, h[0], c->mid_cnt, (int)mid_words(c), c->gave);
     LAUNCHCHK();
   }
   if (hidden) *hidden = a.hout;

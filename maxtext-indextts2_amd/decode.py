@@ -76,6 +76,8 @@ def main(argv: Sequence[str]) -> None:
 
   for i in range(_NUM_STREAMS):   # Get results, decode.py:175-179
     results = [int(t.get_result_at_slot(i).tokens.item()) for t in sampled_tokens_list]
+    if engine.exchange_status() != 0:
+      raise RuntimeError("a bounded wait between blocks of a launch gave up: the generated ids are not to be trusted")
     print(f"Input ids ({true_length}) -> {len(results)} generated ids: {results}")
     if mapping is not None:
       print(f"audio codes: {mapping.to_audio(np.array(results)).tolist()}")

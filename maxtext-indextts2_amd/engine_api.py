@@ -5,8 +5,8 @@ maxengine.py:506-518 / :915-926 and read as `t.get_result_at_slot(i).tokens.item
 `first_token.data`, `.log_prob` at tests/maxengine_test.py:111-164."""
 from __future__ import annotations
 
-from dataclasses import dataclass
-from typing import Any, Optional, Tuple
+from dataclasses import dataclass, field
+from typing import Any, Callable, Optional, Tuple
 
 import numpy as np
 
@@ -28,6 +28,11 @@ class ResultTokens:
   length_idx: Tuple[int, int]
   samples_per_slot: int
   log_prob: Optional[Any] = None
+  # raises if the engine found the pass behind `data` to have gone wrong; called once `data` is on the host, and not part of what the result is
+  check: Optional[Callable[[], None]] = field(default=None, repr=False, compare=False)
+
+  def __getstate__(self):
+    return dict(self.__dict__, check=None)
 
   def convert_to_numpy(self) -> "ResultTokens":
     d = self.data
@@ -36,6 +41,8 @@ class ResultTokens:
     lp = self.log_prob
     if lp is not None and hasattr(lp, "detach"):
       lp = lp.detach().cpu().numpy()
+    if self.check is not None:
+      self.check()
     return ResultTokens(np.asarray(d), self.tokens_idx, self.valid_idx, self.length_idx, self.samples_per_slot, lp)
 
   def get_result_at_slot(self, slot: int) -> SlotData:

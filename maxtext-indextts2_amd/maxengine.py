@@ -15,6 +15,7 @@ from __future__ import annotations
 import ctypes
 import dataclasses
 import os
+import weakref
 from typing import Any, Dict, Optional, Tuple
 
 import numpy as np
@@ -154,6 +155,8 @@ class MaxEngine(engine_api.Engine):
     self._result = torch.zeros((B, 3), dtype=torch.int32, device=self.device)
     self._first = torch.zeros((1,), dtype=torch.int32, device=self.device)
     self._page_failures = 0
+    alive = weakref.ref(self)                            # (a result does not keep the engine)
+    self._result_check = lambda: alive() and alive()._check_waits()
     self._recurrent = any(_architectures.carries_state(l) for l in config.hybrid_layers) if config.decoder_block == "hybrid" else False
     self._status_host = torch.zeros((4,), dtype=torch.int32).pin_memory()   # deferred reservation check of the packed prefill
     self._status_event = None
@@ -177,7 +180,14 @@ class MaxEngine(engine_api.Engine):
     ev.record(torch.cuda.current_stream())
     self._status_event, self._status_what = ev, what
 
+  def _check_waits(self) -> None:
+    """Raises, once, if a bounded wait between blocks of a launch gave up in a pass that has ended: that pass's results are wrong, and so is what it cached.
+    Looks at a word in host memory and waits for nothing."""
+    if self._ctx:
+      _lib.check(self.lib.ixt_wait_check(self._ctx))
+
   def _settle_pages(self) -> None:
+    self._check_waits()
     ev = self._status_event
     if ev is None:
       return
@@ -195,13 +205,11 @@ class MaxEngine(engine_api.Engine):
     out = (ctypes.c_int32 * 4)()
     _lib.check(self.lib.ixt_pages_status(self._ctx, out, 0, ctypes.c_void_p(_stream_ptr())))
     self._raise_if_new_failure(out[0], out[1], what)
-    if self.exchange_status() != 0:     # the stream is synchronised here anyway: the cheapest place to notice a decode step that went wrong
-      raise _lib.IxtError(f"{what}: a wait inside a launch of the few-rows path gave up in an earlier generate step (ixt_exchange_status); "
-                          "the tokens of that step are not to be trusted")
+    self._check_waits()     # the stream is synchronised here anyway
 
   def exchange_status(self, reset: bool = True) -> int:
-    """1 if a bounded wait of the few-rows path (blocks of one launch that wait for each other: split decode attention, whole steps)
-    ever gave up since the last reset -- the numbers of that step are wrong --, else 0.  Synchronises the stream."""
+    """1 if a bounded wait between blocks of a launch (split decode attention, whole steps, what lies between two attentions, products handed from block to block)
+    gave up in a pass so far -- its numbers are wrong -- and no call has raised for it yet, else 0.  Synchronises the stream."""
     out = (ctypes.c_int32 * 1)()
     _lib.check(self.lib.ixt_exchange_status(self._ctx, out, 1 if reset else 0, ctypes.c_void_p(_stream_ptr())))
     return int(out[0])
@@ -322,7 +330,7 @@ class MaxEngine(engine_api.Engine):
     generated = torch.zeros((1, 1), dtype=torch.int32, device=self.device)
     data = torch.cat([first, torch.ones_like(first), generated], dim=1)
     token_logp = self._token_logp(logits, first) if self.config.return_log_prob else None     # maxengine.py:502-505
-    result = engine_api.ResultTokens(data=data, tokens_idx=(0, 1), valid_idx=(1, 2), length_idx=(2, 3), log_prob=token_logp, samples_per_slot=1)
+    result = engine_api.ResultTokens(data=data, tokens_idx=(0, 1), valid_idx=(1, 2), length_idx=(2, 3), log_prob=token_logp, samples_per_slot=1, check=self._result_check)
     next_pos = torch.full((1, 1), start + true_length, dtype=torch.int32, device=self.device)
     prefix = {
         "logits": logits,
@@ -347,7 +355,7 @@ class MaxEngine(engine_api.Engine):
     generated = torch.zeros((num_samples, 1), dtype=torch.int32, device=self.device)
     data = torch.cat([first, torch.ones_like(first), generated], dim=1)
     logp = res1.log_prob.expand(num_samples, 1).contiguous() if res1.log_prob is not None else None      # maxengine.py:684-689
-    result = engine_api.ResultTokens(data=data, tokens_idx=(0, 1), valid_idx=(1, 2), length_idx=(2, 3), log_prob=logp, samples_per_slot=num_samples)
+    result = engine_api.ResultTokens(data=data, tokens_idx=(0, 1), valid_idx=(1, 2), length_idx=(2, 3), log_prob=logp, samples_per_slot=num_samples, check=self._result_check)
     prefix = dict(prefix, tokens=first, generated_tokens=generated)
     return prefix, result
 
@@ -406,7 +414,7 @@ class MaxEngine(engine_api.Engine):
     for i in range(n):
       data = torch.cat([tokens[i], torch.ones_like(tokens[i]), generated[i]], dim=1)
       results.append(engine_api.ResultTokens(data=data, tokens_idx=(0, 1), valid_idx=(1, 2), length_idx=(2, 3),
-                                             log_prob=logps[i:i + 1] if logps is not None else None, samples_per_slot=1))
+                                             log_prob=logps[i:i + 1] if logps is not None else None, samples_per_slot=1, check=self._result_check))
     prefill_results = {"logits": logits, "next_pos": next_pos, "generated_tokens": generated, "tokens": tokens, "prompt_logp": prompt_logp}
     cache = PagedCacheHandle(self, None, 0, groups=[B + i for i in range(n)], lengths=lens)
     return cache, prefill_results, results
@@ -487,7 +495,7 @@ class MaxEngine(engine_api.Engine):
                                      ctypes.c_void_p(self._result.data_ptr()), lg_ptr, ctypes.c_void_p(_stream_ptr())))
     data = self._result.clone()
     token_logp = self._token_logp(lg, data[:, 0:1]) if self.config.return_log_prob else None   # maxengine.py:907-910 (idle slots: of their stale logits)
-    result = engine_api.ResultTokens(data=data, tokens_idx=(0, 1), valid_idx=(1, 2), length_idx=(2, 3), log_prob=token_logp, samples_per_slot=1)
+    result = engine_api.ResultTokens(data=data, tokens_idx=(0, 1), valid_idx=(1, 2), length_idx=(2, 3), log_prob=token_logp, samples_per_slot=1, check=self._result_check)
     return decode_state, result
 
   # ------------------------------------------------------------------ insert
@@ -497,6 +505,7 @@ class MaxEngine(engine_api.Engine):
     del request_id
     if slot < 0 or slot >= self._B:
       raise ValueError(f"slot {slot} out of range [0, {self._B})")
+    self._check_waits()
     handle = prefix["cache"]
     st = ctypes.c_void_p(_stream_ptr())
     if isinstance(handle, PagedCacheHandle) and handle.slot is not None and handle.length > 0:

@@ -192,3 +192,71 @@ def test_beside_another_process():
     assert other.wait(30) == 0
   assert [r.step() for _ in range(4)] == [STEP] * 4
   assert np.array_equal(r.result(), want)
+
+
+# ---- waits that give up
+def _give_up(r, polls):
+  H.lib.check(r.eng.lib.ixt_set_option(r.eng._ctx, b"wait_polls", polls))
+
+
+GEMMA = dict(model_name="gemma2-tiny", sliding_window_size=64)
+
+
+@pytest.mark.parametrize("shape,form,keys", [(FEW, STEP, {}), (SOME, MID, {}), ((5, 512, 8, 4, 128, 512), SPLIT, GEMMA)], ids=["step", "mid", "split"])
+def test_a_wait_that_gives_up_is_reported(shape, form, keys):
+  """No looks at all: what is handed out says so, the next call raises, once, and passes behind it are right again."""
+  import torch
+  r = Run(shape, 9, 20, **keys)
+  for _ in range(5):
+    assert r.step() == form
+  want = r.result()
+  r.begin()
+  _give_up(r, 0)
+  assert r.step() == form
+  torch.cuda.synchronize()
+  assert not r.tokens[0][:, 1].any()                     # not valid
+  with pytest.raises(H.lib.IxtError, match="gave up"):
+    r.step()
+  _give_up(r, 1 << 20)
+  r.begin()                                              # reported: the prompts again
+  for _ in range(5):
+    assert r.step() == form
+  assert r.tokens[0][:, 1].all()
+  assert np.array_equal(r.result(), want)
+
+
+@pytest.mark.parametrize("late", ["convert", "insert", "prefill", "prefill_concat", "insert_partial", "step"])
+def test_where_it_is_reported(late):
+  """Whatever the engine is asked for next says what happened to the pass before."""
+  import torch
+  keys = dict(ixt_staging_groups=2, ixt_max_packed_rows=24, use_chunked_prefill=True) if late in ("prefill_concat", "insert_partial", "step") else {}
+  r = Run((2,) + FEW[1:], 10, 20, **keys)
+  toks = H.synth.synth_prompt(r.cfg.vocab_size, 12, 3)[0]
+  packed = dict(params=r.params, padded_tokens=np.tile(toks[:4], 2), decoder_positions=np.tile(np.arange(4, dtype=np.int32), 2), decoder_segment_ids=np.repeat(np.arange(2) + 1, 4).astype(np.int32),
+                start_pos=np.array([0, 4], np.int32), true_lengths=np.array([4, 4], np.int32), num_prompts=2)
+  with torch.cuda.stream(r.stream):
+    cache, prefix, _ = r.eng.prefill_concat(**packed) if keys else (None, None, None)
+    torch.cuda.synchronize()
+    _give_up(r, 0)
+    if late == "convert":
+      prefix, result = r.eng.prefill(params=r.params, padded_tokens=toks, true_length=12, slot=0)
+    elif late == "insert":
+      prefix, result = r.eng.prefill(params=r.params, padded_tokens=toks, true_length=12, slot=0)
+    else:
+      r.state, result = r.eng.generate(r.params, r.state)
+    if late != "convert":
+      torch.cuda.synchronize()
+    with pytest.raises(H.lib.IxtError, match="gave up"):
+      if late == "convert":
+        result.convert_to_numpy()
+      elif late == "insert":
+        r.eng.insert(prefix, r.state, 0)
+      elif late == "prefill":
+        r.eng.prefill(params=r.params, padded_tokens=toks, true_length=12, slot=0)
+      elif late == "prefill_concat":
+        r.eng.prefill_concat(**packed)
+      elif late == "insert_partial":
+        r.eng.insert_partial(prefix, r.state, cache, [0, 1], num_prompts=2)
+      else:
+        r.eng.step([(0, 0, toks[:3], [2])])
+  assert r.eng.exchange_status() == 0                    # reported once
