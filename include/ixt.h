@@ -246,9 +246,9 @@ int ixt_pages_status_async(ixt_ctx* ctx, int32_t* host_out4, void* stream);
  * ixt_exchange_status: synchronises `stream`; out1 (HOST) = 1 if a wait gave up that was not reported yet, else 0; reset != 0 takes it as reported. */
 int ixt_wait_check(ixt_ctx* ctx);
 int ixt_exchange_status(ixt_ctx* ctx, int32_t* out1, int reset, void* stream);
-/* The forms of launches that the last pass enqueued took, of those whose blocks wait for each other (IXT_FORM_*, ORed; out1: HOST).  Two passes of different contexts that are on a GPU
- * at the same time never both take one of these: the later one takes the forms without waits, with the same results (so do passes on a stream that the caller captures). */
-enum { IXT_FORM_STEP = 1, IXT_FORM_MID = 2, IXT_FORM_SPLIT = 4 };
+/* The forms of launches that the last pass (or ixt_op_dot) enqueued took, of those whose blocks wait for each other (IXT_FORM_*, ORed; out1: HOST).  Two passes of different contexts that are on a GPU
+ * at the same time never both take one of the first three: the later one takes the forms without waits, with the same results (so do passes on a stream that the caller captures). */
+enum { IXT_FORM_STEP = 1, IXT_FORM_MID = 2, IXT_FORM_SPLIT = 4, IXT_FORM_PARTS = 8 };
 int ixt_pass_forms(ixt_ctx* ctx, int32_t* out1);
 /* Recurrent layers (IXT_BLOCK_HYBRID): rows that did not start where their group's state stands (nor at position 0), or a second run of rows of one
  * group in one call, are left idle and counted; out1 (HOST) = their number of runs since the last reset.  Synchronises `stream`. */

@@ -646,7 +646,6 @@ extern "C" int ixt_exchange_status(ixt_ctx* c, int32_t* out1, int reset, void* s
   hipStream_t st = (hipStream_t)stream;
   HIPCHK(hipStreamSynchronize(st));
   *out1 = reset ? __atomic_exchange_n(c->fault, 0, __ATOMIC_ACQ_REL) : __atomic_load_n(c->fault, __ATOMIC_ACQUIRE);
-  if (reset && *out1 != 0) HIPCHK(hipMemsetAsync(c->ring_flags, 0, sizeof(int32_t) * RING_FLAGS, st));
   return IXT_OK;
 }
 extern "C" int ixt_wait_check(ixt_ctx* c) {
@@ -844,6 +843,7 @@ int launch_ring(ixt_ctx* c, int epi, const bf16_t* x, const bf16_t* w, int K, in
   if (epi == GEPI_F32 && split) rc = RING_T(2, 4, 4, 2, 2, 4, GEPI_F32, 1);
   else if (epi == GEPI_F32 && e.rb_exp == nullptr && !wring && c->ring_cfg == 0 && ring_parts_fit(c, cfg, R, N, K)) {
     GemmEpi ep = e;
+    c->forms |= IXT_FORM_PARTS;
     ep.flags = c->ring_flags; ep.wait = c->wait();
     rc = ring_launch_t<2, 4, 4, 1, 2, 5, GEPI_F32, 2>(x, w, K, N, R, chains, wring, ep, st, wave_cols);
   }
@@ -2162,6 +2162,7 @@ static int transpose_rows(ixt_ctx* c, const bf16_t* x, int R, int K, hipStream_t
 
 extern "C" int ixt_op_dot(ixt_ctx* c, const uint16_t* x, const uint16_t* w, float* out, int R, int K, int N, void* stream) {
   if (!c || !x || !w || !out || R <= 0) return set_err(IXT_ERR_INVALID, "bad argument");
+  c->forms = 0;
   hipStream_t st = (hipStream_t)stream;
   if (K % IXT_MK || N % 16) return set_err(IXT_ERR_UNSUPPORTED, "dot: K %% 32 or N %% 16");
   if ((size_t)((K + IXT_CHAIN - 1) / IXT_CHAIN) * R * N > c->part_floats && (size_t)R * N > c->part_floats)

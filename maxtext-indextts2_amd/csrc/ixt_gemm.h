@@ -116,6 +116,7 @@ __device__ __forceinline__ void ring_wait_chunks(int younger) {
 // index on the same XCD (gridDim.x is a multiple of 8), which has started before it; the waits are bounded all the same.  For few tiles of a long K: 256 x 2304 outputs, K 9216, 41 us in
 // one part (144 tiles of 64 x 64 for 256 CUs), 35 in three equal ones (72 of 128 x 64), 31 with a chain more for each later part.
 #define RING_KEEP 7
+#define RING_LEFT 2              // a flag whose taker gave up: its setter clears it, so that the next launch finds zeros whatever happened
 //   grid = (8 ceil(ncolg / 8) zb, SPLIT 1 ? chains : SPLIT 2 ? parts : 1), block 64 WR WC, dynamic LDS = NS (WC CT + WR RB) KS KiB.
 //   Row groups of one column group are block ids b, b + 8, ..: same XCD, the weights meet in its L2.
 //   F8 (ixt_fp8.h): both operands are e4m3 fragments of 64 k (still 1 KiB: the ring moves them exactly as bf16 fragments of 32 k); a fragment
@@ -302,9 +303,16 @@ __global__ __launch_bounds__(WR * WC * 64, 2) void k_gemm_ring(const u32x4* __re
     };
     int32_t* flag = e.flags + ((size_t)blockIdx.x * NW + wave) * parts;
     float* p;
+    bool ready = true;
     if (part > 0) {
       for (int it = 0; __hip_atomic_load(flag + part - 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0;) {
-        if (++it > e.wait.polls) { ixt_gave_up(e.wait); break; }
+        if (++it > e.wait.polls) {
+          int seen = 0;
+          if (lane == 0) __hip_atomic_compare_exchange_strong(flag + part - 1, &seen, RING_LEFT, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          ready = __builtin_amdgcn_readfirstlane(seen) != 0;
+          if (!ready) ixt_gave_up(e.wait);
+          break;
+        }
         __builtin_amdgcn_s_sleep(1);
       }
       asm volatile("" ::: "memory");
@@ -325,7 +333,7 @@ __global__ __launch_bounds__(WR * WC * 64, 2) void k_gemm_ring(const u32x4* __re
 #pragma unroll
             for (int b = 0; b < RB; ++b) tot[i][b] = tot[i][b] + keep[q][i][b];
         }
-      if (lane == 0) __hip_atomic_store(flag + part - 1, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (lane == 0 && ready) __hip_atomic_store(flag + part - 1, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     if (part < parts - 1) {
 #pragma unroll
@@ -334,7 +342,8 @@ __global__ __launch_bounds__(WR * WC * 64, 2) void k_gemm_ring(const u32x4* __re
         for (int b = 0; b < RB; ++b)
           if (place(i, b, p)) stg16_agent(p, tot[i][b]);
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      if (lane == 0) __hip_atomic_store(flag + part, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (lane == 0 && __hip_atomic_exchange(flag + part, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == RING_LEFT)
+        __hip_atomic_store(flag + part, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);      // nobody takes it any more
       return;
     }
   }

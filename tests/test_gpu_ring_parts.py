@@ -40,3 +40,27 @@ def test_parts_equal_whole_sums(wide, R, K, N):
     H.lib.check(eng.lib.ixt_set_option(eng._ctx, b"ring_parts", 1))
     assert torch.equal(got[0].view(torch.int32), got[1].view(torch.int32)), launch
   assert eng.exchange_status() == 0
+
+
+def test_a_hand_over_that_gave_up_leaves_nothing_behind(wide):
+  """Takers that do not wait at all, then launches with patience, which must not find a word of the late hand-over."""
+  torch, eng = wide["torch"], wide["eng"]
+  g = torch.Generator(device="cuda").manual_seed(3)
+  x, w = (torch.randn(shape, generator=g, device="cuda").mul_(f).bfloat16() for shape, f in (((256, 9216), 1.0), ((9216, 2304), 0.05)))
+
+  def run(polls, parts=1):
+    for name, value in ((b"wait_polls", polls), (b"ring_parts", parts)):
+      H.lib.check(eng.lib.ixt_set_option(eng._ctx, name, value))
+    out = torch.full((256, 2304), float("nan"), device="cuda")
+    H.lib.check(eng.lib.ixt_op_dot(eng._ctx, _vp(x), _vp(w), _vp(out), 256, 9216, 2304, _st(torch)))
+    return out.view(torch.int32)
+
+  try:
+    whole = run(1 << 20, 0)
+    for _ in range(4):
+      run(0)
+      assert torch.equal(run(1 << 20), whole)
+    assert eng.exchange_status() == 1                     # (with no look at all some taker was early)
+  finally:
+    for name, value in ((b"wait_polls", 1 << 20), (b"ring_parts", 1)):
+      H.lib.check(eng.lib.ixt_set_option(eng._ctx, name, value))
