@@ -766,7 +766,7 @@ static int ring_pick(const ixt_ctx* c, int epi, int R, int N, bool routed, bool 
 // tile picked, which is one round
 static bool ring_parts_fit(const ixt_ctx* c, int cfg, int R, int N, int K) {
   const int n = (K + IXT_CHAIN - 1) / IXT_CHAIN, colg = (N + 63) / 64, zb = (R + 127) / 128, longest = n - ((RING_PARTS - 1) * n / RING_PARTS - 1);
-  const int per_xcd = (colg + 7) / 8 * zb, one = cfg == 5 ? 31 : cfg == 3 ? 22 : cfg == 6 ? 19 : 0;
+  const int per_xcd = (colg + 7) / 8 * zb, one = cfg == 5 ? 31 : cfg == 3 ? 22 : 0;
   return c->ring_flags != nullptr && c->ring_parts && one > 0 && n >= 2 * RING_PARTS && longest <= RING_KEEP && per_xcd * RING_PARTS <= 32 && (size_t)per_xcd * 8 * 8 * RING_PARTS <= RING_FLAGS &&
          8 * longest * 44 + 300 < 8 * n * one;
 }

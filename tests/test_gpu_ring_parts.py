@@ -1,10 +1,12 @@
 """f32 sums of few tiles over a long K, three blocks a tile: against the oracle's bits and against one block a tile, several launches behind one another (the words
-through which blocks hand their sums on are zero between launches); ragged rows and columns, a short last chain, seventeen and eighteen chains."""
+through which blocks hand their sums on are zero between launches); ragged rows and columns, short last chains, six to eighteen chains."""
+import ctypes
+
 import numpy as np
 import pytest
 
 import helpers as H
-from test_gpu_ops import _dot_case, _st, _vp
+from test_gpu_ops import _st, _vp
 
 pytestmark = pytest.mark.gpu
 
@@ -18,10 +20,33 @@ def wide():
   return {"eng": eng, "O": O, "torch": torch}
 
 
-@pytest.mark.parametrize("R,K,N", [(130, 9216, 48), (200, 8448, 80), (250, 9088, 16), (256, 8704, 32)])
+PARTS = 8
+
+
+def _forms(eng):
+  out = ctypes.c_int32(-1)
+  H.lib.check(eng.lib.ixt_pass_forms(eng._ctx, ctypes.byref(out)))
+  return out.value
+
+
+# rows, K, columns: 6, 7, 8 chains (a part of one chain or two) and 11 beside tiles of 64 x 64, 12 and 16 beside 64 x 32, 17 and 18 beside both; short last chains, ragged rows and columns
+CASES = [(256, 3072, 2304), (200, 3456, 2064), (193, 4096, 2560), (250, 5504, 2320), (190, 6144, 2000), (300, 6144, 1520), (161, 8192, 1600), (256, 8448, 2304), (129, 8576, 2064),
+         (250, 9088, 2304), (256, 9216, 2048)]
+
+
+@pytest.mark.parametrize("R,K,N", CASES)
 def test_parts_against_the_oracle(wide, R, K, N):
+  """Rows at the edges of the tiles, every column."""
+  torch, eng, O = wide["torch"], wide["eng"], wide["O"]
   rng = np.random.default_rng(R + K + N)
-  _dot_case(wide, H.rand_bf16(rng, (R, K)), H.rand_bf16(rng, (K, N), 0.05))
+  x, w = H.rand_bf16(rng, (R, K)), H.rand_bf16(rng, (K, N), 0.05)
+  rows = sorted({0, 15, 16, 63, 64, 127, 128, R - 2, R - 1})
+  ref, some = np.zeros((len(rows), N), np.float32), np.ascontiguousarray(x[rows])
+  O.lib().orc_dot_rows(O._p(some, O._u16p), K, len(rows), O._p(w, O._u16p), K, N, O._p(ref, O._f32p), N)
+  xd, wd, out = H.dev_bf16(x), H.dev_bf16(w), torch.empty((R, N), dtype=torch.float32, device="cuda")
+  H.lib.check(eng.lib.ixt_op_dot(eng._ctx, _vp(xd), _vp(wd), _vp(out), R, K, N, _st(torch)))
+  assert _forms(eng) == PARTS
+  assert np.array_equal(out.cpu().numpy()[rows].view(np.uint32), ref.view(np.uint32))
 
 
 @pytest.mark.parametrize("R,K,N", [(256, 9216, 2304), (129, 9216, 2064), (190, 8320, 2000)])
@@ -36,6 +61,7 @@ def test_parts_equal_whole_sums(wide, R, K, N):
       H.lib.check(eng.lib.ixt_set_option(eng._ctx, b"ring_parts", parts))
       out = torch.full((R, N), float("nan"), device="cuda")
       H.lib.check(eng.lib.ixt_op_dot(eng._ctx, _vp(x), _vp(w), _vp(out), R, K, N, _st(torch)))
+      assert _forms(eng) == (PARTS if parts else 0)
       got.append(out)
     H.lib.check(eng.lib.ixt_set_option(eng._ctx, b"ring_parts", 1))
     assert torch.equal(got[0].view(torch.int32), got[1].view(torch.int32)), launch
