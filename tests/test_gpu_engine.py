@@ -1,6 +1,8 @@
 """GPU parity, engine level: MaxEngine (HIP) against OracleEngine (CPU) through the reference's call order
 (decode.py:133-184): prefill -> init_decode_state -> insert -> generate loop.  Bar: token ids, logits (f32 bit
 patterns), K/V cache contents and PageState are all bit-exact."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -17,8 +19,8 @@ def assert_pages_equal(eng, orc):
     assert np.array_equal(st[f], getattr(orc.page_state, f)), f
 
 
-def run_pair(cfg, weights, prompts, steps, use_graph=True, check_logits=True, chunks=None, options=None, sampling_ranges=None):
-  """prompts: list of (padded_tokens, true_length) one per slot (len <= batch).  Returns HIP token matrix."""
+def run_pair(cfg, weights, prompts, steps, use_graph=True, check_logits=True, chunks=None, options=None, sampling_ranges=None, forms=None):
+  """prompts: list of (padded_tokens, true_length) one per slot (len <= batch).  forms: what ixt_pass_forms has to say of the last step.  Returns HIP token matrix."""
   import torch
   eng, params = H.make_engine(cfg, weights)
   for name, value in (options or {}).items():
@@ -28,12 +30,12 @@ def run_pair(cfg, weights, prompts, steps, use_graph=True, check_logits=True, ch
     eng.set_sampling_ranges(sampling_ranges)
     orc.set_sampling_ranges(sampling_ranges)
   try:
-    return _run_pair(cfg, eng, params, orc, prompts, steps, check_logits, chunks)
+    return _run_pair(cfg, eng, params, orc, prompts, steps, check_logits, chunks, forms)
   finally:
     orc.set_sampling_ranges([])
 
 
-def _run_pair(cfg, eng, params, orc, prompts, steps, check_logits, chunks):
+def _run_pair(cfg, eng, params, orc, prompts, steps, check_logits, chunks, forms=None):
   import torch
   B = int(cfg.per_device_batch_size)
   prefixes, oprefixes = [], []
@@ -90,7 +92,11 @@ def _run_pair(cfg, eng, params, orc, prompts, steps, check_logits, chunks):
     kg, vg = eng.gather_kv(H.sublayers(cfg) - 1, slot, n)
     ko, vo = orc.model.gather_kv(H.sublayers(cfg) - 1, orc.page_state.page_map[slot], n)
     assert np.array_equal(H.bits(kg), ko) and np.array_equal(H.bits(vg), vo)
-  assert eng.exchange_status() == 0      # no bounded wait of the split decode attention gave up
+  assert eng.exchange_status() == 0      # no bounded wait gave up
+  if forms is not None:
+    took = ctypes.c_int32(-1)
+    H.lib.check(eng.lib.ixt_pass_forms(eng._ctx, ctypes.byref(took)))
+    assert took.value == forms
   del eng
   torch.cuda.synchronize()
   return np.stack(out, 0)

@@ -17,7 +17,7 @@ CASES = [
     (32, 1152, 4, 4, 64, 4608, 5, 2),
     (33, 768, 12, 12, 64, 2048, 40, 2),
     (48, 2048, 16, 16, 128, 7168, 3, 1),
-    (49, 512, 20, 10, 128, 1024, 6, 2),
+    (49, 1536, 20, 10, 128, 8192, 3, 1),
     (64, 1536, 2, 2, 128, 8192, 3, 2),
     (57, 2048, 4, 4, 128, 4736, 4, 2),
     (48, 128, 4, 4, 64, 256, 33, 2),
@@ -32,8 +32,8 @@ def test_decode_rows(case):
   rng = np.random.default_rng(rows)
   lengths = [longest, 1, max(1, longest - 1)] + [int(n) for n in rng.integers(1, longest + 1, rows - 4)]      # one slot stays idle
   prompts = [(H.synth.synth_prompt(cfg.vocab_size, longest, i)[0], n) for i, n in enumerate(lengths)]
-  one = run_pair(cfg, w, prompts, steps=4)
-  assert np.array_equal(one, run_pair(cfg, w, prompts, steps=4, options={"mid_rows": 0}))
+  one = run_pair(cfg, w, prompts, steps=4, forms=2)
+  assert np.array_equal(one, run_pair(cfg, w, prompts, steps=4, options={"mid_rows": 0}, forms=0))
 
 
 @pytest.mark.parametrize("rope", ["default", "llama3.1"])

@@ -38,8 +38,8 @@ def test_steps_as_one_launch(case):
   rng = np.random.default_rng(rows)
   lengths = [longest, 1, max(1, longest - 1)][:rows] + [int(n) for n in rng.integers(1, longest + 1, max(0, rows - 4))]      # from four rows on one slot stays idle
   prompts = [(H.synth.synth_prompt(cfg.vocab_size, longest, i)[0], n) for i, n in enumerate(lengths)]
-  one = run_pair(cfg, w, prompts, steps=5)
-  assert np.array_equal(one, run_pair(cfg, w, prompts, steps=5, options={"small_step": 0}))
+  one = run_pair(cfg, w, prompts, steps=5, forms=1)
+  assert np.array_equal(one, run_pair(cfg, w, prompts, steps=5, options={"small_step": 0}, forms=0))
 
 
 @pytest.mark.parametrize("rope", ["default", "llama3.1"])
