@@ -523,40 +523,13 @@ struct SplitWs {
 // invalidate is needed -- measured: with __threadfence() / acquire fences around the counter a one-utterance step took 1.64 instead of 1.05 ms).
 __device__ __forceinline__ void ixt_xst(float* p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ __forceinline__ float ixt_xld(const float* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
-// Eight agent-scope loads IN FLIGHT together (v[i] = p[i * stride], i < n <= 8; the rest 0).  The compiler waits for every relaxed atomic
-// load before it issues the next one (a 33-term sum took 33 memory round trips: Gemma-2 decode 4.5 -> 5.1 ms per step), so these are written
-// out: the loads, then ONE wait that owns all eight registers -- no use of a value can be scheduled in front of it.  n is wave-uniform.
-__device__ __forceinline__ void ixt_xld8(const float* p, size_t stride, int n, float (&v)[8]) {
+// Sixteen agent-scope loads IN FLIGHT together: v[i] = p[min(i, n - 1) * stride], 1 <= n <= 16, p in the workspace.  The compiler waits for every relaxed atomic
+// load before it issues the next one (a 33-term sum took 33 memory round trips: Gemma-2 decode 4.5 -> 5.1 ms per step); buffer loads with the same scope it counts.
+__device__ __forceinline__ void ixt_xld16(const SplitWs& w, const float* p, size_t stride, int n, float (&v)[16]) {
+  const __amdgpu_buffer_rsrc_t ws = __builtin_amdgcn_make_buffer_rsrc(w.ws, 0, -1, 0x00027000);
+  const int at = (int)((p - w.ws) * sizeof(float));
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    v[i] = 0.0f;
-    if (i < n) asm volatile("global_load_dword %0, %1, off sc1" : "=v"(v[i]) : "v"(p + (size_t)i * stride) : "memory");
-  }
-  asm volatile("s_waitcnt vmcnt(0)" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7]) : : "memory");
-}
-__device__ __forceinline__ void ixt_xld16(const float* p, size_t stride, int n, float (&v)[16]) {
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    v[i] = 0.0f;
-    if (i < n) asm volatile("global_load_dword %0, %1, off sc1" : "=v"(v[i]) : "v"(p + (size_t)i * stride) : "memory");
-  }
-  asm volatile("s_waitcnt vmcnt(0)" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7]),
-               "+v"(v[8]), "+v"(v[9]), "+v"(v[10]), "+v"(v[11]), "+v"(v[12]), "+v"(v[13]), "+v"(v[14]), "+v"(v[15]) : : "memory");
-}
-// two such batches (two output elements of a thread) behind ONE wait
-__device__ __forceinline__ void ixt_xld16x2(const float* p0, const float* p1, size_t stride, int n, float (&v)[16], float (&u)[16]) {
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    v[i] = 0.0f; u[i] = 0.0f;
-    if (i < n) {
-      asm volatile("global_load_dword %0, %1, off sc1" : "=v"(v[i]) : "v"(p0 + (size_t)i * stride) : "memory");
-      asm volatile("global_load_dword %0, %1, off sc1" : "=v"(u[i]) : "v"(p1 + (size_t)i * stride) : "memory");
-    }
-  }
-  asm volatile("s_waitcnt vmcnt(0)" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7]),
-               "+v"(v[8]), "+v"(v[9]), "+v"(v[10]), "+v"(v[11]), "+v"(v[12]), "+v"(v[13]), "+v"(v[14]), "+v"(v[15]) : : "memory");
-  asm volatile("" : "+v"(u[0]), "+v"(u[1]), "+v"(u[2]), "+v"(u[3]), "+v"(u[4]), "+v"(u[5]), "+v"(u[6]), "+v"(u[7]),
-               "+v"(u[8]), "+v"(u[9]), "+v"(u[10]), "+v"(u[11]), "+v"(u[12]), "+v"(u[13]), "+v"(u[14]), "+v"(u[15]) : : "memory");   // (after the wait: volatile statements keep their order)
+  for (int i = 0; i < 16; ++i) v[i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(ws, at + min(i, n - 1) * (int)(stride * sizeof(float)), 0, 1 << 4));     // sc1
 }
 __device__ __forceinline__ void ixt_arrive_and_wait(int32_t* cnt, int target, const IxtWait& w, int tid) {
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this thread's exchange stores have completed (at agent scope: they are sc1 stores)
@@ -717,7 +690,7 @@ __global__ __launch_bounds__(256) void k_attn_split(DecAttnArgs a, SplitWs w) {
   ixt_arrive_and_wait(cnt, S, w.wait, tid);
   if (tid < GQ) {
     float mv[16];
-    ixt_xld16(gmx + tid * 16, 1, S, mv);
+    ixt_xld16(w, gmx + tid * 16, 1, S, mv);
     float m = mv[0];
 #pragma unroll
     for (int i = 1; i < 16; ++i) if (i < S) m = fmaxf(m, mv[i]);
@@ -816,7 +789,8 @@ __global__ __launch_bounds__(256) void k_attn_split(DecAttnArgs a, SplitWs w) {
       float t0 = 0.0f, t1 = 0.0f;
       for (int sb = 0; sb < nsb; sb += 16) {
         float sv[16], su[16];
-        ixt_xld16x2(gsb + ((size_t)q0 * g.nsb_max + sb) * HD + d0, gsb + ((size_t)q1 * g.nsb_max + sb) * HD + d1, HD, min(16, nsb - sb), sv, su);
+        ixt_xld16(w, gsb + ((size_t)q0 * g.nsb_max + sb) * HD + d0, HD, min(16, nsb - sb), sv);
+        ixt_xld16(w, gsb + ((size_t)q1 * g.nsb_max + sb) * HD + d1, HD, min(16, nsb - sb), su);
 #pragma unroll
         for (int k = 0; k < 16; ++k) if (sb + k < nsb) { t0 = t0 + sv[k]; t1 = t1 + su[k]; }
       }
@@ -829,7 +803,7 @@ __global__ __launch_bounds__(256) void k_attn_split(DecAttnArgs a, SplitWs w) {
       float t = 0.0f;
       for (int sb = 0; sb < nsb; sb += 16) {
         float sv[16];
-        ixt_xld16(gsb + ((size_t)q * g.nsb_max + sb) * HD + d, HD, min(16, nsb - sb), sv);
+        ixt_xld16(w, gsb + ((size_t)q * g.nsb_max + sb) * HD + d, HD, min(16, nsb - sb), sv);
 #pragma unroll
         for (int k = 0; k < 16; ++k) if (sb + k < nsb) t = t + sv[k];
       }

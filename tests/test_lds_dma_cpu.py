@@ -94,3 +94,11 @@ def test_wide_stores_are_followed_by_a_wait_state():
           found += 1
           assert re.search(r"\\n\\ts_nop \d", text[at.end():]), (n, text)
   assert found > 0
+
+
+def test_no_load_of_memory_into_registers_in_asm():
+  """The compiler takes the registers of such a load as written at once: a copy of one, or another use of it, may come ahead of the wait."""
+  for n in sorted(os.listdir(build.CSRC)):
+    with open(os.path.join(build.CSRC, n), encoding="utf-8") as f:
+      for text in re.findall(r'asm(?: volatile)?\s*\(\s*"((?:[^"\\]|\\.)*)"', f.read()):
+        assert not re.search(r"(?:global|buffer|flat|scratch)_load_(?!lds)", text), (n, text)
