@@ -11,6 +11,7 @@
 #include <stdlib.h>
 
 #include <mutex>
+#include <thread>
 
 static thread_local char g_err[512] = "";
 int set_err(int code, const char* fmt, ...) {
@@ -387,7 +388,6 @@ extern "C" int ixt_create(const ixt_config* cfg, ixt_ctx** out) {
   if (!hybrid) {
     if (hipEventCreateWithFlags(&x->pass_event, hipEventDisableTiming) != hipSuccess) return fail(set_err(IXT_ERR_HIP, "event"));
     x->gate = device_gate();
-    if (x->gate) x->gate->join(x, x->pass_event, [] { return hipDeviceSynchronize() == hipSuccess; });
   }
   *out = x;
   return IXT_OK;
@@ -1979,29 +1979,23 @@ class WaitPass {
     c->forms = 0;
     if (c->gate == nullptr || !takes_waits(c, R, decode)) return;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
-      (void)hipGetLastError();
-      return;
-    }
+    if (!quietly(hipStreamIsCapturing(st, &cap)) || cap != hipStreamCaptureStatusNone) return;
     in_ = true;
-    c->may_wait = c->gate->enter(c, [](void* event) {
-      const bool ended = hipEventQuery((hipEvent_t)event) == hipSuccess;
-      if (!ended) (void)hipGetLastError();       // (not ready)
-      return ended;
-    });
+    const IxtGate::Lane lane(st, st == hipStreamPerThread ? std::this_thread::get_id() : std::thread::id());
+    c->may_wait = c->gate->enter(c, lane, c->pass_event, [](void* event) { return quietly(hipEventQuery((hipEvent_t)event)); }, [] { return quietly(hipDeviceSynchronize()); });
   }
   ~WaitPass() {
     if (!in_) return;
     c_->may_wait = false;
-    c_->gate->leave(c_, [this](void* event) {
-      const bool marked = hipEventRecord((hipEvent_t)event, st_) == hipSuccess;
-      if (!marked) (void)hipGetLastError();
-      return marked;
-    });
+    c_->gate->leave(c_, [this](void* event) { return quietly(hipEventRecord((hipEvent_t)event, st_)); });
   }
   WaitPass(const WaitPass&) = delete;
 
  private:
+  static bool quietly(hipError_t e) {            // (no error of the calls behind it)
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e == hipSuccess;
+  }
   ixt_ctx* c_;
   hipStream_t st_;
   bool in_ = false;

@@ -1,7 +1,7 @@
 // ixt_gate.h -- which pass may take the launches whose blocks wait for each other (k_step, k_mid, k_attn_split).
 //
 // One such grid ends beside anything that ends by itself (ixt_step.h, ixt_small.h).  Two of them need not: each could hold the compute units that a block of the other has to start on.  So a pass takes these
-// forms only while no other context has a pass on the GPU, and otherwise the forms without waits, which give the same bits.  Nobody stands still for the answer.  (A turn that
+// forms only while no other context has a pass on another stream of the GPU, and otherwise the forms without waits, which give the same bits.  Nobody stands still for the answer.  (A turn that
 // kernels wait for needs a launch behind them to give it on, which a hardware queue shared with another stream may hold back, or which an error on the way may never send.)
 //
 // That the other's pass counts whatever its form is a matter of speed: a grid of k_step beside launches of another pass slows both.  Two engines of the 1B model on two streams, ms for
@@ -20,69 +20,53 @@
 #include <map>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <utility>
 
 class IxtGate {
  public:
+  using Lane = std::pair<const void*, std::thread::id>;      // a stream; the thread where the handle means another stream in each
   explicit IxtGate(std::string lock_file = "") : file_(std::move(lock_file)) {}
-  // Context `who` comes, with an event of its own (any pointer).  `settle` waits for the GPU: passes of a context that was alone have no event behind them.
-  template <typename Settle>
-  void join(const void* who, void* event, Settle settle) {
-    std::map<const void*, long> open;
-    {
-      std::lock_guard<std::mutex> lk(mu_);
-      users_[who].event = event;
-      for (auto& u : users_)
-        if (u.second.state == OPEN) open[u.first] = u.second.passes;
-    }
-    if (open.empty() || !settle()) return;
+  // A pass of `who` (the caller orders those of one context) is about to be enqueued on stream `lane`: may it take the forms that wait?  leave() follows in either case.
+  // event: the context's own, for leave() to record; ended: has all in front of its last record ended?  settle: waits for the GPU; for passes without an event behind them.
+  template <typename Ended, typename Settle>
+  bool enter(const void* who, Lane lane, void* event, Ended ended, Settle settle) {
     std::lock_guard<std::mutex> lk(mu_);
-    for (auto& o : open) {
-      auto u = users_.find(o.first);
-      if (u != users_.end() && u->second.state == OPEN && u->second.passes == o.second) u->second.state = NONE;
+    bool alone = true, settled = false;
+    for (auto& u : users_) {
+      User& other = u.second;
+      if (u.first == who || other.state == NONE || other.lane == lane) continue;       // (passes of one stream run one after the other)
+      lanes_ = true;
+      if (other.state == OPEN && !settled) settled = settle();
+      if ((other.state == OPEN && settled) || (other.state == MARKED && ended(other.event))) other.state = NONE;
+      else alone = false;
     }
+    users_[who] = User{BEGUN, lane, event};
+    return alone && claim();
+  }
+  // It is enqueued; `mark` records the event behind it, which passes are spared (3 us of the host) until a second stream is seen.
+  template <typename Mark>
+  void leave(const void* who, Mark mark) {
+    std::lock_guard<std::mutex> lk(mu_);
+    User& me = users_[who];
+    me.state = lanes_ && mark(me.event) ? MARKED : OPEN;
   }
   // `who` is about to go, with nothing of it left on the GPU
   void forget(const void* who) {
     std::lock_guard<std::mutex> lk(mu_);
     users_.erase(who);
-    for (auto& u : users_)
-      if (u.second.passes > 0) return;
-    if (fd_ >= 0) (void)close(fd_);              // (and with it the lock)
+    if (users_.size() < 2) lanes_ = false;
+    if (!users_.empty() || fd_ < 0) return;
+    (void)close(fd_);                            // (and with it the lock)
     fd_ = -1;
-  }
-  // A pass of `who` (the caller orders those of one context) is about to be enqueued: may it take the forms that wait?  leave() follows in either case.
-  // `ended`: has everything in front of the last record of this event ended?
-  template <typename Ended>
-  bool enter(const void* who, Ended ended) {
-    std::lock_guard<std::mutex> lk(mu_);
-    bool alone = true;
-    for (auto& u : users_) {
-      if (u.first == who) continue;
-      if (u.second.state == MARKED && ended(u.second.event)) u.second.state = NONE;
-      alone = alone && u.second.state == NONE;
-    }
-    User& me = users_[who];
-    me.state = OPEN;
-    ++me.passes;
-    return alone && claim();
-  }
-  // It is enqueued; `mark` records the event behind it, which the only context of a GPU is spared (3 us of a pass).
-  template <typename Mark>
-  void leave(const void* who, Mark mark) {
-    std::lock_guard<std::mutex> lk(mu_);
-    User& me = users_[who];
-    if (users_.size() < 2) return;
-    if (mark(me.event)) me.state = MARKED;
-    else ++me.passes;                            // (a join that is waiting for the GPU may have begun before this pass)
   }
 
  private:
-  enum State { NONE, OPEN, MARKED };             // of a context's last pass: ended; enqueued or being enqueued; with the event behind it
+  enum State { NONE, BEGUN, OPEN, MARKED };      // of a context's last pass: it has ended; is being enqueued; is enqueued; with the event behind it
   struct User {
-    void* event = nullptr;
     State state = NONE;
-    long passes = 0;
+    Lane lane{};
+    void* event = nullptr;
   };
   // the file's lock.  A record lock: a child of fork() has no part in it, and cannot keep it.
   bool claim() {
@@ -104,7 +88,8 @@ class IxtGate {
   }
 
   std::mutex mu_;
-  std::map<const void*, User> users_;
+  std::map<const void*, User> users_;            // contexts whose passes asked
+  bool lanes_ = false;           // on different streams
   const std::string file_;
   int fd_ = -1;
 };

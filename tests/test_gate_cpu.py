@@ -1,5 +1,5 @@
 """The rule that keeps launches whose blocks wait for each other apart (csrc/ixt_gate.h), built for the host by itself and driven by threads: a pass may take them
-only while no other context's pass can be on the GPU, nobody stands still for the answer, and no path of errors leaves the gate shut."""
+only while no other context's pass can be on another stream of the GPU, nobody stands still for the answer, and no path of errors leaves the gate shut."""
 import os
 import shutil
 import signal
@@ -28,76 +28,69 @@ static auto broken = [](void*) { return false; };
 
 static const char* file;
 
+static IxtGate::Lane lane(long n) { return IxtGate::Lane(reinterpret_cast<void*>(n), std::thread::id()); }
+static int settles = 0;
+static auto settle = [] { ++settles; return true; };
+static auto cannot = [] { return false; };
+
 static int rules() {
   IxtGate g(file);
   Event a, b, c;
-  int settled = 0;
-  auto settle = [&] { ++settled; return true; };
-  g.join(&a, &a, settle);
-  CHECK(g.enter(&a, ended)); g.leave(&a, mark);
-  CHECK(a.ended);                                        // alone: no event
-  CHECK(g.enter(&a, ended)); g.leave(&a, mark);          // its own passes are in order
-  g.join(&b, &b, settle);
-  CHECK(settled == 1);                                   // a's last pass has no event: waited for
-  CHECK(g.enter(&b, ended)); g.leave(&b, mark);
-  CHECK(!b.ended);
-  CHECK(!g.enter(&a, ended)); g.leave(&a, mark);         // b's may still run
-  CHECK(!g.enter(&b, ended)); g.leave(&b, mark);         // so may a's
+  auto in = [&](Event& e, long n) { return g.enter(&e, lane(n), &e, ended, settle); };
+  auto out = [&](Event& e) { g.leave(&e, mark); };
+  CHECK(in(a, 1)); out(a);
+  CHECK(in(a, 2)); out(a);                               // its own passes are in order
+  CHECK(in(b, 2)); out(b);                               // so are those of one stream
+  CHECK(a.ended && b.ended && settles == 0);             // no event, no look
+  CHECK(in(c, 3)); out(c);
+  CHECK(settles == 1 && !c.ended);                       // passes without an event on another stream: waited for, once
+  CHECK(!in(a, 2)); out(a);                              // c's may still run
+  CHECK(!in(c, 3)); out(c);                              // so may a's
   a.ended = true;
-  CHECK(g.enter(&b, ended));
-  bool other = true;                                     // another thread, while b's pass is being enqueued: refused, at once
-  std::thread([&] { other = g.enter(&a, ended); g.leave(&a, mark); }).join();
+  CHECK(in(c, 3));                                       // (b's were waited for)
+  bool other = true;                                     // another thread, while c's pass is being enqueued: refused, at once
+  std::thread([&] { other = in(a, 2); out(a); }).join();
   CHECK(!other);
-  g.leave(&b, mark);
-  b.ended = a.ended = true;
-  CHECK(g.enter(&b, ended)); g.leave(&b, broken);        // nothing tells when this one has ended
-  CHECK(!g.enter(&a, ended)); g.leave(&a, mark);
+  out(c);
+  CHECK(in(a, 3)); out(a);                               // behind c's, on its stream
+  a.ended = c.ended = true;
+  CHECK(in(b, 1)); g.leave(&b, broken);                  // nothing tells when this one has ended
+  CHECK(!g.enter(&a, lane(2), &a, ended, cannot)); out(a);
   a.ended = true;
-  CHECK(g.enter(&b, ended)); g.leave(&b, mark);          // until the next one
-  b.ended = true;
-  CHECK(g.enter(&a, ended)); g.leave(&a, broken);
-  g.forget(&a);                                          // or its context goes
-  CHECK(g.enter(&b, ended)); g.leave(&b, mark);
-  g.join(&c, &c, [&] { return false; });                 // the GPU cannot be waited for: b's pass counts as on its way
-  CHECK(!g.enter(&c, ended)); g.leave(&c, mark);
+  CHECK(in(c, 3) && settles == 2); out(c);               // but the GPU can be waited for
+  c.ended = true;
+  CHECK(in(b, 1)); g.leave(&b, broken);
+  g.forget(&b);                                          // or its context goes
+  CHECK(g.enter(&a, lane(2), &a, ended, cannot)); out(a);
+  g.forget(&c);
+  CHECK(g.enter(&a, lane(1), &a, ended, cannot));
+  a.ended = true; out(a);
+  CHECK(a.ended);                                        // alone again: no event
   return 0;
 }
 
-// A context comes while another's pass is being enqueued: that pass gets an event.
-static int joined_in_between() {
-  IxtGate g(file);
-  Event a, b;
-  auto never = [] { return false; };
-  g.join(&a, &a, never);
-  CHECK(g.enter(&a, ended));
-  g.join(&b, &b, [&] { g.leave(&a, mark); return true; });   // (enqueued while the other waits for the GPU: not covered by that wait)
-  CHECK(!a.ended && !g.enter(&b, ended));
-  return 0;
-}
-
-// contexts on threads of their own; a pass stays on the "GPU" for a while after it was enqueued
+// contexts on threads and streams of their own; a pass stays on the "GPU" for a while after it was enqueued
 static int apart() {
   IxtGate g(file);
   std::atomic<long> until[4], waiting[4];                // ends of the last pass, and of the last one with blocks that wait
   std::atomic<int> running{-1}, bad{0}, in{0};
   auto now = [] { return (long)std::chrono::steady_clock::now().time_since_epoch().count(); };
   auto over = [&](void* e) { return now() >= *static_cast<std::atomic<long>*>(e); };
-  for (int k = 0; k < 4; ++k) { until[k] = waiting[k] = 0; g.join(&until[k], &until[k], [] { return true; }); }
+  auto all_over = [&] { for (auto& u : until) while (now() < u) {} return true; };
+  for (int k = 0; k < 4; ++k) until[k] = waiting[k] = 0;
   std::vector<std::thread> ts;
   for (int k = 0; k < 4; ++k)
     ts.emplace_back([&, k] {
       for (int i = 0; i < 3000; ++i) {
-        const bool may = g.enter(&until[k], over);
+        const bool may = g.enter(&until[k], lane(k), &until[k], over, all_over);
         if (may) {
           const int before = running.exchange(k);
           if (before >= 0 && before != k && now() < waiting[before]) ++bad;
           ++in;
         }
-        g.leave(&until[k], [&](void*) {
-          until[k] = std::max(until[k].load(), now()) + (may ? 20000 : 2000);      // (behind its pass before)
-          if (may) waiting[k] = until[k].load();
-          return true;
-        });
+        until[k] = std::max(until[k].load(), now()) + (may ? 20000 : 2000);      // (behind its pass before)
+        if (may) waiting[k] = until[k].load();
+        g.leave(&until[k], [&](void*) { return i % 16 != 15; });
         if (i % 4 == k) std::this_thread::sleep_for(std::chrono::microseconds(30));
       }
     });
@@ -108,11 +101,10 @@ static int apart() {
 // argv: file, and "hold" to keep the lock until a line comes in, or "ask": may a pass take the waiting forms?
 int main(int argc, char** argv) {
   file = argv[1];
-  if (argc == 2) return rules() || joined_in_between() || apart();
+  if (argc == 2) return rules() || apart();
   IxtGate g(file);
   Event a;
-  auto ask = [&] { const bool may = g.enter(&a, ended); g.leave(&a, mark); return may; };
-  g.join(&a, &a, [] { return true; });
+  auto ask = [&] { const bool may = g.enter(&a, lane(1), &a, ended, settle); g.leave(&a, mark); return may; };
   std::printf("%d\n", (int)ask());
   std::fflush(stdout);
   if (argv[2][0] == 'h') {

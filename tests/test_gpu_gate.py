@@ -28,9 +28,9 @@ class Run:
   """One engine with its prompts prefilled and inserted, on a stream of its own."""
   alive = []
 
-  def __init__(self, shape, seed, steps, **keys):
+  def __init__(self, shape, seed, steps, stream=None, **keys):
     import torch
-    self.torch, self.stream, self.tokens = torch, torch.cuda.Stream(), []
+    self.torch, self.stream, self.tokens = torch, stream or torch.cuda.Stream(), []
     self.cfg = _config(*shape, 12 + steps, 2, **keys)
     self.eng, self.params = H.make_engine(self.cfg, H.synth.synth_weights(self.cfg, seed))
     Run.alive.append(self.eng)
@@ -80,6 +80,21 @@ def test_a_pass_beside_another():
   for r, n, tokens in zip((a, b), (63, 62), got):
     r.begin()
     for _ in range(n):
+      r.step()
+      r.stream.synchronize()
+    assert np.array_equal(tokens, r.result())
+
+
+def test_engines_on_one_stream():
+  """Passes of one stream run one after the other: all with waits, however many are on their way."""
+  a = Run(FEW, 1, 130)
+  b = Run(SOME, 2, 130, stream=a.stream)
+  for _ in range(40):
+    assert a.step() == STEP and b.step() == MID
+  got = [a.result(), b.result()]
+  for r, tokens in zip((a, b), got):
+    r.begin()
+    for _ in range(40):
       r.step()
       r.stream.synchronize()
     assert np.array_equal(tokens, r.result())
