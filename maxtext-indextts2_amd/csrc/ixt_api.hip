@@ -1982,7 +1982,8 @@ class WaitPass {
     if (!quietly(hipStreamIsCapturing(st, &cap)) || cap != hipStreamCaptureStatusNone) return;
     in_ = true;
     const IxtGate::Lane lane(st, st == hipStreamPerThread ? std::this_thread::get_id() : std::thread::id());
-    c->may_wait = c->gate->enter(c, lane, c->pass_event, [](void* event) { return quietly(hipEventQuery((hipEvent_t)event)); }, [] { return quietly(hipDeviceSynchronize()); });
+    c->may_wait = c->gate->enter(c, lane, c->pass_event, [](void* event) { return Relaxed(), quietly(hipEventQuery((hipEvent_t)event)); },
+                                 [] { return Relaxed(), quietly(hipDeviceSynchronize()); });
   }
   ~WaitPass() {
     if (!in_) return;
@@ -1992,6 +1993,12 @@ class WaitPass {
   WaitPass(const WaitPass&) = delete;
 
  private:
+  // a question to the GPU is no part of a capture that another thread has under way, and must not end it
+  struct Relaxed {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    Relaxed() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+    ~Relaxed() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  };
   static bool quietly(hipError_t e) {            // (no error of the calls behind it)
     if (e != hipSuccess) (void)hipGetLastError();
     return e == hipSuccess;

@@ -179,6 +179,45 @@ def test_a_stream_that_the_caller_captures(shape):
   assert np.array_equal(torch.stack(got).cpu().numpy(), want)
 
 
+def test_beside_a_capture_of_another_thread():
+  """Looking whether another engine's passes have ended does not end a capture that another thread has under way."""
+  import torch
+  a, b, c = Run(FEW, 1, 40), Run(FEW, 2, 40), Run(SOME, 3, 40)
+  alone = []
+  for r in (a, b, c):
+    for _ in range(24):
+      r.step()
+    alone.append(r.result())
+    r.begin()
+  x, graph, errors = torch.zeros(64, device="cuda"), torch.cuda.CUDAGraph(), []
+
+  def work():
+    try:
+      for _ in range(8):
+        for r in (a, a, b, b, c, c, c):
+          r.step()
+      for r, n in ((a, 8), (b, 8)):
+        for _ in range(n):
+          r.step()
+    except Exception as e:  # pylint: disable=broad-except
+      errors.append(e)
+
+  x.add_(0.0)
+  torch.cuda.synchronize()
+  with torch.cuda.graph(graph):
+    x.add_(1.0)
+    t = threading.Thread(target=work)
+    t.start()
+    t.join(60)
+    x.add_(1.0)
+  assert not errors and not t.is_alive()
+  for _ in range(3):
+    graph.replay()
+  for r, want in zip((a, b, c), alone):
+    assert np.array_equal(r.result(), want)
+  assert x.cpu().tolist() == [6.0] * 64
+
+
 HOLD = """
 import fcntl, os, sys
 fd = os.open(sys.argv[1], os.O_RDWR | os.O_CREAT, 0o666)
