@@ -115,6 +115,7 @@ __device__ __forceinline__ void ring_wait_chunks(int younger) {
 // registers, takes the sum so far from the part before it, wave by wave, adds its own in order and hands it on; the last one stores it.  Progress: a part waits for a block of lower
 // index on the same XCD (gridDim.x is a multiple of 8), which has started before it; the waits are bounded all the same.  For few tiles of a long K: 256 x 2304 outputs, K 9216, 41 us in
 // one part (144 tiles of 64 x 64 for 256 CUs), 35 in three equal ones (72 of 128 x 64), 31 with a chain more for each later part.
+// RING_KEEP holds up to 18 chains, the longest that was measured (163 of 256 registers); a sum of more goes to one block a tile.
 #define RING_KEEP 7
 #define RING_LEFT 2              // a flag whose taker gave up: its setter clears it, so that the next launch finds zeros whatever happened
 //   grid = (8 ceil(ncolg / 8) zb, SPLIT 1 ? chains : SPLIT 2 ? parts : 1), block 64 WR WC, dynamic LDS = NS (WC CT + WR RB) KS KiB.

@@ -10,7 +10,7 @@
 // The norms are phases of their own, a wave a row: every block norming all rows, as k_step does for up to 16, would cost 8 us at 64.
 //
 // Measured, 1B model, ms a pass, a launch a phase -> this: decode steps (32 a pass, 300 keys) of 17 slots 43.5 -> 36.3, 32 slots 46.3 -> 38.8, 33 slots 45.8 -> 41.4, 64 slots 52.6 ->
-// 49.1; a prompt of 17 tokens 1.24 -> 1.05, of 57 1.34 -> 1.28.  A launch of 48 rows takes 43 us: output projection 12 (the weights of all phases are on their way beside it), norms 4 each, units 7,
+// 49.1; a prompt of 17 tokens 1.24 -> 1.05, of 57 1.35 -> 1.25.  A launch of 48 rows takes 43 us: output projection 12 (the weights of all phases are on their way beside it), norms 4 each, units 7,
 // down projection 10, QKV 6; 20 us of weights lie beside them.  What took it there from 59: whole lines from the norms, the down projection's weights in the L2s ahead of time and
 // its row groups in two blocks (3 us), angles ahead of the wait, QKV over twice the blocks (2 us; the CUs are free for its weights only when the down projection ends).  Tried
 // without gain: QKV's weights pulled into the L2s by waves of the down projection that have no unit (+8 us: their block ends later), the pull of the down projection's weights held back until the output projection

@@ -73,8 +73,11 @@ static MidPlan mid_plan(const ixt_ctx* c, int R) {
   return p;
 }
 static bool step_model(const ixt_ctx* c) { return !c->moe && !c->gemma && !c->fp8 && c->L >= 1; }
-// Four row groups only where the weights of a layer are worth the phases' ends: ms a pass of 32 steps, a launch a phase / k_mid, 64 slots of the 1B model (121 MB a layer) 52.6 / 49.1, of the
-// 134M model (14 MB) 22.5 / 22.9; 33 of it 18.4 / 17.6, 20 19.3 / 16.2
+// Four row groups only where the weights of a layer are worth the phases' ends.  ms a step, a launch a phase / k_mid, eight layers of so many MB each (heads of 64 or 128, 60 to 270 keys):
+//            14             29             45             63             116
+//   48 rows  0.400 / 0.382  0.436 / 0.409  0.480 / 0.451  0.516 / 0.472  0.600 / 0.532
+//   49       0.406 / 0.411  0.437 / 0.442  0.485 / 0.486  0.520 / 0.500  0.614 / 0.571
+//   64       0.412 / 0.416  0.441 / 0.445  0.492 / 0.496  0.534 / 0.515  0.641 / 0.593
 bool mid_fits(const ixt_ctx* c, int R) {
   const size_t layer = ((size_t)c->E * (c->NQKV + 2 * c->F) + (size_t)(c->QN + c->F) * c->E) * sizeof(bf16_t);
   return c->mid_ws != nullptr && R >= 17 && R <= std::min(layer >= (size_t)48 << 20 ? 64 : 48, c->mid_rows) && mid_plan(c, R).ok;

@@ -57,6 +57,9 @@ __device__ __forceinline__ void ixt_k_operands(const u32x4& w, uint32_t sel, flo
 // of the transpose.  Tried without gain: the keys of the next super-block requested ahead, page numbers in a register, a priority for half of the waves;
 // 4-byte loads of the keys that need no lane swaps (2.3 x slower).  Keys and values widened to f32 by a launch ahead take another 15 % off here and cost 11 to 22 us for 1024 to
 // 3900 keys: level up to 2048.
+// What the bound of two or three blocks a CU leaves no register for goes through scratch.  Registers spilled, heads of 128: <2, 1> 31 to 39, <4, 1> 16 to 30, <8, 3> 19 to 29, <8, 4> 75 to 89; heads of
+// 256: 31 to 42, 20 to 32, 26 to 37, 82 to 86; heads of 64: <8, 4> 47 to 55, <2, 1> up to 6; the other forms none.  Scratch's loads and stores stand in the counter of the fetches, too; what they cost is not
+// measured.
 // Measured against k_attn_tile, 16 heads of 128, 1024 rows at <= 1024 / 2048 / 3072 keys 282 / 860 / 1143 us; before the instructions above and the forms
 // <4, 2> and <8, 3>: 112 / 215 / 351, now 88 / 195 / 302.  828 rows at <= 3900 keys 1496, 448, 411 us (57 TFLOP/s).  8 heads of 256 on 4, 256 rows at <= 3000 keys: 151 -> 130 us.
 // 8 packed prompts (1525 rows, <= 251 keys) 128.6, 68.8, 67.6: two waves per block for <= 256 keys, with four, two of them had nothing to do (90.2 us).
