@@ -101,9 +101,9 @@ static DeviceGate* device_gate() {
   int dev = 0;
   char bus[64] = "";
   if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetPCIBusId(bus, sizeof(bus), dev) != hipSuccess) return nullptr;
-  const std::string file = std::string("/tmp/libixt-gpu-") + bus + ".lock";
+  const std::string file = std::string("/libixt-gpu-") + bus + ".lock";
   std::lock_guard<std::mutex> lk(mu);
-  return &gates.try_emplace(file, file).first->second;
+  return &gates.try_emplace(file, std::vector<std::string>{"/tmp" + file, "/dev/shm" + file}).first->second;
 }
 
 static int sdot_set_attributes();

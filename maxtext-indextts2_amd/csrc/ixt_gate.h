@@ -8,7 +8,7 @@
 // a step of both, 1 + 1 / 8 + 8 / 48 + 48 / 1 + 48 slots: a turn for the waiting forms 1.24 / 1.55 / 2.79 / 2.05, one pass with them and the other without 1.44 / 1.78 / 2.64 / 2.13, both without 1.32 / 1.60 / 2.42 / 2.04.
 //
 // Between processes a record lock on a file per GPU does the same, for as long as a process has contexts whose passes asked for these forms; the others' passes take the forms without waits.
-// Processes that do not see each other's /tmp are not told apart: there the waits' bounds end them, and the caller gets an error.
+// Processes that do not see each other's file are not told apart: there the waits' bounds end them, and the caller gets an error.
 //
 // Host code of its own: no GPU header.
 #pragma once
@@ -22,11 +22,13 @@
 #include <string>
 #include <thread>
 #include <utility>
+#include <vector>
 
 class IxtGate {
  public:
   using Lane = std::pair<const void*, std::thread::id>;      // a stream; the thread where the handle means another stream in each
-  explicit IxtGate(std::string lock_file = "") : file_(std::move(lock_file)) {}
+  // the first of the files that can be opened counts; none: no pass takes the forms that wait
+  explicit IxtGate(std::vector<std::string> lock_files) : files_(std::move(lock_files)) {}
   // A pass of `who` (the caller orders those of one context) is about to be enqueued on stream `lane`: may it take the forms that wait?  leave() follows in either case.
   // event: the context's own, for leave() to record; ended: has all in front of its last record ended?  settle: waits for the GPU; for passes without an event behind them.
   template <typename Ended, typename Settle>
@@ -70,26 +72,28 @@ class IxtGate {
   };
   // the file's lock.  A record lock: a child of fork() has no part in it, and cannot keep it.
   bool claim() {
-    if (fd_ >= 0) return true;
-    int fd = open(file_.c_str(), O_RDWR | O_CLOEXEC | O_NOFOLLOW);
-    if (fd < 0 && errno == ENOENT) {
-      fd = open(file_.c_str(), O_RDWR | O_CLOEXEC | O_NOFOLLOW | O_CREAT, 0666);
-      if (fd >= 0) (void)fchmod(fd, 0666);       // for the processes of other users
+    for (size_t i = 0; i < files_.size() && fd_ < 0; ++i) {
+      int fd = open(files_[i].c_str(), O_RDWR | O_CLOEXEC | O_NOFOLLOW);
+      if (fd < 0 && errno == ENOENT) {
+        fd = open(files_[i].c_str(), O_RDWR | O_CLOEXEC | O_NOFOLLOW | O_CREAT, 0666);
+        if (fd >= 0) (void)fchmod(fd, 0666);     // for the processes of other users
+      }
+      if (fd < 0) continue;
+      struct flock whole = {};
+      whole.l_type = F_WRLCK;
+      whole.l_whence = SEEK_SET;
+      if (fcntl(fd, F_SETLK, &whole) != 0) {
+        (void)close(fd);
+        return false;
+      }
+      fd_ = fd;
     }
-    struct flock whole = {};
-    whole.l_type = F_WRLCK;
-    whole.l_whence = SEEK_SET;
-    if (fd >= 0 && fcntl(fd, F_SETLK, &whole) != 0) {
-      (void)close(fd);
-      fd = -1;
-    }
-    fd_ = fd;
     return fd_ >= 0;
   }
 
   std::mutex mu_;
   std::map<const void*, User> users_;            // contexts whose passes asked
   bool lanes_ = false;           // on different streams
-  const std::string file_;
+  const std::vector<std::string> files_;
   int fd_ = -1;
 };

@@ -17,6 +17,8 @@ PROGRAM = r"""
 #include <atomic>
 #include <chrono>
 #include <cstdio>
+#include <sstream>
+#include <string>
 #include <thread>
 #include <vector>
 #define CHECK(x) do { if (!(x)) { std::printf("line %d: %s\n", __LINE__, #x); return 1; } } while (0)
@@ -26,7 +28,7 @@ static auto ended = [](void* e) { return static_cast<Event*>(e)->ended; };
 static auto mark = [](void* e) { static_cast<Event*>(e)->ended = false; return true; };
 static auto broken = [](void*) { return false; };
 
-static const char* file;
+static std::vector<std::string> files;
 
 static IxtGate::Lane lane(long n) { return IxtGate::Lane(reinterpret_cast<void*>(n), std::thread::id()); }
 static int settles = 0;
@@ -34,7 +36,7 @@ static auto settle = [] { ++settles; return true; };
 static auto cannot = [] { return false; };
 
 static int rules() {
-  IxtGate g(file);
+  IxtGate g(files);
   Event a, b, c;
   auto in = [&](Event& e, long n) { return g.enter(&e, lane(n), &e, ended, settle); };
   auto out = [&](Event& e) { g.leave(&e, mark); };
@@ -71,7 +73,7 @@ static int rules() {
 
 // contexts on threads and streams of their own; a pass stays on the "GPU" for a while after it was enqueued
 static int apart() {
-  IxtGate g(file);
+  IxtGate g(files);
   std::atomic<long> until[4], waiting[4];                // ends of the last pass, and of the last one with blocks that wait
   std::atomic<int> running{-1}, bad{0}, in{0};
   auto now = [] { return (long)std::chrono::steady_clock::now().time_since_epoch().count(); };
@@ -98,11 +100,12 @@ static int apart() {
   CHECK(bad == 0 && in > 0);
   return 0;
 }
-// argv: file, and "hold" to keep the lock until a line comes in, or "ask": may a pass take the waiting forms?
+// argv: files (a colon between them), and "hold" to keep the lock until a line comes in, or "ask": may a pass take the waiting forms?
 int main(int argc, char** argv) {
-  file = argv[1];
+  std::stringstream names(argv[1]);
+  for (std::string n; std::getline(names, n, ':');) files.push_back(n);
   if (argc == 2) return rules() || apart();
-  IxtGate g(file);
+  IxtGate g(files);
   Event a;
   auto ask = [&] { const bool may = g.enter(&a, lane(1), &a, ended, settle); g.leave(&a, mark); return may; };
   std::printf("%d\n", (int)ask());
@@ -172,5 +175,6 @@ def test_a_process_that_dies_lets_go(program, tmp_path):
 def test_no_file_no_waits(program, tmp_path):
   """Where the lock cannot be taken at all, or the file is somebody's link, a pass takes the forms without waits."""
   assert _ask(program, str(tmp_path / "none" / "lock")) == "0"
+  assert _ask(program, f"{tmp_path}/none/lock:{tmp_path}/second") == "1" and os.path.exists(tmp_path / "second") and not os.path.exists(tmp_path / "none")
   os.symlink(tmp_path / "target", tmp_path / "link")
   assert _ask(program, str(tmp_path / "link")) == "0"
