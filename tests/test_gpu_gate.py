@@ -44,6 +44,12 @@ class Run:
         self.state = self.eng.insert(prefix, self.state, slot)
     self.torch.cuda.synchronize()
 
+  def hold(self):
+    """Something in front of the next steps, so that they are still on their way when others are asked for."""
+    with self.torch.cuda.stream(self.stream):
+      self.torch.cuda._sleep(20_000_000)
+    return self
+
   def step(self):
     with self.torch.cuda.stream(self.stream):
       self.state, result = self.eng.generate(self.params, self.state)
@@ -68,12 +74,14 @@ def closed():
 def test_a_pass_beside_another():
   """While passes of another engine are on their way an engine takes the forms without waits; behind them, and alone, those with."""
   a, b = Run(FEW, 1, 130), Run(SOME, 2, 130)
+  a.hold()
   assert [a.step() for _ in range(60)] == [STEP] * 60
-  assert b.step() == 0 and a.step() == 0
+  assert b.hold().step() == 0 and a.step() == 0
   a.result()
   b.result()
+  b.hold()
   assert [b.step() for _ in range(60)] == [MID] * 60
-  assert a.step() == 0 and b.step() == 0
+  assert a.hold().step() == 0 and b.step() == 0
   b.result()
   assert a.step() == STEP
   got = [a.result(), b.result()]
@@ -137,8 +145,8 @@ def test_split_attention_beside_whole_steps(beside):
     assert [r.step() for _ in range(60)] == [form] * 60
     alone.append(r.result())
     r.begin()
-  seen = set()
-  for _ in range(60):
+  seen = {split.hold().step(), other.hold().step()}
+  for _ in range(59):
     seen |= {split.step(), other.step()}
   assert 0 in seen
   for r, want in zip((split, other), alone):
