@@ -468,7 +468,7 @@ def roofline(args, wl, eng, cfg, nums, prompts, B):
   build_id = lib.ixt_build_id().decode()
   traffic, traffic_src, mfma, stale = None, None, None, None
   import glob
-  for pmc in sorted(glob.glob(os.path.join(ROOT, "profiles", "*pmc*.json")), reverse=True):      # newest round first
+  for pmc in sorted(glob.glob(os.path.join(ROOT, "profiles", "*pmc*.json")), reverse=True):
     try:
       pj = json.load(open(pmc))
     except Exception:  # pylint: disable=broad-except
