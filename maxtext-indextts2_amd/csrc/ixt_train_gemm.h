@@ -2,12 +2,18 @@
 // contiguous one, f32 accumulation.
 //
 // Block = (16 MI WM) x (16 NI WN), waves WM x WN, 32 k at a time through a ring of NS LDS slots filled by LDS-DMA; a wave's tile is 16 MI x 16 NI.
-// What bounds it: LDS reads against matrix cores.  Per 32 k a wave reads MI + NI KiB and issues MI NI products of 16 cycles; eight waves of 128 x 64
-// read 96 KiB (768 cycles of the LDS) under 1024 cycles of products, four of 64 x 64 32 KiB (256) under 256: hence the 256 x 256 block wherever
-// its tiles fill the chip.  With few tiles a wave is alone on its SIMD and bound by its own instructions: smaller tiles, more waves (gemm_launch has
-// the rule).  The next 32 k are read from LDS and fetched from memory between the rows of products, not in front of them.
-// Measured (bf16): 16384 x 2048 x 7168 1.06 PFLOP/s, its input gradient 1.12, its weight gradient 1.13, 8192^3 1.24 (0.45 - 0.53 with 128 x 128 x 64
-// tiles staged through registers; torch's product of 8192^3 1.37 on this card); without the fetches 1.4 - 1.7.
+// What bounds it: the matrix units at the clock that the card's power leaves them.  Random operands, 256 x 256 blocks: 1068 cycles of products per 32 k, 1136 with the
+// LDS reads and the fetches beside them and nothing else (1.55 PFLOP/s at 1.64 GHz), 1340 to 1450 here at 1.5 to 1.8 GHz.  Per 32 k a wave reads MI + NI KiB for MI NI products of
+// 16 cycles, which is why the largest block is taken wherever its tiles fill the chip.  With few tiles a wave is alone on its SIMD and bound by its own instructions: smaller tiles,
+// more waves (gemm_launch has the rule).  So what counts is what stands between the products:
+//   the next 32 k are read from LDS and fetched from memory between the rows of products, not in front of them;
+//   the steps that fetch whole chunks are a loop of their own without a branch (a branch a fetch: 1515 cycles instead of 1400);
+//   the block's barrier stands behind a step's first products, which cover the last reads and the waves' skew (2 to 4 % of long reductions);
+//   a row of 32 k is half a line of 128 bytes: where an operand's k is contiguous (PAIR), both halves are fetched one behind the other, every second step, so that the second comes
+//   from the L1 (fetches alone 593 cycles per 32 KiB, 1110 with the halves a step apart; five slots instead of four).
+// Measured (us, with a launch's start and end), before these three and the stores of 16 bytes / now: 4096 x 4096, K 8192, k contiguous 232 / 205, of one operand 243 / 229, by columns 231 / 216;
+// 16384 x 8192, K 2048 531 / 477; 128 x 128 blocks, 4096 x 2048, K 4096 86 / 68; 64 x 64, 2048 x 768, K 4096 31.8 / 26.8.  Sums onto an f32 C (256 x 256 tiles): 20 us of a tile's 80
+// are its 512 KiB, all CUs at once, at 6.5 TB/s.
 //   k contiguous:   slot image [row][32 k], four 16-byte pieces a row, piece c of row r at c ^ ((r >> 2) & 3): the 16 rows a half wave reads lie on
 //                   disjoint banks
 //   row contiguous: slot image [k][row], 32-byte pieces, piece u of row k at u ^ (k & 7) (64 rows: u ^ (k / 2 & 3)); ds_read_tr16 hands a 4 x 16 block to 16 lanes column-wise, so
@@ -22,6 +28,8 @@
 // another in the block and join a second set of accumulators, in the same order: no partial C in memory, no kernel that adds them, one launch.
 #pragma once
 #include "ixt_device.h"
+
+#include <type_traits>
 
 typedef float tf32x4 __attribute__((ext_vector_type(4)));
 typedef short tbf16x8 __attribute__((ext_vector_type(8)));
@@ -51,10 +59,11 @@ static __device__ const uint32_t tg_zero[4] = {0u, 0u, 0u, 0u};
 
 template <bool TA, bool TB, int MI, int NI, int WM, int WN, int NS, bool FOLD = false>
 __global__ __launch_bounds__(WM * WN * 64, 2) void k_tgemm(TGemm g) {
+  constexpr bool PAIR = !TA || !TB;
   constexpr int BM = 16 * MI * WM, BN = 16 * NI * WN, NW = WM * WN;
   constexpr int NA = BM / 16, NB = BN / 16, NJ = (NA + NB) / NW;          // KiB of a chunk; a wave fetches NJ of them
   constexpr int SLOT = (BM + BN) * 32;                                    // elements
-  static_assert(NA % NW == 0 && NB % NW == 0, "a fetch is of one operand");
+  static_assert(NA % NW == 0 && NB % NW == 0 && NS == (PAIR ? 5 : 4), "a fetch is of one operand; pairs: two chunks being read, three ahead");
   extern __shared__ __attribute__((aligned(16))) bf16_t lds[];            // [NS][A image | B image]
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, r16 = lane & 15, q = lane >> 4;
   const int wm = wave / WN, wn = wave % WN;
@@ -108,26 +117,24 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void k_tgemm(TGemm g) {
     }
   }
   const int chunks1 = (segend - segk + 31) >> 5, chunks = FOLD ? g.nsum * chunks1 : chunks1;
+  const int whole = !FOLD ? (segend - segk) >> 5 : (segend & 31) == 0 ? chunks : 0;      // chunks from the first on that end within K
   int sum = 0;                                                            // FOLD: the product that is fetched
-  bool whole = false;
-  auto next_chunk = [&]() {                                               // past the last chunk: zeros, so that the counts stay
-    whole = segk + 32 <= segend;
-  };
   const uint32_t lds0 = (uint32_t)(uintptr_t)((__attribute__((address_space(3))) bf16_t*)lds);
-  auto issue = [&](int slot, int j) {                                     // piece j of this wave's share of the next chunk; the waits are counted in the loop
+  struct Chunk { const char *a, *b; int k; };                             // a chunk to fetch: its first row of either operand, its first k
+  // piece j of this wave's share; the waits are counted in the loop.  A chunk that reaches past the last k fetches zeros there (edge), so that the counts stay
+  auto issue = [&](int slot, int j, const Chunk& c, auto edge) {
     const bool isa = j * NW < NA;
     const uint32_t dst = __builtin_amdgcn_readfirstlane(lds0 + (uint32_t)(slot * SLOT + (wave + NW * j) * 512) * 2u);
-    if (whole) {
-      lds_dma16(dst, isa ? pa : pb, off[j]);
+    if constexpr (!edge.value) {
+      lds_dma16(dst, isa ? c.a : c.b, off[j]);
     } else {
-      const char* p = (isa ? pa : pb) + off[j];
       int k, x;
       place(isa ? TA : TB, isa ? BM : BN, isa ? wave + NW * j : wave + NW * j - NA, k, x);
-      if (segk + k >= segend) p = reinterpret_cast<const char*>(tg_zero);
-      lds_dma16(dst, p);
+      lds_dma16(dst, c.k + k >= segend ? reinterpret_cast<const char*>(tg_zero) : (isa ? c.a : c.b) + off[j]);
     }
   };
-  auto advance = [&]() {
+  auto next_chunk = [&]() -> Chunk {
+    const Chunk c{pa, pb, segk};
     segk += 32; pa += adva; pb += advb;
     if constexpr (FOLD) {
       if (segk >= segend && sum + 1 < g.nsum) {
@@ -137,6 +144,7 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void k_tgemm(TGemm g) {
         pb = reinterpret_cast<const char*>(g.B[sum] + (TB ? (long)n0 : (long)n0 * g.ldb[0]));
       }
     }
+    return c;
   };
   const int trf = (r16 >> 2) | (q & 1) << 2;                              // k & 7 of the lane's row in a transposed read: 4 q + r16 / 4
   auto operand = [&](const bf16_t* img, int x, int bx, bool tr) -> tbf16x8 {
@@ -163,41 +171,64 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void k_tgemm(TGemm g) {
 #pragma unroll
     for (int j = 0; j < NI; ++j) acc[i][j] = tf32x4(0.0f);
   tbf16x8 fa[MI], fb[2][NI];
+  if constexpr (PAIR) {
 #pragma unroll
-  for (int c = 0; c < NS; ++c) {
-    next_chunk();
+    for (int c = 0; c < 4; c += 2) {
+      const Chunk lo = next_chunk(), hi = next_chunk();
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) issue(c, j);
-    advance();
+      for (int j = 0; j < NJ; ++j) { issue(c, j, lo, std::true_type()); issue(c + 1, j, hi, std::true_type()); }
+    }
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * NJ) : "memory");
+  } else {
+#pragma unroll
+    for (int c = 0; c < NS; ++c) {
+      const Chunk lo = next_chunk();
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) issue(c, j, lo, std::true_type());
+    }
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 1) * NJ) : "memory");
   }
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 1) * NJ) : "memory");
   lds_barrier();
 #pragma unroll
   for (int j = 0; j < NI; ++j) fb[0][j] = row_b(0, j);
 #pragma unroll
   for (int i = 0; i < MI; ++i) fa[i] = row_a(0, i);
-  auto step = [&](int c, int cur) {
-    // chunk c + 1 has landed once the (NS - 2) younger ones are all that is outstanding; this wave's reads of chunk c are done, so behind the
-    // barrier its slot can be filled again
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((NS - 2) * NJ) : "memory");
-    lds_barrier();
-    next_chunk();
-    const int nxt = (c + 1) % NS, old = c % NS;
-    // a row of products, then a share of the reads of chunk c + 1 and of the fetches of chunk c + NS: they ride under the products
+  int slot = 0;                                                           // of chunk c
+  auto step = [&](auto cur_, auto edge) {
+    constexpr int cur = cur_.value;
+    const int old = slot, older = slot == 0 ? NS - 1 : slot - 1, nxt = slot + 1 == NS ? 0 : slot + 1;
+    slot = nxt;
+    constexpr bool fetch = !PAIR || cur == 0;
+    Chunk lo{}, hi{};
+    if constexpr (fetch) lo = next_chunk();
+    if constexpr (PAIR && fetch) hi = next_chunk();
+    // a row of products, then a share of the reads of chunk c + 1 and of the fetches (of chunk c + NS; PAIR: for an even c, of chunks c + 4 and c + 5): they ride
+    // under the products
 #pragma unroll
     for (int i = 0; i < MI; ++i) {
 #pragma unroll
       for (int j = 0; j < NI; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[cur][j], fa[i], acc[i][j], 0, 0, 0);
+      if (i == 0) {
+        // chunk c + 1 has landed once those behind it (PAIR: the pair behind its own) are all that is outstanding; this wave's reads of chunk c are done, so
+        // behind the barrier its slot can be filled again.  Behind the first products: they cover the last reads and the waves' skew
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(PAIR ? 2 * NJ : (NS - 2) * NJ) : "memory");
+        lds_barrier();
+      }
       fa[i] = row_a(nxt, i);
 #pragma unroll
       for (int j = 0; j < NI; ++j)
         if (j * MI / NI == i) fb[cur ^ 1][j] = row_b(nxt, j);
+      if constexpr (fetch) {
 #pragma unroll
-      for (int j = 0; j < NJ; ++j)
-        if (j * MI / NJ == i) issue(old, j);
+        for (int j = 0; j < NJ; ++j)
+          if (j * MI / NJ == i) {
+            issue(PAIR ? older : old, j, lo, edge);
+            if constexpr (PAIR) issue(old, j, hi, edge);
+          }
+      }
       __builtin_amdgcn_sched_barrier(0);
     }
-    advance();
   };
   tf32x4 tot[FOLD ? MI : 1][FOLD ? NI : 1];
   int next = FOLD && g.fold > 0 ? g.fold : chunks1;
@@ -216,12 +247,18 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void k_tgemm(TGemm g) {
       next += done < chunks1 ? g.fold : chunks1;
     }
   };
-  for (int c = 0; c < chunks; c += 2) {                                   // (an odd count: the last products are with zeros)
-    step(c, 0);
-    fold(c + 1);
-    step(c + 1, 1);
-    fold(c + 2);
-  }
+  int c = 0;
+  auto steps = [&](int end, auto edge) {                                  // (an odd count: the last products are with zeros)
+    for (; c < end; c += 2) {
+      step(std::integral_constant<int, 0>(), edge);
+      fold(c + 1);
+      step(std::integral_constant<int, 1>(), edge);
+      fold(c + 2);
+    }
+  };
+  // steps that fetch whole chunks, without a branch between the products (one a fetch cost 300 cycles of 1500 a step), then the others
+  steps((whole - 4) & ~1, std::false_type());                             // (steps c and c + 1 fetch chunks c + 4 and c + 5)
+  steps(chunks, std::true_type());
   if constexpr (FOLD) {
 #pragma unroll
     for (int i = 0; i < MI; ++i)
@@ -230,42 +267,56 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void k_tgemm(TGemm g) {
   }
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");             // nothing may land in LDS that the next block owns
   // lane: m = r16, n = 4 q + register
-  const int out = g.out, nw = n0 + wn * NI * 16 + q * 4;
+  const int out = g.out, m1 = m0 + wm * MI * 16 + r16, nw = n0 + wn * NI * 16;
+  if (out == TG_F32 || out == TG_F32_ADD) {
+    float* c = reinterpret_cast<float*>(g.C[prob]) + (g.parts > 1 ? part * g.cpart[prob] : zc) + nw + q * 4;
+    constexpr int AHEAD = MI < 4 ? MI : 4;                                // rows of the old sums in flight (one at a time: 20 us a tile of 256 x 256, eight waits)
+    tf32x4 old[AHEAD][NI];
+    auto load = [&](int i) {
 #pragma unroll
-  for (int i = 0; i < MI; ++i) {
-    const int m = m0 + (wm * MI + i) * 16 + r16;
-    if (m >= g.M) continue;
-    const long row = (long)m * g.ldc[prob] + nw;
-    if (out == TG_F32 || out == TG_F32_ADD) {
-      float* c = reinterpret_cast<float*>(g.C[prob]) + (g.parts > 1 ? part * g.cpart[prob] : zc) + row;
+      for (int j = 0; j < NI; ++j)
+        old[i % AHEAD][j] = m1 + i * 16 < g.M && nw + j * 16 + q * 4 < N ? *reinterpret_cast<const tf32x4*>(c + (long)(m1 + i * 16) * g.ldc[prob] + j * 16) : tf32x4(0.0f);
+    };
+    if (out == TG_F32_ADD) {
+#pragma unroll
+      for (int i = 0; i < AHEAD; ++i) load(i);
+    }
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
       if (out == TG_F32_ADD) {
-        tf32x4 old[NI];
 #pragma unroll
-        for (int j = 0; j < NI; ++j) old[j] = nw + j * 16 < N ? *reinterpret_cast<const tf32x4*>(c + j * 16) : tf32x4(0.0f);
-#pragma unroll
-        for (int j = 0; j < NI; ++j) acc[i][j] = old[j] + acc[i][j];
+        for (int j = 0; j < NI; ++j) acc[i][j] = old[i % AHEAD][j] + acc[i][j];
+        if (i + AHEAD < MI) load(i + AHEAD);
       }
 #pragma unroll
       for (int j = 0; j < NI; ++j)
-        if (nw + j * 16 < N) *reinterpret_cast<tf32x4*>(c + j * 16) = acc[i][j];
-    } else {
-      bf16_t* c = reinterpret_cast<bf16_t*>(g.C[prob]) + zc + row;
-      if (out == TG_BF16_RES) {
-        uint2 h[NI];
+        if (m1 + i * 16 < g.M && nw + j * 16 + q * 4 < N) *reinterpret_cast<tf32x4*>(c + (long)(m1 + i * 16) * g.ldc[prob] + j * 16) = acc[i][j];
+    }
+    return;
+  }
+  // bf16: two column tiles at a time; a swap of lane groups leaves every lane eight columns of one of them, 16 bytes to store and 64 side by side (256 x 256:
+  // 4.1 us for stores of 8 bytes)
+  static_assert(NI % 2 == 0, "pairs of column tiles");
+  const int ns = nw + (q & 1) * 16 + (q >> 1) * 8;
 #pragma unroll
-        for (int j = 0; j < NI; ++j) h[j] = nw + j * 16 < N ? *reinterpret_cast<const uint2*>(g.R + row + j * 16) : make_uint2(0u, 0u);
+  for (int i = 0; i < MI; ++i) {
+    const int m = m1 + i * 16;
+    const long row = (long)m * g.ldc[prob];
 #pragma unroll
-        for (int j = 0; j < NI; ++j) {
-          acc[i][j][0] = bflo(h[j].x) + rbf(acc[i][j][0]); acc[i][j][1] = bfhi(h[j].x) + rbf(acc[i][j][1]);
-          acc[i][j][2] = bflo(h[j].y) + rbf(acc[i][j][2]); acc[i][j][3] = bfhi(h[j].y) + rbf(acc[i][j][3]);
+    for (int j = 0; j < NI; j += 2) {
+      uint2 o[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        tf32x4 v = acc[i][j + h];
+        if (out == TG_BF16_RES) {
+          const int n = nw + (j + h) * 16 + q * 4;
+          const uint2 r = m < g.M && n < N ? *reinterpret_cast<const uint2*>(g.R + row + n) : make_uint2(0u, 0u);
+          v[0] = bflo(r.x) + rbf(v[0]); v[1] = bfhi(r.x) + rbf(v[1]); v[2] = bflo(r.y) + rbf(v[2]); v[3] = bfhi(r.y) + rbf(v[3]);
         }
+        o[h].x = pack2(f2bf(v[0]), f2bf(v[1])); o[h].y = pack2(f2bf(v[2]), f2bf(v[3]));
       }
-#pragma unroll
-      for (int j = 0; j < NI; ++j) {
-        uint2 o;
-        o.x = pack2(f2bf(acc[i][j][0]), f2bf(acc[i][j][1])); o.y = pack2(f2bf(acc[i][j][2]), f2bf(acc[i][j][3]));
-        if (nw + j * 16 < N) *reinterpret_cast<uint2*>(c + j * 16) = o;
-      }
+      const auto x = __builtin_amdgcn_permlane16_swap(o[0].x, o[1].x, false, false), y = __builtin_amdgcn_permlane16_swap(o[0].y, o[1].y, false, false);
+      if (m < g.M && ns + j * 16 < N) *reinterpret_cast<uint4*>(reinterpret_cast<bf16_t*>(g.C[prob]) + zc + row + ns + j * 16) = make_uint4(x[0], y[0], x[1], y[1]);
     }
   }
 }
