@@ -13,8 +13,9 @@
 // What bounds it: a 128 x 128 tile fetches as many bytes a chunk as the CU's 64 B a cycle bring in the time of its products (512 cycles of each per 64 k;
 // measured 31 TB/s over the chip from L2), and a fetch that finds the queue full holds its wave and the MFMAs behind it.  256 x 128 tiles need 3/4 of
 // that and win wherever the launch has enough of them: 14336 columns, K 2048, 1525 rows: 122 us (735 TFLOP/s) with 128 x 128 tiles whose chunk was
-// read and then multiplied, 112 with the reads under the products, 102 (881 TFLOP/s) with 256 x 128.  Tried without gain: the fetches of a SIMD's two waves in
-// different halves of a chunk, hot weights, chunk-contiguous operands.
+// read and then multiplied, 112 with the reads under the products, 107 and now 100 with the steps that refill a loop of their own, without a branch, and the barrier behind a
+// step's first products.  256 x 128 tiles take 1250 to 1310 cycles per 64 k of which the products are 1068, at 1.6 to 2.3 GHz: the card's power sets the clock.  Tried without gain: the
+// fetches of a SIMD's two waves in different halves of a chunk, hot weights, chunk-contiguous operands.
 //
 // Epilogues (EPI):
 //   GEPI_F32      f32 [slice][R][N] (op-level entry point, split-K form)
@@ -29,6 +30,7 @@
 //                 head columns are stored pair-interleaved (qk_col): a 16-column tile holds features 8j..8j+7 and half+8j..half+8j+7,
 //                 so the two RoPE partners of a feature sit in lanes l and l ^ 32 of one accumulator register.
 #pragma once
+#include <type_traits>
 
 enum { GEPI_F32 = 0, GEPI_UNEMBED = 1, GEPI_RESID = 2, GEPI_SWIGLU = 3, GEPI_QKV = 4, GEPI_TANHNORM = 5, GEPI_ACT = 6 };
 
@@ -208,18 +210,13 @@ __global__ __launch_bounds__(WR * WC * 64, 2) void k_gemm_ring(const u32x4* __re
   int fill = 0;
   // One k-step: products of the fragments in registers, with the reads of the next step's fragments and the refill of the slot that was read out last dealt
   // between them, so that the matrix cores, the LDS and the fetches run side by side (reading a chunk and then multiplying it took turns: 1 500 cycles a
-  // 64-k chunk of a 128 x 128 tile, of which the products are 512).  Ahead of a chunk's last step its fragments are all in registers and the next chunk has
-  // to be there: one counted wait and one barrier a chunk, behind which its slot is free for chunk ch + NS.
-  auto step = [&](int ch, int ks, int cur) {
-    const bool last = ks == KS - 1;
-    if (last) {
-      ring_wait_chunks<NJ, NS - 2>(che - ch - 2);
-      lds_barrier();
-      refill = ch + NS < che;
-      fill = slot;
-      slot = slot + 1 == NS ? 0 : slot + 1;
-    }
-    const int nks = last ? 0 : ks + 1, from = ks == KS - 1 ? 0 : ks + 1;   // `from`: position of this step among the KS steps of a refill
+  // 64-k chunk of a 128 x 128 tile, of which the products are 512).  Behind the first products of a chunk's last step its fragments are all in registers and the
+  // next chunk has to be there: one counted wait and one barrier a chunk, behind which its slot is free for chunk ch + NS.  STEADY: there is such a chunk, and
+  // there was one in the chunk before; the steps of these are a loop without a branch.
+  auto step = [&](int ch, auto ks_, int cur, auto steady) {
+    constexpr int ks = ks_.value;
+    constexpr bool last = ks == KS - 1;
+    constexpr int nks = last ? 0 : ks + 1, from = nks;                // `from`: position of this step among the KS steps of a refill
 #pragma unroll
     for (int i = 0; i < CT; ++i) {
 #pragma unroll
@@ -233,19 +230,28 @@ __global__ __launch_bounds__(WR * WC * 64, 2) void k_gemm_ring(const u32x4* __re
           acc[i][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[i], xf[cur][b], acc[i][b], 0, 0, 0);
         }
       }
+      if (last && i == 0) {
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (steady.value) ring_wait<(NS - 2) * NJ>();
+        else ring_wait_chunks<NJ, NS - 2>(che - ch - 2);
+        lds_barrier();
+        if constexpr (!steady.value) refill = ch + NS < che;
+        fill = slot;
+        slot = slot + 1 == NS ? 0 : slot + 1;
+      }
       wf[i] = wfrag(slot, nks, i);
 #pragma unroll
       for (int b = 0; b < RB; ++b)
         if (b * CT / RB == i) xf[cur ^ 1][b] = xfrag(slot, nks, b);
       const int gi = from * CT + i;
-      if (refill) {
+      if (steady.value || refill) {
 #pragma unroll
         for (int j = 0; j < NJ; ++j)
           if (j * (KS * CT) / NJ == gi) issue(fill, j);
       }
       __builtin_amdgcn_sched_barrier(0);
     }
-    if (refill && from == KS - 1) advance();
+    if (from == KS - 1 && (steady.value || refill)) advance();
   };
   // a 512-k chain is complete
   auto chain_end = [&](int ch) {
@@ -268,18 +274,32 @@ __global__ __launch_bounds__(WR * WC * 64, 2) void k_gemm_ring(const u32x4* __re
 #pragma unroll
       for (int b = 0; b < RB; ++b) { tot[i][b] = tot[i][b] + acc[i][b]; acc[i][b] = f32x4(0.0f); }
   };
+  auto chunk = [&](int ch, auto steady) {
+    step(ch, std::integral_constant<int, 0>(), 0, steady);
+    if constexpr (KS > 1) step(ch, std::integral_constant<int, 1 % KS>(), 1, steady);
+    if constexpr (KS > 2) { step(ch, std::integral_constant<int, 2 % KS>(), 0, steady); step(ch, std::integral_constant<int, 3 % KS>(), 1, steady); }
+  };
+  static_assert(KS == 1 || KS == 2 || KS == 4, "steps of a chunk");
   if constexpr (KS == 1) {                                      // (an even number of chunks: K is a multiple of 128)
-    for (int ch = chb; ch < che; ch += 2) {
-      step(ch, 0, 0);
-      step(ch + 1, 0, 1);
+    auto two = [&](int ch, auto steady) {
+      step(ch, std::integral_constant<int, 0>(), 0, steady);
+      step(ch + 1, std::integral_constant<int, 0>(), 1, steady);
       if (((ch + 2) % CPC) == 0 || ch + 2 == che) chain_end(ch);
-    }
+    };
+    int ch = chb;
+    for (; ch + 1 + NS < che; ch += 2) two(ch, std::true_type());
+    for (; ch < che; ch += 2) two(ch, std::false_type());
   } else if (SPLIT != 2 || part == 0) {
-    for (int ch = chb; ch < che; ++ch) {
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) step(ch, ks, ks & 1);
+    auto one = [&](int ch, auto steady) {
+      chunk(ch, steady);
       if (((ch + 1) % CPC) == 0 || ch + 1 == che) chain_end(ch);
+    };
+    int ch = chb;
+    one(ch++, std::false_type());
+    if (refill) {                                               // (chunk ch - 1 + NS has begun to come)
+      for (; ch + NS < che; ++ch) one(ch, std::true_type());
     }
+    for (; ch < che; ++ch) one(ch, std::false_type());
   }
   if constexpr (SPLIT == 2) {
     static_assert(EPI == GEPI_F32 && KS > 1 && !F8, "parts of f32 sums");
@@ -287,10 +307,7 @@ __global__ __launch_bounds__(WR * WC * 64, 2) void k_gemm_ring(const u32x4* __re
     if (part > 0) {
 #pragma unroll
       for (int q = 0; q < RING_KEEP; ++q) {
-        for (int ch = chb + q * CPC; ch < min(che, chb + (q + 1) * CPC); ++ch) {
-#pragma unroll
-          for (int ks = 0; ks < KS; ++ks) step(ch, ks, ks & 1);
-        }
+        for (int ch = chb + q * CPC; ch < min(che, chb + (q + 1) * CPC); ++ch) chunk(ch, std::false_type());
 #pragma unroll
         for (int i = 0; i < CT; ++i)
 #pragma unroll
