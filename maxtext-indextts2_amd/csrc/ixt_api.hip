@@ -366,6 +366,8 @@ extern "C" int ixt_create(const ixt_config* cfg, ixt_ctx** out) {
   x->fault_dev = (int32_t*)fault_dev;
   A(dmalloc(x, &x->ring_flags, (size_t)RING_FLAGS));
   if (hipMemset(x->ring_flags, 0, sizeof(int32_t) * RING_FLAGS) != hipSuccess) return fail(set_err(IXT_ERR_HIP, "flags"));
+  A(dmalloc(x, &x->gate_tables, (size_t)IXT_GATE_BYTES));          // (bf16: two tables)
+  hipLaunchKernelGGL(k_gate_tables, dim3((IXT_GATE_BYTES + 255) / 256), dim3(256), 0, 0, x->gate_tables);
   A(dmalloc(x, &x->row_slot, (size_t)R));
   A(dmalloc(x, &x->row_pos, (size_t)R));
   A(dmalloc(x, &x->row_active, (size_t)R));
@@ -781,7 +783,7 @@ template <int WR, int WC, int RB, int CT, int KS, int NS, int EPI, int SPLIT, bo
 static int ring_launch_o(const bf16_t* x, const bf16_t* w, int K, int N, int R, int chains, int wring, const GemmEpi& e, hipStream_t st, int* wave_cols) {
   constexpr int TC = WC * CT, TR = WR * RB;
   const int ncolg = (N / 16 + TC - 1) / TC, zb = (R + 16 * TR - 1) / (16 * TR);
-  constexpr size_t lds = (size_t)NS * (TC + TR) * KS * 1024;
+  constexpr size_t lds = (size_t)NS * (TC + TR) * KS * 1024 + (EPI == GEPI_SWIGLU ? IXT_GATE_BYTES : 0);
   static bool attr_done = false;
   if (!attr_done) {   // more than 64 KiB of dynamic LDS needs the attribute once per kernel
     HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gemm_ring<WR, WC, RB, CT, KS, NS, EPI, SPLIT, false, ONCE>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
@@ -805,9 +807,11 @@ static int ring_launch_t(const bf16_t* x, const bf16_t* w, int K, int N, int R, 
 
 // x in xidx layout, w in widx layout (wring: ring layout); the epilogue's operands in `e`.  split (GEPI_F32 only): one f32 slice per
 // 512-k chain.  wave_cols (GEPI_UNEMBED): entries per row of the (max, index) arrays.
-int launch_ring(ixt_ctx* c, int epi, const bf16_t* x, const bf16_t* w, int K, int N, int R, const GemmEpi& e, bool split, hipStream_t st, int wring,
+int launch_ring(ixt_ctx* c, int epi, const bf16_t* x, const bf16_t* w, int K, int N, int R, const GemmEpi& epilogue, bool split, hipStream_t st, int wring,
                 int* wave_cols) {
   if (K % IXT_KALIGN || N % 16) return set_err(IXT_ERR_UNSUPPORTED, "ring gemm: K %% 128 or N %% 16");
+  GemmEpi e = epilogue;
+  e.gate = c->gate_tables + (e.glu < 0 ? IXT_GATE_BYTES / 2 : 0);
   const int chains = (K + IXT_CHAIN - 1) / IXT_CHAIN;
   const int cfg = ring_pick(c, epi, R, N, e.rb_exp != nullptr, wring != 0);
   if (epi == GEPI_UNEMBED && (size_t)R * ring_pairs(cfg, N) > c->amax_cap) return set_err(IXT_ERR_INVALID, "argmax workspace too small");
@@ -851,6 +855,7 @@ int launch_ring(ixt_ctx* c, int epi, const bf16_t* x, const bf16_t* w, int K, in
   else if (epi == GEPI_RESID) RING(GEPI_RESID)
   else if (epi == GEPI_TANHNORM) RING(GEPI_TANHNORM)
   else if (epi == GEPI_ACT) RING(GEPI_ACT)
+  else if (epi == GEPI_QKV && e.g.rope32) RING(GEPI_QKV32)
   else if (epi == GEPI_QKV) RING(GEPI_QKV)
   else if (epi == GEPI_UNEMBED) RING_PAIRS(GEPI_UNEMBED)
   else if (epi == GEPI_SWIGLU) RING_PAIRS(GEPI_SWIGLU)

@@ -69,10 +69,10 @@ __device__ __forceinline__ float ixt_log(float x) {
   return __builtin_fmaf(fe, 0.693145751953125f, __builtin_fmaf(fe, 1.42860682030941723212e-6f, lf));
 }
 
+__device__ __forceinline__ float ixt_sigmoid(float a) { return rbf(1.0f / (1.0f + ixt_exp(-a))); }
 // MlpBlock gate: bf16(bf16(a * bf16(sigmoid(a))) * b)
 __device__ __forceinline__ bf16_t ixt_swiglu(float a, float b) {
-  float sg = rbf(1.0f / (1.0f + ixt_exp(-a)));
-  float u = rbf(a * sg);
+  float u = rbf(a * ixt_sigmoid(a));
   return f2bf(u * b);
 }
 
@@ -99,13 +99,30 @@ __device__ __forceinline__ float ixt_tanh(float x) {
 
 // Gemma MlpBlock gate (mlp_activations ["gelu", "linear"], linears.py:449-464; jax.nn.gelu approximate=True on bf16 values, every
 // primitive rounded to bf16): cdf = 0.5 (1 + tanh(c (a + 0.044715 a^3))), bf16(bf16(a * cdf) * b)
-__device__ __forceinline__ bf16_t ixt_geglu(float a, float b) {
+__device__ __forceinline__ float ixt_gelu_cdf(float a) {
   const float x3 = rbf(rbf(a * a) * a);
   const float u = rbf(a + rbf(0.044677734375f * x3));       // bf16(0.044715)
   const float th = rbf(ixt_tanh(rbf(0.796875f * u)));       // bf16(sqrt(2 / pi))
-  const float cdf = rbf(0.5f * rbf(1.0f + th));
-  const float g = rbf(a * cdf);
+  return rbf(0.5f * rbf(1.0f + th));
+}
+__device__ __forceinline__ bf16_t ixt_geglu(float a, float b) {
+  const float g = rbf(a * ixt_gelu_cdf(a));
   return f2bf(g * b);
+}
+
+// A gate whose argument is a bf16 value `a` is bf16(a * w(a)), w(a) a bf16 value that depends on `a` alone: bf16(sigmoid(a)), or Gemma's cdf.  Table of w over
+// sign and 2^-10 <= |a| <= 2^7; below, w is its value at 2^-10 of that sign (1/2: what is added to 1/2 or 1 is less than half a step of bf16), above, its
+// value at 2^7 (ixt_exp clamps its argument at 80, tanh is 1 from 10 on).
+#define IXT_GATE_LO ((127 - 10) << 7)
+#define IXT_GATE_N (17 * 128 + 1)                    // of one sign
+#define IXT_GATE_BYTES 9216                          // both, in whole KiB
+__device__ __forceinline__ int ixt_gate_at(uint32_t a) {
+  return min(max((int)(a & 0x7fffu), IXT_GATE_LO), IXT_GATE_LO + IXT_GATE_N - 1) - IXT_GATE_LO + (int)(a >> 15) * IXT_GATE_N;
+}
+// ixt_swiglu / ixt_geglu of bf16(t0) and bf16(t1), bit for bit
+__device__ __forceinline__ bf16_t ixt_gate(const bf16_t* table, float t0, float t1) {
+  const bf16_t a = f2bf(t0);
+  return f2bf(rbf(bf2f(a) * bf2f(table[ixt_gate_at(a)])) * rbf(t1));
 }
 
 // gated units in f32, by kind (IXT_GLU_*).  1: g = min(a, limit), u = clamp(b, -limit, limit), g sigmoid(1.702 g) (u + 1); 2: tanh form of gelu, as

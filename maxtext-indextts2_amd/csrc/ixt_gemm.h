@@ -16,6 +16,8 @@
 // read and then multiplied, 112 with the reads under the products, 107 and now 100 with the steps that refill a loop of their own, without a branch, and the barrier behind a
 // step's first products.  256 x 128 tiles take 1250 to 1310 cycles per 64 k of which the products are 1068, at 1.6 to 2.3 GHz: the card's power sets the clock.  Tried without gain: the
 // fetches of a SIMD's two waves in different halves of a chunk, hot weights, chunk-contiguous operands.
+// What a launch spends beside its chunks (256 x 128, 128 x 128): 2 to 3.5 us until the first one is there, and the epilogue, before and now: residual 6.5 and 3.4 -> 2.4 and 1.1 us (loads, then
+// stores of 16 bytes), gated unit 4.5 and 2.3 -> 2.7 and 1.5 (ixt_gate), Gemma's 12 -> 2.7, q, k, v 10.7 and 6.0 -> 6.7 and 3.1.
 //
 // Epilogues (EPI):
 //   GEPI_F32      f32 [slice][R][N] (op-level entry point, split-K form)
@@ -29,10 +31,11 @@
 //   GEPI_QKV      bf16(t), RoPE (embeddings.py:277-315), q -> qbuf, k / v -> the row's page (paged_attention.py:446-471).  Q and K
 //                 head columns are stored pair-interleaved (qk_col): a 16-column tile holds features 8j..8j+7 and half+8j..half+8j+7,
 //                 so the two RoPE partners of a feature sit in lanes l and l ^ 32 of one accumulator register.
+//   GEPI_QKV32    the same with rope_type "llama3.1" (a kernel of its own: its code in the other's way costs every wave instruction fetches)
 #pragma once
 #include <type_traits>
 
-enum { GEPI_F32 = 0, GEPI_UNEMBED = 1, GEPI_RESID = 2, GEPI_SWIGLU = 3, GEPI_QKV = 4, GEPI_TANHNORM = 5, GEPI_ACT = 6 };
+enum { GEPI_F32 = 0, GEPI_UNEMBED = 1, GEPI_RESID = 2, GEPI_SWIGLU = 3, GEPI_QKV = 4, GEPI_TANHNORM = 5, GEPI_ACT = 6, GEPI_QKV32 = 7 };
 
 // GEPI_TANHNORM: an f32 residual stream between tanh norms, x <- x + post(t), act = bf16(pre(x)), norm(y) = tanh(alpha y) w + b feature by feature (w
 // null: no norm).  Nothing in it looks at a row's other features, so it needs no launch of its own.
@@ -81,6 +84,21 @@ __device__ __forceinline__ void tanhnorm_epi(const TanhNormEpi& n, bf16_t* act, 
   *reinterpret_cast<uint2*>(act + xidx(row, col, n.Ep)) = o;
 }
 
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+// A lane of an accumulator tile holds four columns of one row (8 bytes of bf16): lane group q columns 4 q ..  The tiles of two row blocks, a swap of lane groups apart, are
+// 16 bytes a lane: eight columns, 8 (q / 2) .., of the first block on even groups, of the second on odd ones.  rows_split undoes it.
+__device__ __forceinline__ u32x4 rows_pair(const uint2& lo, const uint2& hi) {
+  const auto x = __builtin_amdgcn_permlane16_swap(lo.x, hi.x, false, false), y = __builtin_amdgcn_permlane16_swap(lo.y, hi.y, false, false);
+  return u32x4{x[0], y[0], x[1], y[1]};
+}
+__device__ __forceinline__ void rows_split(const u32x4& m, uint2& lo, uint2& hi) {
+  const auto x = __builtin_amdgcn_permlane16_swap(m.x, m.z, false, false), y = __builtin_amdgcn_permlane16_swap(m.y, m.w, false, false);
+  lo = make_uint2(x[0], y[0]); hi = make_uint2(x[1], y[1]);
+}
+// A value that is there from here on.  An epilogue loads, then fences, computes, fences, and then stores: a store under a condition is a block of its own, and a wait
+// in it for a load (or a load behind it) is one for every store before it, too.  128 x 128, residual: 3.4 us for eight stores that waited for each other, 1.1 with all at once.
+template <typename T> __device__ __forceinline__ void epi_fence(T& v) { asm volatile("" : "+v"(v)); }
+
 struct GemmEpi {
   float* out;                                           // F32: [slices][R][N]; UNEMBED: rounded logits [R][N] or nullptr
   float* amax_val; int32_t* amax_idx; ColRanges cr;     // UNEMBED: [R][WC ncolg]
@@ -95,6 +113,7 @@ struct GemmEpi {
   size_t sstride;                                       // F8 + routed experts: floats between two experts' column scales
   TanhNormEpi tn;                                       // TANHNORM (with act)
   int glu; float glu_limit; const float* act_par;       // ACT: the unit's kind and its numbers; SWIGLU: glu > 0 takes that gated unit of the f32 totals instead (ixt_glu), glu < 0 ixt_geglu
+  const bf16_t* gate;                                   // SWIGLU, glu <= 0: the gate's table (ixt_gate), IXT_GATE_BYTES
   int32_t* flags;                                       // SPLIT 2: a word a wave of a tile and part, zero between launches
   IxtWait wait;
   const int32_t* rb_exp; size_t wstride;                // routed experts: expert of every 16-row block (-1: none), 16-byte units between experts' kernels
@@ -120,7 +139,7 @@ __device__ __forceinline__ void ring_wait_chunks(int younger) {
 // RING_KEEP holds up to 18 chains, the longest that was measured (163 of 256 registers); a sum of more goes to one block a tile.
 #define RING_KEEP 7
 #define RING_LEFT 2              // a flag whose taker gave up: its setter clears it, so that the next launch finds zeros whatever happened
-//   grid = (8 ceil(ncolg / 8) zb, SPLIT 1 ? chains : SPLIT 2 ? parts : 1), block 64 WR WC, dynamic LDS = NS (WC CT + WR RB) KS KiB.
+//   grid = (8 ceil(ncolg / 8) zb, SPLIT 1 ? chains : SPLIT 2 ? parts : 1), block 64 WR WC, dynamic LDS = NS (WC CT + WR RB) KS KiB and, for SWIGLU, the gate's table.
 //   Row groups of one column group are block ids b, b + 8, ..: same XCD, the weights meet in its L2.
 //   F8 (ixt_fp8.h): both operands are e4m3 fragments of 64 k (still 1 KiB: the ring moves them exactly as bf16 fragments of 32 k); a fragment
 //   feeds two v_mfma_f32_16x16x32_fp8_fp8; at the end of every 512-k chain the accumulator is scaled by (a_rc s_n) before it joins the total.
@@ -184,6 +203,12 @@ __global__ __launch_bounds__(WR * WC * 64, 2) void k_gemm_ring(const u32x4* __re
     else lds_dma16<ONCE>(dst, pw, off[j]);
   };
   auto advance = [&]() { pw += wadv; px += (size_t)KS * 1024; };
+  bf16_t* const gate = reinterpret_cast<bf16_t*>(st + NS * NF * 64);
+  if constexpr (EPI == GEPI_SWIGLU) {                           // (older than every chunk: the first wait covers it)
+    if (e.glu <= 0) {
+      for (int p = wave; p < IXT_GATE_BYTES / 1024; p += NW) lds_dma16(lds0 + (uint32_t)(NS * NF + p) * 1024u, e.gate, (uint32_t)(p * 1024 + lane * 16));
+    }
+  }
 #pragma unroll
   for (int c = 0; c < NS; ++c)
     if (chb + c < che) {
@@ -191,6 +216,21 @@ __global__ __launch_bounds__(WR * WC * 64, 2) void k_gemm_ring(const u32x4* __re
       for (int j = 0; j < NJ; ++j) issue(c, j);
       advance();
     }
+  // QKV: the positions of the rows, and of a store's rows (PR row blocks, one for even and one for odd lane groups).  Behind the first fetches, in whose time they come; the first
+  // counted wait waits for as many pieces more
+  constexpr bool ROWS = EPI == GEPI_QKV || EPI == GEPI_QKV32;
+  constexpr int PR = RB % 2 == 0 && EPI == GEPI_QKV ? 2 : 1;
+  const int odd = PR == 2 ? cq & 1 : 0;
+  int pos[ROWS ? RB : 1], spos[ROWS ? RB / PR : 1], page[ROWS ? RB / PR : 1], act[ROWS ? RB / PR : 1];
+  if constexpr (ROWS) {
+#pragma unroll
+    for (int b = 0; b < RB; ++b) pos[b] = e.row_pos[min((rowg * TR + wr * RB + b) * 16 + r_in, R - 1)];
+#pragma unroll
+    for (int b = 0; b < RB; b += PR) {
+      const int at = min((rowg * TR + wr * RB + b + odd) * 16 + r_in, R - 1);
+      spos[b / PR] = e.row_pos[at]; page[b / PR] = e.row_slot[at]; act[b / PR] = e.row_active[at];      // (no use of them here: it would be a wait)
+    }
+  }
   f32x4 acc[CT][RB], tot[CT][RB];
 #pragma unroll
   for (int i = 0; i < CT; ++i)
@@ -410,19 +450,51 @@ __global__ __launch_bounds__(WR * WC * 64, 2) void k_gemm_ring(const u32x4* __re
       }
     }
   } else if constexpr (EPI == GEPI_RESID) {
+    if constexpr (RB % 2 == 0) {
+      u32x4 m[CT][RB / 2];
+      auto at = [&](int i, int b) {
+        const int tile = min(colg * TC + wc * CT + i, ntile - 1), row = min((rowg * TR + wr * RB + b + (cq & 1)) * 16 + r_in, R - 1);
+        return (size_t)row * N + tile * 16 + 8 * (cq >> 1);
+      };
 #pragma unroll
-    for (int i = 0; i < CT; ++i) {
-      const int tile = colg * TC + wc * CT + i;
+      for (int i = 0; i < CT; ++i)
 #pragma unroll
-      for (int b = 0; b < RB; ++b) {
-        const int row = (rowg * TR + wr * RB + b) * 16 + r_in;
-        if (tile < ntile && row < R) {
-          const size_t o = (size_t)row * N + tile * 16 + cq * 4;
-          const uint2 hv = *reinterpret_cast<const uint2*>(e.h_in + o);
-          uint2 ov;
-          ov.x = pack2(f2bf(bflo(hv.x) + rbf(tot[i][b][0])), f2bf(bfhi(hv.x) + rbf(tot[i][b][1])));
-          ov.y = pack2(f2bf(bflo(hv.y) + rbf(tot[i][b][2])), f2bf(bfhi(hv.y) + rbf(tot[i][b][3])));
-          *reinterpret_cast<uint2*>(e.h_out + o) = ov;
+        for (int b = 0; b < RB; b += 2) m[i][b / 2] = *reinterpret_cast<const u32x4*>(e.h_in + at(i, b));
+#pragma unroll
+      for (int i = 0; i < CT; ++i)
+#pragma unroll
+        for (int b = 0; b < RB; b += 2) {
+          uint2 h[2];
+          rows_split(m[i][b / 2], h[0], h[1]);
+#pragma unroll
+          for (int k = 0; k < 2; ++k) {
+            const f32x4& t = tot[i][b + k];
+            h[k].x = pack2(f2bf(bflo(h[k].x) + rbf(t[0])), f2bf(bfhi(h[k].x) + rbf(t[1])));
+            h[k].y = pack2(f2bf(bflo(h[k].y) + rbf(t[2])), f2bf(bfhi(h[k].y) + rbf(t[3])));
+          }
+          m[i][b / 2] = rows_pair(h[0], h[1]);
+          epi_fence(m[i][b / 2]);
+        }
+#pragma unroll
+      for (int i = 0; i < CT; ++i)
+#pragma unroll
+        for (int b = 0; b < RB; b += 2)
+          if (colg * TC + wc * CT + i < ntile && (rowg * TR + wr * RB + b + (cq & 1)) * 16 + r_in < R) *reinterpret_cast<u32x4*>(e.h_out + at(i, b)) = m[i][b / 2];
+    } else {
+#pragma unroll
+      for (int i = 0; i < CT; ++i) {
+        const int tile = colg * TC + wc * CT + i;
+#pragma unroll
+        for (int b = 0; b < RB; ++b) {
+          const int row = (rowg * TR + wr * RB + b) * 16 + r_in;
+          if (tile < ntile && row < R) {
+            const size_t o = (size_t)row * N + tile * 16 + cq * 4;
+            const uint2 hv = *reinterpret_cast<const uint2*>(e.h_in + o);
+            uint2 ov;
+            ov.x = pack2(f2bf(bflo(hv.x) + rbf(tot[i][b][0])), f2bf(bfhi(hv.x) + rbf(tot[i][b][1])));
+            ov.y = pack2(f2bf(bflo(hv.y) + rbf(tot[i][b][2])), f2bf(bfhi(hv.y) + rbf(tot[i][b][3])));
+            *reinterpret_cast<uint2*>(e.h_out + o) = ov;
+          }
         }
       }
     }
@@ -452,101 +524,156 @@ __global__ __launch_bounds__(WR * WC * 64, 2) void k_gemm_ring(const u32x4* __re
       }
     }
   } else if constexpr (EPI == GEPI_SWIGLU) {
+    static_assert(RB % 2 == 0, "pairs of row blocks");
     const int F = N >> 1;
+    u32x4 m[CT / 2][RB / 2];
 #pragma unroll
-    for (int i = 0; i < CT; i += 2) {
-      const int tile = colg * TC + wc * CT + i;             // even: wi_0 tile tile/2; tile + 1: wi_1 tile tile/2
+    for (int i = 0; i < CT; i += 2)                         // tile even: wi_0 tile tile/2; tile + 1: wi_1 tile tile/2
+#pragma unroll
+      for (int b = 0; b < RB; b += 2) {
+        uint2 o[2];
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+          bf16_t v[4];
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            v[j] = e.glu > 0 ? f2bf(ixt_glu(e.glu, tot[i][b + k][j], tot[i + 1][b + k][j], e.glu_limit)) : ixt_gate(gate, tot[i][b + k][j], tot[i + 1][b + k][j]);
+          o[k].x = pack2(v[0], v[1]); o[k].y = pack2(v[2], v[3]);
+        }
+        m[i / 2][b / 2] = rows_pair(o[0], o[1]);
+        epi_fence(m[i / 2][b / 2]);
+      }
+#pragma unroll
+    for (int i = 0; i < CT; i += 2)
+#pragma unroll
+      for (int b = 0; b < RB; b += 2) {
+        const int tile = colg * TC + wc * CT + i, row = (rowg * TR + wr * RB + b + (cq & 1)) * 16 + r_in;
+        if (tile + 1 < ntile && row < R) *reinterpret_cast<u32x4*>(e.act + xidx(row, (tile >> 1) * 16 + 8 * (cq >> 1), F)) = m[i / 2][b / 2];
+      }
+  } else if constexpr (EPI == GEPI_QKV || EPI == GEPI_QKV32) {
+    const AttnGeom& g = e.g;
+    const int half = g.hd >> 1, tph = g.hd >> 4;                // tiles per head
+    // section (q, k, v), head in it and tile in that of the wave's column tiles
+    int sect[CT], hh[CT], th[CT];
+    hh[0] = (colg * TC + wc * CT) / tph;
+    th[0] = colg * TC + wc * CT - hh[0] * tph;
+#pragma unroll
+    for (int i = 1; i < CT; ++i) {
+      const bool next = th[i - 1] + 1 == tph;
+      hh[i] = hh[i - 1] + next;
+      th[i] = next ? 0 : th[i - 1] + 1;
+    }
+#pragma unroll
+    for (int i = 0; i < CT; ++i) {
+      sect[i] = hh[i] < g.nq ? 0 : hh[i] < g.nq + g.nkv ? 1 : 2;
+      hh[i] -= sect[i] == 0 ? 0 : sect[i] == 1 ? g.nq : g.nq + g.nkv;
+    }
+    bool kv[RB / PR];
+#pragma unroll
+    for (int b = 0; b < RB / PR; ++b) {
+      kv[b] = (rowg * TR + wr * RB + b * PR + odd) * 16 + r_in < R && act[b] != 0;
+      const int chunk = spos[b] / g.P;
+      spos[b] -= chunk * g.P;                                   // from here on: the token in its page
+      page[b] = e.page_map[kv[b] ? (size_t)page[b] * g.mpg + chunk : 0];
+    }
+    // pair-interleaved tile: lanes cq 0,1 hold x1 = features 8 th + 4 (cq & 1) + j, lanes cq 2,3 the partners x2 = half + the same
+    if constexpr (EPI == GEPI_QKV) {
+      uint2 sn[CT][RB], cs[CT][RB];                             // (of value tiles, too: not used)
+      const uint32_t sign = cq < 2 ? 0x80008000u : 0u;
+#pragma unroll
+      for (int b = 0; b < RB; ++b) {
+        const size_t at = (size_t)pos[b] * half + 4 * (cq & 1);
+#pragma unroll
+        for (int i = 0; i < CT; ++i) {
+          sn[i][b] = *reinterpret_cast<const uint2*>(e.rope_sin + at + 8 * th[i]);
+          cs[i][b] = *reinterpret_cast<const uint2*>(e.rope_cos + at + 8 * th[i]);
+        }
+      }
+      typedef typename std::conditional<PR == 2, u32x4, u32x2>::type Piece;
+      Piece m[CT][RB / PR];
+#pragma unroll
+      for (int i = 0; i < CT; ++i) {
+        if (sect[i] < 2) {
+          // first half: bf16(bf16(x1 c) - bf16(x2 s)); second half: bf16(bf16(x2 c) + bf16(x1 s)); two features at a time
+#pragma unroll
+          for (int b = 0; b < RB; ++b) {
+#pragma unroll
+            for (int j = 0; j < 4; j += 2) {
+              const uint32_t v = pack2(f2bf(tot[i][b][j]), f2bf(tot[i][b][j + 1])), c = j ? cs[i][b].y : cs[i][b].x, s = (j ? sn[i][b].y : sn[i][b].x) ^ sign;
+              const auto x = __builtin_amdgcn_permlane32_swap(v, v, false, false);                                     // x1 and x2, on either partner
+              const uint32_t other = cq < 2 ? x[1] : x[0];
+              const uint32_t a = pack2(f2bf(bflo(v) * bflo(c)), f2bf(bfhi(v) * bfhi(c))), d = pack2(f2bf(bflo(other) * bflo(s)), f2bf(bfhi(other) * bfhi(s)));
+              tot[i][b][j] = bflo(a) + bflo(d);
+              tot[i][b][j + 1] = bfhi(a) + bfhi(d);
+            }
+          }
+        }
+        if (sect[i] == 0 && e.q_scalar != 0.0f) {
+#pragma unroll
+          for (int b = 0; b < RB; ++b)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) tot[i][b][j] = rbf(tot[i][b][j]) * e.q_scalar;
+        }
+#pragma unroll
+        for (int b = 0; b < RB; b += PR) {
+          uint2 o[PR];
+#pragma unroll
+          for (int k = 0; k < PR; ++k) {
+            const f32x4& t = tot[i][b + k];
+            o[k] = make_uint2(pack2(f2bf(t[0]), f2bf(t[1])), pack2(f2bf(t[2]), f2bf(t[3])));
+          }
+          if constexpr (PR == 2) m[i][b / 2] = rows_pair(o[0], o[1]);
+          else { m[i][b].x = o[0].x; m[i][b].y = o[0].y; }
+          epi_fence(m[i][b / PR]);
+        }
+      }
+      const int qfeat = (cq >= 2 ? half : 0) + (PR == 2 ? 0 : 4 * (cq & 1)), vfeat = PR == 2 ? 8 * (cq >> 1) : 4 * cq;
+#pragma unroll
+      for (int b = 0; b < RB / PR; ++b) {
+        const int row = (rowg * TR + wr * RB + b * PR + odd) * 16 + r_in;
+        bf16_t* const qp = e.qbuf + (size_t)row * g.nq * g.hd + qfeat;
+        bf16_t* const kp = e.kpages + kpage_off(g, page[b], 0, qfeat >> 3, spos[b]) + (qfeat & 7);
+        bf16_t* const vp = e.vpages + vpage_off(g, page[b], 0, spos[b]) + vfeat;
+#pragma unroll
+        for (int i = 0; i < CT; ++i)
+          if (colg * TC + wc * CT + i < ntile && (sect[i] == 0 ? row < R : kv[b])) {
+            bf16_t* const to = sect[i] == 0 ? qp + hh[i] * g.hd + 8 * th[i] : sect[i] == 1 ? kp + (hh[i] * (g.hd >> 3) + th[i]) * g.P * 8 : vp + hh[i] * g.P * g.hd + 16 * th[i];
+            *reinterpret_cast<Piece*>(to) = m[i][b];
+          }
+      }
+    } else {   // rope_type "llama3.1": f32 tables, one rounding (ixt_rope_pair); the lane's four de-interleaved features are every second feature of the model's order (ixt_qk_feat)
 #pragma unroll
       for (int b = 0; b < RB; ++b) {
         const int row = (rowg * TR + wr * RB + b) * 16 + r_in;
-        if (tile + 1 < ntile && row < R) {
-          const int f0 = (tile >> 1) * 16 + cq * 4;
-          bf16_t o[4];
 #pragma unroll
-          for (int j = 0; j < 4; ++j)
-            o[j] = e.glu > 0 ? f2bf(ixt_glu(e.glu, tot[i][b][j], tot[i + 1][b][j], e.glu_limit)) : e.glu < 0 ? ixt_geglu(rbf(tot[i][b][j]), rbf(tot[i + 1][b][j]))
-                                                                                                          : ixt_swiglu(rbf(tot[i][b][j]), rbf(tot[i + 1][b][j]));
-          uint2 ov;
-          ov.x = pack2(o[0], o[1]); ov.y = pack2(o[2], o[3]);
-          *reinterpret_cast<uint2*>(e.act + xidx(row, f0, F)) = ov;
-        }
-      }
-    }
-  } else if constexpr (EPI == GEPI_QKV) {
-    const AttnGeom& g = e.g;
-    const int half = g.hd >> 1, tph = g.hd >> 4;                // tiles per head
-    const int QN = g.nq * g.hd, KN = g.nkv * g.hd;
+        for (int i = 0; i < CT; ++i) {
+          const int fi = 8 * th[i] + 4 * (cq & 1);
+          float v[4];
 #pragma unroll
-    for (int b = 0; b < RB; ++b) {
-      const int row = (rowg * TR + wr * RB + b) * 16 + r_in;
-      const bool row_ok = row < R;
-      const int pos = row_ok ? e.row_pos[row] : 0;
-      const bool wr_kv = row_ok && e.row_active[row] != 0;
-      int page = 0;
-      if (wr_kv) page = e.page_map[(size_t)e.row_slot[row] * g.mpg + pos / g.P];
-      const int tok = pos % g.P;
-#pragma unroll
-      for (int i = 0; i < CT; ++i) {
-        const int tile = colg * TC + wc * CT + i;
-        const int col0 = tile * 16;
-        float v[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] = rbf(tot[i][b][j]);
-        const bool is_v = col0 >= QN + KN;
-        const int hh = col0 / g.hd, th = tile % tph;            // head (q heads, then k heads, then v heads), tile inside the head
-        if (!is_v) {
-          // pair-interleaved tile: lanes cq 0,1 hold x1 = features 8 th + 4 (cq & 1) + j, lanes cq 2,3 the partners x2 = half + the same
-          const int fi = 8 * th + 4 * (cq & 1);
-          if (g.rope32) {   // rope_type "llama3.1": f32 tables, one rounding (ixt_rope_pair)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
+          for (int j = 0; j < 4; ++j) {
+            v[j] = rbf(tot[i][b][j]);
+            if (sect[i] < 2) {
               const float other = __shfl_xor(v[j], 32, 64);
               float o1, o2;
-              ixt_rope_pair(1, e.rope_sin, e.rope_cos, (size_t)pos * half + fi + j, cq < 2 ? v[j] : other, cq < 2 ? other : v[j], o1, o2);
+              ixt_rope_pair(1, e.rope_sin, e.rope_cos, (size_t)pos[b] * half + fi + j, cq < 2 ? v[j] : other, cq < 2 ? other : v[j], o1, o2);
               v[j] = cq < 2 ? o1 : o2;
             }
+            if (sect[i] == 0 && e.q_scalar != 0.0f) v[j] = rbf(v[j] * e.q_scalar);
+          }
+          if (colg * TC + wc * CT + i >= ntile || !(sect[i] == 0 ? row < R : kv[b])) continue;
+          if (sect[i] == 2) {
+            uint2 ov;
+            ov.x = pack2(f2bf(v[0]), f2bf(v[1])); ov.y = pack2(f2bf(v[2]), f2bf(v[3]));
+            *reinterpret_cast<uint2*>(e.vpages + vpage_off(g, page[b], hh[i], spos[b]) + th[i] * 16 + cq * 4) = ov;
           } else {
-          float sn[4], cs[4];
-          {
-            const uint2 sv = *reinterpret_cast<const uint2*>(e.rope_sin + (size_t)pos * half + fi);
-            const uint2 cv = *reinterpret_cast<const uint2*>(e.rope_cos + (size_t)pos * half + fi);
-            sn[0] = bflo(sv.x); sn[1] = bfhi(sv.x); sn[2] = bflo(sv.y); sn[3] = bfhi(sv.y);
-            cs[0] = bflo(cv.x); cs[1] = bfhi(cv.x); cs[2] = bflo(cv.y); cs[3] = bfhi(cv.y);
-          }
+            const int feat = (cq >= 2 ? half : 0) + fi;
 #pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const float other = __shfl_xor(v[j], 32, 64);
-            // first half: bf16(bf16(x1 c) - bf16(x2 s)); second half: bf16(bf16(x2 c) + bf16(x1 s))
-            v[j] = cq < 2 ? rbf(rbf(v[j] * cs[j]) - rbf(other * sn[j])) : rbf(rbf(v[j] * cs[j]) + rbf(other * sn[j]));
+            for (int j = 0; j < 4; ++j) {
+              const int f = ixt_qk_feat(1, feat + j, half);
+              if (sect[i] == 0) e.qbuf[((size_t)row * g.nq + hh[i]) * g.hd + f] = f2bf(v[j]);
+              else e.kpages[kpage_off(g, page[b], hh[i], f >> 3, spos[b]) + (f & 7)] = f2bf(v[j]);
+            }
           }
-          }
-        }
-        if (hh < g.nq && e.q_scalar != 0.0f) {
-#pragma unroll
-          for (int j = 0; j < 4; ++j) v[j] = rbf(v[j] * e.q_scalar);
-        }
-        if (tile >= ntile || !row_ok) continue;
-        uint2 ov;
-        ov.x = pack2(f2bf(v[0]), f2bf(v[1])); ov.y = pack2(f2bf(v[2]), f2bf(v[3]));
-        if (g.rope32 && !is_v) {   // llama3.1: the lane's four de-interleaved features are every second feature of the model's order (ixt_qk_feat)
-          const int feat = (cq >= 2 ? half : 0) + 8 * th + 4 * (cq & 1);
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const int fn_ = ixt_qk_feat(1, feat + j, half);
-            if (hh < g.nq) e.qbuf[((size_t)row * g.nq + hh) * g.hd + fn_] = f2bf(v[j]);
-            else if (wr_kv) e.kpages[kpage_off(g, page, hh - g.nq, fn_ >> 3, tok) + (fn_ & 7)] = f2bf(v[j]);
-          }
-        } else if (hh < g.nq) {
-          const int feat = (cq >= 2 ? half : 0) + 8 * th + 4 * (cq & 1);
-          *reinterpret_cast<uint2*>(e.qbuf + ((size_t)row * g.nq + hh) * g.hd + feat) = ov;
-        } else if (!is_v) {
-          if (wr_kv) {
-            const int feat = (cq >= 2 ? half : 0) + 8 * th + 4 * (cq & 1);
-            *reinterpret_cast<uint2*>(e.kpages + kpage_off(g, page, hh - g.nq, feat >> 3, tok) + (feat & 7)) = ov;
-          }
-        } else if (wr_kv) {
-          const int feat = th * 16 + cq * 4;
-          *reinterpret_cast<uint2*>(e.vpages + vpage_off(g, page, hh - g.nq - g.nkv, tok) + feat) = ov;
         }
       }
     }

@@ -128,6 +128,7 @@ struct ixt_ctx {
   int small_prefetch_blocks = 64;
   int ring_parts = 1;        // f32 sums of few tiles over a long K: three blocks a tile (k_gemm_ring, SPLIT 2)
   int32_t* ring_flags = nullptr;
+  bf16_t* gate_tables = nullptr;   // k_gate_tables
   int small_step = 1;        // few rows: all layers in one launch (k_step) where the shapes allow; 0: five launches a layer
   struct StepLayer* step_layers = nullptr;   // [L] in HBM
   bf16_t* step_ws = nullptr;

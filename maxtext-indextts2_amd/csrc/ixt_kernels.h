@@ -2381,4 +2381,12 @@ __global__ void k_copy_convert(const T* src, bf16_t* dst, int64_t rows, int64_t 
   else dst[r * ldd + c] = src[i];
 }
 
+// the gates' tables (ixt_gate_at), one behind the other: ixt_swiglu's, ixt_geglu's
+static __global__ void k_gate_tables(bf16_t* out) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x, n = IXT_GATE_BYTES / 2, r = i % n;
+  if (i >= 2 * n) return;
+  const float a = bf2f((bf16_t)(IXT_GATE_LO + r % IXT_GATE_N | r / IXT_GATE_N << 15));
+  out[i] = r >= 2 * IXT_GATE_N ? 0 : f2bf(i < n ? ixt_sigmoid(a) : ixt_gelu_cdf(a));
+}
+
 #include "ixt_gemm.h"
