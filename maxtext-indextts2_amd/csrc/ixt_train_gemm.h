@@ -12,8 +12,7 @@
 //   a row of 32 k is half a line of 128 bytes: where an operand's k is contiguous (PAIR), both halves are fetched one behind the other, every second step, so that the second comes
 //   from the L1 (fetches alone 593 cycles per 32 KiB, 1110 with the halves a step apart; five slots instead of four).
 // Measured (us, with a launch's start and end), before these three and the stores of 16 bytes / now: 4096 x 4096, K 8192, k contiguous 232 / 205, of one operand 243 / 229, by columns 231 / 216;
-// 16384 x 8192, K 2048 531 / 477; 128 x 128 blocks, 4096 x 2048, K 4096 86 / 68; 64 x 64, 2048 x 768, K 4096 31.8 / 26.8.  Sums onto an f32 C (256 x 256 tiles): 20 us of a tile's 80
-// are its 512 KiB, all CUs at once, at 6.5 TB/s.
+// 16384 x 8192, K 2048 531 / 477; 128 x 128 blocks, 4096 x 2048, K 4096 86 / 68; 64 x 64, 2048 x 768, K 4096 31.8 / 26.8.
 //   k contiguous:   slot image [row][32 k], four 16-byte pieces a row, piece c of row r at c ^ ((r >> 2) & 3): the 16 rows a half wave reads lie on
 //                   disjoint banks
 //   row contiguous: slot image [k][row], 32-byte pieces, piece u of row k at u ^ (k & 7) (64 rows: u ^ (k / 2 & 3)); ds_read_tr16 hands a 4 x 16 block to 16 lanes column-wise, so
@@ -266,57 +265,90 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void k_tgemm(TGemm g) {
       for (int j = 0; j < NI; ++j) acc[i][j] = tot[i][j];
   }
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");             // nothing may land in LDS that the next block owns
-  // lane: m = r16, n = 4 q + register
+  // lane: m = r16, n = 4 q + register.  A tile that lies inside C has an epilogue without conditions: a load or a store under one is a block of its own, where a wait for a
+  // load is one for every store before it (256 x 256: sums onto C 20 us a tile, 12 now; with a residual 13 and 7.2)
   const int out = g.out, m1 = m0 + wm * MI * 16 + r16, nw = n0 + wn * NI * 16;
-  if (out == TG_F32 || out == TG_F32_ADD) {
-    float* c = reinterpret_cast<float*>(g.C[prob]) + (g.parts > 1 ? part * g.cpart[prob] : zc) + nw + q * 4;
-    constexpr int AHEAD = MI < 4 ? MI : 4;                                // rows of the old sums in flight (one at a time: 20 us a tile of 256 x 256, eight waits)
-    tf32x4 old[AHEAD][NI];
-    auto load = [&](int i) {
+  auto epilogue = [&](auto inside_) {
+    constexpr bool inside = inside_.value;
+    if (out == TG_F32 || out == TG_F32_ADD) {
+      const long ld = g.ldc[prob];
+      float* c = reinterpret_cast<float*>(g.C[prob]) + (g.parts > 1 ? part * g.cpart[prob] : zc) + (long)m1 * ld + nw + q * 4;
+      auto in = [&](int i, int j) { return inside || (m1 + i * 16 < g.M && nw + j * 16 + q * 4 < N); };
+      constexpr int AHEAD = MI < 4 ? MI : 4;                              // rows of the old sums in flight
+      tf32x4 old[AHEAD][NI];
+      auto load = [&](int i) {
 #pragma unroll
-      for (int j = 0; j < NI; ++j)
-        old[i % AHEAD][j] = m1 + i * 16 < g.M && nw + j * 16 + q * 4 < N ? *reinterpret_cast<const tf32x4*>(c + (long)(m1 + i * 16) * g.ldc[prob] + j * 16) : tf32x4(0.0f);
+        for (int j = 0; j < NI; ++j) old[i % AHEAD][j] = in(i, j) ? *reinterpret_cast<const tf32x4*>(c + i * 16 * ld + j * 16) : tf32x4(0.0f);
+      };
+      if (out == TG_F32_ADD) {
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i) load(i);
+#pragma unroll
+        for (int i = 0; i < MI; ++i) {
+#pragma unroll
+          for (int j = 0; j < NI; ++j) {
+            acc[i][j] = old[i % AHEAD][j] + acc[i][j];
+            if (in(i, j)) *reinterpret_cast<tf32x4*>(c + i * 16 * ld + j * 16) = acc[i][j];
+          }
+          if (i + AHEAD < MI) load(i + AHEAD);
+          __builtin_amdgcn_sched_barrier(0);                              // (a row's addresses at a time: all of them are 64 registers)
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < MI; ++i) {
+#pragma unroll
+          for (int j = 0; j < NI; ++j)
+            if (in(i, j)) *reinterpret_cast<tf32x4*>(c + i * 16 * ld + j * 16) = acc[i][j];
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+      return;
+    }
+    // bf16: two column tiles at a time; a swap of lane groups leaves every lane eight columns of one of them, 16 bytes to store and 64 side by side (256 x 256:
+    // 4.1 us for stores of 8 bytes, 2.4)
+    static_assert(NI % 2 == 0, "pairs of column tiles");
+    const int ns = nw + (q & 1) * 16 + (q >> 1) * 8;
+    const long at = zc + (long)m1 * g.ldc[prob] + ns;
+    auto in = [&](int i, int j) { return inside || (m1 + i * 16 < g.M && ns + j * 16 < N); };
+    auto pair = [&](const uint2& lo, const uint2& hi) -> uint4 {
+      const auto x = __builtin_amdgcn_permlane16_swap(lo.x, hi.x, false, false), y = __builtin_amdgcn_permlane16_swap(lo.y, hi.y, false, false);
+      return make_uint4(x[0], y[0], x[1], y[1]);
     };
-    if (out == TG_F32_ADD) {
+    if (out == TG_BF16_RES) {
+      // (the pair of a pair is the pair's halves again)
+      constexpr int STEP = MI < 4 ? MI : 4;
 #pragma unroll
-      for (int i = 0; i < AHEAD; ++i) load(i);
+      for (int i0 = 0; i0 < MI; i0 += STEP) {
+        uint4 r[STEP][NI / 2];
+#pragma unroll
+        for (int i = 0; i < STEP; ++i)
+#pragma unroll
+          for (int j = 0; j < NI; j += 2) r[i][j / 2] = in(i0 + i, j) ? *reinterpret_cast<const uint4*>(g.R + at + (i0 + i) * 16 * g.ldc[prob] + j * 16) : make_uint4(0u, 0u, 0u, 0u);
+#pragma unroll
+        for (int i = 0; i < STEP; ++i)
+#pragma unroll
+          for (int j = 0; j < NI; j += 2) {
+            const uint4 h = pair(make_uint2(r[i][j / 2].x, r[i][j / 2].y), make_uint2(r[i][j / 2].z, r[i][j / 2].w));
+            const uint2 hh[2] = {make_uint2(h.x, h.y), make_uint2(h.z, h.w)};
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+              tf32x4& v = acc[i0 + i][j + k];
+              v[0] = bflo(hh[k].x) + rbf(v[0]); v[1] = bfhi(hh[k].x) + rbf(v[1]); v[2] = bflo(hh[k].y) + rbf(v[2]); v[3] = bfhi(hh[k].y) + rbf(v[3]);
+            }
+          }
+      }
     }
 #pragma unroll
     for (int i = 0; i < MI; ++i) {
-      if (out == TG_F32_ADD) {
 #pragma unroll
-        for (int j = 0; j < NI; ++j) acc[i][j] = old[i % AHEAD][j] + acc[i][j];
-        if (i + AHEAD < MI) load(i + AHEAD);
+      for (int j = 0; j < NI; j += 2) {
+        const tf32x4 &v = acc[i][j], &w = acc[i][j + 1];
+        const uint4 o = pair(make_uint2(pack2(f2bf(v[0]), f2bf(v[1])), pack2(f2bf(v[2]), f2bf(v[3]))), make_uint2(pack2(f2bf(w[0]), f2bf(w[1])), pack2(f2bf(w[2]), f2bf(w[3]))));
+        if (in(i, j)) *reinterpret_cast<uint4*>(reinterpret_cast<bf16_t*>(g.C[prob]) + at + i * 16 * g.ldc[prob] + j * 16) = o;
       }
-#pragma unroll
-      for (int j = 0; j < NI; ++j)
-        if (m1 + i * 16 < g.M && nw + j * 16 + q * 4 < N) *reinterpret_cast<tf32x4*>(c + (long)(m1 + i * 16) * g.ldc[prob] + j * 16) = acc[i][j];
+      __builtin_amdgcn_sched_barrier(0);
     }
-    return;
-  }
-  // bf16: two column tiles at a time; a swap of lane groups leaves every lane eight columns of one of them, 16 bytes to store and 64 side by side (256 x 256:
-  // 4.1 us for stores of 8 bytes)
-  static_assert(NI % 2 == 0, "pairs of column tiles");
-  const int ns = nw + (q & 1) * 16 + (q >> 1) * 8;
-#pragma unroll
-  for (int i = 0; i < MI; ++i) {
-    const int m = m1 + i * 16;
-    const long row = (long)m * g.ldc[prob];
-#pragma unroll
-    for (int j = 0; j < NI; j += 2) {
-      uint2 o[2];
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        tf32x4 v = acc[i][j + h];
-        if (out == TG_BF16_RES) {
-          const int n = nw + (j + h) * 16 + q * 4;
-          const uint2 r = m < g.M && n < N ? *reinterpret_cast<const uint2*>(g.R + row + n) : make_uint2(0u, 0u);
-          v[0] = bflo(r.x) + rbf(v[0]); v[1] = bfhi(r.x) + rbf(v[1]); v[2] = bflo(r.y) + rbf(v[2]); v[3] = bfhi(r.y) + rbf(v[3]);
-        }
-        o[h].x = pack2(f2bf(v[0]), f2bf(v[1])); o[h].y = pack2(f2bf(v[2]), f2bf(v[3]));
-      }
-      const auto x = __builtin_amdgcn_permlane16_swap(o[0].x, o[1].x, false, false), y = __builtin_amdgcn_permlane16_swap(o[0].y, o[1].y, false, false);
-      if (m < g.M && ns + j * 16 < N) *reinterpret_cast<uint4*>(reinterpret_cast<bf16_t*>(g.C[prob]) + zc + row + ns + j * 16) = make_uint4(x[0], y[0], x[1], y[1]);
-    }
-  }
+  };
+  if (m0 + BM <= g.M && n0 + BN <= N) epilogue(std::true_type());
+  else epilogue(std::false_type());
 }
