@@ -1,6 +1,6 @@
 // ixt_tile_attn.h -- prefill attention on the f32 matrix units, for pages of 32 tokens.
 //
-// v_mfma_f32_16x16x4_f32 adds its four products to the accumulator one after the other, k ascending, each step one IEEE fma (subnormals kept): on
+// v_mfma_f32_16x16x4_f32 (and v_mfma_f32_16x16x1_4b_f32, four blocks of one product) adds its four products to the accumulator one after the other, k ascending, each step one IEEE fma (subnormals kept): on
 // 10^6 cells of random bf16 and f32 operands, down to subnormal sums, its result is the chain of four fmaf bit for bit.  So the contract's chains --
 // a score is one fma chain over d, an output one fma chain over the tokens of a page -- run on it unchanged, at 140 TFLOP/s where the vector units'
 // chains (k_attn_tile) reached 17.
@@ -10,6 +10,7 @@
 #include <type_traits>
 
 typedef float ixt_f32x4 __attribute__((ext_vector_type(4)));
+typedef float ixt_f32x16 __attribute__((ext_vector_type(16)));
 
 // rows 1 and 3 of `a` (16 lanes each) against rows 0 and 2 of `b` / the upper half of `a` against the lower half of `b`
 __device__ __forceinline__ void ixt_swap16(uint32_t& a, uint32_t& b) {
@@ -21,32 +22,20 @@ __device__ __forceinline__ void ixt_swap32(uint32_t& a, uint32_t& b) {
   a = r[0]; b = r[1];
 }
 
-// 32 consecutive d of 16 keys, lane (key, c) holding the bf16 d = 8 c .. 8 c + 7, as the matrix operands of eight steps: out[s] on lane (key, c) is
-// d = 4 s + c.  `sel`: v_perm selector of the lane's half of a dword, as f32.
-__device__ __forceinline__ void ixt_k_operands(const u32x4& w, uint32_t sel, float (&out)[8]) {
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    uint32_t a = h ? w.z : w.x, b = h ? w.w : w.y;
-    ixt_swap32(a, b);
-    uint32_t a1 = a, b1 = b;
-    ixt_swap16(a, a1);
-    ixt_swap16(b, b1);
-    out[0 + h] = __uint_as_float(__builtin_amdgcn_perm(a, 0u, sel)); out[2 + h] = __uint_as_float(__builtin_amdgcn_perm(a1, 0u, sel));
-    out[4 + h] = __uint_as_float(__builtin_amdgcn_perm(b, 0u, sel)); out[6 + h] = __uint_as_float(__builtin_amdgcn_perm(b1, 0u, sel));
-  }
-}
-
 // block = (kv head, 16 query vectors = 16 / GQ consecutive rows x GQ heads), NW waves.  Super-block (4 pages, 128 keys) n NW + w belongs to wave w in
 // round n; its 128 x 16 scores stay in that wave's registers from the score products to the output products, so the keys one block holds are
 // 128 NW NR and nothing of them goes through LDS or memory.
-//   Scores: matrix rows = keys, columns = query vectors.  Row i of tile t is token 4 t + i % 4 of page i / 4: a lane then holds the 32 tokens of ONE
-//   page (its 16-lane group) for one query vector, and the page's sum of exponentials is a sum over its own registers, in order.  K is read once, 16
-//   bytes a lane, and turned into operands by lane swaps; the query operand comes from LDS, one read per eight products.
+//   Scores: matrix rows = keys, columns = query vectors, one d a step (16x16x1: four blocks of 16 keys, each with the operand of its own lane group).  Row i
+//   of block b is token 4 t + i % 4 of page i / 4, t = b and 4 + b: a lane then holds the 32 tokens of ONE page (its 16-lane group) for one query vector, and
+//   the page's sum of exponentials is a sum over its own registers, in order.  K is read once, 16 bytes a lane: eight d of the lane's own key, operands as they are
+//   (with four d a step, 16x16x4, they had to change lanes first, 18 vector instructions for eight products instead of 8: 33.7 us of a block's 103 in <8, 4>, now 28, which is
+//   the products' own time).  The query operand comes from LDS, 16 bytes for four steps.
 //   Softmax: max over lanes and waves; page sums meet in LDS and every lane adds its vector's in page order.  e / l with one reciprocal per lane:
 //   two corrections of the quotient give the correctly rounded one where no remainder is subnormal (e >= 2^-96); otherwise the divide itself.
 //   Outputs: matrix rows = value columns, P as the other operand after a 4 x 4 transpose of lane groups and registers.  A lane's 16 bytes of V are 8
 //   columns of one token: column 8 i + x belongs to row i of tile x.  Page chains start from zero, four pages add up in order; the super-blocks of a
-//   round meet in LDS, where the thread that owns (vector, column) adds them in order.
+//   round meet in LDS, where the thread that owns (vector, column) adds them in order: with two buffers there, one barrier a round (four, half of the columns at
+//   a time, took 3 us more of the 103).
 // A key that a row does not see has P = +0 (k_attn_tile says why that is exact); tokens past the end are re-reads of the last one.
 // Rows of other page groups in the tile are worked off group by group, dealt among `shares` blocks.  grid = (kv heads, tiles, parts x shares): parts = 1 or
 // the number of 128-column parts of a value (the two halves of head_dim 256 in two blocks, each taking the scores anew), shares = 1 or more, both for
@@ -54,28 +43,32 @@ __device__ __forceinline__ void ixt_k_operands(const u32x4& w, uint32_t sel, flo
 // Bound by the matrix units and the vector units TOGETHER: an f32 product and a vector instruction of the same SIMD take turns, whichever waves they belong to (products
 // alone 150 TFLOP/s; one bf16 -> f32 conversion in front of each 116, eight in front of eight 129).  So what counts is vector instructions: operands of a
 // step converted together, no mask where every row sees every key (sees_all; the selects of a score were a branch each), weights rounded and packed two at a time ahead
-// of the transpose.  Tried without gain: the keys of the next super-block requested ahead, page numbers in a register, a priority for half of the waves;
-// 4-byte loads of the keys that need no lane swaps (2.3 x slower).  Keys and values widened to f32 by a launch ahead take another 15 % off here and cost 11 to 22 us for 1024 to
-// 3900 keys: level up to 2048.
-// What the bound of two or three blocks a CU leaves no register for goes through scratch.  Registers spilled, heads of 128: <2, 1> 31 to 39, <4, 1> 16 to 30, <8, 3> 19 to 29, <8, 4> 75 to 89; heads of
-// 256: 31 to 42, 20 to 32, 26 to 37, 82 to 86; heads of 64: <8, 4> 47 to 55, <2, 1> up to 6; the other forms none.  Scratch's loads and stores stand in the counter of the fetches, too; what they cost is not
-// measured.
-// Measured against k_attn_tile, 16 heads of 128, 1024 rows at <= 1024 / 2048 / 3072 keys 282 / 860 / 1143 us; before the instructions above and the forms
-// <4, 2> and <8, 3>: 112 / 215 / 351, now 88 / 195 / 302.  828 rows at <= 3900 keys 1496, 448, 411 us (57 TFLOP/s).  8 heads of 256 on 4, 256 rows at <= 3000 keys: 151 -> 130 us.
-// 8 packed prompts (1525 rows, <= 251 keys) 128.6, 68.8, 67.6: two waves per block for <= 256 keys, with four, two of them had nothing to do (90.2 us).
+// of the transpose.  A block of <8, 4> at 3072 to 3900 keys: 4.1 us until the first scores, 28 scores, 12 maxima and exponentials, 5 weights, 43 outputs (their products: 27 and 27); the
+// clock stays at 2.2 to 2.4 GHz.  Tried without gain: a priority for half of the waves; values by 16x16x1 products, too, four pages at a time from weights as they lie (286
+// against 293 us at <= 3072 keys, but 403 against 375 at <= 3900 and 118 against 117 with heads of 256: the sums of four pages leave no registers); a whole page of values
+// ahead (spills: 316 us).  Keys and values widened to f32 by a launch ahead: level up to 2048 keys.
+// What the bound of two or three blocks a CU leaves no register for goes through scratch.  Registers spilled, heads of 128: <2, 1> 32, <8, 3> 23, <8, 4> 76; heads of 256: <8, 3> 33.
+// Measured against k_attn_tile, 16 heads of 128, 1024 rows at <= 1024 / 2048 / 3072 keys 282 / 860 / 1143 us, before the scores' 16x16x1 products and the exchange with one barrier
+// 92 / 212 / 310, now 87 / 198 / 293.  828 rows at <= 3900 keys 1496, 408, 375 us (63 TFLOP/s).  8 heads of 256 on 4, 256 rows at <= 1756 / 2756 keys: 88 / 131, 79 / 117 us.
+// Prompts of <= 256 keys: two waves per block; with four, two of them had nothing to do (eight packed ones, 1525 rows: 90.2 us against 67.6).
+// Buffers of the exchange: with two a round has one barrier (another one's sums are read while the next is written); one where there is one round, or where two
+// would take a CU's second block away.
+constexpr int mtile_buffers(int hd, int nw, int nr) { return nr > 1 && (nw == 8 || hd <= 128) ? 2 : 1; }
+constexpr size_t mtile_lds(int hd, int nw, int nr) { return (size_t)mtile_buffers(hd, nw, nr) * nw * 16 * ((hd >= 128 ? 128 : hd) + 4) * 4; }
 template <int HD, int GQ, int NW, int NR>
 __global__ __launch_bounds__(NW * 64, NR == 1 && NW <= 4 ? 3 : 2) void k_attn_mtile(TileAttnArgs a) {
   constexpr int TQ = 16 / GQ;
   constexpr int NB = HD / 32;
   constexpr int VW = HD >= 128 ? 128 : HD;     // value columns of one output pass
   constexpr int NE = VW / 16;                  // matrix tiles of them
-  constexpr int NEH = NE / 2, CH = VW / 2, OP = CH + 4;
-  constexpr int NTOT = 16 * CH / (NW * 64);    // (vector, column) totals per thread and half
+  constexpr int OP = VW + 4, NTOT = 16 * VW / (NW * 64);       // a vector's pitch of the exchange; (vector, column) totals per thread
+  constexpr int NBUF = mtile_buffers(HD, NW, NR);
   static_assert(16 % GQ == 0 && HD % 64 == 0 && (HD <= 128 || HD % 128 == 0), "tile geometry");
-  __shared__ __attribute__((aligned(16))) float qs[HD / 4 * 64];         // step s, lane l: d = 4 s + l / 16 of vector l % 16
+  constexpr int QP = HD + 4;                                             // a vector's pitch: 16 lanes read 16 bytes of 16 vectors without a bank conflict
+  __shared__ __attribute__((aligned(16))) float qs[16 * QP];
   __shared__ float psum[NW * NR * 4 * 16];                               // [page][vector]
   __shared__ float wmax[NW * 16];
-  __shared__ __attribute__((aligned(16))) float ob[NW * 16 * OP];        // [wave][vector][half the columns]
+  extern __shared__ __attribute__((aligned(16))) float ob[];             // [buffer][wave][vector][columns]
   __shared__ int s_pos[TQ], s_slot[TQ];
   const AttnGeom& g = a.g;
   const int kvh = blockIdx.x, r0 = (gridDim.y - 1 - blockIdx.y) * TQ;    // the rows with the most keys first
@@ -91,11 +84,9 @@ __global__ __launch_bounds__(NW * 64, NR == 1 && NW <= 4 ? 3 : 2) void k_attn_mt
   for (int it = tid; it < 16 * (HD / 8); it += NW * 64) {
     const int v = it & 15, c = it >> 4;
     const u32x4 w = *reinterpret_cast<const u32x4*>(a.qbuf + ((size_t)min(r0 + v / GQ, a.R - 1) * g.nq + kvh * GQ + v % GQ) * HD + c * 8);
-#pragma unroll
-    for (int x = 0; x < 4; ++x) {
-      qs[(2 * c + (x >> 1)) * 64 + (2 * x & 3) * 16 + v] = bflo(w[x]);
-      qs[(2 * c + (x >> 1)) * 64 + ((2 * x & 3) + 1) * 16 + v] = bfhi(w[x]);
-    }
+    float4* q = reinterpret_cast<float4*>(qs + v * QP + c * 8);
+    q[0] = make_float4(bflo(w[0]), bfhi(w[0]), bflo(w[1]), bfhi(w[1]));
+    q[1] = make_float4(bflo(w[2]), bfhi(w[2]), bflo(w[3]), bfhi(w[3]));
   }
   __syncthreads();
   unsigned pending = 0;
@@ -107,7 +98,6 @@ __global__ __launch_bounds__(NW * 64, NR == 1 && NW <= 4 ? 3 : 2) void k_attn_mt
       for (int idx = tid; idx < GQ * HD; idx += NW * 64) a.out[xidx(r0 + i, kvh * GQ * HD + idx, n_out)] = 0;
     }
   }
-  const uint32_t sel = (lg & 1) ? 0x07060c0cu : 0x05040c0cu;
   int turn = 0;                                          // whose group comes next
   while (pending != 0) {
     // the rows of the leader's page group
@@ -139,49 +129,61 @@ __global__ __launch_bounds__(NW * 64, NR == 1 && NW <= 4 ? 3 : 2) void k_attn_mt
     auto sees_all = [&](int sb) { return sb * 128 + 127 <= posmin && (a.window <= 0 || posmax - a.window < sb * 128); };
 
     // ---- scores
-    ixt_f32x4 S[NR][8];
+    ixt_f32x16 S[NR][2];                                 // register 4 (t % 4) + r of half t / 4: token 4 t + r of the lane's page
     float mx = -INFINITY, mn = INFINITY;
 #pragma unroll
     for (int n = 0; n < NR; ++n) {
       const int sb = n * NW + wave;
-#pragma unroll
-      for (int t = 0; t < 8; ++t) S[n][t] = ixt_f32x4(0.0f);
+      S[n][0] = S[n][1] = ixt_f32x16(0.0f);
       if (sb < nsb) {
-        const bf16_t* kp = a.kpages + kpage_off(g, prow[min(4 * sb + (i16 >> 2), pages_all - 1)], kvh, lg, i16 & 3);
+        // lane (i16, lg) loads token 4 t + i16 % 4 of page i16 / 4, t = lg and 4 + lg
+        const bf16_t* kp = a.kpages + kpage_off(g, prow[min(4 * sb + (i16 >> 2), pages_all - 1)], kvh, 0, 4 * lg + (i16 & 3));
         u32x4 kr[2][8];
+        auto fetch = [&](int k, int b) {
 #pragma unroll
-        for (int t = 0; t < 8; ++t) kr[0][t] = *reinterpret_cast<const u32x4*>(kp + t * 32);
-#pragma unroll
-        for (int b = 0; b < NB; ++b) {
-          if (b + 1 < NB) {                              // the next 32 d fly while these are multiplied
-#pragma unroll
-            for (int t = 0; t < 8; ++t) kr[(b + 1) & 1][t] = *reinterpret_cast<const u32x4*>(kp + (b + 1) * 1024 + t * 32);
-          }
-          float q8[8];
-#pragma unroll
-          for (int s = 0; s < 8; ++s) q8[s] = qs[(8 * b + s) * 64 + lane];
+          for (int t = 0; t < 8; ++t) kr[k][t] = *reinterpret_cast<const u32x4*>(kp + b * 1024 + (t >> 1) * 256 + (t & 1) * 128);
+        };
+        auto products = [&](int k, int b) {              // 32 d of 128 keys, eight d's operands at a time: the scores need the registers
           __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-          for (int t = 0; t < 8; t += 2) {
+          for (int c = 0; c < 4; ++c) {
+            const float* q = qs + i16 * QP + b * 32 + c * 8;
+            const float4 q0 = *reinterpret_cast<const float4*>(q), q1 = *reinterpret_cast<const float4*>(q + 4);
+            const float q8[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
             float x[8], y[8];
-            ixt_k_operands(kr[b & 1][t], sel, x);
-            ixt_k_operands(kr[b & 1][t + 1], sel, y);
+#pragma unroll
+            for (int s = 0; s < 8; ++s) {
+              x[s] = s & 1 ? bfhi(kr[k][2 * c][s >> 1]) : bflo(kr[k][2 * c][s >> 1]);
+              y[s] = s & 1 ? bfhi(kr[k][2 * c + 1][s >> 1]) : bflo(kr[k][2 * c + 1][s >> 1]);
+              asm volatile("" : "+v"(x[s]), "+v"(y[s]));
+            }
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int s = 0; s < 8; ++s) {
-              S[n][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[s], q8[s], S[n][t], 0, 0, 0);
-              S[n][t + 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(y[s], q8[s], S[n][t + 1], 0, 0, 0);
+              S[n][0] = __builtin_amdgcn_mfma_f32_16x16x1f32(x[s], q8[s], S[n][0], 0, 0, 0);
+              S[n][1] = __builtin_amdgcn_mfma_f32_16x16x1f32(y[s], q8[s], S[n][1], 0, 0, 0);
             }
-            __builtin_amdgcn_sched_barrier(0);           // two tiles' operands at a time: the scores need the registers
+            __builtin_amdgcn_sched_barrier(0);
           }
+        };
+        fetch(0, 0);
+        fetch(1, 1);
+#pragma unroll 1
+        for (int b = 2; b < NB; b += 2) {                // the next 32 d fly while these are multiplied
+          products(0, b - 2);
+          fetch(0, b);
+          products(1, b - 1);
+          fetch(1, b + 1);
         }
+        products(0, NB - 2);
+        products(1, NB - 1);
         // lane (vector i16, group lg): register r of tile t is token 4 t + r of page 4 sb + lg
         const int lim = mypos - sb * 128 - lg * 32, lo = a.window > 0 ? lim - a.window : -1;
         if (a.cap > 0.0f) {
 #pragma unroll
           for (int t = 0; t < 8; ++t) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) S[n][t][r] = ixt_tanh(S[n][t][r] / a.cap) * a.cap;
+            for (int r = 0; r < 4; ++r) S[n][t >> 2][4 * (t & 3) + r] = ixt_tanh(S[n][t >> 2][4 * (t & 3) + r] / a.cap) * a.cap;
             __builtin_amdgcn_sched_barrier(0);
           }
         }
@@ -191,8 +193,8 @@ __global__ __launch_bounds__(NW * 64, NR == 1 && NW <= 4 ? 3 : 2) void k_attn_mt
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
               const int k = 4 * t + r;
-              mn = fminf(mn, S[n][t][r]);
-              mx = fmaxf(mx, !masked.value || (k <= lim && k > lo) ? S[n][t][r] : -INFINITY);
+              mn = fminf(mn, S[n][t >> 2][4 * (t & 3) + r]);
+              mx = fmaxf(mx, !masked.value || (k <= lim && k > lo) ? S[n][t >> 2][4 * (t & 3) + r] : -INFINITY);
             }
             __builtin_amdgcn_sched_barrier(0);
           }
@@ -220,9 +222,9 @@ __global__ __launch_bounds__(NW * 64, NR == 1 && NW <= 4 ? 3 : 2) void k_attn_mt
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
               const int k = 4 * t + r;
-              const float e = ixt_exp(S[n][t][r] - mx);
-              S[n][t][r] = !masked.value || (k <= lim && k > lo) ? e : 0.0f;
-              sacc = sacc + S[n][t][r];
+              const float e = ixt_exp(S[n][t >> 2][4 * (t & 3) + r] - mx);
+              S[n][t >> 2][4 * (t & 3) + r] = !masked.value || (k <= lim && k > lo) ? e : 0.0f;
+              sacc = sacc + S[n][t >> 2][4 * (t & 3) + r];
             }
             __builtin_amdgcn_sched_barrier(0);
           }
@@ -249,7 +251,7 @@ __global__ __launch_bounds__(NW * 64, NR == 1 && NW <= 4 ? 3 : 2) void k_attn_mt
 #pragma unroll
           for (int t = 0; t < 8; ++t) {
             // bf16 pairs of tokens of the lane's page -> pairs of pages, lane group = token
-            uint32_t u = pack2(f2bf(quotient(S[n][t][0])), f2bf(quotient(S[n][t][1]))), v = pack2(f2bf(quotient(S[n][t][2])), f2bf(quotient(S[n][t][3])));
+            uint32_t u = pack2(f2bf(quotient(S[n][t >> 2][4 * (t & 3) + 0])), f2bf(quotient(S[n][t >> 2][4 * (t & 3) + 1]))), v = pack2(f2bf(quotient(S[n][t >> 2][4 * (t & 3) + 2])), f2bf(quotient(S[n][t >> 2][4 * (t & 3) + 3])));
             ixt_swap32(u, v);                            // u: pages 0, 1, v: pages 2, 3; lane groups 0, 1: tokens 0 and 1, 2, 3: tokens 2 and 3
             uint32_t u1 = u, v1 = v;
             ixt_swap16(u, u1);
@@ -269,9 +271,15 @@ __global__ __launch_bounds__(NW * 64, NR == 1 && NW <= 4 ? 3 : 2) void k_attn_mt
     });
     // ---- outputs
     for (int part = part0; part < HD / VW; part += a.parts) {
-      float tot[2][NTOT];
+      float tot[NTOT];
+      int nsb_t[NTOT];                                   // super-blocks of the total's row
 #pragma unroll
-      for (int k = 0; k < NTOT; ++k) { tot[0][k] = 0.0f; tot[1][k] = 0.0f; }
+      for (int k = 0; k < NTOT; ++k) {
+        const int v = (tid + k * NW * 64) / VW;
+        tot[k] = 0.0f;
+        nsb_t[k] = ((grp >> (v / GQ)) & 1u) ? (((s_pos[v / GQ] + 32) >> 5) + IXT_SB - 1) / IXT_SB : 0;
+      }
+      const int nsb_min = (((posmin + 32) >> 5) + IXT_SB - 1) / IXT_SB;
 #pragma unroll
       for (int n = 0; n < NR; ++n) {
         if (n * NW >= nsb) break;
@@ -340,34 +348,36 @@ __global__ __launch_bounds__(NW * 64, NR == 1 && NW <= 4 ? 3 : 2) void k_attn_mt
           }
         }
         // lane: vector i16, columns NE (4 lg + r) + x
+        float* const buf = ob + (NBUF == 2 ? n & 1 : 0) * NW * 16 * OP;
+        if (NBUF == 1) __syncthreads();
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          __syncthreads();
+        for (int r = 0; r < 4; ++r)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            float* o = ob + (wave * 16 + i16) * OP + (4 * lg + r) * NEH;
-            if constexpr (NEH == 4) *reinterpret_cast<float4*>(o) = make_float4(ss[h * NEH][r], ss[h * NEH + 1][r], ss[h * NEH + 2][r], ss[h * NEH + 3][r]);
-            else *reinterpret_cast<float2*>(o) = make_float2(ss[h * NEH][r], ss[h * NEH + 1][r]);
-          }
-          __syncthreads();
+          for (int x = 0; x < NE; x += 4) *reinterpret_cast<float4*>(buf + (wave * 16 + i16) * OP + (4 * lg + r) * NE + x) = make_float4(ss[x][r], ss[x + 1][r], ss[x + 2][r], ss[x + 3][r]);
+        __syncthreads();
+        if ((n + 1) * NW <= nsb_min) {                   // every row has all of the round
 #pragma unroll
           for (int k = 0; k < NTOT; ++k) {
-            const int idx = tid + k * NW * 64, v = idx / CH, c = idx % CH;
-            const int nsb_v = ((grp >> (v / GQ)) & 1u) ? (((s_pos[v / GQ] + 32) >> 5) + IXT_SB - 1) / IXT_SB : 0;
+            const int idx = tid + k * NW * 64, at = idx / VW * OP + idx % VW;
+#pragma unroll
+            for (int w = 0; w < NW; ++w) tot[k] = tot[k] + buf[w * 16 * OP + at];
+          }
+        } else {
+#pragma unroll
+          for (int k = 0; k < NTOT; ++k) {
+            const int idx = tid + k * NW * 64, at = idx / VW * OP + idx % VW;
 #pragma unroll
             for (int w = 0; w < NW; ++w)
-              if (n * NW + w < nsb_v) tot[h][k] = tot[h][k] + ob[(w * 16 + v) * OP + c];
+              if (n * NW + w < nsb_t[k]) tot[k] = tot[k] + buf[w * 16 * OP + at];
           }
         }
       }
 #pragma unroll
-      for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int k = 0; k < NTOT; ++k) {
-          const int idx = tid + k * NW * 64, v = idx / CH, c = idx % CH;
-          const int d = part * VW + c / NEH * NE + h * NEH + c % NEH;
-          if ((grp >> (v / GQ)) & 1u) a.out[xidx(r0 + v / GQ, (kvh * GQ + v % GQ) * HD + d, n_out)] = f2bf(tot[h][k]);
-        }
+      for (int k = 0; k < NTOT; ++k) {
+        const int idx = tid + k * NW * 64, v = idx / VW, c = idx % VW;
+        if ((grp >> (v / GQ)) & 1u) a.out[xidx(r0 + v / GQ, (kvh * GQ + v % GQ) * HD + part * VW + c, n_out)] = f2bf(tot[k]);
+      }
+      if (NBUF == 2 && part + a.parts < HD / VW) __syncthreads();      // (the next part's first buffer may be this one's last)
     }
     __syncthreads();                                     // the LDS arrays are reused by the next group
   }

@@ -3,6 +3,13 @@
 
 #include <algorithm>
 
+template <int HD, int GQ, int NW, int NR>
+static void mtile_launch(const dim3& grid, const TileAttnArgs& ta, hipStream_t st) {
+  constexpr size_t lds = mtile_lds(HD, NW, NR);
+  static const hipError_t room = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_attn_mtile<HD, GQ, NW, NR>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  (void)room;                                            // (a launch without room for its LDS fails, and the caller looks at that)
+  hipLaunchKernelGGL((k_attn_mtile<HD, GQ, NW, NR>), grid, dim3(NW * 64), lds, st, ta);
+}
 // The smallest form that holds the call's longest prefix (ta.lmax keys, at most 4096).
 template <int HD, int GQ>
 static void mtile_attn_t(TileAttnArgs ta, hipStream_t st) {
@@ -13,17 +20,17 @@ static void mtile_attn_t(TileAttnArgs ta, hipStream_t st) {
   // took 2.40 ms a step of four sub-layers (per-vector units: 2.35), dealt out 1.84; 16 heads of 128, four layers: 64 keys 2.45 -> 1.77, 1500 keys 4.50 -> 2.58
   ta.parts = HD > 128 && blocks <= 128 ? HD / 128 : 1;
   const dim3 grid(ta.g.nkv, tiles, ta.parts * std::min(TQ, std::max(1, 256 / (blocks * ta.parts))));
-  if (ta.lmax <= 256) hipLaunchKernelGGL((k_attn_mtile<HD, GQ, 2, 1>), grid, dim3(128), 0, st, ta);
-  else if (ta.lmax <= 512) hipLaunchKernelGGL((k_attn_mtile<HD, GQ, 4, 1>), grid, dim3(256), 0, st, ta);
+  if (ta.lmax <= 256) mtile_launch<HD, GQ, 2, 1>(grid, ta, st);
+  else if (ta.lmax <= 512) mtile_launch<HD, GQ, 4, 1>(grid, ta, st);
   // more than one block a CU: two of four waves side by side (256 registers a wave; one block's softmax and exchange under the other's products), else all the waves a CU has room
   // for in one.  16 heads of 128 at <= 1024 keys, us of <8, 1> / <4, 2>: 256 blocks 32.0 / 37.8, 320 61.2 / 57.9, 512 64.0 / 58.1, 1024 105 / 88.  With twice the keys two blocks' scores
   // take every register: level
-  else if (ta.lmax <= 1024 && (int)(grid.x * grid.y * ta.parts) > 256) hipLaunchKernelGGL((k_attn_mtile<HD, GQ, 4, 2>), grid, dim3(256), 0, st, ta);
-  else if (ta.lmax <= 1024) hipLaunchKernelGGL((k_attn_mtile<HD, GQ, 8, 1>), grid, dim3(512), 0, st, ta);
-  else if (ta.lmax <= 2048) hipLaunchKernelGGL((k_attn_mtile<HD, GQ, 8, 2>), grid, dim3(512), 0, st, ta);
+  else if (ta.lmax <= 1024 && (int)(grid.x * grid.y * ta.parts) > 256) mtile_launch<HD, GQ, 4, 2>(grid, ta, st);
+  else if (ta.lmax <= 1024) mtile_launch<HD, GQ, 8, 1>(grid, ta, st);
+  else if (ta.lmax <= 2048) mtile_launch<HD, GQ, 8, 2>(grid, ta, st);
   // (the scores of three rounds leave registers that those of four do not: 1024 rows at <= 3072 keys 322 -> 302 us)
-  else if (ta.lmax <= 3072) hipLaunchKernelGGL((k_attn_mtile<HD, GQ, 8, 3>), grid, dim3(512), 0, st, ta);
-  else hipLaunchKernelGGL((k_attn_mtile<HD, GQ, 8, 4>), grid, dim3(512), 0, st, ta);
+  else if (ta.lmax <= 3072) mtile_launch<HD, GQ, 8, 3>(grid, ta, st);
+  else mtile_launch<HD, GQ, 8, 4>(grid, ta, st);
 }
 bool launch_mtile_attn(const TileAttnArgs& ta, int hd, int gq, hipStream_t st) {
 #define ATT(HD_, GQ_) if (hd == HD_ && gq == GQ_) { mtile_attn_t<HD_, GQ_>(ta, st); return true; }
