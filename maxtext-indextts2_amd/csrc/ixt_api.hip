@@ -312,7 +312,8 @@ extern "C" int ixt_create(const ixt_config* cfg, ixt_ctx** out) {
     x->part_floats = full > split ? full : split;
     A(dmalloc(x, &x->part, x->part_floats));
   }
-  A(dmalloc(x, &x->scores, (size_t)R * x->Q * x->Tmax));
+  // (whole tiles of 16 query vectors and whole super-blocks of keys: k_attn_mscores)
+  A(dmalloc(x, &x->scores, (size_t)((R + 15) & ~15) * x->Q * ((x->Tmax + 127) & ~127)));
   A(dmalloc(x, &x->pvpart, (size_t)R * x->Q * x->nsb_max * x->D));
   x->amax_cap = (size_t)x->NLmax * std::max(4, (V + 15) / 16);   // (ring_pairs)
   A(dmalloc(x, &x->amax_val, x->amax_cap));
@@ -1271,6 +1272,7 @@ static int launch_attention_tile(ixt_ctx* c, int layer, int R, int len_hint, hip
     TileAttnArgs ta;
     ta.row_slot = c->row_slot; ta.row_pos = c->row_pos; ta.row_active = c->row_active; ta.page_map = c->ps.page_map;
     ta.qbuf = c->qbuf; ta.kpages = c->kpages_l[layer]; ta.vpages = c->vpages_l[layer]; ta.out = c->ao; ta.g = c->geom; ta.R = R; ta.lmax = lmax; ta.cap = cap; ta.window = window;
+    ta.scores = c->one_segment ? c->scores : nullptr;
     if (launch_mtile_attn(ta, c->D, c->GQ, st)) { LAUNCHCHK(); return IXT_OK; }
   }
   const bool wide = tile_attn_lds(c, 16, lmax) <= 150 * 1024 && c->D <= 128;   // (head_dim 256 with 16 vectors: 100+ bytes of scratch per lane)

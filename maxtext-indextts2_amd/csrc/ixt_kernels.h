@@ -1733,6 +1733,7 @@ struct TileAttnArgs {
   float cap;                          // > 0: score = ixt_tanh(score / cap) * cap before the max (attn_logits_soft_cap, attentions.py:1257-1259), as k_attn_pv
   int window;                         // > 0: keys j <= pos - window are invisible (LOCAL_SLIDING, attentions.py:625-631): e_j = p_j = +0, every sum unchanged
   int parts;                          // k_attn_mtile: blocks that share a value's columns
+  float* scores;                      // k_attn_mscores: its output, as many floats as row blocks of 16 vectors x keys (of whole super-blocks); nullptr: the rows are of several page groups
 };
 bool launch_mtile_attn(const TileAttnArgs& ta, int hd, int gq, hipStream_t st);   // ixt_tile_attn.hip; false: no such head geometry
 typedef uint32_t ixt_u32x16 __attribute__((ext_vector_type(16)));

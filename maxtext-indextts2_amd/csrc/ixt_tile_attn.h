@@ -22,6 +22,51 @@ __device__ __forceinline__ void ixt_swap32(uint32_t& a, uint32_t& b) {
   a = r[0]; b = r[1];
 }
 
+// The scores of a super-block: 128 keys against 16 query vectors.  kp: token 4 lg + i16 % 4 of page i16 / 4 of it; q: the lane's vector in LDS.  Register 4 (t % 4) + r of half t / 4: token
+// 4 t + r of the lane's page (page lg), vector i16.
+template <int HD>
+__device__ __forceinline__ void mtile_scores(const bf16_t* kp, const float* q, ixt_f32x16& S0, ixt_f32x16& S1) {
+  constexpr int NB = HD / 32;
+  u32x4 kr[2][8];
+  auto fetch = [&](int k, int b) {
+#pragma unroll
+    for (int t = 0; t < 8; ++t) kr[k][t] = *reinterpret_cast<const u32x4*>(kp + b * 1024 + (t >> 1) * 256 + (t & 1) * 128);
+  };
+  auto products = [&](int k, int b) {              // 32 d of 128 keys, eight d's operands at a time: the scores need the registers
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const float* qp = q + b * 32 + c * 8;
+      const float4 q0 = *reinterpret_cast<const float4*>(qp), q1 = *reinterpret_cast<const float4*>(qp + 4);
+      const float q8[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
+      float x[8], y[8];
+#pragma unroll
+      for (int s = 0; s < 8; ++s) {
+        x[s] = s & 1 ? bfhi(kr[k][2 * c][s >> 1]) : bflo(kr[k][2 * c][s >> 1]);
+        y[s] = s & 1 ? bfhi(kr[k][2 * c + 1][s >> 1]) : bflo(kr[k][2 * c + 1][s >> 1]);
+        asm volatile("" : "+v"(x[s]), "+v"(y[s]));
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int s = 0; s < 8; ++s) {
+        S0 = __builtin_amdgcn_mfma_f32_16x16x1f32(x[s], q8[s], S0, 0, 0, 0);
+        S1 = __builtin_amdgcn_mfma_f32_16x16x1f32(y[s], q8[s], S1, 0, 0, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  fetch(0, 0);
+  fetch(1, 1);
+#pragma unroll 1
+  for (int b = 2; b < NB; b += 2) {                // the next 32 d fly while these are multiplied
+    products(0, b - 2);
+    fetch(0, b);
+    products(1, b - 1);
+    fetch(1, b + 1);
+  }
+  products(0, NB - 2);
+  products(1, NB - 1);
+}
 // block = (kv head, 16 query vectors = 16 / GQ consecutive rows x GQ heads), NW waves.  Super-block (4 pages, 128 keys) n NW + w belongs to wave w in
 // round n; its 128 x 16 scores stay in that wave's registers from the score products to the output products, so the keys one block holds are
 // 128 NW NR and nothing of them goes through LDS or memory.
@@ -51,14 +96,71 @@ __device__ __forceinline__ void ixt_swap32(uint32_t& a, uint32_t& b) {
 // Measured against k_attn_tile, 16 heads of 128, 1024 rows at <= 1024 / 2048 / 3072 keys 282 / 860 / 1143 us, before the scores' 16x16x1 products and the exchange with one barrier
 // 92 / 212 / 310, now 87 / 198 / 293.  828 rows at <= 3900 keys 1496, 408, 375 us (63 TFLOP/s).  8 heads of 256 on 4, 256 rows at <= 1756 / 2756 keys: 88 / 131, 79 / 117 us.
 // Prompts of <= 256 keys: two waves per block; with four, two of them had nothing to do (eight packed ones, 1525 rows: 90.2 us against 67.6).
+__device__ __forceinline__ void mtile_cap(ixt_f32x16& S0, ixt_f32x16& S1, float cap) {
+#pragma unroll
+  for (int k = 0; k < 16; ++k) {
+    S0[k] = ixt_tanh(S0[k] / cap) * cap;
+    S1[k] = ixt_tanh(S1[k] / cap) * cap;
+    if ((k & 1) == 1) __builtin_amdgcn_sched_barrier(0);
+  }
+}
+// Where a launch's (kv head, tile) blocks leave half of the CUs idle, the scores go ahead of it in a launch of their own, a tile's super-blocks dealt among gridDim.z blocks, and
+// k_attn_mtile<.., GIVEN> finds them in memory, 8 KiB a super-block, as its lanes hold them: two blocks that share a value's columns no longer take every score both (Gemma-2 2B, 3000
+// tokens by 256: 22.1 ms of attention launches of more than 512 keys, now 7.2 of scores and 10.4 of values).  The rows of a tile are of one page group (the caller's promise: one segment), idle ones among them.
+__device__ __forceinline__ size_t mscores_at(const TileAttnArgs& a, int tile, int kvh, int sb) {
+  return (((size_t)tile * a.g.nkv + kvh) * ((a.lmax + 127) >> 7) + sb) * 2048;
+}
+template <int HD, int GQ>
+__global__ __launch_bounds__(512, 2) void k_attn_mscores(TileAttnArgs a) {
+  constexpr int TQ = 16 / GQ, QP = HD + 4, NW = 8;
+  __shared__ __attribute__((aligned(16))) float qs[16 * QP];
+  __shared__ int s_pos[TQ], s_slot[TQ];
+  const AttnGeom& g = a.g;
+  const int kvh = blockIdx.x, r0 = (gridDim.y - 1 - blockIdx.y) * TQ;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, i16 = lane & 15, lg = lane >> 4;
+  if (tid < TQ) {
+    const int r = r0 + tid;
+    const bool ok = r < a.R && a.row_active[r] != 0;
+    s_pos[tid] = ok ? a.row_pos[r] : -1;
+    s_slot[tid] = ok ? a.row_slot[r] : -1;
+  }
+  for (int it = tid; it < 16 * (HD / 8); it += NW * 64) {
+    const int v = it & 15, c = it >> 4;
+    const u32x4 w = *reinterpret_cast<const u32x4*>(a.qbuf + ((size_t)min(r0 + v / GQ, a.R - 1) * g.nq + kvh * GQ + v % GQ) * HD + c * 8);
+    float4* q = reinterpret_cast<float4*>(qs + v * QP + c * 8);
+    q[0] = make_float4(bflo(w[0]), bfhi(w[0]), bflo(w[1]), bfhi(w[1]));
+    q[1] = make_float4(bflo(w[2]), bfhi(w[2]), bflo(w[3]), bfhi(w[3]));
+  }
+  __syncthreads();
+  int posmax = -1, slot = 0;
+#pragma unroll
+  for (int i = 0; i < TQ; ++i) {
+    const int ps = __builtin_amdgcn_readfirstlane(s_pos[i]);
+    if (ps >= 0 && ps < a.lmax && ps > posmax) { posmax = ps; slot = __builtin_amdgcn_readfirstlane(s_slot[i]); }
+  }
+  if (posmax < 0) return;
+  const int pages_all = (posmax + 32) >> 5, nsb = (pages_all + IXT_SB - 1) / IXT_SB;
+  const int32_t* prow = a.page_map + (size_t)slot * g.mpg;
+  for (int sb = wave * gridDim.z + blockIdx.z; sb < nsb; sb += NW * gridDim.z) {
+    ixt_f32x16 S0 = ixt_f32x16(0.0f), S1 = ixt_f32x16(0.0f);
+    mtile_scores<HD>(a.kpages + kpage_off(g, prow[min(4 * sb + (i16 >> 2), pages_all - 1)], kvh, 0, 4 * lg + (i16 & 3)), qs + i16 * QP, S0, S1);
+    if (a.cap > 0.0f) mtile_cap(S0, S1, a.cap);
+    float4* sp = reinterpret_cast<float4*>(a.scores + mscores_at(a, r0 / TQ, kvh, sb)) + lane;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      sp[k * 64] = make_float4(S0[4 * k], S0[4 * k + 1], S0[4 * k + 2], S0[4 * k + 3]);
+      sp[(4 + k) * 64] = make_float4(S1[4 * k], S1[4 * k + 1], S1[4 * k + 2], S1[4 * k + 3]);
+    }
+  }
+}
 // Buffers of the exchange: with two a round has one barrier (another one's sums are read while the next is written); one where there is one round, or where two
 // would take a CU's second block away.
 constexpr int mtile_buffers(int hd, int nw, int nr) { return nr > 1 && (nw == 8 || hd <= 128) ? 2 : 1; }
 constexpr size_t mtile_lds(int hd, int nw, int nr) { return (size_t)mtile_buffers(hd, nw, nr) * nw * 16 * ((hd >= 128 ? 128 : hd) + 4) * 4; }
-template <int HD, int GQ, int NW, int NR>
+// GIVEN: the scores are in memory (k_attn_mscores, the same rows)
+template <int HD, int GQ, int NW, int NR, bool GIVEN = false>
 __global__ __launch_bounds__(NW * 64, NR == 1 && NW <= 4 ? 3 : 2) void k_attn_mtile(TileAttnArgs a) {
   constexpr int TQ = 16 / GQ;
-  constexpr int NB = HD / 32;
   constexpr int VW = HD >= 128 ? 128 : HD;     // value columns of one output pass
   constexpr int NE = VW / 16;                  // matrix tiles of them
   constexpr int OP = VW + 4, NTOT = 16 * VW / (NW * 64);       // a vector's pitch of the exchange; (vector, column) totals per thread
@@ -81,7 +183,7 @@ __global__ __launch_bounds__(NW * 64, NR == 1 && NW <= 4 ? 3 : 2) void k_attn_mt
     s_pos[tid] = ok ? a.row_pos[r] : -1;
     s_slot[tid] = ok ? a.row_slot[r] : -1;
   }
-  for (int it = tid; it < 16 * (HD / 8); it += NW * 64) {
+  for (int it = GIVEN ? 16 * (HD / 8) : tid; it < 16 * (HD / 8); it += NW * 64) {
     const int v = it & 15, c = it >> 4;
     const u32x4 w = *reinterpret_cast<const u32x4*>(a.qbuf + ((size_t)min(r0 + v / GQ, a.R - 1) * g.nq + kvh * GQ + v % GQ) * HD + c * 8);
     float4* q = reinterpret_cast<float4*>(qs + v * QP + c * 8);
@@ -136,57 +238,19 @@ __global__ __launch_bounds__(NW * 64, NR == 1 && NW <= 4 ? 3 : 2) void k_attn_mt
       const int sb = n * NW + wave;
       S[n][0] = S[n][1] = ixt_f32x16(0.0f);
       if (sb < nsb) {
-        // lane (i16, lg) loads token 4 t + i16 % 4 of page i16 / 4, t = lg and 4 + lg
-        const bf16_t* kp = a.kpages + kpage_off(g, prow[min(4 * sb + (i16 >> 2), pages_all - 1)], kvh, 0, 4 * lg + (i16 & 3));
-        u32x4 kr[2][8];
-        auto fetch = [&](int k, int b) {
+        if constexpr (GIVEN) {
+          const float4* sp = reinterpret_cast<const float4*>(a.scores + mscores_at(a, r0 / TQ, kvh, sb)) + lane;
 #pragma unroll
-          for (int t = 0; t < 8; ++t) kr[k][t] = *reinterpret_cast<const u32x4*>(kp + b * 1024 + (t >> 1) * 256 + (t & 1) * 128);
-        };
-        auto products = [&](int k, int b) {              // 32 d of 128 keys, eight d's operands at a time: the scores need the registers
-          __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-          for (int c = 0; c < 4; ++c) {
-            const float* q = qs + i16 * QP + b * 32 + c * 8;
-            const float4 q0 = *reinterpret_cast<const float4*>(q), q1 = *reinterpret_cast<const float4*>(q + 4);
-            const float q8[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
-            float x[8], y[8];
-#pragma unroll
-            for (int s = 0; s < 8; ++s) {
-              x[s] = s & 1 ? bfhi(kr[k][2 * c][s >> 1]) : bflo(kr[k][2 * c][s >> 1]);
-              y[s] = s & 1 ? bfhi(kr[k][2 * c + 1][s >> 1]) : bflo(kr[k][2 * c + 1][s >> 1]);
-              asm volatile("" : "+v"(x[s]), "+v"(y[s]));
-            }
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int s = 0; s < 8; ++s) {
-              S[n][0] = __builtin_amdgcn_mfma_f32_16x16x1f32(x[s], q8[s], S[n][0], 0, 0, 0);
-              S[n][1] = __builtin_amdgcn_mfma_f32_16x16x1f32(y[s], q8[s], S[n][1], 0, 0, 0);
-            }
-            __builtin_amdgcn_sched_barrier(0);
+          for (int k = 0; k < 8; ++k) {
+            const float4 v = sp[k * 64];
+            S[n][k >> 2][4 * (k & 3)] = v.x; S[n][k >> 2][4 * (k & 3) + 1] = v.y; S[n][k >> 2][4 * (k & 3) + 2] = v.z; S[n][k >> 2][4 * (k & 3) + 3] = v.w;
           }
-        };
-        fetch(0, 0);
-        fetch(1, 1);
-#pragma unroll 1
-        for (int b = 2; b < NB; b += 2) {                // the next 32 d fly while these are multiplied
-          products(0, b - 2);
-          fetch(0, b);
-          products(1, b - 1);
-          fetch(1, b + 1);
+        } else {
+          mtile_scores<HD>(a.kpages + kpage_off(g, prow[min(4 * sb + (i16 >> 2), pages_all - 1)], kvh, 0, 4 * lg + (i16 & 3)), qs + i16 * QP, S[n][0], S[n][1]);
+          if (a.cap > 0.0f) mtile_cap(S[n][0], S[n][1], a.cap);
         }
-        products(0, NB - 2);
-        products(1, NB - 1);
         // lane (vector i16, group lg): register r of tile t is token 4 t + r of page 4 sb + lg
         const int lim = mypos - sb * 128 - lg * 32, lo = a.window > 0 ? lim - a.window : -1;
-        if (a.cap > 0.0f) {
-#pragma unroll
-          for (int t = 0; t < 8; ++t) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) S[n][t >> 2][4 * (t & 3) + r] = ixt_tanh(S[n][t >> 2][4 * (t & 3) + r] / a.cap) * a.cap;
-            __builtin_amdgcn_sched_barrier(0);
-          }
-        }
         auto range = [&](auto masked) {
 #pragma unroll
           for (int t = 0; t < 8; ++t) {

@@ -3,12 +3,12 @@
 
 #include <algorithm>
 
-template <int HD, int GQ, int NW, int NR>
+template <int HD, int GQ, int NW, int NR, bool GIVEN = false>
 static void mtile_launch(const dim3& grid, const TileAttnArgs& ta, hipStream_t st) {
   constexpr size_t lds = mtile_lds(HD, NW, NR);
-  static const hipError_t room = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_attn_mtile<HD, GQ, NW, NR>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  static const hipError_t room = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_attn_mtile<HD, GQ, NW, NR, GIVEN>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   (void)room;                                            // (a launch without room for its LDS fails, and the caller looks at that)
-  hipLaunchKernelGGL((k_attn_mtile<HD, GQ, NW, NR>), grid, dim3(NW * 64), lds, st, ta);
+  hipLaunchKernelGGL((k_attn_mtile<HD, GQ, NW, NR, GIVEN>), grid, dim3(NW * 64), lds, st, ta);
 }
 // The smallest form that holds the call's longest prefix (ta.lmax keys, at most 4096).
 template <int HD, int GQ>
@@ -20,6 +20,18 @@ static void mtile_attn_t(TileAttnArgs ta, hipStream_t st) {
   // took 2.40 ms a step of four sub-layers (per-vector units: 2.35), dealt out 1.84; 16 heads of 128, four layers: 64 keys 2.45 -> 1.77, 1500 keys 4.50 -> 2.58
   ta.parts = HD > 128 && blocks <= 128 ? HD / 128 : 1;
   const dim3 grid(ta.g.nkv, tiles, ta.parts * std::min(TQ, std::max(1, 256 / (blocks * ta.parts))));
+  // two blocks a value and rows of one page group: the scores once, by a launch of their own on all CUs (256 rows, 8 heads of 256 on 4, <= 1024 / 2048 / 3072 keys: 45.6,
+  // 74.3, 112 us, now 22.0, 33.6, 54.6 and the scores before them, 27.0 in the mean; at <= 512 keys the second launch costs what it gives)
+  if constexpr (HD > 128) {
+    if (ta.parts > 1 && ta.scores != nullptr && ta.lmax > 512) {
+      hipLaunchKernelGGL((k_attn_mscores<HD, GQ>), dim3(ta.g.nkv, tiles, std::min(8, std::max(2, 256 / blocks))), dim3(512), 0, st, ta);
+      if (ta.lmax <= 1024) mtile_launch<HD, GQ, 8, 1, true>(grid, ta, st);
+      else if (ta.lmax <= 2048) mtile_launch<HD, GQ, 8, 2, true>(grid, ta, st);
+      else if (ta.lmax <= 3072) mtile_launch<HD, GQ, 8, 3, true>(grid, ta, st);
+      else mtile_launch<HD, GQ, 8, 4, true>(grid, ta, st);
+      return;
+    }
+  }
   if (ta.lmax <= 256) mtile_launch<HD, GQ, 2, 1>(grid, ta, st);
   else if (ta.lmax <= 512) mtile_launch<HD, GQ, 4, 1>(grid, ta, st);
   // more than one block a CU: two of four waves side by side (256 registers a wave; one block's softmax and exchange under the other's products), else all the waves a CU has room

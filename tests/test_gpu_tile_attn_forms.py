@@ -23,7 +23,8 @@ def test_two_blocks_a_cu(model, hd, nq, nkv, window, option, length, chunk):
   _same(_prefill_long(cfg, w, toks, chunk, {option: 1, "attn_tile_min_rows": 1}), _prefill_long(cfg, w, toks, chunk, {option: 0}))
 
 
-@pytest.mark.parametrize("nq,nkv,window,length,chunk", [(8, 4, 4096, 3330, 256), (8, 4, 700, 3330, 250), (4, 4, 2100, 3072, 256), (8, 2, 4096, 3073, 130)])
+@pytest.mark.parametrize("nq,nkv,window,length,chunk", [(8, 4, 4096, 3330, 256), (8, 4, 700, 3330, 250), (4, 4, 2100, 3072, 256), (8, 2, 4096, 3073, 130),
+                                                        (8, 4, 4096, 1025, 40), (4, 4, 30, 545, 17)])
 def test_heads_of_256_at_many_keys(nq, nkv, window, length, chunk):
   cfg = H.make_config(model_name="gemma2-tiny", override_model_config=True, head_dim=256, base_num_query_heads=nq, base_num_kv_heads=nkv, sliding_window_size=window,
                       base_num_decoder_layers=1, per_device_batch_size=1.0, use_chunked_prefill=True, prefill_chunk_size=256, max_prefill_predict_length=256,
