@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 typedef uint16_t bf16_t;
 
 #define IXT_MK 32      // k per matrix instruction (v_mfma_f32_16x16x32_bf16)
@@ -196,3 +198,25 @@ __device__ __forceinline__ void ixt_gave_up(const IxtWait& w) {
 // agent-scope (L1-bypassing) accesses for state one wave re-reads after writing it
 __device__ __forceinline__ int ldg_i32(const int32_t* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ __forceinline__ void stg_i32(int32_t* p, int v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+
+// v of the lane 1, 2, 4, 8, 16, 32 away combined with this lane's, in the order of the xor-butterfly of the canonical sums: from 4 on the lanes of a group hold the same
+// value already, so that any lane of the other group will do (row_half_mirror, row_mirror, swaps of rows and halves), and no step goes through LDS.
+template <typename F> __device__ __forceinline__ float xor_butterfly(float v, F f) {
+  auto dpp = [](float x, auto ctrl) { return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), decltype(ctrl)::value, 0xf, 0xf, true)); };
+  v = f(v, dpp(v, std::integral_constant<int, 0xb1>()));           // quad_perm 1 0 3 2
+  v = f(v, dpp(v, std::integral_constant<int, 0x4e>()));           // quad_perm 2 3 0 1
+  v = f(v, dpp(v, std::integral_constant<int, 0x141>()));          // row_half_mirror
+  v = f(v, dpp(v, std::integral_constant<int, 0x140>()));          // row_mirror
+  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = f(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return f(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+__device__ __forceinline__ float xor_sum(float v) { return xor_butterfly(v, [](float x, float y) { return x + y; }); }
+
+// The row of block b where a block takes a row of R and writes it to an operand (xidx: 16 bytes of a line of eight rows at a time): the eight rows of a line go to blocks that the
+// dispatcher deals to one XCD, so that its L2 holds the line whole when it is written back (with
+// sums over the lanes that need no LDS, us before / now: k_rownorm of 1592 rows of 2048 7.8 / 5.9, of 1024 6.5 / 5.2; k_gnorm of 256 rows of 2304 6.3 / 5.1).
+__device__ __forceinline__ int row_of_block(int b, int R) {
+  return (b | 63) < R ? (b & ~63) + (b & 7) * 8 + (b >> 3 & 7) : b;
+}

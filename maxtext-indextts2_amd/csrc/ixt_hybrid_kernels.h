@@ -70,11 +70,7 @@ struct Slices {             // a dot's output; bias: one number per column joins
   __host__ __device__ __forceinline__ Slices from(int c) const { Slices s = *this; s.p += c; if (bias != nullptr) s.bias += c; return s; }
 };
 
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) v += __shfl_xor(v, off, 64);
-  return v;
-}
+__device__ __forceinline__ float wave_sum(float v) { return xor_sum(v); }
 // sum over the 16 lanes of a DPP row, every lane ends up with it
 __device__ __forceinline__ float row16_sum(float v) {
   v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128, 0xf, 0xf, false));   // row_ror:8

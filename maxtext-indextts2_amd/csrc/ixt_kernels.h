@@ -638,7 +638,7 @@ __global__ __launch_bounds__(256) void k_rownorm(RowNormArgs a) {
   extern __shared__ __attribute__((aligned(16))) float smem[];
   float* hrow = smem;            // [E]
   float* blk = smem + a.E;       // [<=64]
-  const int r = blockIdx.x, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int r = row_of_block(blockIdx.x, gridDim.x), tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int E = a.E, nch = E / 8, nblk = (nch + 63) / 64;
   const bf16_t* src = nullptr;
   if (MODE == 0) src = a.embedding + (size_t)a.tokens[r] * E;
@@ -689,8 +689,7 @@ __global__ __launch_bounds__(256) void k_rownorm(RowNormArgs a) {
       }
     }
     if (b < nblk) {
-#pragma unroll
-      for (int off = 1; off < 64; off <<= 1) v = v + __shfl_xor(v, off, 64);
+      v = xor_sum(v);
       if (lane == 0) blk[b] = v;
     }
   }
@@ -846,8 +845,7 @@ static __global__ __launch_bounds__(64) void k_qkv_finalize(QkvArgs a) {
         ss = __builtin_fmaf(x, x, ss);
       }
     }
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) ss = ss + __shfl_xor(ss, off, 64);
+    ss = xor_sum(ss);
     const float total = 0.0f + ss;
     nr = 1.0f / sqrtf(total / (float)g.hd + a.eps);
   }

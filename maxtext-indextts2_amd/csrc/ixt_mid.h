@@ -318,7 +318,7 @@ __device__ __forceinline__ void mid_norm(const MidArgs& a, int blk, u32x4* sx) {
 #pragma unroll
       for (int j = 0; j < 8; ++j) v = __builtin_fmaf(f[j], f[j], v);
       v = b * 64 + lane < nch ? v : 0.0f;
-      v = step_butterfly(v, [](float x, float y) { return x + y; });
+      v = xor_sum(v);
       total = b * 64 < nch ? total + v : total;
     }
     const float rs = 1.0f / sqrtf(total / (float)a.E + a.eps);

@@ -39,8 +39,7 @@ static __global__ __launch_bounds__(1024) void k_moe_route(const bf16_t* xn, con
 #pragma unroll
             for (int j = 0; j < 8; ++j) a = __builtin_fmaf(x[j], bf2f(gv[u][j]), a);
           }
-#pragma unroll
-          for (int off = 1; off < 64; off <<= 1) a = a + __shfl_xor(a, off, 64);
+          a = xor_sum(a);
           total = total + a;
         }
       }
@@ -106,8 +105,7 @@ __global__ __launch_bounds__(1024) void k_moe_route_blocks(const bf16_t* xn, con
 #pragma unroll
     for (int e = 0; e < NEXP; ++e) {
       float t = a[e];
-#pragma unroll
-      for (int off = 1; off < 64; off <<= 1) t = t + __shfl_xor(t, off, 64);
+      t = xor_sum(t);
       if (lane == 0) part[b][e] = t;
     }
   }

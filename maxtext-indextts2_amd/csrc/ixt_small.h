@@ -122,8 +122,7 @@ __global__ __launch_bounds__(1024) void k_sdot(SdotArgs a) {
 #pragma unroll
         for (int j = 0; j < 8; ++j) v = __builtin_fmaf(h[j], h[j], v);
       }
-#pragma unroll
-      for (int off = 1; off < 64; off <<= 1) v = v + __shfl_xor(v, off, 64);
+      v = xor_sum(v);
       if (lane == 0) blk[row * nblk + b] = v;
     }
     __syncthreads();

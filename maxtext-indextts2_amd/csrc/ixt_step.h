@@ -91,20 +91,6 @@ __device__ __forceinline__ void step_wait(const int32_t* cnt, int n, const IxtWa
   asm volatile("" ::: "memory");
 }
 
-// v of the lane 1, 2, 4, 8, 16, 32 away combined with this lane's, in the order of the xor-butterfly of the canonical sums: from 4 on the lanes of a group hold the same
-// value already, so that any lane of the other group will do (row_half_mirror, row_mirror, swaps of rows and halves), and no step goes through LDS.
-template <typename F> __device__ __forceinline__ float step_butterfly(float v, F f) {
-  auto dpp = [](float x, auto ctrl) { return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), decltype(ctrl)::value, 0xf, 0xf, true)); };
-  v = f(v, dpp(v, std::integral_constant<int, 0xb1>()));           // quad_perm 1 0 3 2
-  v = f(v, dpp(v, std::integral_constant<int, 0x4e>()));           // quad_perm 2 3 0 1
-  v = f(v, dpp(v, std::integral_constant<int, 0x141>()));          // row_half_mirror
-  v = f(v, dpp(v, std::integral_constant<int, 0x140>()));          // row_mirror
-  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  v = f(__uint_as_float(a[0]), __uint_as_float(a[1]));
-  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return f(__uint_as_float(b[0]), __uint_as_float(b[1]));
-}
-
 // One block of a projection: `tpb` tiles of 16 columns x the chains of K, one (tile, chain) a wave: 16 KB of weights in its registers.  NORM: the rows are normed on
 // the way into LDS, as k_sdot does.
 template <int PHASE>
@@ -219,7 +205,7 @@ __device__ __forceinline__ void step_dot(const StepArgs& a, int layer, int blk, 
 #pragma unroll
         for (int j = 0; j < 8; ++j) v = __builtin_fmaf(h[j], h[j], v);
         v = ch < nch ? v : 0.0f;
-        v = step_butterfly(v, [](float x, float y) { return x + y; });
+        v = xor_sum(v);
         if (lane == 0) bsum[u] = v;
       }
     }
@@ -498,14 +484,14 @@ __device__ __forceinline__ void step_attn(const StepArgs& a, int layer, int blk,
   vload(2 * wave + hw);
 #pragma unroll
   for (int q = 0; q < GQ; ++q) {
-    mx[q] = step_butterfly(mx[q], [](float x, float y) { return fmaxf(x, y); });
+    mx[q] = xor_butterfly(mx[q], [](float x, float y) { return fmaxf(x, y); });
     if (lane == 0) wred[q * STEP_NW + wave] = mx[q];
   }
   __syncthreads();
 #pragma unroll
   for (int q = 0; q < GQ; ++q) {
     float m = wred[q * STEP_NW + (lane & (aw - 1))];
-    m = step_butterfly(m, [](float x, float y) { return fmaxf(x, y); });
+    m = xor_butterfly(m, [](float x, float y) { return fmaxf(x, y); });
     float* e = ebuf + (size_t)q * tp;
 #pragma unroll 1
     for (int j = j0; j - lane < kv_len; j += nt) e[j] = ixt_exp(e[j] - m);
