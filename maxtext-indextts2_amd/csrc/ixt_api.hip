@@ -1325,6 +1325,8 @@ SdotPlan sdot_plan(const ixt_ctx* c, int epi, bool norm, int K, int N, int R) {
   while (tpb > 1 && p.chains * tpb > 16) tpb -= (epi == GEPI_SWIGLU ? 2 : 1);
   if (tpb > ntile) tpb = ntile;
   p.tpb = tpb;
+  // tiles for half of the CUs at most: half a tile a block (2048 columns; from 129 tiles on whole ones fill more than half of the chip, and twice the blocks would read the rows twice as often)
+  p.half = (epi == GEPI_F32 || epi == GEPI_TANHNORM) && !norm && tpb == 1 && ntile <= 128;
   const int nblk = (K / 8 + 63) / 64;
   p.lds = ((size_t)(K / 8) << p.rpl) * 16 + (size_t)p.chains * tpb * 1024 + (norm ? 1024 + (size_t)(K / 8) * 16 : 0);
   p.ok = R >= 1 && R <= 16 && R * nblk <= 240 && K % IXT_MK == 0 && N % 16 == 0 && p.chains * tpb <= 16 && tpb >= 1 && (epi != GEPI_SWIGLU || tpb % 2 == 0) && p.lds <= 150 * 1024;
@@ -1333,7 +1335,15 @@ SdotPlan sdot_plan(const ixt_ctx* c, int epi, bool norm, int K, int N, int R) {
 
 template <int EPI, bool NORM>
 static int sdot_t(const SdotArgs& a, const SdotPlan& p, hipStream_t st) {
-  hipLaunchKernelGGL((k_sdot<EPI, NORM>), dim3(a.main_blocks + (a.pf_n ? p.pf_blocks : 0)), dim3(64 * p.chains * p.tpb), p.lds, st, a);
+  const dim3 grid(a.main_blocks + (a.pf_n ? p.pf_blocks : 0)), block(64 * p.chains * p.tpb);
+  if constexpr ((EPI == GEPI_F32 || EPI == GEPI_TANHNORM) && !NORM) {
+    if (p.half) {
+      hipLaunchKernelGGL((k_sdot<EPI, NORM, true>), grid, block, p.lds, st, a);
+      LAUNCHCHK();
+      return IXT_OK;
+    }
+  }
+  hipLaunchKernelGGL((k_sdot<EPI, NORM>), grid, block, p.lds, st, a);
   LAUNCHCHK();
   return IXT_OK;
 }
@@ -1342,9 +1352,10 @@ static int sdot_t(const SdotArgs& a, const SdotPlan& p, hipStream_t st) {
 static int sdot_set_attributes() {
   static bool done = false;
   if (done) return IXT_OK;
-#define SATTR(E_, N_) HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_sdot<E_, N_>), hipFuncAttributeMaxDynamicSharedMemorySize, 156 * 1024))
+#define SATTR(E_, ...) HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_sdot<E_, __VA_ARGS__>), hipFuncAttributeMaxDynamicSharedMemorySize, 156 * 1024))
   SATTR(GEPI_QKV, true); SATTR(GEPI_QKV, false); SATTR(GEPI_RESID, true); SATTR(GEPI_RESID, false);
   SATTR(GEPI_SWIGLU, true); SATTR(GEPI_SWIGLU, false); SATTR(GEPI_F32, true); SATTR(GEPI_F32, false); SATTR(GEPI_TANHNORM, false); SATTR(GEPI_ACT, false);
+  SATTR(GEPI_F32, false, true); SATTR(GEPI_TANHNORM, false, true);
 #undef SATTR
   done = true;
   return IXT_OK;
@@ -1352,13 +1363,14 @@ static int sdot_set_attributes() {
 
 // x: NORM: hidden rows [R][K] row-major (+ scale); else activations in xidx layout.  w: widx layout.
 int launch_sdot(ixt_ctx* c, int epi, bool norm, const bf16_t* x, const bf16_t* scale, const bf16_t* w, int K, int N, int R, const GemmEpi& e,
-                       hipStream_t st, const bf16_t* pf, size_t pf_elems) {
+                       hipStream_t st, const bf16_t* pf, size_t pf_elems, const SdotSide* side) {
   SdotPlan p = sdot_plan(c, epi, norm, K, N, R);
   if (!p.ok) return set_err(IXT_ERR_UNSUPPORTED, "sdot: %d rows x K %d x N %d does not fit the few-rows form", R, K, N);
   SdotArgs a;
   a.x = x; a.scale = scale; a.eps = c->cfg.normalization_layer_epsilon; a.w = reinterpret_cast<const u32x4*>(w);
   a.K = K; a.N = N; a.R = R; a.rpl = p.rpl; a.tpb = p.tpb; a.chains = p.chains; a.e = e;
-  a.main_blocks = (N / 16 + p.tpb - 1) / p.tpb;
+  if (side != nullptr) a.side = *side;
+  a.main_blocks = p.half ? N / 8 : (N / 16 + p.tpb - 1) / p.tpb;
   const bool prefetch = c->small_prefetch && pf != nullptr && pf_elems > 0;
   a.pf = prefetch ? reinterpret_cast<const u32x4*>(pf) : nullptr;
   a.pf_n = prefetch ? pf_elems / 8 : 0;

@@ -44,9 +44,13 @@ struct SdotArgs {
   int K, N, R, rpl, tpb, chains;
   GemmEpi e;
   const u32x4* pf; size_t pf_n; int main_blocks;   // prefetch: blocks main_blocks .. gridDim.x - 1 stream pf[0 .. pf_n) (16-byte units)
+  SdotSide side;
 };
 
-template <int EPI, bool NORM>
+// HALF: a block takes eight columns of a tile, so that a product of few tiles still runs on all CUs.  A wave's load is two steps of those columns (whole lines of 128 bytes): lanes
+// 8 .. 15 of each group of 16 hold the second, and a rotation of the groups by eight lanes brings it to the rows of the first; rows 8 .. 15 of the products are never stored.
+// 8 rows, 2048 columns, K 2048 and 7168 in turn: 7.9 us a launch by whole tiles (128 blocks), now 6.9; 4 rows, 1024 columns, K 1024 and 3584 with the tanh norm: 6.4 -> 6.0.
+template <int EPI, bool NORM, bool HALF = false>
 __global__ __launch_bounds__(1024) void k_sdot(SdotArgs a) {
   extern __shared__ __attribute__((aligned(16))) u32x4 sx[];
   const int tid = threadIdx.x, nthr = blockDim.x, lane = tid & 63;
@@ -59,7 +63,7 @@ __global__ __launch_bounds__(1024) void k_sdot(SdotArgs a) {
   const int nsteps = K >> 5, ntile = N >> 4, nch = K >> 3;
   const int rpl = a.rpl, Rp = 1 << rpl;
   const int t = wave % tpb, c = wave / tpb;
-  const int tile = blockIdx.x * tpb + t;
+  const int tile = HALF ? (int)blockIdx.x >> 1 : (int)blockIdx.x * tpb + t, half8 = HALF ? ((int)blockIdx.x & 1) * 8 : 0;      // (HALF: tpb is 1)
   const bool tile_ok = tile < ntile;
   const int r_in = lane & 15, cq = lane >> 4;
   f32x4* red = reinterpret_cast<f32x4*>(sx + ((size_t)nch << rpl));     // [chains][tpb][64]
@@ -82,13 +86,14 @@ __global__ __launch_bounds__(1024) void k_sdot(SdotArgs a) {
 
   // this wave's chain of weight fragments: all sixteen in flight
   const int s0 = c * 16, cs = min(16, nsteps - s0);
-  const u32x4* wbase = a.w + ((size_t)(tile_ok ? tile : 0) * nsteps + s0) * 64 + lane;
+  const u32x4* wbase = a.w + ((size_t)(tile_ok ? tile : 0) * nsteps + s0) * 64 + (HALF ? cq * 16 + half8 + (lane & 7) : lane);
   const bool full = tile_ok && cs == 16;      // the usual case: a whole chain, no per-step conditions anywhere
-  u32x4 wv[16];
+  constexpr int NWV = HALF ? 8 : 16;
+  u32x4 wv[NWV];
   // (a short last chain re-reads its last fragment for the steps it does not have, a block past the last tile reads tile 0: valid
   // addresses, values never used -- one unconditional load sequence for every wave)
 #pragma unroll
-  for (int s = 0; s < 16; ++s) wv[s] = __builtin_nontemporal_load(wbase + (size_t)min(s, cs - 1) * 64);
+  for (int s = 0; s < NWV; ++s) wv[s] = __builtin_nontemporal_load(wbase + (size_t)min(HALF ? 2 * s + (lane >> 3 & 1) : s, cs - 1) * 64);
 
 #pragma unroll
   for (int u = 0; u < 8; ++u) {
@@ -154,16 +159,27 @@ __global__ __launch_bounds__(1024) void k_sdot(SdotArgs a) {
   f32x4 acc = f32x4(0.0f);
   {
     const u32x4* xb = sx + (((size_t)s0 * 4 + cq) << rpl) + (r_in & (Rp - 1));
+    auto fragment = [&](int s) {
+      if constexpr (!HALF) return wv[s];
+      else {
+        u32x4 f = wv[s >> 1];
+        if (s & 1) {
+          auto turned = [](uint32_t v) { return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x128, 0xf, 0xf, true); };      // row_ror:8
+          f = u32x4{turned(f.x), turned(f.y), turned(f.z), turned(f.w)};
+        }
+        return f;
+      }
+    };
     if (full) {
 #pragma unroll
       for (int s = 0; s < 16; ++s) {
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wv[s]), __builtin_bit_cast(bf16x8, xb[(size_t)(s * 4) << rpl]), acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, fragment(s)), __builtin_bit_cast(bf16x8, xb[(size_t)(s * 4) << rpl]), acc, 0, 0, 0);
         if ((s & 3) == 3) __builtin_amdgcn_sched_barrier(0);   // at most four operand reads ahead of their MFMAs: 64 registers hold the weight fragments
       }
     } else if (tile_ok) {
 #pragma unroll
       for (int s = 0; s < 16; ++s)
-        if (s < cs) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wv[s]), __builtin_bit_cast(bf16x8, xb[(size_t)(s * 4) << rpl]), acc, 0, 0, 0);
+        if (s < cs) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, fragment(s)), __builtin_bit_cast(bf16x8, xb[(size_t)(s * 4) << rpl]), acc, 0, 0, 0);
     }
   }
   red[((size_t)c * tpb + t) * 64 + lane] = acc;
@@ -176,12 +192,25 @@ __global__ __launch_bounds__(1024) void k_sdot(SdotArgs a) {
     if (EPI == GEPI_SWIGLU) tot2 = tot2 + red[((size_t)cc * tpb + t + 1) * 64 + lane];
   }
   const int row = r_in;
-  const bool row_ok = row < R;
+  const bool row_ok = row < R && (!HALF || cq < 2);
 
   if constexpr (EPI == GEPI_F32) {
-    if (row_ok) *reinterpret_cast<float4*>(a.e.out + (size_t)row * N + tile * 16 + cq * 4) = make_float4(tot[0], tot[1], tot[2], tot[3]);
+    const int col = tile * 16 + half8 + cq * 4;
+    if (row_ok) {
+      *reinterpret_cast<float4*>(a.e.out + (size_t)row * N + col) = make_float4(tot[0], tot[1], tot[2], tot[3]);
+      if (a.side.x != nullptr) {
+        const SdotSide& sd = a.side;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int k = (unsigned)(col + j - sd.a) < (unsigned)sd.na ? col + j - sd.a : (unsigned)(col + j - sd.b) < (unsigned)sd.nb ? sd.na + col + j - sd.b : -1;
+          if (k >= 0) sd.x[xidx(row, k, sd.Kp)] = f2bf(tot[j]);
+        }
+        if (col < 8)                                   // (the first columns' lanes: all rows, two of them a row)
+          for (int k = sd.na + sd.nb + (col >> 2); k < sd.Kp; k += 2) sd.x[xidx(row, k, sd.Kp)] = 0;
+      }
+    }
   } else if constexpr (EPI == GEPI_TANHNORM) {
-    if (row_ok) tanhnorm_epi(a.e.tn, a.e.act, row, tile * 16 + cq * 4, tot);
+    if (row_ok) tanhnorm_epi(a.e.tn, a.e.act, row, tile * 16 + half8 + cq * 4, tot);
   } else if constexpr (EPI == GEPI_ACT) {
     if (row_ok) {
       uint2 ov;

@@ -171,6 +171,13 @@ def test_dot_small_rows_kernel(ctx, R, K, N, tpb):
     H.lib.check(eng.lib.ixt_set_option(eng._ctx, b"small_tpb", 0))
 
 
+@pytest.mark.parametrize("R,K,N", [(1, 128, 2048), (8, 640, 2048), (8, 7168, 2032), (16, 1152, 2048), (8, 1152, 2064)])
+def test_dot_small_rows_half_tiles(ctx, R, K, N):
+  """The few-rows form takes half a tile a block up to 128 tiles (two steps of weights a load, the second turned by eight lanes), whole ones from 129 on; whole and short last chains.
+  The canonical sum, bit for bit."""
+  test_dot_small_rows_kernel(ctx, R, K, N, 0)
+
+
 @pytest.mark.parametrize("spread,zero_frac", [(4, 0.0), (12, 0.2), (40, 0.05)])
 def test_dot_wide_exponents_and_zeros(ctx, spread, zero_frac):
   """The matrix-core arithmetic truncates small products against the largest one of each 8-k step: exercise wide exponent
