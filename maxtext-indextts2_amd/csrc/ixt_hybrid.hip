@@ -571,6 +571,7 @@ int hybrid_init(ixt_ctx* c) {
         const int N = up_to(l.out_gate ? L.g_off + g.H * l.vdim : L.d_off + g.rank + g.dr, 16);
         dotsz(m->Ep, N);
         if (l.out_gate || l.q_rank > 0) upd(part2, std::max((size_t)R * N, (size_t)std::min(R, 128) * N * ((m->Ep + IXT_CHAIN - 1) / IXT_CHAIN)));
+        else upd(part2, (size_t)std::min(R, 16) * N * ((m->Ep + IXT_CHAIN - 1) / IXT_CHAIN));      // (k_latent_front)
         if (l.q_rank > 0) { dotsz(up_to(l.q_rank, IXT_KALIGN), NQ); upd(act_k, up_to(l.q_rank, IXT_KALIGN)); }
       }
       upd(part, (size_t)g.H * Rp * ukn);                                    // several slices only below 128 rows
@@ -742,15 +743,17 @@ int hybrid_copy_group(ixt_ctx* c, int src, int dst, int npages, hipStream_t st) 
 }
 
 // ---------------------------------------------------------------------------------------------------- the forward pass
-template <typename T> static int hdot(ixt_ctx* c, const T* x, const HMat& w, int R, float* out, size_t out_floats, hipStream_t st, Slices* res);
-template <> int hdot<bf16_t>(ixt_ctx* c, const bf16_t* x, const HMat& w, int R, float* out, size_t out_floats, hipStream_t st, Slices* res) {
+// side: asks for columns as the next operand, too; its x is nullptr afterwards where the form does not have that
+template <typename T> static int hdot(ixt_ctx* c, const T* x, const HMat& w, int R, float* out, size_t out_floats, hipStream_t st, Slices* res, SdotSide* side = nullptr);
+template <> int hdot<bf16_t>(ixt_ctx* c, const bf16_t* x, const HMat& w, int R, float* out, size_t out_floats, hipStream_t st, Slices* res, SdotSide* side) {
   if (R <= c->small_rows && (size_t)R * w.Np <= out_floats && w.Np <= 65536 && sdot_plan(c, GEPI_F32, false, w.Kp, w.Np, R).ok) {     // few rows: one slice
     GemmEpi e{};
     e.out = out;
-    TRY(launch_sdot(c, GEPI_F32, false, x, nullptr, (const bf16_t*)w.w, w.Kp, w.Np, R, e, st));
+    TRY(launch_sdot(c, GEPI_F32, false, x, nullptr, (const bf16_t*)w.w, w.Kp, w.Np, R, e, st, nullptr, 0, side));
     *res = Slices{out, 1, (size_t)R * w.Np, w.Np};
     return IXT_OK;
   }
+  if (side != nullptr) side->x = nullptr;
   DotResult dr;
   TRY(launch_dot(c, x, (const bf16_t*)w.w, w.Kp, w.Np, R, out, out_floats, false, st, &dr));
   *res = Slices{out, dr.slices, dr.slice_stride, w.Np};
@@ -774,7 +777,8 @@ static int launch_dot32(const float* x, const HMat& w, size_t wstride, int R, co
   *res = Slices{out, (int)grid.z, (size_t)R * w.Np, w.Np};
   return IXT_OK;
 }
-template <> int hdot<float>(ixt_ctx*, const float* x, const HMat& w, int R, float* out, size_t out_floats, hipStream_t st, Slices* res) {
+template <> int hdot<float>(ixt_ctx*, const float* x, const HMat& w, int R, float* out, size_t out_floats, hipStream_t st, Slices* res, SdotSide* side) {
+  if (side != nullptr) side->x = nullptr;
   return launch_dot32(x, w, 0, R, nullptr, out, out_floats, st, res);
 }
 // a product of few columns over a long K, some rows: whole-K blocks would leave most of the chip idle, so the reduction is cut into slices (128 x 160 outputs, K
@@ -892,9 +896,9 @@ static int latent_launch(bool tall, int H, int splits, LatentAttnArgs a, hipStre
   LAUNCHCHK();
   return IXT_OK;
 }
-// queries (slices in latent space + rotated parts) over the paged latents -> the value latents, act(T) row h Rp + r
+// queries (slices in latent space + rotated parts) over the paged latents -> the value latents, act(T) row h Rp + r; apart (nullptr: no): the key splits may stay apart, its number of them (1: they did not)
 template <typename T>
-static int latent_attention(ixt_ctx* c, const HLayer& L, const Slices& qa, int R, int Rp, bool decode, int len_hint, hipStream_t st) {
+static int latent_attention(ixt_ctx* c, const HLayer& L, const Slices& qa, int R, int Rp, bool decode, int len_hint, hipStream_t st, int* apart) {
   HybridModel* m = c->hy;
   const LatentGeom& g = L.lg;
   const int Kp = up_to(g.rankp, IXT_KALIGN);
@@ -918,7 +922,8 @@ static int latent_attention(ixt_ctx* c, const HLayer& L, const Slices& qa, int R
         else rc = latent_launch<32, 2>(tall, g.H, splits, a, st);
       }
       TRY(rc);
-      if (splits > 1) {
+      if (apart != nullptr) *apart = splits;
+      else if (splits > 1) {
         hipLaunchKernelGGL(k_latent_combine, dim3(R, g.H), dim3(128), 0, st, m->po, m->pml, splits, g.rankp, g.H, Rp, c->row_active, (bf16_t*)m->olat, Kp);
         LAUNCHCHK();
       }
@@ -937,7 +942,11 @@ static int hybrid_mixer_latent(ixt_ctx* c, const HLayer& L, const HLayer& W, int
   HybridModel* m = c->hy;
   const LatentGeom& g = L.lg;
   Slices t, in;
-  const bool kept = L.c.out_gate || L.c.q_rank > 0;              // the input projection outlives the next dots
+  // few rows: the cache entry beside the key up-projection, and all that lies between the attention and the output projection, a launch each
+  const bool few = sizeof(T) == 2 && R <= 16 && latent_mfma_fits(*m, g);
+  const bool front = few && L.c.q_rank == 0 && W.uk.Kp <= IXT_CHAIN && (size_t)R * W.in.Np <= m->part2_floats && (size_t)g.H * Rp * W.uk.Np <= c->part_floats;
+  const bool back = few && W.uv.Kp <= IXT_CHAIN;
+  const bool kept = L.c.out_gate || L.c.q_rank > 0 || front;     // the input projection outlives the next dots
   TRY(hdot<T>(c, (const T*)m->xb, W.in, R, kept ? m->part2 : c->part, kept ? m->part2_floats : c->part_floats, st, &in));
   t = in;
   if (L.c.q_rank > 0) {
@@ -945,11 +954,32 @@ static int hybrid_mixer_latent(ixt_ctx* c, const HLayer& L, const HLayer& W, int
     LAUNCHCHK();
     TRY(hdot<T>(c, (const T*)m->act, W.uq, R, c->part, c->part_floats, st, &t));
   }
-  hipLaunchKernelGGL((k_latent_prep<T>), dim3(R, 1 + (g.H + 3) / 4), dim3(256), 0, st, in, t, L.d_off, g, W.cnorm, m->eps, L.rope_cos, L.rope_sin, c->row_slot, c->row_pos, c->row_active,
-                     c->ps.page_map, (T*)L.pages, (T*)m->qx, W.uk.Kp, Rp, (T*)m->qr);
-  LAUNCHCHK();
-  TRY(hdot_grouped<T>(c, (const T*)m->qx, W.uk, W.uk_stride, g.H * Rp, Rp, m->head_rb, c->part, c->part_floats, st, &t));
-  TRY(latent_attention<T>(c, L, t, R, Rp, decode, len_hint, st));
+  const LatentPrepArgs<T> pa{in, t, L.d_off, g, W.cnorm, m->eps, L.rope_cos, L.rope_sin, c->row_slot, c->row_pos, c->row_active, c->ps.page_map, (T*)L.pages, front ? nullptr : (T*)m->qx, W.uk.Kp, Rp,
+                             (T*)m->qr};
+  if constexpr (sizeof(T) == 2) {
+    if (front) {
+      const LatentUpArgs ua{reinterpret_cast<const u32x4*>(W.uk.w), W.uk_stride / 8, W.uk.Np, c->part, R};
+      hipLaunchKernelGGL(k_latent_front, dim3(R * (1 + (g.H + 3) / 4) + g.H * ((W.uk.Np + 127) / 128)), dim3(256), (size_t)W.uk.Kp * 32, st, pa, ua);
+      LAUNCHCHK();
+      t = Slices{c->part, 1, (size_t)g.H * Rp * W.uk.Np, W.uk.Np};
+    }
+  }
+  if (!front) {
+    hipLaunchKernelGGL((k_latent_prep<T>), dim3(R, 1 + (g.H + 3) / 4), dim3(256), 0, st, pa);
+    LAUNCHCHK();
+    TRY(hdot_grouped<T>(c, (const T*)m->qx, W.uk, W.uk_stride, g.H * Rp, Rp, m->head_rb, c->part, c->part_floats, st, &t));
+  }
+  int splits = 1;
+  TRY(latent_attention<T>(c, L, t, R, Rp, decode, len_hint, st, back ? &splits : nullptr));
+  if constexpr (sizeof(T) == 2) {
+    if (back) {
+      const LatentOutArgs oa{splits > 1 ? m->po : nullptr, m->pml, splits, g.rankp, (const bf16_t*)m->olat, Rp, reinterpret_cast<const u32x4*>(W.uv.w), W.uv_stride / 8, W.uv.Kp, W.uv.Np, g.H, R, L.c.vdim,
+                             L.c.out_gate ? in : Slices{}, L.g_off, c->row_active, (bf16_t*)m->act, W.o.Kp};
+      hipLaunchKernelGGL(k_latent_out, dim3(g.H, (W.uv.Np + 31) / 32), dim3(512), (size_t)W.uv.Kp * 32, st, oa);
+      LAUNCHCHK();
+      return IXT_OK;
+    }
+  }
   TRY(hdot_grouped<T>(c, (const T*)m->olat, W.uv, W.uv_stride, g.H * Rp, Rp, m->head_rb, c->part, c->part_floats, st, &t));
   hipLaunchKernelGGL((k_heads_x<T>), dim3(R, (W.o.Kp + 255) / 256), dim3(256), 0, st, t, g.H, L.c.vdim, Rp, L.c.out_gate ? in : Slices{}, L.g_off, (T*)m->act, W.o.Kp);
   LAUNCHCHK();
@@ -994,9 +1024,13 @@ static int hybrid_mixer_delta(ixt_ctx* c, const HLayer& L, const HLayer& W, int 
   HybridModel* m = c->hy;
   const DeltaGeom& g = L.dg;
   Slices t, t2;
-  TRY(hdot<T>(c, (const T*)m->xb, W.in, R, c->part, c->part_floats, st, &t));
-  hipLaunchKernelGGL((k_lowrank_x<T>), dim3(R), dim3(128), 0, st, t, g, (T*)m->act, W.low.Kp);
-  LAUNCHCHK();
+  SdotSide low;                                                    // the low-rank columns as an operand: by the product itself, or a launch behind it
+  if constexpr (sizeof(T) == 2) low = SdotSide{(bf16_t*)m->act, g.oa, g.ra, g.og, g.rg, W.low.Kp};
+  TRY(hdot<T>(c, (const T*)m->xb, W.in, R, c->part, c->part_floats, st, &t, &low));
+  if (low.x == nullptr) {
+    hipLaunchKernelGGL((k_lowrank_x<T>), dim3(R), dim3(128), 0, st, t, g, (T*)m->act, W.low.Kp);
+    LAUNCHCHK();
+  }
   TRY(hdot<T>(c, (const T*)m->act, W.low, R, m->part2, m->part2_floats, st, &t2));
   if (single) {            // every row is a segment of one token
     DeltaStepArgs da{t, t2, g, W.cq, W.ck, W.cv, W.a_log, W.dt_bias, W.onorm, m->eps, c->row_active, c->row_slot, c->row_pos, m->parity, L.tails, L.state};

@@ -808,15 +808,24 @@ struct LatentGeom {
 // (heads of dn + dr, columns from 0 on) -> unrotated parts head-major as the operand of the key up-projection (row h Rp + r), rotated parts qr
 // [R][H][rotp].  rope: f32 [position][dr / 2] cos, sin.  grid (R, 1 + ceil(H / 4)), block 256: y = 0 the cache entry, y > 0 four heads (a wave each).
 template <typename T>
-__global__ __launch_bounds__(256) void k_latent_prep(Slices t, Slices tq, int d_off, LatentGeom g, const float* __restrict__ cnorm, float eps, const float* __restrict__ rope_cos,
-                                                     const float* __restrict__ rope_sin, const int32_t* __restrict__ row_slot, const int32_t* __restrict__ row_pos,
-                                                     const int32_t* __restrict__ row_active, const int32_t* __restrict__ page_map, T* __restrict__ pages, T* __restrict__ qx,
-                                                     int dnp, int Rp, T* __restrict__ qr) {
+struct LatentPrepArgs {
+  Slices t, tq; int d_off; LatentGeom g; const float* cnorm; float eps; const float *rope_cos, *rope_sin;
+  const int32_t *row_slot, *row_pos, *row_active, *page_map;
+  T *pages, *qx; int dnp, Rp; T* qr;                   // qx nullptr: the unrotated parts stay where they are
+};
+template <typename T>
+__device__ __forceinline__ void latent_prep(const LatentPrepArgs<T>& a, int r, int y) {
   __shared__ float red[4];
-  const int r = blockIdx.x, half = g.dr >> 1;
-  const bool act = row_active[r] != 0;
-  const int pos = act ? row_pos[r] : 0;
-  if (blockIdx.y == 0) {
+  const Slices &t = a.t, &tq = a.tq;
+  const LatentGeom& g = a.g;
+  const float *__restrict__ cnorm = a.cnorm, *__restrict__ rope_cos = a.rope_cos, *__restrict__ rope_sin = a.rope_sin;
+  const int32_t *__restrict__ row_slot = a.row_slot, *__restrict__ page_map = a.page_map;
+  T *__restrict__ pages = a.pages, *__restrict__ qx = a.qx, *__restrict__ qr = a.qr;
+  const int half = g.dr >> 1, d_off = a.d_off, dnp = a.dnp, Rp = a.Rp;
+  const float eps = a.eps;
+  const bool act = a.row_active[r] != 0;
+  const int pos = act ? a.row_pos[r] : 0;
+  if (y == 0) {
     if (!act) return;
     float ss = 0.0f;
     for (int k = threadIdx.x; k < g.rank; k += 256) { const float v = t.at(r, d_off + k); ss = fmaf(v, v, ss); }
@@ -832,10 +841,10 @@ __global__ __launch_bounds__(256) void k_latent_prep(Slices t, Slices tq, int d_
     }
     return;
   }
-  const int h = (blockIdx.y - 1) * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int h = (y - 1) * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (h >= g.H) return;
   const int c0 = h * (g.dn + g.dr);
-  for (int k = lane; k < dnp; k += 64) act_store1(qx, h * Rp + r, k, dnp, k < g.dn ? tq.at(r, c0 + k) : 0.0f);
+  for (int k = lane; k < dnp && qx != nullptr; k += 64) act_store1(qx, h * Rp + r, k, dnp, k < g.dn ? tq.at(r, c0 + k) : 0.0f);
   T* qo = qr + ((size_t)r * g.H + h) * g.rotp;
   for (int i = lane; i < g.rotp / 2; i += 64) {
     float a = 0.0f, b = 0.0f;
@@ -846,6 +855,47 @@ __global__ __launch_bounds__(256) void k_latent_prep(Slices t, Slices tq, int d_
     }
     qo[2 * i] = from_f<T>(a); qo[2 * i + 1] = from_f<T>(b);
   }
+}
+template <typename T>
+__global__ __launch_bounds__(256) void k_latent_prep(LatentPrepArgs<T> a) { latent_prep(a, blockIdx.x, blockIdx.y); }
+// Up to 16 rows (bf16): the same and, beside it, the unrotated parts through the key up-projection, which needs nothing of it: out, head-major slices (row h Rp + r, Np columns), may not lie
+// where tq does.  Two launches took 4.3 and 4.2 us (8 rows, 16 heads, rank 512), this 5.3.  grid R (1 + ceil(H / 4)) + H ceil(Np / 128), block 256, LDS 2 dnp 16 bytes: behind the blocks above, block = (head, eight tiles of
+// its columns), a wave two of them.
+struct LatentUpArgs { const u32x4* w; size_t wstride; int Np; float* out; int R; };
+static __global__ __launch_bounds__(256) void k_latent_front(LatentPrepArgs<bf16_t> a, LatentUpArgs u) {
+  extern __shared__ __attribute__((aligned(16))) u32x4 lx[];       // pieces of eight features of a row: [dnp / 8][16]
+  const LatentGeom& g = a.g;
+  const int per = 1 + (g.H + 3) / 4, first = u.R * per, tid = threadIdx.x, lane = tid & 63;
+  if ((int)blockIdx.x < first) { latent_prep(a, blockIdx.x / per, blockIdx.x % per); return; }
+  const int per_head = (u.Np + 127) >> 7, b = blockIdx.x - first, h = b / per_head, t0 = (b % per_head) * 8 + __builtin_amdgcn_readfirstlane(tid >> 6) * 2;
+  const int nsteps = a.dnp >> 5, ntile = u.Np >> 4;
+  u32x4 wv[2][16];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const u32x4* wb = u.w + (size_t)h * u.wstride + (size_t)min(t0 + i, ntile - 1) * nsteps * 64 + lane;
+#pragma unroll
+    for (int s = 0; s < 16; ++s)
+      if (s < nsteps) wv[i][s] = wb[(size_t)s * 64];
+  }
+  const int c0 = h * (g.dn + g.dr);
+  for (int i = tid; i < u.R * a.dnp; i += 256) {
+    const int r = i / a.dnp, k = i - r * a.dnp;
+    reinterpret_cast<bf16_t*>(lx)[((k >> 3) * 16 + r) * 8 + (k & 7)] = k < g.dn ? f2bf(a.tq.at(r, c0 + k)) : (bf16_t)0;
+  }
+  __syncthreads();
+  f32x4 acc[2] = {f32x4(0.0f), f32x4(0.0f)};
+#pragma unroll
+  for (int s = 0; s < 16; ++s)
+    if (s < nsteps) {
+      const bf16x8 x = __builtin_bit_cast(bf16x8, lx[s * 64 + lane]);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wv[i][s]), x, acc[i], 0, 0, 0);
+    }
+  const int row = lane & 15;
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+    if (row < u.R && t0 + i < ntile)
+      *reinterpret_cast<float4*>(u.out + ((size_t)h * a.Rp + row) * u.Np + (t0 + i) * 16 + (lane >> 4) * 4) = make_float4(acc[i][0], acc[i][1], acc[i][2], acc[i][3]);
 }
 
 // n columns of a projection from c0 on, RMS-normed with a plain weight, as the next dot's operand.  grid R, block 256.
@@ -1240,17 +1290,22 @@ __global__ __launch_bounds__(256, 2) void k_latent_decode(LatentAttnArgs a) {
     if (wave == 0 && cq == 0) { a.part_ml[pi * 2] = m; a.part_ml[pi * 2 + 1] = l; }
   }
 }
-// Key splits (<= 16) of one (row, head): ml = {maximum, sum} per split -> fac[s] = what split s's weighted sum counts for (threads 0 .. 63 work, all call)
+// Key splits (<= 16) of one (row, head): ml = {maximum, sum} per split -> what split s's weighted sum counts for (s = lane % 16; a whole wave)
+__device__ __forceinline__ float split_factor(const float* __restrict__ ml, int nsplit, int lane) {
+  const int s = lane & 15;
+  const float ms = s < nsplit ? ml[s * 2] : -INFINITY, ls = s < nsplit ? ml[s * 2 + 1] : 0.0f;
+  float mm = ms;
+#pragma unroll
+  for (int off = 1; off < 16; off <<= 1) mm = fmaxf(mm, __shfl_xor(mm, off, 64));
+  const float f = ms == -INFINITY ? 0.0f : exp2f(ms - mm);      // a split without a key of its own
+  const float ll = row16_sum(ls * f);
+  return f / ll;
+}
+// (threads 0 .. 63 work, all call)
 __device__ __forceinline__ void split_factors(const float* __restrict__ ml, int nsplit, int tid, float* fac /*[16] LDS*/) {
   if (tid < 64) {
-    const int s = tid & 15;
-    const float ms = s < nsplit ? ml[s * 2] : -INFINITY, ls = s < nsplit ? ml[s * 2 + 1] : 0.0f;
-    float mm = ms;
-#pragma unroll
-    for (int off = 1; off < 16; off <<= 1) mm = fmaxf(mm, __shfl_xor(mm, off, 64));
-    const float f = ms == -INFINITY ? 0.0f : exp2f(ms - mm);      // a split without a key of its own
-    const float ll = row16_sum(ls * f);
-    if (tid < 16) fac[s] = f / ll;
+    const float f = split_factor(ml, nsplit, tid);
+    if (tid < 16) fac[tid] = f;
   }
   __syncthreads();
 }
@@ -1282,6 +1337,81 @@ static __global__ __launch_bounds__(128) void k_latent_combine(const float* __re
     act_store4(out, h * Rp + r, c, Kp, v);
   }
 }
+// Up to 16 rows (bf16): the key splits of every head put together, the values' up-projection of the head and its gate, act of the output projection's, in one launch: k_latent_combine,
+// k_dotb and k_heads_x one behind the other took 4.1, 4.2 and 2.5 us
+// (8 rows, 16 heads of 128, rank 512, five splits; a launch behind another costs 4 us whatever it does), this 6.3.  Block = (head, two tiles of its columns): a wave requests a tile's weights, all eight put the row's latents together.
+// o (nullptr: `olat`, one split): [R][H][nsplit][cols].  rows without a token: zeros.  grid (H, ceil(Np / 32)), block 512, LDS 2 Kp 16 bytes.
+struct LatentOutArgs {
+  const float *o, *ml; int nsplit, cols;
+  const bf16_t* olat; int Rp;
+  const u32x4* w; size_t wstride; int Kp, Np;          // per head: Kp x Np, Kp <= IXT_CHAIN
+  int H, R, n;                                         // n: value dims of a head
+  Slices gate; int g0;
+  const int32_t* row_active;
+  bf16_t* out; int out_Kp;
+};
+static __global__ __launch_bounds__(512) void k_latent_out(LatentOutArgs a) {
+  extern __shared__ __attribute__((aligned(16))) u32x4 lx[];       // pieces of eight latents of a row: [Kp / 8][16]
+  __shared__ float fac[16][16];
+  __shared__ int live[16];
+  const int h = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int nsteps = a.Kp >> 5, tile = blockIdx.y * 2 + wave, row = lane & 15, cq = lane >> 4, col = tile * 16 + cq * 4;
+  const bool dots = wave < 2 && tile * 16 < a.Np;
+  u32x4 wv[16];
+  float gate[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  if (dots) {
+    const u32x4* wb = a.w + (size_t)h * a.wstride + (size_t)tile * nsteps * 64 + lane;
+#pragma unroll
+    for (int s = 0; s < 16; ++s) wv[s] = wb[(size_t)min(s, nsteps - 1) * 64];
+    if (a.gate.n > 0) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (row < a.R && col + j < a.n) gate[j] = a.gate.at(row, a.g0 + h * a.n + col + j);
+    }
+  }
+  for (int r = wave; r < a.R; r += 8) {
+    const int on = a.row_active[r];
+    const float f = a.o != nullptr && on ? split_factor(a.ml + ((size_t)r * a.H + h) * a.nsplit * 2, a.nsplit, lane) : 0.0f;
+    if (lane < 16) fac[r][lane] = f;
+    if (lane == 0) live[r] = on;
+  }
+  __syncthreads();
+  const int quads = a.Kp >> 2;
+  for (int i = tid; i < a.R * quads; i += 512) {
+    const int r = i / quads, c = (i - r * quads) * 4;
+    uint2 u = {0, 0};
+    if (live[r] && c < a.cols) {
+      if (a.o != nullptr) {
+        float v[4];
+        split_sum4(a.o + ((size_t)r * a.H + h) * a.nsplit * a.cols + c, a.cols, a.nsplit, fac[r], v);
+        u = uint2{pack2(f2bf(v[0]), f2bf(v[1])), pack2(f2bf(v[2]), f2bf(v[3]))};
+      } else u = *reinterpret_cast<const uint2*>(a.olat + xidx(h * a.Rp + r, c, a.Kp));
+    }
+    reinterpret_cast<uint2*>(lx)[((c >> 3) * 16 + r) * 2 + (c >> 2 & 1)] = u;
+  }
+  __syncthreads();
+  if (dots) {
+    f32x4 acc = f32x4(0.0f);
+#pragma unroll
+    for (int s = 0; s < 16; ++s)
+      if (s < nsteps) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wv[s]), __builtin_bit_cast(bf16x8, lx[s * 64 + lane]), acc, 0, 0, 0);
+    if (row < a.R) {
+      float v[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = a.gate.n > 0 ? acc[j] * f32_sigmoid(gate[j]) : acc[j];
+      if ((a.n & 3) == 0) {
+        if (col < a.n) act_store4(a.out, row, h * a.n + col, a.out_Kp, v);
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (col + j < a.n) act_store1(a.out, row, h * a.n + col + j, a.out_Kp, v[j]);
+      }
+    }
+  }
+  if (h == a.H - 1 && blockIdx.y == 0)
+    for (int k = a.H * a.n + lane; k < a.out_Kp; k += 64)
+      for (int r = wave; r < a.R; r += 8) act_store1(a.out, r, k, a.out_Kp, 0.0f);
+}
 // head-major slices (row h Rp + r, n columns each) -> act of the output projection: column h n + c, times sigmoid of gate column g0 + h n + c (gate.n ==
 // 0: none).  grid (R, ceil(Kp / 256)), block 256.
 template <typename T>
@@ -1303,7 +1433,7 @@ struct DeltaGeom {
   int og2;                                  // column of the output gate in the second low-rank product (decays start at 0)
   int C;                                    // convolution channels = 2 KH d + H dv (q, k, v)
 };
-// the two low-rank activations side by side as ONE operand (the second matrices form a block diagonal).  grid R, block 128.
+// the two low-rank activations side by side as ONE operand (the second matrices form a block diagonal), where the projection's form does not leave it itself (SdotSide: 3.5 us less).  grid R, block 128.
 template <typename T>
 __global__ __launch_bounds__(128) void k_lowrank_x(Slices t, DeltaGeom g, T* __restrict__ out, int Kp) {
   const int r = blockIdx.x;

@@ -69,6 +69,14 @@ def test_latent_attention_alone(tmp_path, name, dtype):
   one_layer(tmp_path, VH.with_mlp(LATENTS[name], None), dtype, n=75, portions=((1,), (33, 2), (7, 1, 40)))
 
 
+@pytest.mark.parametrize("layer", [dict(heads=3, dim=24, rot=16, vdim=20, rank=40, window=300), dict(heads=5, dim=10, rot=6, vdim=6, rank=130, window=70),
+                                   dict(heads=17, dim=136, rot=32, vdim=48, rank=500, window=40)])
+def test_few_rows_of_latent_attention(tmp_path, layer):
+  """Up to 16 rows take the cache entry beside the key up-projection, and the key splits beside the values' up-projection, as one launch each; 17 the launches of their own.  Value
+  dims that are no multiple of four, one and several key splits, one tile of latents and several.  bfloat16's tolerance (rounding of operands)."""
+  one_layer(tmp_path, VH.with_mlp(VH.latent(**layer), None), "bfloat16", n=96, portions=((16,), (50, 17, 16, 13), (80, 1)))
+
+
 DELTAS = {
     "one head": VH.delta(heads=1, kv_heads=1, dim=8, vdim=8, conv=2),
     "shared keys": VH.delta(heads=6, kv_heads=2, dim=20, vdim=12, conv=4),
