@@ -238,15 +238,15 @@ static int attn_gemm(hipStream_t st, bool ta, bool tb, const bf16_t* A, long lda
   return ta ? gemm_launch<true, true, 64>(st, g) : gemm_launch<false, true, 64>(st, g);
 }
 static void softmax_fwd(hipStream_t st, const float* scores, const int32_t* seg, bf16_t* P, int S, int B, int H) {
-  const dim3 grid(S, B * H);
-  if (S <= 512) hipLaunchKernelGGL(k_t_softmax_fwd_reg<2>, grid, dim3(256), 0, st, scores, seg, P, S, H);
-  else if (S <= 2048) hipLaunchKernelGGL(k_t_softmax_fwd_reg<8>, grid, dim3(256), 0, st, scores, seg, P, S, H);
+  const dim3 grid(S, B * H), waves((S + 3) / 4, B * H);
+  if (S <= 512) hipLaunchKernelGGL(k_t_softmax_fwd_wave<2>, waves, dim3(256), 0, st, scores, seg, P, S, H);
+  else if (S <= 2048) hipLaunchKernelGGL(k_t_softmax_fwd_wave<8>, waves, dim3(256), 0, st, scores, seg, P, S, H);
   else if (S <= 4096) hipLaunchKernelGGL(k_t_softmax_fwd_reg<16>, grid, dim3(256), 0, st, scores, seg, P, S, H);
   else hipLaunchKernelGGL(k_t_softmax_fwd, grid, dim3(256), 0, st, scores, seg, P, S, H);
 }
 static void softmax_bwd(hipStream_t st, const float* dP, const bf16_t* P, bf16_t* dS, int S, int BH) {
-  const dim3 grid(S, BH);
-  if (S <= 512) hipLaunchKernelGGL(k_t_softmax_bwd_reg<2>, grid, dim3(256), 0, st, dP, P, dS, S);
+  const dim3 grid(S, BH), waves((S + 3) / 4, BH);
+  if (S <= 512) hipLaunchKernelGGL(k_t_softmax_bwd_wave<2>, waves, dim3(256), 0, st, dP, P, dS, S);
   else if (S <= 2048) hipLaunchKernelGGL(k_t_softmax_bwd_reg<8>, grid, dim3(256), 0, st, dP, P, dS, S);
   else if (S <= 4096) hipLaunchKernelGGL(k_t_softmax_bwd_reg<16>, grid, dim3(256), 0, st, dP, P, dS, S);
   else hipLaunchKernelGGL(k_t_softmax_bwd, grid, dim3(256), 0, st, dP, P, dS, S);

@@ -42,9 +42,21 @@ static __global__ void k_t_cast_bf16(const float* __restrict__ src, bf16_t* __re
   *reinterpret_cast<uint2*>(dst + blockIdx.y * ld + i) = make_uint2(pack2(f2bf(v.x), f2bf(v.y)), pack2(f2bf(v.z), f2bf(v.w)));
 }
 
+// the sum over the lanes, with those 32, 16, .. 1 away in turn (from 8 on any lane of the other group will do: the lanes of a group hold the same value)
+__device__ __forceinline__ float t_wave_sum(float v) {
+  auto ror = [](float x, auto ctrl) { return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), decltype(ctrl)::value, 0xf, 0xf, true)); };
+  const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+  const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = __uint_as_float(b[0]) + __uint_as_float(b[1]);
+  v += ror(v, std::integral_constant<int, 0x128>());
+  v += ror(v, std::integral_constant<int, 0x124>());
+  v += ror(v, std::integral_constant<int, 0x122>());
+  v += ror(v, std::integral_constant<int, 0x121>());
+  return v;
+}
 __device__ __forceinline__ float t_block_sum(float v, float* red) {   // 256 threads
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+  v = t_wave_sum(v);
   __syncthreads();
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
   __syncthreads();
@@ -233,6 +245,74 @@ static __global__ __launch_bounds__(256) void k_t_softmax_fwd(const float* __res
     p[j] = on ? f2bf(ixt_exp(s[j] - m) / l) : (bf16_t)0;
   }
 }
+// A wave a row, for rows of at most 256 MAXV <= 2048 columns: no wave waits for another (a block a row: 25.7 us for 48 heads of 512 x 512, 510 for 128 of 2048 x 2048, now 14.4 and 390).  The sums are
+// those of the block: lane L adds up what threads L, L + 64, .. of it would, and their waves' sums are added in the same order.
+template <int MAXV>
+static __global__ __launch_bounds__(256) void k_t_softmax_fwd_wave(const float* __restrict__ sc, const int32_t* __restrict__ seg, bf16_t* __restrict__ P, int S, int H) {
+  __shared__ __attribute__((aligned(16))) bf16_t tiles[4][256 * MAXV];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), row = blockIdx.x * 4 + wave;
+  if (row >= S) return;                                    // whole wave: no barrier in here
+  const long bh = blockIdx.y, b = bh / H;
+  const float* s = sc + (bh * S + row) * S;
+  const int32_t* sg = seg + b * S;
+  bf16_t* tile = tiles[wave];
+  const int myseg = sg[row], nv = row / 256 + 1;
+  float v[MAXV][4], m = -INFINITY;
+  int g[MAXV][4];
+#pragma unroll
+  for (int i = 0; i < MAXV; ++i)
+    if (i < nv) {                                          // every load at once
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        const int j = min(i * 256 + w * 64 + lane, row);
+        v[i][w] = s[j]; g[i][w] = sg[j];
+      }
+    }
+  uint32_t on = 0;
+#pragma unroll
+  for (int i = 0; i < MAXV; ++i)
+    if (i < nv) {
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        const bool see = i * 256 + w * 64 + lane <= row && g[i][w] == myseg;
+        on |= see ? 1u << (i * 4 + w) : 0u;
+        m = fmaxf(m, see ? v[i][w] : -INFINITY);
+      }
+    }
+  m = xor_butterfly(m, [](float x, float y) { return fmaxf(x, y); });
+  float l[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  bool small = false;
+#pragma unroll
+  for (int i = 0; i < MAXV; ++i)
+    if (i < nv) {
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        const bool see = on >> (i * 4 + w) & 1u;
+        v[i][w] = see ? ixt_exp(v[i][w] - m) : 0.0f;
+        small = small || (see && v[i][w] < 0x1p-96f);
+        l[w] += v[i][w];
+      }
+    }
+  const float sum = t_wave_sum(l[0]) + t_wave_sum(l[1]) + t_wave_sum(l[2]) + t_wave_sum(l[3]), rl = 1.0f / sum;
+  auto write = [&](auto quotient) {
+#pragma unroll
+    for (int i = 0; i < MAXV; ++i)
+      if (i < nv) {
+#pragma unroll
+        for (int w = 0; w < 4; ++w) tile[i * 256 + w * 64 + lane] = f2bf(quotient(v[i][w]));
+      }
+  };
+  // the quotient by the reciprocal and two corrections, the last of which rounds as a division does where no residue is lost below the normal numbers
+  if (__any(small)) write([&](float e) { return e / sum; });
+  else write([&](float e) {
+    float q = e * rl;
+    q = __builtin_fmaf(__builtin_fmaf(-q, sum, e), rl, q);
+    return __builtin_fmaf(__builtin_fmaf(-q, sum, e), rl, q);
+  });
+  const int n = min(S, nv * 256);
+  bf16_t* out = P + (bh * S + row) * S;
+  for (int j = lane * 8; j < n; j += 512) *reinterpret_cast<u32x4*>(out + j) = *reinterpret_cast<const u32x4*>(tile + j);
+}
 template <int MAXV>
 static __global__ __launch_bounds__(256) void k_t_softmax_fwd_reg(const float* __restrict__ sc, const int32_t* __restrict__ seg, bf16_t* __restrict__ P, int S, int H) {
   __shared__ float red[4];
@@ -286,6 +366,53 @@ static __global__ __launch_bounds__(256) void k_t_softmax_bwd(const float* __res
     const float p = j <= row ? bf2f(P[base + j]) : 0.0f;
     dS[base + j] = j <= row ? f2bf(p * (dP[base + j] - dot)) : (bf16_t)0;
   }
+}
+// a wave a row, as k_t_softmax_fwd_wave: 48 heads of 512 x 512 20.8 us by blocks, now 13.1; 128 of 2048 x 2048, where a wave would hold 32 columns a lane, 413 by blocks and 444 so
+template <int MAXV>
+static __global__ __launch_bounds__(256) void k_t_softmax_bwd_wave(const float* __restrict__ dP, const bf16_t* __restrict__ P, bf16_t* __restrict__ dS, int S) {
+  __shared__ __attribute__((aligned(16))) bf16_t tiles[4][256 * MAXV];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), row = blockIdx.x * 4 + wave;
+  if (row >= S) return;                                    // whole wave: no barrier in here
+  bf16_t* tile = tiles[wave];
+  const int nv = row / 256 + 1, n = min(S, nv * 256);
+  const long base = ((long)blockIdx.y * S + row) * S;
+  float g[MAXV][4];
+  u32x4 p[MAXV / 2];
+#pragma unroll
+  for (int i = 0; i < MAXV; ++i)
+    if (i < nv) {
+#pragma unroll
+      for (int w = 0; w < 4; ++w) g[i][w] = dP[base + min(i * 256 + w * 64 + lane, row)];
+    }
+#pragma unroll
+  for (int i = 0; i < MAXV / 2; ++i)
+    if (i * 512 + lane * 8 < n) p[i] = *reinterpret_cast<const u32x4*>(P + base + i * 512 + lane * 8);
+#pragma unroll
+  for (int i = 0; i < MAXV / 2; ++i)
+    if (i * 512 + lane * 8 < n) *reinterpret_cast<u32x4*>(tile + i * 512 + lane * 8) = p[i];
+  float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int i = 0; i < MAXV; ++i)
+    if (i < nv) {
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        const int j = i * 256 + w * 64 + lane;
+        const bool in = j <= row;
+        s[w] += (in ? g[i][w] : 0.0f) * (in ? bf2f(tile[j]) : 0.0f);
+      }
+    }
+  const float dot = t_wave_sum(s[0]) + t_wave_sum(s[1]) + t_wave_sum(s[2]) + t_wave_sum(s[3]);
+#pragma unroll
+  for (int i = 0; i < MAXV; ++i)
+    if (i < nv) {
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        const int j = i * 256 + w * 64 + lane;
+        const bool in = j <= row;
+        tile[j] = f2bf((in ? bf2f(tile[j]) : 0.0f) * ((in ? g[i][w] : 0.0f) - dot));
+      }
+    }
+  for (int j = lane * 8; j < n; j += 512) *reinterpret_cast<u32x4*>(dS + base + j) = *reinterpret_cast<const u32x4*>(tile + j);
 }
 template <int MAXV>
 static __global__ __launch_bounds__(256) void k_t_softmax_bwd_reg(const float* __restrict__ dP, const bf16_t* __restrict__ P, bf16_t* __restrict__ dS, int S) {

@@ -26,6 +26,10 @@ SHAPES = {
     "large attention tiles": dict(base_emb_dim=72, base_num_query_heads=16, base_num_kv_heads=16, head_dim=128, base_mlp_dim=136, vocab_size=264, max_target_length=264, per_device_batch_size=16.0),
     # a vocabulary of an odd number of 128-byte lines: its rows lie as far apart as they are long, also from 4096 columns on
     "odd lines": dict(base_emb_dim=72, base_num_query_heads=2, base_num_kv_heads=2, head_dim=64, base_mlp_dim=136, vocab_size=4160, max_target_length=72, per_device_batch_size=2.0),
+    # softmax by a wave a row: the last rows of 512 columns' form, a few columns beyond it and beyond 1024
+    "softmax 512": dict(base_emb_dim=64, base_num_query_heads=3, base_num_kv_heads=3, head_dim=64, base_mlp_dim=72, vocab_size=264, max_target_length=504, per_device_batch_size=1.0),
+    "softmax 520": dict(base_emb_dim=64, base_num_query_heads=1, base_num_kv_heads=1, head_dim=64, base_mlp_dim=72, vocab_size=264, max_target_length=520, per_device_batch_size=2.0),
+    "softmax 1032": dict(base_emb_dim=64, base_num_query_heads=2, base_num_kv_heads=1, head_dim=64, base_mlp_dim=72, vocab_size=264, max_target_length=1032, per_device_batch_size=1.0),
     # one row, shorter than any tile
     "short": dict(base_emb_dim=64, base_num_query_heads=2, base_num_kv_heads=1, head_dim=64, base_mlp_dim=72, vocab_size=264, max_target_length=8, per_device_batch_size=1.0),
 }
