@@ -251,6 +251,23 @@ static void softmax_bwd(hipStream_t st, const float* dP, const bf16_t* P, bf16_t
   else if (S <= 4096) hipLaunchKernelGGL(k_t_softmax_bwd_reg<16>, grid, dim3(256), 0, st, dP, P, dS, S);
   else hipLaunchKernelGGL(k_t_softmax_bwd, grid, dim3(256), 0, st, dP, P, dS, S);
 }
+// Rows of 16384 columns and more by sixteen waves (32000 columns 82 -> 76 us for 2048 rows); where two such blocks a CU would have more in work than the memory-side cache holds beside what
+// is written, the LDS keeps it to one (264192 columns: 804 us by two, 737 by one, 971 by blocks of four waves).
+static int xent(hipStream_t st, const bf16_t* logits, const int32_t* targets, const int32_t* seg, bf16_t* dlog, float* row_loss, int n, int V, long ld) {
+  if (V < 16384) {
+    hipLaunchKernelGGL(k_t_xent, dim3(n), dim3(256), 0, st, logits, targets, seg, dlog, row_loss, V, ld);
+  } else {
+    constexpr int two = 2 * 8192 * sizeof(float), one = 96 * 1024;
+    static bool attr_done = false;
+    if (!attr_done) {
+      TCHK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_t_xent_wide), hipFuncAttributeMaxDynamicSharedMemorySize, one));
+      attr_done = true;
+    }
+    hipLaunchKernelGGL(k_t_xent_wide, dim3(n), dim3(1024), (size_t)V * sizeof(bf16_t) * 512 > (size_t)192 << 20 ? one : two, st, logits, targets, seg, dlog, row_loss, V, ld);
+  }
+  TLAUNCH();
+  return IXT_OK;
+}
 // TL_DX: n is the reduction (the layer's outputs), c of the first entry the result; ldw: where the rows of w (TL_XW: and of c) lie further apart than n
 struct TOperand { const bf16_t* x; const bf16_t* w; void* c; int n; long ldw = 0; };
 // TL_DX of several entries: the sum of their products.
@@ -397,7 +414,7 @@ extern "C" int ixt_train_forward_backward(ixt_trainer* t, const int32_t* inputs,
     const int n = T - t0 < t->Tc ? T - t0 : t->Tc;
     const bf16_t* xn = t->xn_f + (long)t0 * E;
     TTRY(gemm(st, TL_XW, n, E, {{xn, pb + t->o_logits, t->logits, V, t->Vp}}, TG_BF16, E));
-    hipLaunchKernelGGL(k_t_xent, dim3(n), dim3(256), 0, st, reinterpret_cast<const bf16_t*>(t->logits), targets + t0, targets_segmentation + t0, t->dlog, t->row_loss + t0, V, t->Vp);
+    TTRY(xent(st, reinterpret_cast<const bf16_t*>(t->logits), targets + t0, targets_segmentation + t0, t->dlog, t->row_loss + t0, n, V, t->Vp));
     // d xn_f = dlogits . W^T ; dW += xn_f^T . dlogits
     TTRY(gemm(st, TL_DX, n, V, {{t->dlog, pb + t->o_logits, t->dxn + (long)t0 * E, V, t->Vp}}, TG_F32, t->Vp, E, nullptr, t->scores, V >= 65536 ? (size_t)B * H * S * S : 0));   // (the score buffer is idle)
     TTRY(gemm(st, TL_DW, E, n, {{xn, t->dlog, t->g + t->o_logits, V, t->Vp}}, t0 == 0 ? TG_F32 : TG_F32_ADD, E));

@@ -537,6 +537,85 @@ static __global__ __launch_bounds__(256) void k_t_xent(const bf16_t* __restrict_
   }
 }
 
+// The same for wide rows, a block of sixteen waves a row and CU: the rows in work (256 of 528 KB) stay in the memory-side cache between the three passes over them
+// (2048 rows of 264192 columns: 971 us a chunk with eight blocks of four waves on a CU, all 2048 rows in work at once and 4.3 GB from memory; now 737).
+// The terms of the sum are worked out 16 bytes of logits a thread and added up by the four waves of the form above, column by column in its order.  grid = Tc, block 1024.
+static __global__ __launch_bounds__(1024) void k_t_xent_wide(const bf16_t* __restrict__ logits, const int32_t* __restrict__ targets, const int32_t* __restrict__ tseg,
+                                                      bf16_t* __restrict__ dlogits, float* __restrict__ row_loss, int V, long ld) {
+  extern __shared__ __attribute__((aligned(16))) float term[];   // [2][8192]
+  __shared__ float red[16];
+  const long row = blockIdx.x;
+  const int tid = threadIdx.x, wave = tid >> 6;
+  const bf16_t* l = logits + row * ld;
+  auto load = [&](int j) { return *reinterpret_cast<const u32x4*>(l + min(j, V - 8)); };      // (V a multiple of 8; past the end: the last eight again)
+  float m = -INFINITY;
+  for (int j = tid * 8; j < V; j += 4 * 8192) {
+    u32x4 w[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) w[u] = load(j + u * 8192);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      float v[8];
+      t_unpack8(w[u], v);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) m = fmaxf(m, v[k]);
+    }
+  }
+  m = xor_butterfly(m, [](float x, float y) { return fmaxf(x, y); });
+  if ((tid & 63) == 0) red[wave] = m;
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < 16; ++k) m = fmaxf(m, red[k]);
+  float s = 0.0f;
+  u32x4 w = load(tid * 8);
+  int buf = 0;
+  for (int j0 = 0; j0 < V; j0 += 8192, buf ^= 8192) {
+    float v[8];
+    t_unpack8(w, v);
+    w = load(j0 + 8192 + tid * 8);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = ixt_exp(v[k] - m);
+    float4* to = reinterpret_cast<float4*>(term + buf + tid * 8);
+    to[0] = make_float4(v[0], v[1], v[2], v[3]); to[1] = make_float4(v[4], v[5], v[6], v[7]);
+    __syncthreads();                                     // (the other buffer is written next: one barrier per tile)
+    if (wave < 4) {
+      const int n = min(32, (V - j0 - tid + 255) >> 8);  // rows of 256 columns that hold this thread's
+      if (n == 32) {
+#pragma unroll
+        for (int i = 0; i < 32; ++i) s += term[buf + i * 256 + tid];
+      } else {
+        for (int i = 0; i < n; ++i) s += term[buf + i * 256 + tid];
+      }
+    }
+  }
+  __syncthreads();
+  s = t_wave_sum(s);
+  if (wave < 4 && (tid & 63) == 0) red[wave] = s;
+  __syncthreads();
+  s = red[0] + red[1] + red[2] + red[3];
+  const float wt = tseg[row] != 0 ? 1.0f : 0.0f;
+  const int tg = targets[row];
+  if (tid == 0) row_loss[row] = wt * (logf(s) + m - bf2f(l[tg]));
+  const float inv = wt / s;
+  for (int j = tid * 8; j < V; j += 2 * 8192) {
+    const u32x4 x[2] = {load(j), load(j + 8192)};
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int at = j + u * 8192;
+      if (at >= V) continue;
+      float v[8];
+      t_unpack8(x[u], v);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[k] = ixt_exp(v[k] - m) * inv;
+      if ((unsigned)(tg - at) < 8u) {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v[k] -= at + k == tg ? wt : 0.0f;
+      }
+      *reinterpret_cast<u32x4*>(dlogits + row * ld + at) = t_pack8(v);
+    }
+  }
+}
+
 // out[i] = 1 where s[i] != 0 (the weight of a target position, train.py:308-309)
 static __global__ void k_t_nonzero(const int32_t* __restrict__ s, float* __restrict__ out, long n) {
   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;

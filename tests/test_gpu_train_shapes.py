@@ -30,6 +30,10 @@ SHAPES = {
     "softmax 512": dict(base_emb_dim=64, base_num_query_heads=3, base_num_kv_heads=3, head_dim=64, base_mlp_dim=72, vocab_size=264, max_target_length=504, per_device_batch_size=1.0),
     "softmax 520": dict(base_emb_dim=64, base_num_query_heads=1, base_num_kv_heads=1, head_dim=64, base_mlp_dim=72, vocab_size=264, max_target_length=520, per_device_batch_size=2.0),
     "softmax 1032": dict(base_emb_dim=64, base_num_query_heads=2, base_num_kv_heads=1, head_dim=64, base_mlp_dim=72, vocab_size=264, max_target_length=1032, per_device_batch_size=1.0),
+    # the loss by sixteen waves a row: the fewest columns, a ragged last tile of 8192 columns, one block a CU
+    "vocabulary 16384": dict(base_emb_dim=64, base_num_query_heads=2, base_num_kv_heads=1, head_dim=64, base_mlp_dim=72, vocab_size=16384, max_target_length=24, per_device_batch_size=1.0),
+    "vocabulary 24584": dict(base_emb_dim=64, base_num_query_heads=2, base_num_kv_heads=1, head_dim=64, base_mlp_dim=72, vocab_size=24584, max_target_length=24, per_device_batch_size=2.0),
+    "vocabulary 200072": dict(base_emb_dim=64, base_num_query_heads=2, base_num_kv_heads=1, head_dim=64, base_mlp_dim=72, vocab_size=200072, max_target_length=16, per_device_batch_size=1.0),
     # one row, shorter than any tile
     "short": dict(base_emb_dim=64, base_num_query_heads=2, base_num_kv_heads=1, head_dim=64, base_mlp_dim=72, vocab_size=264, max_target_length=8, per_device_batch_size=1.0),
 }
