@@ -86,7 +86,7 @@ bool heads_mfma_sizes(int d, int maps, int dv, bool f32, int* dkp, int* dvp);
 
 // What surrounds a sublayer: the norms behind it and in front of the next one, its own hyper-connection and the next one's (nullptr: there is none), the
 // token shift in front of the next one.  to_cat: the next thing is the start of a pass, which takes x as it is
-struct Around { NormW post, pre; const float *hc, *hc_next; const float* mu = nullptr; float* shift = nullptr; bool to_cat = false; };
+struct Around { NormW post, pre; const float *hc, *hc_next; const float* mu = nullptr; float* shift = nullptr; bool to_cat = false, to_head = false; };
 // A sublayer's output: slices t, or the weighted sum of a row's expert outputs among them (pos, wts, top); add, times addw, and bias, times fbias, join it.
 // fresh: it takes the place of x
 struct SubOut { Slices t, add; const float* addw; const int32_t* pos; const float* wts; int top; const float* bias = nullptr; float fbias = 1.0f; bool fresh = false; };

@@ -1090,14 +1090,14 @@ static int hybrid_moe(ixt_ctx* c, const HLayer& L, const HLayer& W, int R, hipSt
   return hdot_grouped<T>(c, (const T*)m->mhact, W.down, W.down_stride, rows_g, align, m->mrb, c->part, c->part_floats, st, out);
 }
 
-// logits of rows lrows[i] (or lrow0 + i) of the residual stream, NLmax at a time
+// logits of rows lrows[i] (or lrow0 + i) of the residual stream, NLmax at a time; normed: all rows, and their norm is there
 template <typename T>
-static int hybrid_logits(ixt_ctx* c, int R, int lrow0, int nl, const int32_t* lrows, int32_t* argmax_out, float* logits_out, hipStream_t st) {
+static int hybrid_logits(ixt_ctx* c, int R, int lrow0, int nl, const int32_t* lrows, int32_t* argmax_out, float* logits_out, hipStream_t st, bool normed = false) {
   HybridModel* m = c->hy;
   const int nblk = (m->V + 1023) / 1024;
   for (int i0 = 0; i0 < nl; i0 += c->NLmax) {
     const int n = std::min(c->NLmax, nl - i0);
-    TRY((hybrid_final_norm<T>(c, R, n, lrows ? lrows + i0 : nullptr, lrow0 + i0, st)));
+    if (!normed) TRY((hybrid_final_norm<T>(c, R, n, lrows ? lrows + i0 : nullptr, lrow0 + i0, st)));
     Slices t;
     TRY(hdot<T>(c, (const T*)m->xn, m->head, n, c->part, c->part_floats, st, &t));
     hipLaunchKernelGGL(k_head_post, dim3(nblk, n), dim3(256), 0, st, t, m->V, m->logit_scale, c->sample_cols, logits_out ? logits_out + (size_t)i0 * m->V : nullptr, c->amax_val, c->amax_idx);
@@ -1117,7 +1117,7 @@ static int hybrid_dot_norm(ixt_ctx* c, const T* v, const HMat& w, const Around& 
     const bool small = R <= c->small_rows && sdot_plan(c, GEPI_TANHNORM, false, w.Kp, w.Np, R).ok;
     if (m->norm_kind == IXT_NORM_TANH && m->streams == 0 && ar.mu == nullptr && !ar.to_cat && bias == nullptr && (small || R >= c->ring_min_rows)) {
       GemmEpi e{};
-      e.act = (bf16_t*)m->xb;
+      e.act = (bf16_t*)(ar.to_head ? m->xn : m->xb);
       e.tn = TanhNormEpi{post.w, post.b, post.alpha, pre.w, pre.b, pre.alpha, m->x, routed && pre.w != nullptr ? m->h32 : nullptr, m->E, m->Ep};
       if (small) return launch_sdot(c, GEPI_TANHNORM, false, v, nullptr, (const bf16_t*)w.w, w.Kp, w.Np, R, e, st);
       return launch_ring(c, GEPI_TANHNORM, v, (const bf16_t*)w.w, w.Kp, w.Np, R, e, false, st);
@@ -1143,8 +1143,10 @@ static int forward_rows_hybrid_t(ixt_ctx* c, int R, const int32_t* tokens, int l
     const HLayer& W = m->layers[m->layers[i].src];
     return Around{none, W.n1, nullptr, W.hc1, W.mu, m->layers[i].shift, false};
   };
-  auto before = [&](size_t i) {                                    // what a sublayer in front of run i leaves (the head's norm is taken of the wanted rows only)
-    if (i >= m->layers.size()) return Around{none, none, nullptr, nullptr};
+  // every row is wanted (decode): the last sublayer leaves the head's operand itself, a launch less (4.7 us of 8 rows)
+  const bool normed = nl == R && lrow0 == 0 && lrows == nullptr && R <= c->NLmax && m->streams == 0;
+  auto before = [&](size_t i) {                                    // what a sublayer in front of run i leaves (of a few wanted rows the head's norm is a launch of its own)
+    if (i >= m->layers.size()) return Around{none, normed ? m->fnorm : none, nullptr, nullptr, nullptr, nullptr, false, normed};
     if (m->layers[i].c.loop_pass >= 0) return Around{none, none, nullptr, nullptr, nullptr, nullptr, true};
     return entry(i);
   };
@@ -1194,7 +1196,7 @@ static int forward_rows_hybrid_t(ixt_ctx* c, int R, const int32_t* tokens, int l
     }
   }
   c->h_final_rows = R;
-  if (nl > 0) TRY((hybrid_logits<T>(c, R, lrow0, nl, lrows, argmax_out, logits_out, st)));
+  if (nl > 0) TRY((hybrid_logits<T>(c, R, lrow0, nl, lrows, argmax_out, logits_out, st, normed)));
   return IXT_OK;
 }
 int forward_rows_hybrid(ixt_ctx* c, int R, const int32_t* tokens, int len_hint, int lrow0, int nl, const int32_t* lrows, int32_t* argmax_out, float* logits_out, bool decode,

@@ -236,7 +236,7 @@ static __global__ __launch_bounds__(1024) void k_segments(int R, int32_t* row_ac
     if (row_active[r] && starts(r)) last = r;
   s_last[tid] = last;
   __syncthreads();
-  for (int off = 1; off < 1024; off <<= 1) {               // inclusive maximum over the threads before and at this one
+  for (int off = 1; off < min(R, 1024); off <<= 1) {       // inclusive maximum over the threads before and at this one (threads behind R hold none; all ten steps took 3 us)
     const int v = tid >= off ? s_last[tid - off] : -1;
     __syncthreads();
     s_last[tid] = max(s_last[tid], v);

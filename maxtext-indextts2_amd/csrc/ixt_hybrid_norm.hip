@@ -8,7 +8,7 @@ int hybrid_norm(ixt_ctx* c, const SubOut& o, const Around& ar, bool routed, int 
   HybridModel* m = c->hy;
   const bool later = ar.mu != nullptr && !single;
   float* h32 = (routed || later) && ar.pre.w != nullptr ? m->h32 : nullptr;
-  T* to = later ? nullptr : (T*)(ar.to_cat ? m->cat : m->xb);
+  T* to = later ? nullptr : (T*)(ar.to_head ? m->xn : ar.to_cat ? m->cat : m->xb);
   const ShiftArgs sh = ar.mu != nullptr && single ? ShiftArgs{ar.mu, ar.shift, c->row_slot, c->row_pos, c->row_active, m->parity} : ShiftArgs{};
   const HyperW hc{ar.hc_next, ar.hc ? ar.hc + HC_MAX : nullptr, ar.hc ? ar.hc + 2 * HC_MAX : nullptr};
   const SubNormArgs a{o.t, o.add, o.addw, o.pos, o.wts, o.top, ar.post, ar.pre, m->eps, m->E, m->Ep, m->streams, hc, o.bias, o.fbias, o.fresh ? 1 : 0, sh, ar.to_cat ? 2 * m->Ep : m->Ep};
