@@ -1312,7 +1312,7 @@ static int launch_attention_partials(ixt_ctx* c, int layer, int R, int len_hint,
 }
 
 // ---- few rows: k_sdot / k_attn_small (ixt_small.h)
-SdotPlan sdot_plan(const ixt_ctx* c, int epi, bool norm, int K, int N, int R) {
+SdotPlan sdot_plan(const ixt_ctx* c, int epi, bool norm, int K, int N, int R, bool rows) {
   SdotPlan p{};
   p.chains = (K + IXT_CHAIN - 1) / IXT_CHAIN;
   p.rpl = 0;
@@ -1321,19 +1321,21 @@ SdotPlan sdot_plan(const ixt_ctx* c, int epi, bool norm, int K, int N, int R) {
   // tiles per block: the blocks of a norm-fused launch each norm the rows for themselves, two tiles share that (QKV at C2, 8 rows:
   // 11.3 us with two tiles per block against 14.3 with one; the plain forms are fastest with one: profiles/r03_b8_by_grid.txt)
   int tpb = c->small_tpb > 0 ? c->small_tpb : ((epi == GEPI_SWIGLU || norm) ? 2 : 1);
+  if (rows) tpb = epi == GEPI_SWIGLU ? 4 : 2;               // (SDOT_ROWS rows: two units of a row a wave, four where a CU has one block)
   if (epi == GEPI_SWIGLU && (tpb & 1)) ++tpb;
   while (tpb > 1 && p.chains * tpb > 16) tpb -= (epi == GEPI_SWIGLU ? 2 : 1);
-  if (tpb > ntile) tpb = ntile;
+  if (tpb > ntile && !rows) tpb = ntile;
   p.tpb = tpb;
   // tiles for half of the CUs at most: half a tile a block (2048 columns; from 129 tiles on whole ones fill more than half of the chip, and twice the blocks would read the rows twice as often)
-  p.half = (epi == GEPI_F32 || epi == GEPI_TANHNORM) && !norm && tpb == 1 && ntile <= 128;
+  p.half = (epi == GEPI_F32 || epi == GEPI_TANHNORM) && !norm && !rows && tpb == 1 && ntile <= 128;
   const int nblk = (K / 8 + 63) / 64;
-  p.lds = ((size_t)(K / 8) << p.rpl) * 16 + (size_t)p.chains * tpb * 1024 + (norm ? 1024 + (size_t)(K / 8) * 16 : 0);
+  p.lds = ((size_t)(K / 8) << p.rpl) * 16 + (size_t)p.chains * tpb * 1024 + (rows ? 1024 : norm ? 1024 + (size_t)(K / 8) * 16 : 0);
   p.ok = R >= 1 && R <= 16 && R * nblk <= 240 && K % IXT_MK == 0 && N % 16 == 0 && p.chains * tpb <= 16 && tpb >= 1 && (epi != GEPI_SWIGLU || tpb % 2 == 0) && p.lds <= 150 * 1024;
+  if (rows) p.ok = p.ok && R <= SDOT_ROWS && K <= 2048 && tpb == (epi == GEPI_SWIGLU ? 4 : 2) && (epi == GEPI_SWIGLU || epi == GEPI_F32);
   return p;
 }
 
-template <int EPI, bool NORM>
+template <int EPI, int NORM>
 static int sdot_t(const SdotArgs& a, const SdotPlan& p, hipStream_t st) {
   const dim3 grid(a.main_blocks + (a.pf_n ? p.pf_blocks : 0)), block(64 * p.chains * p.tpb);
   if constexpr ((EPI == GEPI_F32 || EPI == GEPI_TANHNORM) && !NORM) {
@@ -1355,7 +1357,7 @@ static int sdot_set_attributes() {
 #define SATTR(E_, ...) HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_sdot<E_, __VA_ARGS__>), hipFuncAttributeMaxDynamicSharedMemorySize, 156 * 1024))
   SATTR(GEPI_QKV, true); SATTR(GEPI_QKV, false); SATTR(GEPI_RESID, true); SATTR(GEPI_RESID, false);
   SATTR(GEPI_SWIGLU, true); SATTR(GEPI_SWIGLU, false); SATTR(GEPI_F32, true); SATTR(GEPI_F32, false); SATTR(GEPI_TANHNORM, false); SATTR(GEPI_ACT, false);
-  SATTR(GEPI_F32, false, true); SATTR(GEPI_TANHNORM, false, true);
+  SATTR(GEPI_F32, false, true); SATTR(GEPI_TANHNORM, false, true); SATTR(GEPI_F32, 2); SATTR(GEPI_SWIGLU, 2);
 #undef SATTR
   done = true;
   return IXT_OK;
@@ -1363,13 +1365,14 @@ static int sdot_set_attributes() {
 
 // x: NORM: hidden rows [R][K] row-major (+ scale); else activations in xidx layout.  w: widx layout.
 int launch_sdot(ixt_ctx* c, int epi, bool norm, const bf16_t* x, const bf16_t* scale, const bf16_t* w, int K, int N, int R, const GemmEpi& e,
-                       hipStream_t st, const bf16_t* pf, size_t pf_elems, const SdotSide* side) {
-  SdotPlan p = sdot_plan(c, epi, norm, K, N, R);
+                       hipStream_t st, const bf16_t* pf, size_t pf_elems, const SdotSide* side, const SdotRows* rows) {
+  SdotPlan p = sdot_plan(c, epi, norm, K, N, R, rows != nullptr);
   if (!p.ok) return set_err(IXT_ERR_UNSUPPORTED, "sdot: %d rows x K %d x N %d does not fit the few-rows form", R, K, N);
   SdotArgs a;
   a.x = x; a.scale = scale; a.eps = c->cfg.normalization_layer_epsilon; a.w = reinterpret_cast<const u32x4*>(w);
   a.K = K; a.N = N; a.R = R; a.rpl = p.rpl; a.tpb = p.tpb; a.chains = p.chains; a.e = e;
   if (side != nullptr) a.side = *side;
+  if (rows != nullptr) a.rows = *rows;
   a.main_blocks = p.half ? N / 8 : (N / 16 + p.tpb - 1) / p.tpb;
   const bool prefetch = c->small_prefetch && pf != nullptr && pf_elems > 0;
   a.pf = prefetch ? reinterpret_cast<const u32x4*>(pf) : nullptr;
@@ -1377,7 +1380,8 @@ int launch_sdot(ixt_ctx* c, int epi, bool norm, const bf16_t* x, const bf16_t* s
   p.pf_blocks = c->small_prefetch_blocks;
   const int ti = timing_begin(c, st, (double)K * N * 2.0 + (double)R * K * 2.0);
   int rc = IXT_ERR_UNSUPPORTED;
-  if (epi == GEPI_QKV) rc = norm ? sdot_t<GEPI_QKV, true>(a, p, st) : sdot_t<GEPI_QKV, false>(a, p, st);
+  if (rows != nullptr) rc = epi == GEPI_SWIGLU ? sdot_t<GEPI_SWIGLU, 2>(a, p, st) : sdot_t<GEPI_F32, 2>(a, p, st);
+  else if (epi == GEPI_QKV) rc = norm ? sdot_t<GEPI_QKV, true>(a, p, st) : sdot_t<GEPI_QKV, false>(a, p, st);
   else if (epi == GEPI_RESID) rc = norm ? sdot_t<GEPI_RESID, true>(a, p, st) : sdot_t<GEPI_RESID, false>(a, p, st);
   else if (epi == GEPI_SWIGLU) rc = norm ? sdot_t<GEPI_SWIGLU, true>(a, p, st) : sdot_t<GEPI_SWIGLU, false>(a, p, st);
   else if (epi == GEPI_F32) rc = norm ? sdot_t<GEPI_F32, true>(a, p, st) : sdot_t<GEPI_F32, false>(a, p, st);

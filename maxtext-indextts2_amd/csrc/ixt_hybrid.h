@@ -62,7 +62,10 @@ struct HybridModel {
   HMat loop_in;
   float* loop_step = nullptr;                    // [passes][Ep]
   // workspaces
-  float *x = nullptr, *part2 = nullptr, *h32 = nullptr;      // h32: a routed layer's normed input in f32
+  float *x = nullptr, *x0 = nullptr, *x1 = nullptr;          // the residual stream: x0 between passes, inside one either (SdotRows)
+  float *ride_t = nullptr;                       // a sublayer's output whose norm the next product takes in
+  struct { bool on = false; const float *t = nullptr, *w = nullptr; int ldt = 0; } ride;
+  float *part2 = nullptr, *h32 = nullptr;      // h32: a routed layer's normed input in f32
   size_t part2_floats = 0;
   void *cat = nullptr;                           // a loop: act of [x | embedding output], Ep columns each
   void* scan_t = nullptr;                        // the operand of a scan's third projection

@@ -676,7 +676,8 @@ int hybrid_init(ixt_ctx* c) {
   m->part2_floats = part2; TRY(h_allocf(c, &m->part2, part2 + 4));
   m->part3_floats = part3; TRY(h_allocf(c, &m->part3, part3 + 4));
   TRY(h_alloc(c, &m->scan_t, (scan_t + 8) * m->esz)); TRY(h_allocf(c, &m->scan_u, scan_u + 4)); TRY(h_allocf(c, &m->scan_sum, scan_s + 4));
-  TRY(h_allocf(c, &m->x, (size_t)R * std::max(1, m->streams) * m->E));
+  TRY(h_allocf(c, &m->x0, (size_t)R * std::max(1, m->streams) * m->E)); TRY(h_allocf(c, &m->x1, (size_t)SDOT_ROWS * m->E)); TRY(h_allocf(c, &m->ride_t, (size_t)SDOT_ROWS * up_to(m->E, 16)));
+  m->x = m->x0;
   TRY(h_allocf(c, &m->ret_u, ret_u + 4)); TRY(h_allocf(c, &m->chunk, max_chunks)); TRY(h_allocf(c, &m->sgate, (size_t)R + 4));
   TRY(h_alloc(c, &m->xb, (size_t)Rp * m->Ep * m->esz));
   TRY(h_alloc(c, &m->act, (size_t)Rp * act_k * m->esz));
@@ -743,16 +744,34 @@ int hybrid_copy_group(ixt_ctx* c, int src, int dst, int npages, hipStream_t st) 
 }
 
 // ---------------------------------------------------------------------------------------------------- the forward pass
+// A sublayer's output, its RMS norm and the residual inside the next product, every block for itself, under its weights' way (few rows): a launch less
+template <typename T> static bool norm_rides(ixt_ctx* c, const HMat& w, const Around& ar, bool routed, int R, const float* bias, const HMat* next, int epi) {
+  const HybridModel* m = c->hy;
+  return sizeof(T) == 2 && next != nullptr && m->norm_kind == IXT_NORM_RMS && m->streams == 0 && m->E == m->Ep && R <= std::min(SDOT_ROWS, c->small_rows) && m->tap == nullptr && !routed && ar.mu == nullptr &&
+         !ar.to_cat && !ar.to_head && ar.post.w != nullptr && ar.pre.w == nullptr && bias == nullptr && next->Np <= 65536 && sdot_plan(c, GEPI_F32, false, w.Kp, w.Np, R).ok && sdot_plan(c, epi, false, next->Kp, next->Np, R, true).ok;
+}
+// a pending norm's rows for the product of operand x, whose launch leaves the residual stream in the other buffer
+static bool take_ride(HybridModel* m, const void* x, SdotRows* rows) {
+  if (!m->ride.on || x != m->xb) return false;
+  float* to = m->x == m->x0 ? m->x1 : m->x0;
+  *rows = SdotRows{m->x, m->ride.t, m->ride.w, to, m->ride.ldt, m->eps};
+  m->x = to;
+  m->ride.on = false;
+  return true;
+}
 // side: asks for columns as the next operand, too; its x is nullptr afterwards where the form does not have that
 template <typename T> static int hdot(ixt_ctx* c, const T* x, const HMat& w, int R, float* out, size_t out_floats, hipStream_t st, Slices* res, SdotSide* side = nullptr);
 template <> int hdot<bf16_t>(ixt_ctx* c, const bf16_t* x, const HMat& w, int R, float* out, size_t out_floats, hipStream_t st, Slices* res, SdotSide* side) {
-  if (R <= c->small_rows && (size_t)R * w.Np <= out_floats && w.Np <= 65536 && sdot_plan(c, GEPI_F32, false, w.Kp, w.Np, R).ok) {     // few rows: one slice
+  SdotRows rows;
+  const bool riding = take_ride(c->hy, x, &rows);
+  if (R <= c->small_rows && (size_t)R * w.Np <= out_floats && w.Np <= 65536 && sdot_plan(c, GEPI_F32, false, w.Kp, w.Np, R, riding).ok) {     // few rows: one slice
     GemmEpi e{};
     e.out = out;
-    TRY(launch_sdot(c, GEPI_F32, false, x, nullptr, (const bf16_t*)w.w, w.Kp, w.Np, R, e, st, nullptr, 0, side));
+    TRY(launch_sdot(c, GEPI_F32, false, x, nullptr, (const bf16_t*)w.w, w.Kp, w.Np, R, e, st, nullptr, 0, side, riding ? &rows : nullptr));
     *res = Slices{out, 1, (size_t)R * w.Np, w.Np};
     return IXT_OK;
   }
+  if (riding) return set_err(IXT_ERR_INVALID, "a product that does not take its rows' norm in");
   if (side != nullptr) side->x = nullptr;
   DotResult dr;
   TRY(launch_dot(c, x, (const bf16_t*)w.w, w.Kp, w.Np, R, out, out_floats, false, st, &dr));
@@ -851,11 +870,14 @@ template <> int hglu<bf16_t>(ixt_ctx* c, const bf16_t* x, const HMat& w, size_t 
     e.act = out; e.glu = kind; e.glu_limit = limit; e.rb_exp = rb; e.wstride = stride / 8;
     return launch_ring(c, GEPI_SWIGLU, x, (const bf16_t*)w.w, w.Kp, w.Np, rows, e, false, st);
   }
-  if (!rb && rows <= c->small_rows && sdot_plan(c, GEPI_SWIGLU, false, w.Kp, w.Np, rows).ok) {
+  SdotRows apart;
+  const bool riding = !rb && take_ride(c->hy, x, &apart);
+  if (!rb && rows <= c->small_rows && sdot_plan(c, GEPI_SWIGLU, false, w.Kp, w.Np, rows, riding).ok) {
     GemmEpi e{};
     e.act = out; e.glu = kind; e.glu_limit = limit;
-    return launch_sdot(c, GEPI_SWIGLU, false, x, nullptr, (const bf16_t*)w.w, w.Kp, w.Np, rows, e, st);
+    return launch_sdot(c, GEPI_SWIGLU, false, x, nullptr, (const bf16_t*)w.w, w.Kp, w.Np, rows, e, st, nullptr, 0, nullptr, riding ? &apart : nullptr);
   }
+  if (riding) return set_err(IXT_ERR_INVALID, "a product that does not take its rows' norm in");
   const int rowblocks = (rows + 15) / 16, nrb = rb ? 1 : (rowblocks >= 3 ? 4 : rowblocks), zblocks = (rowblocks + nrb - 1) / nrb, ntile = w.Np / 16;
   dim3 grid((((ntile + 3) / 4 + 7) / 8) * 8 * zblocks, 1, 1);
   const u32x4 *xp = reinterpret_cast<const u32x4*>(x), *wp = reinterpret_cast<const u32x4*>(w.w);
@@ -1107,10 +1129,10 @@ static int hybrid_logits(ixt_ctx* c, int R, int lrow0, int nl, const int32_t* lr
   return IXT_OK;
 }
 
-// a sublayer's last product and what follows it: x <- x + post(W v), the next operand pre(x).  Tanh norms ride in the product's epilogue where the whole
+// a sublayer's last product and what follows it: x <- x + post(W v), the next operand pre(x); next, epi: the one product that takes it (nullptr: none, or several).  Tanh norms ride in the product's epilogue where the whole
 // sum is in one place.
 template <typename T>
-static int hybrid_dot_norm(ixt_ctx* c, const T* v, const HMat& w, const Around& ar, bool routed, int R, bool single, const float* bias, float fbias, hipStream_t st) {
+static int hybrid_dot_norm(ixt_ctx* c, const T* v, const HMat& w, const Around& ar, bool routed, int R, bool single, const float* bias, float fbias, const HMat* next, int epi, hipStream_t st) {
   HybridModel* m = c->hy;
   [[maybe_unused]] const NormW &post = ar.post, &pre = ar.pre;
   if constexpr (sizeof(T) == 2) {
@@ -1124,6 +1146,11 @@ static int hybrid_dot_norm(ixt_ctx* c, const T* v, const HMat& w, const Around& 
     }
   }
   Slices t;
+  if (norm_rides<T>(c, w, ar, routed, R, bias, next, epi)) {
+    TRY(hdot<T>(c, v, w, R, m->ride_t, (size_t)SDOT_ROWS * w.Np, st, &t));
+    m->ride.on = true; m->ride.t = t.p; m->ride.ldt = t.ncols; m->ride.w = post.w;
+    return IXT_OK;
+  }
   TRY(hdot<T>(c, v, w, R, c->part, c->part_floats, st, &t));
   SubOut o{t};
   o.bias = bias; o.fbias = fbias;
@@ -1138,6 +1165,7 @@ static int forward_rows_hybrid_t(ixt_ctx* c, int R, const int32_t* tokens, int l
   if (m->recurrent || m->maxH > 0)
     hipLaunchKernelGGL(k_segments, dim3(1), dim3(1024), 0, st, R, c->row_active, c->row_slot, c->row_pos, m->row_seg, m->row_j, m->seg, m->chunk, m->nseg, m->state_len, m->parity, m->claim, c->G,
                      m->recurrent ? 1 : 0, m->err, m->head_rb, m->maxH * (Rp / 16), Rp / 16);
+  m->x = m->x0; m->ride.on = false;
   const NormW none{};
   auto entry = [&](size_t i) {                                     // what stands in front of the mixer of run i
     const HLayer& W = m->layers[m->layers[i].src];
@@ -1172,11 +1200,15 @@ static int forward_rows_hybrid_t(ixt_ctx* c, int R, const int32_t* tokens, int l
     const bool ffn = L.c.ffn != IXT_FFN_NONE;
     Around ar1 = ffn ? Around{none, W.n2, nullptr, W.hc2} : before(i + 1), ar2 = before(i + 1);
     ar1.post = W.n1b; ar1.hc = W.hc1; ar2.post = W.n2b; ar2.hc = W.hc2;
-    TRY((hybrid_dot_norm<T>(c, (const T*)m->act, W.o, ar1, L.c.ffn == IXT_FFN_MOE, R, decode, W.obias, L.c.mix_scale, st)));
+    const HLayer* behind = i + 1 < m->layers.size() ? &m->layers[i + 1] : nullptr;      // whose first product is the one that reads the rows
+    if (behind && (behind->c.loop_pass >= 0 || behind->c.mixer == IXT_MIX_SCAN || column_mixer(behind->c))) behind = nullptr;
+    const HMat* in = behind ? &m->layers[behind->src].in : nullptr;
+    const bool unit = L.c.ffn == IXT_FFN_DENSE && L.c.glu < IXT_ACT_RELU2;
+    TRY((hybrid_dot_norm<T>(c, (const T*)m->act, W.o, ar1, L.c.ffn == IXT_FFN_MOE, R, decode, W.obias, L.c.mix_scale, unit ? &W.gu : ffn ? nullptr : in, unit ? GEPI_SWIGLU : GEPI_F32, st)));
     if (L.c.ffn == IXT_FFN_DENSE) {
       TRY(L.c.glu < IXT_ACT_RELU2 ? hglu<T>(c, (const T*)m->xb, W.gu, 0, R, 0, nullptr, L.c.glu, L.c.glu_limit, (T*)m->hact, st)
                                   : hact_unit<T>(c, (const T*)m->xb, W.gu, 0, R, 0, nullptr, L.c.glu, W.unit_par, (T*)m->hact, st));
-      TRY((hybrid_dot_norm<T>(c, (const T*)m->hact, W.down, ar2, false, R, decode, nullptr, 1.0f, st)));
+      TRY((hybrid_dot_norm<T>(c, (const T*)m->hact, W.down, ar2, false, R, decode, nullptr, 1.0f, in, GEPI_F32, st)));
     } else if (L.c.ffn == IXT_FFN_MOE) {
       Slices t, shared{};
       const float* addw = L.c.shared_gate ? m->sgate : nullptr;

@@ -424,7 +424,7 @@ struct SubNormArgs {
   const float* bias; float fbias; int fresh; ShiftArgs shift; int Kp;      // Kp: columns of the operand's rows
 };
 template <typename T, int NI, int KIND, int SM>
-__global__ __launch_bounds__(256) void k_sub_norm(SubNormArgs a, float* __restrict__ x, T* __restrict__ xb, float* __restrict__ h32) {
+__global__ __launch_bounds__(256) void k_sub_norm(SubNormArgs a, float* x, float* xo, T* __restrict__ xb, float* __restrict__ h32) {      // xo: where x goes (streams: x itself)
   __shared__ float red[4];
   const Slices &t = a.t, &add = a.add;
   const int32_t* __restrict__ pos = a.pos;
@@ -578,11 +578,11 @@ __global__ __launch_bounds__(256) void k_sub_norm(SubNormArgs a, float* __restri
       if (vec) {
 #pragma unroll
         for (int q = 0; q < 8; q += 4)
-          if (k0 + q < E) *reinterpret_cast<float4*>(x + (size_t)r * E + k0 + q) = make_float4(xv[i][q], xv[i][q + 1], xv[i][q + 2], xv[i][q + 3]);
+          if (k0 + q < E) *reinterpret_cast<float4*>(xo + (size_t)r * E + k0 + q) = make_float4(xv[i][q], xv[i][q + 1], xv[i][q + 2], xv[i][q + 3]);
       } else {
 #pragma unroll
         for (int j = 0; j < 8; ++j)
-          if (k0 + j < E) x[(size_t)r * E + k0 + j] = xv[i][j];
+          if (k0 + j < E) xo[(size_t)r * E + k0 + j] = xv[i][j];
       }
     }
   }

@@ -6,13 +6,14 @@
 template <typename T>
 int hybrid_norm(ixt_ctx* c, const SubOut& o, const Around& ar, bool routed, int R, bool single, hipStream_t st) {
   HybridModel* m = c->hy;
+  if (m->ride.on) return set_err(IXT_ERR_INVALID, "a norm is pending");
   const bool later = ar.mu != nullptr && !single;
   float* h32 = (routed || later) && ar.pre.w != nullptr ? m->h32 : nullptr;
   T* to = later ? nullptr : (T*)(ar.to_head ? m->xn : ar.to_cat ? m->cat : m->xb);
   const ShiftArgs sh = ar.mu != nullptr && single ? ShiftArgs{ar.mu, ar.shift, c->row_slot, c->row_pos, c->row_active, m->parity} : ShiftArgs{};
   const HyperW hc{ar.hc_next, ar.hc ? ar.hc + HC_MAX : nullptr, ar.hc ? ar.hc + 2 * HC_MAX : nullptr};
   const SubNormArgs a{o.t, o.add, o.addw, o.pos, o.wts, o.top, ar.post, ar.pre, m->eps, m->E, m->Ep, m->streams, hc, o.bias, o.fbias, o.fresh ? 1 : 0, sh, ar.to_cat ? 2 * m->Ep : m->Ep};
-#define HNORM_S(NI_, KIND_, SM_) hipLaunchKernelGGL((k_sub_norm<T, NI_, KIND_, SM_>), dim3(R), dim3(256), 0, st, a, m->x, to, h32)
+#define HNORM_S(NI_, KIND_, SM_) hipLaunchKernelGGL((k_sub_norm<T, NI_, KIND_, SM_>), dim3(R), dim3(256), 0, st, a, m->x, m->x0, to, h32)
 #define HNORM(NI_, KIND_) do { if (m->streams == 0) HNORM_S(NI_, KIND_, 0); else if (m->streams <= 4) HNORM_S(NI_, KIND_, 4); else HNORM_S(6, KIND_, HC_MAX); } while (0)
 #define HNORM_K(NI_) do { if (m->norm_kind == IXT_NORM_TANH) HNORM(NI_, IXT_NORM_TANH); else if (m->norm_kind == IXT_NORM_LAYER) HNORM(NI_, IXT_NORM_LAYER); else if (m->norm_kind == IXT_NORM_ONE) HNORM(NI_, IXT_NORM_ONE); else HNORM(NI_, IXT_NORM_RMS); } while (0)
   if (m->Ep <= 2048) HNORM_K(1); else if (m->Ep <= 4096) HNORM_K(2); else if (m->Ep <= 8192) HNORM_K(4); else HNORM_K(6);
@@ -20,6 +21,7 @@ int hybrid_norm(ixt_ctx* c, const SubOut& o, const Around& ar, bool routed, int 
 #undef HNORM
 #undef HNORM_S
   LAUNCHCHK();
+  if (o.t.n > 0) m->x = m->x0;
   if (later) {
     hipLaunchKernelGGL((k_token_shift<T>), dim3(R), dim3(256), 0, st, m->h32, ar.mu, ar.shift, m->row_seg, m->row_j, m->seg, m->E, m->Ep, (T*)m->xb);
     LAUNCHCHK();

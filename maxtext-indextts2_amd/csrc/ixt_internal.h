@@ -203,12 +203,15 @@ static int dmalloc(ixt_ctx* c, T** p, size_t n) {
 struct DotResult { int slices; size_t slice_stride; int ntiles; };
 // k_sdot: columns [a, a + na) and [b, b + nb) of an f32 result side by side as the next dot's operand, too (zeros up to Kp); x nullptr: none
 struct SdotSide { bf16_t* x = nullptr; int a = 0, na = 0, b = 0, nb = 0, Kp = 0; };
+// k_sdot: rows that are still apart: x + t / rms(t) (1 + w) is the residual stream (f32, to x_out, by one block) and the operand.  x_out != x
+struct SdotRows { const float *x, *t, *w; float* x_out; int ldt; float eps; };
+#define SDOT_ROWS 8             // rows of that form
 struct SdotPlan { int chains, tpb, rpl; size_t lds; bool ok, half; int pf_blocks; };
 int launch_ring(ixt_ctx* c, int epi, const bf16_t* x, const bf16_t* w, int K, int N, int R, const GemmEpi& e, bool split, hipStream_t st, int wring = 0, int* wave_cols = nullptr);
 int launch_dot(ixt_ctx* c, const bf16_t* x, const bf16_t* w, int K, int N, int R, float* out, size_t out_floats, bool force_full, hipStream_t st, DotResult* res, bool no_ring = false);
-SdotPlan sdot_plan(const ixt_ctx* c, int epi, bool norm, int K, int N, int R);
+SdotPlan sdot_plan(const ixt_ctx* c, int epi, bool norm, int K, int N, int R, bool rows = false);
 int launch_sdot(ixt_ctx* c, int epi, bool norm, const bf16_t* x, const bf16_t* scale, const bf16_t* w, int K, int N, int R, const GemmEpi& e, hipStream_t st,
-                const bf16_t* pf = nullptr, size_t pf_elems = 0, const SdotSide* side = nullptr);
+                const bf16_t* pf = nullptr, size_t pf_elems = 0, const SdotSide* side = nullptr, const SdotRows* rows = nullptr);
 // ---- few rows, all layers in one launch (ixt_step.hip)
 int step_init(ixt_ctx* c);
 bool step_fits(const ixt_ctx* c, int R);

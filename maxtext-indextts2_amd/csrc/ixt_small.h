@@ -36,6 +36,10 @@ __device__ __forceinline__ void ixt_prefetch(const u32x4* __restrict__ p, size_t
   }
 }
 
+__device__ __forceinline__ void rows_load8(const float* __restrict__ p, float* o) {       // p % 16 bytes == 0
+  const float4 u = *reinterpret_cast<const float4*>(p), v = *reinterpret_cast<const float4*>(p + 4);
+  o[0] = u.x; o[1] = u.y; o[2] = u.z; o[3] = u.w; o[4] = v.x; o[5] = v.y; o[6] = v.z; o[7] = v.w;
+}
 struct SdotArgs {
   const bf16_t* x;       // NORM = false: [K/8][16][8] (xidx layout, row block 0); NORM = true: hidden rows [R][K] row-major
   const bf16_t* scale;   // NORM: RMSNorm scale [K]
@@ -45,13 +49,17 @@ struct SdotArgs {
   GemmEpi e;
   const u32x4* pf; size_t pf_n; int main_blocks;   // prefetch: blocks main_blocks .. gridDim.x - 1 stream pf[0 .. pf_n) (16-byte units)
   SdotSide side;
+  SdotRows rows;         // NORM = 2
 };
 
 // HALF: a block takes eight columns of a tile, so that a product of few tiles still runs on all CUs.  A wave's load is two steps of those columns (whole lines of 128 bytes): lanes
 // 8 .. 15 of each group of 16 hold the second, and a rotation of the groups by eight lanes brings it to the rows of the first; rows 8 .. 15 of the products are never stored.
 // 8 rows, 2048 columns, K 2048 and 7168 in turn: 7.9 us a launch by whole tiles (128 blocks), now 6.9; 4 rows, 1024 columns, K 1024 and 3584 with the tanh norm: 6.4 -> 6.0.
-template <int EPI, bool NORM, bool HALF = false>
-__global__ __launch_bounds__(1024) void k_sdot(SdotArgs a) {
+// NORM 1: RMSNorm of bf16 rows [R][K]; 2: SdotRows, up to SDOT_ROWS rows, K <= 2048, every block for itself while its weights come.  Gated units of 8 rows, K 2048, 14336 columns: 13.2 us behind
+// a launch of 4.1 that took the norm, now 14.9 alone (sixteen waves a block, so that a wave has two units of a row beside its 16 KB of weights); 6416 columns 8.4 behind 4.1, now 10.4 (eight
+// waves, four units).
+template <int EPI, int NORM, bool HALF = false>
+__global__ __launch_bounds__(NORM == 2 && EPI == GEPI_F32 ? 512 : 1024) void k_sdot(SdotArgs a) {
   extern __shared__ __attribute__((aligned(16))) u32x4 sx[];
   const int tid = threadIdx.x, nthr = blockDim.x, lane = tid & 63;
   if ((int)blockIdx.x >= a.main_blocks) {        // a prefetch block (whole block: no barrier is skipped)
@@ -77,12 +85,28 @@ __global__ __launch_bounds__(1024) void k_sdot(SdotArgs a) {
   const int np = nch << rpl;
   auto xsrc = [&](int p) -> const u32x4* {
     p = min(p, np - 1);
-    if constexpr (NORM) return reinterpret_cast<const u32x4*>(a.x + (size_t)min(p & (Rp - 1), R - 1) * K + (size_t)(p >> rpl) * 8);
+    if constexpr (NORM == 1) return reinterpret_cast<const u32x4*>(a.x + (size_t)min(p & (Rp - 1), R - 1) * K + (size_t)(p >> rpl) * 8);
     else return reinterpret_cast<const u32x4*>(a.x) + (size_t)(p >> rpl) * 16 + (p & (Rp - 1));
   };
-  u32x4 x0[8];
+  u32x4 x0[NORM == 2 ? 1 : 8];
+  if constexpr (NORM != 2) {
 #pragma unroll
-  for (int u = 0; u < 8; ++u) x0[u] = *xsrc(tid + u * nthr);
+    for (int u = 0; u < 8; ++u) x0[u] = *xsrc(tid + u * nthr);
+  }
+  // NORM 2: units of (row, 512 features), a lane eight of them; a wave's units are of the same features
+  constexpr int NU = NORM != 2 ? 1 : EPI == GEPI_F32 ? 4 : 2;
+  const int uch = (wave % chains) * 64 + lane, nw = nthr >> 6;
+  float rx[NU][8], rt[NU][8], pw[NORM == 2 ? 8 : 1];
+  if constexpr (NORM == 2) {
+    const int at = min(uch, nch - 1) * 8;
+#pragma unroll
+    for (int i = 0; i < NU; ++i) {
+      const int row = min((wave + i * nw) / chains, R - 1);
+      rows_load8(a.rows.t + (size_t)row * a.rows.ldt + at, rt[i]);
+      rows_load8(a.rows.x + (size_t)row * K + at, rx[i]);
+    }
+    rows_load8(a.rows.w + at, pw);
+  }
 
   // this wave's chain of weight fragments: all sixteen in flight
   const int s0 = c * 16, cs = min(16, nsteps - s0);
@@ -95,13 +119,44 @@ __global__ __launch_bounds__(1024) void k_sdot(SdotArgs a) {
 #pragma unroll
   for (int s = 0; s < NWV; ++s) wv[s] = __builtin_nontemporal_load(wbase + (size_t)min(HALF ? 2 * s + (lane >> 3 & 1) : s, cs - 1) * 64);
 
+  if constexpr (NORM == 2) {
+    // the sums as k_sub_norm takes them: a lane's eight, the lanes of 512 features, the features' four blocks in pairs
 #pragma unroll
-  for (int u = 0; u < 8; ++u) {
-    const int p = tid + u * nthr;
-    if (p < np) sx[p] = x0[u];
+    for (int i = 0; i < NU; ++i) {
+      const int row = (wave + i * nw) / chains;
+      float ss = 0.0f;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) ss = fmaf(rt[i][j], rt[i][j], ss);
+      ss = xor_sum(uch < nch ? ss : 0.0f);
+      if (lane == 0 && row < R) blk[row * 4 + wave % chains] = ss;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < NU; ++i) {
+      const int row = (wave + i * nw) / chains;
+      float q[4];
+#pragma unroll
+      for (int b = 0; b < 4; ++b) q[b] = b < chains ? blk[min(row, R - 1) * 4 + min(b, chains - 1)] : 0.0f;
+      const float s = 1.0f / sqrtf(((q[0] + q[1]) + (q[2] + q[3])) / (float)K + a.rows.eps);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) rx[i][j] = rx[i][j] + rt[i][j] * s * (1.0f + pw[j]);
+      if (row < R && uch < nch) {
+        sx[(uch << rpl) + row] = u32x4{pack2(f2bf(rx[i][0]), f2bf(rx[i][1])), pack2(f2bf(rx[i][2]), f2bf(rx[i][3])), pack2(f2bf(rx[i][4]), f2bf(rx[i][5])), pack2(f2bf(rx[i][6]), f2bf(rx[i][7]))};
+        if (blockIdx.x == 0) {
+          float4* o = reinterpret_cast<float4*>(a.rows.x_out + (size_t)row * K + uch * 8);
+          o[0] = make_float4(rx[i][0], rx[i][1], rx[i][2], rx[i][3]); o[1] = make_float4(rx[i][4], rx[i][5], rx[i][6], rx[i][7]);
+        }
+      }
+    }
+  } else {
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int p = tid + u * nthr;
+      if (p < np) sx[p] = x0[u];
+    }
   }
 #pragma unroll 1
-  for (int p0 = tid + 8 * nthr; p0 < np; p0 += 4 * nthr) {   // more than 8 pieces per thread (many rows): further rounds of 4
+  for (int p0 = tid + 8 * nthr; p0 < np && NORM != 2; p0 += 4 * nthr) {   // more than 8 pieces per thread (many rows): further rounds of 4
     u32x4 tmp[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) tmp[u] = *xsrc(p0 + u * nthr);
@@ -111,7 +166,7 @@ __global__ __launch_bounds__(1024) void k_sdot(SdotArgs a) {
       if (p < np) sx[p] = tmp[u];
     }
   }
-  if constexpr (NORM) {
+  if constexpr (NORM == 1) {
     // RMSNorm (normalizations.py:57-70) in the canonical order of k_rownorm: chunk of 8 = one fma chain, block of 64 chunks by
     // xor-butterfly, blocks added in order; y = bf16(x r), out = bf16(y scale).  Every block norms the rows for itself.
     for (int i = tid; i < nch; i += nthr) ssc[i] = *reinterpret_cast<const u32x4*>(a.scale + i * 8);

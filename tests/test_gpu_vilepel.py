@@ -77,6 +77,27 @@ def test_few_rows_of_latent_attention(tmp_path, layer):
   one_layer(tmp_path, VH.with_mlp(VH.latent(**layer), None), "bfloat16", n=96, portions=((16,), (50, 17, 16, 13), (80, 1)))
 
 
+@pytest.mark.parametrize("width", [128, 1152, 2048])
+def test_few_rows_take_a_norm_into_the_next_product(tmp_path, width):
+  """Up to eight rows of whole 128s of features: a sublayer's norm and the residual are part of the next product's launch, unless the residual stream is tapped.  The same bits, for one row, an
+  odd number of them, eight, and nine (which take the launches of their own)."""
+  cfg = VH.model([VH.with_mlp(VH.delta(), VH.dense(ff=200)), VH.with_mlp(VH.latent(), None), VH.with_mlp(VH.latent(), VH.dense(ff=136)), VH.with_mlp(VH.delta(), VH.moe()),
+                  VH.with_mlp(VH.delta(), VH.dense())], width=width)
+  w = VH.random_weights(cfg, 7)
+  eng, _ = VH.engine(VH.write_model(tmp_path, cfg, w), dtype="bfloat16")
+  t = VH.tokens(cfg, 40, 8)
+  tap = torch.zeros(40 * len(cfg["layers"]) * width, device="cuda")
+  out = []
+  for tapped in (True, False):
+    s = VH.scheduler(eng)
+    VH.H.lib.check(eng.lib.ixt_set_residual_tap(eng._ctx, ctypes.c_void_p(tap.data_ptr()) if tapped else None, tap.numel() if tapped else 0))
+    out.append(VH.run_portions(s, "r", t, (1, 5, 8, 9, 1, 1, 7, 8)))
+    s.release("r")
+  eng.close()
+  assert np.array_equal(out[0], out[1])
+  VH.check(out[1], V.forward(cfg, w, t), "bfloat16")
+
+
 DELTAS = {
     "one head": VH.delta(heads=1, kv_heads=1, dim=8, vdim=8, conv=2),
     "shared keys": VH.delta(heads=6, kv_heads=2, dim=20, vdim=12, conv=4),
