@@ -204,7 +204,7 @@ enum { TL_XW, TL_DX, TL_DW };
 template <bool TA, bool TB, int BM, int BN = BM, bool FOLD = false>
 static int gemm_launch(hipStream_t st, TGemm& g) {
   // waves and their tiles: 256 x 256: 2 x 4 of 128 x 64; 256 x 128: 4 x 2 and 128 x 128: 2 x 2 of 64 x 64; 128 x 64: 4 of 32 x 64; 64 x 64: 2 x 2 of 32 x 32
-  constexpr int WM = BN == BM ? 2 : 4, WN = BN == 256 ? 4 : BN == 64 && BM == 128 ? 1 : 2, MI = BM / 16 / WM, NI = BN / 16 / WN, NS = TA && TB ? 4 : 5, lds = NS * (BM + BN) * 64;
+  constexpr int WM = BN == BM ? 2 : 4, WN = BN == 256 ? 4 : BN == 64 && BM == 128 ? 1 : 2, MI = BM / 16 / WM, NI = BN / 16 / WN, NS = 4, lds = (TA && TB ? NS : NS + 1) * (BM + BN) * 64;
   const auto kernel = k_tgemm<TA, TB, MI, NI, WM, WN, NS, FOLD>;
   static bool attr_done = false;
   if (!attr_done) {

@@ -1,7 +1,7 @@
 // ixt_train_gemm.h -- the matrix products of the training step: C[m][n] (+)= sum_k A(m, k) B(k, n), bf16 operands of which either index may be the
 // contiguous one, f32 accumulation.
 //
-// Block = (16 MI WM) x (16 NI WN), waves WM x WN, 32 k at a time through a ring of NS LDS slots filled by LDS-DMA; a wave's tile is 16 MI x 16 NI.
+// Block = (16 MI WM) x (16 NI WN), waves WM x WN, 32 k at a time through a ring of NS LDS slots (one more for pairs, below) filled by LDS-DMA; a wave's tile is 16 MI x 16 NI.
 // What bounds it: the matrix units at the clock that the card's power leaves them.  Random operands, 256 x 256 blocks: 1068 cycles of products per 32 k, 1136 with the
 // LDS reads and the fetches beside them and nothing else (1.55 PFLOP/s at 1.64 GHz), 1340 to 1450 here at 1.5 to 1.8 GHz.  Per 32 k a wave reads MI + NI KiB for MI NI products of
 // 16 cycles, which is why the largest block is taken wherever its tiles fill the chip.  With few tiles a wave is alone on its SIMD and bound by its own instructions: smaller tiles,
@@ -59,11 +59,12 @@ static __device__ const uint32_t tg_zero[4] = {0u, 0u, 0u, 0u};
 template <bool TA, bool TB, int MI, int NI, int WM, int WN, int NS, bool FOLD = false>
 __global__ __launch_bounds__(WM * WN * 64, 2) void k_tgemm(TGemm g) {
   constexpr bool PAIR = !TA || !TB;
+  constexpr int SLOTS = PAIR ? NS + 1 : NS;                               // pairs: two chunks being read, three ahead
   constexpr int BM = 16 * MI * WM, BN = 16 * NI * WN, NW = WM * WN;
   constexpr int NA = BM / 16, NB = BN / 16, NJ = (NA + NB) / NW;          // KiB of a chunk; a wave fetches NJ of them
   constexpr int SLOT = (BM + BN) * 32;                                    // elements
-  static_assert(NA % NW == 0 && NB % NW == 0 && NS == (PAIR ? 5 : 4), "a fetch is of one operand; pairs: two chunks being read, three ahead");
-  extern __shared__ __attribute__((aligned(16))) bf16_t lds[];            // [NS][A image | B image]
+  static_assert(NA % NW == 0 && NB % NW == 0 && NS == 4, "a fetch is of one operand; the counts of the waits");
+  extern __shared__ __attribute__((aligned(16))) bf16_t lds[];            // [SLOTS][A image | B image]
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, r16 = lane & 15, q = lane >> 4;
   const int wm = wave / WN, wn = wave % WN;
   // XCD x takes a run of tiles (part by part); eight row tiles share their columns' operand
@@ -195,7 +196,7 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void k_tgemm(TGemm g) {
   int slot = 0;                                                           // of chunk c
   auto step = [&](auto cur_, auto edge) {
     constexpr int cur = cur_.value;
-    const int old = slot, older = slot == 0 ? NS - 1 : slot - 1, nxt = slot + 1 == NS ? 0 : slot + 1;
+    const int old = slot, older = slot == 0 ? SLOTS - 1 : slot - 1, nxt = slot + 1 == SLOTS ? 0 : slot + 1;
     slot = nxt;
     constexpr bool fetch = !PAIR || cur == 0;
     Chunk lo{}, hi{};
