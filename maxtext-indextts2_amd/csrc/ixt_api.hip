@@ -1667,7 +1667,7 @@ static int moe_experts_routed(ixt_ctx* c, const LayerW& w, const bf16_t* x, cons
       const int ti = timing_begin(c, st, (double)K * N * 2.0 * c->NEL + (double)rows_g * K * 2.0 + out_bytes);
       dim3 grid((((nwaves + 3) / 4 + 7) / 8) * 8 * zblocks, 1, 1);
       hipLaunchKernelGGL(kern, grid, dim3(256), (size_t)64 * 1024, st, reinterpret_cast<const u32x4*>(xin), reinterpret_cast<const u32x4*>(wbase), K, N, rows_g, out, nwaves, zblocks,
-                         c->moe_rbexp, wstride, 0, 0.0f, (const float*)nullptr);
+                         c->moe_rbexp, wstride, 0, 0.0f, (const float*)nullptr, (const int32_t*)nullptr, 0);
       timing_end(c, st, ti);
     };
     if ((size_t)rows_g * E > c->part_floats) return set_err(IXT_ERR_INVALID, "moe: output workspace too small");
@@ -1680,13 +1680,13 @@ static int moe_experts_routed(ixt_ctx* c, const LayerW& w, const bf16_t* x, cons
   }
   if (align == 16) {
     const int zblocks = rows_g / 16;
-    auto dotg = [&](const bf16_t* xin, const bf16_t* wbase, size_t wstride, int K, int N) -> int {
+    auto dotg = [&](const bf16_t* xin, const bf16_t* wbase, size_t wstride, int K, int N, bool live) -> int {      // live: rows with a copy only
       const int chains = (K + IXT_CHAIN - 1) / IXT_CHAIN, nwaves = N / 16;
       if ((size_t)chains * rows_g * N > c->part_floats) return set_err(IXT_ERR_INVALID, "moe: slice workspace too small");
       const int ti = timing_begin(c, st, (double)K * N * 2.0 * c->NEL + (double)rows_g * K * 2.0 + (double)chains * rows_g * N * 4.0);
       dim3 grid((((nwaves + 3) / 4 + 7) / 8) * 8 * zblocks, chains, 1);
       hipLaunchKernelGGL((k_dotb<1, true, true>), grid, dim3(256), (size_t)16 * 1024, st, reinterpret_cast<const u32x4*>(xin), reinterpret_cast<const u32x4*>(wbase), K, N,
-                         rows_g, c->part, nwaves, zblocks, c->moe_rbexp, wstride);
+                         rows_g, c->part, nwaves, zblocks, c->moe_rbexp, wstride, 0, 0.0f, nullptr, live ? c->moe_cnt : nullptr, c->NEL);
       timing_end(c, st, ti);
       LAUNCHCHK();
       return chains;
@@ -1701,12 +1701,12 @@ static int moe_experts_routed(ixt_ctx* c, const LayerW& w, const bf16_t* x, cons
       timing_end(c, st, ti);
       LAUNCHCHK();
     } else {
-      ch = dotg(c->moe_xg, w.ewi[0], wi_stride, E, 2 * F);
+      ch = dotg(c->moe_xg, w.ewi[0], wi_stride, E, 2 * F, false);
       if (ch < 0) return ch;
       hipLaunchKernelGGL(k_swiglu_part, dim3((F + 2047) / 2048, rows_g), dim3(256), 0, st, c->part, ch, (size_t)rows_g * 2 * F, F, c->moe_hact, c->moe_rbexp);
       LAUNCHCHK();
     }
-    ch = dotg(c->moe_hact, w.ewout[0], wo_stride, F, E);
+    ch = dotg(c->moe_hact, w.ewout[0], wo_stride, F, E, true);
     if (ch < 0) return ch;
     res->slices = ch; res->slice_stride = (size_t)rows_g * E; res->ntiles = E / 16;
     return IXT_OK;

@@ -83,7 +83,8 @@ __host__ __device__ __forceinline__ int qk_col(int i, int half) {
 //   SPLIT (one chain per block, 256 threads): the slab loads are issued BEFORE the weight loads -- loads return in order, so
 //   the L2-resident slab lands and is written to LDS while the weight fragments are still on their way from HBM.
 //   Routed experts (rb_exp != nullptr; NRB = 1): row block rb belongs to expert rb_exp[rb], whose kernels start wstride 16-byte units after
-//   wt; a row block of no expert (-1) leaves at once (k_moe_plan, ixt_moe_kernels.h).
+//   wt; a row block of no expert (-1) leaves at once (k_moe_plan, ixt_moe_kernels.h).  cnt_off: the plan's counts and offsets; the slices' rows behind an expert's last copy are not
+//   written (8 tokens, two of 8 experts each: 59 MB of slices beside 940 of weights, 162 us; now 7, and 138).
 //   EPI = 1 (whole-K blocks only): the columns are interleaved (wi_0, wi_1) tiles (k_tile_w mode 2) and `out` is the bf16 activation buffer of the
 //   next dot (glu: that gated unit of the f32 totals instead, ixt_glu): the odd wave of a pair hands its totals to the even one through LDS, which writes bf16(bf16(a * bf16(sigmoid a)) * b) in the x layout
 //   (linears.py:331-361) -- no f32 slice leaves the chip (routed experts at decode: 132 MB of slices per layer and the kernel that re-read them).
@@ -91,7 +92,8 @@ __host__ __device__ __forceinline__ int qk_col(int i, int half) {
 template <int NRB, bool SPLIT, bool NT, int EPI = 0>
 __global__ __launch_bounds__(256, 2) void k_dotb(const u32x4* __restrict__ xt, const u32x4* __restrict__ wt, int K, int N, int R,
                                                  float* __restrict__ out, int nwaves, int zblocks, const int32_t* __restrict__ rb_exp = nullptr,
-                                                 size_t wstride = 0, int glu = 0, float glu_limit = 0.0f, const float* __restrict__ act_par = nullptr) {
+                                                 size_t wstride = 0, int glu = 0, float glu_limit = 0.0f, const float* __restrict__ act_par = nullptr,
+                                                 const int32_t* __restrict__ cnt_off = nullptr, int n_exp = 0) {
   extern __shared__ __attribute__((aligned(16))) u32x4 xs[];   // [NRB][16 steps][64 lanes]
   const int tid = threadIdx.x, nthr = blockDim.x, wpb = nthr >> 6;
   const int wave = tid >> 6, lane = tid & 63;
@@ -107,10 +109,14 @@ __global__ __launch_bounds__(256, 2) void k_dotb(const u32x4* __restrict__ xt, c
   const int r_in = lane & 15, cq = lane >> 4;
   const bool tile_ok = tile < nwaves;
   const u32x4* wbase = wt + (size_t)(tile_ok ? tile : 0) * nsteps * 64 + lane;
+  int rows_out = R;
   if (rb_exp != nullptr) {
     const int ex = rb_exp[rb0];
     if (ex < 0) return;                                  // the whole block: no barrier is skipped
     wbase += (size_t)ex * wstride;
+    if constexpr (SPLIT) {
+      if (cnt_off != nullptr) rows_out = min(R, cnt_off[ex] + cnt_off[n_exp + ex]);
+    }
   }
   f32x4 tot[NRB];
 #pragma unroll
@@ -169,7 +175,7 @@ __global__ __launch_bounds__(256, 2) void k_dotb(const u32x4* __restrict__ xt, c
 #pragma unroll
       for (int b = 0; b < NRB; ++b) {
         const int row = (rb0 + b) * 16 + r_in;
-        if (tile_ok && row < R)
+        if (tile_ok && row < rows_out)
           *reinterpret_cast<float4*>(out + ((size_t)c * R + row) * N + tile * 16 + cq * 4) = make_float4(acc[b][0], acc[b][1], acc[b][2], acc[b][3]);
       }
     } else {
