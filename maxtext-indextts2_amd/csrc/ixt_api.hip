@@ -1640,7 +1640,7 @@ static int moe_experts_routed(ixt_ctx* c, const LayerW& w, const bf16_t* x, cons
         const int ti_ = timing_begin(c, st, (double)K * N * c->NEL + (double)rows_g * K + (double)chains * rows_g * N * 4.0);
         dim3 grid((((nwaves + 3) / 4 + 7) / 8) * 8 * zblocks, chains, 1);
         hipLaunchKernelGGL((k_dotb8<1>), grid, dim3(256), (size_t)8192, st, reinterpret_cast<const u32x4*>(c->x8), reinterpret_cast<const u32x4*>(t.w8), c->xs8, t.s, K, N,
-                           rows_g, c->part, nwaves, zblocks, c->moe_rbexp, w8stride, sstride);
+                           rows_g, c->part, nwaves, zblocks, c->moe_rbexp, w8stride, sstride, c->moe_cnt, c->NEL);
         timing_end(c, st, ti_);
         LAUNCHCHK();
         return chains;
@@ -1653,7 +1653,7 @@ static int moe_experts_routed(ixt_ctx* c, const LayerW& w, const bf16_t* x, cons
     };
     int ch = dot8g(c->moe_xg, ti, E, 2 * F, (size_t)2 * F);
     if (ch < 0) return ch;
-    hipLaunchKernelGGL(k_swiglu_part, dim3((F + 2047) / 2048, rows_g), dim3(256), 0, st, c->part, ch, (size_t)rows_g * 2 * F, F, c->moe_hact, c->moe_rbexp);
+    hipLaunchKernelGGL(k_swiglu_part, dim3((F + 2047) / 2048, rows_g), dim3(256), 0, st, c->part, ch, (size_t)rows_g * 2 * F, F, c->moe_hact, c->moe_rbexp, align == 16 ? c->moe_cnt : nullptr, c->NEL);
     LAUNCHCHK();
     ch = dot8g(c->moe_hact, to, F, E, (size_t)E);
     if (ch < 0) return ch;

@@ -93,7 +93,7 @@ static __global__ __launch_bounds__(64) void k_f8_quant_x(const bf16_t* __restri
 template <int NRB>
 __global__ __launch_bounds__(256, 2) void k_dotb8(const u32x4* __restrict__ x8, const u32x4* __restrict__ w8, const float* __restrict__ xscale,
                                                   const float* __restrict__ wscale, int K, int N, int R, float* __restrict__ out, int nwaves, int zblocks,
-                                                  const int32_t* __restrict__ rb_exp = nullptr, size_t wstride = 0, size_t sstride = 0) {
+                                                  const int32_t* __restrict__ rb_exp = nullptr, size_t wstride = 0, size_t sstride = 0, const int32_t* __restrict__ cnt_off = nullptr, int n_exp = 0) {
   extern __shared__ __attribute__((aligned(16))) u32x4 xs[];   // [NRB][8 fragments][64 lanes]
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -105,11 +105,13 @@ __global__ __launch_bounds__(256, 2) void k_dotb8(const u32x4* __restrict__ x8, 
   const int f0 = c * 8, cf = min(8, nfr - f0);                 // (K % 64 == 0: a last chain of 256 k has 4 fragments)
   const int r_in = lane & 15, cq = lane >> 4;
   const bool tile_ok = tile < nwaves;
+  int rows_out = R;
   if (rb_exp != nullptr) {
     const int ex = rb_exp[rb0];
     if (ex < 0) return;                                        // the whole block: no barrier is skipped
     w8 += (size_t)ex * wstride;
     wscale += (size_t)ex * sstride;
+    if (cnt_off != nullptr) rows_out = min(R, cnt_off[ex] + cnt_off[n_exp + ex]);      // rows that hold a copy (k_dotb)
   }
   // activation fragments of this chain first (L2), then the weights (HBM): loads return in order
   u32x4 xq[NRB * 2];
@@ -149,7 +151,7 @@ __global__ __launch_bounds__(256, 2) void k_dotb8(const u32x4* __restrict__ x8, 
 #pragma unroll
   for (int b = 0; b < NRB; ++b) {
     const int row = (rb0 + b) * 16 + r_in;
-    if (row < R) {
+    if (row < rows_out) {
       const float a = xscale[(size_t)row * nchains + c];
       *reinterpret_cast<float4*>(out + ((size_t)c * R + row) * N + tile * 16 + cq * 4) =
           make_float4(acc[b][0] * (a * sn.x), acc[b][1] * (a * sn.y), acc[b][2] * (a * sn.z), acc[b][3] * (a * sn.w));

@@ -724,10 +724,13 @@ __global__ __launch_bounds__(256) void k_rownorm(RowNormArgs a) {
 // 16-byte store: 8 consecutive features of a row are one lane's fragment bytes in the dot kernel's x layout).
 // =====================================================================================================
 static __global__ __launch_bounds__(256) void k_swiglu_part(const float* part, int slices, size_t slice_stride, int F,
-                                                      bf16_t* out /*[R][F] in xidx layout*/, const int32_t* rb_exp = nullptr) {
+                                                      bf16_t* out /*[R][F] in xidx layout*/, const int32_t* rb_exp = nullptr, const int32_t* cnt_off = nullptr, int n_exp = 0) {
   const int f0 = (blockIdx.x * 256 + threadIdx.x) * 8, r = blockIdx.y;
   if (f0 >= F) return;
-  if (rb_exp != nullptr && rb_exp[r >> 4] < 0) return;      // routed experts: a row block nobody's copies live in
+  if (rb_exp != nullptr) {                                  // routed experts: a row block nobody's copies live in, a row behind an expert's last copy
+    const int ex = rb_exp[r >> 4];
+    if (ex < 0 || (cnt_off != nullptr && r >= cnt_off[ex] + cnt_off[n_exp + ex])) return;
+  }
   const float* p = part + (size_t)r * 2 * F;
   float a[8], b[8];
 #pragma unroll
