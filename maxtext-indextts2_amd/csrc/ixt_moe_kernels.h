@@ -177,7 +177,23 @@ static __global__ __launch_bounds__(1024) void k_moe_plan(const int32_t* idx /*[
   __shared__ int s_base, s_off;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   for (int i = tid; i < nrb_cap; i += 1024) rb_exp[i] = -1;
-  for (int i = tid; i < npairs; i += 1024) pos[i] = -1;     // a copy of no resident expert (expert-parallel padding) stays without a row
+  if (npairs <= 64) {                                       // a wave has all pairs: no barriers an expert (16 pairs of 8 experts: 7.2 us -> 4.6)
+    __syncthreads();
+    if (wave > 0) return;
+    const int mine = lane < npairs ? idx[lane] - e0 : -1;
+    int place = -1, off = 0;                                // -1: a copy of no resident expert (expert-parallel padding) stays without a row
+    for (int e = 0; e < n_exp; ++e) {
+      const unsigned long long bal = __ballot(mine == e);
+      const int n = __popcll(bal);
+      if (mine == e) place = off + __popcll(bal & ((1ull << lane) - 1ull));
+      if (lane < (n + 15) >> 4) rb_exp[(off >> 4) + lane] = e;
+      if (lane == 0) { cnt_off[e] = n; cnt_off[n_exp + e] = off; }
+      off += (n + align - 1) / align * align;
+    }
+    if (lane < npairs) pos[lane] = place;
+    return;
+  }
+  for (int i = tid; i < npairs; i += 1024) pos[i] = -1;     // (as above)
   if (tid == 0) s_off = 0;
   __syncthreads();
   for (int e = 0; e < n_exp; ++e) {

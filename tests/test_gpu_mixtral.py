@@ -57,6 +57,14 @@ def test_mixtral_expert_counts(ne, k):
   run_pair(cfg, w, prompts, steps=10)
 
 
+@pytest.mark.parametrize("ne,k,lengths", [(8, 2, (32, 33)), (2, 1, (40, 17)), (4, 4, (16, 17))])
+def test_mixtral_copies_at_the_ends_of_blocks(ne, k, lengths):
+  """64 copies, whose plan a wave makes, and the few more that take the block's; experts with one copy behind a block of 16 rows: the slices' last rows that are written.  Bit for bit."""
+  cfg = _cfg(per_device_batch_size=2.0, num_experts=ne, num_experts_per_tok=k)
+  w = H.synth.synth_weights(cfg, 8)
+  run_pair(cfg, w, [(_prompt(cfg.vocab_size, 48, 70 + s), n) for s, n in enumerate(lengths)], steps=3)
+
+
 def test_mixtral_many_rows():
   """130 decode slots and a 150-row prefill: the per-expert dots take their >= 128-row forms."""
   cfg = H.make_config("mixtral-tiny", max_prefill_predict_length=160, max_target_length=192, per_device_batch_size=130.0, pagedattn_num_pages=130 * 24 + 8,
