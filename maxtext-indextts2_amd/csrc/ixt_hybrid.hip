@@ -744,11 +744,14 @@ int hybrid_copy_group(ixt_ctx* c, int src, int dst, int npages, hipStream_t st) 
 }
 
 // ---------------------------------------------------------------------------------------------------- the forward pass
+// gated units of rows that are no routed experts' copies: by the ring product (ring_min_rows is an option, from 1 on), which takes its rows as an operand
+static bool units_by_ring(const ixt_ctx* c, int rows) { return rows >= c->ring_min_rows; }
 // A sublayer's output, its RMS norm and the residual inside the next product, every block for itself, under its weights' way (few rows): a launch less
 template <typename T> static bool norm_rides(ixt_ctx* c, const HMat& w, const Around& ar, bool routed, int R, const float* bias, const HMat* next, int epi) {
   const HybridModel* m = c->hy;
   return sizeof(T) == 2 && next != nullptr && m->norm_kind == IXT_NORM_RMS && m->streams == 0 && m->E == m->Ep && R <= std::min(SDOT_ROWS, c->small_rows) && m->tap == nullptr && !routed && ar.mu == nullptr &&
-         !ar.to_cat && !ar.to_head && ar.post.w != nullptr && ar.pre.w == nullptr && bias == nullptr && next->Np <= 65536 && sdot_plan(c, GEPI_F32, false, w.Kp, w.Np, R).ok && sdot_plan(c, epi, false, next->Kp, next->Np, R, true).ok;
+         !ar.to_cat && !ar.to_head && ar.post.w != nullptr && ar.pre.w == nullptr && bias == nullptr && next->Np <= 65536 && !(epi == GEPI_SWIGLU && units_by_ring(c, R)) &&
+         sdot_plan(c, GEPI_F32, false, w.Kp, w.Np, R).ok && sdot_plan(c, epi, false, next->Kp, next->Np, R, true).ok;
 }
 // a pending norm's rows for the product of operand x, whose launch leaves the residual stream in the other buffer
 static bool take_ride(HybridModel* m, const void* x, SdotRows* rows) {
@@ -865,7 +868,8 @@ template <> int hact_unit<float>(ixt_ctx* c, const float* x, const HMat& w, size
 // gate | up product with the gated unit (IXT_GLU_*) behind it -> act(T) of the down product
 template <typename T> static int hglu(ixt_ctx* c, const T* x, const HMat& w, size_t stride, int rows, int group_rows, const int32_t* rb, int kind, float limit, T* out, hipStream_t st);
 template <> int hglu<bf16_t>(ixt_ctx* c, const bf16_t* x, const HMat& w, size_t stride, int rows, int group_rows, const int32_t* rb, int kind, float limit, bf16_t* out, hipStream_t st) {
-  if (rb ? group_rows % 128 == 0 : rows >= c->ring_min_rows) {
+  if (rb ? group_rows % 128 == 0 : units_by_ring(c, rows)) {
+    if (c->hy->ride.on && x == c->hy->xb) return set_err(IXT_ERR_INVALID, "a product that does not take its rows' norm in");
     GemmEpi e{};
     e.act = out; e.glu = kind; e.glu_limit = limit; e.rb_exp = rb; e.wstride = stride / 8;
     return launch_ring(c, GEPI_SWIGLU, x, (const bf16_t*)w.w, w.Kp, w.Np, rows, e, false, st);

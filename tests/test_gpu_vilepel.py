@@ -98,6 +98,28 @@ def test_few_rows_take_a_norm_into_the_next_product(tmp_path, width):
   VH.check(out[1], V.forward(cfg, w, t), "bfloat16")
 
 
+@pytest.mark.parametrize("last", ["routed", "dense"])
+def test_units_by_the_ring_take_no_norm_in(tmp_path, last):
+  """ring_min_rows of 1: the gated units of a few rows go by the ring product, which reads its rows from memory, so the norm in front of them is a launch of its own.  The same bits as with a tapped
+  residual stream, where every norm is one, and the restatement at bfloat16's tolerance."""
+  cfg = VH.model([VH.with_mlp(VH.delta(), VH.dense(ff=200)), VH.with_mlp(VH.latent(), None), VH.with_mlp(VH.latent(), VH.dense(ff=136)),
+                  VH.with_mlp(VH.delta(), VH.moe() if last == "routed" else VH.dense())], width=256)
+  w = VH.random_weights(cfg, 9)
+  eng, _ = VH.engine(VH.write_model(tmp_path, cfg, w), dtype="bfloat16")
+  H.lib.check(eng.lib.ixt_set_option(eng._ctx, b"ring_min_rows", 1))
+  t = VH.tokens(cfg, 40, 8)
+  tap = torch.zeros(40 * len(cfg["layers"]) * 256, device="cuda")
+  out = []
+  for tapped in (True, False):
+    s = VH.scheduler(eng)
+    VH.H.lib.check(eng.lib.ixt_set_residual_tap(eng._ctx, ctypes.c_void_p(tap.data_ptr()) if tapped else None, tap.numel() if tapped else 0))
+    out.append(VH.run_portions(s, "r", t, (1, 5, 8, 9, 1, 1, 7, 8)))
+    s.release("r")
+  eng.close()
+  assert np.array_equal(out[0], out[1])
+  VH.check(out[1], V.forward(cfg, w, t), "bfloat16")
+
+
 DELTAS = {
     "one head": VH.delta(heads=1, kv_heads=1, dim=8, vdim=8, conv=2),
     "shared keys": VH.delta(heads=6, kv_heads=2, dim=20, vdim=12, conv=4),
