@@ -214,6 +214,13 @@ template <typename F> __device__ __forceinline__ float xor_butterfly(float v, F 
 }
 __device__ __forceinline__ float xor_sum(float v) { return xor_butterfly(v, [](float x, float y) { return x + y; }); }
 
+// between LDS writes of a wave's lanes and reads of other lanes of it: the hardware keeps a wave's LDS accesses in order, this keeps the compiler to it (no instruction)
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // The row of block b where a block takes a row of R and writes it to an operand (xidx: 16 bytes of a line of eight rows at a time): the eight rows of a line go to blocks that the
 // dispatcher deals to one XCD, so that its L2 holds the line whole when it is written back (with
 // sums over the lanes that need no LDS, us before / now: k_rownorm of 1592 rows of 2048 7.8 / 5.9, of 1024 6.5 / 5.2; k_gnorm of 256 rows of 2304 6.3 / 5.1).

@@ -309,6 +309,7 @@ static __global__ __launch_bounds__(256) void k_t_softmax_fwd_wave(const float* 
     q = __builtin_fmaf(__builtin_fmaf(-q, sum, e), rl, q);
     return __builtin_fmaf(__builtin_fmaf(-q, sum, e), rl, q);
   });
+  wave_lds_sync();
   const int n = min(S, nv * 256);
   bf16_t* out = P + (bh * S + row) * S;
   for (int j = lane * 8; j < n; j += 512) *reinterpret_cast<u32x4*>(out + j) = *reinterpret_cast<const u32x4*>(tile + j);
@@ -390,6 +391,7 @@ static __global__ __launch_bounds__(256) void k_t_softmax_bwd_wave(const float* 
 #pragma unroll
   for (int i = 0; i < MAXV / 2; ++i)
     if (i * 512 + lane * 8 < n) *reinterpret_cast<u32x4*>(tile + i * 512 + lane * 8) = p[i];
+  wave_lds_sync();
   float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
   for (int i = 0; i < MAXV; ++i)
@@ -412,6 +414,7 @@ static __global__ __launch_bounds__(256) void k_t_softmax_bwd_wave(const float* 
         tile[j] = f2bf((in ? bf2f(tile[j]) : 0.0f) * ((in ? g[i][w] : 0.0f) - dot));
       }
     }
+  wave_lds_sync();
   for (int j = lane * 8; j < n; j += 512) *reinterpret_cast<u32x4*>(dS + base + j) = *reinterpret_cast<const u32x4*>(tile + j);
 }
 template <int MAXV>

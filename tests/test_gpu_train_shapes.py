@@ -63,3 +63,47 @@ def test_train_step_at_tile_edges(shape):
   assert abs(m["learning/loss"] - o["learning/loss"]) <= 2e-3 * abs(o["learning/loss"]), (m["learning/loss"], o["learning/loss"])
   del trainer
   torch.cuda.synchronize()
+
+
+def step_and_oracle(cfg, params, batch):
+  """One step of the trainer and of the oracle: their metrics, and the gradients of both."""
+  import torch
+  tr = importlib.import_module("maxtext-indextts2_amd.train")
+  trainer = tr.Trainer(cfg)
+  trainer.load_params(params)
+  m = trainer.train_step(batch)
+  o = TO.TrainOracle(cfg, params).train_step(batch)
+  grads = {k: v.clone().cpu() / (o["learning/total_weights"] + 1e-8) for k, v in trainer.param_views(trainer.grads).items()}
+  del trainer
+  torch.cuda.synchronize()
+  return m, grads, o
+
+
+def one_step(cfg, params, batch, names=None):
+  """The loss and the gradients (`names`: of these tensors) at the tolerances above."""
+  m, grads, o = step_and_oracle(cfg, params, batch)
+  assert abs(m["learning/loss"] - o["learning/loss"]) <= 1e-4 * abs(o["learning/loss"]), (m["learning/loss"], o["learning/loss"])
+  for k in names or grads:
+    err = float((grads[k] - o["grads"][k]).norm()) / (float(o["grads"][k].norm()) + 1e-12)
+    assert err < 2e-2, (k, err)
+
+
+@pytest.mark.parametrize("drop", [58.0, 80.0])
+@pytest.mark.parametrize("length", [264, 520])
+def test_softmax_of_peaked_rows(length, drop):
+  """Scores that lie `drop` below a row's others: weights down to 2^-94, whose quotients go by the reciprocal, and below 2^-96, for which the row is divided.  One token in seven has a key that
+  every query scores so; all others have ordinary scores, and their probabilities, the loss and the gradients are what the oracle's are."""
+  cfg = train_config(base_emb_dim=64, base_num_query_heads=2, base_num_kv_heads=2, head_dim=64, base_mlp_dim=72, vocab_size=264, max_target_length=length, per_device_batch_size=2.0)
+  params = f32_params(cfg, 8)
+  emb = params["params/token_embedder/embedding"].reshape(264, 64)
+  emb[:, :2] = 0.0
+  emb *= (62.0 / (emb**2).sum(1, keepdims=True))**0.5       # every token's norm divides features 0 and 1 by the same
+  emb[:, 0], emb[7, 1] = 1.0, 1.0
+  a = "params/decoder/layers_0/self_attention/"
+  q, k = params[a + "query/kernel"].reshape(64, 2, 64), params[a + "key/kernel"].reshape(64, 2, 64)
+  for p in (q, k):
+    p[:, :, 31], p[:, :, 63] = 0.0, 0.0                      # the slowest pair of the rotation: 0.07 over 520 positions
+  q[0, :, 31], k[1, :, 31] = 8.0, -drop / 8.0
+  b = packed_batch(cfg, 41)
+  b["inputs"][:, 3::7] = 7
+  one_step(cfg, params, b)
