@@ -786,11 +786,7 @@ static int ring_launch_o(const bf16_t* x, const bf16_t* w, int K, int N, int R, 
   constexpr int TC = WC * CT, TR = WR * RB;
   const int ncolg = (N / 16 + TC - 1) / TC, zb = (R + 16 * TR - 1) / (16 * TR);
   constexpr size_t lds = (size_t)NS * (TC + TR) * KS * 1024 + (EPI == GEPI_SWIGLU ? IXT_GATE_BYTES : 0);
-  static bool attr_done = false;
-  if (!attr_done) {   // more than 64 KiB of dynamic LDS needs the attribute once per kernel
-    HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gemm_ring<WR, WC, RB, CT, KS, NS, EPI, SPLIT, false, ONCE>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    attr_done = true;
-  }
+  HIPCHK((lds_room<&k_gemm_ring<WR, WC, RB, CT, KS, NS, EPI, SPLIT, false, ONCE>>(lds)));
   dim3 grid(((ncolg + 7) / 8) * 8 * zb, SPLIT == 2 ? RING_PARTS : SPLIT ? chains : 1, 1);
   hipLaunchKernelGGL((k_gemm_ring<WR, WC, RB, CT, KS, NS, EPI, SPLIT, false, ONCE>), grid, dim3(WR * WC * 64), lds, st, reinterpret_cast<const u32x4*>(x),
                      reinterpret_cast<const u32x4*>(w), K, N, R, ncolg, zb, wring, e);
@@ -886,11 +882,7 @@ static int ring_launch8_t(const uint8_t* x8, const uint8_t* w8, int K, int N, in
   constexpr int TC = WC * CT, TR = WR * RB;
   const int ncolg = (N / 16 + TC - 1) / TC, zb = (R + 16 * TR - 1) / (16 * TR);
   constexpr size_t lds = (size_t)NS * (TC + TR) * KS * 1024;
-  static bool attr_done = false;
-  if (!attr_done) {
-    HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gemm_ring<WR, WC, RB, CT, KS, NS, GEPI_F32, 0, true>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    attr_done = true;
-  }
+  HIPCHK((lds_room<&k_gemm_ring<WR, WC, RB, CT, KS, NS, GEPI_F32, 0, true>>(lds)));
   hipLaunchKernelGGL((k_gemm_ring<WR, WC, RB, CT, KS, NS, GEPI_F32, 0, true>), dim3(((ncolg + 7) / 8) * 8 * zb), dim3(WR * WC * 64), lds, st,
                      reinterpret_cast<const u32x4*>(x8), reinterpret_cast<const u32x4*>(w8), K, N, R, ncolg, zb, 0, e);
   LAUNCHCHK();
@@ -1244,11 +1236,7 @@ static void launch_decode_attn(ixt_ctx* c, int layer, int R, const DotResult& dr
 // len_hint keys do not fit the LDS (the caller takes the per-row kernels).
 template <int HD, int GQ, int NQ>
 static int tile_attn_t(ixt_ctx* c, int layer, int R, int lmax, size_t lds, hipStream_t st, float cap, int window) {
-  static bool attr_done = false;
-  if (!attr_done) {   // up to 160 KiB of dynamic LDS: the attribute once per kernel
-    HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_attn_tile<HD, GQ, NQ>), hipFuncAttributeMaxDynamicSharedMemorySize, 156 * 1024));
-    attr_done = true;
-  }
+  HIPCHK((lds_room<&k_attn_tile<HD, GQ, NQ>>(156 * 1024)));
   TileAttnArgs ta;
   ta.row_slot = c->row_slot; ta.row_pos = c->row_pos; ta.row_active = c->row_active; ta.page_map = c->ps.page_map;
   ta.qbuf = c->qbuf; ta.kpages = c->kpages_l[layer]; ta.vpages = c->vpages_l[layer]; ta.out = c->ao; ta.g = c->geom; ta.R = R; ta.lmax = lmax; ta.cap = cap; ta.window = window;
@@ -1351,16 +1339,13 @@ static int sdot_t(const SdotArgs& a, const SdotPlan& p, hipStream_t st) {
   return IXT_OK;
 }
 
-// up to 156 KiB of dynamic LDS (the down projection keeps R x mlp_dim activations on chip): the attribute once per kernel, at ixt_create
+// up to 156 KiB of dynamic LDS (the down projection keeps R x mlp_dim activations on chip): asked for at ixt_create
 static int sdot_set_attributes() {
-  static bool done = false;
-  if (done) return IXT_OK;
-#define SATTR(E_, ...) HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_sdot<E_, __VA_ARGS__>), hipFuncAttributeMaxDynamicSharedMemorySize, 156 * 1024))
+#define SATTR(E_, ...) HIPCHK((lds_room<&k_sdot<E_, __VA_ARGS__>>(156 * 1024)))
   SATTR(GEPI_QKV, true); SATTR(GEPI_QKV, false); SATTR(GEPI_RESID, true); SATTR(GEPI_RESID, false);
   SATTR(GEPI_SWIGLU, true); SATTR(GEPI_SWIGLU, false); SATTR(GEPI_F32, true); SATTR(GEPI_F32, false); SATTR(GEPI_TANHNORM, false); SATTR(GEPI_ACT, false);
   SATTR(GEPI_F32, false, true); SATTR(GEPI_TANHNORM, false, true); SATTR(GEPI_F32, 2); SATTR(GEPI_SWIGLU, 2);
 #undef SATTR
-  done = true;
   return IXT_OK;
 }
 

@@ -1,12 +1,23 @@
 // ixt_device.h -- scalar numerics shared by every kernel ("IXT-MFMA-v2").
 // Compiled with -ffp-contract=off: a*b+c never fuses; every fused multiply-add is an explicit fmaf.
 #pragma once
+#include "ixt_lds_room.h"
+
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
 #include <type_traits>
 
 typedef uint16_t bf16_t;
+
+// room for `bytes` of dynamic LDS in launches of Kernel on the current device, asked for once a device
+template <auto Kernel> static inline hipError_t lds_room(size_t bytes) {
+  static IxtLdsRoom room;
+  int device = -1;
+  const hipError_t e = hipGetDevice(&device);
+  if (e != hipSuccess) return e;
+  return (hipError_t)room.ask(device, bytes, [&] { return (int)hipFuncSetAttribute(reinterpret_cast<const void*>(Kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes); });
+}
 
 #define IXT_MK 32      // k per matrix instruction (v_mfma_f32_16x16x32_bf16)
 #define IXT_CHAIN 512  // k per accumulator chain of the canonical dot = the unit of a split-K slice

@@ -905,12 +905,8 @@ template <> int hglu<float>(ixt_ctx* c, const float* x, const HMat& w, size_t st
 template <int RT, int RS>
 static int latent_launch(bool tall, int H, int splits, LatentAttnArgs a, hipStream_t st) {
   constexpr size_t tile = LatentTile<RT, RS>::BYTES;
-  static bool attr_done = false;
-  if (!attr_done) {
-    HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_latent_attn<RT, RS>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)(2 * tile)));
-    HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_latent_decode<RT, RS>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)tile));
-    attr_done = true;
-  }
+  if (tall) HIPCHK((lds_room<&k_latent_attn<RT, RS>>(2 * tile)));
+  else HIPCHK((lds_room<&k_latent_decode<RT, RS>>(tile)));
   if (tall) {
     a.HB = std::min(H, 64); a.NQ = std::max(1, 64 / a.HB);
     hipLaunchKernelGGL((k_latent_attn<RT, RS>), dim3((a.R + a.NQ - 1) / a.NQ, (H + a.HB - 1) / a.HB), dim3(256), 2 * tile, st, a);

@@ -15,11 +15,7 @@ bool heads_mfma_sizes(int d, int maps, int dv, bool f32, int* dkp, int* dvp) {
 template <int DK, int DV, int MAPS>
 static int heads_prompt_launch(HeadsAttnArgs a, hipStream_t st) {
   constexpr int lds = 2 * 64 * (DK + DV) * 2;
-  static bool attr_done = false;
-  if (!attr_done) {
-    HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_heads_prompt<DK, DV, MAPS>), hipFuncAttributeMaxDynamicSharedMemorySize, lds));
-    attr_done = true;
-  }
+  HIPCHK((lds_room<&k_heads_prompt<DK, DV, MAPS>>(lds)));
   const int GQ = a.g.H / a.g.G;
   a.HB = std::min(GQ, 64 / MAPS); a.NQ = 64 / MAPS / a.HB; a.hchunks = (GQ + a.HB - 1) / a.HB;
   hipLaunchKernelGGL((k_heads_prompt<DK, DV, MAPS>), dim3(a.g.G * a.hchunks, (a.R + a.NQ - 1) / a.NQ), dim3(256), lds, st, a);
@@ -30,12 +26,8 @@ template <int DK, int DV, int MAPS>
 static int heads_launch(bool tall, bool fused, int splits, HeadsAttnArgs a, hipStream_t st) {
   if (tall) return heads_prompt_launch<DK, DV, MAPS>(a, st);
   constexpr int lds = 64 * (DK + DV) * 2;
-  static bool attr_done = false;
-  if (!attr_done) {
-    HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_heads_decode<DK, DV, true, MAPS>), hipFuncAttributeMaxDynamicSharedMemorySize, lds));
-    HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_heads_decode<DK, DV, false, MAPS>), hipFuncAttributeMaxDynamicSharedMemorySize, lds));
-    attr_done = true;
-  }
+  if (fused) HIPCHK((lds_room<&k_heads_decode<DK, DV, true, MAPS>>(lds)));
+  else HIPCHK((lds_room<&k_heads_decode<DK, DV, false, MAPS>>(lds)));
   const dim3 grid(a.R, a.g.G * a.hchunks, splits);
   if (fused) hipLaunchKernelGGL((k_heads_decode<DK, DV, true, MAPS>), grid, dim3(256), lds, st, a);
   else hipLaunchKernelGGL((k_heads_decode<DK, DV, false, MAPS>), grid, dim3(256), lds, st, a);
@@ -69,11 +61,7 @@ template <int DK, int DV>
 static int pair_launch(const HeadsAttnArgs& a, int splits, const RetArgs& b, const HeadsRope& rope, hipStream_t st) {
   constexpr int lds = 64 * (DK + DV) * 2;
   const size_t need = std::max((size_t)lds, ret_step_lds(b.g));
-  static size_t most = 0;
-  if (need > most) {
-    HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_pair_decode<DK, DV>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)need));
-    most = need;
-  }
+  HIPCHK((lds_room<&k_pair_decode<DK, DV>>(need)));
   hipLaunchKernelGGL((k_pair_decode<DK, DV>), dim3(a.R * (b.g.H + a.g.G * a.hchunks * splits)), dim3(256), need, st, a, splits, b, rope, a.Kp);
   LAUNCHCHK();
   return IXT_OK;

@@ -61,12 +61,8 @@ int scan_rank(ixt_ctx* c, const HLayer& W, const Slices& low, int R, hipStream_t
 }
 template <typename T, int SPL, int LPC>
 static int scan_chunks(ixt_ctx* c, const ScanArgs& a, int R, int nseg_max, int Kp, hipStream_t st) {
-  static bool attr_done = false;
-  if (!attr_done) {
-    HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_scan_sums<T, SPL, LPC>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)scan_lds<SPL, LPC, false>()));
-    HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_scan_out<T, SPL, LPC>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)scan_lds<SPL, LPC, true>()));
-    attr_done = true;
-  }
+  HIPCHK((lds_room<&k_scan_sums<T, SPL, LPC>>(scan_lds<SPL, LPC, false>())));
+  HIPCHK((lds_room<&k_scan_out<T, SPL, LPC>>(scan_lds<SPL, LPC, true>())));
   constexpr int CB = 256 / LPC;
   const ScanGeom& g = a.g;
   const int chunks = R / SEG_CHUNK + nseg_max;

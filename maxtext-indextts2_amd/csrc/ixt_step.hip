@@ -39,11 +39,7 @@ static StepPlan step_plan(const ixt_ctx* c, int R) {
 }
 template <int HD, int GQ>
 static int launch_step_t(const StepArgs& a, int L, size_t lds, hipStream_t st) {
-  static bool attr_done = false;
-  if (!attr_done) {
-    HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_step<HD, GQ>), hipFuncAttributeMaxDynamicSharedMemorySize, STEP_LDS));
-    attr_done = true;
-  }
+  HIPCHK((lds_room<&k_step<HD, GQ>>(STEP_LDS)));
   hipLaunchKernelGGL((k_step<HD, GQ>), dim3((unsigned)(L * a.per_layer)), dim3(STEP_NW * 64), lds, st, a);
   LAUNCHCHK();
   return IXT_OK;
@@ -128,14 +124,10 @@ int launch_step(ixt_ctx* c, int R, const int32_t* tokens, int fresh, const bf16_
   return set_err(IXT_ERR_UNSUPPORTED, "step geometry hd=%d gq=%d", c->D, c->GQ);
 }
 
-static int launch_mid_t(const MidArgs& a, int G, int blocks, size_t lds, hipStream_t st) {
-  const auto kernel = G == 2 ? &k_mid<2> : G == 3 ? &k_mid<3> : &k_mid<4>;
-  static bool attr_done[5] = {};
-  if (!attr_done[G]) {
-    HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 2 * MID_BUF_STEPS * 1024));
-    attr_done[G] = true;
-  }
-  hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(MID_NW * 64), lds, st, a);
+template <int G>
+static int launch_mid_t(const MidArgs& a, int blocks, size_t lds, hipStream_t st) {
+  HIPCHK((lds_room<&k_mid<G>>(2 * MID_BUF_STEPS * 1024)));
+  hipLaunchKernelGGL(k_mid<G>, dim3((unsigned)blocks), dim3(MID_NW * 64), lds, st, a);
   LAUNCHCHK();
   return IXT_OK;
 }
@@ -175,5 +167,5 @@ int launch_mid(ixt_ctx* c, int R, int l, const int32_t* tokens, bool final, cons
   }
   if (hidden) *hidden = a.hout;
   if (normed) *normed = a.xn1;
-  return launch_mid_t(a, G, blocks, p.lds, st);
+  return G == 2 ? launch_mid_t<2>(a, blocks, p.lds, st) : G == 3 ? launch_mid_t<3>(a, blocks, p.lds, st) : launch_mid_t<4>(a, blocks, p.lds, st);
 }

@@ -6,8 +6,7 @@
 template <int HD, int GQ, int NW, int NR, bool GIVEN = false>
 static void mtile_launch(const dim3& grid, const TileAttnArgs& ta, hipStream_t st) {
   constexpr size_t lds = mtile_lds(HD, NW, NR);
-  static const hipError_t room = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_attn_mtile<HD, GQ, NW, NR, GIVEN>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  (void)room;                                            // (a launch without room for its LDS fails, and the caller looks at that)
+  if (lds_room<&k_attn_mtile<HD, GQ, NW, NR, GIVEN>>(lds) != hipSuccess) return;      // (the runtime's last error, which the caller looks at)
   hipLaunchKernelGGL((k_attn_mtile<HD, GQ, NW, NR, GIVEN>), grid, dim3(NW * 64), lds, st, ta);
 }
 // The smallest form that holds the call's longest prefix (ta.lmax keys, at most 4096).

@@ -206,11 +206,7 @@ static int gemm_launch(hipStream_t st, TGemm& g) {
   // waves and their tiles: 256 x 256: 2 x 4 of 128 x 64; 256 x 128: 4 x 2 and 128 x 128: 2 x 2 of 64 x 64; 128 x 64: 4 of 32 x 64; 64 x 64: 2 x 2 of 32 x 32
   constexpr int WM = BN == BM ? 2 : 4, WN = BN == 256 ? 4 : BN == 64 && BM == 128 ? 1 : 2, MI = BM / 16 / WM, NI = BN / 16 / WN, NS = 4, lds = (TA && TB ? NS : NS + 1) * (BM + BN) * 64;
   const auto kernel = k_tgemm<TA, TB, MI, NI, WM, WN, NS, FOLD>;
-  static bool attr_done = false;
-  if (!attr_done) {
-    TCHK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds));
-    attr_done = true;
-  }
+  TCHK((lds_room<&k_tgemm<TA, TB, MI, NI, WM, WN, NS, FOLD>>(lds)));
   if (g.nb1 == 0) g.nb1 = g.nb2 = 1;
   g.mt = (g.M + BM - 1) / BM;
   for (int i = 0; i < 3; ++i) g.nt[i] = i < g.nprob ? (g.N[i] + BN - 1) / BN : 0;
@@ -258,11 +254,7 @@ static int xent(hipStream_t st, const bf16_t* logits, const int32_t* targets, co
     hipLaunchKernelGGL(k_t_xent, dim3(n), dim3(256), 0, st, logits, targets, seg, dlog, row_loss, V, ld);
   } else {
     constexpr int two = 2 * 8192 * sizeof(float), one = 96 * 1024;
-    static bool attr_done = false;
-    if (!attr_done) {
-      TCHK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_t_xent_wide), hipFuncAttributeMaxDynamicSharedMemorySize, one));
-      attr_done = true;
-    }
+    TCHK(lds_room<&k_t_xent_wide>(one));
     hipLaunchKernelGGL(k_t_xent_wide, dim3(n), dim3(1024), (size_t)V * sizeof(bf16_t) * 512 > (size_t)192 << 20 ? one : two, st, logits, targets, seg, dlog, row_loss, V, ld);
   }
   TLAUNCH();
