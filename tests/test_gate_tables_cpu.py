@@ -1,11 +1,21 @@
 """The gates of the units' ring products come from tables of 2 x 2177 weights (csrc/ixt_device.h, ixt_gate_at): bf16(a w(a)) with w(a) taken where |a| is clamped to
 2^-10 .. 2^7.  Every bf16 value of a, infinities included, against the oracle's gate: the clamp takes nothing away.  Bits are compared, there is no tolerance."""
+import os
+import re
+
 import numpy as np
 import pytest
 
+import helpers as H
 from oracle import oracle as O
 
-LO, N = (127 - 10) << 7, 17 * 128 + 1
+
+def constant(name):
+  with open(os.path.join(H.importlib.import_module("maxtext-indextts2_amd.build").CSRC, "ixt_device.h"), encoding="utf-8") as f:
+    return eval(re.search(rf"#define {name} (.*?)(//|\n)", f.read()).group(1), {"__builtins__": {}})
+
+
+LO, N = constant("IXT_GATE_LO"), constant("IXT_GATE_N")
 f32 = np.float32
 
 

@@ -107,3 +107,17 @@ def test_softmax_of_peaked_rows(length, drop):
   b = packed_batch(cfg, 41)
   b["inputs"][:, 3::7] = 7
   one_step(cfg, params, b)
+
+
+@pytest.mark.parametrize("vocab", [264, 16392, 200072])
+def test_loss_of_rows_with_an_infinite_logit(vocab):
+  """A logit of -inf in every row, in the loss by four waves a row and by sixteen (two blocks a CU and one): it adds nothing to the sum, and the loss and the logits kernel's gradient are the oracle's."""
+  cfg = train_config(base_emb_dim=64, base_num_query_heads=2, base_num_kv_heads=1, head_dim=64, base_mlp_dim=72, vocab_size=vocab, max_target_length=24, per_device_batch_size=1.0)
+  params = f32_params(cfg, 8)
+  params["params/token_embedder/embedding"].reshape(vocab, 64)[:, 0] = 12.0
+  out = "params/decoder/logits_dense/kernel"
+  w = params[out].reshape(64, vocab)
+  w[:, vocab - 3], w[0, vocab - 3] = 0.0, -3e38
+  b = packed_batch(cfg, 41)
+  b["targets"][b["targets"] == vocab - 3] = 5
+  one_step(cfg, params, b, [out])
