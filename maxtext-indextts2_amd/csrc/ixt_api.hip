@@ -737,8 +737,9 @@ static void timing_end(ixt_ctx* c, hipStream_t st, int idx) {
 // chunk takes, in units of 10 ns, measured on 9 numbers of rows (128 .. 2048) x 8 projections (K 2048 .. 9216, N 2048 .. 18432) -- tile 4: 100, 1: 62, 2: 44,
 // 5: 31 (52 for two blocks of a CU), 3: 22, 6: 19, 7: 66 (122 for two).  The least estimate is within 6 % of the fastest tile on all but 3 of these 72
 // (within 12 %); the rule that looked at the number of 128 x 128 tiles alone took 62 us where this takes 40 (256 x 2304 outputs, K 9216) and 122 where this
-// takes 102 (1525 x 14336, K 2048).  With the products' present loops a chunk takes 60, 45, 31, 21, 14, 13 and 43 of these units (73 for two of
-// tile 7, 32 of tile 5), and a round 230 to 660 beside its chunks: the rule is 1.4 % off the fastest tile in the geometric mean of such launches, one with the new figures 0.8 %.
+// takes 102 (1525 x 14336, K 2048).
+// These are the times of the products' former loops.  With the present ones a chunk takes 60, 45, 31, 21, 14, 13 and 43 (73 for two of tile 7, 32 of tile 5), and a round 230 to 660 beside its
+// chunks, which no single figure a tile stands for: by the figures below the tile is 1.4 % off the fastest in the geometric mean of such launches, by a rule of two figures a tile 0.8 %.
 static int ring_pick(const ixt_ctx* c, int epi, int R, int N, bool routed, bool wring) {
   if (c->ring_cfg >= 1 && c->ring_cfg <= 7 && !(epi == GEPI_SWIGLU && (c->ring_cfg == 3 || c->ring_cfg == 6)) && !(epi == GEPI_UNEMBED && c->ring_cfg != 1) && !(routed && c->ring_cfg == 4) &&
       !(wring && c->ring_cfg == 7)) return c->ring_cfg;

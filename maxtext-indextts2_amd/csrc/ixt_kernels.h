@@ -84,7 +84,7 @@ __host__ __device__ __forceinline__ int qk_col(int i, int half) {
 //   the L2-resident slab lands and is written to LDS while the weight fragments are still on their way from HBM.
 //   Routed experts (rb_exp != nullptr; NRB = 1): row block rb belongs to expert rb_exp[rb], whose kernels start wstride 16-byte units after
 //   wt; a row block of no expert (-1) leaves at once (k_moe_plan, ixt_moe_kernels.h).  cnt_off: the plan's counts and offsets; the slices' rows behind an expert's last copy are not
-//   written (8 tokens, two of 8 experts each: 59 MB of slices beside 940 of weights, 162 us; now 7, and 138).
+//   written (8 tokens, two of 8 experts each: 59 MB of slices beside 870 of weights, those of the 7.4 experts that had a token, 162 us; now 7, and 138).
 //   EPI = 1 (whole-K blocks only): the columns are interleaved (wi_0, wi_1) tiles (k_tile_w mode 2) and `out` is the bf16 activation buffer of the
 //   next dot (glu: that gated unit of the f32 totals instead, ixt_glu): the odd wave of a pair hands its totals to the even one through LDS, which writes bf16(bf16(a * bf16(sigmoid a)) * b) in the x layout
 //   (linears.py:331-361) -- no f32 slice leaves the chip (routed experts at decode: 132 MB of slices per layer and the kernel that re-read them).

@@ -57,7 +57,8 @@ struct SdotArgs {
 // 8 rows, 2048 columns, K 2048 and 7168 in turn: 7.9 us a launch by whole tiles (128 blocks), now 6.9; 4 rows, 1024 columns, K 1024 and 3584 with the tanh norm: 6.4 -> 6.0.
 // NORM 1: RMSNorm of bf16 rows [R][K]; 2: SdotRows, up to SDOT_ROWS rows, K <= 2048, every block for itself while its weights come.  Gated units of 8 rows, K 2048, 14336 columns: 13.2 us behind
 // a launch of 4.1 that took the norm, now 14.9 alone (sixteen waves a block, so that a wave has two units of a row beside its 16 KB of weights); 6416 columns 8.4 behind 4.1, now 10.4 (eight
-// waves, four units).
+// waves, four units).  Always eight rows' units: fewer rows' are read again.  32 decode steps of the benchmark's Vilepel with and without, ms: one row 17.76 / 16.65, four 18.32 / 17.41, eight 19.45 / 18.85
+// (width 2048), 11.93 / 11.08, 12.77 / 11.88, 13.84 / 13.12 (width 1024).
 template <int EPI, int NORM, bool HALF = false>
 __global__ __launch_bounds__(NORM == 2 && EPI == GEPI_F32 ? 512 : 1024) void k_sdot(SdotArgs a) {
   extern __shared__ __attribute__((aligned(16))) u32x4 sx[];

@@ -67,35 +67,7 @@ __device__ __forceinline__ void mtile_scores(const bf16_t* kp, const float* q, i
   products(0, NB - 2);
   products(1, NB - 1);
 }
-// block = (kv head, 16 query vectors = 16 / GQ consecutive rows x GQ heads), NW waves.  Super-block (4 pages, 128 keys) n NW + w belongs to wave w in
-// round n; its 128 x 16 scores stay in that wave's registers from the score products to the output products, so the keys one block holds are
-// 128 NW NR and nothing of them goes through LDS or memory.
-//   Scores: matrix rows = keys, columns = query vectors, one d a step (16x16x1: four blocks of 16 keys, each with the operand of its own lane group).  Row i
-//   of block b is token 4 t + i % 4 of page i / 4, t = b and 4 + b: a lane then holds the 32 tokens of ONE page (its 16-lane group) for one query vector, and
-//   the page's sum of exponentials is a sum over its own registers, in order.  K is read once, 16 bytes a lane: eight d of the lane's own key, operands as they are
-//   (with four d a step, 16x16x4, they had to change lanes first, 18 vector instructions for eight products instead of 8: 33.7 us of a block's 103 in <8, 4>, now 28, which is
-//   the products' own time).  The query operand comes from LDS, 16 bytes for four steps.
-//   Softmax: max over lanes and waves; page sums meet in LDS and every lane adds its vector's in page order.  e / l with one reciprocal per lane:
-//   two corrections of the quotient give the correctly rounded one where no remainder is subnormal (e >= 2^-96); otherwise the divide itself.
-//   Outputs: matrix rows = value columns, P as the other operand after a 4 x 4 transpose of lane groups and registers.  A lane's 16 bytes of V are 8
-//   columns of one token: column 8 i + x belongs to row i of tile x.  Page chains start from zero, four pages add up in order; the super-blocks of a
-//   round meet in LDS, where the thread that owns (vector, column) adds them in order: with two buffers there, one barrier a round (four, half of the columns at
-//   a time, took 3 us more of the 103).
-// A key that a row does not see has P = +0 (k_attn_tile says why that is exact); tokens past the end are re-reads of the last one.
-// Rows of other page groups in the tile are worked off group by group, dealt among `shares` blocks.  grid = (kv heads, tiles, parts x shares): parts = 1 or
-// the number of 128-column parts of a value (the two halves of head_dim 256 in two blocks, each taking the scores anew), shares = 1 or more, both for
-// launches that leave CUs idle otherwise.
-// Bound by the matrix units and the vector units TOGETHER: an f32 product and a vector instruction of the same SIMD take turns, whichever waves they belong to (products
-// alone 150 TFLOP/s; one bf16 -> f32 conversion in front of each 116, eight in front of eight 129).  So what counts is vector instructions: operands of a
-// step converted together, no mask where every row sees every key (sees_all; the selects of a score were a branch each), weights rounded and packed two at a time ahead
-// of the transpose.  A block of <8, 4> at 3072 to 3900 keys: 4.1 us until the first scores, 28 scores, 12 maxima and exponentials, 5 weights, 43 outputs (their products: 27 and 27); the
-// clock stays at 2.2 to 2.4 GHz.  Tried without gain: a priority for half of the waves; values by 16x16x1 products, too, four pages at a time from weights as they lie (286
-// against 293 us at <= 3072 keys, but 403 against 375 at <= 3900 and 118 against 117 with heads of 256: the sums of four pages leave no registers); a whole page of values
-// ahead (spills: 316 us).  Keys and values widened to f32 by a launch ahead: level up to 2048 keys.
-// What the bound of two or three blocks a CU leaves no register for goes through scratch.  Registers spilled, heads of 128: <2, 1> 32, <8, 3> 23, <8, 4> 76; heads of 256: <8, 3> 33.
-// Measured against k_attn_tile, 16 heads of 128, 1024 rows at <= 1024 / 2048 / 3072 keys 282 / 860 / 1143 us, before the scores' 16x16x1 products and the exchange with one barrier
-// 92 / 212 / 310, now 87 / 198 / 293.  828 rows at <= 3900 keys 1496, 408, 375 us (63 TFLOP/s).  8 heads of 256 on 4, 256 rows at <= 1756 / 2756 keys: 88 / 131, 79 / 117 us.
-// Prompts of <= 256 keys: two waves per block; with four, two of them had nothing to do (eight packed ones, 1525 rows: 90.2 us against 67.6).
+// the soft cap of a super-block's scores
 __device__ __forceinline__ void mtile_cap(ixt_f32x16& S0, ixt_f32x16& S1, float cap) {
 #pragma unroll
   for (int k = 0; k < 16; ++k) {
@@ -157,6 +129,35 @@ __global__ __launch_bounds__(512, 2) void k_attn_mscores(TileAttnArgs a) {
 // would take a CU's second block away.
 constexpr int mtile_buffers(int hd, int nw, int nr) { return nr > 1 && (nw == 8 || hd <= 128) ? 2 : 1; }
 constexpr size_t mtile_lds(int hd, int nw, int nr) { return (size_t)mtile_buffers(hd, nw, nr) * nw * 16 * ((hd >= 128 ? 128 : hd) + 4) * 4; }
+// block = (kv head, 16 query vectors = 16 / GQ consecutive rows x GQ heads), NW waves.  Super-block (4 pages, 128 keys) n NW + w belongs to wave w in
+// round n; its 128 x 16 scores stay in that wave's registers from the score products to the output products, so the keys one block holds are
+// 128 NW NR and nothing of them goes through LDS or memory.
+//   Scores: matrix rows = keys, columns = query vectors, one d a step (16x16x1: four blocks of 16 keys, each with the operand of its own lane group).  Row i
+//   of block b is token 4 t + i % 4 of page i / 4, t = b and 4 + b: a lane then holds the 32 tokens of ONE page (its 16-lane group) for one query vector, and
+//   the page's sum of exponentials is a sum over its own registers, in order.  K is read once, 16 bytes a lane: eight d of the lane's own key, operands as they are
+//   (with four d a step, 16x16x4, they had to change lanes first, 18 vector instructions for eight products instead of 8: 33.7 us of a block's 103 in <8, 4>, now 28, which is
+//   the products' own time).  The query operand comes from LDS, 16 bytes for four steps.
+//   Softmax: max over lanes and waves; page sums meet in LDS and every lane adds its vector's in page order.  e / l with one reciprocal per lane:
+//   two corrections of the quotient give the correctly rounded one where no remainder is subnormal (e >= 2^-96); otherwise the divide itself.
+//   Outputs: matrix rows = value columns, P as the other operand after a 4 x 4 transpose of lane groups and registers.  A lane's 16 bytes of V are 8
+//   columns of one token: column 8 i + x belongs to row i of tile x.  Page chains start from zero, four pages add up in order; the super-blocks of a
+//   round meet in LDS, where the thread that owns (vector, column) adds them in order: with two buffers there, one barrier a round (four, half of the columns at
+//   a time, took 3 us more of the 103).
+// A key that a row does not see has P = +0 (k_attn_tile says why that is exact); tokens past the end are re-reads of the last one.
+// Rows of other page groups in the tile are worked off group by group, dealt among `shares` blocks.  grid = (kv heads, tiles, parts x shares): parts = 1 or
+// the number of 128-column parts of a value (the two halves of head_dim 256 in two blocks, each taking the scores anew), shares = 1 or more, both for
+// launches that leave CUs idle otherwise.
+// Bound by the matrix units and the vector units TOGETHER: an f32 product and a vector instruction of the same SIMD take turns, whichever waves they belong to (products
+// alone 150 TFLOP/s; one bf16 -> f32 conversion in front of each 116, eight in front of eight 129).  So what counts is vector instructions: operands of a
+// step converted together, no mask where every row sees every key (sees_all; the selects of a score were a branch each), weights rounded and packed two at a time ahead
+// of the transpose.  A block of <8, 4> at 3072 to 3900 keys: 4.1 us until the first scores, 28 scores, 12 maxima and exponentials, 5 weights, 43 outputs (their products: 27 and 27); the
+// clock stays at 2.2 to 2.4 GHz.  Tried without gain: a priority for half of the waves; values by 16x16x1 products, too, four pages at a time from weights as they lie (286
+// against 293 us at <= 3072 keys, but 403 against 375 at <= 3900 and 118 against 117 with heads of 256: the sums of four pages leave no registers); a whole page of values
+// ahead (spills: 316 us).  Keys and values widened to f32 by a launch ahead: level up to 2048 keys.
+// What the bound of two or three blocks a CU leaves no register for goes through scratch.  Registers spilled, heads of 128: <2, 1> 32, <8, 3> 23, <8, 4> 76; heads of 256: <8, 3> 33.
+// Measured against k_attn_tile, 16 heads of 128, 1024 rows at <= 1024 / 2048 / 3072 keys 282 / 860 / 1143 us, before the scores' 16x16x1 products and the exchange with one barrier
+// 92 / 212 / 310, now 87 / 198 / 293.  828 rows at <= 3900 keys 1496, 408, 375 us (63 TFLOP/s).  8 heads of 256 on 4, 256 rows at <= 1756 / 2756 keys: 88 / 131, 79 / 117 us.
+// Prompts of <= 256 keys: two waves per block; with four, two of them had nothing to do (eight packed ones, 1525 rows: 90.2 us against 67.6).
 // GIVEN: the scores are in memory (k_attn_mscores, the same rows)
 template <int HD, int GQ, int NW, int NR, bool GIVEN = false>
 __global__ __launch_bounds__(NW * 64, NR == 1 && NW <= 4 ? 3 : 2) void k_attn_mtile(TileAttnArgs a) {
