@@ -357,9 +357,10 @@ extern "C" int ixt_create(const ixt_config* cfg, ixt_ctx** out) {
     }
   }
   }
-  A(dmalloc(x, &x->gave, (size_t)1));
+  A(dmalloc(x, &x->gave, (size_t)2));
   void *fault = nullptr, *fault_dev = nullptr;
-  if (hipMemset(x->gave, 0, sizeof(int32_t)) != hipSuccess || hipHostMalloc(&fault, 64, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess)
+  const int32_t words[2] = {0, x->B};
+  if (hipMemcpy(x->gave, words, sizeof(words), hipMemcpyHostToDevice) != hipSuccess || hipHostMalloc(&fault, 64, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess)
     return fail(set_err(IXT_ERR_HIP, "words of the waits"));
   x->fault = (int32_t*)fault;
   *x->fault = 0;
@@ -1065,6 +1066,14 @@ int launch_dot(ixt_ctx* c, const bf16_t* x, const bf16_t* w, int K, int N, int R
 // routed blocks' QKV and O start at ring_min_rows.
 static int ring_model_rows(const ixt_ctx* c, bool decode) { return c->ring_min_rows > 128 ? c->ring_min_rows : std::min(c->ring_min_rows, c->ring_mid_rows + (decode ? 16 : 0)); }
 
+// the tokens of R rows out of their sampling pairs (nullptr: nobody wants them)
+int launch_argmax(ixt_ctx* c, int R, int pairs, int32_t* argmax_out, hipStream_t st) {
+  c->pairs = pairs;
+  if (argmax_out == nullptr || c->leave_pairs) return IXT_OK;
+  hipLaunchKernelGGL(k_argmax_final, dim3(R), dim3(256), 0, st, c->amax_val, c->amax_idx, pairs, argmax_out);
+  LAUNCHCHK();
+  return IXT_OK;
+}
 // logits (optional store) + greedy argmax for R rows of normed hidden states
 static int launch_unembed(ixt_ctx* c, const bf16_t* yT, int R, float* logits_out, int32_t* argmax_out, hipStream_t st) {
   const int K = c->E, N = c->V;
@@ -1073,9 +1082,7 @@ static int launch_unembed(ixt_ctx* c, const bf16_t* yT, int R, float* logits_out
     e.out = logits_out; e.amax_val = c->amax_val; e.amax_idx = c->amax_idx; e.cr = c->sample_cols;
     int wave_cols = 0;
     TRY(launch_ring(c, GEPI_UNEMBED, yT, c->logits_w, K, N, R, e, false, st, 0, &wave_cols));
-    hipLaunchKernelGGL(k_argmax_final, dim3(R), dim3(256), 0, st, c->amax_val, c->amax_idx, wave_cols, argmax_out);
-    LAUNCHCHK();
-    return IXT_OK;
+    return launch_argmax(c, R, wave_cols, argmax_out, st);
   }
   if (R >= c->gemm_min_rows && c->unembed_gemm) {   // many rows: the tiled GEMM with the sampling epilogue (weights pulled through L2 half as often)
     const int ntile_ = N / 16, ncolg = (ntile_ + 7) / 8, zb = (R + 127) / 128;
@@ -1085,9 +1092,7 @@ static int launch_unembed(ixt_ctx* c, const bf16_t* yT, int R, float* logits_out
     if (zb == 1) hipLaunchKernelGGL((k_gemm<true, 4, 1, 0>), grid, dim3(256), (size_t)64 * 1024, st, reinterpret_cast<const u32x4*>(yT), reinterpret_cast<const u32x4*>(c->logits_w), K, N, R, logits_out, ncolg, zb, c->amax_val, c->amax_idx, c->sample_cols);
     else hipLaunchKernelGGL((k_gemm<false, 4, 1, 0>), grid, dim3(256), (size_t)64 * 1024, st, reinterpret_cast<const u32x4*>(yT), reinterpret_cast<const u32x4*>(c->logits_w), K, N, R, logits_out, ncolg, zb, c->amax_val, c->amax_idx, c->sample_cols);
     timing_end(c, st, ti);
-    hipLaunchKernelGGL(k_argmax_final, dim3(R), dim3(256), 0, st, c->amax_val, c->amax_idx, 2 * ncolg, argmax_out);
-    LAUNCHCHK();
-    return IXT_OK;
+    return launch_argmax(c, R, 2 * ncolg, argmax_out, st);
   }
   const int ntile = N / 16, nwaves = (ntile + 3) / 4;
   const int rowblocks = (R + 15) / 16;
@@ -1107,9 +1112,7 @@ static int launch_unembed(ixt_ctx* c, const bf16_t* yT, int R, float* logits_out
   if (nrb == 4) UNEMB(4); else if (nrb == 2) UNEMB(2); else UNEMB(1);
 #undef UNEMB
   timing_end(c, st, ti);
-  hipLaunchKernelGGL(k_argmax_final, dim3(R), dim3(256), 0, st, c->amax_val, c->amax_idx, nwaves, argmax_out);
-  LAUNCHCHK();
-  return IXT_OK;
+  return launch_argmax(c, R, nwaves, argmax_out, st);
 }
 
 template <int HD, int GQ>
@@ -1481,11 +1484,7 @@ static int launch_logits_post(ixt_ctx* c, float* lg, int nl, int normalize, floa
   if ((size_t)nl * nblk > c->amax_cap) return set_err(IXT_ERR_INVALID, "argmax workspace too small");
   hipLaunchKernelGGL(k_logits_post, dim3(nblk, nl), dim3(256), 0, st, lg, c->V, normalize, sqrtf((float)c->E), cap, c->sample_cols, c->amax_val, c->amax_idx);
   LAUNCHCHK();
-  if (argmax_out != nullptr) {
-    hipLaunchKernelGGL(k_argmax_final, dim3(nl), dim3(256), 0, st, c->amax_val, c->amax_idx, nblk, argmax_out);
-    LAUNCHCHK();
-  }
-  return IXT_OK;
+  return launch_argmax(c, nl, nblk, argmax_out, st);
 }
 
 static int launch_gnorm(const GNormArgs& ga, int R, hipStream_t st) {
@@ -1578,11 +1577,12 @@ static int forward_rows_gemma2(ixt_ctx* c, int R, const int32_t* tokens, int len
     if (nl > c->NLmax) return set_err(IXT_ERR_INVALID, "too many logits rows (%d > %d)", nl, c->NLmax);
     if (!all_rows) TRY(launch_rownorm(c, 2, nl, nullptr, nullptr, lrows ? hcur : hcur + (size_t)lrow0 * E, nullptr, c->final_norm, c->xn, st, 1, lrows));
     float* lg = logits_out ? logits_out : c->glogits;
-    TRY(launch_unembed(c, c->xn, nl, lg, argmax_out, st));
     // decoders.py:552-565: the division and the cap belong to the tied head
     const int normalize = cf.logits_via_embedding && cf.normalize_embedding_logits;
     const float cap = cf.logits_via_embedding ? cf.final_logits_soft_cap : 0.0f;
-    if (normalize || cap > 0.0f) TRY(launch_logits_post(c, lg, nl, normalize, cap, argmax_out, st));
+    const bool post = normalize || cap > 0.0f;                  // (the tokens are those of the capped logits)
+    TRY(launch_unembed(c, c->xn, nl, lg, post ? nullptr : argmax_out, st));
+    if (post) TRY(launch_logits_post(c, lg, nl, normalize, cap, argmax_out, st));
   }
   c->h_final = hcur; c->h_final_rows = R;
   return IXT_OK;
@@ -2085,12 +2085,16 @@ extern "C" int ixt_prefill_rows(ixt_ctx* c, int n_rows, const int32_t* tokens_de
   return forward_rows(c, n_rows, tokens_dev, max_len, 0, n_logits, c->lrows, first_tokens_dev, logits_dev, false, st);
 }
 
-static int decode_rows(ixt_ctx* c, const int32_t* tokens_dev, const int32_t* pos_dev, int32_t* next_tokens_dev, float* logits_dev, int check_len,
+// advance: the pages take a token first (ixt_generate), and a row's position has to be its group's last
+static int decode_rows(ixt_ctx* c, const int32_t* tokens_dev, const int32_t* pos_dev, int32_t* next_tokens_dev, float* logits_dev, bool advance,
                        hipStream_t st) {
-  hipLaunchKernelGGL(k_rows_decode, dim3(1), dim3(c->B <= 1024 ? ((c->B + 63) / 64) * 64 : 1024), 0, st, c->row_slot, c->row_pos, c->row_active, c->row_tok,
-                     tokens_dev, pos_dev, c->ps.has_active_page, c->ps.num_pages_used, c->ps.sequence_lengths, check_len, c->P, c->Tmax, c->B);
+  const bool plain = c->may_wait && c->hy == nullptr && !c->gemma;
+  const bool step = plain && small_path_ok(c, c->B) && takes_step(c, c->B, true), mid = plain && !small_path_ok(c, c->B) && takes_mid(c, c->B);
+  const FrontRows f = step ? step_front(c) : mid ? mid_front(c) : FrontRows{};
+  hipLaunchKernelGGL(k_decode_front, dim3(step || mid ? 1 + c->B : 1), dim3(256), 0, st, c->ps, advance ? 1 : 0, c->row_slot, c->row_pos, c->row_active, c->row_tok, tokens_dev, pos_dev, c->Tmax, c->B, f,
+                     c->gave);
   LAUNCHCHK();
-  return forward_rows(c, c->B, c->row_tok, c->Tmax, 0, c->B, nullptr, next_tokens_dev, logits_dev, true, st);
+  return forward_rows(c, c->B, step || mid ? nullptr : c->row_tok, c->Tmax, 0, c->B, nullptr, next_tokens_dev, logits_dev, true, st);
 }
 
 extern "C" int ixt_decode_step(ixt_ctx* c, const int32_t* tokens_dev, const int32_t* pos_dev, int32_t* next_tokens_dev, float* logits_dev, void* stream) {
@@ -2098,17 +2102,14 @@ extern "C" int ixt_decode_step(ixt_ctx* c, const int32_t* tokens_dev, const int3
   TRY(ixt_wait_check(c));
   if (c->B > 1024) return set_err(IXT_ERR_UNSUPPORTED, "max_slots > 1024");
   const WaitPass pass(c, c->B, true, (hipStream_t)stream);
-  return decode_rows(c, tokens_dev, pos_dev, next_tokens_dev, logits_dev, 0, (hipStream_t)stream);
+  return decode_rows(c, tokens_dev, pos_dev, next_tokens_dev, logits_dev, false, (hipStream_t)stream);
 }
 
-static int generate_body(ixt_ctx* c, int32_t* tokens_dev, int32_t* next_pos_dev, int32_t* generated_dev, int32_t* result_data_dev, float* logits_dev,
-                         hipStream_t st) {
-  hipLaunchKernelGGL(k_pages_advance, dim3(1), dim3(64), 0, st, c->ps);
-  LAUNCHCHK();
-  TRY(decode_rows(c, tokens_dev, next_pos_dev, c->new_tok, logits_dev, 1, st));
-  hipLaunchKernelGGL(k_generate_epilogue, dim3(1), dim3(((c->B + 63) / 64) * 64), 0, st, c->new_tok, tokens_dev, next_pos_dev, generated_dev, result_data_dev, c->B, c->gave);
-  LAUNCHCHK();
-  return IXT_OK;
+static int generate_body(ixt_ctx* c, const int32_t* tokens_dev, const int32_t* next_pos_dev, float* logits_dev, hipStream_t st) {
+  c->leave_pairs = true;
+  const int rc = decode_rows(c, tokens_dev, next_pos_dev, c->new_tok, logits_dev, true, st);
+  c->leave_pairs = false;
+  return rc;
 }
 
 extern "C" int ixt_generate(ixt_ctx* c, int32_t* tokens_dev, int32_t* next_pos_dev, int32_t* generated_dev, int32_t* result_data_dev, float* logits_dev,
@@ -2118,10 +2119,18 @@ extern "C" int ixt_generate(ixt_ctx* c, int32_t* tokens_dev, int32_t* next_pos_d
   if (c->B > 1024) return set_err(IXT_ERR_UNSUPPORTED, "max_slots > 1024");
   hipStream_t st = (hipStream_t)stream;
   const WaitPass pass(c, c->B, true, st);
-  if (!c->cfg.use_hip_graph || c->timing) return generate_body(c, tokens_dev, next_pos_dev, generated_dev, result_data_dev, logits_dev, st);
+  const auto finish = [&](int pairs) -> int {
+    hipLaunchKernelGGL(k_decode_finish, dim3(c->B), dim3(256), 0, st, c->amax_val, c->amax_idx, pairs, tokens_dev, next_pos_dev, generated_dev, result_data_dev, c->gave, c->gave + 1);
+    LAUNCHCHK();
+    return IXT_OK;
+  };
+  if (!c->cfg.use_hip_graph || c->timing) {
+    TRY(generate_body(c, tokens_dev, next_pos_dev, logits_dev, st));
+    return finish(c->pairs);
+  }
   if (!ixt_weights_complete(c)) return set_err(IXT_ERR_NOT_LOADED, "weights incomplete");
   char key[160];
-  snprintf(key, sizeof(key), "%p/%p/%p/%p/%p/%d", (void*)tokens_dev, (void*)next_pos_dev, (void*)generated_dev, (void*)result_data_dev, (void*)logits_dev, c->may_wait ? 1 : 0);
+  snprintf(key, sizeof(key), "%p/%p/%p/%d", (void*)tokens_dev, (void*)next_pos_dev, (void*)logits_dev, c->may_wait ? 1 : 0);
   auto it = c->graphs.find(key);
   if (it == c->graphs.end()) {
     // capture on a private stream so the caller's stream state is untouched
@@ -2130,7 +2139,7 @@ extern "C" int ixt_generate(ixt_ctx* c, int32_t* tokens_dev, int32_t* next_pos_d
     hipGraph_t graph = nullptr;
     HIPCHK(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
     c->capturing = true;
-    int rc = generate_body(c, tokens_dev, next_pos_dev, generated_dev, result_data_dev, logits_dev, cs);
+    int rc = generate_body(c, tokens_dev, next_pos_dev, logits_dev, cs);
     c->capturing = false;
     hipError_t e = hipStreamEndCapture(cs, &graph);
     if (rc != IXT_OK || e != hipSuccess) {
@@ -2140,6 +2149,7 @@ extern "C" int ixt_generate(ixt_ctx* c, int32_t* tokens_dev, int32_t* next_pos_d
     }
     GraphEntry ge;
     ge.forms = c->forms;
+    ge.pairs = c->pairs;
     e = hipGraphInstantiate(&ge.exec, graph, nullptr, nullptr, 0);
     (void)hipGraphDestroy(graph);
     (void)hipStreamDestroy(cs);
@@ -2152,7 +2162,7 @@ extern "C" int ixt_generate(ixt_ctx* c, int32_t* tokens_dev, int32_t* next_pos_d
   }
   HIPCHK(hipGraphLaunch(it->second.exec, st));
   c->forms = it->second.forms;
-  return IXT_OK;
+  return finish(it->second.pairs);
 }
 
 // --------------------------------------------------------------------------------------- op-level

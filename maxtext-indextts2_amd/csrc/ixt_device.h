@@ -199,7 +199,7 @@ template <typename V> __device__ __forceinline__ void stg16_agent(void* p, const
 }
 
 // Waits of a block for another one of its launch are bounded: `polls` looks, then the block says so and goes on.  `gave` is the pass's own word on the device (cleared in front of a pass; who
-// sees it set waits no more, and k_generate_epilogue marks the result), `fault` the context's in host memory, which the next call reports.
+// sees it set waits no more, and k_decode_finish marks the result), `fault` the context's in host memory, which the next call reports.
 struct IxtWait { int32_t *gave, *fault; int polls; };
 __device__ __forceinline__ void ixt_gave_up(const IxtWait& w) {
   __hip_atomic_store(w.gave, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

@@ -1123,8 +1123,8 @@ static int hybrid_logits(ixt_ctx* c, int R, int lrow0, int nl, const int32_t* lr
     Slices t;
     TRY(hdot<T>(c, (const T*)m->xn, m->head, n, c->part, c->part_floats, st, &t));
     hipLaunchKernelGGL(k_head_post, dim3(nblk, n), dim3(256), 0, st, t, m->V, m->logit_scale, c->sample_cols, logits_out ? logits_out + (size_t)i0 * m->V : nullptr, c->amax_val, c->amax_idx);
-    if (argmax_out) hipLaunchKernelGGL(k_argmax_final, dim3(n), dim3(256), 0, st, c->amax_val, c->amax_idx, nblk, argmax_out + i0);
     LAUNCHCHK();
+    TRY(launch_argmax(c, n, nblk, argmax_out ? argmax_out + i0 : nullptr, st));
   }
   return IXT_OK;
 }

@@ -37,7 +37,7 @@ struct TimingPair { hipEvent_t a, b; double bytes; int family; };   // family: 0
 
 struct GraphEntry {
   hipGraphExec_t exec;
-  int forms = 0;
+  int forms = 0, pairs = 0;
 };
 
 struct HybridModel;           // IXT_BLOCK_HYBRID (ixt_hybrid.h)
@@ -180,12 +180,15 @@ struct ixt_ctx {
   std::vector<TimingPair> tpairs;
   size_t tused = 0;
   // bounded waits between blocks of a launch (IxtWait)
-  int32_t *gave = nullptr, *fault = nullptr, *fault_dev = nullptr;   // fault: pinned host memory, and what the GPU knows it by
+  int32_t *gave = nullptr, *fault = nullptr, *fault_dev = nullptr;   // gave[1]: k_decode_finish's blocks to come; fault: pinned host memory, and what the GPU knows it by
   int wait_polls = 1 << 20;     // (0.5 to 1 s)
   IxtWait wait() const { return IxtWait{gave, fault_dev, wait_polls}; }
   // graphs keyed by the pointer tuple of ixt_generate
   std::map<std::string, GraphEntry> graphs;
   bool capturing = false;
+  // the sampling pairs of the pass being enqueued are left to k_decode_finish, so many a row (launch_argmax)
+  bool leave_pairs = false;
+  int pairs = 0;
   std::vector<void*> allocs;
 };
 
@@ -216,5 +219,8 @@ int launch_sdot(ixt_ctx* c, int epi, bool norm, const bf16_t* x, const bf16_t* s
 int step_init(ixt_ctx* c);
 bool step_fits(const ixt_ctx* c, int R);
 bool mid_fits(const ixt_ctx* c, int R);
+int launch_argmax(ixt_ctx* c, int R, int pairs, int32_t* argmax_out, hipStream_t st);
+FrontRows step_front(const ixt_ctx* c);
+FrontRows mid_front(const ixt_ctx* c);
 int launch_mid(ixt_ctx* c, int R, int l, const int32_t* tokens, bool final, const bf16_t** hidden, const bf16_t** normed, hipStream_t st);
 int launch_step(ixt_ctx* c, int R, const int32_t* tokens, int fresh, const bf16_t** hidden, hipStream_t st);

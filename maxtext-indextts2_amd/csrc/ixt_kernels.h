@@ -574,13 +574,11 @@ static __global__ void k_transpose_x(const bf16_t* x, bf16_t* xT, int R, int K) 
   if (k < K) xT[xidx(r, k, K)] = x[(size_t)r * K + k];
 }
 
-// final (max, first index) over the per-tile pairs.  grid = R, block 256.
-static __global__ __launch_bounds__(256) void k_argmax_final(const float* __restrict__ amax_val, const int32_t* __restrict__ amax_idx, int ntiles, int32_t* out_idx) {
+// (max, first index) over a row's per-tile pairs, on thread 0 of a block of 256
+__device__ __forceinline__ int argmax_row(const float* __restrict__ pv, const int32_t* __restrict__ pi, int ntiles) {
   __shared__ float bv[4];
   __shared__ int bi[4];
-  const int r = blockIdx.x, tid = threadIdx.x;
-  const float* pv = amax_val + (size_t)r * ntiles;
-  const int32_t* pi = amax_idx + (size_t)r * ntiles;
+  const int tid = threadIdx.x;
   float best = -INFINITY;
   int bidx = 0x7fffffff;
   auto take = [&](float v, int i2) { if (v > best || (v == best && i2 < bidx)) { best = v; bidx = i2; } };
@@ -604,8 +602,13 @@ static __global__ __launch_bounds__(256) void k_argmax_final(const float* __rest
   __syncthreads();
   if (tid == 0) {
     for (int w = 1; w < 4; ++w) take(bv[w], bi[w]);
-    out_idx[r] = bidx == 0x7fffffff ? 0 : bidx;
   }
+  return bidx == 0x7fffffff ? 0 : bidx;
+}
+// grid = R, block 256.
+static __global__ __launch_bounds__(256) void k_argmax_final(const float* __restrict__ amax_val, const int32_t* __restrict__ amax_idx, int ntiles, int32_t* out_idx) {
+  const int r = blockIdx.x, best = argmax_row(amax_val + (size_t)r * ntiles, amax_idx + (size_t)r * ntiles, ntiles);
+  if (threadIdx.x == 0) out_idx[r] = best;
 }
 
 // h_out = bf16(h_in + bf16(sum of slices))  (llama2.py:127, :157).  grid = (ceil(E/256), R), block 128, 2 columns per thread.
@@ -2126,41 +2129,6 @@ static __global__ void k_rows_packed(int32_t* row_slot, int32_t* row_pos, int32_
     row_slot[i] = ok ? g : 0; row_pos[i] = ok ? pos : 0; row_active[i] = (ok && pos / P < num_pages_used[g]) ? 1 : 0;
   }
 }
-// Decode rows: slot i at position pos[i] (the caller's decode_state["next_pos"]).  Active only when the page manager agrees: the slot
-// has an active page, the position is inside max_target_length and inside the pages granted so far (a page the pool could not grant
-// deactivates the row instead of letting it write through a stale page_map entry), and -- check_len, ixt_generate -- the position is
-// the one the page manager has just advanced to (sequence_lengths - 1): a slot that was prefilled but not inserted yet carries the
-// previous occupant's next_pos and stays idle until MaxEngine.insert.
-static __global__ void k_rows_decode(int32_t* row_slot, int32_t* row_pos, int32_t* row_active, int32_t* row_tok,
-                              const int32_t* tokens, const int32_t* pos, const int32_t* has_active, const int32_t* num_pages_used,
-                              const int32_t* sequence_lengths, int check_len, int P, int Tmax, int B) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < B) {
-    const int p = pos[i];
-    bool act = has_active[i] != 0 && p >= 0 && p < Tmax && p / P < num_pages_used[i];
-    if (check_len) act = act && p == sequence_lengths[i] - 1;
-    row_slot[i] = i; row_pos[i] = act ? p : 0; row_active[i] = act ? 1 : 0; row_tok[i] = tokens[i];
-  }
-}
-// maxengine.py:913-935
-// gave: a wait of the pass gave up, its tokens are not valid (one block: cleared for the next pass)
-static __global__ void k_generate_epilogue(const int32_t* new_tok, int32_t* tokens, int32_t* next_pos, int32_t* generated,
-                                    int32_t* result, int B, int32_t* gave) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  const int bad = *gave;
-  __syncthreads();
-  if (i == 0) *gave = 0;
-  if (i < B) {
-    tokens[i] = new_tok[i];
-    next_pos[i] = next_pos[i] + 1;
-    const int gnew = generated[i] + 1;
-    generated[i] = gnew;
-    result[i * 3 + 0] = new_tok[i];
-    result[i * 3 + 1] = bad ? 0 : 1;
-    result[i * 3 + 2] = gnew;
-  }
-}
-
 // =====================================================================================================
 // PageState kernels (inference/page_manager.py), one wave each, state in HBM.
 // =====================================================================================================
@@ -2302,10 +2270,7 @@ static __global__ __launch_bounds__(64) void k_pages_reserve(PageStateDev s, int
 
 // page_manager.py:331-412: every active group advances one token; groups that cross a page boundary take the next free page,
 // in group order
-static __global__ __launch_bounds__(64) void k_pages_advance(PageStateDev s) {
-  __shared__ int32_t need[IXT_MAX_GROUPS];
-  __shared__ int32_t got[IXT_MAX_GROUPS];
-  const int lane = threadIdx.x;
+static __device__ void wave_pages_advance(PageStateDev s, int lane, int32_t* need, int32_t* got) {
   int m = 0;
   for (int base = 0; base < s.decode_groups; base += 64) {
     const int g = base + lane;
@@ -2323,10 +2288,10 @@ static __global__ __launch_bounds__(64) void k_pages_advance(PageStateDev s) {
     m += __popcll(mask);
   }
   if (m == 0) return;
-  __syncthreads();
+  wave_lds_sync();
   const int found = wave_take_free(s, lane, m, got);
-  __syncthreads();
-  if (lane == 0 && found < m) s.status[2] = s.status[2] + (m - found);   // these rows stay idle (k_rows_decode) until a page is free
+  wave_lds_sync();
+  if (lane == 0 && found < m) s.status[2] = s.status[2] + (m - found);   // these rows stay idle (k_decode_front) until a page is free
   for (int k = lane; k < found; k += 64) {
     const int gg = need[k], nf = got[k];
     const int used = s.num_pages_used[gg];
@@ -2334,6 +2299,56 @@ static __global__ __launch_bounds__(64) void k_pages_advance(PageStateDev s) {
     s.num_pages_used[gg] = used + 1;
     s.active_page[gg] = nf;
   }
+}
+static __global__ __launch_bounds__(64) void k_pages_advance(PageStateDev s) {
+  __shared__ int32_t need[IXT_MAX_GROUPS], got[IXT_MAX_GROUPS];
+  wave_pages_advance(s, threadIdx.x, need, got);
+}
+// What stands in front of a decode pass, one launch instead of three.  Block 0: the page advance (ixt_generate) and the rows, slot i at position pos[i] (the caller's decode_state["next_pos"]).  Active only when the page manager agrees: the slot
+// has an active page, the position is inside max_target_length and inside the pages granted so far (a page the pool could not grant
+// deactivates the row instead of letting it write through a stale page_map entry), and -- check_len, ixt_generate -- the position is
+// the one the page manager has just advanced to (sequence_lengths - 1): a slot that was prefilled but not inserted yet carries the
+// previous occupant's next_pos and stays idle until MaxEngine.insert.
+// Blocks 1 + i, where the pass's first launch is k_step or k_mid: the embedding of row i, and zeros in that launch's counters.  gave: of the pass to come.
+// grid = 1 (+ B), block 256
+struct FrontRows { const bf16_t* embedding; bf16_t* h0; int E; int32_t* cnt; int ncnt; };
+__device__ __forceinline__ void front_row(const FrontRows& f, int row, int rows, int token) {
+  const bf16_t* src = f.embedding + (size_t)token * f.E;
+  for (int i = threadIdx.x; i < f.E / 8; i += 256) *reinterpret_cast<u32x4*>(f.h0 + (size_t)row * f.E + i * 8) = *reinterpret_cast<const u32x4*>(src + i * 8);
+  for (int i = row * 256 + threadIdx.x; i < f.ncnt; i += rows * 256) f.cnt[(size_t)i * 32] = 0;
+}
+static __global__ __launch_bounds__(256) void k_decode_front(PageStateDev s, int advance, int32_t* row_slot, int32_t* row_pos, int32_t* row_active, int32_t* row_tok, const int32_t* tokens, const int32_t* pos,
+                                                             int Tmax, int B, FrontRows f, int32_t* gave) {
+  __shared__ int32_t need[IXT_MAX_GROUPS], got[IXT_MAX_GROUPS];
+  if (blockIdx.x > 0) return front_row(f, blockIdx.x - 1, B, tokens[blockIdx.x - 1]);
+  if (threadIdx.x == 0) *gave = 0;
+  if (advance && threadIdx.x < 64) wave_pages_advance(s, threadIdx.x, need, got);
+  __syncthreads();
+  for (int i = threadIdx.x; i < B; i += 256) {
+    const int p = pos[i];
+    bool act = s.has_active_page[i] != 0 && p >= 0 && p < Tmax && p / s.P < s.num_pages_used[i];
+    if (advance) act = act && p == s.sequence_lengths[i] - 1;
+    row_slot[i] = i; row_pos[i] = act ? p : 0; row_active[i] = act ? 1 : 0; row_tok[i] = tokens[i];
+  }
+}
+// Behind it: a slot's token out of the sampling pairs of its row, and the slot's state (maxengine.py:913-935).  By a launch of its own behind the step's graph, into the caller's own result rows
+// instead of three launches; with the one in front, a step of one row 651 -> 642 us, of eight 812 -> 802, of 48 1632 -> 1620.  gave: a wait of the pass gave up, its tokens are not valid; the last block clears it.  left: blocks to
+// come, as many as slots between launches.  grid = B, block 256
+static __global__ __launch_bounds__(256) void k_decode_finish(const float* __restrict__ amax_val, const int32_t* __restrict__ amax_idx, int ntiles, int32_t* tokens, int32_t* next_pos, int32_t* generated,
+                                                              int32_t* result, int32_t* gave, int32_t* left) {
+  const int i = blockIdx.x;
+  int at = 0, made = 0, bad = 0;
+  if (threadIdx.x == 0) { at = next_pos[i]; made = generated[i]; bad = ldg_i32(gave); }
+  const int tok = argmax_row(amax_val + (size_t)i * ntiles, amax_idx + (size_t)i * ntiles, ntiles);
+  if (threadIdx.x != 0) return;
+  tokens[i] = tok;
+  next_pos[i] = at + 1;
+  generated[i] = made + 1;
+  result[i * 3 + 0] = tok;
+  result[i * 3 + 1] = bad ? 0 : 1;
+  result[i * 3 + 2] = made + 1;
+  if (!bad) return;                                             // (all blocks see the same word: it is set before the launch, and cleared behind the last one's read)
+  if (__hip_atomic_fetch_add(left, -1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 1) { stg_i32(left, gridDim.x); stg_i32(gave, 0); }
 }
 static __global__ void k_pages_set_active(PageStateDev s, int g, int v) { s.has_active_page[g] = v; }
 

@@ -607,10 +607,8 @@ __global__ __launch_bounds__(STEP_NW * 64, STEP_NW / 4) void k_step(StepArgs a) 
   step_dot<STEP_DOWN>(a, layer, b - a.nblk[STEP_UP], step_lds);
 }
 
-// rows of the embedding in front of the first layer; the counters of the launch behind it, and the pass's word of waits given up
-__global__ __launch_bounds__(256) void k_step_begin(const int32_t* tokens, const bf16_t* embedding, int E, bf16_t* h0, int32_t* cnt, int ncnt, int32_t* gave) {
-  const bf16_t* src = embedding + (size_t)tokens[blockIdx.x] * E;
-  for (int i = threadIdx.x; i < E / 8; i += 256) *reinterpret_cast<u32x4*>(h0 + (size_t)blockIdx.x * E + i * 8) = *reinterpret_cast<const u32x4*>(src + i * 8);
-  for (int i = blockIdx.x * 256 + threadIdx.x; i < ncnt; i += gridDim.x * 256) cnt[(size_t)i * 32] = 0;
+// rows of the embedding in front of the first layer; the counters of the launch behind it, and the pass's word of waits given up.  (Decode rows: k_decode_front.)
+static __global__ __launch_bounds__(256) void k_step_begin(const int32_t* tokens, FrontRows f, int32_t* gave) {
+  front_row(f, blockIdx.x, gridDim.x, tokens[blockIdx.x]);
   if (blockIdx.x == 0 && threadIdx.x == 0) *gave = 0;
 }

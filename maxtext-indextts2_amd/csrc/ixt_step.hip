@@ -102,7 +102,9 @@ int step_init(ixt_ctx* c) {
   return IXT_OK;
 }
 bool step_fits(const ixt_ctx* c, int R) { return c->step_ok && step_plan(c, R).ok; }
-// every layer of R rows; *hidden = the rows behind the last one.  fresh: step_attn
+FrontRows step_front(const ixt_ctx* c) { return FrontRows{c->embedding, c->h_a, c->E, c->step_cnt, c->L * STEP_PHASES * STEP_NS}; }
+FrontRows mid_front(const ixt_ctx* c) { return FrontRows{c->embedding, c->mid_ws, c->E, c->mid_cnt, (int)mid_words(c)}; }
+// every layer of R rows (tokens nullptr: what step_front names is done); *hidden = the rows behind the last one.  fresh: step_attn
 int launch_step(ixt_ctx* c, int R, const int32_t* tokens, int fresh, const bf16_t** hidden, hipStream_t st) {
   const StepPlan p = step_plan(c, R);
   c->forms |= IXT_FORM_STEP;
@@ -115,8 +117,10 @@ int launch_step(ixt_ctx* c, int R, const int32_t* tokens, int fresh, const bf16_
   a.eps = c->cfg.normalization_layer_epsilon;
   a.row_slot = c->row_slot; a.row_pos = c->row_pos; a.row_active = c->row_active; a.page_map = c->ps.page_map;
   a.rope_sin = c->rope_sin; a.rope_cos = c->rope_cos; a.g = c->geom;
-  hipLaunchKernelGGL(k_step_begin, dim3(R), dim3(256), 0, st, tokens, c->embedding, c->E, c->h_a, c->step_cnt, c->L * STEP_PHASES * STEP_NS, c->gave);
-  LAUNCHCHK();
+  if (tokens != nullptr) {
+    hipLaunchKernelGGL(k_step_begin, dim3(R), dim3(256), 0, st, tokens, step_front(c), c->gave);
+    LAUNCHCHK();
+  }
   *hidden = c->step_ws + (size_t)c->L * a.lstride - (size_t)16 * c->E;
 #define ST(HD_, GQ_) if (c->D == HD_ && c->GQ == GQ_) return launch_step_t<HD_, GQ_>(a, c->L, p.lds, st);
   ST(128, 1) ST(128, 2) ST(64, 1) ST(64, 2)
@@ -161,8 +165,8 @@ int launch_mid(ixt_ctx* c, int R, int l, const int32_t* tokens, bool final, cons
     if (here) before = i;
     blocks += a.nblk[i];
   }
-  if (l < 0) {
-    hipLaunchKernelGGL(k_step_begin, dim3(R), dim3(256), 0, st, tokens, c->embedding, c->E, h[0], c->mid_cnt, (int)mid_words(c), c->gave);
+  if (l < 0 && tokens != nullptr) {
+    hipLaunchKernelGGL(k_step_begin, dim3(R), dim3(256), 0, st, tokens, mid_front(c), c->gave);
     LAUNCHCHK();
   }
   if (hidden) *hidden = a.hout;

@@ -152,7 +152,6 @@ class MaxEngine(engine_api.Engine):
     self.page_state = self.page_manager.get_initial_page_state()
     self.rng = None
     self._params_loaded = False
-    self._result = torch.zeros((B, 3), dtype=torch.int32, device=self.device)
     self._first = torch.zeros((1,), dtype=torch.int32, device=self.device)
     self._page_failures = 0
     alive = weakref.ref(self)                            # (a result does not keep the engine)
@@ -489,11 +488,11 @@ class MaxEngine(engine_api.Engine):
       lg = torch.empty((self._B, 1, self.config.vocab_size), dtype=torch.float32, device=self.device)
       decode_state["logits"] = lg
     lg_ptr = ctypes.c_void_p(lg.data_ptr()) if isinstance(lg, torch.Tensor) else None
+    data = torch.empty((self._B, 3), dtype=torch.int32, device=self.device)
     _lib.check(self.lib.ixt_generate(self._ctx, ctypes.c_void_p(decode_state["tokens"].data_ptr()),
                                      ctypes.c_void_p(decode_state["next_pos"].data_ptr()),
                                      ctypes.c_void_p(decode_state["generated_tokens"].data_ptr()),
-                                     ctypes.c_void_p(self._result.data_ptr()), lg_ptr, ctypes.c_void_p(_stream_ptr())))
-    data = self._result.clone()
+                                     ctypes.c_void_p(data.data_ptr()), lg_ptr, ctypes.c_void_p(_stream_ptr())))
     token_logp = self._token_logp(lg, data[:, 0:1]) if self.config.return_log_prob else None   # maxengine.py:907-910 (idle slots: of their stale logits)
     result = engine_api.ResultTokens(data=data, tokens_idx=(0, 1), valid_idx=(1, 2), length_idx=(2, 3), log_prob=token_logp, samples_per_slot=1, check=self._result_check)
     return decode_state, result
