@@ -5,6 +5,7 @@
 #include "../../include/ixt_train.h"
 #include "ixt_kernels.h"
 #include "ixt_train_kernels.h"
+#include "ixt_train_attn.h"
 
 #include <hip/hip_runtime.h>
 #include <math.h>
@@ -62,11 +63,15 @@ struct ixt_trainer {
   std::vector<LayerAct> act;
   bf16_t *h_final = nullptr, *xn_f = nullptr, *rope_sin = nullptr, *rope_cos = nullptr;
   float* r_f = nullptr;
+  bool walk = false;        // attention by ixt_train_attn.h: heads of 64 or 128, rows of at most TA_MOST tokens, operands of a batch row and weights of a head within the reach of a 32-bit offset
+  long Sp;                  // columns between rows of P and dS: S, or whole tiles of 64, an odd number of them (walk)
+  int2* reach = nullptr;
   // workspaces
   float *scores = nullptr, *dh = nullptr, *dxn = nullptr, *logits = nullptr, *row_loss = nullptr, *scal = nullptr, *part = nullptr, *norm_part = nullptr;   // norm_part: [norms][blocks][E], rows of at most 1024 (rmsnorm_bwd)
   bf16_t *dS = nullptr, *d_ao = nullptr, *dq = nullptr, *dk = nullptr, *dv = nullptr, *dact = nullptr, *da = nullptr, *db = nullptr, *dlog = nullptr,
          *dy_bf = nullptr;
   float *dkf = nullptr, *dvf = nullptr;   // grouped-query attention: dK / dV summed over a group's query heads in f32 before they round to bf16
+  size_t scores_n = 0;
   std::vector<void*> allocs;
 };
 
@@ -125,25 +130,34 @@ extern "C" int ixt_train_create(const ixt_train_config* c, ixt_trainer** out) {
   auto fail = [&](int code) { ixt_train_destroy(t); return code; };
 #define A(expr) do { rc = (expr); if (rc != IXT_OK) return fail(rc); } while (0)
   const size_t T = t->T, S = t->S, BH = (size_t)t->B * t->H;
+  t->Sp = ((long)S + 63) / 64 * 64;
+  t->Sp += t->Sp / 64 % 2 == 0 ? 64 : 0;
+  t->walk = (t->D == 64 || t->D == 128) && S <= TA_MOST && S * (size_t)(QN > t->Sp ? QN : t->Sp) * 2 < (size_t)1 << 32;
+  if (!t->walk) t->Sp = S;
   A(tmalloc(t, &t->pb, (size_t)t->total + (size_t)E * (t->Vp - V)));
   t->act.resize(t->L);
   for (int i = 0; i < t->L; ++i) {
     LayerAct& a = t->act[i];
     A(tmalloc(t, &a.h_in, T * E)); A(tmalloc(t, &a.xn1, T * E)); A(tmalloc(t, &a.q, T * QN)); A(tmalloc(t, &a.k, T * KN)); A(tmalloc(t, &a.v, T * KN));
-    A(tmalloc(t, &a.P, BH * S * S)); A(tmalloc(t, &a.ao, T * QN)); A(tmalloc(t, &a.h_mid, T * E)); A(tmalloc(t, &a.xn2, T * E));
+    A(tmalloc(t, &a.P, BH * S * t->Sp)); A(tmalloc(t, &a.ao, T * QN)); A(tmalloc(t, &a.h_mid, T * E)); A(tmalloc(t, &a.xn2, T * E));
     A(tmalloc(t, &a.a, T * F)); A(tmalloc(t, &a.b, T * F)); A(tmalloc(t, &a.act, T * F)); A(tmalloc(t, &a.r1, T)); A(tmalloc(t, &a.r2, T));
   }
   A(tmalloc(t, &t->h_final, T * E)); A(tmalloc(t, &t->xn_f, T * E)); A(tmalloc(t, &t->r_f, T));
-  A(tmalloc(t, &t->scores, BH * S * S)); A(tmalloc(t, &t->dh, T * E)); A(tmalloc(t, &t->dxn, T * E));
+  // (behind the logits the scores hold the parts of a cut product, too)
+  t->scores_n = t->walk ? (V >= 65536 ? (size_t)4 * t->Tc * E : 0) : BH * S * S;
+  if (t->scores_n > 0) A(tmalloc(t, &t->scores, t->scores_n));
+  A(tmalloc(t, &t->dh, T * E)); A(tmalloc(t, &t->dxn, T * E));
   // (a chunk's logits are bf16, at the front of a buffer of f32 words that holds the parts of cut weight gradients later on)
   A(tmalloc(t, &t->logits, (size_t)t->Tc * V)); A(tmalloc(t, &t->dlog, (size_t)t->Tc * t->Vp)); A(tmalloc(t, &t->row_loss, T)); A(tmalloc(t, &t->scal, (size_t)16));
   A(tmalloc(t, &t->part, (size_t)4096));
   // The norms' scale gradients without atomics, for rows of at most 1024: at 2048 x 768 the atomics are 10 of a launch's 23 us, and the parts 39 MB for 25 norms.
   // 33 norms of 16384 x 2048 would take 277 MB for 13 of 145 us, 0.2 % of a step: wider rows keep the atomics, and with them last bits that vary from run to run.
   if (E <= 1024) A(tmalloc(t, &t->norm_part, (size_t)(2 * t->L + 1) * norm_blocks(t->T) * E));
-  A(tmalloc(t, &t->dS, BH * S * S)); A(tmalloc(t, &t->d_ao, T * QN)); A(tmalloc(t, &t->dq, T * QN)); A(tmalloc(t, &t->dk, T * KN));
+  A(tmalloc(t, &t->dS, BH * S * t->Sp));
+  if (t->walk) A(tmalloc(t, &t->reach, (size_t)t->B * 64));
+  A(tmalloc(t, &t->d_ao, T * QN)); A(tmalloc(t, &t->dq, T * QN)); A(tmalloc(t, &t->dk, T * KN));
   A(tmalloc(t, &t->dv, T * KN));
-  if (t->G > 1) { A(tmalloc(t, &t->dkf, T * KN)); A(tmalloc(t, &t->dvf, T * KN)); } A(tmalloc(t, &t->dact, T * F)); A(tmalloc(t, &t->da, T * F)); A(tmalloc(t, &t->db, T * F)); A(tmalloc(t, &t->dy_bf, T * E));
+  if (t->G > 1 && !t->walk) { A(tmalloc(t, &t->dkf, T * KN)); A(tmalloc(t, &t->dvf, T * KN)); } A(tmalloc(t, &t->dact, T * F)); A(tmalloc(t, &t->da, T * F)); A(tmalloc(t, &t->db, T * F)); A(tmalloc(t, &t->dy_bf, T * E));
 #undef A
   // RoPE tables: the same host recipe as the decode path (embeddings.py:270-307)
   {
@@ -232,6 +246,37 @@ static int attn_gemm(hipStream_t st, bool ta, bool tb, const bf16_t* A, long lda
   if (N > 64 && blocks(256, 128) >= 512) return ta ? gemm_launch<true, true, 256, 128>(st, g) : gemm_launch<false, true, 256, 128>(st, g);
   if (blocks(128, 64) >= 200) return ta ? gemm_launch<true, true, 128, 64>(st, g) : gemm_launch<false, true, 128, 64>(st, g);
   return ta ? gemm_launch<true, true, 64>(st, g) : gemm_launch<false, true, 64>(st, g);
+}
+// attention by walks (ixt_train_attn.h): forward, the queries' gradients, behind them the keys' and values'
+enum { TA_FWD, TA_DQ, TA_DKV };
+template <int D, int N>
+static int attn_back_t(hipStream_t st, const TAttn& a, int what) {
+  const int heads = a.B * (what == TA_DKV ? a.KVH : a.H);
+  const dim3 grid((unsigned)((heads + 7) / 8 * 8 * ((a.S + 64 * N - 1) / (64 * N))));
+  TCHK((lds_room<&k_t_attn_dq<D, N>>(TA_LDS(D, 4))));
+  TCHK((lds_room<&k_t_attn_dkv<D, N>>(TA_LDS_DKV(D, N))));
+  if (what == TA_DQ) hipLaunchKernelGGL((k_t_attn_dq<D, N>), grid, dim3(256), TA_LDS(D, 4), st, a);
+  else hipLaunchKernelGGL((k_t_attn_dkv<D, N>), grid, dim3(256), TA_LDS_DKV(D, N), st, a);
+  TLAUNCH();
+  return IXT_OK;
+}
+// Rows of at most 512 tokens: a wave holds its scores (48 heads of 64 x 512: 18.8 us; by three walks 32).
+template <int D>
+static int attn_forward_t(hipStream_t st, const TAttn& a) {
+  const dim3 grid((unsigned)((a.B * a.H + 7) / 8 * 8 * ((a.S + 63) / 64)));
+  TCHK((lds_room<&k_t_attn_fwd<D, true>>(TA_LDS(D, 4))));
+  if (a.S <= 64 * TA_HELD) hipLaunchKernelGGL((k_t_attn_fwd<D, true>), grid, dim3(256), TA_LDS(D, 4), st, a);
+  else hipLaunchKernelGGL((k_t_attn_fwd<D, false>), grid, dim3(256), TA_LDS(D, 3), st, a);
+  TLAUNCH();
+  return IXT_OK;
+}
+// Back: 32 rows a wave where that leaves two blocks a CU, 16 below (us queries' and keys' gradients, 32 / 16 rows: 192 blocks of 128 rows, heads of 64 24.2 14.2 / 19.2 11.9; 2048 blocks, heads of 128
+// 392 251 / 482 298; heads of 64, 1536 blocks 251 159 / 272 157)
+static int attn_walk(hipStream_t st, const TAttn& a, int D, int what) {
+  if (what == TA_FWD) return D == 64 ? attn_forward_t<64>(st, a) : attn_forward_t<128>(st, a);
+  const bool wide = (long)a.B * (what == TA_DKV ? a.KVH : a.H) * ((a.S + 127) / 128) >= 512;
+  if (D == 64) return wide ? attn_back_t<64, 2>(st, a, what) : attn_back_t<64, 1>(st, a, what);
+  return wide ? attn_back_t<128, 2>(st, a, what) : attn_back_t<128, 1>(st, a, what);
 }
 static void softmax_fwd(hipStream_t st, const float* scores, const int32_t* seg, bf16_t* P, int S, int B, int H) {
   const dim3 grid(S, B * H), waves((S + 3) / 4, B * H);
@@ -383,15 +428,21 @@ extern "C" int ixt_train_forward_backward(ixt_trainer* t, const int32_t* inputs,
     const ixt_trainer::LOff& o = t->lo[l];
     hipLaunchKernelGGL(k_t_rmsnorm_fwd, dim3(T), dim3(256), 0, st, a.h_in, pb + o.ln1, a.xn1, a.r1, E, eps);
     TTRY(gemm(st, TL_XW, T, E, {{a.xn1, pb + o.wq, a.q, QN}, {a.xn1, pb + o.wk, a.k, KN}, {a.xn1, pb + o.wv, a.v, KN}}, TG_BF16, E));
-    hipLaunchKernelGGL((k_t_rope<false>), EW((long)T * (H + KVH) * (D / 8)), a.q, a.k, positions, t->rope_sin, t->rope_cos, H, KVH, D, (long)T);
+    const auto rope = t->walk ? k_t_rope<false, true> : k_t_rope<false, false>;
+    hipLaunchKernelGGL(rope, EW((long)T * (H + KVH) * (D / 8)), a.q, a.k, positions, t->rope_sin, t->rope_cos, H, KVH, D, (long)T);
     // scores[b,h] = Q_h K_(h / G)^T (sm_scale 1: the query kernel carries 1/sqrt(d), attentions.py:1900-1904).  Grouped-query attention
     // (attentions.py:1206-1271: query heads reshaped to [kv heads, G]): query head kvh G + g of every kv head in launch g, batches (b, kvh).
-    const long SS = (long)S * S;
-    for (int g = 0; g < G; ++g)
-      TTRY(attn_gemm(st, false, false, a.q + (long)g * D, HD, a.k, KN, t->scores + g * SS, S, S, S, D, TG_F32, TC_LOWER, B, KVH, (long)S * HD, (long)G * D, (long)S * KN, D, H * SS, G * SS));
-    softmax_fwd(st, t->scores, segmentation, a.P, S, B, H);
-    for (int g = 0; g < G; ++g)
-      TTRY(attn_gemm(st, false, true, a.P + g * SS, S, a.v, KN, a.ao + (long)g * D, HD, S, D, S, TG_BF16, TC_K_TO_ROW, B, KVH, H * SS, G * SS, (long)S * KN, D, (long)S * HD, (long)G * D));
+    const TAttn ta{a.q, a.k, a.v, segmentation, a.P, a.ao, t->reach, t->d_ao, t->dS, t->dq, t->dk, t->dv, B, S, H, KVH, t->Sp};
+    if (t->walk) {
+      TTRY(attn_walk(st, ta, D, TA_FWD));
+    } else {
+      const long SS = (long)S * S;
+      for (int g = 0; g < G; ++g)
+        TTRY(attn_gemm(st, false, false, a.q + (long)g * D, HD, a.k, KN, t->scores + g * SS, S, S, S, D, TG_F32, TC_LOWER, B, KVH, (long)S * HD, (long)G * D, (long)S * KN, D, H * SS, G * SS));
+      softmax_fwd(st, t->scores, segmentation, a.P, S, B, H);
+      for (int g = 0; g < G; ++g)
+        TTRY(attn_gemm(st, false, true, a.P + g * SS, S, a.v, KN, a.ao + (long)g * D, HD, S, D, S, TG_BF16, TC_K_TO_ROW, B, KVH, H * SS, G * SS, (long)S * KN, D, (long)S * HD, (long)G * D));
+    }
     TTRY(gemm(st, TL_XW, T, QN, {{a.ao, pb + o.wo, a.h_mid, E}}, TG_BF16_RES, QN, 0, a.h_in));
     hipLaunchKernelGGL(k_t_rmsnorm_fwd, dim3(T), dim3(256), 0, st, a.h_mid, pb + o.ln2, a.xn2, a.r2, E, eps);
     TTRY(gemm(st, TL_XW, T, E, {{a.xn2, pb + o.wi0, a.a, F}, {a.xn2, pb + o.wi1, a.b, F}}, TG_BF16, E));
@@ -408,7 +459,7 @@ extern "C" int ixt_train_forward_backward(ixt_trainer* t, const int32_t* inputs,
     TTRY(gemm(st, TL_XW, n, E, {{xn, pb + t->o_logits, t->logits, V, t->Vp}}, TG_BF16, E));
     TTRY(xent(st, reinterpret_cast<const bf16_t*>(t->logits), targets + t0, targets_segmentation + t0, t->dlog, t->row_loss + t0, n, V, t->Vp));
     // d xn_f = dlogits . W^T ; dW += xn_f^T . dlogits
-    TTRY(gemm(st, TL_DX, n, V, {{t->dlog, pb + t->o_logits, t->dxn + (long)t0 * E, V, t->Vp}}, TG_F32, t->Vp, E, nullptr, t->scores, V >= 65536 ? (size_t)B * H * S * S : 0));   // (the score buffer is idle)
+    TTRY(gemm(st, TL_DX, n, V, {{t->dlog, pb + t->o_logits, t->dxn + (long)t0 * E, V, t->Vp}}, TG_F32, t->Vp, E, nullptr, t->scores, V >= 65536 ? t->scores_n : 0));   // (the score buffer is idle)
     TTRY(gemm(st, TL_DW, E, n, {{xn, t->dlog, t->g + t->o_logits, V, t->Vp}}, t0 == 0 ? TG_F32 : TG_F32_ADD, E));
   }
   hipLaunchKernelGGL(k_t_reduce, dim3(1), dim3(256), 0, st, t->row_loss, (long)T, 0, loss_and_weights_dev, 0);
@@ -435,31 +486,38 @@ extern "C" int ixt_train_forward_backward(ixt_trainer* t, const int32_t* inputs,
     // attention: h_mid = h_in + out(ao)
     TTRY(gemm(st, TL_DX, T, E, {{t->dy_bf, pb + o.wo, t->d_ao, E}}, TG_BF16, E, QN));                    // d ao = dy . Wo^T
     TTRY(gemm(st, TL_DW, QN, T, {{a.ao, t->dy_bf, t->g + o.wo, E}}, TG_F32, QN, 0, nullptr, spare, spare_n));   // d Wo = ao^T . dy
-    // dP = d_ao V^T (f32) ; dV = P^T d_ao ; dS = P o (dP - rowsum(dP o P)) ; dQ = dS K ; dK = dS^T Q.  With G query heads per kv head, dV and dK
-    // are the sums over the group: accumulated in f32 over the G launches, rounded to bf16 once.
-    const long SS = (long)S * S;
-    for (int g = 0; g < G; ++g)
-      TTRY(attn_gemm(st, false, false, t->d_ao + (long)g * D, HD, a.v, KN, t->scores + g * SS, S, S, S, D, TG_F32, TC_LOWER, B, KVH, (long)S * HD, (long)G * D, (long)S * KN, D, H * SS, G * SS));
-    if (G == 1) {
-      TTRY(attn_gemm(st, true, true, a.P, S, t->d_ao, HD, t->dv, HD, S, D, S, TG_BF16, TC_K_FROM_ROW, B, H, H * SS, SS, (long)S * HD, D, (long)S * HD, D));
+    if (t->walk) {
+      const TAttn ta{a.q, a.k, a.v, segmentation, a.P, a.ao, t->reach, t->d_ao, t->dS, t->dq, t->dk, t->dv, B, S, H, KVH, t->Sp};
+      TTRY(attn_walk(st, ta, D, TA_DQ));
+      TTRY(attn_walk(st, ta, D, TA_DKV));
     } else {
+      // dP = d_ao V^T (f32) ; dV = P^T d_ao ; dS = P o (dP - rowsum(dP o P)) ; dQ = dS K ; dK = dS^T Q.  With G query heads per kv head, dV and dK
+      // are the sums over the group: accumulated in f32 over the G launches, rounded to bf16 once.
+      const long SS = (long)S * S;
       for (int g = 0; g < G; ++g)
-        TTRY(attn_gemm(st, true, true, a.P + g * SS, S, t->d_ao + (long)g * D, HD, t->dvf, KN, S, D, S, g > 0 ? TG_F32_ADD : TG_F32, TC_K_FROM_ROW, B, KVH, H * SS, G * SS, (long)S * HD,
-                       (long)G * D, (long)S * KN, D));
-      hipLaunchKernelGGL(k_t_f32_to_bf16, EW((long)T * KN / 8), t->dvf, t->dv, (long)T * KN);
-    }
-    softmax_bwd(st, t->scores, a.P, t->dS, S, B * H);
-    for (int g = 0; g < G; ++g)
-      TTRY(attn_gemm(st, false, true, t->dS + g * SS, S, a.k, KN, t->dq + (long)g * D, HD, S, D, S, TG_BF16, TC_K_TO_ROW, B, KVH, H * SS, G * SS, (long)S * KN, D, (long)S * HD, (long)G * D));
-    if (G == 1) {
-      TTRY(attn_gemm(st, true, true, t->dS, S, a.q, HD, t->dk, HD, S, D, S, TG_BF16, TC_K_FROM_ROW, B, H, H * SS, SS, (long)S * HD, D, (long)S * HD, D));
-    } else {
+        TTRY(attn_gemm(st, false, false, t->d_ao + (long)g * D, HD, a.v, KN, t->scores + g * SS, S, S, S, D, TG_F32, TC_LOWER, B, KVH, (long)S * HD, (long)G * D, (long)S * KN, D, H * SS, G * SS));
+      if (G == 1) {
+        TTRY(attn_gemm(st, true, true, a.P, S, t->d_ao, HD, t->dv, HD, S, D, S, TG_BF16, TC_K_FROM_ROW, B, H, H * SS, SS, (long)S * HD, D, (long)S * HD, D));
+      } else {
+        for (int g = 0; g < G; ++g)
+          TTRY(attn_gemm(st, true, true, a.P + g * SS, S, t->d_ao + (long)g * D, HD, t->dvf, KN, S, D, S, g > 0 ? TG_F32_ADD : TG_F32, TC_K_FROM_ROW, B, KVH, H * SS, G * SS, (long)S * HD,
+                         (long)G * D, (long)S * KN, D));
+        hipLaunchKernelGGL(k_t_f32_to_bf16, EW((long)T * KN / 8), t->dvf, t->dv, (long)T * KN);
+      }
+      softmax_bwd(st, t->scores, a.P, t->dS, S, B * H);
       for (int g = 0; g < G; ++g)
-        TTRY(attn_gemm(st, true, true, t->dS + g * SS, S, a.q + (long)g * D, HD, t->dkf, KN, S, D, S, g > 0 ? TG_F32_ADD : TG_F32, TC_K_FROM_ROW, B, KVH, H * SS, G * SS, (long)S * HD,
-                       (long)G * D, (long)S * KN, D));
-      hipLaunchKernelGGL(k_t_f32_to_bf16, EW((long)T * KN / 8), t->dkf, t->dk, (long)T * KN);
+        TTRY(attn_gemm(st, false, true, t->dS + g * SS, S, a.k, KN, t->dq + (long)g * D, HD, S, D, S, TG_BF16, TC_K_TO_ROW, B, KVH, H * SS, G * SS, (long)S * KN, D, (long)S * HD, (long)G * D));
+      if (G == 1) {
+        TTRY(attn_gemm(st, true, true, t->dS, S, a.q, HD, t->dk, HD, S, D, S, TG_BF16, TC_K_FROM_ROW, B, H, H * SS, SS, (long)S * HD, D, (long)S * HD, D));
+      } else {
+        for (int g = 0; g < G; ++g)
+          TTRY(attn_gemm(st, true, true, t->dS + g * SS, S, a.q + (long)g * D, HD, t->dkf, KN, S, D, S, g > 0 ? TG_F32_ADD : TG_F32, TC_K_FROM_ROW, B, KVH, H * SS, G * SS, (long)S * HD,
+                         (long)G * D, (long)S * KN, D));
+        hipLaunchKernelGGL(k_t_f32_to_bf16, EW((long)T * KN / 8), t->dkf, t->dk, (long)T * KN);
+      }
     }
-    hipLaunchKernelGGL((k_t_rope<true>), EW((long)T * (H + KVH) * (D / 8)), t->dq, t->dk, positions, t->rope_sin, t->rope_cos, H, KVH, D, (long)T);
+    const auto rope = t->walk ? k_t_rope<true, true> : k_t_rope<true, false>;
+    hipLaunchKernelGGL(rope, EW((long)T * (H + KVH) * (D / 8)), t->dq, t->dk, positions, t->rope_sin, t->rope_cos, H, KVH, D, (long)T);
     // d xn1 = dq Wq^T + dk Wk^T + dv Wv^T
     TTRY(gemm(st, TL_DX, T, QN, {{t->dq, pb + o.wq, t->dxn, QN}, {t->dk, pb + o.wk, t->dxn, KN}, {t->dv, pb + o.wv, t->dxn, KN}}, TG_F32, QN, E, nullptr, spare, spare_n));
     TTRY(gemm(st, TL_DW, E, T, {{a.xn1, t->dq, t->g + o.wq, QN}, {a.xn1, t->dk, t->g + o.wk, KN}, {a.xn1, t->dv, t->g + o.wv, KN}}, TG_F32, E, 0, nullptr, spare, spare_n));

@@ -188,9 +188,13 @@ static __global__ void k_t_sum_parts(const float* __restrict__ parts, int nparts
   *reinterpret_cast<float4*>(out + i) = t;
 }
 
+// Where the walks over keys (ixt_train_attn.h) have features i .. i + 3 of a head, i a multiple of 4: of every 32 the runs of four 0, 4, 1, 5, 2, 6, 3, 7, so that a lane's 16 bytes are the
+// two runs that a product of k_tgemm puts on it.
+__device__ __forceinline__ int ta_place4(int i) { return (i & ~31) + ((i >> 2 & 3) << 3) + (i >> 4 & 1) * 4; }
 // RoPE (embeddings.py:277-315) on q bf16 [T][H][D] and k [T][KVH][D] with per-token positions; INV: the transposed rotation (backward).  A thread turns
-// four pairs (D % 8 == 0).  grid = ceil(T (H + KVH) (D / 8) / 256), block 256.
-template <bool INV>
+// four pairs (D % 8 == 0).  RUNS (heads of 64 and 128): features in the order of ta_place4 on the attention's side; a head's threads are lanes of one wave, whose loads stand in front of its
+// stores.  grid = ceil(T (H + KVH) (D / 8) / 256), block 256.
+template <bool INV, bool RUNS>
 __global__ void k_t_rope(bf16_t* __restrict__ q, bf16_t* __restrict__ k, const int32_t* __restrict__ pos, const bf16_t* __restrict__ sn, const bf16_t* __restrict__ cs, int H, int KVH,
                          int D, long T) {
   const int quads = D / 8, half = D / 2;
@@ -198,9 +202,11 @@ __global__ void k_t_rope(bf16_t* __restrict__ q, bf16_t* __restrict__ k, const i
   const long t = id / ((H + KVH) * quads);
   if (t >= T) return;
   const int in = (int)(id - t * ((H + KVH) * quads)), h = in / quads, i = (in - h * quads) * 4;
-  bf16_t* p = (h < H ? q + (t * H + h) * D : k + (t * KVH + h - H) * D) + i;
+  bf16_t* const head = h < H ? q + (t * H + h) * D : k + (t * KVH + h - H) * D;
+  const bf16_t* const from = head + (RUNS && INV ? ta_place4(i) : i);
+  bf16_t* const to = head + (RUNS && !INV ? ta_place4(i) : i);
   const long at = (long)pos[t] * half + i;
-  const uint2 a = *reinterpret_cast<const uint2*>(p), b = *reinterpret_cast<const uint2*>(p + half), sw = *reinterpret_cast<const uint2*>(sn + at), cw = *reinterpret_cast<const uint2*>(cs + at);
+  const uint2 a = *reinterpret_cast<const uint2*>(from), b = *reinterpret_cast<const uint2*>(from + half), sw = *reinterpret_cast<const uint2*>(sn + at), cw = *reinterpret_cast<const uint2*>(cs + at);
   const float x1[4] = {bflo(a.x), bfhi(a.x), bflo(a.y), bfhi(a.y)}, x2[4] = {bflo(b.x), bfhi(b.x), bflo(b.y), bfhi(b.y)};
   const float s[4] = {bflo(sw.x), bfhi(sw.x), bflo(sw.y), bfhi(sw.y)}, c[4] = {bflo(cw.x), bfhi(cw.x), bflo(cw.y), bfhi(cw.y)};
   bf16_t u[4], v[4];
@@ -209,8 +215,9 @@ __global__ void k_t_rope(bf16_t* __restrict__ q, bf16_t* __restrict__ k, const i
     if (!INV) { u[j] = f2bf(rbf(x1[j] * c[j]) - rbf(x2[j] * s[j])); v[j] = f2bf(rbf(x2[j] * c[j]) + rbf(x1[j] * s[j])); }
     else { u[j] = f2bf(x1[j] * c[j] + x2[j] * s[j]); v[j] = f2bf(x2[j] * c[j] - x1[j] * s[j]); }
   }
-  *reinterpret_cast<uint2*>(p) = make_uint2(pack2(u[0], u[1]), pack2(u[2], u[3]));
-  *reinterpret_cast<uint2*>(p + half) = make_uint2(pack2(v[0], v[1]), pack2(v[2], v[3]));
+  if constexpr (RUNS) wave_lds_sync();                     // (orders the compiler; the hardware has the wave's loads in front of its stores anyway)
+  *reinterpret_cast<uint2*>(to) = make_uint2(pack2(u[0], u[1]), pack2(u[2], u[3]));
+  *reinterpret_cast<uint2*>(to + half) = make_uint2(pack2(v[0], v[1]), pack2(v[2], v[3]));
 }
 
 // Attention softmax over scores f32 [BH][S][S] with the train-mode mask (attentions.py:586-618: same segment AND col <= row), P bf16 out.  Columns up to
