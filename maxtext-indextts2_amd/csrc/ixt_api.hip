@@ -374,7 +374,7 @@ extern "C" int ixt_create(const ixt_config* cfg, ixt_ctx** out) {
   A(dmalloc(x, &x->row_pos, (size_t)R));
   A(dmalloc(x, &x->row_active, (size_t)R));
   A(dmalloc(x, &x->row_tok, (size_t)R));
-  A(dmalloc(x, &x->new_tok, (size_t)R));
+  A(dmalloc(x, &x->new_tok, (size_t)R)); A(dmalloc(x, &x->row_order, (size_t)R));
   A(dmalloc(x, &x->lrows, (size_t)x->NLmax));
   A(dmalloc(x, &x->kptrs_d, (size_t)L));
   A(dmalloc(x, &x->vptrs_d, (size_t)L));
@@ -1211,6 +1211,8 @@ static void launch_scores_pv(ixt_ctx* c, int layer, int R, int len_hint, hipStre
   hipLaunchKernelGGL((k_attn_pv<HD, GQ>), dim3(R, g.nkv, nchunk), dim3(256), lds, st, pa);
 }
 
+// Decode rows of so many blocks (two on a CU) go longest first: k_decode_front leaves their order.  With fewer there is one wave of blocks or less than one, and no order is better than another.
+static bool attn_in_order(const ixt_ctx* c, int R) { return (long)R * c->geom.nkv >= 512; }
 template <int HD, int GQ>
 static void launch_decode_attn(ixt_ctx* c, int layer, int R, const DotResult& dr, bool newtok, bool decode, hipStream_t st) {
   const AttnGeom& g = c->geom;
@@ -1229,7 +1231,8 @@ static void launch_decode_attn(ixt_ctx* c, int layer, int R, const DotResult& dr
   const size_t lds = sizeof(float) * ((size_t)GQ * HD + 2 * HD + (size_t)GQ * ((g.Tmax + 3) & ~3) + ((g.mpg + 3) & ~3) + 8 + (size_t)g.nsb_max * HD);
   // streamed past the caches where the launch is bound by the memory's rate: with fewer blocks its latency counts, and that is longer (10.7 -> 12.1 us for 16 blocks,
   // 3 % of a step at 384 blocks of 12 heads)
-  const bool once = decode && (long)R * g.nkv >= 512;
+  const bool once = decode && attn_in_order(c, R);
+  if (once) da.row_order = c->row_order;
   if (newtok && once) hipLaunchKernelGGL((k_attn_decode<HD, GQ, true, true>), dim3(g.nkv, R), dim3(256), lds, st, da);
   else if (newtok) hipLaunchKernelGGL((k_attn_decode<HD, GQ, true, false>), dim3(g.nkv, R), dim3(256), lds, st, da);
   else if (once) hipLaunchKernelGGL((k_attn_decode<HD, GQ, false, true>), dim3(g.nkv, R), dim3(256), lds, st, da);
@@ -2092,7 +2095,7 @@ static int decode_rows(ixt_ctx* c, const int32_t* tokens_dev, const int32_t* pos
   const bool step = plain && small_path_ok(c, c->B) && takes_step(c, c->B, true), mid = plain && !small_path_ok(c, c->B) && takes_mid(c, c->B);
   const FrontRows f = step ? step_front(c) : mid ? mid_front(c) : FrontRows{};
   hipLaunchKernelGGL(k_decode_front, dim3(step || mid ? 1 + c->B : 1), dim3(256), 0, st, c->ps, advance ? 1 : 0, c->row_slot, c->row_pos, c->row_active, c->row_tok, tokens_dev, pos_dev, c->Tmax, c->B, f,
-                     c->gave);
+                     c->gave, attn_in_order(c, c->B) ? c->row_order : nullptr);
   LAUNCHCHK();
   return forward_rows(c, c->B, step || mid ? nullptr : c->row_tok, c->Tmax, 0, c->B, nullptr, next_tokens_dev, logits_dev, true, st);
 }
