@@ -732,28 +732,30 @@ static void timing_end(ixt_ctx* c, hipStream_t st, int idx) {
 // --------------------------------------------------------------------------------------- LDS-ring GEMM (ixt_gemm.h)
 // Tiles (rows x columns): 1 = 128 x 128 (8 waves as 2 x 4, 4 slots of 32 KiB), 2 = 128 x 64 (8 waves, 5 x 24 KiB), 3 = 64 x 32 (4 waves, 6 x 24 KiB,
 // 128-k chunks), 4 = 256 x 128 (8 waves of 64 x 64, 3 x 48 KiB), 5 = 64 x 64 (4 waves, 4 x 16 KiB: two blocks share a CU), 6 = 64 x 16 (4 waves, 6 x 20 KiB,
-// 128-k chunks), 7 = 128 x 128 with 32-k chunks (4 x 16 KiB, two blocks share a CU).
+// 128-k chunks), 7 = 128 x 128 with 32-k chunks (4 x 16 KiB, two blocks share a CU), 8 = 128 x 192 (8 waves of 64 x 48, 3 x 40 KiB; not for gate pairs, an even number of a wave's column tiles).
 //
 // A launch takes as many rounds as its fullest XCD has blocks for its 32 CUs, and a round of one tile takes the same time whatever the sizes: what one 64-k
 // chunk takes, in units of 10 ns, measured on 9 numbers of rows (128 .. 2048) x 8 projections (K 2048 .. 9216, N 2048 .. 18432) -- tile 4: 100, 1: 62, 2: 44,
 // 5: 31 (52 for two blocks of a CU), 3: 22, 6: 19, 7: 66 (122 for two).  The least estimate is within 6 % of the fastest tile on all but 3 of these 72
 // (within 12 %); the rule that looked at the number of 128 x 128 tiles alone took 62 us where this takes 40 (256 x 2304 outputs, K 9216) and 122 where this
-// takes 102 (1525 x 14336, K 2048).
+// takes 102 (1525 x 14336, K 2048).  Tile 8 (90) came later: what 256 x 128 leaves on a part of the CUs fills them all (6144 outputs, K 2048: 1024 rows 192 tiles -> 256, QKV 41.0 -> 34.7 us, 828 rows 41.1 -> 33.0;
+// 1592 rows, 2 rounds of 52 a XCD against tile 7's 78: 64.0 and 62.4).  192 x 128, whose odd row block of a wave is stored by itself: QKV 63.9 for 1592 rows, gated units 104.9 against 100.9, not taken.
 // These are the times of the products' former loops.  With the present ones a chunk takes 60, 45, 31, 21, 14, 13 and 43 (73 for two of tile 7, 32 of tile 5), and a round 230 to 660 beside its
 // chunks, which no single figure a tile stands for: by the figures below the tile is 1.4 % off the fastest in the geometric mean of such launches, by a rule of two figures a tile 0.8 %.
 static int ring_pick(const ixt_ctx* c, int epi, int R, int N, bool routed, bool wring) {
-  if (c->ring_cfg >= 1 && c->ring_cfg <= 7 && !(epi == GEPI_SWIGLU && (c->ring_cfg == 3 || c->ring_cfg == 6)) && !(epi == GEPI_UNEMBED && c->ring_cfg != 1) && !(routed && c->ring_cfg == 4) &&
-      !(wring && c->ring_cfg == 7)) return c->ring_cfg;
+  if (c->ring_cfg >= 1 && c->ring_cfg <= 8 && !(epi == GEPI_SWIGLU && (c->ring_cfg == 3 || c->ring_cfg == 6 || c->ring_cfg == 8)) && !(epi == GEPI_UNEMBED && c->ring_cfg != 1) &&
+      !(routed && c->ring_cfg == 4) && !(wring && c->ring_cfg >= 7)) return c->ring_cfg;
   if (routed) {   // every expert's rows are one or two groups of 128, whatever the launch's total: the blocks that have work are not known here
     const long b1 = (long)((N + 127) / 128) * ((R + 127) / 128), b2 = (long)((N + 63) / 64) * ((R + 127) / 128);
     return b1 >= 192 ? 1 : b2 >= 160 || epi == GEPI_SWIGLU ? 2 : 3;
   }
-  static const struct { int id, rows, cols, one, two; } tiles[] = {{4, 256, 128, 100, 0}, {7, 128, 128, 66, 122}, {1, 128, 128, 62, 0}, {2, 128, 64, 44, 0},
+  static const struct { int id, rows, cols, one, two; } tiles[] = {{4, 256, 128, 100, 0}, {8, 128, 192, 90, 0}, {7, 128, 128, 66, 122}, {1, 128, 128, 62, 0}, {2, 128, 64, 44, 0},
                                                                     {5, 64, 64, 31, 52},  {3, 64, 32, 22, 0},     {6, 64, 16, 19, 0}};
   int best = 1;
   long least = -1;
   for (const auto& t : tiles) {
     if ((epi == GEPI_SWIGLU && t.cols < 64) || (epi == GEPI_UNEMBED && t.cols < 64)) continue;   // gate pairs are two column tiles of a wave; few waves a row for the sampling
+    if (t.id == 8 && (epi == GEPI_SWIGLU || epi == GEPI_UNEMBED || wring)) continue;
     if ((t.id == 7 && (!c->ring_two_per_cu || wring)) || (t.id == 4 && epi == GEPI_UNEMBED && !c->unembed_tall)) continue;
     const long per_xcd = (long)(((N + t.cols - 1) / t.cols + 7) / 8) * ((R + t.rows - 1) / t.rows);
     long cost;
@@ -838,6 +840,7 @@ int launch_ring(ixt_ctx* c, int epi, const bf16_t* x, const bf16_t* w, int K, in
     case 2: rc = RING_T(2, 4, 4, 1, 2, 5, EPI_, 0); break;                 \
     case 3: rc = RING_T(2, 2, 2, 1, 4, 6, EPI_, 0); break;                 \
     case 6: rc = RING_T(4, 1, 1, 1, 4, 6, EPI_, 0); break;                 \
+    case 8: rc = RING_T(2, 4, 4, 3, 2, 3, EPI_, 0); break;                 \
   }
 #define RING_PAIRS(EPI_)                                                   \
   switch (cfg) {                                                           \
