@@ -128,7 +128,8 @@ __global__ __launch_bounds__(512, 2) void k_attn_mscores(TileAttnArgs a) {
 // Buffers of the exchange: with two a round has one barrier (another one's sums are read while the next is written); one where there is one round, or where two
 // would take a CU's second block away.
 constexpr int mtile_buffers(int hd, int nw, int nr) { return nr > 1 && (nw == 8 || hd <= 128) ? 2 : 1; }
-constexpr size_t mtile_lds(int hd, int nw, int nr) { return (size_t)mtile_buffers(hd, nw, nr) * nw * 16 * ((hd >= 128 ? 128 : hd) + 4) * 4; }
+constexpr int mtile_width(int hd) { return hd >= 128 ? 128 : hd; }        // value columns of one output pass
+constexpr size_t mtile_lds(int hd, int nw, int nr, int vw) { return (size_t)mtile_buffers(hd, nw, nr) * nw * 16 * (vw + 4) * 4; }
 // block = (kv head, 16 query vectors = 16 / GQ consecutive rows x GQ heads), NW waves.  Super-block (4 pages, 128 keys) n NW + w belongs to wave w in
 // round n; its 128 x 16 scores stay in that wave's registers from the score products to the output products, so the keys one block holds are
 // 128 NW NR and nothing of them goes through LDS or memory.
@@ -159,14 +160,13 @@ constexpr size_t mtile_lds(int hd, int nw, int nr) { return (size_t)mtile_buffer
 // 92 / 212 / 310, now 87 / 198 / 293.  828 rows at <= 3900 keys 1496, 408, 375 us (63 TFLOP/s).  8 heads of 256 on 4, 256 rows at <= 1756 / 2756 keys: 88 / 131, 79 / 117 us.
 // Prompts of <= 256 keys: two waves per block; with four, two of them had nothing to do (eight packed ones, 1525 rows: 90.2 us against 67.6).
 // GIVEN: the scores are in memory (k_attn_mscores, the same rows)
-template <int HD, int GQ, int NW, int NR, bool GIVEN = false>
+template <int HD, int GQ, int NW, int NR, bool GIVEN = false, int VW = mtile_width(HD)>
 __global__ __launch_bounds__(NW * 64, NR == 1 && NW <= 4 ? 3 : 2) void k_attn_mtile(TileAttnArgs a) {
   constexpr int TQ = 16 / GQ;
-  constexpr int VW = HD >= 128 ? 128 : HD;     // value columns of one output pass
   constexpr int NE = VW / 16;                  // matrix tiles of them
   constexpr int OP = VW + 4, NTOT = 16 * VW / (NW * 64);       // a vector's pitch of the exchange; (vector, column) totals per thread
   constexpr int NBUF = mtile_buffers(HD, NW, NR);
-  static_assert(16 % GQ == 0 && HD % 64 == 0 && (HD <= 128 || HD % 128 == 0), "tile geometry");
+  static_assert(16 % GQ == 0 && HD % VW == 0 && VW % 64 == 0 && VW <= 128, "tile geometry");
   constexpr int QP = HD + 4;                                             // a vector's pitch: 16 lanes read 16 bytes of 16 vectors without a bank conflict
   __shared__ __attribute__((aligned(16))) float qs[16 * QP];
   __shared__ float psum[NW * NR * 4 * 16];                               // [page][vector]
