@@ -71,7 +71,7 @@ struct HybridModel {
   void* scan_t = nullptr;                        // the operand of a scan's third projection
   float *part3 = nullptr, *scan_u = nullptr, *scan_sum = nullptr;
   size_t part3_floats = 0;
-  void *xb = nullptr, *act = nullptr, *hact = nullptr, *xn = nullptr, *qx = nullptr, *qr = nullptr, *olat = nullptr, *xg = nullptr, *mhact = nullptr;
+  void *xb = nullptr, *act = nullptr, *hact = nullptr, *xn = nullptr, *qx = nullptr, *qr = nullptr, *olat = nullptr, *xg = nullptr, *mhact = nullptr, *lowx = nullptr;
   float *dq = nullptr, *dk = nullptr, *dkq = nullptr, *dv = nullptr, *dec = nullptr, *beta = nullptr, *dout = nullptr, *mw = nullptr, *msum = nullptr, *po = nullptr, *pml = nullptr, *ret_u = nullptr, *sgate = nullptr;
   int32_t *midx = nullptr, *mpos = nullptr, *mrb = nullptr;
   int moe_cap = 0;

@@ -681,7 +681,7 @@ int hybrid_init(ixt_ctx* c) {
   TRY(h_allocf(c, &m->ret_u, ret_u + 4)); TRY(h_allocf(c, &m->chunk, max_chunks)); TRY(h_allocf(c, &m->sgate, (size_t)R + 4));
   TRY(h_alloc(c, &m->xb, (size_t)Rp * m->Ep * m->esz));
   TRY(h_alloc(c, &m->act, (size_t)Rp * act_k * m->esz));
-  TRY(h_alloc(c, &m->hact, (size_t)Rp * (hact_k + 8) * m->esz));
+  TRY(h_alloc(c, &m->hact, (size_t)Rp * (hact_k + 8) * m->esz)); TRY(h_alloc(c, &m->lowx, (size_t)16 * DELTA_LOW_K * m->esz));
   TRY(h_alloc(c, &m->xn, (size_t)up_to(c->NLmax, 128) * m->Ep * m->esz));
   TRY(h_alloc(c, &m->qx, (qx_e + 8) * m->esz)); TRY(h_alloc(c, &m->qr, (qr_e + 8) * m->esz)); TRY(h_alloc(c, &m->olat, (olat_e + 8) * m->esz));
   TRY(h_alloc(c, &m->xg, (xg_e + 8) * m->esz)); TRY(h_alloc(c, &m->mhact, (mh_e + 8) * m->esz));
@@ -1046,19 +1046,25 @@ static int hybrid_mixer_delta(ixt_ctx* c, const HLayer& L, const HLayer& W, int 
   HybridModel* m = c->hy;
   const DeltaGeom& g = L.dg;
   Slices t, t2;
+  // a token a row and few rows: the low-rank columns' own product is k_delta_step's, whose blocks write m->act while others still read its operand
+  const bool inside = sizeof(T) == 2 && single && R <= 16 && W.low.Kp <= DELTA_LOW_K && g.d % 16 == 0 && g.dv % 16 == 0;
+  T* const lowx = (T*)(inside ? m->lowx : m->act);
   SdotSide low;                                                    // the low-rank columns as an operand: by the product itself, or a launch behind it
-  if constexpr (sizeof(T) == 2) low = SdotSide{(bf16_t*)m->act, g.oa, g.ra, g.og, g.rg, W.low.Kp};
+  if constexpr (sizeof(T) == 2) low = SdotSide{lowx, g.oa, g.ra, g.og, g.rg, W.low.Kp};
   TRY(hdot<T>(c, (const T*)m->xb, W.in, R, c->part, c->part_floats, st, &t, &low));
   if (low.x == nullptr) {
-    hipLaunchKernelGGL((k_lowrank_x<T>), dim3(R), dim3(128), 0, st, t, g, (T*)m->act, W.low.Kp);
+    hipLaunchKernelGGL((k_lowrank_x<T>), dim3(R), dim3(128), 0, st, t, g, lowx, W.low.Kp);
     LAUNCHCHK();
   }
-  TRY(hdot<T>(c, (const T*)m->act, W.low, R, m->part2, m->part2_floats, st, &t2));
+  if (!inside) TRY(hdot<T>(c, (const T*)m->act, W.low, R, m->part2, m->part2_floats, st, &t2));
   if (single) {            // every row is a segment of one token
-    DeltaStepArgs da{t, t2, g, W.cq, W.ck, W.cv, W.a_log, W.dt_bias, W.onorm, m->eps, c->row_active, c->row_slot, c->row_pos, m->parity, L.tails, L.state};
-    const dim3 grid(R, g.H);
-    const size_t lds = sizeof(float) * (3 * g.dp + 2 * g.dv);
-#define HSTEP(RP_) case RP_: hipLaunchKernelGGL((k_delta_step<T, RP_>), grid, dim3(256), lds, st, da, (T*)m->act, W.o.Kp); break
+    DeltaStepArgs da{t, t2, g, W.cq, W.ck, W.cv, W.a_log, W.dt_bias, W.onorm, m->eps, c->row_active, c->row_slot, c->row_pos, m->parity, L.tails, L.state,
+                     (const u32x4*)lowx, (const u32x4*)W.low.w, W.low.Kp};
+    const dim3 grid(g.H, R);
+    const size_t lds = sizeof(float) * (3 * g.dp + 2 * g.dv + (inside ? g.d + g.dv : 0));
+#define HSTEP(RP_) case RP_: \
+    if constexpr (sizeof(T) == 2) if (inside) { hipLaunchKernelGGL((k_delta_step<T, RP_, true>), grid, dim3(512), lds, st, da, (T*)m->act, W.o.Kp); break; } \
+    hipLaunchKernelGGL((k_delta_step<T, RP_, false>), grid, dim3(512), lds, st, da, (T*)m->act, W.o.Kp); break
     switch (g.dp / 16) { HSTEP(1); HSTEP(2); HSTEP(4); HSTEP(8); HSTEP(16); HSTEP(32); default: return set_err(IXT_ERR_UNSUPPORTED, "delta rule: %d key dims", g.d); }
 #undef HSTEP
     LAUNCHCHK();
