@@ -1214,8 +1214,8 @@ static void launch_scores_pv(ixt_ctx* c, int layer, int R, int len_hint, hipStre
   hipLaunchKernelGGL((k_attn_pv<HD, GQ>), dim3(R, g.nkv, nchunk), dim3(256), lds, st, pa);
 }
 
-// Decode rows of so many blocks (two on a CU) go longest first: k_decode_front leaves their order.  With fewer there is one wave of blocks or less than one, and no order is better than another.
-static bool attn_in_order(const ixt_ctx* c, int R) { return (long)R * c->geom.nkv >= 512; }
+// Decode rows of two to eight blocks a CU go longest first: k_decode_front leaves their order.  (k_attn_decode has both sides' figures; with fewer blocks there is one a CU or less, and no order.)
+static bool attn_in_order(const ixt_ctx* c, int R) { return (long)R * c->geom.nkv >= 512 && (long)R * c->geom.nkv <= 2048; }
 template <int HD, int GQ>
 static void launch_decode_attn(ixt_ctx* c, int layer, int R, const DotResult& dr, bool newtok, bool decode, hipStream_t st) {
   const AttnGeom& g = c->geom;
@@ -1234,12 +1234,14 @@ static void launch_decode_attn(ixt_ctx* c, int layer, int R, const DotResult& dr
   const size_t lds = sizeof(float) * ((size_t)GQ * HD + 2 * HD + (size_t)GQ * ((g.Tmax + 3) & ~3) + ((g.mpg + 3) & ~3) + 8 + (size_t)g.nsb_max * HD);
   // streamed past the caches where the launch is bound by the memory's rate: with fewer blocks its latency counts, and that is longer (10.7 -> 12.1 us for 16 blocks,
   // 3 % of a step at 384 blocks of 12 heads)
-  const bool once = decode && attn_in_order(c, R);
-  if (once) da.row_order = c->row_order;
-  if (newtok && once) hipLaunchKernelGGL((k_attn_decode<HD, GQ, true, true>), dim3(g.nkv, R), dim3(256), lds, st, da);
-  else if (newtok) hipLaunchKernelGGL((k_attn_decode<HD, GQ, true, false>), dim3(g.nkv, R), dim3(256), lds, st, da);
-  else if (once) hipLaunchKernelGGL((k_attn_decode<HD, GQ, false, true>), dim3(g.nkv, R), dim3(256), lds, st, da);
-  else hipLaunchKernelGGL((k_attn_decode<HD, GQ, false, false>), dim3(g.nkv, R), dim3(256), lds, st, da);
+  const bool once = decode && (long)R * g.nkv >= 512;
+  da.row_order = c->row_order;
+#define ATT(NEW_, ONCE_, ORD_) hipLaunchKernelGGL((k_attn_decode<HD, GQ, NEW_, ONCE_, ORD_>), dim3(g.nkv, R), dim3(256), lds, st, da)
+  if (decode && attn_in_order(c, R)) { if (newtok) ATT(true, true, true); else ATT(false, true, true); }
+  else if (newtok) { if (once) ATT(true, true, false); else ATT(true, false, false); }
+  else if (once) ATT(false, true, false);
+  else ATT(false, false, false);
+#undef ATT
 }
 
 // prefill rows (q in qbuf, K/V already in the pages): NQ query vectors per block share every K / V load.  false: the score rows of

@@ -88,7 +88,8 @@ struct ixt_ctx {
   bf16_t* wt_op = nullptr;  // ixt_op_dot: the caller's row-major kernel in the tiled weight layout (grown on demand)
   size_t wt_cap = 0;
   size_t part_floats = 0;
-  int32_t *row_slot = nullptr, *row_pos = nullptr, *row_active = nullptr, *row_tok = nullptr, *new_tok = nullptr, *row_order = nullptr;
+  int32_t *row_slot = nullptr, *row_pos = nullptr, *row_active = nullptr, *row_tok = nullptr, *new_tok = nullptr;
+  int2* row_order = nullptr;
   AttnGeom geom{};
   // timing
   bool timing = false;

@@ -1231,7 +1231,7 @@ struct DecAttnArgs {
   bf16_t* out;        // [R][nq*hd] in xidx layout
   AttnGeom g;
   const bf16_t* qbuf; // NEWTOK = false: [R][nq][hd] finalised queries
-  const int32_t* row_order = nullptr;   // the row of a block's place (nullptr: that row)
+  const int2* row_order = nullptr;      // a place's row, which is its slot, too, and position (-1: idle)
   int rows;           // k_attn_small: blocks with blockIdx.y >= rows are prefetch blocks
   const u32x4* pf; size_t pf_n;
 };
@@ -1245,18 +1245,20 @@ template <bool ONCE> __device__ __forceinline__ u32x4 kv_load(const bf16_t* p) {
 // NEWTOK = false: prefill rows: q comes from qbuf and every key / value from the pages (k_qkv_finalize ran before this launch).
 // ONCE: no other row reads this row's pages (decode rows), so the 1 KiB of a load never comes back: streamed past the caches (256 rows of 350 to 700 keys:
 // 225 -> 197 us, 5.2 -> 6.0 TB/s; 48 rows 42.3 -> 40.0).  The rows of a prompt share theirs.
-// Blocks take their rows longest first (row_order; sums are a row's own): a long row among the last ones ran on alone, and 48 rows of 300 to 630 keys, whose 768 blocks are on
-// the chip at once, were spread over the CUs as they came.  48 rows 39.5 -> 37.4 us, 256 rows 196.4 -> 192.8 (6.1 TB/s).  Every second run of blocks the other way round,
-// so that those of a CU add up alike, gave no more: 37.3 and 193 for runs of 4, 8, 16 and 32 rows.
-template <int HD, int GQ, bool NEWTOK, bool ONCE>
+// ORDERED: rows longest first (row_order: a place holds all that a block asks for first; sums are a row's own).  With at most eight blocks a CU a long row among the last ones ran on alone, and 48 rows of
+// 300 to 630 keys, whose 768 blocks are on the chip at once, were spread over the CUs as they came; heads of 128, 16 a row, us by place / longest first: 33 rows of <= 900 keys 43.5 / 42.1, 48 of
+// <= 630 39.5 / 37.4, 64 of <= 600 51.1 / 48.0, 128 of <= 900 126.5 / 121.7, 100 of <= 200 34.5 / 34.3; 12 heads of 64, 64 rows of <= 100 13.9 / 13.3.  Every second run of blocks the other way round,
+// so that those of a CU add up alike, gave no more.  With more blocks it costs as often as it gives: 256 rows of <= 400 / 500 / 700 keys 113.6 / 134.4 / 191.0 by place, 117.6 / 142.2 / 188.4 in order.
+template <int HD, int GQ, bool NEWTOK, bool ONCE, bool ORDERED = false>
 __global__ __launch_bounds__(256) void k_attn_decode(DecAttnArgs a) {
   extern __shared__ __attribute__((aligned(16))) float sm[];
   const AttnGeom& g = a.g;
   // heads fastest: the 16 blocks of a row read 16 adjacent 8 KiB pieces of each page
-  const int kvh = blockIdx.x, r = ONCE && a.row_order != nullptr ? a.row_order[blockIdx.y] : (int)blockIdx.y;
+  const int2 place = ORDERED ? a.row_order[blockIdx.y] : make_int2(blockIdx.y, 0);
+  const int kvh = blockIdx.x, r = place.x;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int n_out = g.nq * HD;
-  if (!a.row_active[r]) {
+  if (ORDERED ? place.y < 0 : !a.row_active[r]) {
     for (int i = tid; i < GQ * HD; i += 256) a.out[xidx(r, kvh * GQ * HD + i, n_out)] = 0;
     return;
   }
@@ -1268,13 +1270,13 @@ __global__ __launch_bounds__(256) void k_attn_decode(DecAttnArgs a) {
   float* psum = ebuf + (size_t)GQ * tp;         // [mpg]
   float* wred = psum + ((g.mpg + 3) & ~3);        // [8]
   float* sbs = wred + 8;                        // [nsb_max][HD] super-block sums of the head being finished
-  const int pos = a.row_pos[r];
+  const int pos = ORDERED ? place.y : a.row_pos[r];
   const int kv_len = pos + 1;
   const int pages = (kv_len + g.P - 1) / g.P;
   const int nsb = (pages + IXT_SB - 1) / IXT_SB;
   const int ppw = 64 / g.P;
   constexpr int half = HD / 2;
-  const int32_t* prow = a.page_map + (size_t)a.row_slot[r] * g.mpg;
+  const int32_t* prow = a.page_map + (size_t)(ORDERED ? r : a.row_slot[r]) * g.mpg;
   const int QN = g.nq * HD, KN = g.nkv * HD;
 
   // Score work of this wave as a flat list of half tiles: tile i = keys of pages (wave + 4 i) ppw .., half h = d-chunks
@@ -2314,7 +2316,7 @@ static __global__ __launch_bounds__(64) void k_pages_advance(PageStateDev s) {
 // deactivates the row instead of letting it write through a stale page_map entry), and -- check_len, ixt_generate -- the position is
 // the one the page manager has just advanced to (sequence_lengths - 1): a slot that was prefilled but not inserted yet carries the
 // previous occupant's next_pos and stays idle until MaxEngine.insert.
-// row_order (or nullptr): the rows as k_attn_decode's blocks take them, longest first, equals in order, idle rows last.  B * B compares out of the LDS: 12.4 us instead of 4.6 at 256 rows.
+// row_order (or nullptr): the rows as k_attn_decode's blocks take them, longest first, equals in order, idle rows last.  B * B compares out of the LDS: 6.3 us instead of 4.7 at 200 rows (12.4 with two keys a compare).
 // Blocks 1 + i, where the pass's first launch is k_step or k_mid: the embedding of row i, and zeros in that launch's counters.  gave: of the pass to come.
 // grid = 1 (+ B), block 256
 struct FrontRows { const bf16_t* embedding; bf16_t* h0; int E; int32_t* cnt; int ncnt; };
@@ -2324,7 +2326,7 @@ __device__ __forceinline__ void front_row(const FrontRows& f, int row, int rows,
   for (int i = row * 256 + threadIdx.x; i < f.ncnt; i += rows * 256) f.cnt[(size_t)i * 32] = 0;
 }
 static __global__ __launch_bounds__(256) void k_decode_front(PageStateDev s, int advance, int32_t* row_slot, int32_t* row_pos, int32_t* row_active, int32_t* row_tok, const int32_t* tokens, const int32_t* pos,
-                                                             int Tmax, int B, FrontRows f, int32_t* gave, int32_t* row_order) {
+                                                             int Tmax, int B, FrontRows f, int32_t* gave, int2* row_order) {
   __shared__ __attribute__((aligned(16))) int32_t need[IXT_MAX_GROUPS], got[IXT_MAX_GROUPS];
   if (blockIdx.x > 0) return front_row(f, blockIdx.x - 1, B, tokens[blockIdx.x - 1]);
   if (threadIdx.x == 0) *gave = 0;
@@ -2335,19 +2337,22 @@ static __global__ __launch_bounds__(256) void k_decode_front(PageStateDev s, int
     bool act = s.has_active_page[i] != 0 && p >= 0 && p < Tmax && p / s.P < s.num_pages_used[i];
     if (advance) act = act && p == s.sequence_lengths[i] - 1;
     row_slot[i] = i; row_pos[i] = act ? p : 0; row_active[i] = act ? 1 : 0; row_tok[i] = tokens[i];
-    need[i] = act ? p : -1;                                     // (nobody else's: the page advance is through)
+    need[i] = (min(act ? p + 1 : 0, (1 << 18) - 1) << 12) + IXT_MAX_GROUPS - 1 - i;      // longer rows first, equals in order (nobody else's: the page advance is through)
   }
   if (row_order == nullptr) return;                             // whole block
-  for (int i = B + threadIdx.x; i < ((B + 3) & ~3); i += 256) need[i] = -2;
+  for (int i = B + threadIdx.x; i < ((B + 15) & ~15); i += 256) need[i] = -1;
   __syncthreads();
   for (int i = threadIdx.x; i < B; i += 256) {
     const int mine = need[i];
     int at = 0;
-    for (int j = 0; j < B; j += 4) {
-      const int4 v = *reinterpret_cast<const int4*>(need + j);
-      at += (v.x > mine || (v.x == mine && j < i)) + (v.y > mine || (v.y == mine && j + 1 < i)) + (v.z > mine || (v.z == mine && j + 2 < i)) + (v.w > mine || (v.w == mine && j + 3 < i));
+    for (int j = 0; j < B; j += 16) {
+      int4 v[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) v[k] = *reinterpret_cast<const int4*>(need + j + 4 * k);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) at += (v[k].x > mine) + (v[k].y > mine) + (v[k].z > mine) + (v[k].w > mine);
     }
-    row_order[at] = i;
+    row_order[at] = make_int2(i, row_active[i] ? row_pos[i] : -1);        // (its own stores)
   }
 }
 // Behind it: a slot's token out of the sampling pairs of its row, and the slot's state (maxengine.py:913-935).  By a launch of its own behind the step's graph, into the caller's own result rows

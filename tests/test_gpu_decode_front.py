@@ -17,9 +17,9 @@ def test_steps_with_an_idle_slot(slots):
   run_pair(cfg, H.synth.synth_weights(cfg, slots), prompts, steps=6)
 
 
-@pytest.mark.parametrize("slots, heads", [(33, 16), (130, 4), (128, 4), (256, 2)])
+@pytest.mark.parametrize("slots, heads", [(33, 16), (130, 4), (128, 4), (256, 2), (257, 8)])
 def test_rows_of_mixed_lengths(slots, heads):
-  """512 blocks of attention and more: rows go to them longest first; short, long, equal and idle ones among each other."""
+  """512 to 2048 blocks of attention: rows go to them longest first; short, long, equal and idle ones among each other.  More: as they lie."""
   cfg = H.make_config(per_device_batch_size=float(slots), max_prefill_predict_length=64, max_target_length=96, pagedattn_num_pages=5 * slots + 3, pagedattn_tokens_per_page=32,
                       base_num_decoder_layers=1, base_num_query_heads=heads, base_num_kv_heads=heads)
   prompts = [(H.synth.synth_prompt(cfg.vocab_size, 64, i)[0], 1 + (37 * i) % 64 if i % 3 else 40) for i in range(slots - 1)]
