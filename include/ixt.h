@@ -397,7 +397,7 @@ int ixt_set_sampling_ranges(ixt_ctx* ctx, const int32_t* lo_hi, int nranges);
  *   "ring_mid_rows"          passes of the Gemma blocks and prompts' passes of the llama blocks take it from this many rows (default 17), decode steps of the
  *                            llama blocks and unembeddings from 16 more, unless ring_min_rows is above 128
  *   "ring_cfg"               0 (default): tile chosen per shape; 1: 128 x 128, 2: 128 rows x 64 columns, 3: 64 x 32, 4: 256 x 128, 5: 64 x 64,
- *                            6: 64 x 16, 7: 128 x 128 with 32-k chunks, two blocks on a CU
+ *                            6: 64 x 16, 7: 128 x 128 with 32-k chunks, two blocks on a CU, 8: 128 x 192 (not gated units, unembeddings and the ring layout)
  *   "ring_split"             1: ixt_op_dot's ring GEMM runs split over the 512-k chains (one f32 slice per chain)
  *   "ring_wlayout"           1: ixt_op_dot stores its weights in the ring layout ([n/128][k/64][16 fragments]: one sequential stream per block)
  *   "attn_tile"              1 (default): prefill calls of at least "attn_tile_min_rows" rows (default 64) run the tiled attention, 16 (other
