@@ -138,11 +138,6 @@ __device__ __forceinline__ uint32_t ta_pack2(float lo, float hi) {      // one v
 __device__ __forceinline__ tbf16x8 ta_pack(const tf32x4& a, const tf32x4& b) {
   return __builtin_bit_cast(tbf16x8, u32x4{ta_pack2(a[0], a[1]), ta_pack2(a[2], a[3]), ta_pack2(b[0], b[1]), ta_pack2(b[2], b[3])});
 }
-__device__ __forceinline__ float ta_max3(float a, float b, float c) {     // (fmaxf quiets each operand first: two more a score)
-  float r;
-  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-  return r;
-}
 // ixt_exp of a number that is not positive: the same value by an instruction less (the whole number out of the sum's last bits instead of a conversion and a scaling)
 __device__ __forceinline__ float ta_exp(float x) {
   x = fmaxf(x, -80.0f);
@@ -270,7 +265,7 @@ __global__ __launch_bounds__(256, HELD ? 2 : D == 64 ? 4 : 3) void k_t_attn_fwd(
   float m = -3e38f, sum = 0.0f, rsum;
   auto highest = [&](const tf32x4 (&s)[4]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int kt = 0; kt < 4; ++kt) m = ta_max3(ta_max3(m, s[kt][0], s[kt][1]), s[kt][2], s[kt][3]);
+    for (int kt = 0; kt < 4; ++kt) m = fmaxf(fmaxf(fmaxf(fmaxf(m, s[kt][0]), s[kt][1]), s[kt][2]), s[kt][3]);      // (two instructions)
   };
   auto exps = [&](tf32x4 (&s)[4]) __attribute__((always_inline)) {
 #pragma unroll

@@ -102,3 +102,11 @@ def test_no_load_of_memory_into_registers_in_asm():
     with open(os.path.join(build.CSRC, n), encoding="utf-8") as f:
       for text in re.findall(r'asm(?: volatile)?\s*\(\s*"((?:[^"\\]|\\.)*)"', f.read()):
         assert not re.search(r"(?:global|buffer|flat|scratch)_load_(?!lds)", text), (n, text)
+
+
+def test_no_vector_arithmetic_in_asm():
+  """A matrix product's result may be read only some wait states behind it; the compiler keeps them for the instructions that it knows, and in asm knows none."""
+  for n in sorted(os.listdir(build.CSRC)):
+    with open(os.path.join(build.CSRC, n), encoding="utf-8") as f:
+      for text in re.findall(r'asm(?: volatile)?\s*\(\s*"((?:[^"\\]|\\.)*)"', f.read()):
+        assert not re.search(r"\bv_\w+", text), (n, text)
