@@ -29,6 +29,12 @@ typedef struct ixt_trainer ixt_trainer;
 const char* ixt_train_last_error(void);
 /* maxtext_utils.setup_training_state (state shapes) + activation workspaces for one batch of [batch, seq_len]. */
 int ixt_train_create(const ixt_train_config* cfg, ixt_trainer** out);
+/* The same with a say in how attention goes: IXT_TRAIN_ATTENTION_AUTO is ixt_train_create; _WALK: scores, softmax and products in one launch (head_dim 64 or 128, seq_len at
+ * most 4096; IXT_ERR_UNSUPPORTED elsewhere); _MEMORY: one behind the other, through memory (any size). */
+#define IXT_TRAIN_ATTENTION_AUTO 0
+#define IXT_TRAIN_ATTENTION_WALK 1
+#define IXT_TRAIN_ATTENTION_MEMORY 2
+int ixt_train_create_attention(const ixt_train_config* cfg, int attention, ixt_trainer** out);
 int ixt_train_destroy(ixt_trainer* t);
 /* The flat parameter layout: `count` tensors, tensor i = `numel` f32 values at `offset` (elements) of the flat buffers, row-major with
  * MaxText's kernel shapes; `name` is the unscanned tree path ("params/decoder/layers_3/mlp/wi_0/kernel"). */

@@ -93,7 +93,9 @@ static void add_param(ixt_trainer* t, const std::string& name, long numel, long*
   t->total += (numel + 63) / 64 * 64;   // 256-byte aligned segments
 }
 
-extern "C" int ixt_train_create(const ixt_train_config* c, ixt_trainer** out) {
+extern "C" int ixt_train_create(const ixt_train_config* c, ixt_trainer** out) { return ixt_train_create_attention(c, IXT_TRAIN_ATTENTION_AUTO, out); }
+extern "C" int ixt_train_create_attention(const ixt_train_config* c, int attention, ixt_trainer** out) {
+  if (attention < IXT_TRAIN_ATTENTION_AUTO || attention > IXT_TRAIN_ATTENTION_MEMORY) return t_set_err(IXT_ERR_INVALID, "train step: attention %d", attention);
   if (!c || !out) return t_set_err(IXT_ERR_INVALID, "null argument");
   if (c->num_kv_heads <= 0 || c->num_query_heads % c->num_kv_heads) return t_set_err(IXT_ERR_INVALID, "train step: num_query_heads %% num_kv_heads != 0");
   if (c->head_dim % 8 || c->emb_dim % 8 || c->mlp_dim % 8 || c->vocab_size % 8 || c->seq_len % 8)
@@ -133,6 +135,8 @@ extern "C" int ixt_train_create(const ixt_train_config* c, ixt_trainer** out) {
   t->Sp = ((long)S + 63) / 64 * 64;
   t->Sp += t->Sp / 64 % 2 == 0 ? 64 : 0;
   t->walk = (t->D == 64 || t->D == 128) && S <= TA_MOST && S * (size_t)(QN > t->Sp ? QN : t->Sp) * 2 < (size_t)1 << 32;
+  if (attention == IXT_TRAIN_ATTENTION_WALK && !t->walk) return fail(t_set_err(IXT_ERR_UNSUPPORTED, "train step: no walks over the keys with heads of %d, %d tokens a row", t->D, t->S));
+  if (attention == IXT_TRAIN_ATTENTION_MEMORY) t->walk = false;
   if (!t->walk) t->Sp = S;
   A(tmalloc(t, &t->pb, (size_t)t->total + (size_t)E * (t->Vp - V)));
   t->act.resize(t->L);

@@ -267,32 +267,46 @@ __global__ __launch_bounds__(256, HELD ? 2 : D == 64 ? 4 : 3) void k_t_attn_fwd(
 #pragma unroll
     for (int kt = 0; kt < 4; ++kt) m = fmaxf(fmaxf(fmaxf(fmaxf(m, s[kt][0]), s[kt][1]), s[kt][2]), s[kt][3]);      // (two instructions)
   };
-  auto exps = [&](tf32x4 (&s)[4]) __attribute__((always_inline)) {
+  // least: a lane's least one (of keys that are not seen, too) as a word, whose order is that of numbers that are not negative
+  auto exps = [&](tf32x4 (&s)[4], int& least) __attribute__((always_inline)) {
 #pragma unroll
     for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) s[kt][i] = ta_exp(s[kt][i] - m);
+      for (int i = 0; i < 4; ++i) {
+        s[kt][i] = ta_exp(s[kt][i] - m);
+        least = min(least, __float_as_int(s[kt][i]));
+      }
   };
+  const int most = 0x7fffffff;
+  auto small = [](int least) __attribute__((always_inline)) { return __any(least < __float_as_int(0x1p-96f)); };
   tf32x4 o[DT];
 #pragma unroll
   for (int d = 0; d < DT; ++d) o[d] = tf32x4(0.0f);
   bf16_t* const prow = t.P + ((long)bh * S + row) * t.ld + 8 * q;         // (to the end of the tile: zeros past the last key)
   const bool real = qw + r16 < S;
+  // with a weight below 2^-96 among them they are divided, as k_t_softmax_fwd_wave has it (the quotient by 1 that follows changes nothing)
+  auto divide = [&](tf32x4 (&s)[4]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) s[kt][i] = s[kt][i] / sum;
+  };
   auto zeros = [&](int k0) __attribute__((always_inline)) {
     if (real) *reinterpret_cast<u32x4*>(prow + k0) = *reinterpret_cast<u32x4*>(prow + k0 + 32) = u32x4(0u);
   };
-  // weights of the tile of the keys from k0 on, and their product with its values
-  auto values = [&](tf32x4 (&s)[4], uint32_t img, int k0) __attribute__((always_inline)) {
+  // weights of the tile of the keys from k0 on, and their product with its values.  The quotient by the reciprocal and two corrections, the last of which rounds as a division does where no residue
+  // is lost below the normal numbers
+  auto values = [&](tf32x4 (&s)[4], float by, float rby, uint32_t img, int k0) __attribute__((always_inline)) {
 #pragma unroll
     for (int st = 0; st < 2; ++st) {
 #pragma unroll
       for (int kt = 2 * st; kt < 2 * st + 2; ++kt)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {                                     // the quotient by the reciprocal and two corrections, as k_t_softmax_fwd_wave has it
+        for (int i = 0; i < 4; ++i) {
           const float e = s[kt][i];
-          float x = e * rsum;
-          x = __builtin_fmaf(__builtin_fmaf(-x, sum, e), rsum, x);
-          s[kt][i] = __builtin_fmaf(__builtin_fmaf(-x, sum, e), rsum, x);
+          float x = e * rby;
+          x = __builtin_fmaf(__builtin_fmaf(-x, by, e), rby, x);
+          s[kt][i] = __builtin_fmaf(__builtin_fmaf(-x, by, e), rby, x);
         }
       const tbf16x8 p = ta_pack(s[2 * st], s[2 * st + 1]);
       if (real) *reinterpret_cast<u32x4*>(prow + k0 + st * 32) = __builtin_bit_cast(u32x4, p);
@@ -331,17 +345,21 @@ __global__ __launch_bounds__(256, HELD ? 2 : D == 64 ? 4 : 3) void k_t_attn_fwd(
       }
 #pragma unroll
       for (int j = 0; j < TA_HELD; ++j) {
-        if (who[j] == TA_SOME) unseen(s[j], see[j], -INFINITY);
-        if (who[j] != TA_NONE) highest(s[j]);
+        if (who[j] == TA_ALL) highest(s[j]);
+        if (who[j] != TA_SOME) continue;
+        tf32x4 seen[4] = {s[j][0], s[j][1], s[j][2], s[j][3]};           // (the scores stay: least would be that of -INFINITY)
+        unseen(seen, see[j], -INFINITY);
+        highest(seen);
       }
       m = ta_max4(m);
+      int least = most;
 #pragma unroll
       for (int j = 0; j < TA_HELD; ++j) {
         if (who[j] == TA_NONE) {
 #pragma unroll
           for (int kt = 0; kt < 4; ++kt) s[j][kt] = tf32x4(0.0f);
         } else {
-          exps(s[j]);
+          exps(s[j], least);
           if (who[j] == TA_SOME) unseen(s[j], see[j], 0.0f);
         }
       }
@@ -349,6 +367,11 @@ __global__ __launch_bounds__(256, HELD ? 2 : D == 64 ? 4 : 3) void k_t_attn_fwd(
 #pragma unroll
       for (int w = 0; w < 4; ++w) run[w] = ta_run(s[w][0] + s[w + 4][0], s[w][1] + s[w + 4][1], s[w][2] + s[w + 4][2], s[w][3] + s[w + 4][3]);
       sum = run[0] + run[1] + run[2] + run[3];
+      if (__builtin_expect(small(least), false)) {
+#pragma unroll
+        for (int j = 0; j < TA_HELD; ++j) divide(s[j]);
+        sum = 1.0f;
+      }
       rsum = 1.0f / sum;
       const int vbuf = ((in.last - from) / 2 + 1) & 1;                    // the stage that the first values came to
 #pragma unroll
@@ -361,7 +384,7 @@ __global__ __launch_bounds__(256, HELD ? 2 : D == 64 ? 4 : 3) void k_t_attn_fwd(
         for (int u = 0; u < 2; ++u) {
           if (j + u < in.first || j + u > in.last) continue;              // (in front of and behind what is kept)
           if (who[2 * p + u] == TA_NONE) zeros(j * 64 + u * 64);
-          else values(s[2 * p + u], (uint32_t)((buf * 2 + u) * IMG * 2), j * 64 + u * 64);
+          else values(s[2 * p + u], sum, rsum, (uint32_t)((buf * 2 + u) * IMG * 2), j * 64 + u * 64);
         }
       }
     }
@@ -401,7 +424,8 @@ __global__ __launch_bounds__(256, HELD ? 2 : D == 64 ? 4 : 3) void k_t_attn_fwd(
       }
       const int who = scores(s, see, (uint32_t)(img * IMG * 2), k0, skj);
       if (who != TA_NONE) {
-        exps(s);
+        int least;
+        exps(s, least = most);
         if (who == TA_SOME) unseen(s, see, 0.0f);
 #pragma unroll
         for (int kt = 0; kt < 4; ++kt) l[kt] += s[kt];
@@ -430,8 +454,11 @@ __global__ __launch_bounds__(256, HELD ? 2 : D == 64 ? 4 : 3) void k_t_attn_fwd(
       ta_here(skj);
       if (j < in.last) keys.fetch(next, k0 + 64);
       const int who = scores(s, see, (uint32_t)(img * IMG * 2), k0, skj);
-      if (who != TA_NONE) exps(s);
+      int least = most;
+      if (who != TA_NONE) exps(s, least);
       if (who == TA_SOME) unseen(s, see, 0.0f);
+      const bool divided = small(least);
+      if (__builtin_expect(divided, false)) divide(s);
       if (j < in.last) {
         asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(TaStage<D>::NJ) : "memory");   // the values
         lds_barrier();
@@ -441,7 +468,7 @@ __global__ __launch_bounds__(256, HELD ? 2 : D == 64 ? 4 : 3) void k_t_attn_fwd(
         ta_turn();
       }
       if (who == TA_NONE) zeros(k0);
-      else values(s, (uint32_t)(v * IMG * 2), k0);
+      else values(s, divided ? 1.0f : sum, divided ? 1.0f : rsum, (uint32_t)(v * IMG * 2), k0);
       img = next;
     }
   }

@@ -50,6 +50,7 @@ def _signatures(lib):
   vp, ci, cf = ctypes.c_void_p, ctypes.c_int, ctypes.c_float
   lib.ixt_train_last_error.restype = ctypes.c_char_p
   lib.ixt_train_create.argtypes, lib.ixt_train_create.restype = [ctypes.POINTER(IxtTrainConfig), ctypes.POINTER(vp)], ci
+  lib.ixt_train_create_attention.argtypes, lib.ixt_train_create_attention.restype = [ctypes.POINTER(IxtTrainConfig), ci, ctypes.POINTER(vp)], ci
   lib.ixt_train_destroy.argtypes = [vp]
   lib.ixt_train_total_numel.argtypes, lib.ixt_train_total_numel.restype = [vp], ctypes.c_int64
   lib.ixt_train_param_count.argtypes, lib.ixt_train_param_count.restype = [vp], ci
@@ -78,7 +79,8 @@ def _sp():
 
 
 class Trainer:
-  def __init__(self, config: Any, batch: Optional[int] = None, seq_len: Optional[int] = None, logits_chunk: int = 0, exchange: str = "auto"):
+  def __init__(self, config: Any, batch: Optional[int] = None, seq_len: Optional[int] = None, logits_chunk: int = 0, exchange: str = "auto", attention: str = "auto"):
+    """attention: "auto", "walk" or "memory" (ixt_train_create_attention)."""
     if not torch.cuda.is_available():
       raise _lib.IxtError("Trainer needs a ROCm GPU: there is no CPU path")
     if str(config.rope_type).lower() != "default":
@@ -95,7 +97,7 @@ class Trainer:
     c.rope_min_timescale, c.rope_max_timescale = float(config.rope_min_timescale), float(config.rope_max_timescale)
     c.batch, c.seq_len, c.logits_chunk = self.B, self.S, int(logits_chunk)
     self._h = ctypes.c_void_p()
-    _check(self.lib, self.lib.ixt_train_create(ctypes.byref(c), ctypes.byref(self._h)))
+    _check(self.lib, self.lib.ixt_train_create_attention(ctypes.byref(c), ("auto", "walk", "memory").index(attention), ctypes.byref(self._h)))
     n = int(self.lib.ixt_train_total_numel(self._h))
     z = lambda: torch.zeros((n,), dtype=torch.float32, device=self.device)
     self.params, self.grads, self.mu, self.nu = z(), z(), z(), z()

@@ -65,3 +65,53 @@ def test_wide_walks():
   for k, g in grads.items():
     ref = o["grads"][k]
     assert float((g - ref).norm()) <= 2e-2 * float(ref.norm()) + 1e-12, k
+
+
+def loss_and_gradients(cfg, params, batch, attention):
+  import torch
+  tr = importlib.import_module("maxtext-indextts2_amd.train")
+  trainer = tr.Trainer(cfg, attention=attention)
+  trainer.load_params(params)
+  loss = trainer.forward_backward(batch).clone()
+  grads = {k: v.clone() for k, v in trainer.param_views(trainer.grads).items()}
+  del trainer
+  torch.cuda.synchronize()
+  return loss, grads
+
+
+# (score of a small weight, score of another one): behind the largest, 0, the quotients e^small / (1 + e^other) lie so near the middle of two bf16 numbers that a quotient by the reciprocal and
+# two corrections, of whose residues the last bits are lost below 2^-149, rounds to the other one of them
+NEAR_THE_MIDDLE = [(-74.8192139, -0.589346707), (-74.8979492, -0.433190912), (-75.588623, -2.45409417), (-75.5889893, -0.0813442543), (-76.536499, -0.188589051), (-76.6171875, -0.341206789),
+                   (-76.8988037, -1.67407274), (-76.9376221, -0.160699293), (-77.0887451, -2.77235889), (-77.1809082, -3.24232554), (-77.3969727, -0.267132759), (-77.4521484, -0.107146807)]
+
+
+@pytest.mark.parametrize("length", [64, 584])
+def test_small_weights_are_quotients(length):
+  """Weights below 2^-96: a division, as through memory.  Segments of three tokens, each a feature of its own (their norm is 8): the largest score, another one, and the query, whose own score is
+  the small one; a score is three bf16 features of a key.  The gradient of the value kernel has the small weight times the output's gradient in the query's row."""
+  import torch
+  cfg = train_config(base_emb_dim=64, base_num_query_heads=1, base_num_kv_heads=1, head_dim=64, base_mlp_dim=72, vocab_size=264, max_target_length=length, per_device_batch_size=1.0,
+                     base_num_decoder_layers=1)
+  params, n = f32_params(cfg, 8), len(NEAR_THE_MIDDLE)
+  params["params/token_embedder/embedding"].reshape(264, 64)[:64] = np.eye(64)
+  a = "params/decoder/layers_0/self_attention/"
+  q, k = params[a + "query/kernel"].reshape(64, 64), params[a + "key/kernel"].reshape(64, 64)
+  q[:], k[:] = 0.0, 0.0
+  q[:, :3] = 0.125
+  params["params/decoder/layers_0/pre_self_attention_layer_norm/scale"][:] = 1.0
+  for token, score in enumerate(np.float32([0.0] + [x for pair in NEAR_THE_MIDDLE for x in pair[::-1]])):
+    for part in range(3):
+      cut = np.float32(score).view(np.uint32) & np.uint32(0xffff0000)
+      k[token, part] = cut.view(np.float32) / 8
+      score -= cut.view(np.float32)
+    assert score == 0.0
+  b = AT.synthetic_batch(cfg, 7)
+  at = np.arange(3 * n)
+  for key, value in (("inputs", np.stack([0 * at[::3], 1 + 2 * at[:n], 2 + 2 * at[:n]], 1).reshape(-1)), ("inputs_segmentation", 1 + at // 3), ("targets_segmentation", at % 3 // 2)):
+    b[key][:] = 0
+    b[key][0, :3 * n] = value
+  b["inputs_position"][:] = 0
+  (loss, grads), (want, ref) = (loss_and_gradients(cfg, params, b, how) for how in ("walk", "memory"))
+  v = a + "value/kernel"
+  assert torch.equal(loss, want) and bool((ref[v].view(64, 64)[2:2 + 2 * n:2].abs().amax(1) > 0).all())
+  assert torch.equal(grads[v], ref[v])
