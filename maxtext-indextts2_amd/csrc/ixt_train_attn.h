@@ -1,8 +1,9 @@
 // ixt_train_attn.h -- causal attention of the training step, heads of 64 and 128: scores, softmax and products in one launch forward, two backward.
 //
-// Every number is the one that products and softmax through memory give (k_tgemm, k_t_softmax_*), bit for bit: the same products of 32 features or rows in the same order, the same exponentials, row
-// sums in the same order.  (16 layers of bf16 carry any other last bit on to every gradient: with weights and sums rounded elsewhere, as precise, a step's gradients differed by as much as either is
-// from 64 bits.)
+// With a query head a kv head every number is the one that products and softmax through memory give (k_tgemm, k_t_softmax_*), bit for bit: the same products of 32 features or rows in the same
+// order, the same exponentials, row sums in the same order, the same quotients.  (16 layers of bf16 carry any other last bit on to every gradient: with weights and sums rounded elsewhere, as precise, a
+// step's gradients differed by as much as either is from 64 bits.)  With groups of query heads that holds for the outputs and the queries' gradients; dK and dV of a group are one chain of f32 sums
+// over its heads here, a sum a head, added up in f32, there.
 // Forward: a wave has 16 queries in registers and walks the keys, 64 at a time: S^T = K Q^T, so that a lane holds the scores of ONE query (four keys a register quad) and hands its
 // weights to O^T += V^T P^T as they are.  Three walks: maxima; sums of exponentials; weights, which go to memory for the way back, and outputs.  Rows of at most 512 tokens are held and walked once.
 // Backward: k_t_attn_dq is the same walk over P and dP = dO V^T, twice: the rows' sums, then dS, to memory, and dQ; k_t_attn_dkv the transposed one, a wave 16 N keys, of P and dS.

@@ -79,6 +79,55 @@ def loss_and_gradients(cfg, params, batch, attention):
   return loss, grads
 
 
+def walks_and_memory(cfg, segments, seed):
+  """Both ways over the same batch; no token twice, whose rows of the embedding's gradient would be added up in any order."""
+  rng, b = np.random.default_rng(seed), AT.synthetic_batch(cfg, 7)
+  rows, length = b["inputs"].shape
+  b["inputs"][:] = rng.permutation(int(cfg.vocab_size))[:rows * length].reshape(rows, length)
+  b["inputs_segmentation"][:] = [SEGMENTS[segments](length, rng) for _ in range(rows)]
+  b["targets_segmentation"][:] = b["inputs_segmentation"]
+  b["inputs_position"][:] = np.arange(length)
+  params = f32_params(cfg, 11)
+  return [loss_and_gradients(cfg, params, b, how) for how in ("walk", "memory")]
+
+
+@pytest.mark.parametrize("segments", list(SEGMENTS))
+@pytest.mark.parametrize("dim,heads,length,rows", [(64, 2, 64, 2), (64, 3, 136, 1), (64, 2, 512, 1), (64, 4, 584, 2), (64, 1, 2056, 1), (128, 2, 128, 1), (128, 1, 520, 1), (128, 1, 1096, 1)])
+def test_walks_give_the_numbers_of_the_products_through_memory(dim, heads, length, rows, segments):
+  """A query head a kv head: the loss and every gradient bit for bit, so that no row of any tile can be wrong."""
+  import torch
+  cfg = train_config(base_emb_dim=64, base_num_query_heads=heads, base_num_kv_heads=heads, head_dim=dim, base_mlp_dim=72, vocab_size=(rows * length + 8) // 8 * 8, max_target_length=length,
+                     per_device_batch_size=float(rows), base_num_decoder_layers=2)
+  (loss, grads), (want, ref) = walks_and_memory(cfg, segments, length + dim)
+  assert torch.equal(loss, want)
+  assert [k for k in grads if not torch.equal(grads[k], ref[k])] == []
+
+
+# 512 blocks of 128 rows of query heads, of kv heads, of neither: 32 rows a wave on the way back for queries, for both, for neither
+@pytest.mark.parametrize("dim,heads,kv,length,rows", [(64, 4, 2, 584, 1), (128, 6, 2, 136, 2), (64, 16, 8, 200, 16), (128, 16, 4, 200, 16), (64, 32, 16, 200, 16), (128, 32, 16, 200, 16)])
+def test_groups_of_query_heads(dim, heads, kv, length, rows):
+  """The gradients of keys and values are added up over a group in one chain of f32 sums by the walk, and head by head through memory.  Both round to bf16 once: of two f32 sums of at most 4800
+  terms some 2^-24 4800^(1/2) of the sum apart, one in a thousand lands on another bf16 number, 2^-8 of its size away; 2^-8 1000^(-1/2) = 1.2e-4 of the norm, and nothing else of one layer differs."""
+  import torch
+  cfg = train_config(base_emb_dim=64, base_num_query_heads=heads, base_num_kv_heads=kv, head_dim=dim, base_mlp_dim=72, vocab_size=(rows * length + 8) // 8 * 8, max_target_length=length,
+                     per_device_batch_size=float(rows), base_num_decoder_layers=1)
+  (loss, grads), (want, ref) = walks_and_memory(cfg, "packed", length + dim)
+  assert torch.equal(loss, want)
+  for k in grads:
+    if any(part in k for part in ("key/", "value/", "token_embedder", "pre_self_attention")):
+      assert float((grads[k] - ref[k]).norm()) <= 5e-4 * float(ref[k].norm()), k
+    else:
+      assert torch.equal(grads[k], ref[k]), k
+
+
+def test_walks_are_refused_where_there_are_none():
+  tr = importlib.import_module("maxtext-indextts2_amd.train")
+  for dim, length in ((32, 64), (64, 4104)):
+    cfg = train_config(base_emb_dim=64, head_dim=dim, base_mlp_dim=72, vocab_size=264, max_target_length=length, per_device_batch_size=1.0, base_num_decoder_layers=1)
+    with pytest.raises(NotImplementedError):
+      tr.Trainer(cfg, attention="walk")
+
+
 # (score of a small weight, score of another one): behind the largest, 0, the quotients e^small / (1 + e^other) lie so near the middle of two bf16 numbers that a quotient by the reciprocal and
 # two corrections, of whose residues the last bits are lost below 2^-149, rounds to the other one of them
 NEAR_THE_MIDDLE = [(-74.8192139, -0.589346707), (-74.8979492, -0.433190912), (-75.588623, -2.45409417), (-75.5889893, -0.0813442543), (-76.536499, -0.188589051), (-76.6171875, -0.341206789),
