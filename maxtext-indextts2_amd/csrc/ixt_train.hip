@@ -13,6 +13,7 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <algorithm>
 #include <initializer_list>
 #include <string>
 #include <vector>
@@ -63,7 +64,7 @@ struct ixt_trainer {
   std::vector<LayerAct> act;
   bf16_t *h_final = nullptr, *xn_f = nullptr, *rope_sin = nullptr, *rope_cos = nullptr;
   float* r_f = nullptr;
-  bool walk = false;        // attention by ixt_train_attn.h: heads of 64 or 128, rows of at most TA_MOST tokens, operands of a batch row and weights of a head within the reach of a 32-bit offset
+  bool walk = false;        // attention by ixt_train_attn.h (walk_pays): heads of 64 or 128, rows of at most TA_MOST tokens, operands of a batch row and weights of a head within the reach of a 32-bit offset
   long Sp;                  // columns between rows of P and dS: S, or whole tiles of 64, an odd number of them (walk)
   int2* reach = nullptr;
   // workspaces
@@ -93,6 +94,19 @@ static void add_param(ixt_trainer* t, const std::string& name, long numel, long*
   t->total += (numel + 63) / 64 * 64;   // 256-byte aligned segments
 }
 
+// Walks over the keys (ixt_train_attn.h) where they are the faster way.  A row of tokens is walked by one block of 64 rows after the other's start, 64 keys behind 64, three times: with few blocks the
+// chip waits for the longest walk, while the products through memory have tiles of all keys at once; the more query heads a kv head has, the more launches these take.  us a layer (width 256, forward
+// and backward, all tokens of one segment), walks / through memory, one row: 16 heads of 128, 512 tokens 205 / 195, 1024 297 / 288, 1536 406 / 414, 2048 499 / 579; 12 heads of 64, 512 tokens 159 / 160,
+// 1024 224 / 216, 1536 296 / 302; 4 heads of 128, 128 tokens 122 / 124, 4096 719 / 608; 2 heads of 64, 256 tokens 120 / 122, 4096 528 / 409.  In groups of two, 4 heads of 64, 576 tokens 173 / 186, 2048
+// 343 / 320; 8 heads of 128, 512 tokens 189 / 195, 2048 454 / 435; in groups of four, 8 heads of 128, 1024 tokens 321 / 331.  Of 398 such shapes (1 to 128 heads, 64 to 4096 tokens, groups of 1 to 32) the
+// rule takes the slower way by more than 1 % for 11, by 13 % at most (4 heads of 128 in one group, 576 tokens); walks alone would for 106, by up to twice the time.
+static bool walk_pays(long heads, int G, int D, int S) {
+  const bool narrow = D == 64;
+  if (S <= (narrow ? 256 : 128)) return true;
+  const long blocks = heads * ((S + 63) / 64);
+  if (G > 1) return S <= 512 || heads * G >= (narrow ? 16 : 32) || blocks >= 512;
+  return blocks >= (S <= 512 ? (narrow ? 64 : 192) : (narrow ? 288 : 320));
+}
 extern "C" int ixt_train_create(const ixt_train_config* c, ixt_trainer** out) { return ixt_train_create_attention(c, IXT_TRAIN_ATTENTION_AUTO, out); }
 extern "C" int ixt_train_create_attention(const ixt_train_config* c, int attention, ixt_trainer** out) {
   if (attention < IXT_TRAIN_ATTENTION_AUTO || attention > IXT_TRAIN_ATTENTION_MEMORY) return t_set_err(IXT_ERR_INVALID, "train step: attention %d", attention);
@@ -136,7 +150,7 @@ extern "C" int ixt_train_create_attention(const ixt_train_config* c, int attenti
   t->Sp += t->Sp / 64 % 2 == 0 ? 64 : 0;
   t->walk = (t->D == 64 || t->D == 128) && S <= TA_MOST && S * (size_t)(QN > t->Sp ? QN : t->Sp) * 2 < (size_t)1 << 32;
   if (attention == IXT_TRAIN_ATTENTION_WALK && !t->walk) return fail(t_set_err(IXT_ERR_UNSUPPORTED, "train step: no walks over the keys with heads of %d, %d tokens a row", t->D, t->S));
-  if (attention == IXT_TRAIN_ATTENTION_MEMORY) t->walk = false;
+  if (attention == IXT_TRAIN_ATTENTION_MEMORY || (attention == IXT_TRAIN_ATTENTION_AUTO && !walk_pays((long)t->B * t->H, t->G, t->D, t->S))) t->walk = false;
   if (!t->walk) t->Sp = S;
   A(tmalloc(t, &t->pb, (size_t)t->total + (size_t)E * (t->Vp - V)));
   t->act.resize(t->L);
@@ -147,8 +161,8 @@ extern "C" int ixt_train_create_attention(const ixt_train_config* c, int attenti
     A(tmalloc(t, &a.a, T * F)); A(tmalloc(t, &a.b, T * F)); A(tmalloc(t, &a.act, T * F)); A(tmalloc(t, &a.r1, T)); A(tmalloc(t, &a.r2, T));
   }
   A(tmalloc(t, &t->h_final, T * E)); A(tmalloc(t, &t->xn_f, T * E)); A(tmalloc(t, &t->r_f, T));
-  // (behind the logits the scores hold the parts of a cut product, too)
-  t->scores_n = t->walk ? (V >= 65536 ? (size_t)4 * t->Tc * E : 0) : BH * S * S;
+  // (behind the logits the scores hold the parts of a cut product, too: whichever way attention goes, the cut stays a matter of the shape alone)
+  t->scores_n = std::max(t->walk ? (size_t)0 : BH * S * S, V >= 65536 ? (size_t)4 * t->Tc * E : (size_t)0);
   if (t->scores_n > 0) A(tmalloc(t, &t->scores, t->scores_n));
   A(tmalloc(t, &t->dh, T * E)); A(tmalloc(t, &t->dxn, T * E));
   // (a chunk's logits are bf16, at the front of a buffer of f32 words that holds the parts of cut weight gradients later on)

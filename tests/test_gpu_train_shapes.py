@@ -65,11 +65,11 @@ def test_train_step_at_tile_edges(shape):
   torch.cuda.synchronize()
 
 
-def step_and_oracle(cfg, params, batch):
+def step_and_oracle(cfg, params, batch, attention="auto"):
   """One step of the trainer and of the oracle: their metrics, and the gradients of both."""
   import torch
   tr = importlib.import_module("maxtext-indextts2_amd.train")
-  trainer = tr.Trainer(cfg)
+  trainer = tr.Trainer(cfg, attention=attention)
   trainer.load_params(params)
   m = trainer.train_step(batch)
   o = TO.TrainOracle(cfg, params).train_step(batch)

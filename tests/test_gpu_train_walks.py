@@ -34,7 +34,7 @@ def test_walks(dim, heads, kv, length, rows, segments):
     b["inputs_segmentation"][r] = seg
     b["targets_segmentation"][r] = seg
     b["inputs_position"][r] = np.arange(length)
-  m, grads, o = step_and_oracle(cfg, f32_params(cfg, 11), b)
+  m, grads, o = step_and_oracle(cfg, f32_params(cfg, 11), b, "walk")
   assert abs(m["learning/loss"] - o["learning/loss"]) <= 1e-4 * abs(o["learning/loss"])
   for k, g in grads.items():
     ref = o["grads"][k]
@@ -60,7 +60,7 @@ def test_wide_walks():
   b = AT.synthetic_batch(cfg, 9)
   b["inputs_segmentation"][:] = (np.arange(152)[None] < 152 - 9 * np.arange(16)[:, None]).astype(np.int32)
   b["targets_segmentation"][:] = b["inputs_segmentation"]
-  m, grads, o = step_and_oracle(cfg, f32_params(cfg, 12), b)
+  m, grads, o = step_and_oracle(cfg, f32_params(cfg, 12), b, "walk")
   assert abs(m["learning/loss"] - o["learning/loss"]) <= 1e-4 * abs(o["learning/loss"])
   for k, g in grads.items():
     ref = o["grads"][k]
@@ -79,7 +79,7 @@ def loss_and_gradients(cfg, params, batch, attention):
   return loss, grads
 
 
-def walks_and_memory(cfg, segments, seed):
+def walks_and_memory(cfg, segments, seed, ways=("walk", "memory")):
   """Both ways over the same batch; no token twice, whose rows of the embedding's gradient would be added up in any order."""
   rng, b = np.random.default_rng(seed), AT.synthetic_batch(cfg, 7)
   rows, length = b["inputs"].shape
@@ -88,7 +88,7 @@ def walks_and_memory(cfg, segments, seed):
   b["targets_segmentation"][:] = b["inputs_segmentation"]
   b["inputs_position"][:] = np.arange(length)
   params = f32_params(cfg, 11)
-  return [loss_and_gradients(cfg, params, b, how) for how in ("walk", "memory")]
+  return [loss_and_gradients(cfg, params, b, way) for way in ways]
 
 
 @pytest.mark.parametrize("segments", list(SEGMENTS))
@@ -164,3 +164,25 @@ def test_small_weights_are_quotients(length):
   v = a + "value/kernel"
   assert torch.equal(loss, want) and bool((ref[v].view(64, 64)[2:2 + 2 * n:2].abs().amax(1) > 0).all())
   assert torch.equal(grads[v], ref[v])
+
+
+# (the last shape that goes through memory and the first that is walked, of rows beyond 512 tokens, of 512, and in groups)
+@pytest.mark.parametrize("dim,heads,kv,length,rows", [(64, 7, 7, 640, 4), (64, 8, 8, 576, 4), (128, 8, 8, 640, 3), (128, 8, 8, 640, 4), (64, 9, 9, 448, 1), (64, 10, 10, 448, 1), (128, 12, 12, 512, 1),
+                                                      (128, 12, 12, 512, 2), (64, 6, 3, 520, 1), (64, 8, 4, 520, 1), (128, 14, 7, 520, 1), (128, 16, 8, 520, 1)])
+def test_either_way_by_sizes(dim, heads, kv, length, rows):
+  """What is taken without a word about it has the loss of both and the gradients of one of them, bit for bit."""
+  import torch
+  cfg = train_config(base_emb_dim=64, base_num_query_heads=heads, base_num_kv_heads=kv, head_dim=dim, base_mlp_dim=72, vocab_size=(rows * length + 8) // 8 * 8, max_target_length=length,
+                     per_device_batch_size=float(rows), base_num_decoder_layers=1)
+  (got, taken), *both = walks_and_memory(cfg, "packed", length, ("auto", "walk", "memory"))
+  assert all(torch.equal(got, loss) for loss, _ in both)
+  assert any(all(torch.equal(taken[k], way[k]) for k in taken) for _, way in both)
+
+
+def test_large_vocabularies_cut_their_sums_alike():
+  """From 65536 columns the gradient of the normed rows is cut in four parts, which the scores' buffer holds; short rows have few scores."""
+  import torch
+  cfg = train_config(base_emb_dim=64, base_num_query_heads=1, base_num_kv_heads=1, head_dim=64, base_mlp_dim=72, vocab_size=65536, max_target_length=64, per_device_batch_size=1.0,
+                     base_num_decoder_layers=1)
+  (loss, grads), (want, ref) = walks_and_memory(cfg, "packed", 3)
+  assert torch.equal(loss, want) and [k for k in grads if not torch.equal(grads[k], ref[k])] == []
