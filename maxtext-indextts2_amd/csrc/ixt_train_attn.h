@@ -263,7 +263,7 @@ __global__ __launch_bounds__(256, HELD ? 2 : D == 64 ? 4 : 3) void k_t_attn_fwd(
 #pragma unroll
       for (int i = 0; i < 4; ++i) s[kt][i] = see >> (kt * 4 + i) & 1u ? s[kt][i] : with;
   };
-  float m = -3e38f, sum = 0.0f, rsum;
+  float m = -INFINITY, sum = 0.0f, rsum;
   auto highest = [&](const tf32x4 (&s)[4]) __attribute__((always_inline)) {
 #pragma unroll
     for (int kt = 0; kt < 4; ++kt) m = fmaxf(fmaxf(fmaxf(fmaxf(m, s[kt][0]), s[kt][1]), s[kt][2]), s[kt][3]);      // (two instructions)

@@ -186,3 +186,27 @@ def test_large_vocabularies_cut_their_sums_alike():
                      base_num_decoder_layers=1)
   (loss, grads), (want, ref) = walks_and_memory(cfg, "packed", 3)
   assert torch.equal(loss, want) and [k for k in grads if not torch.equal(grads[k], ref[k])] == []
+
+
+@pytest.mark.parametrize("length", [64, 584])
+def test_rows_of_lowest_scores(length):
+  """A row all of whose scores lie below -3e38, as through memory: its own maximum is taken off them.  Two tokens a segment, the second one's weights are 1 and e^-80, not two halves."""
+  import torch
+  cfg = train_config(base_emb_dim=64, base_num_query_heads=1, base_num_kv_heads=1, head_dim=64, base_mlp_dim=72, vocab_size=264, max_target_length=length, per_device_batch_size=1.0,
+                     base_num_decoder_layers=1)
+  params = f32_params(cfg, 8)
+  params["params/token_embedder/embedding"].reshape(264, 64)[:64] = np.eye(64)
+  a = "params/decoder/layers_0/self_attention/"
+  q, k = params[a + "query/kernel"].reshape(64, 64), params[a + "key/kernel"].reshape(64, 64)
+  q[:], k[:] = 0.0, 0.0
+  q[:, 0] = 0.125
+  params["params/decoder/layers_0/pre_self_attention_layer_norm/scale"][:] = 1.0
+  k[0, 0], k[1, 0] = -0.9375 * 2.0**125, -0.96875 * 2.0**125         # (a token's norm is 8: scores of -3.19e38 and -3.30e38)
+  b = AT.synthetic_batch(cfg, 7)
+  at = np.arange(length)
+  b["inputs"][:], b["inputs_segmentation"][:], b["inputs_position"][:] = at % 2, 1 + at // 2, 0
+  b["targets_segmentation"][:] = 1
+  (loss, grads), (want, ref) = (loss_and_gradients(cfg, params, b, how) for how in ("walk", "memory"))
+  v = a + "value/kernel"
+  assert torch.equal(loss, want) and bool(torch.isfinite(want).all())
+  assert torch.equal(grads[v], ref[v]) and float(ref[v].norm()) > 0
