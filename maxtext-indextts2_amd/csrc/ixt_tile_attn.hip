@@ -1,4 +1,5 @@
 // ixt_tile_attn.hip -- launches of k_attn_mtile (an object of its own: it compiles beside the others).
+#include "ixt_rounds.h"
 #include "ixt_tile_attn.h"
 
 #include <algorithm>
@@ -36,13 +37,13 @@ static void mtile_attn_t(TileAttnArgs ta, hipStream_t st) {
       return;
     }
   }
-  // Heads of 128, a block a CU (below): what is left behind the last whole round of 256 blocks, at most half of one, goes by two blocks a value and scores ahead, too: the first
-  // rows, whose keys are the fewest.  16 heads, us: 100 rows at <= 1124 / 2148 / 3172 keys 44.8 / 69.7 / 100.4, now 25.5 / 39.0 / 61.0 and the scores before them 14.5 / 20.0 / 25.9; 828 rows at
-  // <= 3900 keys, 3 rounds and 64 blocks, 421, now 316 + 57 + 16.  The other rows by moved pointers: a first row as the kernel's argument spills 36 bytes more, 330 instead of 316.
+  // Heads of 128, a block a CU (below): what is left behind the last whole round of 256 blocks, at most half of one, goes by two blocks a value and scores ahead, too (tiles_split): the
+  // first rows, whose keys are the fewest.  16 heads, us: 100 rows at <= 1124 / 2148 / 3172 keys 44.8 / 69.7 / 100.4, now 25.5 / 39.0 / 61.0 and the scores before them 14.5 / 20.0 / 25.9; 828
+  // rows at <= 3900 keys, 3 rounds and 64 blocks, 345, now 281 + 44 + 10.  The other rows by moved pointers: a first row as the kernel's argument spills 36 bytes more, 330 instead of 316.
   if constexpr (HD == 128) {
     constexpr int PER16 = 16 / TQ;                       // tiles of 16 rows, the unit of `out`
-    const int round = std::max(1, 256 / ta.g.nkv), over = tiles < round ? tiles : tiles % round / PER16 * PER16;
-    if (ta.scores != nullptr && ta.lmax > 1024 && over > 0 && over * ta.g.nkv <= 128) {
+    const int over = ta.scores != nullptr && ta.lmax > 1024 ? tiles_split(tiles, ta.g.nkv, PER16, ta.lmax - ta.R) : 0;
+    if (over > 0) {
       TileAttnArgs rest = ta;
       rest.parts = 2;
       rest.R = std::min(ta.R, over * TQ);

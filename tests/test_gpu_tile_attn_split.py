@@ -10,8 +10,9 @@ from test_gpu_tile_attn_matrix import _same
 pytestmark = pytest.mark.gpu
 
 
-# (16 kv heads: 16 tiles a round; tiles of 16, 8 and 4 rows)
-@pytest.mark.parametrize("nq,nkv,length,chunk", [(16, 16, 1400, 340), (16, 16, 2500, 350), (16, 16, 3500, 500), (32, 16, 1500, 170), (32, 16, 1300, 301), (16, 4, 2300, 300)])
+# (16 kv heads: 16 tiles a round; tiles of 16, 8 and 4 rows.  Chunks of 300, 170 and 260 rows behind 2560 keys and more: split in part, in units of 1, 2 and 4 tiles, 20 heads in rounds that they do not fill)
+@pytest.mark.parametrize("nq,nkv,length,chunk", [(16, 16, 1400, 340), (16, 16, 2500, 350), (16, 16, 3500, 500), (32, 16, 1500, 170), (32, 16, 1300, 301), (16, 4, 2300, 300),
+                                                  (16, 16, 3400, 300), (16, 4, 3400, 300), (32, 16, 3250, 170), (20, 20, 3200, 260)])
 def test_split_tiles_equal_the_row_kernel(nq, nkv, length, chunk):
   cfg = H.make_config(base_emb_dim=256, base_num_query_heads=nq, base_num_kv_heads=nkv, head_dim=128, base_mlp_dim=384, base_num_decoder_layers=1,
                       vocab_size=1024, model_name="default", per_device_batch_size=1.0, use_chunked_prefill=True, prefill_chunk_size=512,
