@@ -1041,6 +1041,11 @@ static int hybrid_mixer_scan(ixt_ctx* c, const HLayer& L, const HLayer& W, int R
   return scan_mix<T>(c, L, W, in, low, dt, R, nseg_max, single, st);
 }
 
+// Waves of a block of k_delta_step, key dimensions rounded up to 16 RP.  Eight shorten the block's own chain; a CU has two of them where it has three of four (RP 8: 89 and 131 registers), one where it
+// has two (RP 32), and of few value columns half of their lanes have none.  us, four / eight waves, bf16, key x value size: 128 x 128, 136 blocks 12.2 / 10.9, 512 18.9 / 18.2, 544 23.0 / 24.0, 768 23.8 /
+// 26.8, 1024 39.7 / 34.6, 2048 68.6 / 67.2; 64 x 64, 512 blocks 10.2 / 10.3, 768 12.1 / 12.6, 2048 23.2 / 27.6; 32 x 128, 1600 blocks 19.1 / 23.9; 256 x 256, 800 blocks 109 / 106; 512 x 512, 256 blocks 123 /
+// 118, 400 205 / 214.  float32 alike.
+static int delta_step_waves(int RP, long blocks) { return RP <= 4 ? (blocks > 512 ? 4 : 8) : RP == 8 ? (blocks > 512 && blocks <= 768 ? 4 : 8) : RP == 32 && blocks > 256 ? 4 : 8; }
 template <typename T>
 static int hybrid_mixer_delta(ixt_ctx* c, const HLayer& L, const HLayer& W, int R, int nseg_max, bool single, hipStream_t st) {
   HybridModel* m = c->hy;
@@ -1062,11 +1067,15 @@ static int hybrid_mixer_delta(ixt_ctx* c, const HLayer& L, const HLayer& W, int 
                      (const u32x4*)lowx, (const u32x4*)W.low.w, W.low.Kp};
     const dim3 grid(g.H, R);
     const size_t lds = sizeof(float) * (3 * g.dp + 2 * g.dv + (inside ? g.d + g.dv : 0));
+    const bool four = !inside && delta_step_waves(g.dp / 16, (long)R * g.H) == 4;
+#define HSTEP_L(RP_, LOW_, NW_) hipLaunchKernelGGL((k_delta_step<T, RP_, LOW_, NW_>), grid, dim3(64 * NW_), lds, st, da, (T*)m->act, W.o.Kp); break
 #define HSTEP(RP_) case RP_: \
-    if constexpr (sizeof(T) == 2) if (inside) { hipLaunchKernelGGL((k_delta_step<T, RP_, true>), grid, dim3(512), lds, st, da, (T*)m->act, W.o.Kp); break; } \
-    hipLaunchKernelGGL((k_delta_step<T, RP_, false>), grid, dim3(512), lds, st, da, (T*)m->act, W.o.Kp); break
+    if constexpr (sizeof(T) == 2) if (inside) { HSTEP_L(RP_, true, 8); } \
+    if constexpr (RP_ != 16) if (four) { HSTEP_L(RP_, false, 4); } \
+    HSTEP_L(RP_, false, 8)
     switch (g.dp / 16) { HSTEP(1); HSTEP(2); HSTEP(4); HSTEP(8); HSTEP(16); HSTEP(32); default: return set_err(IXT_ERR_UNSUPPORTED, "delta rule: %d key dims", g.d); }
 #undef HSTEP
+#undef HSTEP_L
     LAUNCHCHK();
     return IXT_OK;
   }

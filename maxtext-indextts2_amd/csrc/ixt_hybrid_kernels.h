@@ -1647,13 +1647,14 @@ __global__ __launch_bounds__(256) void k_delta_scan(DeltaScanArgs a) {
 }
 
 // One token per row (decode): everything between the projections of a gated-delta layer in one launch.  Block = (head, row): its whole state matrix is
-// requested first and travels while the convolutions, unit vectors, decays and the step size are computed; then the recurrence on 32 columns at a
+// requested first and travels while the convolutions, unit vectors, decays and the step size are computed; then the recurrence on 4 NW columns at a
 // time, the head's norm and output gate.  A query / key head that several heads share is computed by each of them; the first one keeps its tail.
 // LOW (bf16, at most 16 rows): the second low-rank product's columns of the head, too, instead of a launch in front: its operand `x` holds all rows, and a row's sums are those of
-// k_sdot (one product after the other, k ascending).  The weights of a head, at most 128 KB for 256 columns, are shared by its blocks, which are on one XCD; they come beside the state, and what bounds the block is the chain
-// of its loads, barriers and sums: 8 rows x 16 heads of 128 x 128 12.0 us, as without them, where the launch in front took 4.8 and its start.  Eight waves a block, half the state's columns each has of
-// four.  More rows than a 16-row operand, more low-rank columns than a wave's registers hold and heads that share a column tile leave the product to its launch.
-// grid (H, R), block 512, dynamic LDS = (3 dp + 2 dv, LOW + d + dv) floats.
+// k_sdot (one product after the other, k ascending).  The weights of a head, at most 128 KB for 256 columns, are shared by its blocks, which are on one XCD where the heads are a multiple of 8; they come
+// beside the state, and what bounds the block is the chain of its loads, barriers and sums: 8 rows x 16 heads of 128 x 128 12.0 us, as without them, where the launch in front took 4.8 and its start.
+// More rows than a 16-row operand, more low-rank columns than a wave's registers hold and heads that share a column tile leave the product to its launch.
+// NW: eight waves a block, half the state's columns each has of four (delta_step_waves).
+// grid (H, R), block 64 NW, dynamic LDS = (3 dp + 2 dv, LOW + d + dv) floats.
 #define DELTA_LOW_K 256
 struct DeltaStepArgs {
   Slices t, t2; DeltaGeom g;
@@ -1663,11 +1664,11 @@ struct DeltaStepArgs {
   float *tails, *state;
   const u32x4 *x, *w; int lowK;                                // LOW: fragments of 16 rows, of 16 columns; k, at most DELTA_LOW_K
 };
-template <typename T, int RP, bool LOW>
-__global__ __launch_bounds__(512) void k_delta_step(DeltaStepArgs a, T* __restrict__ out, int Kp) {
-  constexpr int DP = 16 * RP, NJ = RP <= 8 ? 4 : (RP == 16 ? 2 : 1);      // columns in flight per lane
+template <typename T, int RP, bool LOW, int NW>
+__global__ __launch_bounds__(64 * NW) void k_delta_step(DeltaStepArgs a, T* __restrict__ out, int Kp) {
+  constexpr int DP = 16 * RP, NT = 64 * NW, NC = 4 * NW, NJ = (RP <= 8 ? 32 : RP == 16 ? 16 : 8) / NW;      // columns of a block's round; a lane has NJ of them in flight
   extern __shared__ __attribute__((aligned(16))) float lm[];
-  __shared__ float red[8], red2[8];
+  __shared__ float red[NW], red2[NW];
   float *qs = lm, *ks = lm + DP, *gs = lm + 2 * DP, *vs = lm + 3 * DP, *os = vs + a.g.dv, *ls = os + a.g.dv;
   const DeltaGeom& g = a.g;
   const int r = blockIdx.y, h = blockIdx.x, kh = h / (g.H / g.KH), tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, sub = lane & 15, cl = wave * 4 + (lane >> 4);
@@ -1677,7 +1678,7 @@ __global__ __launch_bounds__(512) void k_delta_step(DeltaStepArgs a, T* __restri
   auto fetch = [&](int i0) __attribute__((always_inline)) {               // two of the head's column tiles a wave
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
-      const int i = min(i0 + wave + 8 * k, ltiles - 1), tile = i < dtiles ? h * dtiles + i : ((g.og2 + h * g.dv) >> 4) + i - dtiles;
+      const int i = min(i0 + wave + NW * k, ltiles - 1), tile = i < dtiles ? h * dtiles + i : ((g.og2 + h * g.dv) >> 4) + i - dtiles;
 #pragma unroll
       for (int s = 0; s < LS; ++s)
         if (s < nsteps) wf[k][s] = a.w[((size_t)tile * nsteps + s) * 64 + lane];
@@ -1696,7 +1697,7 @@ __global__ __launch_bounds__(512) void k_delta_step(DeltaStepArgs a, T* __restri
   float S[NJ][RP];
 #pragma unroll
   for (int j = 0; j < NJ; ++j) {
-    const int col = cl + 32 * j;
+    const int col = cl + NC * j;
 #pragma unroll
     for (int i = 0; i < RP; ++i) S[j][i] = (start > 0 && col < g.dv) ? sp[(size_t)col * DP + delta_row<RP>(sub, i)] : 0.0f;
   }
@@ -1706,11 +1707,11 @@ __global__ __launch_bounds__(512) void k_delta_step(DeltaStepArgs a, T* __restri
   float* tail_out = tb + (size_t)(par ^ 1) * tsz;
   const float gate0 = !LOW && tid < g.dv ? a.t2.at(r, g.og2 + h * g.dv + tid) : 0.0f, beta_z = a.t.at(r, g.ob + h), ea = expf(a.a_log[h]);
   if constexpr (LOW) {
-    for (int i0 = 0; i0 < ltiles; i0 += 16) {
+    for (int i0 = 0; i0 < ltiles; i0 += 2 * NW) {
       if (i0 > 0) fetch(i0);
 #pragma unroll
       for (int k = 0; k < 2; ++k) {
-        const int i = i0 + wave + 8 * k;
+        const int i = i0 + wave + NW * k;
         f32x4 acc = f32x4(0.0f);
 #pragma unroll
         for (int s = 0; s < LS; ++s)
@@ -1726,7 +1727,7 @@ __global__ __launch_bounds__(512) void k_delta_step(DeltaStepArgs a, T* __restri
   const bool first = h % (g.H / g.KH) == 0;          // of the heads that share a query / key head
   float qq = 0.0f, kk = 0.0f;
   // one channel per thread and round: queries, keys, decays, values side by side
-  for (int i = tid; i < 3 * DP + g.dv; i += 512) {
+  for (int i = tid; i < 3 * DP + g.dv; i += NT) {
     const int kind = i < DP ? 0 : (i < 2 * DP ? 1 : (i < 3 * DP ? 2 : 3)), c = i - kind * DP;
     float x = 0.0f;
     if (kind == 2) {
@@ -1746,10 +1747,14 @@ __global__ __launch_bounds__(512) void k_delta_step(DeltaStepArgs a, T* __restri
   if (lane == 0) { red[wave] = qq; red2[wave] = kk; }
   __syncthreads();
   if constexpr (LOW) {                       // (every thread is here or none)
-    for (int c = tid; c < g.d; c += 512) gs[c] = decay(c, ls[c]);
+    for (int c = tid; c < g.d; c += NT) gs[c] = decay(c, ls[c]);
   }
-  auto eight = [](const float* v) { return ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7])); };
-  const float qn = 1.0f / sqrtf(eight(red) + 1e-6f) * (1.0f / sqrtf((float)g.d)), kn = 1.0f / sqrtf(eight(red2) + 1e-6f);
+  auto total = [](const float* v) {
+    float t = (v[0] + v[1]) + (v[2] + v[3]);
+    if constexpr (NW == 8) t += (v[4] + v[5]) + (v[6] + v[7]);
+    return t;
+  };
+  const float qn = 1.0f / sqrtf(total(red) + 1e-6f) * (1.0f / sqrtf((float)g.d)), kn = 1.0f / sqrtf(total(red2) + 1e-6f);
   if constexpr (LOW) __syncthreads();
   float qv[RP], kv[RP], gv[RP], qk = 0.0f;
 #pragma unroll
@@ -1759,18 +1764,18 @@ __global__ __launch_bounds__(512) void k_delta_step(DeltaStepArgs a, T* __restri
     qk = fmaf(qv[i], kv[i], qk);
   }
   qk = row16_sum(qk);
-  for (int c0 = 0; c0 < g.dv; c0 += 32 * NJ) {
+  for (int c0 = 0; c0 < g.dv; c0 += NC * NJ) {
     if (c0 > 0) {
 #pragma unroll
       for (int j = 0; j < NJ; ++j) {
-        const int col = c0 + cl + 32 * j;
+        const int col = c0 + cl + NC * j;
 #pragma unroll
         for (int i = 0; i < RP; ++i) S[j][i] = (start > 0 && col < g.dv) ? sp[(size_t)col * DP + delta_row<RP>(sub, i)] : 0.0f;
       }
     }
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
-      const int col = c0 + cl + 32 * j;
+      const int col = c0 + cl + NC * j;
       float ax = 0.0f, bx = 0.0f;
 #pragma unroll
       for (int i = 0; i < RP; ++i) { S[j][i] *= gv[i]; ax = fmaf(kv[i], S[j][i], ax); bx = fmaf(qv[i], S[j][i], bx); }
@@ -1786,15 +1791,15 @@ __global__ __launch_bounds__(512) void k_delta_step(DeltaStepArgs a, T* __restri
   }
   __syncthreads();
   float ss = 0.0f;
-  for (int c = tid; c < g.dv; c += 512) ss = fmaf(os[c], os[c], ss);
+  for (int c = tid; c < g.dv; c += NT) ss = fmaf(os[c], os[c], ss);
   ss = wave_sum(ss);
   if (lane == 0) red[wave] = ss;
   __syncthreads();
-  const float rs = 1.0f / sqrtf(eight(red) / (float)g.dv + a.eps);
-  for (int c = tid; c < g.dv; c += 512)
-    act_store1(out, r, h * g.dv + c, Kp, os[c] * rs * a.nw[c] * f32_sigmoid(LOW ? ls[g.d + c] : c < 512 ? gate0 : a.t2.at(r, g.og2 + h * g.dv + c)));
+  const float rs = 1.0f / sqrtf(total(red) / (float)g.dv + a.eps);
+  for (int c = tid; c < g.dv; c += NT)
+    act_store1(out, r, h * g.dv + c, Kp, os[c] * rs * a.nw[c] * f32_sigmoid(LOW ? ls[g.d + c] : c < NT ? gate0 : a.t2.at(r, g.og2 + h * g.dv + c)));
   if (h == g.H - 1)
-    for (int k = g.H * g.dv + tid; k < Kp; k += 512) act_store1(out, r, k, Kp, 0.0f);
+    for (int k = g.H * g.dv + tid; k < Kp; k += NT) act_store1(out, r, k, Kp, 0.0f);
 }
 
 // read-out: o / rms(o) * norm * sigmoid(gate) per head -> the output projection's operand (column h dv + c).  grid (R, ceil(H / 4)), block 256.

@@ -44,3 +44,10 @@ def test_sizes(tmp_path, heads, kv_heads, dim, vdim):
 def test_rows(tmp_path, slots):
   """Two layers of different low-rank columns: each row's own sums, nothing of the other layer's operand."""
   decoded(tmp_path, [VH.with_mlp(VH.delta(heads=3, kv_heads=3, dim=32, vdim=48, conv=3), None), VH.with_mlp(VH.delta(heads=2, kv_heads=1, dim=64, vdim=160, conv=4), None)], slots, 12)
+
+
+# (33 rows; key sizes 16, 64, 128 and 512.  528 blocks or 264: four waves a block; 792 and, with key size 256, any: eight)
+@pytest.mark.parametrize("heads,kv_heads,dim,vdim", [(16, 16, 16, 48), (16, 8, 48, 80), (16, 16, 128, 32), (24, 24, 120, 24), (16, 4, 144, 16), (8, 8, 264, 48)])
+def test_waves_of_a_block(tmp_path, heads, kv_heads, dim, vdim):
+  """More blocks than two a CU: by four waves where three blocks of them, but two of eight, are on a CU, or where a head has too few value columns for eight."""
+  decoded(tmp_path, [VH.with_mlp(VH.delta(heads=heads, kv_heads=kv_heads, dim=dim, vdim=vdim, conv=4), None)], 33, 4)
