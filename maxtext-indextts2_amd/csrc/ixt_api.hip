@@ -739,7 +739,9 @@ static void timing_end(ixt_ctx* c, hipStream_t st, int idx) {
 // 5: 31 (52 for two blocks of a CU), 3: 22, 6: 19, 7: 66 (122 for two).  The least estimate is within 6 % of the fastest tile on all but 3 of these 72
 // (within 12 %); the rule that looked at the number of 128 x 128 tiles alone took 62 us where this takes 40 (256 x 2304 outputs, K 9216) and 122 where this
 // takes 102 (1525 x 14336, K 2048).  Tile 8 (90) came later: what 256 x 128 leaves on a part of the CUs fills them all (6144 outputs, K 2048: 1024 rows 192 tiles -> 256, QKV 41.0 -> 34.7 us, 828 rows 41.1 -> 33.0;
-// 1592 rows, 2 rounds of 52 a XCD against tile 7's 78: 64.0 and 62.4).  192 x 128, whose odd row block of a wave is stored by itself: QKV 63.9 for 1592 rows, gated units 104.9 against 100.9, not taken.
+// 1592 rows, 2 rounds of 52 a XCD against tile 7's 78: 64.0 and 62.4).  Its 90 is of the present loops, not of the former ones; taken among the others' figures it is the faster one in every epilogue, us
+// of tile 8 / of what is taken without it: residuals 1600 x 2304 39.9 / 43.6, 1100 x 4096 46.2 / 47.9; tanh norms 1300 x 3072 46.9 / 55.8, 1600 x 2304 50.0 / 56.4; units without a gate 700 x 6144 29.4 / 33.1,
+// 300 x 14336 30.7 / 37.1; QKV, llama3.1 positions, 700 x 6144 50.8 / 61.7.  192 x 128, whose odd row block of a wave is stored by itself: QKV 63.9 for 1592 rows, gated units 104.9 against 100.9, not taken.
 // These are the times of the products' former loops.  With the present ones a chunk takes 60, 45, 31, 21, 14, 13 and 43 (73 for two of tile 7, 32 of tile 5), and a round 230 to 660 beside its
 // chunks, which no single figure a tile stands for: by the figures below the tile is 1.4 % off the fastest in the geometric mean of such launches, by a rule of two figures a tile 0.8 %.
 static int ring_pick(const ixt_ctx* c, int epi, int R, int N, bool routed, bool wring) {
