@@ -22,11 +22,12 @@ SHAPES = {
     "cut reductions": dict(base_emb_dim=768, base_num_query_heads=12, base_num_kv_heads=12, head_dim=64, base_mlp_dim=2048, vocab_size=6152, max_target_length=768, per_device_batch_size=3.0),
     # sums of two and of three products in 128 x 128 tiles (4096 x 832), reductions that end inside a chunk
     "sums in large tiles": dict(base_emb_dim=832, base_num_query_heads=13, base_num_kv_heads=13, head_dim=64, base_mlp_dim=1032, vocab_size=264, max_target_length=512, per_device_batch_size=8.0),
-    # enough heads for the attention's largest tiles (256 x 256 scores, 256 x 128 outputs), rows 8 beyond a tile
+    # many heads, rows 8 beyond a tile: walks of 32 rows a wave on the way back; through memory the largest tiles (256 x 256 scores, 256 x 128 outputs)
     "large attention tiles": dict(base_emb_dim=72, base_num_query_heads=16, base_num_kv_heads=16, head_dim=128, base_mlp_dim=136, vocab_size=264, max_target_length=264, per_device_batch_size=16.0),
     # a vocabulary of an odd number of 128-byte lines: its rows lie as far apart as they are long, also from 4096 columns on
     "odd lines": dict(base_emb_dim=72, base_num_query_heads=2, base_num_kv_heads=2, head_dim=64, base_mlp_dim=136, vocab_size=4160, max_target_length=72, per_device_batch_size=2.0),
-    # softmax by a wave a row: the last rows of 512 columns' form, a few columns beyond it and beyond 1024
+    # walks of 512 tokens at most, which hold their scores, and of a few more; through memory (test_attention_through_memory_at_tile_edges) the softmax by a wave a row, the last rows of 512 columns'
+    # form, a few columns beyond it and beyond 1024
     "softmax 512": dict(base_emb_dim=64, base_num_query_heads=3, base_num_kv_heads=3, head_dim=64, base_mlp_dim=72, vocab_size=264, max_target_length=504, per_device_batch_size=1.0),
     "softmax 520": dict(base_emb_dim=64, base_num_query_heads=1, base_num_kv_heads=1, head_dim=64, base_mlp_dim=72, vocab_size=264, max_target_length=520, per_device_batch_size=2.0),
     "softmax 1032": dict(base_emb_dim=64, base_num_query_heads=2, base_num_kv_heads=1, head_dim=64, base_mlp_dim=72, vocab_size=264, max_target_length=1032, per_device_batch_size=1.0),
@@ -79,18 +80,29 @@ def step_and_oracle(cfg, params, batch, attention="auto"):
   return m, grads, o
 
 
-def one_step(cfg, params, batch, names=None):
+def one_step(cfg, params, batch, names=None, attention="auto"):
   """The loss and the gradients (`names`: of these tensors) at the tolerances above."""
-  m, grads, o = step_and_oracle(cfg, params, batch)
+  m, grads, o = step_and_oracle(cfg, params, batch, attention)
   assert abs(m["learning/loss"] - o["learning/loss"]) <= 1e-4 * abs(o["learning/loss"]), (m["learning/loss"], o["learning/loss"])
   for k in names or grads:
     err = float((grads[k] - o["grads"][k]).norm()) / (float(o["grads"][k].norm()) + 1e-12)
     assert err < 2e-2, (k, err)
 
 
+# 256 x 256 scores and 256 x 128 outputs; 128 x 128 scores and 128 x 64 outputs, of narrow heads and of wide ones; the softmax by a wave a row
+@pytest.mark.parametrize("sizes", ["large attention tiles", "softmax 512", "softmax 520", "softmax 1032", dict(base_num_query_heads=16, base_num_kv_heads=16, head_dim=64),
+                                   dict(base_num_query_heads=24, base_num_kv_heads=24, head_dim=96), dict(base_num_query_heads=32, base_num_kv_heads=16, head_dim=160)], ids=str)
+def test_attention_through_memory_at_tile_edges(sizes):
+  """The way that heads of other sizes and longer rows take, at the sizes of its larger tiles."""
+  sizes = SHAPES[sizes] if isinstance(sizes, str) else dict(base_emb_dim=72, base_mlp_dim=136, vocab_size=264, max_target_length=136, per_device_batch_size=8.0, **sizes)
+  cfg = train_config(**sizes)
+  one_step(cfg, f32_params(cfg, 8), packed_batch(cfg, 41), attention="memory")
+
+
+@pytest.mark.parametrize("attention", ["auto", "memory"])
 @pytest.mark.parametrize("drop", [58.0, 80.0])
 @pytest.mark.parametrize("length", [264, 520])
-def test_softmax_of_peaked_rows(length, drop):
+def test_softmax_of_peaked_rows(length, drop, attention):
   """Scores that lie `drop` below a row's others: weights down to 2^-94, whose quotients go by the reciprocal, and below 2^-96, for which the row is divided.  One token in seven has a key that
   every query scores so; all others have ordinary scores, and their probabilities, the loss and the gradients are what the oracle's are."""
   cfg = train_config(base_emb_dim=64, base_num_query_heads=2, base_num_kv_heads=2, head_dim=64, base_mlp_dim=72, vocab_size=264, max_target_length=length, per_device_batch_size=2.0)
@@ -106,7 +118,7 @@ def test_softmax_of_peaked_rows(length, drop):
   q[0, :, 31], k[1, :, 31] = 8.0, -drop / 8.0
   b = packed_batch(cfg, 41)
   b["inputs"][:, 3::7] = 7
-  one_step(cfg, params, b)
+  one_step(cfg, params, b, attention=attention)
 
 
 @pytest.mark.parametrize("vocab", [264, 16392, 200072])
