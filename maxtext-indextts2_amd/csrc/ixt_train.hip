@@ -271,9 +271,9 @@ template <int D, int N>
 static int attn_back_t(hipStream_t st, const TAttn& a, int what) {
   const int heads = a.B * (what == TA_DKV ? a.KVH : a.H);
   const dim3 grid((unsigned)((heads + 7) / 8 * 8 * ((a.S + 64 * N - 1) / (64 * N))));
-  TCHK((lds_room<&k_t_attn_dq<D, N>>(TA_LDS(D, 4))));
+  TCHK((lds_room<&k_t_attn_dq<D, N>>(TA_LDS_IMAGES(D, 4))));
   TCHK((lds_room<&k_t_attn_dkv<D, N>>(TA_LDS_DKV(D, N))));
-  if (what == TA_DQ) hipLaunchKernelGGL((k_t_attn_dq<D, N>), grid, dim3(256), TA_LDS(D, 4), st, a);
+  if (what == TA_DQ) hipLaunchKernelGGL((k_t_attn_dq<D, N>), grid, dim3(256), TA_LDS_IMAGES(D, 4), st, a);
   else hipLaunchKernelGGL((k_t_attn_dkv<D, N>), grid, dim3(256), TA_LDS_DKV(D, N), st, a);
   TLAUNCH();
   return IXT_OK;

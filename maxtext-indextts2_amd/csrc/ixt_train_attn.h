@@ -31,7 +31,8 @@ struct TAttn {
   long ld;
 };
 #define TA_MOST 4096                                    // tokens of a row (a word of 64 tiles)
-#define TA_LDS(D, IMAGES) ((IMAGES) * 64 * (D) * 2 + 32)   // images of 64 rows, ta_range's words
+#define TA_LDS_IMAGES(D, N) ((N) * 64 * (D) * 2)        // images of 64 rows
+#define TA_LDS(D, N) (TA_LDS_IMAGES(D, N) + 32)         // behind them ta_range's words
 #define TA_LDS_DKV(D, N) (2 * (2 * 32 * (D) * 2 + 2 * 32 * 64 * (N) * 2))   // two stages of 32 rows: queries, dO, P, dS
 template <int D>
 __device__ __forceinline__ int ta_swizzle(int row) {    // D / 8 pieces a row; of rows that share their low four bits it is the same
@@ -484,7 +485,7 @@ __global__ __launch_bounds__(256, HELD ? 2 : D == 64 ? 4 : 3) void k_t_attn_fwd(
 template <int D, int N>
 __global__ __launch_bounds__(256, 2) void k_t_attn_dq(TAttn t) {
   constexpr int KS = D / 32, DT = D / 16, IMG = 64 * D;
-  extern __shared__ __attribute__((aligned(16))) bf16_t lds[];            // four images, 8 words of ta_range
+  extern __shared__ __attribute__((aligned(16))) bf16_t lds[];            // four images
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, r16 = lane & 15, q = lane >> 4, S = t.S;
   int bh, nth;
   const int tiles = (S + 64 * N - 1) / (64 * N);
