@@ -9,10 +9,11 @@
 // Backward: k_t_attn_dq is the same walk over P and dP = dO V^T, twice: the rows' sums, then dS, to memory, and dQ; k_t_attn_dkv the transposed one, a wave 16 N keys, of P and dS.
 // What a walk need not look at: tiles beyond the diagonal, tiles in front of and behind the block's segments (ta_range; `reach` keeps them), and for a wave of one segment those of others: rows of
 // padding see none of the tokens.
-// What bounds it: forward, vector instructions: 17 a score for its exponential and the sum, 22 for the exponential and the quotient.  k_t_attn_dq: 0.35 GB of P twice and of dS once beside three
+// What bounds it: forward, vector instructions: 17 a score for its exponential and the sum, 23 for the exponential, the least one and the quotient.  k_t_attn_dq: 0.35 GB of P twice and of dS once beside three
 // products; k_t_attn_dkv the two of them once and two products.  LDS: stages of images of 64 (32) rows, filled by LDS-DMA a stage ahead, a barrier a stage.
-// Measured (us a layer, forward / dP, softmax's gradient, dQ / dK, dV; a fifth of the rows padding), through memory, before, and now: 128 heads of 128 x 2048 tokens 1018 / 1035 / 382, 446 / 392 / 250;
-// 48 heads of 64 x 512 43 / 37 / 17, 19 / 19 / 12.
+// Measured (us a layer, forward / dP, softmax's gradient, dQ / dK, dV; a fifth of the rows padding), through memory, before, and now: 128 heads of 128 x 2048 tokens 1018 / 1035 / 382, 462 / 392 / 250 (the
+// forward 449 before it looked for weights to divide); 48 heads of 64 x 512 43 / 37 / 17, 21 / 19 / 12.  In whole steps, whose rows
+// are half to all tokens, 464 / 430 / 258 and 22 / 20 / 13.
 //
 // Image: 16-byte pieces, piece c of row r at c ^ ta_swizzle(r): 16 rows at one piece (ds_read_b128), and 8 rows at one pair of pieces (ds_read_tr16_b64, columns to
 // lanes), lie on disjoint banks.  (Lanes step along a row by an exclusive or of addresses: the images lie at a multiple of 256 bytes, in front of everything else in LDS.)
